@@ -159,7 +159,7 @@ int ss2d_selective_scan_fwd_maps(const ss2d_scan_params *params, const void *x_t
  *               ZERO-INITIALISED by the caller (accumulated with atomics over the rows that share them);
  *               dD / ddelta_bias NULL exactly when D / delta_bias is NULL.
  * The forward states are recomputed inside the kernel, so the forward's `x` output is not needed.
- * Returns SS2D_ENOTSUP when ceil(seqlen/512) * dstate exceeds ~3000 (per-pass states kept in LDS).
+ * Returns SS2D_ENOTSUP for more than 32 states when ceil(seqlen/512) * dstate exceeds ~3000 (per-pass states kept in LDS).
  */
 typedef struct ss2d_scan_bwd_params {
     int32_t batch, dim, seqlen, dstate, n_groups, delta_dim;

@@ -57,6 +57,15 @@ CASES = [
     (1, 27, 1, 1, 520, 9, True),           # 27 channels in chunks of 14 + 13, delta rows shared by three channels
     (1, 24, 1, 1, 3136, None, True),       # one state, 7 passes, 6 channels per wavefront (pass-major kernel)
     (2, 10, 1, 1, 100, None, False),       # the same kernel without softplus, wavefronts with 3 and 2 channels
+    (3, 14, 2, 1, 49, None, True),         # rows that fit 64 lanes: one position per lane
+    (2, 12, 1, 1, 196, 4, True),           # one pass of 4 positions per lane; delta rows shared by three channels
+    (2, 9, 1, 1, 255, None, True),         # the same with rows that are read element by element
+    (1, 40, 1, 1, 4100, None, True),       # 9 passes, the last one 4 positions long; workgroups of 4 channels
+    (2, 10, 1, 2, 256, None, True),        # exactly one pass; one wavefront with two of its four states
+    (1, 8, 2, 5, 257, None, True),         # one position into the second pass; the last wavefront has one state
+    (2, 30, 1, 16, 784, None, True),       # 16 states, 4 passes, 30 channels in workgroups of 4 and fewer
+    (1, 6, 1, 32, 60, 2, False),           # the most states of this kernel, one position per lane, no softplus
+    (1, 4, 2, 40, 300, None, True),        # more: a wavefront per row
 ]
 
 
@@ -85,6 +94,18 @@ def test_scan_bwd_16bit_inputs(dtype, dout_float, dim, G):
     want = torch_ref.selective_scan_grads(u.float(), delta.float(), A, B.float(), C.float(), D, bias, dout.float(), True)
     got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, True, 1)
     assert got[0].dtype == dtype and got[1].dtype == dtype and got[3].dtype == dtype and got[2].dtype == torch.float32
+    compare(got, want, 3e-2, "16-bit")
+
+
+@pytest.mark.parametrize("dtype,dout_float", [(torch.bfloat16, True), (torch.float16, False)])
+@pytest.mark.parametrize("N,L", [(1, 196), (1, 49), (1, 1100), (16, 784), (16, 196), (16, 49), (3, 333)])
+def test_scan_bwd_16bit_row_lengths(N, L, dtype, dout_float):
+    """Every positions-per-lane variant of the register-summing kernels with 16-bit rows (bound: as above)."""
+    print("CASE scan-bwd-16-rows", N, L, dtype, dout_float, flush=True)
+    u, delta, A, B, C, D, bias, dout = make(N + L, 2, 20, 2, N, L, dtype)
+    dout = dout if dout_float else dout.to(dtype)
+    want = torch_ref.selective_scan_grads(u.float(), delta.float(), A, B.float(), C.float(), D, bias, dout.float(), True)
+    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, True, 1)
     compare(got, want, 3e-2, "16-bit")
 
 
