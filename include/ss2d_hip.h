@@ -235,6 +235,21 @@ int ss2d_cross_scan_1b1(const void *x, void *y, int B, int C, int H, int W, int 
                         int64_t y_dir_stride, int64_t y_chan_stride, void *stream);
 
 /*
+ * x_proj in scan order: the projection of SS2Dv2.forward_corev2 (classification/models/vmamba.py:605-607) applied to the map
+ * itself, each direction's rows written in ITS scan order (cross_scan1b1_fwd, csm_triton.py:88-131) -- what x_proj on the
+ * four scan-ordered copies of x would give.
+ *   x (B,D,H,W) contiguous; weight (4,C,D) contiguous, 16-byte aligned; both bf16 or fp16 (dtype)
+ *   out[k*out_dir_stride + c*out_chan_stride + b*out_batch_stride + j] = sum_d weight[k,c,d] * x[b,d,r_k(j)], fp32 sums,
+ *   rounded once; j in [0, Hp*Wp), r_k as in ss2d_cross_scan_1b1 on the Hp x Wp map whose top-left H x W part is x and
+ *   whose added positions project to 0.
+ * mask_row in [0, C] inserts a row at that index (the rows from there on move up by one) that is 1 at the added positions
+ * and 0 elsewhere; -1: none.  Returns SS2D_ENOTSUP for fp32, D not a multiple of 8, C > 96, maps of fewer than 8 positions or
+ * more than 2^31 elements per image.
+ */
+int ss2d_x_proj(const void *x, const void *weight, void *out, int B, int D, int C, int H, int W, int Hp, int Wp, int mask_row,
+                int64_t out_dir_stride, int64_t out_chan_stride, int64_t out_batch_stride, int dtype, void *stream);
+
+/*
  * Fused SS2D core for dstate = 1: CrossScan -> selective scan (softplus, fp32 state, fp32 "oflex" output) ->
  * CrossMerge in one kernel.  Replaces the three calls of SS2Dv2.forward_corev2
  * (classification/models/vmamba.py:604, 625-633, 638: cross_scan_fn, selective_scan, cross_merge_fn) for

@@ -156,6 +156,36 @@ def ss2d_core_hip(x, delta, Bs, Cs, As, Ds=None, delta_bias=None, delta_softplus
     return y
 
 
+X_PROJ_MAX_ROWS = 96
+
+
+def x_proj_fits(x, weight):
+    """True when ss2d_x_proj takes this map (B, D, H, W) and these weights (4, C, D)."""
+    return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype and x.shape[1] % 8 == 0
+            and x.shape[1] > 0 and weight.shape[1] <= X_PROJ_MAX_ROWS and x.shape[2] * x.shape[3] >= 8
+            and x.shape[1] * x.shape[2] * x.shape[3] < 2 ** 31 and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
+
+
+def x_proj_hip(x, weight, out, padded=None, mask_row=-1):
+    """weight (4, C, D) applied to the map x (B, D, H, W), each direction's rows in its scan order, written into ``out``: a
+    (B, 4, C', L') view with contiguous rows (any batch / direction / row strides), L' = H' * W' of the ``padded`` size
+    (default: H, W), C' = C, or C + 1 with a row at index ``mask_row`` that is 1 at the added positions (ss2d_x_proj)."""
+    _check(x.is_cuda and x.dim() == 4 and weight.dim() == 3 and weight.shape[0] == 4 and weight.shape[2] == x.shape[1],
+           "x_proj expects x (B, D, H, W) and weight (4, C, D)")
+    _check(x.dtype == weight.dtype == out.dtype and x.dtype in _DTYPE_CODE, "x_proj: one 16-bit dtype")
+    B, D, H, W = x.shape
+    Hp, Wp = padded or (H, W)
+    C = weight.shape[1]
+    _check(tuple(out.shape) == (B, 4, C + (mask_row >= 0), Hp * Wp) and (out.stride(3) == 1 or out.shape[3] == 1),
+           "x_proj: out must be a (B, 4, rows, L) view with contiguous rows")
+    x, weight = x.contiguous(), weight.contiguous()
+    with torch.cuda.device(x.device):
+        rc = _lib.lib().ss2d_x_proj(x.data_ptr(), weight.data_ptr(), out.data_ptr(), B, D, C, H, W, Hp, Wp, mask_row, out.stride(1),
+                                    out.stride(2), out.stride(0), _DTYPE_CODE[x.dtype], torch.cuda.current_stream(x.device).cuda_stream)
+    _lib.check(rc, "ss2d_x_proj")
+    return out
+
+
 DT_PROJ_MAX_RANK = 48
 
 

@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from ._lib import SS2D_ENOTSUP, Ss2dError
 from .core import (DT_PROJ_MAX_RANK, core_fits, core_mask_pads_hip, dt_proj_hip, embed_maps_hip, padded_map_size,
-                   ss2d_core_hip)
+                   ss2d_core_hip, x_proj_fits, x_proj_hip)
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
 from .conv import dwconv3x3_silu_hip
@@ -214,8 +214,11 @@ class SS2D(nn.Module):
         direction's rows in that direction's order.  x_proj then reads the map once instead of its four copies."""
         B, D, H, W = x.shape
         K, L, R, N = self.k_group, H * W, self.dt_rank, self.d_state
-        proj = torch.bmm(consts["Wx_all"], x.reshape(B, D, L)).view(B, K, R + 2 * N, H, W)
-        x_dbl = cross_scan_fn(proj, in_channel_first=True, out_channel_first=True, one_by_one=True, scans=0)   # (B, K, R+2N, L)
+        if x_proj_fits(x, self.x_proj_weight) and not needs_grad(x, self.x_proj_weight):
+            x_dbl = x_proj_hip(x, self.x_proj_weight, x.new_empty((B, K, R + 2 * N, L)))
+        else:
+            proj = torch.bmm(consts["Wx_all"], x.reshape(B, D, L)).view(B, K, R + 2 * N, H, W)
+            x_dbl = cross_scan_fn(proj, in_channel_first=True, out_channel_first=True, one_by_one=True, scans=0)   # (B, K, R+2N, L)
         dts, Bs, Cs = torch.split(x_dbl, [R, N, N], dim=2)
         dts = dts.reshape(B * K, R, L)
         if dts.dtype != torch.float32 and R <= DT_PROJ_MAX_RANK and not needs_grad(dts, self.dt_projs_weight):
@@ -245,24 +248,28 @@ class SS2D(nn.Module):
             x = embed_maps_hip(x.contiguous().view(B * D, H0, W0), padded[0], padded[1]).view(B, D, padded[0], padded[1])
         H, W = x.shape[2], x.shape[3]
         L = H * W
-        proj = torch.bmm(consts["Wx_all"], x.view(B, D, L))                                   # (B, K*C, L)
         # Rows of B*L positions start on 16-byte boundaries only if B*L is a multiple of the 16-byte vector: maps with
         # an odd (or 2, 4 mod 8) number of positions get room for a few images more, which nothing reads back --
         # dt_proj and the kernel's delta stream then keep their 16-byte accesses.
-        vec = 16 // proj.element_size()
+        vec = 16 // x.element_size()
         unit = vec // math.gcd(L, vec)
         Bp = (B + unit - 1) // unit * unit
         # On a padded map the step of the added positions must be 0: the 16-bit dt_proj on the matrix cores writes -1e30
         # (-65504 in fp16) there instead of the projection (a mask of those positions in each direction's order), and the
         # softplus of that is exactly 0.  Otherwise ss2d_core_mask_pads writes -inf into delta afterwards, a scattered
         # pass over its rows.
-        x_dbl = proj.new_empty((K, C, B, L)) if Bp == B else proj.new_zeros((K, C, Bp, L))
-        cross_scan_1b1_hip(proj.view(B, K, C, H, W), out=x_dbl[:, :, :B].permute(2, 0, 1, 3))
+        x_dbl = x.new_empty((K, C, B, L)) if Bp == B else x.new_zeros((K, C, Bp, L))
+        x_dbl_rows = x_dbl[:, :, :B].permute(2, 0, 1, 3)
+        if x_proj_fits(x, self.x_proj_weight):
+            x_proj_hip(x, self.x_proj_weight, x_dbl_rows)
+        else:
+            proj = torch.bmm(consts["Wx_all"], x.view(B, D, L))                               # (B, K*C, L)
+            cross_scan_1b1_hip(proj.view(B, K, C, H, W), out=x_dbl_rows)
         dts = x_dbl[:, :R].reshape(K, R, Bp * L)
         if dts.dtype != torch.float32 and R <= DT_PROJ_MAX_RANK:
             if padded is not None:
-                big = -65504.0 if proj.dtype == torch.float16 else -1e30
-                delta = dt_proj_hip(dts, self.dt_projs_weight, _pad_mask(H0, W0, H, W, Bp, proj.device), big).view(K, D, Bp, L)
+                big = -65504.0 if x.dtype == torch.float16 else -1e30
+                delta = dt_proj_hip(dts, self.dt_projs_weight, _pad_mask(H0, W0, H, W, Bp, x.device), big).view(K, D, Bp, L)
             else:
                 delta = dt_proj_hip(dts, self.dt_projs_weight).view(K, D, Bp, L)
         else:
