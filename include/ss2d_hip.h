@@ -250,6 +250,13 @@ int ss2d_x_proj(const void *x, const void *weight, void *out, int B, int D, int 
                 int64_t out_dir_stride, int64_t out_chan_stride, int64_t out_batch_stride, int dtype, void *stream);
 
 /*
+ * The same projection in single precision (fp32 operands and sums), any D > 0 and C; the map as it is
+ * (no padding, no mask row).
+ */
+int ss2d_x_proj_f32(const float *x, const float *weight, float *out, int B, int D, int C, int H, int W, int64_t out_dir_stride,
+                    int64_t out_chan_stride, int64_t out_batch_stride, void *stream);
+
+/*
  * Fused SS2D core for dstate = 1: CrossScan -> selective scan (softplus, fp32 state, fp32 "oflex" output) ->
  * CrossMerge in one kernel.  Replaces the three calls of SS2Dv2.forward_corev2
  * (classification/models/vmamba.py:604, 625-633, 638: cross_scan_fn, selective_scan, cross_merge_fn) for
@@ -400,6 +407,10 @@ int ss2d_stem_conv_ln_gelu(const void *x, const void *weight, const int64_t *wei
  */
 int ss2d_dt_proj(const void *x, const void *weight, void *delta, int K, int D, int R, int64_t N, int64_t x_dir_stride,
                  int64_t x_rank_stride, int dtype, void *stream);
+
+/* The same projection in single precision (fp32 operands and sums); R > 24 returns SS2D_ENOTSUP. */
+int ss2d_dt_proj_f32(const float *x, const float *weight, float *delta, int K, int D, int R, int64_t N, int64_t x_dir_stride,
+                     int64_t x_rank_stride, void *stream);
 
 /*
  * The same projection with chosen positions overwritten: mask is (K, N) 16-bit words, each 0 or 0xffff, and where a word

@@ -211,3 +211,48 @@ def dt_proj_hip(x, weight, mask=None, fill=0.0):
                                             torch.cuda.current_stream(x.device).cuda_stream)
     _lib.check(rc, "ss2d_dt_proj")
     return out
+
+
+def x_proj_f32_fits(x, weight):
+    """True when ss2d_x_proj_f32 takes this map (B, D, H, W) and these weights (4, C, D)."""
+    return (x.is_cuda and x.dtype == weight.dtype == torch.float32 and weight.device == x.device and x.numel() > 0
+            and x.numel() // x.shape[1] < 2 ** 31)
+
+
+def x_proj_f32_hip(x, weight, out):
+    """x_proj_hip in single precision: weight (4, C, D) applied to the map x (B, D, H, W), each direction's rows in its scan
+    order, into ``out``: a (B, 4, C, L) view with contiguous rows (ss2d_x_proj_f32)."""
+    _check(x.is_cuda and x.dim() == 4 and weight.dim() == 3 and weight.shape[0] == 4 and weight.shape[2] == x.shape[1],
+           "x_proj_f32 expects x (B, D, H, W) and weight (4, C, D)")
+    _check(x.dtype == weight.dtype == out.dtype == torch.float32 and weight.device == out.device == x.device,
+           "x_proj_f32: float32 tensors on one device")
+    B, D, H, W = x.shape
+    C = weight.shape[1]
+    _check(tuple(out.shape) == (B, 4, C, H * W) and (out.stride(3) == 1 or out.shape[3] == 1),
+           "x_proj_f32: out must be a (B, 4, rows, L) view with contiguous rows")
+    x, weight = x.contiguous(), weight.contiguous()
+    with torch.cuda.device(x.device):
+        rc = _lib.lib().ss2d_x_proj_f32(x.data_ptr(), weight.data_ptr(), out.data_ptr(), B, D, C, H, W, out.stride(1), out.stride(2),
+                                        out.stride(0), torch.cuda.current_stream(x.device).cuda_stream)
+    _lib.check(rc, "ss2d_x_proj_f32")
+    return out
+
+
+DT_PROJ_F32_MAX_RANK = 24
+
+
+def dt_proj_f32_hip(x, weight):
+    """dt_proj_hip in single precision: x (K, R, N) with contiguous rows, weight (K, D, R) -> (K, D, N) (ss2d_dt_proj_f32)."""
+    _check(x.is_cuda and x.dim() == 3 and weight.dim() == 3 and x.shape[0] == weight.shape[0] and x.shape[1] == weight.shape[2],
+           "dt_proj_f32 expects x (K, R, N) and weight (K, D, R)")
+    _check(x.dtype == weight.dtype == torch.float32 and x.device == weight.device, "dt_proj_f32: float32 tensors on one device")
+    _check(x.stride(2) == 1 or x.size(2) == 1, "x must be contiguous in its last dimension")
+    K, R, N = x.shape
+    D = weight.shape[1]
+    weight = weight.contiguous()
+    out = torch.empty((K, D, N), device=x.device, dtype=x.dtype)
+    with torch.cuda.device(x.device):
+        rc = _lib.lib().ss2d_dt_proj_f32(x.data_ptr(), weight.data_ptr(), out.data_ptr(), K, D, R, N, x.stride(0), x.stride(1),
+                                         torch.cuda.current_stream(x.device).cuda_stream)
+    _lib.check(rc, "ss2d_dt_proj_f32")
+    return out

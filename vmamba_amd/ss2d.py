@@ -21,8 +21,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ._lib import SS2D_ENOTSUP, Ss2dError
-from .core import (DT_PROJ_MAX_RANK, core_fits, core_mask_pads_hip, dt_proj_hip, embed_maps_hip, padded_map_size,
-                   ss2d_core_hip, x_proj_fits, x_proj_hip)
+from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_fits, core_mask_pads_hip, dt_proj_f32_hip, dt_proj_hip,
+                   embed_maps_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_fits, x_proj_hip)
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
 from .conv import dwconv3x3_silu_hip
@@ -216,6 +216,8 @@ class SS2D(nn.Module):
         K, L, R, N = self.k_group, H * W, self.dt_rank, self.d_state
         if x_proj_fits(x, self.x_proj_weight) and not needs_grad(x, self.x_proj_weight):
             x_dbl = x_proj_hip(x, self.x_proj_weight, x.new_empty((B, K, R + 2 * N, L)))
+        elif x_proj_f32_fits(x, self.x_proj_weight) and not needs_grad(x, self.x_proj_weight):
+            x_dbl = x_proj_f32_hip(x, self.x_proj_weight, x.new_empty((B, K, R + 2 * N, L)))
         else:
             proj = torch.bmm(consts["Wx_all"], x.reshape(B, D, L)).view(B, K, R + 2 * N, H, W)
             x_dbl = cross_scan_fn(proj, in_channel_first=True, out_channel_first=True, one_by_one=True, scans=0)   # (B, K, R+2N, L)
@@ -223,6 +225,8 @@ class SS2D(nn.Module):
         dts = dts.reshape(B * K, R, L)
         if dts.dtype != torch.float32 and R <= DT_PROJ_MAX_RANK and not needs_grad(dts, self.dt_projs_weight):
             dts = dt_proj_hip(dts, consts["Wdt"])                     # one (image, direction) problem per weight copy
+        elif dts.dtype == torch.float32 and dts.is_cuda and R <= DT_PROJ_F32_MAX_RANK and not needs_grad(dts, self.dt_projs_weight):
+            dts = dt_proj_f32_hip(dts, consts["Wdt"])
         else:
             dts = torch.bmm(consts["Wdt"], dts)
         return dts.view(B, K * D, L), Bs, Cs
@@ -262,6 +266,8 @@ class SS2D(nn.Module):
         x_dbl_rows = x_dbl[:, :, :B].permute(2, 0, 1, 3)
         if x_proj_fits(x, self.x_proj_weight):
             x_proj_hip(x, self.x_proj_weight, x_dbl_rows)
+        elif x_proj_f32_fits(x, self.x_proj_weight):
+            x_proj_f32_hip(x, self.x_proj_weight, x_dbl_rows)
         else:
             proj = torch.bmm(consts["Wx_all"], x.view(B, D, L))                               # (B, K*C, L)
             cross_scan_1b1_hip(proj.view(B, K, C, H, W), out=x_dbl_rows)
@@ -272,6 +278,8 @@ class SS2D(nn.Module):
                 delta = dt_proj_hip(dts, self.dt_projs_weight, _pad_mask(H0, W0, H, W, Bp, x.device), big).view(K, D, Bp, L)
             else:
                 delta = dt_proj_hip(dts, self.dt_projs_weight).view(K, D, Bp, L)
+        elif dts.dtype == torch.float32 and R <= DT_PROJ_F32_MAX_RANK:
+            delta = dt_proj_f32_hip(dts, self.dt_projs_weight).view(K, D, Bp, L)
         else:
             delta = torch.bmm(self.dt_projs_weight, dts).view(K, D, Bp, L)
             if padded is not None:
