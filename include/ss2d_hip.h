@@ -223,6 +223,25 @@ int ss2d_dwconv3x3_silu(const void *x, const void *weight, const void *bias, voi
                         int dtype, int in_channel_last, int apply_silu, void *stream);
 
 /*
+ * The same on channel-first fp32 maps with the nine products summed in 64 bits: the forward of training.  SS2D_ENOTSUP for
+ * rows so long that two of them, with halo, do not fit 64 KB (more than about 1600 columns).
+ */
+int ss2d_dwconv3x3_silu_f32(const float *x, const float *weight, const float *bias, float *y, int B, int D, int H, int W,
+                            void *stream);
+
+/*
+ * Backward of ss2d_dwconv3x3_silu with apply_silu (in training the reference differentiates the two operators,
+ * classification/models/vmamba.py:656-658): x, dy, dx (B,D,H,W), weight and dweight (D,1,3,3), bias and dbias (D) or NULL, all
+ * of `dtype`, contiguous; sums in fp32 (those of nine products in 64 bits for fp32), rounded once, in a fixed order.  The convolution is
+ * recomputed from x and not rounded before the SiLU.  workspace: ss2d_dwconv3x3_silu_bwd_workspace_bytes(...) bytes of device memory, 4-byte aligned.
+ * SS2D_ENOTSUP (from both): rows so long that two of them, with halo, do not fit 64 KB (more than about 1600 columns).
+ */
+int64_t ss2d_dwconv3x3_silu_bwd_workspace_bytes(int B, int D, int H, int W);
+int ss2d_dwconv3x3_silu_bwd(const void *x, const void *weight, const void *bias, const void *dy, void *dx, void *dweight,
+                            void *dbias, int B, int D, int H, int W, int dtype, void *workspace, int64_t workspace_bytes,
+                            void *stream);
+
+/*
  * CrossScan, one-by-one, scans=0, channel-first: every direction slice of the input is put in ITS scan order.
  * Replaces CrossScanTriton1b1.forward / cross_scan1b1_fwd (classification/models/csm_triton.py:88-131, 400-436).
  *   x (B,4,C,H,W) contiguous -> y[b*y_batch_stride + k*y_dir_stride + c*y_chan_stride + j], j in [0, L):

@@ -25,7 +25,7 @@ from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_fits, core_mask_
                    embed_maps_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_fits, x_proj_hip)
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
-from .conv import dwconv3x3_silu_hip
+from .conv import DwConv3x3SiLU, dwconv3x3_silu_hip, dwconv_silu_trainable
 from .linear import linear_cf_ln_fusable, linear_cf_ln_hip, linear_cl_hip, linear_fusable
 from .norm import (LayerNorm, LayerNorm2d, add_layer_norm_fusable, add_layer_norm_hip, layer_norm_cf_hip,
                    needs_grad)
@@ -66,6 +66,8 @@ class HipLayers:
         fusable = conv2d is not None and conv2d.kernel_size == (3, 3) and conv2d.padding == (1, 1) and conv2d.stride == (1, 1)
         if fusable and not needs_grad(x, conv2d.weight, conv2d.bias):
             return dwconv3x3_silu_hip(x, conv2d.weight, conv2d.bias, in_channel_last=not channel_first, apply_silu=True)
+        if fusable and dwconv_silu_trainable(conv2d, x, not channel_first):
+            return DwConv3x3SiLU.apply(x, conv2d.weight, conv2d.bias, not channel_first)
         if not channel_first:
             x = x.permute(0, 3, 1, 2).contiguous()
         return F.silu(conv2d(x) if conv2d is not None else x)
