@@ -322,6 +322,27 @@ int64_t ss2d_core_workspace_bytes(const ss2d_core_params *params);
 int ss2d_core_fwd_ws(const ss2d_core_params *params, void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
+ * SS2Dv2.forward_corev2 of a one-state block (classification/models/vmamba.py:603-646) in one call: ss2d_x_proj, ss2d_dt_proj,
+ * ss2d_core_fwd_ws and -- with `normalise` -- ss2d_layer_norm_cf as out_norm, enqueued on `stream` (fp32: the _f32 projections).
+ *   x (B,D,H,W); x_proj_weight (4, rank + 2, D); dt_proj_weight (4, D, rank), all of `dtype`; A, D, delta_bias (4*D) fp32
+ *   out   normalise: (B,D,L), or (B,L,D) if out_channel_last, of `dtype`; else the merged map (B,D,L) fp32
+ *   norm_weight, norm_bias (D) of norm_dtype or NULL
+ * Everything contiguous.  workspace: ss2d_forward_core_workspace_bytes(params) bytes, 16-byte aligned, contents irrelevant;
+ * workspace_bytes depends on the sizes and types, and on the pointers' alignment.  Either function returns SS2D_ENOTSUP where
+ * one of the kernels has no variant for the problem.
+ */
+typedef struct ss2d_forward_core_params {
+    int32_t batch, dim, height, width, rank;
+    int32_t dtype, norm_dtype, normalise, out_channel_last;
+    float eps;
+    const void *x, *x_proj_weight, *dt_proj_weight, *A, *D, *delta_bias, *norm_weight, *norm_bias;
+    void *out;
+} ss2d_forward_core_params;
+
+int64_t ss2d_forward_core_workspace_bytes(const ss2d_forward_core_params *params);
+int ss2d_forward_core(const ss2d_forward_core_params *params, void *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * Maps whose sides do not suit the core's vector paths (57 x 58 -- the reference's own check size,
  * classification/models/csm_triton.py:524, 670 -- 75 x 75, 19 x 19 ...) can be embedded by the caller in a map of
  * padded_height x padded_width >= height x width: x = 0 on the added rows / columns, the projections computed on the

@@ -5,6 +5,8 @@ There is no CPU fallback: if the library has not been built, loading fails loudl
 import ctypes
 import os
 
+import torch
+
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "libss2d_hip.so")
 
@@ -22,7 +24,7 @@ EXPORTS = ("ss2d_abi_version", "ss2d_strerror", "ss2d_cross_scan", "ss2d_cross_m
            "ss2d_selective_scan_kernel", "ss2d_selective_scan_fwd_maps",
            "ss2d_layer_norm", "ss2d_add_layer_norm", "ss2d_bias_layer_norm", "ss2d_layer_norm_cf", "ss2d_dwconv3x3_silu",
            "ss2d_dwconv3x3_silu_f32", "ss2d_dwconv3x3_silu_bwd", "ss2d_dwconv3x3_silu_bwd_workspace_bytes", "ss2d_cross_scan_1b1", "ss2d_core_fwd",
-           "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
+           "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_forward_core", "ss2d_forward_core_workspace_bytes", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
            "ss2d_x_proj", "ss2d_x_proj_f32", "ss2d_dt_proj", "ss2d_dt_proj_f32", "ss2d_dt_proj_masked", "ss2d_cross_scan_flex", "ss2d_cross_scan_flex_ws", "ss2d_cross_scan_flex_static", "ss2d_cross_merge_flex",
            "ss2d_selective_scan_bwd", "ss2d_transpose_bcl", "ss2d_mlp_fused", "ss2d_linear_cl", "ss2d_linear_cf_ln", "ss2d_stem_conv_ln_gelu", "ss2d_mean_pool_cl")
 
@@ -63,6 +65,17 @@ class CoreParams(ctypes.Structure):
         + [(n, ctypes.c_void_p) for n in ("x", "delta", "A", "B", "C", "D", "delta_bias", "y")]
         + [(n, ctypes.c_int64) for n in ("delta_dir_stride", "delta_dim_stride", "delta_batch_stride",
                                          "B_dir_stride", "B_batch_stride", "C_dir_stride", "C_batch_stride")]
+    )
+
+
+class ForwardCoreParams(ctypes.Structure):
+    """struct ss2d_forward_core_params (include/ss2d_hip.h)."""
+    _fields_ = (
+        [(n, ctypes.c_int32) for n in ("batch", "dim", "height", "width", "rank", "dtype", "norm_dtype", "normalise",
+                                       "out_channel_last")]
+        + [("eps", ctypes.c_float)]
+        + [(n, ctypes.c_void_p) for n in ("x", "x_proj_weight", "dt_proj_weight", "A", "D", "delta_bias", "norm_weight",
+                                          "norm_bias", "out")]
     )
 
 
@@ -129,6 +142,10 @@ def lib():
         L.ss2d_core_workspace_bytes.argtypes = [ctypes.POINTER(CoreParams)]
         L.ss2d_core_fwd_ws.restype = ctypes.c_int
         L.ss2d_core_fwd_ws.argtypes = [ctypes.POINTER(CoreParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+        L.ss2d_forward_core_workspace_bytes.restype = ctypes.c_int64
+        L.ss2d_forward_core_workspace_bytes.argtypes = [ctypes.POINTER(ForwardCoreParams)]
+        L.ss2d_forward_core.restype = ctypes.c_int
+        L.ss2d_forward_core.argtypes = [ctypes.POINTER(ForwardCoreParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
         L.ss2d_core_embed_maps.restype = ctypes.c_int
         L.ss2d_core_embed_maps.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int,
                                            ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]
@@ -174,6 +191,17 @@ def lib():
             raise ImportError(f"{LIB_PATH}: ABI version {L.ss2d_abi_version()} != expected {ABI_VERSION}; rebuild")
         _lib = L
     return _lib
+
+
+def launch(tensor, fn, *args):
+    """fn(*args, stream): a launch on ``tensor``'s device and torch's current stream there.  The device is switched only where
+    it is not current already, and the stream is asked for as the bare handle: the context manager and Stream object of the
+    usual spelling cost more than the launch."""
+    index = tensor.get_device()
+    if index == torch.cuda.current_device():
+        return fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    with torch.cuda.device(index):
+        return fn(*args, torch._C._cuda_getCurrentRawStream(index))
 
 
 def strerror(code):

@@ -30,10 +30,9 @@ def dwconv3x3_silu_hip(x, weight, bias=None, in_channel_last=False, apply_silu=T
     weight = weight.to(x.dtype).contiguous()
     bias = bias.to(x.dtype).contiguous() if bias is not None else None
     y = torch.empty((B, D, H, W), device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_dwconv3x3_silu(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
-                                            y.data_ptr(), B, D, H, W, _DTYPE_CODE[x.dtype], int(bool(in_channel_last)),
-                                            int(bool(apply_silu)), torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_dwconv3x3_silu, x.data_ptr(), weight.data_ptr(),
+                     bias.data_ptr() if bias is not None else None, y.data_ptr(), B, D, H, W, _DTYPE_CODE[x.dtype],
+                     int(bool(in_channel_last)), int(bool(apply_silu)))
     _lib.check(rc, "ss2d_dwconv3x3_silu")
     return y
 
@@ -56,11 +55,10 @@ def dwconv3x3_silu_bwd_hip(x, weight, bias, dy):
     need = _lib.lib().ss2d_dwconv3x3_silu_bwd_workspace_bytes(B, D, H, W)
     _lib.check(min(need, 0), "ss2d_dwconv3x3_silu_bwd_workspace_bytes")
     workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_dwconv3x3_silu_bwd(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
-                                                dy.data_ptr(), dx.data_ptr(), dweight.data_ptr(),
-                                                dbias.data_ptr() if dbias is not None else None, B, D, H, W, _DTYPE_CODE[x.dtype],
-                                                workspace.data_ptr(), need, torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_dwconv3x3_silu_bwd, x.data_ptr(), weight.data_ptr(),
+                     bias.data_ptr() if bias is not None else None, dy.data_ptr(), dx.data_ptr(), dweight.data_ptr(),
+                     dbias.data_ptr() if dbias is not None else None, B, D, H, W, _DTYPE_CODE[x.dtype], workspace.data_ptr(),
+                     need)
     _lib.check(rc, "ss2d_dwconv3x3_silu_bwd")
     return dx, dweight, dbias
 
@@ -81,9 +79,8 @@ class DwConv3x3SiLU(torch.autograd.Function):
             return dwconv3x3_silu_hip(x, weight, bias, in_channel_last=False, apply_silu=True)
         weight, bias = weight.contiguous(), bias.contiguous() if bias is not None else None
         y = torch.empty_like(x)
-        with torch.cuda.device(x.device):
-            rc = _lib.lib().ss2d_dwconv3x3_silu_f32(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
-                                                    y.data_ptr(), *x.shape, torch.cuda.current_stream(x.device).cuda_stream)
+        rc = _lib.launch(x, _lib.lib().ss2d_dwconv3x3_silu_f32, x.data_ptr(), weight.data_ptr(),
+                         bias.data_ptr() if bias is not None else None, y.data_ptr(), *x.shape)
         _lib.check(rc, "ss2d_dwconv3x3_silu_f32")
         return y
 

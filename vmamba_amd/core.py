@@ -70,10 +70,8 @@ def core_mask_pads_hip(delta, H, W, Hp, Wp):
     columns >= W, in every direction's order (ss2d_core_mask_pads).  In place."""
     _check(delta.is_cuda and delta.dim() == 4 and delta.shape[0] == 4 and delta.shape[3] == Hp * Wp, "delta must be (4, D, B, Hp*Wp) on the GPU")
     _check(delta.dtype in _DTYPE_CODE and (delta.stride(3) == 1 or delta.shape[3] == 1), "delta must be contiguous along the map")
-    with torch.cuda.device(delta.device):
-        rc = _lib.lib().ss2d_core_mask_pads(delta.data_ptr(), delta.shape[2], delta.shape[1], H, W, Hp, Wp, delta.stride(0),
-                                            delta.stride(1), delta.stride(2), _DTYPE_CODE[delta.dtype],
-                                            torch.cuda.current_stream(delta.device).cuda_stream)
+    rc = _lib.launch(delta, _lib.lib().ss2d_core_mask_pads, delta.data_ptr(), delta.shape[2], delta.shape[1], H, W, Hp, Wp,
+                     delta.stride(0), delta.stride(1), delta.stride(2), _DTYPE_CODE[delta.dtype])
     _lib.check(rc, "ss2d_core_mask_pads")
     return delta
 
@@ -89,9 +87,8 @@ def embed_maps_hip(src, dst_rows, dst_cols):
         return dst
     if src.numel() == 0:
         return dst.zero_()
-    with torch.cuda.device(src.device):
-        rc = _lib.lib().ss2d_core_embed_maps(src.data_ptr(), dst.data_ptr(), n, rows, cols, dst_rows, dst_cols, src.element_size(),
-                                             torch.cuda.current_stream(src.device).cuda_stream)
+    rc = _lib.launch(src, _lib.lib().ss2d_core_embed_maps, src.data_ptr(), dst.data_ptr(), n, rows, cols, dst_rows, dst_cols,
+                     src.element_size())
     _lib.check(rc, "ss2d_core_embed_maps")
     return dst
 
@@ -142,18 +139,66 @@ def ss2d_core_hip(x, delta, Bs, Cs, As, Ds=None, delta_bias=None, delta_softplus
     p.delta_dir_stride, p.delta_dim_stride, p.delta_batch_stride = delta.stride(0), delta.stride(1), delta.stride(2)
     p.B_dir_stride, p.B_batch_stride = Bs.stride(0), Bs.stride(1)
     p.C_dir_stride, p.C_batch_stride = Cs.stride(0), Cs.stride(1)
-    with torch.cuda.device(x.device):
-        # maps too large for the single kernel are walked in tiles, twice, through scratch memory of the size the library asks for
-        need = _lib.lib().ss2d_core_workspace_bytes(p)
-        _lib.check(min(need, 0), "ss2d_core_workspace_bytes")
-        stream = torch.cuda.current_stream(x.device).cuda_stream
-        if need > 0:
-            workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
-            rc = _lib.lib().ss2d_core_fwd_ws(p, workspace.data_ptr(), need, stream)
-        else:
-            rc = _lib.lib().ss2d_core_fwd(p, stream)
+    # maps too large for the single kernel are walked in tiles, twice, through scratch memory of the size the library asks for
+    need = _lib.lib().ss2d_core_workspace_bytes(p)
+    _lib.check(min(need, 0), "ss2d_core_workspace_bytes")
+    if need > 0:
+        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+        rc = _lib.launch(x, _lib.lib().ss2d_core_fwd_ws, p, workspace.data_ptr(), need)
+    else:
+        rc = _lib.launch(x, _lib.lib().ss2d_core_fwd, p)
     _lib.check(rc, "ss2d_core_fwd")
     return y
+
+
+def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=None, out_channel_last=False):
+    """x_proj, dt_proj, the fused core and -- with ``norm`` -- out_norm in one call (ss2d_forward_core): x (B,D,H,W),
+    x_proj_weight (4,R+2,D), dt_proj_weight (4,D,R) of one dtype; As, Ds, dt_bias (4*D) fp32; norm a LayerNorm over D.  Returns
+    (B,H,W,D) if ``out_channel_last`` else (B,D,H,W) in x.dtype, the merged map (B,D,L) in fp32 without ``norm``, or None
+    where the kernels have no variant for the call and the separate ones have to be tried."""
+    B, D, H, W = x.shape
+    R = dt_proj_weight.shape[2]
+    code = _DTYPE_CODE.get(x.dtype)
+    if (code is None or x.numel() == 0 or R == 0 or tuple(x_proj_weight.shape) != (4, R + 2, D) or tuple(dt_proj_weight.shape) != (4, D, R)
+            or not As.numel() == Ds.numel() == dt_bias.numel() == 4 * D or padded_map_size(H, W, x.dtype) is not None):
+        return None
+    index = x.get_device()
+    for t in (x_proj_weight, dt_proj_weight):
+        if t.dtype != x.dtype or t.get_device() != index or not t.is_contiguous():
+            return None
+    for t in (As, Ds, dt_bias):
+        if t.dtype != torch.float32 or t.get_device() != index or not t.is_contiguous():
+            return None
+    x = x.contiguous()
+    p = _lib.ForwardCoreParams(B, D, H, W, R, code)
+    if norm is not None:
+        weight, bias = norm.weight, norm.bias
+        for t in (weight, bias):
+            if t is not None and (t.get_device() != index or not t.is_contiguous() or t.numel() != D or t.dtype not in _DTYPE_CODE):
+                return None
+        if weight is not None and bias is not None and weight.dtype != bias.dtype:
+            return None
+        p.normalise, p.out_channel_last, p.eps = 1, int(out_channel_last), norm.eps
+        if weight is not None:
+            p.norm_weight, p.norm_dtype = weight.data_ptr(), _DTYPE_CODE[weight.dtype]
+        if bias is not None:
+            p.norm_bias, p.norm_dtype = bias.data_ptr(), _DTYPE_CODE[bias.dtype]
+        out = x.new_empty((B, H, W, D) if out_channel_last else (B, D, H, W))
+    else:
+        out = torch.empty((B, D, H * W), device=x.device, dtype=torch.float32)
+    p.x, p.x_proj_weight, p.dt_proj_weight = x.data_ptr(), x_proj_weight.data_ptr(), dt_proj_weight.data_ptr()
+    p.A, p.D, p.delta_bias, p.out = As.data_ptr(), Ds.data_ptr(), dt_bias.data_ptr(), out.data_ptr()
+    L = _lib.lib()
+    need = L.ss2d_forward_core_workspace_bytes(p)
+    if need == _lib.SS2D_ENOTSUP:
+        return None
+    _lib.check(min(need, 0), "ss2d_forward_core_workspace_bytes")
+    workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+    rc = _lib.launch(x, L.ss2d_forward_core, p, workspace.data_ptr(), need)
+    if rc == _lib.SS2D_ENOTSUP:
+        return None
+    _lib.check(rc, "ss2d_forward_core")
+    return out
 
 
 X_PROJ_MAX_ROWS = 96
@@ -179,9 +224,8 @@ def x_proj_hip(x, weight, out, padded=None, mask_row=-1):
     _check(tuple(out.shape) == (B, 4, C + (mask_row >= 0), Hp * Wp) and (out.stride(3) == 1 or out.shape[3] == 1),
            "x_proj: out must be a (B, 4, rows, L) view with contiguous rows")
     x, weight = x.contiguous(), weight.contiguous()
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_x_proj(x.data_ptr(), weight.data_ptr(), out.data_ptr(), B, D, C, H, W, Hp, Wp, mask_row, out.stride(1),
-                                    out.stride(2), out.stride(0), _DTYPE_CODE[x.dtype], torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_x_proj, x.data_ptr(), weight.data_ptr(), out.data_ptr(), B, D, C, H, W, Hp, Wp,
+                     mask_row, out.stride(1), out.stride(2), out.stride(0), _DTYPE_CODE[x.dtype])
     _lib.check(rc, "ss2d_x_proj")
     return out
 
@@ -205,10 +249,9 @@ def dt_proj_hip(x, weight, mask=None, fill=0.0):
                and mask.is_contiguous(), "dt_proj: mask must be a contiguous (K, N) int16 tensor on x's device")
     weight = weight.contiguous()
     out = torch.empty((K, D, N), device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_dt_proj_masked(x.data_ptr(), weight.data_ptr(), None if mask is None else mask.data_ptr(), float(fill),
-                                            out.data_ptr(), K, D, R, N, x.stride(0), x.stride(1), _DTYPE_CODE[x.dtype],
-                                            torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_dt_proj_masked, x.data_ptr(), weight.data_ptr(),
+                     None if mask is None else mask.data_ptr(), float(fill), out.data_ptr(), K, D, R, N, x.stride(0),
+                     x.stride(1), _DTYPE_CODE[x.dtype])
     _lib.check(rc, "ss2d_dt_proj")
     return out
 
@@ -231,9 +274,8 @@ def x_proj_f32_hip(x, weight, out):
     _check(tuple(out.shape) == (B, 4, C, H * W) and (out.stride(3) == 1 or out.shape[3] == 1),
            "x_proj_f32: out must be a (B, 4, rows, L) view with contiguous rows")
     x, weight = x.contiguous(), weight.contiguous()
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_x_proj_f32(x.data_ptr(), weight.data_ptr(), out.data_ptr(), B, D, C, H, W, out.stride(1), out.stride(2),
-                                        out.stride(0), torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_x_proj_f32, x.data_ptr(), weight.data_ptr(), out.data_ptr(), B, D, C, H, W,
+                     out.stride(1), out.stride(2), out.stride(0))
     _lib.check(rc, "ss2d_x_proj_f32")
     return out
 
@@ -251,8 +293,7 @@ def dt_proj_f32_hip(x, weight):
     D = weight.shape[1]
     weight = weight.contiguous()
     out = torch.empty((K, D, N), device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_dt_proj_f32(x.data_ptr(), weight.data_ptr(), out.data_ptr(), K, D, R, N, x.stride(0), x.stride(1),
-                                         torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_dt_proj_f32, x.data_ptr(), weight.data_ptr(), out.data_ptr(), K, D, R, N, x.stride(0),
+                     x.stride(1))
     _lib.check(rc, "ss2d_dt_proj_f32")
     return out

@@ -49,8 +49,7 @@ def transpose_bcl_hip(x):
     x = x.contiguous()
     B, R, S = x.shape
     y = x.new_empty((B, S, R))
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_transpose_bcl(x.data_ptr(), y.data_ptr(), B, R, S, x.element_size(), _stream(x))
+    rc = _lib.launch(x, _lib.lib().ss2d_transpose_bcl, x.data_ptr(), y.data_ptr(), B, R, S, x.element_size())
     _lib.check(rc, "ss2d_transpose_bcl")
     return y
 
@@ -65,18 +64,14 @@ def cross_scan_flex_hip(x, in_channel_first=True, out_channel_first=True, one_by
     if in_channel_first != out_channel_first and x.numel():
         y = x.new_empty((B, 4, C, H * W) if out_channel_first else (B, H * W, 4, C))
         staging = torch.empty_like(x)          # one copy of x in the layout of y
-        with torch.cuda.device(x.device):
-            rc = _lib.lib().ss2d_cross_scan_flex_ws(x.data_ptr(), y.data_ptr(), B, C, H, W, x.element_size(),
-                                                    0 if in_channel_first else 1, 0 if out_channel_first else 1,
-                                                    1 if one_by_one else 0, scans, staging.data_ptr(),
-                                                    staging.numel() * staging.element_size(), _stream(x))
+        rc = _lib.launch(x, _lib.lib().ss2d_cross_scan_flex_ws, x.data_ptr(), y.data_ptr(), B, C, H, W, x.element_size(),
+                         0 if in_channel_first else 1, 0 if out_channel_first else 1, 1 if one_by_one else 0, scans,
+                         staging.data_ptr(), staging.numel() * staging.element_size())
         _lib.check(rc, "ss2d_cross_scan_flex_ws")
         return y
     y = x.new_empty((B, 4, C, H * W) if out_channel_first else (B, H * W, 4, C))
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_cross_scan_flex(x.data_ptr(), y.data_ptr(), B, C, H, W, x.element_size(),
-                                             0 if in_channel_first else 1, 0 if out_channel_first else 1,
-                                             1 if one_by_one else 0, scans, _stream(x))
+    rc = _lib.launch(x, _lib.lib().ss2d_cross_scan_flex, x.data_ptr(), y.data_ptr(), B, C, H, W, x.element_size(),
+                     0 if in_channel_first else 1, 0 if out_channel_first else 1, 1 if one_by_one else 0, scans)
     _lib.check(rc, "ss2d_cross_scan_flex")
     return y
 
@@ -104,10 +99,8 @@ def cross_merge_flex_hip(y, in_channel_first=True, out_channel_first=True, one_b
         x = y.new_empty((B, 4, C, L) if in_channel_first else (B, L, 4, C))
     else:
         x = y.new_empty((B, C, L) if in_channel_first else (B, L, C))
-    with torch.cuda.device(y.device):
-        rc = _lib.lib().ss2d_cross_merge_flex(y.data_ptr(), x.data_ptr(), B, C, H, W, _DTYPE_CODE[y.dtype],
-                                              0 if in_channel_first else 1, 0 if out_channel_first else 1,
-                                              1 if one_by_one else 0, scans, order, _stream(y))
+    rc = _lib.launch(y, _lib.lib().ss2d_cross_merge_flex, y.data_ptr(), x.data_ptr(), B, C, H, W, _DTYPE_CODE[y.dtype],
+                     0 if in_channel_first else 1, 0 if out_channel_first else 1, 1 if one_by_one else 0, scans, order)
     _lib.check(rc, "ss2d_cross_merge_flex")
     return x
 
@@ -120,8 +113,7 @@ def cross_scan_hip(x):
     x = x.contiguous()
     B, C, H, W = x.shape
     y = x.new_empty((B, 4, C, H * W))
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_cross_scan(x.data_ptr(), y.data_ptr(), B, C, H, W, x.element_size(), _stream(x))
+    rc = _lib.launch(x, _lib.lib().ss2d_cross_scan, x.data_ptr(), y.data_ptr(), B, C, H, W, x.element_size())
     _lib.check(rc, "ss2d_cross_scan")
     return y
 
@@ -142,9 +134,8 @@ def cross_scan_1b1_hip(x, out=None):
         raise ValueError(f"out must be a {(B, 4, C, H * W)} {x.dtype} tensor on {x.device}")
     if out.numel() and H * W > 1 and out.stride(3) != 1:
         raise ValueError("out must be contiguous in its last dimension")
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_cross_scan_1b1(x.data_ptr(), out.data_ptr(), B, C, H, W, x.element_size(), out.stride(0),
-                                            out.stride(1), out.stride(2), _stream(x))
+    rc = _lib.launch(x, _lib.lib().ss2d_cross_scan_1b1, x.data_ptr(), out.data_ptr(), B, C, H, W, x.element_size(),
+                     out.stride(0), out.stride(1), out.stride(2))
     _lib.check(rc, "ss2d_cross_scan_1b1")
     return out
 
@@ -159,8 +150,7 @@ def cross_merge_hip(ys, order=_lib.MERGE_PAIRWISE):
     ys = ys.contiguous()
     B, K, C, H, W = ys.shape
     out = ys.new_empty((B, C, H * W))
-    with torch.cuda.device(ys.device):
-        rc = _lib.lib().ss2d_cross_merge(ys.data_ptr(), out.data_ptr(), B, C, H, W, _DTYPE_CODE[ys.dtype], order, _stream(ys))
+    rc = _lib.launch(ys, _lib.lib().ss2d_cross_merge, ys.data_ptr(), out.data_ptr(), B, C, H, W, _DTYPE_CODE[ys.dtype], order)
     _lib.check(rc, "ss2d_cross_merge")
     return out
 

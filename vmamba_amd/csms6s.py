@@ -91,8 +91,7 @@ def selective_scan_fwd(u, delta, A, B, C, D=None, delta_bias=None, delta_softplu
     x = torch.empty((batch, dim, n_chunks, dstate * 2), device=u.device, dtype=torch.float32) if want_x else None
 
     p = _scan_params(u, delta, A, B, C, D, delta_bias, delta_softplus, out, x)
-    with torch.cuda.device(u.device):
-        rc = _lib.lib().ss2d_selective_scan_fwd(p, torch.cuda.current_stream(u.device).cuda_stream)
+    rc = _lib.launch(u, _lib.lib().ss2d_selective_scan_fwd, p)
     _lib.check(rc, "ss2d_selective_scan_fwd")
     return [out, x]
 
@@ -127,8 +126,7 @@ def selective_scan_from_map(x, delta, A, B, C, D=None, delta_bias=None, delta_so
     p.in_dtype = _DTYPE_CODE[x.dtype]
     p.u = x.data_ptr()
     p.u_batch_stride, p.u_d_stride = Dm * L, L
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_selective_scan_fwd_maps(p, x_t.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_selective_scan_fwd_maps, p, x_t.data_ptr())
     _lib.check(rc, "ss2d_selective_scan_fwd_maps")
     return out
 
@@ -190,8 +188,7 @@ def selective_scan_bwd(u, delta, A, B, C, D, delta_bias, dout, x=None, delta_sof
     p.C_batch_stride, p.C_group_stride, p.C_dstate_stride = C.stride(0), C.stride(1), C.stride(2)
     p.dout_batch_stride, p.dout_d_stride = dout.stride(0), dout.stride(1)
     if u.numel():
-        with torch.cuda.device(dev):
-            rc = _lib.lib().ss2d_selective_scan_bwd(p, torch.cuda.current_stream(dev).cuda_stream)
+        rc = _lib.launch(u, _lib.lib().ss2d_selective_scan_bwd, p)
         _lib.check(rc, "ss2d_selective_scan_bwd")
     if delta_dim != dim:        # channels sharing a delta row (selective_scan_oflex.cpp:347-352)
         ddelta = ddelta.view(batch, delta_dim, dim // delta_dim, seqlen).sum(2)

@@ -1,0 +1,77 @@
+// forward_core of a one-state block as one call (classification/models/vmamba.py:603-646): x_proj, dt_proj, the fused core and
+// out_norm enqueued back to back.  The kernels are those of the separate entry points; what this saves is the host's share.
+// From Python the four launches, their argument checks, tensors and views took 81 us for one map of 768 x 7 x 7 whose kernels
+// run for 38 -- and most of a 15-block model's time on one image.  One call with one workspace takes the host's share out of
+// everything but the largest batches.
+#include "ss2d_common.h"
+
+namespace ss2d {
+
+struct ForwardCorePlan {
+    int64_t pitch, x_dbl, delta, y, scratch, total;      // row pitch in elements; byte offsets; bytes
+    ss2d_core_params core;
+};
+
+static int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
+
+// base may be NULL while only the size is asked for: stand-in pointers of the same alignment take its place
+static int forward_core_plan(const ss2d_forward_core_params *q, char *base, ForwardCorePlan &p) {
+    if (!q) return SS2D_EINVAL;
+    if (q->batch <= 0 || q->dim <= 0 || q->height <= 0 || q->width <= 0 || q->rank <= 0) return SS2D_EINVAL;
+    if (q->dtype != SS2D_F32 && q->dtype != SS2D_BF16 && q->dtype != SS2D_F16) return SS2D_EINVAL;
+    if (!q->x || !q->x_proj_weight || !q->dt_proj_weight || !q->A || !q->out) return SS2D_EINVAL;
+    const int64_t L = (int64_t)q->height * q->width, D = q->dim, C = q->rank + 2, es = q->dtype == SS2D_F32 ? 4 : 2;
+    // rows of batch * L positions, kept on 16-byte boundaries: the next kernels then keep their vector accesses
+    const int64_t vec = 16 / es;
+    p.pitch = (q->batch * L + vec - 1) / vec * vec;
+    p.x_dbl = 0;
+    p.delta = align256(p.x_dbl + 4 * C * p.pitch * es);
+    p.y = align256(p.delta + 4 * D * p.pitch * es);
+    p.scratch = q->normalise ? align256(p.y + q->batch * D * L * 4) : p.y;
+    char *const at = base ? base : reinterpret_cast<char *>(256);
+    ss2d_core_params &c = p.core;
+    c.batch = q->batch; c.dim = q->dim; c.height = q->height; c.width = q->width;
+    c.in_dtype = q->dtype; c.delta_softplus = 1;
+    c.x = q->x; c.delta = at + p.delta; c.A = q->A; c.D = q->D; c.delta_bias = q->delta_bias;
+    c.B = at + p.x_dbl + (C - 2) * p.pitch * es; c.C = at + p.x_dbl + (C - 1) * p.pitch * es;
+    c.y = q->normalise ? at + p.y : q->out;
+    c.delta_dir_stride = D * p.pitch; c.delta_dim_stride = p.pitch; c.delta_batch_stride = L;
+    c.B_dir_stride = c.C_dir_stride = C * p.pitch; c.B_batch_stride = c.C_batch_stride = L;
+    const int64_t need = ss2d_core_workspace_bytes(&c);
+    if (need < 0) return (int)need;
+    p.total = align256(p.scratch + need);
+    return SS2D_OK;
+}
+
+}  // namespace ss2d
+
+extern "C" int64_t ss2d_forward_core_workspace_bytes(const ss2d_forward_core_params *q) {
+    ss2d::ForwardCorePlan p;
+    const int rc = ss2d::forward_core_plan(q, nullptr, p);
+    return rc != SS2D_OK ? rc : p.total;
+}
+
+extern "C" int ss2d_forward_core(const ss2d_forward_core_params *q, void *workspace, int64_t workspace_bytes, void *stream) {
+    using namespace ss2d;
+    if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return SS2D_EINVAL;
+    ForwardCorePlan p;
+    char *const base = reinterpret_cast<char *>(workspace);
+    int rc = forward_core_plan(q, base, p);
+    if (rc != SS2D_OK) return rc;
+    if (workspace_bytes < p.total) return SS2D_ENOMEM;
+    const int B = q->batch, D = q->dim, H = q->height, W = q->width, R = q->rank, C = R + 2;
+    const int64_t L = (int64_t)H * W, ks = C * p.pitch;
+    void *x_dbl = base + p.x_dbl, *delta = base + p.delta;
+    if (q->dtype == SS2D_F32) {
+        rc = ss2d_x_proj_f32((const float *)q->x, (const float *)q->x_proj_weight, (float *)x_dbl, B, D, C, H, W, ks, p.pitch, L, stream);
+        if (rc == SS2D_OK) rc = ss2d_dt_proj_f32((const float *)x_dbl, (const float *)q->dt_proj_weight, (float *)delta, 4, D, R, p.pitch, ks, p.pitch, stream);
+    } else {
+        rc = ss2d_x_proj(q->x, q->x_proj_weight, x_dbl, B, D, C, H, W, H, W, -1, ks, p.pitch, L, q->dtype, stream);
+        if (rc == SS2D_OK) rc = ss2d_dt_proj(x_dbl, q->dt_proj_weight, delta, 4, D, R, p.pitch, ks, p.pitch, q->dtype, stream);
+    }
+    if (rc == SS2D_OK) rc = ss2d_core_fwd_ws(&p.core, base + p.scratch, p.total - p.scratch, stream);
+    if (rc == SS2D_OK && q->normalise)
+        rc = ss2d_layer_norm_cf(base + p.y, q->norm_weight, q->norm_bias, q->out, B, D, (int)L, q->eps, SS2D_F32, q->norm_dtype,
+                                q->dtype, q->out_channel_last, stream);
+    return rc;
+}

@@ -35,10 +35,8 @@ def linear_cl_hip(x, weight, bias=None, residual=None, ln_weight=None, ln_bias=N
     small = [None if t is None else t.to(x.dtype).contiguous() for t in (ln_weight, ln_bias, bias)]
     keep = [weight.contiguous(), None if residual is None else residual.contiguous()]
     ptr = lambda t: None if t is None else t.data_ptr()
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_linear_cl(x.data_ptr(), ptr(small[0]), ptr(small[1]), float(eps), keep[0].data_ptr(), ptr(small[2]),
-                                       ptr(keep[1]), out.data_ptr(), x.numel() // K, K, N, _DTYPE_CODE[x.dtype],
-                                       torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_linear_cl, x.data_ptr(), ptr(small[0]), ptr(small[1]), float(eps), keep[0].data_ptr(),
+                     ptr(small[2]), ptr(keep[1]), out.data_ptr(), x.numel() // K, K, N, _DTYPE_CODE[x.dtype])
     _lib.check(rc, "ss2d_linear_cl")
     return out
 
@@ -70,9 +68,7 @@ def linear_cf_ln_hip(y, ln_weight, ln_bias, eps, weight, bias=None, residual=Non
         raise ValueError("linear_cf_ln_hip: the LayerNorm weight is required")
     keep = [weight.contiguous(), None if residual is None else residual.contiguous()]
     ptr = lambda t: None if t is None else t.data_ptr()
-    with torch.cuda.device(y.device):
-        rc = _lib.lib().ss2d_linear_cf_ln(y.data_ptr(), ptr(small[0]), ptr(small[1]), float(eps), keep[0].data_ptr(), ptr(small[2]),
-                                          ptr(keep[1]), out.data_ptr(), B, L, K, N, _DTYPE_CODE[dt],
-                                          torch.cuda.current_stream(y.device).cuda_stream)
+    rc = _lib.launch(y, _lib.lib().ss2d_linear_cf_ln, y.data_ptr(), ptr(small[0]), ptr(small[1]), float(eps),
+                     keep[0].data_ptr(), ptr(small[2]), ptr(keep[1]), out.data_ptr(), B, L, K, N, _DTYPE_CODE[dt])
     _lib.check(rc, "ss2d_linear_cf_ln")
     return out

@@ -38,10 +38,8 @@ def mlp_fused_hip(x, w1, b1, w2, b2, residual=None, ln_weight=None, ln_bias=None
     out = torch.empty_like(x)
     ptr = lambda t: None if t is None else t.contiguous().data_ptr()
     keep = [None if t is None else t.to(x.dtype).contiguous() for t in (b1, b2, ln_weight, ln_bias)]
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_mlp_fused(x.data_ptr(), ptr(keep[2]), ptr(keep[3]), float(eps), w1.data_ptr(), ptr(keep[0]),
-                                       w2.data_ptr(), ptr(keep[1]), ptr(residual),
-                                       out.data_ptr(), x.numel() // C, C, _DTYPE_CODE[x.dtype],
-                                       torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_mlp_fused, x.data_ptr(), ptr(keep[2]), ptr(keep[3]), float(eps), w1.data_ptr(),
+                     ptr(keep[0]), w2.data_ptr(), ptr(keep[1]), ptr(residual), out.data_ptr(), x.numel() // C, C,
+                     _DTYPE_CODE[x.dtype])
     _lib.check(rc, "ss2d_mlp_fused")
     return out

@@ -28,11 +28,9 @@ def layer_norm_hip(x, weight, bias, eps=1e-5, out_dtype=None):
     C = x.shape[-1]
     weight, bias, wdt = _params(weight, bias)
     y = torch.empty(x.shape, device=x.device, dtype=out_dtype or x.dtype)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_layer_norm(x.data_ptr(), weight.data_ptr() if weight is not None else None,
-                                        bias.data_ptr() if bias is not None else None, y.data_ptr(),
-                                        x.numel() // max(C, 1), C, eps, _DTYPE_CODE[x.dtype], _DTYPE_CODE[wdt],
-                                        _DTYPE_CODE[y.dtype], torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_layer_norm, x.data_ptr(), weight.data_ptr() if weight is not None else None,
+                     bias.data_ptr() if bias is not None else None, y.data_ptr(), x.numel() // max(C, 1), C, eps,
+                     _DTYPE_CODE[x.dtype], _DTYPE_CODE[wdt], _DTYPE_CODE[y.dtype])
     _lib.check(rc, "ss2d_layer_norm")
     return y
 
@@ -55,11 +53,10 @@ def add_layer_norm_hip(x, residual, weight, bias, eps=1e-5):
     C = x.shape[-1]
     weight, bias, wdt = _params(weight, bias)
     total, y = torch.empty_like(x), torch.empty_like(x)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_add_layer_norm(x.data_ptr(), residual.data_ptr(), weight.data_ptr() if weight is not None else None,
-                                            bias.data_ptr() if bias is not None else None, total.data_ptr(), y.data_ptr(),
-                                            x.numel() // max(C, 1), C, eps, _DTYPE_CODE[x.dtype], _DTYPE_CODE[wdt],
-                                            _DTYPE_CODE[y.dtype], torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_add_layer_norm, x.data_ptr(), residual.data_ptr(),
+                     weight.data_ptr() if weight is not None else None, bias.data_ptr() if bias is not None else None,
+                     total.data_ptr(), y.data_ptr(), x.numel() // max(C, 1), C, eps, _DTYPE_CODE[x.dtype], _DTYPE_CODE[wdt],
+                     _DTYPE_CODE[y.dtype])
     _lib.check(rc, "ss2d_add_layer_norm")
     return total, y
 
@@ -81,11 +78,9 @@ def bias_layer_norm_hip(x, pre_bias, weight, bias, eps=1e-5):
     weight, bias, wdt = _params(weight, bias)
     pre_bias = pre_bias.to(wdt).contiguous()
     y = torch.empty_like(x)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_bias_layer_norm(x.data_ptr(), pre_bias.data_ptr(), weight.data_ptr() if weight is not None else None,
-                                             bias.data_ptr() if bias is not None else None, y.data_ptr(),
-                                             x.numel() // max(C, 1), C, eps, _DTYPE_CODE[x.dtype], _DTYPE_CODE[wdt],
-                                             _DTYPE_CODE[y.dtype], torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_bias_layer_norm, x.data_ptr(), pre_bias.data_ptr(),
+                     weight.data_ptr() if weight is not None else None, bias.data_ptr() if bias is not None else None,
+                     y.data_ptr(), x.numel() // max(C, 1), C, eps, _DTYPE_CODE[x.dtype], _DTYPE_CODE[wdt], _DTYPE_CODE[y.dtype])
     _lib.check(rc, "ss2d_bias_layer_norm")
     return y
 
@@ -105,11 +100,9 @@ def layer_norm_cf_hip(x, weight, bias, eps=1e-5, out_channel_last=False, out_dty
     weight, bias, wdt = _params(weight, bias)
     shape = (B, *spatial, C) if out_channel_last else (B, C, *spatial)
     y = torch.empty(shape, device=x.device, dtype=out_dtype or x.dtype)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_layer_norm_cf(x.data_ptr(), weight.data_ptr() if weight is not None else None,
-                                           bias.data_ptr() if bias is not None else None, y.data_ptr(), B, C, L, eps,
-                                           _DTYPE_CODE[x.dtype], _DTYPE_CODE[wdt], _DTYPE_CODE[y.dtype],
-                                           int(bool(out_channel_last)), torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_layer_norm_cf, x.data_ptr(), weight.data_ptr() if weight is not None else None,
+                     bias.data_ptr() if bias is not None else None, y.data_ptr(), B, C, L, eps, _DTYPE_CODE[x.dtype],
+                     _DTYPE_CODE[wdt], _DTYPE_CODE[y.dtype], int(bool(out_channel_last)))
     _lib.check(rc, "ss2d_layer_norm_cf")
     return y
 

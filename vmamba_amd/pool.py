@@ -24,9 +24,7 @@ def mean_pool_cl_hip(x):
     x = x.contiguous()
     B, L, C = x.shape
     y = torch.empty((B, C), device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_mean_pool_cl(x.data_ptr(), y.data_ptr(), B, L, C, _DTYPE_CODE[x.dtype],
-                                          torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_mean_pool_cl, x.data_ptr(), y.data_ptr(), B, L, C, _DTYPE_CODE[x.dtype])
     _lib.check(rc, "ss2d_mean_pool_cl")
     return y
 

@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from ._lib import SS2D_ENOTSUP, Ss2dError
 from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_fits, core_mask_pads_hip, dt_proj_f32_hip, dt_proj_hip,
-                   embed_maps_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_fits, x_proj_hip)
+                   embed_maps_hip, forward_core_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_fits, x_proj_hip)
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
 from .conv import DwConv3x3SiLU, dwconv3x3_silu_hip, dwconv_silu_trainable
@@ -180,11 +180,12 @@ class SS2D(nn.Module):
                 return pinned[key]
             return cache[key]
         K = self.k_group
-        consts = dict(
-            As=-self.A_logs.float().exp(), Ds=self.Ds.float(), dt_bias=self.dt_projs_bias.reshape(-1).float(),
-            Wx_all=self.x_proj_weight.reshape(1, -1, self.d_inner).expand(batch, -1, -1).contiguous(),
-            Wx=self.x_proj_weight.unsqueeze(0).expand(batch, -1, -1, -1).reshape(batch * K, -1, self.d_inner).contiguous(),
-            Wdt=self.dt_projs_weight.unsqueeze(0).expand(batch, -1, -1, -1).reshape(batch * K, self.d_inner, -1).contiguous())
+        consts = dict(As=-self.A_logs.float().exp(), Ds=self.Ds.float(), dt_bias=self.dt_projs_bias.reshape(-1).float())
+        if batch:                  # 0: a caller that needs no weights repeated over images
+            consts.update(
+                Wx_all=self.x_proj_weight.reshape(1, -1, self.d_inner).expand(batch, -1, -1).contiguous(),
+                Wx=self.x_proj_weight.unsqueeze(0).expand(batch, -1, -1, -1).reshape(batch * K, -1, self.d_inner).contiguous(),
+                Wdt=self.dt_projs_weight.unsqueeze(0).expand(batch, -1, -1, -1).reshape(batch * K, self.d_inner, -1).contiguous())
         if not torch.is_grad_enabled() and not capturing:
             stale = [k for k in cache if k[2] != key[2]]
             for k in stale:
@@ -300,7 +301,26 @@ class SS2D(nn.Module):
         trains = needs_grad(x, self.x_proj_weight, self.dt_projs_weight, self.A_logs, self.Ds, self.dt_projs_bias)
         return self.d_state == 1 and self.fused_core and not trains and core_fits(x.shape[2], x.shape[3], x.dtype)
 
+    def _forward_core_native(self, x, normalise):
+        """forward_core -- or, without ``normalise``, forward_core_fused -- as one call into the library, or None where that
+        does not stand for them: training, a padded map, other layers or an out_norm of another kind, a subclass with its
+        own steps, a shape without a kernel."""
+        cls, norm = type(self), self.out_norm
+        if not (x.is_cuda and x.dim() == 4 and x.numel() > 0 and self._fused_core_applies(x)
+                and cls.forward_core_fused is SS2D.forward_core_fused and cls.finish_core is SS2D.finish_core
+                and cls._inference_constants is SS2D._inference_constants):
+            return None
+        if normalise and not (self.layers is HipLayers and type(norm) is (LayerNorm2d if self.channel_first else LayerNorm)
+                              and norm.normalized_shape == (x.shape[1],) and not needs_grad(norm.weight, norm.bias)):
+            return None
+        consts = self._inference_constants(0)
+        return forward_core_hip(x, self.x_proj_weight, self.dt_projs_weight, consts["As"], consts["Ds"], consts["dt_bias"],
+                                norm if normalise else None, not self.channel_first)
+
     def forward_core(self, x):
+        out = self._forward_core_native(x, True)
+        if out is not None:
+            return out
         B, D, H, W = x.shape
         K, L = self.k_group, H * W
         consts = self._inference_constants(B)
@@ -391,7 +411,9 @@ class SS2D(nn.Module):
             # out_norm, out_proj and the residual add in one kernel, straight from the core's fp32 map
             B, _, H, W = x.shape
             try:
-                y = self.forward_core_fused(x, self._inference_constants(B))                    # (B, D, L) fp32
+                y = self._forward_core_native(x, False)                                         # (B, D, L) fp32
+                if y is None:
+                    y = self.forward_core_fused(x, self._inference_constants(B))
             except Ss2dError as e:          # no fused variant for this shape: forward_core's three-operator path below
                 if e.code != SS2D_ENOTSUP:
                     raise

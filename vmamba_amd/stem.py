@@ -37,9 +37,7 @@ def stem_conv_ln_gelu_hip(x, weight, bias, ln_weight, ln_bias, eps=1e-5):
     ptr = lambda t: None if t is None else t.data_ptr()
     y = torch.empty((B, (H - 1) // 2 + 1, (W - 1) // 2 + 1, C), device=x.device, dtype=x.dtype)
     strides = (ctypes.c_int64 * 4)(*weight.stride())
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().ss2d_stem_conv_ln_gelu(x.data_ptr(), weight.data_ptr(), strides, ptr(bias), ptr(ln_weight), ptr(ln_bias),
-                                               eps, y.data_ptr(), B, H, W, C, _DTYPE_CODE[x.dtype],
-                                               torch.cuda.current_stream(x.device).cuda_stream)
+    rc = _lib.launch(x, _lib.lib().ss2d_stem_conv_ln_gelu, x.data_ptr(), weight.data_ptr(), strides, ptr(bias), ptr(ln_weight),
+                     ptr(ln_bias), eps, y.data_ptr(), B, H, W, C, _DTYPE_CODE[x.dtype])
     _lib.check(rc, "ss2d_stem_conv_ln_gelu")
     return y
