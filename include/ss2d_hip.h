@@ -438,6 +438,15 @@ int ss2d_stem_conv_ln_gelu(const void *x, const void *weight, const int64_t *wei
                            int dtype, void *stream);
 
 /*
+ * Second layer of the patch embedding (classification/models/vmamba.py:1412-1416): y = LayerNorm(conv2d(x, weight, bias;
+ * kernel 3, stride 2, padding 1)) with x (B,H,W,Cin) and y (B,Ho,Wo,Cout) channel-last on 16-byte boundaries, the weight
+ * (Cout,Cin,3,3) through its four strides, bias and LayerNorm parameters (Cout) or NULL; all bf16 or fp16.  The convolution is
+ * rounded to that type before the LayerNorm.  SS2D_ENOTSUP: fp32, any other width than Cin = 48, Cout = 96, inputs of 2 GiB.
+ */
+int ss2d_stem_conv2_ln(const void *x, const void *weight, const int64_t *weight_strides, const void *bias, const void *ln_weight,
+                       const void *ln_bias, float eps, void *y, int B, int H, int W, int Cin, int Cout, int dtype, void *stream);
+
+/*
  * dt_proj of the SS2D core: the per-direction rank-R -> D projection between x_proj and the scan.
  * Replaces the grouped conv1d / einsum of SS2Dv2.forward_corev2 (classification/models/vmamba.py:608-609, 614-615):
  *   delta[k, d, n] = sum_r weight[k, d, r] * x[k*x_dir_stride + r*x_rank_stride + n]

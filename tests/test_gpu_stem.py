@@ -59,3 +59,45 @@ def test_stem_without_affine_parameters_and_rejections():
     with pytest.raises(NotImplementedError):
         stem_conv_ln_gelu_hip(torch.zeros(1, 3, 8, 8).bfloat16(), torch.zeros(48, 3, 3, 3).bfloat16(), None, None, None)
     assert stem_conv_ln_gelu_hip(torch.zeros(0, 3, 8, 8, **bf), torch.zeros(48, 3, 3, 3, **bf), None, None, None).shape == (0, 4, 4, 48)
+
+
+# ---- second layer: conv 48 -> 96 + LayerNorm ----------------------------------------------------------------------
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("channels_last_weight", [False, True])
+@pytest.mark.parametrize("B,H,W", [(2, 56, 56),                  # whole units
+                                   (1, 1, 1), (1, 2, 3), (3, 15, 17),       # odd sides: taps beyond the last row and column
+                                   (1, 16, 130), (5, 9, 8),      # units across rows and images, a short last one
+                                   (3, 224, 160)])               # more units than workgroups
+def test_stem2_matches_conv_layernorm(B, H, W, dtype, channels_last_weight):
+    """The reference rounds the convolution where the kernel does; a difference in its last bit moves a normalised value by a
+    few of its roundings: 2^-7 (bf16) / 2^-10 (fp16) of values of up to about 8 after the affine map."""
+    from vmamba_amd.stem import stem_conv2_ln_hip
+    print("CASE stem2", B, H, W, dtype, channels_last_weight, flush=True)
+    g = torch.Generator().manual_seed(B * 100 + H + W)
+    x = torch.randn(B, 48, H, W, generator=g).to(dtype)
+    w = (torch.randn(96, 48, 3, 3, generator=g) * 0.1).to(dtype)
+    b, gamma, beta = ((torch.randn(96, generator=g) * 0.3 + m).to(dtype) for m in (0, 1, 0))
+    conv = F.conv2d(x.float(), w.float(), b.float(), stride=2, padding=1).to(dtype).float().permute(0, 2, 3, 1)
+    want = F.layer_norm(conv, (96,), gamma.float(), beta.float(), 1e-5)
+    wd = w.to(DEV)
+    if channels_last_weight:
+        wd = wd.contiguous(memory_format=torch.channels_last)
+    got = stem_conv2_ln_hip(x.to(DEV).permute(0, 2, 3, 1).contiguous(), wd, b.to(DEV), gamma.to(DEV), beta.to(DEV), 1e-5)
+    assert got.shape == want.shape and got.dtype == dtype
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert bool(((got.cpu().float() - want).abs() <= 2 * eps * (want.abs() + 8)).all())
+    plain = stem_conv2_ln_hip(x.to(DEV).permute(0, 2, 3, 1).contiguous(), wd, None, None, None, 1e-5)
+    conv = F.conv2d(x.float(), w.float(), stride=2, padding=1).to(dtype).float().permute(0, 2, 3, 1)
+    assert bool(((plain.cpu().float() - F.layer_norm(conv, (96,))).abs() <= 2 * eps * 16).all())
+
+
+def test_stem2_rejections():
+    from vmamba_amd.stem import stem_conv2_ln_hip
+    bf = dict(device=DEV, dtype=torch.bfloat16)
+    with pytest.raises(_lib.Ss2dError) as e:
+        stem_conv2_ln_hip(torch.zeros(1, 4, 4, 64, **bf), torch.zeros(96, 64, 3, 3, **bf), None, None, None)
+    assert e.value.code == _lib.SS2D_ENOTSUP
+    with pytest.raises(RuntimeError):
+        stem_conv2_ln_hip(torch.zeros(1, 4, 4, 48, device=DEV), torch.zeros(96, 48, 3, 3, device=DEV), None, None, None)
+    with pytest.raises(ValueError):
+        stem_conv2_ln_hip(torch.zeros(1, 4, 4, 40, **bf), torch.zeros(96, 48, 3, 3, **bf), None, None, None)

@@ -23,7 +23,7 @@ from .norm import LayerNorm as HipLayerNorm
 from .norm import add_layer_norm_fusable, add_layer_norm_hip, bias_layer_norm_fusable, bias_layer_norm_hip, needs_grad
 from .ss2d import SS2D, HipLayers, Linear2d
 from .pool import GlobalAvgPool2d
-from .stem import stem_conv_ln_gelu_hip, stem_fusable
+from .stem import stem2_fusable, stem_conv2_ln_hip, stem_conv_ln_gelu_hip, stem_fusable
 
 
 class Permute(nn.Module):
@@ -59,6 +59,10 @@ class ConvNormSequence(nn.Sequential):
                 i += 5
             elif i + 2 < len(mods) and self._fusable(x, conv, mods[i + 1], mods[i + 2]):
                 norm = mods[i + 2]
+                if stem2_fusable(x, conv, norm):      # convolution and LayerNorm in one kernel
+                    x = stem_conv2_ln_hip(x.permute(0, 2, 3, 1), conv.weight, conv.bias, norm.weight, norm.bias, norm.eps)
+                    i += 3
+                    continue
                 x = conv._conv_forward(x, conv.weight, None).permute(0, 2, 3, 1)
                 x = bias_layer_norm_hip(x, conv.bias, norm.weight, norm.bias, norm.eps)
                 i += 3
