@@ -327,15 +327,18 @@ int ss2d_core_fwd_ws(const ss2d_core_params *params, void *workspace, int64_t wo
  *   x (B,D,H,W); x_proj_weight (4, rank + 2, D); dt_proj_weight (4, D, rank), all of `dtype`; A, D, delta_bias (4*D) fp32
  *   out   normalise: (B,D,L), or (B,L,D) if out_channel_last, of `dtype`; else the merged map (B,D,L) fp32
  *   norm_weight, norm_bias (D) of norm_dtype or NULL
+ *   padded_height, padded_width   the map's own size, or a larger one to embed it in (ss2d_core_embed_maps; 16-bit types), with
+ *         pad_mask as ss2d_dt_proj_masked takes it for the (4, batch * padded positions) in scan order; the result is cropped
  * Everything contiguous.  workspace: ss2d_forward_core_workspace_bytes(params) bytes, 16-byte aligned, contents irrelevant;
  * workspace_bytes depends on the sizes and types, and on the pointers' alignment.  Either function returns SS2D_ENOTSUP where
  * one of the kernels has no variant for the problem.
  */
 typedef struct ss2d_forward_core_params {
     int32_t batch, dim, height, width, rank;
+    int32_t padded_height, padded_width;
     int32_t dtype, norm_dtype, normalise, out_channel_last;
     float eps;
-    const void *x, *x_proj_weight, *dt_proj_weight, *A, *D, *delta_bias, *norm_weight, *norm_bias;
+    const void *x, *x_proj_weight, *dt_proj_weight, *A, *D, *delta_bias, *norm_weight, *norm_bias, *pad_mask;
     void *out;
 } ss2d_forward_core_params;
 

@@ -71,11 +71,11 @@ class CoreParams(ctypes.Structure):
 class ForwardCoreParams(ctypes.Structure):
     """struct ss2d_forward_core_params (include/ss2d_hip.h)."""
     _fields_ = (
-        [(n, ctypes.c_int32) for n in ("batch", "dim", "height", "width", "rank", "dtype", "norm_dtype", "normalise",
-                                       "out_channel_last")]
+        [(n, ctypes.c_int32) for n in ("batch", "dim", "height", "width", "rank", "padded_height", "padded_width",
+                                       "dtype", "norm_dtype", "normalise", "out_channel_last")]
         + [("eps", ctypes.c_float)]
         + [(n, ctypes.c_void_p) for n in ("x", "x_proj_weight", "dt_proj_weight", "A", "D", "delta_bias", "norm_weight",
-                                          "norm_bias", "out")]
+                                          "norm_bias", "pad_mask", "out")]
     )
 
 

@@ -151,16 +151,20 @@ def ss2d_core_hip(x, delta, Bs, Cs, As, Ds=None, delta_bias=None, delta_softplus
     return y
 
 
-def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=None, out_channel_last=False):
+def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=None, out_channel_last=False, pad_mask=None):
     """x_proj, dt_proj, the fused core and -- with ``norm`` -- out_norm in one call (ss2d_forward_core): x (B,D,H,W),
     x_proj_weight (4,R+2,D), dt_proj_weight (4,D,R) of one dtype; As, Ds, dt_bias (4*D) fp32; norm a LayerNorm over D.  Returns
     (B,H,W,D) if ``out_channel_last`` else (B,D,H,W) in x.dtype, the merged map (B,D,L) in fp32 without ``norm``, or None
-    where the kernels have no variant for the call and the separate ones have to be tried."""
+    where the kernels have no variant for the call and the separate ones have to be tried.  Maps that padded_map_size embeds in
+    larger ones need pad_mask(H, W, padded H, padded W, B, device): the mask dt_proj_hip takes."""
     B, D, H, W = x.shape
     R = dt_proj_weight.shape[2]
     code = _DTYPE_CODE.get(x.dtype)
     if (code is None or x.numel() == 0 or R == 0 or tuple(x_proj_weight.shape) != (4, R + 2, D) or tuple(dt_proj_weight.shape) != (4, D, R)
-            or not As.numel() == Ds.numel() == dt_bias.numel() == 4 * D or padded_map_size(H, W, x.dtype) is not None):
+            or not As.numel() == Ds.numel() == dt_bias.numel() == 4 * D):
+        return None
+    padded = padded_map_size(H, W, x.dtype)
+    if padded is not None and (pad_mask is None or R > DT_PROJ_MAX_RANK):
         return None
     index = x.get_device()
     for t in (x_proj_weight, dt_proj_weight):
@@ -170,7 +174,12 @@ def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=Non
         if t.dtype != torch.float32 or t.get_device() != index or not t.is_contiguous():
             return None
     x = x.contiguous()
-    p = _lib.ForwardCoreParams(B, D, H, W, R, code)
+    p = _lib.ForwardCoreParams(B, D, H, W, R, *(padded or (H, W)), code)
+    if padded is not None:
+        mask = pad_mask(H, W, *padded, B, x.device)
+        _check(mask.get_device() == index and mask.dtype == torch.int16 and mask.is_contiguous()
+               and tuple(mask.shape) == (4, B * padded[0] * padded[1]), "pad_mask: (4, B * L) int16")
+        p.pad_mask = mask.data_ptr()
     if norm is not None:
         weight, bias = norm.weight, norm.bias
         for t in (weight, bias):

@@ -8,7 +8,8 @@
 namespace ss2d {
 
 struct ForwardCorePlan {
-    int64_t pitch, x_dbl, delta, y, scratch, total;      // row pitch in elements; byte offsets; bytes
+    bool padded;
+    int64_t pitch, x, x_dbl, delta, y, out, scratch, total;          // row pitch in elements; byte offsets; bytes
     ss2d_core_params core;
 };
 
@@ -20,21 +21,28 @@ static int forward_core_plan(const ss2d_forward_core_params *q, char *base, Forw
     if (q->batch <= 0 || q->dim <= 0 || q->height <= 0 || q->width <= 0 || q->rank <= 0) return SS2D_EINVAL;
     if (q->dtype != SS2D_F32 && q->dtype != SS2D_BF16 && q->dtype != SS2D_F16) return SS2D_EINVAL;
     if (!q->x || !q->x_proj_weight || !q->dt_proj_weight || !q->A || !q->out) return SS2D_EINVAL;
-    const int64_t L = (int64_t)q->height * q->width, D = q->dim, C = q->rank + 2, es = q->dtype == SS2D_F32 ? 4 : 2;
+    if (q->padded_height < q->height || q->padded_width < q->width) return SS2D_EINVAL;
+    p.padded = q->padded_height > q->height || q->padded_width > q->width;
+    if (p.padded && (q->dtype == SS2D_F32 || !q->pad_mask)) return q->dtype == SS2D_F32 ? SS2D_ENOTSUP : SS2D_EINVAL;
+    const int64_t L = (int64_t)q->padded_height * q->padded_width, D = q->dim, C = q->rank + 2, es = q->dtype == SS2D_F32 ? 4 : 2;
     // rows of batch * L positions, kept on 16-byte boundaries: the next kernels then keep their vector accesses
     const int64_t vec = 16 / es;
     p.pitch = (q->batch * L + vec - 1) / vec * vec;
-    p.x_dbl = 0;
+    // on a padded map delta has to start every image where its mask does
+    if (p.padded && p.pitch != q->batch * L) return SS2D_ENOTSUP;
+    p.x = 0;
+    p.x_dbl = p.padded ? align256(p.x + q->batch * D * L * es) : 0;
     p.delta = align256(p.x_dbl + 4 * C * p.pitch * es);
     p.y = align256(p.delta + 4 * D * p.pitch * es);
-    p.scratch = q->normalise ? align256(p.y + q->batch * D * L * 4) : p.y;
+    p.out = q->normalise || p.padded ? align256(p.y + q->batch * D * L * 4) : p.y;
+    p.scratch = q->normalise && p.padded ? align256(p.out + q->batch * D * L * es) : p.out;
     char *const at = base ? base : reinterpret_cast<char *>(256);
     ss2d_core_params &c = p.core;
-    c.batch = q->batch; c.dim = q->dim; c.height = q->height; c.width = q->width;
+    c.batch = q->batch; c.dim = q->dim; c.height = q->padded_height; c.width = q->padded_width;
     c.in_dtype = q->dtype; c.delta_softplus = 1;
-    c.x = q->x; c.delta = at + p.delta; c.A = q->A; c.D = q->D; c.delta_bias = q->delta_bias;
+    c.x = p.padded ? at + p.x : q->x; c.delta = at + p.delta; c.A = q->A; c.D = q->D; c.delta_bias = q->delta_bias;
     c.B = at + p.x_dbl + (C - 2) * p.pitch * es; c.C = at + p.x_dbl + (C - 1) * p.pitch * es;
-    c.y = q->normalise ? at + p.y : q->out;
+    c.y = q->normalise || p.padded ? at + p.y : q->out;
     c.delta_dir_stride = D * p.pitch; c.delta_dim_stride = p.pitch; c.delta_batch_stride = L;
     c.B_dir_stride = c.C_dir_stride = C * p.pitch; c.B_batch_stride = c.C_batch_stride = L;
     const int64_t need = ss2d_core_workspace_bytes(&c);
@@ -59,19 +67,28 @@ extern "C" int ss2d_forward_core(const ss2d_forward_core_params *q, void *worksp
     int rc = forward_core_plan(q, base, p);
     if (rc != SS2D_OK) return rc;
     if (workspace_bytes < p.total) return SS2D_ENOMEM;
-    const int B = q->batch, D = q->dim, H = q->height, W = q->width, R = q->rank, C = R + 2;
+    const int B = q->batch, D = q->dim, H = q->padded_height, W = q->padded_width, R = q->rank, C = R + 2;
     const int64_t L = (int64_t)H * W, ks = C * p.pitch;
+    const int es = q->dtype == SS2D_F32 ? 4 : 2;
     void *x_dbl = base + p.x_dbl, *delta = base + p.delta;
+    if (p.padded) rc = ss2d_core_embed_maps(q->x, base + p.x, (int64_t)B * D, q->height, q->width, H, W, es, stream);
+    const void *x = p.core.x;
     if (q->dtype == SS2D_F32) {
-        rc = ss2d_x_proj_f32((const float *)q->x, (const float *)q->x_proj_weight, (float *)x_dbl, B, D, C, H, W, ks, p.pitch, L, stream);
+        rc = ss2d_x_proj_f32((const float *)x, (const float *)q->x_proj_weight, (float *)x_dbl, B, D, C, H, W, ks, p.pitch, L, stream);
         if (rc == SS2D_OK) rc = ss2d_dt_proj_f32((const float *)x_dbl, (const float *)q->dt_proj_weight, (float *)delta, 4, D, R, p.pitch, ks, p.pitch, stream);
     } else {
-        rc = ss2d_x_proj(q->x, q->x_proj_weight, x_dbl, B, D, C, H, W, H, W, -1, ks, p.pitch, L, q->dtype, stream);
-        if (rc == SS2D_OK) rc = ss2d_dt_proj(x_dbl, q->dt_proj_weight, delta, 4, D, R, p.pitch, ks, p.pitch, q->dtype, stream);
+        if (rc == SS2D_OK) rc = ss2d_x_proj(x, q->x_proj_weight, x_dbl, B, D, C, H, W, H, W, -1, ks, p.pitch, L, q->dtype, stream);
+        // a step of softplus(fill) = 0 at the added positions
+        if (rc == SS2D_OK) rc = ss2d_dt_proj_masked(x_dbl, q->dt_proj_weight, p.padded ? q->pad_mask : nullptr, q->dtype == SS2D_F16 ? -65504.0f : -1e30f,
+                                                    delta, 4, D, R, p.pitch, ks, p.pitch, q->dtype, stream);
     }
     if (rc == SS2D_OK) rc = ss2d_core_fwd_ws(&p.core, base + p.scratch, p.total - p.scratch, stream);
     if (rc == SS2D_OK && q->normalise)
-        rc = ss2d_layer_norm_cf(base + p.y, q->norm_weight, q->norm_bias, q->out, B, D, (int)L, q->eps, SS2D_F32, q->norm_dtype,
-                                q->dtype, q->out_channel_last, stream);
-    return rc;
+        rc = ss2d_layer_norm_cf(base + p.y, q->norm_weight, q->norm_bias, p.padded ? base + p.out : q->out, B, D, (int)L, q->eps, SS2D_F32,
+                                q->norm_dtype, q->dtype, q->out_channel_last, stream);
+    if (rc != SS2D_OK || !p.padded) return rc;
+    if (!q->normalise) return ss2d_core_embed_maps(base + p.y, q->out, (int64_t)B * D, H, W, q->height, q->width, 4, stream);
+    if (q->out_channel_last)                                         // an image is one map of H rows of W * D elements
+        return ss2d_core_embed_maps(base + p.out, q->out, B, H, (int64_t)W * D, q->height, (int64_t)q->width * D, es, stream);
+    return ss2d_core_embed_maps(base + p.out, q->out, (int64_t)B * D, H, W, q->height, q->width, es, stream);
 }

@@ -303,7 +303,7 @@ class SS2D(nn.Module):
 
     def _forward_core_native(self, x, normalise):
         """forward_core -- or, without ``normalise``, forward_core_fused -- as one call into the library, or None where that
-        does not stand for them: training, a padded map, other layers or an out_norm of another kind, a subclass with its
+        does not stand for them: training, other layers or an out_norm of another kind, a subclass with its
         own steps, a shape without a kernel."""
         cls, norm = type(self), self.out_norm
         if not (x.is_cuda and x.dim() == 4 and x.numel() > 0 and self._fused_core_applies(x)
@@ -315,7 +315,7 @@ class SS2D(nn.Module):
             return None
         consts = self._inference_constants(0)
         return forward_core_hip(x, self.x_proj_weight, self.dt_projs_weight, consts["As"], consts["Ds"], consts["dt_bias"],
-                                norm if normalise else None, not self.channel_first)
+                                norm if normalise else None, not self.channel_first, _pad_mask)
 
     def forward_core(self, x):
         out = self._forward_core_native(x, True)
