@@ -34,8 +34,8 @@ static int forward_core_plan(const ss2d_forward_core_params *q, char *base, Forw
     p.x_dbl = p.padded ? align256(p.x + q->batch * D * L * es) : 0;
     p.delta = align256(p.x_dbl + 4 * C * p.pitch * es);
     p.y = align256(p.delta + 4 * D * p.pitch * es);
-    p.out = q->normalise || p.padded ? align256(p.y + q->batch * D * L * 4) : p.y;
-    p.scratch = q->normalise && p.padded ? align256(p.out + q->batch * D * L * es) : p.out;
+    p.out = p.delta;                                                 // the normalised padded map: four times its room, and read already
+    p.scratch = q->normalise || p.padded ? align256(p.y + q->batch * D * L * 4) : p.y;
     char *const at = base ? base : reinterpret_cast<char *>(256);
     ss2d_core_params &c = p.core;
     c.batch = q->batch; c.dim = q->dim; c.height = q->padded_height; c.width = q->padded_width;
