@@ -179,6 +179,14 @@ typedef struct ss2d_scan_bwd_params {
 int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *params, void *stream);
 
 /*
+ * Around it: up to SS2D_CLEAR_MAX buffers of 4-byte elements on 16-byte boundaries set to zero (the accumulators of the call
+ * above, selective_scan_oflex.cpp:310-330), and two fp32 tensors rounded to bf16 / fp16 (dB and dC, :346), one launch each.
+ */
+#define SS2D_CLEAR_MAX 8
+int ss2d_clear(void *const *ptrs, const int64_t *bytes, int n, void *stream);
+int ss2d_round_pair(const float *src0, void *dst0, int64_t n0, const float *src1, void *dst1, int64_t n1, int dtype, void *stream);
+
+/*
  * LayerNorm over the channel axis, the step after CrossMerge (out_norm) and the block norms of the model.
  * Replaces the torch calls of LayerNorm2d.forward (classification/models/vmamba.py:52-57: permute,
  * F.layer_norm, permute) and of nn.LayerNorm on (B,H,W,C) activations, including the transposition

@@ -131,3 +131,26 @@ def test_scan_bwd_rejections():
     p = _lib.ScanBwdParams()
     assert _lib.lib().ss2d_selective_scan_bwd(p, None) == _lib.SS2D_EINVAL           # dstate 0
     assert _lib.lib().ss2d_selective_scan_bwd(None, None) == _lib.SS2D_EINVAL
+
+
+def test_cleared_accumulators_and_rounded_pair():
+    """ss2d_clear and ss2d_round_pair at their edges: sizes around a thread's 16 bytes and a workgroup's 16 KB, the words behind
+    a buffer untouched, the same bits as torch's conversion."""
+    import ctypes
+    from vmamba_amd import _lib
+    sizes = [1, 3, 4, 5, 4095, 4096, 4097, 12291]
+    store = [torch.full((n + 4,), 7.0, device="cuda") for n in sizes]
+    ptrs, nbytes = (ctypes.c_void_p * 8)(*(t.data_ptr() for t in store)), (ctypes.c_int64 * 8)(*(4 * n for n in sizes))
+    assert _lib.launch(store[0], _lib.lib().ss2d_clear, ptrs, nbytes, 8) == _lib.SS2D_OK
+    for t, n in zip(store, sizes):
+        assert bool((t[:n] == 0).all()) and bool((t[n:] == 7).all())
+    assert _lib.launch(store[0], _lib.lib().ss2d_clear, ptrs, nbytes, 9) == _lib.SS2D_EINVAL
+    for dtype in (torch.bfloat16, torch.float16):
+        for n0, n1 in ((1, 2048), (2047, 9), (2049, 0), (5000, 4096)):
+            a, b = torch.randn(n0, device="cuda") * 300, torch.randn(max(n1, 1), device="cuda")
+            a[0] = float("inf")
+            x, y = (torch.full((n + 8,), 7.0, device="cuda", dtype=dtype) for n in (n0, n1))
+            assert _lib.launch(a, _lib.lib().ss2d_round_pair, a.data_ptr(), x.data_ptr(), n0, b.data_ptr(), y.data_ptr(), n1,
+                               _lib.SS2D_BF16 if dtype == torch.bfloat16 else _lib.SS2D_F16) == _lib.SS2D_OK
+            assert torch.equal(x[:n0], a.to(dtype)) and torch.equal(y[:n1], b[:n1].to(dtype))
+            assert bool((x[n0:] == 7).all()) and bool((y[n1:] == 7).all())

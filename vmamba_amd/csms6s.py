@@ -8,6 +8,8 @@ argument checks are those of selective_scan_fwd / selective_scan_bwd
 with RuntimeError as the reference's TORCH_CHECKs do.  The backward runs on the HIP kernel as well, so the
 operator trains.
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -164,11 +166,11 @@ def selective_scan_bwd(u, delta, A, B, C, D, delta_bias, dout, x=None, delta_sof
     dev = u.device
     du = torch.empty((batch, dim, seqlen), device=dev, dtype=u.dtype)
     ddelta = torch.empty((batch, dim, seqlen), device=dev, dtype=u.dtype)
-    dA = torch.zeros((dim, dstate), device=dev, dtype=torch.float32)
-    dB = torch.zeros((batch, n_groups, dstate, seqlen), device=dev, dtype=torch.float32)
-    dC = torch.zeros((batch, n_groups, dstate, seqlen), device=dev, dtype=torch.float32)
-    dD = torch.zeros((dim,), device=dev, dtype=torch.float32) if D is not None else None
-    dbias = torch.zeros((dim,), device=dev, dtype=torch.float32) if delta_bias is not None else None
+    zeroed = _zeros([(dim, dstate), (batch, n_groups, dstate, seqlen), (batch, n_groups, dstate, seqlen)]
+                    + [(dim,)] * ((D is not None) + (delta_bias is not None)), dev)
+    dA, dB, dC = zeroed[:3]
+    dD = zeroed[3] if D is not None else None
+    dbias = zeroed[-1] if delta_bias is not None else None
 
     p = _lib.ScanBwdParams()
     p.batch, p.dim, p.seqlen, p.dstate, p.n_groups, p.delta_dim = batch, dim, seqlen, dstate, n_groups, delta_dim
@@ -194,7 +196,24 @@ def selective_scan_bwd(u, delta, A, B, C, D, delta_bias, dout, x=None, delta_sof
         ddelta = ddelta.view(batch, delta_dim, dim // delta_dim, seqlen).sum(2)
         if dbias is not None:
             dbias = dbias.view(delta_dim, dim // delta_dim).sum(1)
+    if B.dtype != torch.float32 and dB.numel():
+        dB32, dC32 = dB, dC
+        dB, dC = torch.empty_like(dB32, dtype=B.dtype), torch.empty_like(dC32, dtype=C.dtype)
+        rc = _lib.launch(u, _lib.lib().ss2d_round_pair, dB32.data_ptr(), dB.data_ptr(), dB.numel(), dC32.data_ptr(), dC.data_ptr(),
+                         dC.numel(), _DTYPE_CODE[B.dtype])
+        _lib.check(rc, "ss2d_round_pair")
     return [du, ddelta, dA, dB.to(B.dtype), dC.to(C.dtype), dD, dbias]
+
+
+def _zeros(shapes, device):
+    """fp32 zeros of these shapes, cleared in one launch (ss2d_clear)."""
+    out = [torch.empty(shape, device=device, dtype=torch.float32) for shape in shapes]
+    filled = [t for t in out if t.numel()]
+    if filled:
+        rc = _lib.launch(filled[0], _lib.lib().ss2d_clear, (ctypes.c_void_p * len(filled))(*(t.data_ptr() for t in filled)),
+                         (ctypes.c_int64 * len(filled))(*(4 * t.numel() for t in filled)), len(filled))
+        _lib.check(rc, "ss2d_clear")
+    return out
 
 
 class SelectiveScanHip(torch.autograd.Function):
