@@ -219,6 +219,13 @@ int ss2d_bias_layer_norm(const void *x, const void *pre_bias, const void *weight
                          int C, float eps, int in_dtype, int w_dtype, int out_dtype, void *stream);
 int ss2d_layer_norm_cf(const void *x, const void *weight, const void *bias, void *y, int B, int C, int L, float eps,
                        int in_dtype, int w_dtype, int out_dtype, int out_channel_last, void *stream);
+/*
+ * ss2d_layer_norm_cf of fp32 maps (B,C,H,W) into 16-bit channel-last rows of which only the top-left height x width part of each
+ * map is kept: y (B,height,width,C).  For maps embedded in padded ones.  SS2D_ENOTSUP (use the two steps): maps of up to 1024
+ * positions or no multiple of 4, C no multiple of 8 or beyond 768, other types.
+ */
+int ss2d_layer_norm_cf_crop(const float *x, const void *weight, const void *bias, void *y, int B, int C, int H, int W, int height,
+                            int width, float eps, int w_dtype, int out_dtype, void *stream);
 
 /*
  * Depthwise 3x3 convolution (stride 1, zero padding 1) + optional bias + optional SiLU: the two ops in front of

@@ -14,7 +14,7 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("B,D,H,W", [(1, 768, 7, 7), (3, 192, 14, 14), (2, 96, 28, 28), (5, 48, 9, 8),
                                      (1, 64, 128, 128), (1, 8, 3, 3),
                                      # embedded in larger maps: in LDS, in tiles, a rank without a masked projection, 3 x 5 where padding does not pay
-                                     (2, 96, 19, 19), (3, 64, 25, 42), (1, 32, 123, 125), (1, 800, 9, 9), (2, 16, 3, 5)])
+                                     (2, 96, 19, 19), (3, 64, 25, 42), (1, 96, 57, 58), (1, 192, 33, 35), (1, 384, 34, 33), (1, 768, 33, 33), (1, 32, 123, 125), (1, 800, 9, 9), (2, 16, 3, 5)])
 def test_same_bits(B, D, H, W, dtype, channel_first, monkeypatch):
     print("CASE forward_core", B, D, H, W, dtype, channel_first, flush=True)
     torch.manual_seed(H)

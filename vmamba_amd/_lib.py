@@ -22,7 +22,7 @@ SCAN_KERNEL_NAMES = ("none", "row", "row4", "flat", "small", "chan")
 
 EXPORTS = ("ss2d_abi_version", "ss2d_strerror", "ss2d_cross_scan", "ss2d_cross_merge", "ss2d_selective_scan_fwd",
            "ss2d_selective_scan_kernel", "ss2d_selective_scan_fwd_maps",
-           "ss2d_layer_norm", "ss2d_add_layer_norm", "ss2d_bias_layer_norm", "ss2d_layer_norm_cf", "ss2d_dwconv3x3_silu",
+           "ss2d_layer_norm", "ss2d_add_layer_norm", "ss2d_bias_layer_norm", "ss2d_layer_norm_cf", "ss2d_layer_norm_cf_crop", "ss2d_dwconv3x3_silu",
            "ss2d_dwconv3x3_silu_f32", "ss2d_dwconv3x3_silu_bwd", "ss2d_dwconv3x3_silu_bwd_workspace_bytes", "ss2d_cross_scan_1b1", "ss2d_core_fwd",
            "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_forward_core", "ss2d_forward_core_workspace_bytes", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
            "ss2d_x_proj", "ss2d_x_proj_f32", "ss2d_dt_proj", "ss2d_dt_proj_f32", "ss2d_dt_proj_masked", "ss2d_cross_scan_flex", "ss2d_cross_scan_flex_ws", "ss2d_cross_scan_flex_static", "ss2d_cross_merge_flex",
@@ -127,6 +127,9 @@ def lib():
         L.ss2d_layer_norm_cf.restype = ctypes.c_int
         L.ss2d_layer_norm_cf.argtypes = ([ctypes.c_void_p] * 4 + [ctypes.c_int] * 3 + [ctypes.c_float]
                                          + [ctypes.c_int] * 4 + [ctypes.c_void_p])
+        L.ss2d_layer_norm_cf_crop.restype = ctypes.c_int
+        L.ss2d_layer_norm_cf_crop.argtypes = ([ctypes.c_void_p] * 4 + [ctypes.c_int] * 6 + [ctypes.c_float] + [ctypes.c_int] * 2
+                                              + [ctypes.c_void_p])
         L.ss2d_dwconv3x3_silu.restype = ctypes.c_int
         L.ss2d_dwconv3x3_silu.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 7 + [ctypes.c_void_p]
         L.ss2d_dwconv3x3_silu_f32.restype = ctypes.c_int

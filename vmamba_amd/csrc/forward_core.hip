@@ -83,6 +83,12 @@ extern "C" int ss2d_forward_core(const ss2d_forward_core_params *q, void *worksp
                                                     delta, 4, D, R, p.pitch, ks, p.pitch, q->dtype, stream);
     }
     if (rc == SS2D_OK) rc = ss2d_core_fwd_ws(&p.core, base + p.scratch, p.total - p.scratch, stream);
+    if (rc == SS2D_OK && q->normalise && p.padded && q->out_channel_last) {
+        rc = ss2d_layer_norm_cf_crop((const float *)(base + p.y), q->norm_weight, q->norm_bias, q->out, B, D, H, W, q->height, q->width, q->eps,
+                                     q->norm_dtype, q->dtype, stream);
+        if (rc != SS2D_ENOTSUP) return rc;
+        rc = SS2D_OK;
+    }
     if (rc == SS2D_OK && q->normalise)
         rc = ss2d_layer_norm_cf(base + p.y, q->norm_weight, q->norm_bias, p.padded ? base + p.out : q->out, B, D, (int)L, q->eps, SS2D_F32,
                                 q->norm_dtype, q->dtype, q->out_channel_last, stream);

@@ -382,10 +382,16 @@ __global__ __launch_bounds__(kBlock) void layer_norm_cf_reg_kernel(const in_t *_
 // 4-byte loads of the variant above leave it the bottleneck on short images).  Threads are laid out quads x groups;
 // group g holds channels g, g+kG, ... of its four positions.  Sums cross the groups of a wavefront by lane
 // exchanges and the wavefronts through a few floats of LDS.
-template <typename in_t, typename w_t, typename out_t, bool kOutChannelLast, int kQ, int kG, int kCPL>
+// kCrop (channel-last only): the image is a map of which only the top-left height x width part is wanted; its rows alone are
+// written, as a dense (B, height, width, C).
+struct LnCrop {
+    int32_t height, width;
+    FastDiv by_row;                                  // the whole map's width
+};
+template <typename in_t, typename w_t, typename out_t, bool kOutChannelLast, int kQ, int kG, int kCPL, bool kCrop = false>
 __global__ __launch_bounds__(kBlock) void layer_norm_cf_quad_kernel(const in_t *__restrict__ x, const w_t *__restrict__ weight,
                                                                     const w_t *__restrict__ bias, out_t *__restrict__ y, int C,
-                                                                    int L, int tiles_per_image, int Cp, float eps) {
+                                                                    int L, int tiles_per_image, int Cp, float eps, LnCrop crop) {
     static_assert(kQ * kG == kBlock && kQ <= kWave, "one thread per (position quad, group)");
     constexpr int kTP = 4 * kQ;                      // positions per workgroup
     constexpr int kWaves = kBlock / kWave;
@@ -499,12 +505,19 @@ __global__ __launch_bounds__(kBlock) void layer_norm_cf_quad_kernel(const in_t *
         }
         __syncthreads();
         const int nl = min(kTP, L - l0);
-        out_t *yb = y + ((size_t)b * L + l0) * C;
+        out_t *yb = kCrop ? y + (size_t)b * crop.height * crop.width * C : y + ((size_t)b * L + l0) * C;
         constexpr int kPiece = 16 / (int)sizeof(out_t);            // elements per 16-byte piece; C % kPiece == 0 (host)
         const int pieces = C / kPiece;
         for (int idx = threadIdx.x; idx < nl * pieces; idx += kBlock) {
             const int pp = idx / pieces, cc = (idx - pp * pieces) * kPiece;
-            *reinterpret_cast<uint4 *>(yb + (size_t)pp * C + cc) = *reinterpret_cast<const uint4 *>(ot + pp * Cp + cc);
+            size_t row = (size_t)pp;
+            if constexpr (kCrop) {
+                uint32_t r, c;
+                divmod((uint32_t)(l0 + pp), crop.by_row, r, c);
+                if (r >= (uint32_t)crop.height || c >= (uint32_t)crop.width) continue;
+                row = (size_t)r * crop.width + c;
+            }
+            *reinterpret_cast<uint4 *>(yb + row * C + cc) = *reinterpret_cast<const uint4 *>(ot + pp * Cp + cc);
         }
     }
 }
@@ -813,12 +826,31 @@ static int launch_ln_cf_quad(const void *x, const void *w, const void *b, void *
     if (out_channel_last) {
         const size_t smem = (size_t)kTP * Cp * sizeof(out_t);
         hipLaunchKernelGGL((layer_norm_cf_quad_kernel<in_t, w_t, out_t, true, kQ, kG, kCPL>), dim3((uint32_t)n_wg), dim3(kBlock), smem,
-                           stream, (const in_t *)x, (const w_t *)w, (const w_t *)b, (out_t *)y, C, L, tiles, Cp, eps);
+                           stream, (const in_t *)x, (const w_t *)w, (const w_t *)b, (out_t *)y, C, L, tiles, Cp, eps, LnCrop{});
     } else {
         hipLaunchKernelGGL((layer_norm_cf_quad_kernel<in_t, w_t, out_t, false, kQ, kG, kCPL>), dim3((uint32_t)n_wg), dim3(kBlock), 0,
-                           stream, (const in_t *)x, (const w_t *)w, (const w_t *)b, (out_t *)y, C, L, tiles, Cp, eps);
+                           stream, (const in_t *)x, (const w_t *)w, (const w_t *)b, (out_t *)y, C, L, tiles, Cp, eps, LnCrop{});
     }
     return launch_status();
+}
+
+// fp32 maps normalised into 16-bit channel-last rows, cropped on the way out
+template <typename w_t, typename out_t, int kQ, int kG, int kCPL>
+static int launch_ln_cf_crop(const void *x, const void *w, const void *b, void *y, int B, int C, int L, float eps, const LnCrop &crop,
+                             hipStream_t stream) {
+    constexpr int kTP = 4 * kQ;
+    const int tiles = (L + kTP - 1) / kTP, piece = 16 / (int)sizeof(out_t), Cp = C + piece;
+    hipLaunchKernelGGL((layer_norm_cf_quad_kernel<float, w_t, out_t, true, kQ, kG, kCPL, true>), dim3((uint32_t)((int64_t)B * tiles)),
+                       dim3(kBlock), (size_t)kTP * Cp * sizeof(out_t), stream, (const float *)x, (const w_t *)w, (const w_t *)b,
+                       (out_t *)y, C, L, tiles, Cp, eps, crop);
+    return launch_status();
+}
+template <typename w_t, typename out_t>
+static int ln_cf_crop(const void *x, const void *w, const void *b, void *y, int B, int C, int L, float eps, const LnCrop &crop, hipStream_t s) {
+    if (C <= 96) return launch_ln_cf_crop<w_t, out_t, 16, 16, 6>(x, w, b, y, B, C, L, eps, crop, s);
+    if (C <= 192) return launch_ln_cf_crop<w_t, out_t, 16, 16, 12>(x, w, b, y, B, C, L, eps, crop, s);
+    if (C <= 384) return launch_ln_cf_crop<w_t, out_t, 8, 32, 12>(x, w, b, y, B, C, L, eps, crop, s);
+    return launch_ln_cf_crop<w_t, out_t, 4, 64, 12>(x, w, b, y, B, C, L, eps, crop, s);
 }
 
 // The image variant's split of an image and its launch; false when the shape is not one it covers.
@@ -987,4 +1019,24 @@ extern "C" int ss2d_layer_norm_cf(const void *x, const void *weight, const void 
 #define SS2D_CALL(I, W, O) launch_ln_cf<I, W, O>(x, weight, bias, y, B, C, L, eps, out_channel_last, s)
     SS2D_LN_DISPATCH(SS2D_CALL)
 #undef SS2D_CALL
+}
+
+extern "C" int ss2d_layer_norm_cf_crop(const float *x, const void *weight, const void *bias, void *y, int B, int C, int H, int W,
+                                       int height, int width, float eps, int w_dtype, int out_dtype, void *stream) {
+    using namespace ss2d;
+    if (B < 0 || C < 0 || H < 0 || W < 0 || height < 0 || width < 0 || height > H || width > W) return SS2D_EINVAL;
+    if (!ln_dtype_ok(w_dtype) || !ln_dtype_ok(out_dtype)) return SS2D_EINVAL;
+    if (B == 0 || C == 0 || height == 0 || width == 0) return SS2D_OK;
+    if (!x || !y) return SS2D_EINVAL;
+    const int64_t L = (int64_t)H * W;
+    // where ss2d_layer_norm_cf takes its kernel of position quads: beyond the short images, up to 768 channels.  (57 x 58 maps
+    // embedded in 60 x 60, 48 x 96 of them: the normalisation 24 us and the crop of its result 10; as one 24.)
+    if (L <= 1024 || L % 4 != 0 || C % 8 != 0 || C > 768 || (int64_t)C * L * 4 >= 0x7ffffff0ll || (int64_t)B * ((L + 15) / 16) > 0x7fffffff ||
+        !ln_aligned16(x) || !ln_aligned16(y)) return SS2D_ENOTSUP;
+    const LnCrop crop = {height, width, make_fastdiv((uint32_t)W)};
+    hipStream_t s = (hipStream_t)stream;
+    if (out_dtype == SS2D_BF16 && w_dtype == SS2D_BF16) return ln_cf_crop<bf16_t, bf16_t>(x, weight, bias, y, B, C, (int)L, eps, crop, s);
+    if (out_dtype == SS2D_BF16 && w_dtype == SS2D_F32) return ln_cf_crop<float, bf16_t>(x, weight, bias, y, B, C, (int)L, eps, crop, s);
+    if (out_dtype == SS2D_F16 && w_dtype == SS2D_F16) return ln_cf_crop<f16_t, f16_t>(x, weight, bias, y, B, C, (int)L, eps, crop, s);
+    return SS2D_ENOTSUP;
 }
