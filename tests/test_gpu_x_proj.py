@@ -30,6 +30,9 @@ CASES = [
     (1, 64, 70, 24, 16, None, -1),         # more than 64 output rows
     (1, 96, 8, 256, 200, None, -1),        # large map: tiles in both directions, the last column tile narrower
     (1, 32, 4, 100, 98, None, -1),         # wide map whose width is no multiple of 4: full rows
+    (1, 40, 5, 18, 18, None, -1),          # last tile (9 rows) ends inside a group of four positions, the map does not
+    (2, 48, 26, 66, 66, None, -1),         # the same with two directions a workgroup
+    (24, 64, 12, 58, 58, None, -1),        # five-row tiles, all directions in one workgroup
     (2, 96, 8, 57, 58, (60, 60), 6),       # padded map with a mask row
     (1, 384, 26, 19, 19, (20, 20), -1),    # padded map without one
     (3, 16, 3, 5, 7, (8, 8), 3),           # mask row behind the last row

@@ -119,7 +119,9 @@ __global__ __launch_bounds__(kBlock, kMt == 1 ? 4 : kMt <= 3 ? 3 : 2) void x_pro
 #pragma unroll
             for (int m = 0; m < kMt; ++m) r.a[m] &= keep;
         }
-        if (HW % 4 != 0 && last_h && group == n_groups - 1) {    // uniform
+        // the map's last positions, where the tile does not end on a whole four of them (its size decides that, not the
+        // map's: nine rows of an 18 x 18 map end two positions short).  Uniform.
+        if (n_pos % 4 != 0 && last_h && group == n_groups - 1) {
             const int over = max(0, offset_of(group) - (HW - 4));
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
