@@ -245,6 +245,15 @@ int ss2d_dwconv3x3_silu_f32(const float *x, const float *weight, const float *bi
                             void *stream);
 
 /*
+ * Weight gradient of a projection: dw (N,K) = dy^T x for x (M,K) and dy (M,N), fp32, contiguous, 16-byte aligned; fp32 sums in a
+ * fixed order.  workspace: ss2d_linear_dw_f32_workspace_bytes(...) bytes of device memory, 16-byte aligned.  SS2D_ENOTSUP (from
+ * both): an empty shape, or N or K no multiple of 4.
+ */
+int64_t ss2d_linear_dw_f32_workspace_bytes(int64_t M, int N, int K);
+int ss2d_linear_dw_f32(const float *x, const float *dy, float *dw, int64_t M, int N, int K, void *workspace,
+                       int64_t workspace_bytes, void *stream);
+
+/*
  * Backward of ss2d_dwconv3x3_silu with apply_silu (in training the reference differentiates the two operators,
  * classification/models/vmamba.py:656-658): x, dy, dx (B,D,H,W), weight and dweight (D,1,3,3), bias and dbias (D) or NULL, all
  * of `dtype`, contiguous; sums in fp32 (those of nine products in 64 bits for fp32), rounded once, in a fixed order.  The convolution is

@@ -1,10 +1,12 @@
 """Narrow channel-last projection on the HIP kernel ss2d_linear_cl: out = [LayerNorm](x) W^T + bias + residual.
 
 Stands in, in a channel-last VSS block of width 96, for norm + in_proj and for out_proj + the residual add
-(classification/models/vmamba.py:1225-1228, :648-650, :662) at inference in bf16 / fp16; other widths, fp32 and
-training stay on the PyTorch-ROCm operators.
+(classification/models/vmamba.py:1225-1228, :648-650, :662) at inference in bf16 / fp16; other widths and fp32
+stay on the PyTorch-ROCm operators.  In single-precision training the weight gradient of these projections is a HIP kernel
+(ss2d_linear_dw_f32) where that is the faster one.
 """
 import torch
+import torch.nn as nn
 
 from . import _lib
 
@@ -72,3 +74,56 @@ def linear_cf_ln_hip(y, ln_weight, ln_bias, eps, weight, bias=None, residual=Non
                      keep[0].data_ptr(), ptr(small[2]), ptr(keep[1]), out.data_ptr(), B, L, K, N, _DTYPE_CODE[dt])
     _lib.check(rc, "ss2d_linear_cf_ln")
     return out
+
+
+def linear_dw_hip(x, dy):
+    """dy^T x for x (M, K) and dy (M, N), float32, contiguous: the weight gradient of a projection (ss2d_linear_dw_f32)."""
+    if not (x.is_cuda and dy.device == x.device and x.dtype == dy.dtype == torch.float32 and x.dim() == dy.dim() == 2
+            and x.shape[0] == dy.shape[0]):
+        raise ValueError("linear_dw_hip expects float32 x (M, K) and dy (M, N) on one GPU")
+    x, dy = x.contiguous(), dy.contiguous()
+    (M, K), N = x.shape, dy.shape[1]
+    need = _lib.lib().ss2d_linear_dw_f32_workspace_bytes(M, N, K)
+    _lib.check(min(need, 0), "ss2d_linear_dw_f32_workspace_bytes")
+    workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+    dw = torch.empty((N, K), device=x.device, dtype=x.dtype)
+    rc = _lib.launch(x, _lib.lib().ss2d_linear_dw_f32, x.data_ptr(), dy.data_ptr(), dw.data_ptr(), M, N, K, workspace.data_ptr(), need)
+    _lib.check(rc, "ss2d_linear_dw_f32")
+    return dw
+
+
+def linear_dw_pays(layer, x):
+    """True when LinearDw stands for ``layer(x)`` in training: a plain nn.Linear without bias, hooks or autocast, on float32
+    positions many enough and with outputs few enough that the library leaves most of the chip idle.  12 544 positions, library
+    against kernel in us: 384 x 384 outputs 77 against 54; 576 x 576 104 against 106.  96 x 96 over 200 704: 443 against 141;
+    384 x 384 over 3136: 25 against 28."""
+    if not (type(layer) is nn.Linear and layer.bias is None and x.is_cuda and x.dim() >= 2 and x.dtype == torch.float32):
+        return False
+    weight = layer.weight
+    hooks = (layer._forward_hooks, layer._forward_pre_hooks, layer._backward_hooks, layer._backward_pre_hooks)
+    N, K = weight.shape
+    return (torch.is_grad_enabled() and weight.requires_grad and weight.dtype == x.dtype and weight.device == x.device
+            and x.shape[-1] == K and N % 4 == 0 and K % 4 == 0 and 0 < N * K <= 384 * 384 and x.numel() >= 4096 * K
+            and not any(hooks) and not nn.modules.module._has_any_global_hook() and not torch.is_autocast_enabled())
+
+
+class LinearDw(torch.autograd.Function):
+    """x W^T, plus ``residual`` if one is given, with dW = dy^T x on ss2d_linear_dw_f32."""
+
+    @staticmethod
+    def forward(ctx, x, weight, residual):
+        ctx.save_for_backward(x, weight)
+        if residual is None:
+            return nn.functional.linear(x, weight)
+        return torch.addmm(residual.reshape(-1, weight.shape[0]), x.reshape(-1, weight.shape[1]), weight.t()).view(residual.shape)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        N, K = weight.shape
+        dy2, x2 = dy.reshape(-1, N), x.reshape(-1, K)
+        dx = torch.mm(dy2, weight).view(x.shape) if ctx.needs_input_grad[0] else None
+        dw = None
+        if ctx.needs_input_grad[1]:              # the kernel has no gradient of its own: a second backward goes the library's way
+            dw = torch.mm(dy2.t(), x2) if torch.is_grad_enabled() else linear_dw_hip(x2, dy2)
+        return dx, dw, dy if ctx.needs_input_grad[2] else None

@@ -26,7 +26,7 @@ from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_fits, core_mask_
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
 from .conv import DwConv3x3SiLU, dwconv3x3_silu_hip, dwconv_silu_trainable
-from .linear import linear_cf_ln_fusable, linear_cf_ln_hip, linear_cl_hip, linear_fusable
+from .linear import LinearDw, linear_cf_ln_fusable, linear_cf_ln_hip, linear_cl_hip, linear_dw_pays, linear_fusable
 from .norm import (LayerNorm, LayerNorm2d, add_layer_norm_fusable, add_layer_norm_hip, layer_norm_cf_hip,
                    needs_grad)
 
@@ -401,7 +401,8 @@ class SS2D(nn.Module):
                 and self._narrow(x, self.in_proj, pre_norm.weight, pre_norm.bias)):
             x = linear_cl_hip(x, self.in_proj.weight, self.in_proj.bias, None, pre_norm.weight, pre_norm.bias, pre_norm.eps)
         else:
-            x = self.in_proj(x if pre_norm is None else pre_norm(x))
+            x = x if pre_norm is None else pre_norm(x)
+            x = LinearDw.apply(x, self.in_proj.weight, None) if self.layers is HipLayers and linear_dw_pays(self.in_proj, x) else self.in_proj(x)
         z = None
         if not self.disable_z:
             x, z = x.chunk(2, dim=(1 if self.channel_first else -1))
@@ -426,6 +427,9 @@ class SS2D(nn.Module):
             y = y * z
         if self._narrow(y, self.out_proj, residual):
             return linear_cl_hip(y, self.out_proj.weight, self.out_proj.bias, residual)
+        trains = self.layers is HipLayers and linear_dw_pays(self.out_proj, y) and (residual is None or residual.dtype == y.dtype)
+        if trains:
+            return LinearDw.apply(y, self.out_proj.weight, residual)
         if residual is None:
             return self.out_proj(y)
         if self.channel_first or self.out_proj.bias is not None:
