@@ -33,6 +33,8 @@ CASES = [
     (1, 40, 5, 18, 18, None, -1),          # last tile (9 rows) ends inside a group of four positions, the map does not
     (2, 48, 26, 66, 66, None, -1),         # the same with two directions a workgroup
     (24, 64, 12, 58, 58, None, -1),        # five-row tiles, all directions in one workgroup
+    (1, 40, 3, 65, 1, None, -1),           # one column: the tile before the last ends inside the map's last four positions
+    (1, 32, 8, 137, 1, None, -1),
     (2, 96, 8, 57, 58, (60, 60), 6),       # padded map with a mask row
     (1, 384, 26, 19, 19, (20, 20), -1),    # padded map without one
     (3, 16, 3, 5, 7, (8, 8), 3),           # mask row behind the last row

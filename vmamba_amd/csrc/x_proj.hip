@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kBlock, kMt == 1 ? 4 : kMt <= 3 ? 3 : 2) void x_pro
         return (h0 + r) * p.Wd + w0 + c;
     };
     auto load = [&](int group, int step, Step &r) {
-        const int off = min(offset_of(group), HW - 4);           // the last positions of a map: shifted into place below
+        const int off = min(offset_of(group), HW - 4);           // inside the map: shifted into place below
         const int d0 = step * 32 + 8 * kg;
         const bool in = d0 < p.D;                                // (D is a multiple of 8)
         const uint32_t at_d = (uint32_t)((in ? d0 : 0) * HW + off);      // (D * HW elements fit 31 bits)
@@ -120,8 +120,9 @@ __global__ __launch_bounds__(kBlock, kMt == 1 ? 4 : kMt <= 3 ? 3 : 2) void x_pro
             for (int m = 0; m < kMt; ++m) r.a[m] &= keep;
         }
         // the map's last positions, where the tile does not end on a whole four of them (its size decides that, not the
-        // map's: nine rows of an 18 x 18 map end two positions short).  Uniform.
-        if (n_pos % 4 != 0 && last_h && group == n_groups - 1) {
+        // map's: nine rows of an 18 x 18 map end two positions short).  Not the last tile alone: on a map one position wide
+        // the tile before it ends inside the map's last four positions as well.  Uniform.
+        if (n_pos % 4 != 0 && group == n_groups - 1) {
             const int over = max(0, offset_of(group) - (HW - 4));
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
