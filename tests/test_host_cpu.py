@@ -1,5 +1,6 @@
 """CPU checks of the host-side model code (no kernels run): shapes, parameter inventory and the
 projection identity the SS2D core relies on."""
+import pytest
 import torch
 
 from oracle.ss2d_core_ref import RefSS2D
@@ -156,3 +157,30 @@ def test_with_layout_keeps_keys_values_and_mode():
     assert shared.classifier.head.weight is m.classifier.head.weight
     m.double()
     assert next(shared.parameters()).dtype == torch.float64
+
+
+class _OnGpu:
+    """A CPU tensor that says it lies on cuda:0: what the wrappers ask before any launch, without a GPU."""
+    is_cuda, device = True, torch.device("cuda:0")
+
+    def __init__(self, tensor):
+        self._t = tensor
+
+    def __getattr__(self, name):
+        return getattr(self._t, name)
+
+    def get_device(self):
+        return 0
+
+
+def test_x_proj_wants_its_tensors_on_one_device(monkeypatch):
+    """A weight or a result that lies elsewhere is no operand of a kernel: the dispatch rule says no, the wrapper raises."""
+    from vmamba_amd import _lib
+    from vmamba_amd.core import x_proj_f32_fits, x_proj_f32_hip, x_proj_fits, x_proj_hip
+    monkeypatch.setattr(_lib, "launch", lambda *a: (_ for _ in ()).throw(AssertionError("launched")))
+    for dtype, fits, run in ((torch.bfloat16, x_proj_fits, x_proj_hip), (torch.float32, x_proj_f32_fits, x_proj_f32_hip)):
+        x, weight, out = torch.zeros(1, 16, 4, 4, dtype=dtype), torch.zeros(4, 3, 16, dtype=dtype), torch.zeros(1, 4, 3, 16, dtype=dtype)
+        assert not fits(_OnGpu(x), weight) and fits(_OnGpu(x), _OnGpu(weight))
+        for w, o in ((weight, _OnGpu(out)), (_OnGpu(weight), out)):
+            with pytest.raises(RuntimeError):
+                run(_OnGpu(x), w, o)

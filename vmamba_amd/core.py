@@ -215,8 +215,8 @@ X_PROJ_MAX_ROWS = 96
 
 def x_proj_fits(x, weight):
     """True when ss2d_x_proj takes this map (B, D, H, W) and these weights (4, C, D)."""
-    return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype and x.shape[1] % 8 == 0
-            and x.shape[1] > 0 and weight.shape[1] <= X_PROJ_MAX_ROWS and x.shape[2] * x.shape[3] >= 8
+    return (x.is_cuda and weight.device == x.device and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype
+            and x.shape[1] % 8 == 0 and x.shape[1] > 0 and weight.shape[1] <= X_PROJ_MAX_ROWS and x.shape[2] * x.shape[3] >= 8
             and x.shape[1] * x.shape[2] * x.shape[3] < 2 ** 31 and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
 
 
@@ -227,6 +227,7 @@ def x_proj_hip(x, weight, out, padded=None, mask_row=-1):
     _check(x.is_cuda and x.dim() == 4 and weight.dim() == 3 and weight.shape[0] == 4 and weight.shape[2] == x.shape[1],
            "x_proj expects x (B, D, H, W) and weight (4, C, D)")
     _check(x.dtype == weight.dtype == out.dtype and x.dtype in _DTYPE_CODE, "x_proj: one 16-bit dtype")
+    _check(weight.device == out.device == x.device, "x_proj: tensors on one device")
     B, D, H, W = x.shape
     Hp, Wp = padded or (H, W)
     C = weight.shape[1]
