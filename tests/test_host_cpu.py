@@ -184,3 +184,21 @@ def test_x_proj_wants_its_tensors_on_one_device(monkeypatch):
         for w, o in ((weight, _OnGpu(out)), (_OnGpu(weight), out)):
             with pytest.raises(RuntimeError):
                 run(_OnGpu(x), w, o)
+
+
+def test_convolution_function_and_single_call_core_have_no_cpu_path(monkeypatch):
+    """Neither may hand a host address to a kernel, whichever of its tensors lies on the CPU."""
+    from vmamba_amd import _lib
+    from vmamba_amd.conv import DwConv3x3SiLU
+    from vmamba_amd.core import forward_core_hip
+    monkeypatch.setattr(_lib, "launch", lambda *a: (_ for _ in ()).throw(AssertionError("launched")))
+    x, weight = torch.zeros(1, 16, 4, 4), torch.zeros(16, 1, 3, 3)
+    with pytest.raises(NotImplementedError):
+        DwConv3x3SiLU.apply(x, weight, None, False)
+    ctx = torch.autograd.function.FunctionCtx()
+    for w, b, error in ((weight, None, TypeError), (_OnGpu(weight.half()), None, TypeError), (_OnGpu(weight), weight[:, 0, 0, 0], TypeError),
+                        (_OnGpu(weight[:8]), None, ValueError)):
+        with pytest.raises(error):
+            DwConv3x3SiLU.forward(ctx, _OnGpu(x), w, b, False)
+    with pytest.raises(RuntimeError):
+        forward_core_hip(x, torch.zeros(4, 3, 16), torch.zeros(4, 16, 1), *(torch.zeros(64) for _ in range(3)))

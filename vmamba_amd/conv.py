@@ -69,6 +69,13 @@ class DwConv3x3SiLU(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, bias, channel_last):
+        if not x.is_cuda:
+            raise NotImplementedError("DwConv3x3SiLU: vmamba_amd runs on the GPU only")
+        D = x.shape[3 if channel_last else 1]
+        if tuple(weight.shape) != (D, 1, 3, 3) or (bias is not None and tuple(bias.shape) != (D,)):
+            raise ValueError("DwConv3x3SiLU: expected weight (D,1,3,3) and bias (D)")
+        if x.dtype not in _DTYPE_CODE or any(t is not None and (t.dtype != x.dtype or t.device != x.device) for t in (weight, bias)):
+            raise TypeError("DwConv3x3SiLU: one floating dtype and one device")
         ctx.channel_last = channel_last
         x = x.contiguous()
         if channel_last:

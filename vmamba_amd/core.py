@@ -157,6 +157,7 @@ def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=Non
     (B,H,W,D) if ``out_channel_last`` else (B,D,H,W) in x.dtype, the merged map (B,D,L) in fp32 without ``norm``, or None
     where the kernels have no variant for the call and the separate ones have to be tried.  Maps that padded_map_size embeds in
     larger ones need pad_mask(H, W, padded H, padded W, B, device): the mask dt_proj_hip takes."""
+    _check(x.is_cuda, "forward_core: vmamba_amd runs on the GPU only")
     B, D, H, W = x.shape
     R = dt_proj_weight.shape[2]
     code = _DTYPE_CODE.get(x.dtype)
