@@ -53,6 +53,26 @@ def test_linear_dw_autograd(with_residual):
     assert torch.autograd.grad(dw.sum(), x)[0].shape == x.shape
 
 
+def test_linear_dw_of_views_between_16_byte_boundaries():
+    """x and dy as contiguous views one element into their storage, as slices and the backward of a concatenation give them:
+    the gradients are the layer's own (4096 products of unit size: M * 2^-24 of their magnitudes' sum)."""
+    print("CASE linear_dw unaligned", flush=True)
+    torch.manual_seed(1)
+    layer = nn.Linear(48, 64, bias=False).to(DEV)
+    aligned = [torch.randn(4096, n, device=DEV) for n in (48, 64)]
+    shifted = []
+    for t in aligned:
+        shifted.append(torch.empty(t.numel() + 1, device=DEV)[1:].view(t.shape).copy_(t))
+        assert shifted[-1].is_contiguous() and shifted[-1].data_ptr() % 16 == 4
+    want, size = aligned[1].double().t() @ aligned[0].double(), aligned[1].double().abs().t() @ aligned[0].double().abs()
+    for x, dy in ((shifted[0], aligned[1]), (aligned[0], shifted[1]), shifted):
+        x = x.detach().requires_grad_()
+        assert linear_dw_pays(layer, x)
+        dx, dw = torch.autograd.grad(LinearDw.apply(x, layer.weight, None), [x, layer.weight], dy)
+        assert bool(((dw.double() - want).abs() <= 4096 * 2.0 ** -24 * size).all())
+        assert torch.equal(dx, torch.autograd.grad(layer(x), x, dy)[0])
+
+
 def test_linear_dw_rule():
     layer, x = nn.Linear(48, 64, bias=False).to(DEV), torch.zeros(4096, 48, device=DEV)
     assert linear_dw_pays(layer, x) and not linear_dw_pays(layer, x[:4095]) and not linear_dw_pays(layer, x.half())

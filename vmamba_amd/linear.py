@@ -124,6 +124,10 @@ class LinearDw(torch.autograd.Function):
         dy2, x2 = dy.reshape(-1, N), x.reshape(-1, K)
         dx = torch.mm(dy2, weight).view(x.shape) if ctx.needs_input_grad[0] else None
         dw = None
-        if ctx.needs_input_grad[1]:              # the kernel has no gradient of its own: a second backward goes the library's way
-            dw = torch.mm(dy2.t(), x2) if torch.is_grad_enabled() else linear_dw_hip(x2, dy2)
+        if ctx.needs_input_grad[1]:
+            # the library's product where the kernel does not stand for it: under a second backward (it has no gradient of its
+            # own), and for views that start between 16-byte boundaries, which contiguous() leaves where they are
+            x2, dy2 = x2.contiguous(), dy2.contiguous()
+            kernel = not torch.is_grad_enabled() and (x2.data_ptr() | dy2.data_ptr()) % 16 == 0
+            dw = linear_dw_hip(x2, dy2) if kernel else torch.mm(dy2.t(), x2)
         return dx, dw, dy if ctx.needs_input_grad[2] else None
