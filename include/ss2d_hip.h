@@ -293,6 +293,13 @@ int ss2d_x_proj(const void *x, const void *weight, void *out, int B, int D, int 
                 int64_t out_dir_stride, int64_t out_chan_stride, int64_t out_batch_stride, int dtype, void *stream);
 
 /*
+ * SS2D_OK where ss2d_x_proj takes an unpadded problem of these sizes, SS2D_ENOTSUP where the caller's own product has to: the
+ * conditions above, and rows too wide for LDS (a width that is no multiple of 4 is not cut: from about 700 columns at C = 96,
+ * 1500 at C = 40 and 3600 at C = 16 on).
+ */
+int ss2d_x_proj_applies(int B, int D, int C, int H, int W, int dtype);
+
+/*
  * The same projection in single precision (fp32 operands and sums), any D > 0 and C; the map as it is
  * (no padding, no mask row).
  */

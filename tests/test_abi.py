@@ -177,3 +177,17 @@ def test_torch_extension_shim_loads_and_validates_on_cpu():
     z = torch.zeros(1, 4, 8)
     with pytest.raises(RuntimeError):       # CPU tensors are refused before anything touches a GPU
         ext.fwd(z, z, torch.zeros(4, 1), torch.zeros(1, 4, 1, 8), torch.zeros(1, 4, 1, 8), None, None, True, 1, True)
+
+
+def test_x_proj_says_what_it_takes():
+    """The conditions of ss2d_x_proj from the sizes alone, and that the call itself refuses the same before any launch."""
+    L = _lib.lib()
+    applies = lambda B, D, C, H, W, dtype=_lib.SS2D_BF16: L.ss2d_x_proj_applies(B, D, C, H, W, dtype)
+    taken = [(1, 96, 8, 56, 56), (2, 768, 50, 7, 7), (0, 96, 8, 56, 56), (4, 96, 38, 64, 2000), (64, 96, 8, 64, 2001), (1, 8, 96, 1, 8)]
+    refused = [(1, 12, 8, 56, 56), (1, 96, 97, 56, 56), (1, 96, 8, 1, 7), (1, 96, 38, 64, 2001), (1, 768, 80, 32, 1001), (1, 1 << 20, 8, 64, 64)]
+    assert all(applies(*c) == _lib.SS2D_OK for c in taken)
+    for c in refused:
+        assert applies(*c) == _lib.SS2D_ENOTSUP, c
+        B, D, C, H, W = c
+        assert L.ss2d_x_proj(256, 256, 256, B, D, C, H, W, H, W, -1, C * H * W, H * W, 4 * C * H * W, _lib.SS2D_BF16, None) == _lib.SS2D_ENOTSUP
+    assert applies(1, 96, 8, 56, 56, _lib.SS2D_F32) == _lib.SS2D_ENOTSUP and applies(-1, 96, 8, 56, 56) == _lib.SS2D_EINVAL

@@ -126,6 +126,23 @@ def test_forward_core_on_maps_embedded_in_padded_ones(d_model, B, H, W, channel_
     assert torch.allclose(got.float(), ops.float(), rtol=tol / 2, atol=tol / 2)
 
 
+@pytest.mark.parametrize("d_model,d_state,H,W", [(16, 16, 3, 2001), (512, 1, 1, 2001)])
+def test_forward_core_of_rows_too_wide_for_x_proj(d_model, d_state, H, W):
+    """Rows of a width that is no multiple of 4 and beyond what ss2d_x_proj keeps in LDS: the library's projection, with several
+    states and with one, through the fused core and the three operators (the bf16 bound of the tests above)."""
+    from vmamba_amd.core import x_proj_fits
+    print("CASE core-wide", d_model, d_state, H, W, flush=True)
+    ref, hip = _pair(d_model, d_state)
+    ref, hip = ref.bfloat16(), hip.bfloat16()
+    x = torch.randn(1, d_model, H, W, generator=torch.Generator().manual_seed(8)).bfloat16()
+    assert not x_proj_fits(x.to(DEV), hip.x_proj_weight)
+    with torch.no_grad():
+        want = ref.float().forward_core(x.float())
+        for fused in (True, False):
+            hip.fused_core = fused
+            assert torch.allclose(hip.forward_core(x.to(DEV)).float().cpu(), want, rtol=2e-2, atol=2e-2), f"fused={fused}"
+
+
 def test_block_with_gate_matches():
     print("CASE block-z", flush=True)
     ref, hip = _pair(24, 16, 2.0, disable_z=False)

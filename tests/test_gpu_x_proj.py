@@ -35,6 +35,7 @@ CASES = [
     (24, 64, 12, 58, 58, None, -1),        # five-row tiles, all directions in one workgroup
     (1, 40, 3, 65, 1, None, -1),           # one column: the tile before the last ends inside the map's last four positions
     (1, 32, 8, 137, 1, None, -1),
+    (1, 8, 8, 256, 1931, None, -1),        # a row that fits LDS with two directions, not with four
     (2, 96, 8, 57, 58, (60, 60), 6),       # padded map with a mask row
     (1, 384, 26, 19, 19, (20, 20), -1),    # padded map without one
     (3, 16, 3, 5, 7, (8, 8), 3),           # mask row behind the last row

@@ -211,14 +211,11 @@ def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=Non
     return out
 
 
-X_PROJ_MAX_ROWS = 96
-
-
 def x_proj_fits(x, weight):
     """True when ss2d_x_proj takes this map (B, D, H, W) and these weights (4, C, D)."""
     return (x.is_cuda and weight.device == x.device and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype
-            and x.shape[1] % 8 == 0 and x.shape[1] > 0 and weight.shape[1] <= X_PROJ_MAX_ROWS and x.shape[2] * x.shape[3] >= 8
-            and x.shape[1] * x.shape[2] * x.shape[3] < 2 ** 31 and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+            and _lib.lib().ss2d_x_proj_applies(x.shape[0], x.shape[1], weight.shape[1], x.shape[2], x.shape[3], _DTYPE_CODE[x.dtype]) == _lib.SS2D_OK)
 
 
 def x_proj_hip(x, weight, out, padded=None, mask_row=-1):

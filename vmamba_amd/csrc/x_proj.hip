@@ -319,26 +319,12 @@ static int launch_x_proj(const XProjArgs &a, size_t smem, int m_tiles, hipStream
 
 static int64_t xp_gcd(int64_t a, int64_t b) { while (b) { const int64_t t = a % b; a = b; b = t; } return a < 0 ? -a : a; }
 
-}  // namespace ss2d
-
-extern "C" int ss2d_x_proj(const void *x, const void *weight, void *out, int B, int D, int C, int H, int W, int Hp, int Wp,
-                           int mask_row, int64_t out_dir_stride, int64_t out_chan_stride, int64_t out_batch_stride, int dtype,
-                           void *stream) {
-    using namespace ss2d;
-    if (B < 0 || D < 0 || C < 0 || H < 0 || W < 0 || Hp < H || Wp < W || mask_row > C) return SS2D_EINVAL;
-    if (dtype != SS2D_F32 && dtype != SS2D_BF16 && dtype != SS2D_F16) return SS2D_EINVAL;
-    if (out_dir_stride < 0 || out_chan_stride < 0 || out_batch_stride < 0) return SS2D_EINVAL;
-    if (B == 0 || C == 0 || H == 0 || W == 0) return SS2D_OK;
-    if (!x || !weight || !out) return SS2D_EINVAL;
+// How a problem is cut: everything but the pointers, the output's strides and the stores' width.  SS2D_ENOTSUP: no variant.
+static int x_proj_plan(int B, int D, int C, int H, int W, int Hp, int Wp, int dtype, XProjArgs &a, int &m_tiles, size_t &smem) {
     const int64_t HW = (int64_t)H * W, L = (int64_t)Hp * Wp;
     // 8 channels of a weight row are one 16-byte load; at most 96 output rows (six accumulator tiles)
-    if (dtype == SS2D_F32 || D == 0 || D % 8 != 0 || C > 96 || HW < 8 || L > 0x0fffffff || (int64_t)D * HW > 0x7fffffff ||
-        reinterpret_cast<uintptr_t>(weight) % 16 != 0) return SS2D_ENOTSUP;
-    XProjArgs a;
-    a.x = x; a.W = weight; a.out = out;
+    if (dtype == SS2D_F32 || D == 0 || D % 8 != 0 || C > 96 || HW < 8 || L > 0x0fffffff || (int64_t)D * HW > 0x7fffffff) return SS2D_ENOTSUP;
     a.D = D; a.C = C; a.H = H; a.Wd = W; a.Hp = Hp; a.Wp = Wp;
-    a.mask_row = mask_row < 0 ? -1 : mask_row;
-    a.ks = out_dir_stride; a.cs = out_chan_stride; a.bs = out_batch_stride;
     a.Ce = (C + 1) & ~1;
     // Directions per workgroup: each set reads the map again, from L2, and that re-reading is what bounds the kernel (loads
     // alone, one direction per workgroup: 30 of 37 us at 96 x 56 x 56, batch 128).  As many as four accumulator tiles hold,
@@ -358,6 +344,7 @@ extern "C" int ss2d_x_proj(const void *x, const void *weight, void *out, int B, 
         t = ((H + n - 1) / n + unit - 1) / unit * unit;
         return t > H ? (int64_t)H : t;
     };
+    constexpr int64_t kMostLds = 128 * 1024;
     int64_t Th = 1, row_bytes = 0, total = 0;
     for (;; a.n_dirs /= 2) {
         const int rows = a.n_dirs * a.Ce;
@@ -370,27 +357,61 @@ extern "C" int ss2d_x_proj(const void *x, const void *weight, void *out, int B, 
         auto grid = [&](int64_t t) { return (int64_t)B * (4 / a.n_dirs) * a.tiles_w * ((H + t - 1) / t); };
         while (Th > 16 && grid(Th) < 512) Th = even((Th + 1) / 2);
         total = grid(Th);
-        if (a.n_dirs == 1 || total >= 256) break;
+        if (a.n_dirs == 1 || (total >= 256 && row_bytes * Th <= kMostLds)) break;
     }
-    if (total > 0x7fffffff) return SS2D_ENOTSUP;
+    // a row of a width that is no multiple of 4 is not cut: there is a widest one
+    if (total > 0x7fffffff || row_bytes * Th > kMostLds || Th * a.Tw * a.pitch > (1 << 22)) return SS2D_ENOTSUP;
     a.total = (uint32_t)total;
     a.Th = (int)Th;
     a.tiles_h = (int)((H + Th - 1) / Th);
-    if (row_bytes * Th > 128 * 1024 || Th * a.Tw * a.pitch > (1 << 22)) return SS2D_ENOTSUP;
     const int64_t n_groups = (Th * a.Tw + kXpGroup - 1) / kXpGroup;
     // maps of one or two column groups: the wavefronts split the channels
     const int n_waves = kBlock / kWave;
     a.k_split = 1;
     while (a.k_split * 2 * n_groups <= n_waves && a.k_split * 2 <= a.k_steps) a.k_split *= 2;
     const int rows = a.n_dirs * a.Ce;
-    const int m_tiles = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 48 ? 3 : rows <= 64 ? 4 : 6;
-    size_t smem = ((size_t)row_bytes * Th + 15) & ~(size_t)15;
+    m_tiles = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 48 ? 3 : rows <= 64 ? 4 : 6;
+    smem = ((size_t)row_bytes * Th + 15) & ~(size_t)15;
     if (a.k_split > 1) smem += (size_t)(n_waves / 2) * m_tiles * 4 * kWave * sizeof(floatx4_t);
+    return SS2D_OK;
+}
+
+}  // namespace ss2d
+
+extern "C" int ss2d_x_proj_applies(int B, int D, int C, int H, int W, int dtype) {
+    using namespace ss2d;
+    if (B < 0 || D < 0 || C < 0 || H < 0 || W < 0 || (dtype != SS2D_F32 && dtype != SS2D_BF16 && dtype != SS2D_F16)) return SS2D_EINVAL;
+    if (B == 0 || C == 0 || H == 0 || W == 0) return SS2D_OK;
+    XProjArgs a;
+    int m_tiles;
+    size_t smem;
+    return x_proj_plan(B, D, C, H, W, H, W, dtype, a, m_tiles, smem);
+}
+
+extern "C" int ss2d_x_proj(const void *x, const void *weight, void *out, int B, int D, int C, int H, int W, int Hp, int Wp,
+                           int mask_row, int64_t out_dir_stride, int64_t out_chan_stride, int64_t out_batch_stride, int dtype,
+                           void *stream) {
+    using namespace ss2d;
+    if (B < 0 || D < 0 || C < 0 || H < 0 || W < 0 || Hp < H || Wp < W || mask_row > C) return SS2D_EINVAL;
+    if (dtype != SS2D_F32 && dtype != SS2D_BF16 && dtype != SS2D_F16) return SS2D_EINVAL;
+    if (out_dir_stride < 0 || out_chan_stride < 0 || out_batch_stride < 0) return SS2D_EINVAL;
+    if (B == 0 || C == 0 || H == 0 || W == 0) return SS2D_OK;
+    if (!x || !weight || !out) return SS2D_EINVAL;
+    XProjArgs a;
+    int m_tiles;
+    size_t smem;
+    const int rc = x_proj_plan(B, D, C, H, W, Hp, Wp, dtype, a, m_tiles, smem);
+    if (rc != SS2D_OK) return rc;
+    if (reinterpret_cast<uintptr_t>(weight) % 16 != 0) return SS2D_ENOTSUP;
+    a.x = x; a.W = weight; a.out = out;
+    a.mask_row = mask_row < 0 ? -1 : mask_row;
+    a.ks = out_dir_stride; a.cs = out_chan_stride; a.bs = out_batch_stride;
     // elements per store: what divides every row base, the scan's length and the starts of the tiles' lines
+    const int64_t L = (int64_t)Hp * Wp;
     int64_t g = xp_gcd(xp_gcd(8, a.ks), xp_gcd(a.cs, a.bs));
     g = xp_gcd(g, xp_gcd(L, (int64_t)(reinterpret_cast<uintptr_t>(out) % 16 / 2)));
     if (reinterpret_cast<uintptr_t>(out) % 2 != 0) return SS2D_EINVAL;
-    const int64_t row_start = a.tiles_w == 1 ? Th * Wp : xp_gcd(Wp, a.Tw), col_start = a.tiles_h == 1 ? (int64_t)a.Tw * Hp : xp_gcd(Hp, Th);
+    const int64_t row_start = a.tiles_w == 1 ? (int64_t)a.Th * Wp : xp_gcd(Wp, a.Tw), col_start = a.tiles_h == 1 ? (int64_t)a.Tw * Hp : xp_gcd(Hp, a.Th);
     const int64_t vr = xp_gcd(g, row_start), vc = xp_gcd(g, col_start);
     a.v_row = (int)(vr == 2 ? 1 : vr);
     a.v_col = (int)(vc == 2 ? 1 : vc);
