@@ -287,7 +287,7 @@ int ss2d_cross_scan_1b1(const void *x, void *y, int B, int C, int H, int W, int 
  *   whose added positions project to 0.
  * mask_row in [0, C] inserts a row at that index (the rows from there on move up by one) that is 1 at the added positions
  * and 0 elsewhere; -1: none.  Returns SS2D_ENOTSUP for fp32, D not a multiple of 8, C > 96, maps of fewer than 8 positions or
- * more than 2^31 elements per image.
+ * more than 2^31 elements per image, and where the added positions behind the last tile are millions.
  */
 int ss2d_x_proj(const void *x, const void *weight, void *out, int B, int D, int C, int H, int W, int Hp, int Wp, int mask_row,
                 int64_t out_dir_stride, int64_t out_chan_stride, int64_t out_batch_stride, int dtype, void *stream);

@@ -191,3 +191,12 @@ def test_x_proj_says_what_it_takes():
         B, D, C, H, W = c
         assert L.ss2d_x_proj(256, 256, 256, B, D, C, H, W, H, W, -1, C * H * W, H * W, 4 * C * H * W, _lib.SS2D_BF16, None) == _lib.SS2D_ENOTSUP
     assert applies(1, 96, 8, 56, 56, _lib.SS2D_F32) == _lib.SS2D_ENOTSUP and applies(-1, 96, 8, 56, 56) == _lib.SS2D_EINVAL
+
+
+def test_x_proj_bounds_the_padded_tail():
+    """The last tile writes the added positions behind it, and its index arithmetic is exact below 2^23 items only: a map padded
+    far beyond its size is refused before any launch."""
+    call = lambda C, H, W, Hp, Wp: _lib.lib().ss2d_x_proj(256, 256, 256, 1, 8, C, H, W, Hp, Wp, -1, C * Hp * Wp, Hp * Wp,
+                                                          4 * C * Hp * Wp, _lib.SS2D_BF16, None)
+    for args in ((1, 4, 4, 4096, 4096), (8, 8, 8, 8, 1 << 18), (96, 8, 8, 1 << 18, 8)):
+        assert call(*args) == _lib.SS2D_ENOTSUP, args

@@ -364,6 +364,9 @@ static int x_proj_plan(int B, int D, int C, int H, int W, int Hp, int Wp, int dt
     a.total = (uint32_t)total;
     a.Th = (int)Th;
     a.tiles_h = (int)((H + Th - 1) / Th);
+    // small_divmod's range: the largest tile on the way out, with the added rows and columns that the last one carries
+    const int64_t tail_h = Hp - (int64_t)(a.tiles_h - 1) * Th, tail_w = Wp - (int64_t)(a.tiles_w - 1) * a.Tw;
+    if ((tail_h > Th ? tail_h : Th) * (tail_w > a.Tw ? tail_w : a.Tw) * ((a.Ce / 2 + 3) & ~3) >= 1 << 23) return SS2D_ENOTSUP;
     const int64_t n_groups = (Th * a.Tw + kXpGroup - 1) / kXpGroup;
     // maps of one or two column groups: the wavefronts split the channels
     const int n_waves = kBlock / kWave;
