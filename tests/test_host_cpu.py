@@ -202,3 +202,28 @@ def test_convolution_function_and_single_call_core_have_no_cpu_path(monkeypatch)
             DwConv3x3SiLU.forward(ctx, _OnGpu(x), w, b, False)
     with pytest.raises(RuntimeError):
         forward_core_hip(x, torch.zeros(4, 3, 16), torch.zeros(4, 16, 1), *(torch.zeros(64) for _ in range(3)))
+
+
+def test_observed_layers_are_called_in_training():
+    """A layer whose calls something sees -- a hook of its own, a global one, a forward set on the instance -- is called as a
+    module in training: no kernel stands for it."""
+    from torch.nn.modules import module as nn_module
+    from vmamba_amd.conv import dwconv_silu_trainable
+    from vmamba_amd.linear import linear_dw_pays
+    conv, linear = torch.nn.Conv2d(8, 8, 3, padding=1, groups=8), torch.nn.Linear(8, 8, bias=False)
+
+    def taken():
+        x, rows = _OnGpu(torch.zeros(1, 8, 6, 6)), _OnGpu(torch.zeros(4096, 8))
+        x.device = rows.device = torch.device("cpu")              # the weights' own
+        return [dwconv_silu_trainable(conv, x, False), linear_dw_pays(linear, rows)]
+    see = lambda *args: None
+    assert taken() == [True, True]
+    for register in (nn_module.register_module_forward_hook, nn_module.register_module_forward_pre_hook,
+                     nn_module.register_module_full_backward_hook, conv.register_forward_hook, linear.register_full_backward_hook):
+        handle = register(see)
+        assert taken() == [getattr(register, "__self__", conv) is not conv, getattr(register, "__self__", linear) is not linear]
+        handle.remove()
+    conv.forward, linear.forward = conv.forward, linear.forward
+    assert taken() == [False, False]
+    del conv.forward, linear.forward
+    assert taken() == [True, True]

@@ -8,6 +8,7 @@ import torch
 
 from . import _lib
 from .csm import transpose_bcl_hip
+from .norm import observed
 
 _DTYPE_CODE = {torch.float32: _lib.SS2D_F32, torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 
@@ -108,9 +109,8 @@ def dwconv_silu_trainable(conv2d, x, channel_last):
     if not (type(conv2d) is torch.nn.Conv2d and x.is_cuda and x.dim() == 4 and x.numel() > 0 and x.dtype in _DTYPE_CODE):
         return False
     D, H, W = (x.shape[3], x.shape[1], x.shape[2]) if channel_last else x.shape[1:]
-    hooks = (conv2d._forward_hooks, conv2d._forward_pre_hooks, conv2d._backward_hooks, conv2d._backward_pre_hooks)
     return (conv2d.kernel_size == (3, 3) and conv2d.padding == (1, 1) and conv2d.stride == (1, 1) and conv2d.dilation == (1, 1)
             and conv2d.padding_mode == "zeros" and conv2d.groups == conv2d.in_channels == conv2d.out_channels == D
-            and not any(hooks) and not torch.is_autocast_enabled()
+            and not observed(conv2d) and not torch.is_autocast_enabled()
             and all(t is None or (t.dtype == x.dtype and t.device == x.device) for t in (conv2d.weight, conv2d.bias))
             and _lib.lib().ss2d_dwconv3x3_silu_bwd_workspace_bytes(x.shape[0], D, H, W) > 0)

@@ -9,6 +9,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
+from .norm import observed
 
 _DTYPE_CODE = {torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 FUSED_SHAPES = ((96, 96),)            # (in_features, out_features)
@@ -100,11 +101,10 @@ def linear_dw_pays(layer, x):
     if not (type(layer) is nn.Linear and layer.bias is None and x.is_cuda and x.dim() >= 2 and x.dtype == torch.float32):
         return False
     weight = layer.weight
-    hooks = (layer._forward_hooks, layer._forward_pre_hooks, layer._backward_hooks, layer._backward_pre_hooks)
     N, K = weight.shape
     return (torch.is_grad_enabled() and weight.requires_grad and weight.dtype == x.dtype and weight.device == x.device
             and x.shape[-1] == K and N % 4 == 0 and K % 4 == 0 and 0 < N * K <= 384 * 384 and x.numel() >= 4096 * K
-            and not any(hooks) and not nn.modules.module._has_any_global_hook() and not torch.is_autocast_enabled())
+            and not observed(layer) and not torch.is_autocast_enabled())
 
 
 class LinearDw(torch.autograd.Function):

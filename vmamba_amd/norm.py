@@ -113,6 +113,13 @@ def needs_grad(*tensors):
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
+def observed(layer):
+    """True when something sees or replaces this module's calls -- hooks of its own, global ones, a forward set on the
+    instance: a kernel that stands for the module would go past them, so the module has to be called."""
+    hooks = (layer._forward_hooks, layer._forward_pre_hooks, layer._backward_hooks, layer._backward_pre_hooks)
+    return any(hooks) or nn.modules.module._has_any_global_hook() or "forward" in vars(layer)
+
+
 def _gpu_only(x, what):
     if not x.is_cuda:
         raise NotImplementedError(f"{what}: vmamba_amd runs on the GPU only (got a {x.device.type} tensor)")
