@@ -200,3 +200,24 @@ def test_x_proj_bounds_the_padded_tail():
                                                           4 * C * Hp * Wp, _lib.SS2D_BF16, None)
     for args in ((1, 4, 4, 4096, 4096), (8, 8, 8, 8, 1 << 18), (96, 8, 8, 1 << 18, 8)):
         assert call(*args) == _lib.SS2D_ENOTSUP, args
+
+
+def test_forward_core_says_what_it_takes():
+    """Whatever one of the four kernels refuses, the workspace query refuses: nothing has been launched or allocated then."""
+    def bytes_of(**kw):
+        p = _lib.ForwardCoreParams(batch=2, dim=64, height=8, width=8, rank=4, padded_height=8, padded_width=8, dtype=_lib.SS2D_BF16,
+                                   norm_dtype=_lib.SS2D_BF16, normalise=1, eps=1e-5)
+        for name in ("x", "x_proj_weight", "dt_proj_weight", "A", "D", "delta_bias", "norm_weight", "norm_bias", "out"):
+            setattr(p, name, 4096)
+        for name, value in kw.items():
+            setattr(p, name, value)
+        return _lib.lib().ss2d_forward_core_workspace_bytes(p)
+    F32, BF16, F16 = _lib.SS2D_F32, _lib.SS2D_BF16, _lib.SS2D_F16
+    taken = [{}, dict(rank=48), dict(norm_dtype=F32), dict(dtype=F32, norm_dtype=F32, rank=24), dict(dtype=F32, rank=24), dict(dtype=F16, norm_dtype=F16),
+             dict(dtype=F16, norm_dtype=F32, normalise=0), dict(dtype=F32, norm_dtype=F32, dim=44)]
+    refused = [dict(rank=49), dict(dtype=F32, norm_dtype=F32, rank=25), dict(dtype=F16, norm_dtype=F32), dict(norm_dtype=F16), dict(dim=44),
+               dict(x_proj_weight=4096 + 8), dict(dim=8000), dict(rank=95), dict(dtype=F32, norm_dtype=F32, rank=48, dim=768, height=7, width=7, padded_height=7, padded_width=7)]
+    for kw in taken:
+        assert bytes_of(**kw) > 0, kw
+    for kw in refused:
+        assert bytes_of(**kw) == _lib.SS2D_ENOTSUP, kw

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from vmamba_amd import ss2d
+from vmamba_amd.core import core_fits
 from vmamba_amd.ss2d import SS2D
 
 pytestmark = pytest.mark.gpu
@@ -18,6 +19,8 @@ DEV = "cuda:0"
 def test_same_bits(B, D, H, W, dtype, channel_first, monkeypatch):
     print("CASE forward_core", B, D, H, W, dtype, channel_first, flush=True)
     torch.manual_seed(H)
+    taken, native = [], ss2d.forward_core_hip
+    monkeypatch.setattr(ss2d, "forward_core_hip", lambda *a: taken.append(native(*a)) or taken[-1])
     op = SS2D(d_model=D, channel_first=channel_first).to(DEV).to(dtype).eval()
     with torch.no_grad():
         op.out_norm.weight.uniform_(0.5, 1.5)
@@ -28,6 +31,11 @@ def test_same_bits(B, D, H, W, dtype, channel_first, monkeypatch):
         mixed.load_state_dict(op.state_dict())
         mixed.out_norm.float()                                     # norm parameters of another type than the map's
         got_mixed = mixed.forward_core(x) if dtype != torch.float16 else None      # (the norm kernel has no such pair)
+        # the cases the single call is for are its own, not the separate calls compared with themselves
+        if op.dt_rank <= (24 if dtype == torch.float32 else 48) and core_fits(H, W, dtype):
+            assert len(taken) == 2 + (got_mixed is not None) and all(t is not None for t in taken)
+        else:
+            assert all(t is None for t in taken)
         monkeypatch.setattr(SS2D, "_forward_core_native", lambda self, x, normalise: None)
         assert torch.equal(got, op.forward_core(x)) and torch.equal(turned, op.forward_core(x.transpose(2, 3)))
         assert got_mixed is None or torch.equal(got_mixed, mixed.forward_core(x))

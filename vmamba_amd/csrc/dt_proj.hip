@@ -236,6 +236,13 @@ static int launch_dt_proj(DtArgs a, hipStream_t stream) {
     return launch_status();
 }
 
+static int64_t dt_x_span(int R, int64_t N, int64_t x_rank_stride) { return ((R - 1) * x_rank_stride + N) * 2; }     // bytes of a direction's rows
+
+// fp32 and wide ranks are the library GEMM's; offsets are 31 bits
+bool dt_proj_takes(int D, int R, int64_t N, int64_t x_rank_stride, int dtype) {
+    return dtype != SS2D_F32 && R > 0 && R <= kDtMaxRank && dt_x_span(R, N, x_rank_stride) < 0x7ffffff0ll && (int64_t)D * R * 2 < 0x7ffffff0ll;
+}
+
 }  // namespace ss2d
 
 // The fill value as the 16 bits of the output type (round to nearest even; beyond the type's range: its infinity).
@@ -264,7 +271,7 @@ extern "C" int ss2d_dt_proj_masked(const void *x, const void *weight, const void
     if (dtype != SS2D_F32 && dtype != SS2D_BF16 && dtype != SS2D_F16) return SS2D_EINVAL;
     if (K == 0 || D == 0 || N == 0) return SS2D_OK;
     if (!x || !weight || !delta) return SS2D_EINVAL;
-    if (dtype == SS2D_F32 || R > kDtMaxRank || R == 0) return SS2D_ENOTSUP;   // fp32 and wide ranks: the library GEMM
+    if (!dt_proj_takes(D, R, N, x_rank_stride, dtype)) return SS2D_ENOTSUP;
     DtArgs a;
     a.x = x; a.W = weight; a.out = delta;
     a.mask = mask; a.fill2 = fill_bits16(fill, dtype) * 0x10001u;
@@ -277,9 +284,7 @@ extern "C" int ss2d_dt_proj_masked(const void *x, const void *weight, const void
     a.blocks_per_wave = (int)bpw;
     a.n_pos_chunks = (a.n_blocks + bpw - 1) / bpw;
     a.total_waves = (int64_t)K * a.d_chunks * a.n_pos_chunks;
-    const int64_t x_span = ((int64_t)(R - 1) * x_rank_stride + N) * 2;        // one direction's rows
-    if (x_span >= 0x7ffffff0ll || (int64_t)D * R * 2 >= 0x7ffffff0ll) return SS2D_ENOTSUP;
-    a.x_span_bytes = (uint32_t)x_span;
+    a.x_span_bytes = (uint32_t)dt_x_span(R, N, x_rank_stride);
     a.w_vec = (R % 4 == 0) && (reinterpret_cast<uintptr_t>(weight) % 8 == 0);
     // 16-byte loads of x and stores of delta: rows and bases on 16-byte boundaries
     a.vec_ok = (N % 8 == 0) && (x_dir_stride % 8 == 0) && (x_rank_stride % 8 == 0) &&

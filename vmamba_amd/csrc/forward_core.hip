@@ -13,6 +13,17 @@ struct ForwardCorePlan {
     ss2d_core_params core;
 };
 
+// What a kernel refuses is found here, before a caller has allocated or launched anything.
+static bool forward_core_kernels_take(const ss2d_forward_core_params *q, int64_t pitch) {
+    if (q->dtype == SS2D_F32) {
+        if (!dt_proj_f32_takes(q->rank)) return false;
+    } else if (ss2d_x_proj_applies(q->batch, q->dim, q->rank + 2, q->padded_height, q->padded_width, q->dtype) != SS2D_OK ||
+               reinterpret_cast<uintptr_t>(q->x_proj_weight) % 16 != 0 || !dt_proj_takes(q->dim, q->rank, pitch, pitch, q->dtype)) {
+        return false;
+    }
+    return !q->normalise || layer_norm_cf_takes(q->dim, SS2D_F32, q->norm_dtype, q->dtype);
+}
+
 static int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
 // base may be NULL while only the size is asked for: stand-in pointers of the same alignment take its place
@@ -30,6 +41,7 @@ static int forward_core_plan(const ss2d_forward_core_params *q, char *base, Forw
     p.pitch = (q->batch * L + vec - 1) / vec * vec;
     // on a padded map delta has to start every image where its mask does
     if (p.padded && p.pitch != q->batch * L) return SS2D_ENOTSUP;
+    if (!forward_core_kernels_take(q, p.pitch)) return SS2D_ENOTSUP;
     p.x = 0;
     p.x_dbl = p.padded ? align256(p.x + q->batch * D * L * es) : 0;
     p.delta = align256(p.x_dbl + 4 * C * p.pitch * es);

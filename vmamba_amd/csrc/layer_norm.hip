@@ -978,6 +978,8 @@ static int launch_ln_cf_image(const LnImagePlan &p, const void *x, const void *w
     return launch_status();
 }
 
+constexpr int kLnCfMaxChannels = 156 * 1024 / (5 * (int)sizeof(float));
+
 template <typename in_t, typename w_t, typename out_t>
 static int launch_ln_cf(const void *x, const void *w, const void *b, void *y, int B, int C, int L, float eps,
                         int out_channel_last, hipStream_t stream) {
@@ -1009,7 +1011,7 @@ static int launch_ln_cf(const void *x, const void *w, const void *b, void *y, in
     // in 156 KB of LDS)
     if ((size_t)C * 9 * sizeof(float) <= 48 * 1024)
         return launch_ln_cf_tile<in_t, w_t, out_t, 8>(x, w, b, y, B, C, L, eps, out_channel_last, stream);
-    if ((size_t)C * 5 * sizeof(float) <= 156 * 1024)
+    if (C <= kLnCfMaxChannels)
         return launch_ln_cf_tile<in_t, w_t, out_t, 4>(x, w, b, y, B, C, L, eps, out_channel_last, stream);
     return SS2D_ENOTSUP;
 }
@@ -1028,6 +1030,16 @@ static int launch_ln_cf(const void *x, const void *w, const void *b, void *y, in
         case SS2D_F16 * 9 + SS2D_F32 * 3 + SS2D_F16: return CALL(f16_t, float, f16_t);                      \
         default: return SS2D_ENOTSUP;                                                                        \
     }
+
+bool layer_norm_cf_takes(int C, int in_dtype, int w_dtype, int out_dtype) {
+    if (C > kLnCfMaxChannels) return false;
+    const auto known = [&]() -> int {
+#define SS2D_CALL(I, W, O) SS2D_OK
+        SS2D_LN_DISPATCH(SS2D_CALL)
+#undef SS2D_CALL
+    };
+    return known() == SS2D_OK;
+}
 
 static bool ln_dtype_ok(int d) { return d == SS2D_F32 || d == SS2D_BF16 || d == SS2D_F16; }
 

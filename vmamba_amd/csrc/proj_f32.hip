@@ -227,6 +227,10 @@ static void launch_dt_f32(const DtF32Args &a, bool vec, hipStream_t s) {
     else hipLaunchKernelGGL((dt_proj_f32_kernel<kSteps, false>), dim3(grid), dim3(kBlock), 0, s, a);
 }
 
+// beyond 24 ranks the library's GEMM is level with it (768 x 28 x 28, batch 4, 48 ranks: 29 us either way) or ahead (one
+// map of 7 x 7: 5 us against 9)
+bool dt_proj_f32_takes(int R) { return R > 0 && R <= 24; }
+
 }  // namespace ss2d
 
 extern "C" int ss2d_x_proj_f32(const float *x, const float *weight, float *out, int B, int D, int C, int H, int W,
@@ -263,9 +267,7 @@ extern "C" int ss2d_dt_proj_f32(const float *x, const float *weight, float *delt
     if (K < 0 || D < 0 || R < 0 || N < 0 || x_dir_stride < 0 || x_rank_stride < 0) return SS2D_EINVAL;
     if (K == 0 || D == 0 || N == 0) return SS2D_OK;
     if (!x || !weight || !delta) return SS2D_EINVAL;
-    // beyond 24 ranks the library's GEMM is level with it (768 x 28 x 28, batch 4, 48 ranks: 29 us either way) or ahead (one
-    // map of 7 x 7: 5 us against 9)
-    if (R == 0 || R > 24) return SS2D_ENOTSUP;
+    if (!dt_proj_f32_takes(R)) return SS2D_ENOTSUP;
     DtF32Args a;
     a.x = x; a.W = weight; a.out = delta;
     a.K = K; a.D = D; a.R = R; a.N = N; a.ks = x_dir_stride; a.rs = x_rank_stride;

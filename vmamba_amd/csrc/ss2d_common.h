@@ -208,6 +208,12 @@ __device__ __forceinline__ void layer_norm_tile_rows(uint16_t *tile, int pitch, 
     }
 }
 
+// What the entry points of other files take, from the sizes and types alone (ss2d_dt_proj_masked, ss2d_dt_proj_f32,
+// ss2d_layer_norm_cf): for callers that launch several kernels and have to know before the first.
+bool dt_proj_takes(int D, int R, int64_t N, int64_t x_rank_stride, int dtype);
+bool dt_proj_f32_takes(int R);
+bool layer_norm_cf_takes(int C, int in_dtype, int w_dtype, int out_dtype);
+
 inline int launch_status() { return hipGetLastError() == hipSuccess ? SS2D_OK : SS2D_ELAUNCH; }
 
 }  // namespace ss2d
