@@ -43,10 +43,14 @@ def test_linear_dw_autograd(with_residual):
     y = LinearDw.apply(x, layer.weight, res)
     y_ref = layer(x) if res is None else res + layer(x)
     got, want = torch.autograd.grad(y, wanted, dy), torch.autograd.grad(y_ref, wanted, dy)
-    # M * 2^-24 with the sums' magnitudes of unit-variance products, M = 4096 positions; the others sum 64 of them at most
+    # y and dx are the layer's own products in another call: 48 and 64 of them, n * 2^-24 of the sum of their magnitudes each,
+    # and one more rounding where the residual is added
     assert torch.allclose(y, y_ref, rtol=0, atol=1e-5)
-    for a, b in zip(got, want):
-        assert torch.allclose(a, b, rtol=0, atol=4096 * 2.0 ** -24 * 4096)
+    w, dy2, x2 = layer.weight.detach().double(), dy.double().reshape(-1, 64), x.detach().double().reshape(-1, 48)
+    dx, dw = got[0].double().reshape(-1, 48), got[1].double()
+    assert bool(((dx - dy2 @ w).abs() <= 64 * 2.0 ** -24 * (dy2.abs() @ w.abs())).all())
+    assert bool(((dw - dy2.t() @ x2).abs() <= 4096 * 2.0 ** -24 * (dy2.abs().t() @ x2.abs())).all())
+    assert all(torch.equal(a, b) for a, b in zip(got[2:], want[2:]))                     # the residual's is dy
     # second order: through the library's products
     y = LinearDw.apply(x, layer.weight, res)
     (dw,) = torch.autograd.grad((y * y).sum(), layer.weight, create_graph=True)
