@@ -227,3 +227,17 @@ def test_observed_layers_are_called_in_training():
     assert taken() == [False, False]
     del conv.forward, linear.forward
     assert taken() == [True, True]
+
+
+def test_single_call_core_leaves_steps_of_an_instance_alone(monkeypatch):
+    """A step replaced on the instance is part of what forward_core does, as one of a subclass is: the single call does not stand
+    for it."""
+    from vmamba_amd import ss2d
+    monkeypatch.setattr(ss2d, "forward_core_hip", lambda *args: "called")
+    op, x = ss2d.SS2D(d_model=16), _OnGpu(torch.zeros(1, 16, 8, 8))
+    with torch.no_grad():
+        for step in ("forward_core_fused", "finish_core", "_inference_constants"):
+            assert op._forward_core_native(x, True) == "called"
+            setattr(op, step, getattr(op, step))
+            assert op._forward_core_native(x, True) is None
+            delattr(op, step)

@@ -115,6 +115,9 @@ def _pad_mask(H0, W0, H, W, n_images, device):
     return mask
 
 
+_CORE_STEPS = ("forward_core_fused", "finish_core", "_inference_constants")      # what SS2D._forward_core_native stands for
+
+
 class SS2D(nn.Module):
     """SS2D block: in_proj -> dwconv3x3 -> SiLU -> forward_core -> (gate) -> out_proj.
 
@@ -303,12 +306,12 @@ class SS2D(nn.Module):
 
     def _forward_core_native(self, x, normalise):
         """forward_core -- or, without ``normalise``, forward_core_fused -- as one call into the library, or None where that
-        does not stand for them: training, other layers or an out_norm of another kind, a subclass with its
+        does not stand for them: training, other layers or an out_norm of another kind, a subclass or an instance with its
         own steps, a shape without a kernel."""
         cls, norm = type(self), self.out_norm
         if not (x.is_cuda and x.dim() == 4 and x.numel() > 0 and self._fused_core_applies(x)
                 and cls.forward_core_fused is SS2D.forward_core_fused and cls.finish_core is SS2D.finish_core
-                and cls._inference_constants is SS2D._inference_constants):
+                and cls._inference_constants is SS2D._inference_constants and vars(self).keys().isdisjoint(_CORE_STEPS)):
             return None
         if normalise and not (self.layers is HipLayers and type(norm) is (LayerNorm2d if self.channel_first else LayerNorm)
                               and norm.normalized_shape == (x.shape[1],) and not needs_grad(norm.weight, norm.bias)):
