@@ -36,6 +36,12 @@ CASES = [
     (1, 40, 3, 65, 1, None, -1),           # one column: the tile before the last ends inside the map's last four positions
     (1, 32, 8, 137, 1, None, -1),
     (1, 8, 8, 256, 1931, None, -1),        # a row that fits LDS with two directions, not with four
+    (1, 336, 23, 45, 45, None, -1),        # one odd map: tiles of two rows, channels split in two
+    (1, 768, 50, 28, 28, None, -1),        # one even map: tiles of four rows
+    (2, 64, 10, 56, 56, None, -1),         # from eight rows to four
+    (1, 96, 8, 113, 113, None, -1),        # one row per tile
+    (1, 32, 7, 9, 200, None, -1),          # tiles of half the rows in two columns of tiles
+    (1, 24, 6, 131, 2, None, -1),          # two columns: tiles of 33 rows
     (2, 96, 8, 57, 58, (60, 60), 6),       # padded map with a mask row
     (1, 384, 26, 19, 19, (20, 20), -1),    # padded map without one
     (3, 16, 3, 5, 7, (8, 8), 3),           # mask row behind the last row

@@ -359,6 +359,18 @@ static int x_proj_plan(int B, int D, int C, int H, int W, int Hp, int Wp, int dt
         total = grid(Th);
         if (a.n_dirs == 1 || (total >= 256 && row_bytes * Th <= kMostLds)) break;
     }
+    // Few workgroups walk all channels of a large tile one step after the other while most of the chip idles: tiles of half
+    // the rows -- multiples of 4 where they were, for the wide stores -- double the grid, and from two column groups down the
+    // wavefronts share the channels as well (k_split below).  One image, bf16: 768 x 56 x 56, C = 50 34.5 -> 12.9 us, 336 x 45 x 45,
+    // C = 23 25.2 -> 8.2, 192 x 28 x 28, C = 14 9.3 -> 6.8.  From 160 workgroups on it costs more than it gives (at 192: 48 images
+    // of 384 x 14 x 14, C = 32 11.9 -> 15.3).
+    while (total < 160 && Th > 1 && Th * a.Tw > kXpGroup) {
+        int64_t t = (Th + 1) / 2;
+        if (unit > 1 && t > 2) t = (t + 3) / 4 * 4;
+        if (t >= Th) break;
+        Th = t;
+        total = (int64_t)B * (4 / a.n_dirs) * a.tiles_w * ((H + Th - 1) / Th);
+    }
     // a row of a width that is no multiple of 4 is not cut: there is a widest one
     if (total > 0x7fffffff || row_bytes * Th > kMostLds || Th * a.Tw * a.pitch > (1 << 22)) return SS2D_ENOTSUP;
     a.total = (uint32_t)total;
