@@ -101,3 +101,23 @@ def test_x_proj_refuses():
         x_proj_hip(x, torch.zeros(4, 3, 12, dtype=torch.bfloat16, device=DEV), out)            # D not a multiple of 8
     with pytest.raises(RuntimeError):
         x_proj_hip(x, torch.zeros(4, 3, 12, dtype=torch.float16, device=DEV), out)
+
+
+@pytest.mark.parametrize("D, N, B, side, kernel", [(64, 16, 2, 14, True), (384, 16, 1, 14, True), (768, 16, 1, 7, False),
+                                                   (384, 2, 2, 73, False), (384, 2, 1, 73, True)])
+def test_projections_of_several_states(D, N, B, side, kernel, monkeypatch):
+    """project_from_map on either side of x_proj_pays: the kernel runs where it is the faster one and not beyond, and B and C are
+    the float64 product's on both (bounds as above)."""
+    from vmamba_amd import ss2d
+    torch.manual_seed(D + side)
+    op = ss2d.SS2D(d_model=D, d_state=N).to(DEV, torch.bfloat16).eval()
+    x = torch.randn(B, D, side, side).bfloat16()
+    ran = []
+    monkeypatch.setattr(ss2d, "x_proj_hip", lambda *a: (ran.append(1), x_proj_hip(*a))[1])
+    with torch.no_grad():
+        _, Bs, Cs = op.project_from_map(x.to(DEV), op._inference_constants(B))
+    assert bool(ran) == kernel
+    w, xs = op.x_proj_weight.detach().cpu().double()[:, op.dt_rank:], scan_orders(x.double(), side, side)
+    want, size = torch.matmul(w, xs), torch.matmul(w.abs(), xs.abs())
+    got = torch.cat([Bs, Cs], 2).cpu().double()
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() * (1 + 2.0 ** -8) + D * 2.0 ** -24 * size).all())

@@ -218,6 +218,19 @@ def x_proj_fits(x, weight):
             and _lib.lib().ss2d_x_proj_applies(x.shape[0], x.shape[1], weight.shape[1], x.shape[2], x.shape[3], _DTYPE_CODE[x.dtype]) == _lib.SS2D_OK)
 
 
+def x_proj_pays(x, weight):
+    """False where the library's batched product with the one-by-one CrossScan behind it is the faster way to what ss2d_x_proj
+    gives for a map (B, D, H, W) and weights (4, C, D).  Many rows: beyond C = 64 a workgroup has six accumulator tiles of one
+    direction, reads the weights with every step, and the map is read four times (one image of 768 x 14 x 14, C = 80: 15 us
+    against 10; 48 images of 768 x 28 x 28: 82 against 68).  Many channels on large maps, where the library's product fills the
+    chip and the four readings add up; earlier on odd maps, whose stores are single elements (48 images of 576 x 31 x 31,
+    C = 44: 70 against 47 us; of 192 x 56 x 56, C = 44, the kernel 62 against 77).  Of 690 shapes of 96 to 768 channels with 4 and
+    16 states, the rule's choice is slower by over 3 % on 44, by 1.25 at most; the kernel on all of them on 159, by up to 2.7."""
+    B, D, H, W = x.shape
+    large = 2 << 20 if H * W % 2 else 16 << 20
+    return weight.shape[1] <= 64 and (D < 384 or B * D * H * W < large)
+
+
 def x_proj_hip(x, weight, out, padded=None, mask_row=-1):
     """weight (4, C, D) applied to the map x (B, D, H, W), each direction's rows in its scan order, written into ``out``: a
     (B, 4, C', L') view with contiguous rows (any batch / direction / row strides), L' = H' * W' of the ``padded`` size
