@@ -186,6 +186,27 @@ def test_x_proj_wants_its_tensors_on_one_device(monkeypatch):
                 run(_OnGpu(x), w, o)
 
 
+def test_patch_embedding_kernel_stands_for_plain_convolutions_only():
+    """The second layer's kernel goes past Conv2d._conv_forward: a convolution that computes something else there, or one that
+    autocast runs in another type, is left to itself."""
+    from vmamba_amd.norm import LayerNorm
+    from vmamba_amd.stem import stem2_fusable
+
+    class Standardised(torch.nn.Conv2d):
+        def _conv_forward(self, x, weight, bias):
+            return super()._conv_forward(x, weight - weight.mean((1, 2, 3), keepdim=True), bias)
+
+    x = _OnGpu(torch.zeros(1, 48, 8, 8, dtype=torch.bfloat16).to(memory_format=torch.channels_last))
+    make = lambda cls: cls(48, 96, 3, stride=2, padding=1).bfloat16()
+    plain, norm = make(torch.nn.Conv2d), LayerNorm(96).bfloat16()
+    assert stem2_fusable(x, plain, norm)
+    assert not stem2_fusable(x, make(Standardised), norm)
+    with torch.autocast("cuda", torch.bfloat16):
+        assert not torch.is_autocast_enabled() or stem2_fusable(x, plain, norm)
+    plain._conv_forward = lambda *a: None
+    assert not stem2_fusable(x, plain, norm)
+
+
 def test_convolution_function_and_single_call_core_have_no_cpu_path(monkeypatch):
     """Neither may hand a host address to a kernel, whichever of its tensors lies on the CPU."""
     from vmamba_amd import _lib

@@ -4,6 +4,7 @@ activations (classification/models/vmamba.py:1403-1416)."""
 import ctypes
 
 import torch
+import torch.nn as nn
 
 from . import _lib
 
@@ -49,7 +50,11 @@ _STEM2_MAX_BYTES = 0x7f000000             # the kernel's offsets into the input 
 
 
 def stem2_fusable(x, conv, norm):
-    """True when ss2d_stem_conv2_ln serves this conv / norm pair on x (B, 48, H, W), channel-last in memory."""
+    """True when ss2d_stem_conv2_ln serves this conv / norm pair on x (B, 48, H, W), channel-last in memory: a convolution that
+    computes what nn.Conv2d does, in x's own type."""
+    own = type(conv)._conv_forward is not nn.Conv2d._conv_forward or "_conv_forward" in vars(conv)
+    if own or (torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != x.dtype):
+        return False
     return (x.is_cuda and x.dim() == 4 and x.dtype in _DTYPE_CODE and x.shape[1] == conv.in_channels
             and (conv.in_channels, conv.out_channels) == STEM2_SHAPE and tuple(conv.kernel_size) == (3, 3)
             and tuple(conv.stride) == (2, 2) and tuple(conv.padding) == (1, 1) and tuple(conv.dilation) == (1, 1)
