@@ -4,6 +4,9 @@
 // The library spent 540 us on the three convolution passes of 64 x 384 maps of 14 x 14 in fp32 (the weights' gradient alone
 // 450, a general grouped convolution), more than on any other part of that block's training step; what they move is 58 MB.
 // (Now 27 us forward, 45 backward; the step 3.01 -> 2.36 ms with the two layout changes on this package's transpose.)
+// Forward and backward through autograd against the library, channel-last, batch 64, us: 96 x 56 x 56 fp32 2296 -> 269, bf16
+// 1848 -> 187, fp16 2504 -> 186; 768 x 7 x 7 433 -> 150, 561 -> 149, 342 -> 150; one image of 384 x 14 x 14 183 -> 146, 174 -> 150,
+// 165 -> 146 (the host's share); two of 96 x 256 x 256 1301 -> 269, 1807 -> 203, 1341 -> 205: it serves every map that fits.
 // Here one kernel reads x and dy once and writes dx once: a workgroup owns one channel of several images -- its nine weights'
 // gradients stay in registers over all of them -- and holds their planes in LDS (whole planes where they fit, rows of them
 // with a halo where not), zero-padded so that no tap has a bound to test.  z is recomputed from the same x the weights'

@@ -893,7 +893,9 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
         // wavefronts.  The grid is filled first -- one state: 8 wavefronts per SIMD, as three at a time are resident (96 x 56 x 56,
         // batch 64: 250 us; half as many workgroups: 275); several states: the 2 per SIMD the registers allow -- down to 8
         // channels (57 x 58 maps, batch 16: 109 us; with 4: 119) or, on small problems, 4.  At most 24: no gain beyond, and the
-        // per-channel scalars sit in the lanes of a register.
+        // per-channel scalars sit in the lanes of a register.  Groups of fewer channels leave wavefronts without one and are
+        // still ahead of a wavefront per row: one channel per group, backward through autograd, 64 x 384 rows of 196 positions
+        // 320 -> 95 us, 64 x 768 of 49 224 -> 123, 16 x 96 of 3306 361 -> 109; three 333 -> 77, 230 -> 77, 361 -> 78.
         const int64_t want_wg = (one ? 8192 : 2048) / n_waves, images = (int64_t)q->batch * q->n_groups;
         const int64_t per_8 = images * ((a.dim_per_group + 7) / 8);
         const int64_t least = one && per_8 >= want_wg / 4 ? 8 : 4;

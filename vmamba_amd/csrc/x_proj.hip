@@ -15,7 +15,7 @@
 //   * maps of one or two MFMA column groups (7 x 7 ... 11 x 11) split the channels over the wavefronts instead of the
 //     positions and meet in LDS.
 // 96 x 56 x 56, batch 128: 25-28 us (3.9 TB/s of the 103 MB); 192 x 28 x 28: 45 -> 20; 384 x 14 x 14: 31 -> 16.5;
-// 768 x 7 x 7: 30 -> 17.5; one image of each: 24 -> 9-10.
+// 768 x 7 x 7: 30 -> 17.5; one image of each, replayed from a graph: 9.3 -> 5.8, 9.9 -> 6.8, 22.1 -> 7.6, 20.0 -> 11.5.
 #include <type_traits>
 
 #include "ss2d_common.h"

@@ -6,10 +6,10 @@ channel-first (vmamba.py:493-646, the non-cascade ``cross2d`` branch with ``no_e
 
     CrossScan -> x_proj -> split (dt, B, C) -> dt_proj -> selective scan -> CrossMerge -> out_norm
 
-CrossScan, the selective scan and CrossMerge run on this package's HIP kernels; the two tiny
-projections stay PyTorch-ROCm GEMMs.  B and C are handed to the scan as strided views of the
-projection output: the kernel honours batch/group/state strides, so the reference's
-``.contiguous()`` copies (vmamba.py:621-622) are not needed.
+CrossScan, the selective scan and CrossMerge run on this package's HIP kernels, and so do the two
+narrow projections at inference (PyTorch-ROCm GEMMs in training and where those are faster).  B and C
+are handed to the scan as strided views of the projection output: the kernel honours
+batch/group/state strides, so the reference's ``.contiguous()`` copies (vmamba.py:621-622) are not needed.
 
 Parameter names, shapes and initialisation follow vmamba.py:165-232 and :463-479, so a
 reference state_dict of this block loads as is.
