@@ -103,7 +103,7 @@ def test_x_proj_refuses():
         x_proj_hip(x, torch.zeros(4, 3, 12, dtype=torch.float16, device=DEV), out)
 
 
-@pytest.mark.parametrize("D, N, B, side, kernel", [(64, 16, 2, 14, True), (384, 16, 1, 14, True), (768, 16, 1, 7, False),
+@pytest.mark.parametrize("D, N, B, side, kernel", [(64, 16, 2, 14, True), (384, 16, 1, 14, True), (768, 16, 1, 7, True), (768, 16, 8, 19, False),
                                                    (384, 2, 2, 73, False), (384, 2, 1, 73, True)])
 def test_projections_of_several_states(D, N, B, side, kernel, monkeypatch):
     """project_from_map on either side of x_proj_pays: the kernel runs where it is the faster one and not beyond, and B and C are

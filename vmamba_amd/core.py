@@ -220,15 +220,15 @@ def x_proj_fits(x, weight):
 
 def x_proj_pays(x, weight):
     """False where the library's batched product with the one-by-one CrossScan behind it is the faster way to what ss2d_x_proj
-    gives for a map (B, D, H, W) and weights (4, C, D).  Many rows: beyond C = 64 a workgroup has six accumulator tiles of one
-    direction, reads the weights with every step, and the map is read four times (one image of 768 x 14 x 14, C = 80: 15 us
-    against 10; 48 images of 768 x 28 x 28: 82 against 68).  Many channels on large maps, where the library's product fills the
-    chip and the four readings add up; earlier on odd maps, whose stores are single elements (48 images of 576 x 31 x 31,
-    C = 44: 70 against 47 us; of 192 x 56 x 56, C = 44, the kernel 62 against 77).  Of 690 shapes of 96 to 768 channels with 4 and
-    16 states, the rule's choice is slower by over 3 % on 44, by 1.25 at most; the kernel on all of them on 159, by up to 2.7."""
+    gives for a map (B, D, H, W) and weights (4, C, D).  Many channels on large maps, where the library's product fills the chip
+    and the kernel's four readings of the map add up (48 images of 768 x 28 x 28, C = 56: 60 us against 49); earlier on odd maps,
+    whose stores are single elements (48 images of 576 x 31 x 31, C = 44: 70 against 47; of 192 x 56 x 56, C = 44, the kernel 62
+    against 77), and beyond C = 64, where a workgroup has six accumulator tiles of one direction (48 images of 768 x 28 x 28, C = 80:
+    82 against 68).  On small maps the kernel may be the slower one too (one image of 768 x 14 x 14, C = 80: 15 against 10) but is a
+    launch fewer, and a call that short waits for the host: forward_core there 121 us with the kernel, 153 with the library."""
     B, D, H, W = x.shape
-    large = 2 << 20 if H * W % 2 else 16 << 20
-    return weight.shape[1] <= 64 and (D < 384 or B * D * H * W < large)
+    many = weight.shape[1] > 64
+    return B * D * H * W < (2 << 20 if many or H * W % 2 else 16 << 20) or (D < 384 and not many)
 
 
 def x_proj_hip(x, weight, out, padded=None, mask_row=-1):
