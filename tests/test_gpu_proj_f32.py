@@ -43,3 +43,23 @@ def test_dt_proj_f32(K, D, R, N):
 def test_wide_ranks_are_refused():
     with pytest.raises(RuntimeError):
         dt_proj_f32_hip(torch.zeros(1, 25, 8, device=DEV), torch.zeros(1, 8, 25, device=DEV))
+
+
+@pytest.mark.parametrize("d_state, B, D, H, W, kernel", [(2, 1, 416, 71, 71, True), (2, 1, 416, 73, 71, False), (2, 5, 416, 64, 64, False),
+                                                         (1, 1, 416, 71, 71, True), (1, 1, 416, 73, 71, False), (2, 1, 96, 151, 151, True)])
+def test_projection_on_either_side_of_the_rule(d_state, B, D, H, W, kernel, monkeypatch):
+    """forward_core takes ss2d_x_proj_f32 where x_proj_f32_pays says so and the library's product elsewhere, with one result: the
+    projections differ by D * 2^-24 of their products' magnitudes, some 1e-6 of the output after the scan and the norm."""
+    from vmamba_amd import ss2d
+    torch.manual_seed(D + H)
+    op = ss2d.SS2D(d_model=D, d_state=d_state).cuda().eval()
+    x = torch.nn.functional.silu(torch.randn(B, D, H, W)).cuda()
+    ran, kept = [], ss2d.x_proj_f32_hip
+    monkeypatch.setattr(ss2d, "x_proj_f32_hip", lambda *a: (ran.append(1), kept(*a))[1])
+    with torch.no_grad():
+        got = op.forward_core(x)
+        assert bool(ran) == kernel
+        monkeypatch.setattr(ss2d, "x_proj_f32_pays", lambda *a: not kernel)
+        other = op.forward_core(x)
+        assert len(ran) == 1
+    assert ((got - other).double().norm() / other.double().norm()).item() < 1e-5

@@ -283,6 +283,17 @@ def x_proj_f32_fits(x, weight):
             and x.numel() // x.shape[1] < 2 ** 31)
 
 
+def x_proj_f32_pays(x, weight):
+    """x_proj_pays in single precision.  Few wavefronts share many channels there and load them step by step, single floats on
+    maps of no whole 16-byte pieces: with 384 channels or more the library is ahead from 2 Mi elements on for those (48 images of
+    576 x 17 x 17, one state: forward_core 396 us, with the kernel 413) and from 8 Mi on for the others (16 of 768 x 28 x 28,
+    four states: 341 against 356).  Below, the library's time jumps between neighbouring shapes -- 48 images of 576 x 7 x 7 take it
+    four times the kernel's -- and the call waits for the host; many images of few positions are the kernel's at any size (64 of
+    768 x 14 x 14, C = 50: 72 against 196)."""
+    B, D, H, W = x.shape
+    return D < 384 or H * W < 256 or B * D * H * W < (2 << 20 if H * W % 4 else 8 << 20)
+
+
 def x_proj_f32_hip(x, weight, out):
     """x_proj_hip in single precision: weight (4, C, D) applied to the map x (B, D, H, W), each direction's rows in its scan
     order, into ``out``: a (B, 4, C, L) view with contiguous rows (ss2d_x_proj_f32)."""

@@ -22,8 +22,8 @@ import torch.nn.functional as F
 
 from ._lib import SS2D_ENOTSUP, Ss2dError
 from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_fits, core_mask_pads_hip, dt_proj_f32_hip, dt_proj_hip,
-                   embed_maps_hip, forward_core_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_fits,
-                   x_proj_hip, x_proj_pays)
+                   embed_maps_hip, forward_core_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_f32_pays,
+                   x_proj_fits, x_proj_hip, x_proj_pays)
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
 from .conv import DwConv3x3SiLU, dwconv3x3_silu_hip, dwconv_silu_trainable
@@ -223,7 +223,8 @@ class SS2D(nn.Module):
         K, L, R, N = self.k_group, H * W, self.dt_rank, self.d_state
         if x_proj_pays(x, self.x_proj_weight) and x_proj_fits(x, self.x_proj_weight) and not needs_grad(x, self.x_proj_weight):
             x_dbl = x_proj_hip(x, self.x_proj_weight, x.new_empty((B, K, R + 2 * N, L)))
-        elif x_proj_f32_fits(x, self.x_proj_weight) and not needs_grad(x, self.x_proj_weight):
+        elif (x_proj_f32_fits(x, self.x_proj_weight) and x_proj_f32_pays(x, self.x_proj_weight)
+              and not needs_grad(x, self.x_proj_weight)):
             x_dbl = x_proj_f32_hip(x, self.x_proj_weight, x.new_empty((B, K, R + 2 * N, L)))
         else:
             proj = torch.bmm(consts["Wx_all"], x.reshape(B, D, L)).view(B, K, R + 2 * N, H, W)
@@ -273,7 +274,7 @@ class SS2D(nn.Module):
         x_dbl_rows = x_dbl[:, :, :B].permute(2, 0, 1, 3)
         if x_proj_fits(x, self.x_proj_weight):
             x_proj_hip(x, self.x_proj_weight, x_dbl_rows)
-        elif x_proj_f32_fits(x, self.x_proj_weight):
+        elif x_proj_f32_fits(x, self.x_proj_weight) and x_proj_f32_pays(x, self.x_proj_weight):
             x_proj_f32_hip(x, self.x_proj_weight, x_dbl_rows)
         else:
             proj = torch.bmm(consts["Wx_all"], x.view(B, D, L))                               # (B, K*C, L)
