@@ -104,7 +104,8 @@ def test_x_proj_refuses():
 
 
 @pytest.mark.parametrize("D, N, B, side, kernel", [(64, 16, 2, 14, True), (384, 16, 1, 14, True), (768, 16, 1, 7, True), (768, 16, 8, 19, False),
-                                                   (384, 2, 2, 73, False), (384, 2, 1, 73, True)])
+                                                   (384, 2, 2, 73, False), (384, 2, 1, 73, True),
+                                                   (384, 2, 26, 15, True)])
 def test_projections_of_several_states(D, N, B, side, kernel, monkeypatch):
     """project_from_map on either side of x_proj_pays: the kernel runs where it is the faster one and not beyond, and B and C are
     the float64 product's on both (bounds as above)."""

@@ -225,10 +225,12 @@ def x_proj_pays(x, weight):
     whose stores are single elements (48 images of 576 x 31 x 31, C = 44: 70 against 47; of 192 x 56 x 56, C = 44, the kernel 62
     against 77), and beyond C = 64, where a workgroup has six accumulator tiles of one direction (48 images of 768 x 28 x 28, C = 80:
     82 against 68).  On small maps the kernel may be the slower one too (one image of 768 x 14 x 14, C = 80: 15 against 10) but is a
-    launch fewer, and a call that short waits for the host: forward_core there 121 us with the kernel, 153 with the library."""
+    launch fewer, and a call that short waits for the host: forward_core there 121 us with the kernel, 153 with the library.  Many
+    images of few positions are the kernel's at any size, the library's product of one image being too narrow (128 of 768 x 7 x 7,
+    C = 50: 19 against 25; 64 of 768 x 15 x 15: 28 against 46)."""
     B, D, H, W = x.shape
     many = weight.shape[1] > 64
-    return B * D * H * W < (2 << 20 if many or H * W % 2 else 16 << 20) or (D < 384 and not many)
+    return H * W < 256 or B * D * H * W < (2 << 20 if many or H * W % 2 else 16 << 20) or (D < 384 and not many)
 
 
 def x_proj_hip(x, weight, out, padded=None, mask_row=-1):
