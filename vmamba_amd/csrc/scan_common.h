@@ -43,6 +43,15 @@ struct CoreArgs {
     int64_t dl_ks, dl_ds, dl_bs;        // delta strides over direction, channel, batch (elements)
     int64_t B_ks, B_bs, C_ks, C_bs;     // B / C strides over direction and batch (elements)
     uint32_t B_span_bytes, C_span_bytes;
+    // forward_core only (nullptr elsewhere): the step's ranks as x_proj_pairs writes them instead of delta, strides in dwords
+    const uint32_t *dts;
+    const int32_t *dts_flags;           // flags_per_image words of every image: not 0 where one of the ranks is infinite or NaN
+    int32_t flags_per_image;
+    const uint16_t *Wdt;                // dt_proj's weight (4, D, rank)
+    int64_t dts_ks, dts_ps;
+    int32_t rank;
+    uint32_t dts_span_bytes;
+    uint32_t pad_weight;                // 16 bits: the weight of the rank that is 1 at added positions, 0: there is none
 };
 
 // scan_small.hip: the stand-alone scan for rows of 49 or 196 positions and one state, one segment of a row per lane.
@@ -58,6 +67,19 @@ int launch_core_small(const CoreArgs &a, int in_dtype, hipStream_t stream);
 bool core_tiled_eligible(const CoreArgs &a, int in_dtype);
 int64_t core_tiled_workspace_bytes(const CoreArgs &a);
 int launch_core_tiled(const CoreArgs &a, int in_dtype, void *workspace, hipStream_t stream);
+
+// ss2d_core.hip: the core with dt_proj folded in.  Rows of `dts` (x_proj_pairs) in place of delta; `delta` in q is not read.
+// core_dts_takes: from sizes, types and the alignment of B and C alone.
+struct CoreDts {
+    const void *dts, *weight;
+    int64_t dir_stride, pair_stride;    // dwords
+    int32_t rank;
+    uint32_t pad_weight;                // see CoreArgs
+    const int32_t *flags;
+    int32_t flags_per_image;
+};
+bool core_dts_takes(const ss2d_core_params *q, int rank, bool padded, DtsLayout &layout);
+int core_dts_fwd(const ss2d_core_params *q, const CoreDts &t, hipStream_t stream);
 
 // ---- 8-wide loads / stores ------------------------------------------------------------
 // Eight consecutive elements of a row as they sit in registers before widening: 4 dwords for 16-bit

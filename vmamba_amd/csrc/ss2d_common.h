@@ -153,6 +153,18 @@ __device__ __forceinline__ floatx16_t mfma_32x32x16(f16_t, u32x4_t a, u32x4_t b,
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8_t, a), __builtin_bit_cast(halfx8_t, b), c, 0, 0, 0);
 }
 
+// v_mfma_f32_16x16x32 (gfx950): D (16 x 16) += A (16 x 32) * B (32 x 16).  Lane l supplies A[l % 16][8*(l/16) .. +7] and
+// B[8*(l/16) .. +7][l % 16], and holds D[4*(l/16) + v][l % 16] in accumulator v = 0..3.
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ floatx4_t mfma_16x16x32(bf16_t, u32x4_t a, u32x4_t b, floatx4_t c) {
+    typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ floatx4_t mfma_16x16x32(f16_t, u32x4_t a, u32x4_t b, floatx4_t c) {
+    typedef _Float16 halfx8_t __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8_t, a), __builtin_bit_cast(halfx8_t, b), c, 0, 0, 0);
+}
+
 // LDS traffic of one wavefront is ordered by program order; this keeps the compiler from moving it around when
 // lanes exchange data through a wavefront-private LDS region (no workgroup barrier needed).
 __device__ __forceinline__ void wave_lds_sync() {
@@ -213,6 +225,22 @@ __device__ __forceinline__ void layer_norm_tile_rows(uint16_t *tile, int pitch, 
 bool dt_proj_takes(int D, int R, int64_t N, int64_t x_rank_stride, int dtype);
 bool dt_proj_f32_takes(int R);
 bool layer_norm_cf_takes(int C, int in_dtype, int w_dtype, int out_dtype);
+
+// ss2d_x_proj for one state per channel with the step's ranks in pairs, as the core with dt_proj folded in reads them
+// (core_dts_fwd): per direction ceil((R + padded) / 2) planes of dwords, low half rank 2 p, high half rank 2 p + 1 -- zero where
+// there is none; where x is a map of real_h x real_w with rows or columns of zeros added, rank R is 1 on those --, then the rows B and C.  A plane takes the room of two
+// rows, so that with P planes B is row 2 P.  Strides in 16-bit elements, multiples of 8.  Each of an image's workgroups --
+// x_proj_pairs_workgroups, or 0 where there is no variant -- leaves 0 in its word of `flags`, in the images' order, or not 0 if a rank
+// it wrote is infinite or NaN.
+//   The dwords of a plane stand in the order in which the core reads them (DtsLayout).  A workgroup of it walks the positions of
+// `images` images as one stream, a wavefront per_lane (8 or 16) consecutive positions per lane and 64 lanes at a time; the streams
+// follow one another, and inside each pass of 64 * per_lane positions -- fewer at the stream's end -- come the first four positions of
+// every lane, then the next four, ...: 16 bytes per lane side by side.
+struct DtsLayout { int32_t per_lane, images; };
+inline int dts_planes(int R, bool padded) { return (R + (padded ? 1 : 0) + 1) / 2; }
+int x_proj_pairs_workgroups(int B, int D, int R, int H, int W, int dtype);
+int x_proj_pairs(const void *x, const void *weight, void *out, int32_t *flags, int B, int D, int R, int H, int W, int real_h, int real_w, int64_t dir_stride,
+                 int64_t row_stride, const DtsLayout &layout, int dtype, void *stream);
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? SS2D_OK : SS2D_ELAUNCH; }
 

@@ -73,6 +73,13 @@ template <bool kWide> constexpr int core_items() { return kWide ? 2 * kItems : k
 // a few values that only live before and after the pass loop are then parked in scratch memory), four otherwise.
 template <typename in_t, int kGran, bool kWide> constexpr int core_min_waves() { return sizeof(in_t) == 2 && kGran >= 4 && !kWide ? 6 : 4; }
 
+// With dt_proj folded in the ranks of a pass take more registers than its delta did: four.
+template <typename in_t, int kGran, bool kWide, int kPairs> constexpr int core_waves() {
+    return kPairs > 0 && !kWide ? 4 : core_min_waves<in_t, kGran, kWide>();
+}
+
+constexpr int kCoreMostPairs = 4;  // of ranks that the core with dt_proj folded in takes
+constexpr int kCoreWidePairs = 3;  // ... with 16 positions per lane: four pairs of them spill, 195 us against 99 with 8 (48 x 96 maps of 57 x 58)
 constexpr int kCoreBurst = 2;     // passes whose delta / B / C loads are in flight per wavefront
 
 // What one pass of one lane loads from memory, as it arrives.
@@ -95,8 +102,19 @@ struct CorePassLoads {
 // before its own into the state the round started from, and the plane updates of the whole round happen in the usual two
 // phases (the passes of a round cover different positions, so the forward wavefronts do not meet each other, nor the
 // backward ones).  Two barriers and two update phases per kWpd passes instead of per pass.
-template <typename in_t, bool kSoftplus, int kGran, bool kVecDelta, bool kWide, int kWpd = 1>
-__global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t, kGran, kWide>())) void ss2d_core_kernel(const CoreArgs p, FastDiv divL, FastDiv divW, FastDiv divD, FastDiv divTiles,
+//
+// kPairs > 0: dt_proj folded in.  x_proj leaves the R <= 2 kPairs ranks of the step as dwords of two ranks per position
+// (x_proj_pairs); a lane loads the four dwords of four of its positions as one 16-byte piece per pair of ranks, and
+// v_mfma_f32_16x16x32 puts the four sums over the ranks where they are needed: B's column j holds the pieces of lanes j, j + 16,
+// j + 32, j + 48, 8 values of the contraction each, and row 4 q + v of A is the pair of weights at position v of lane group q's
+// piece and zero elsewhere, so that D[4 q + v][j] -- accumulator v of lane 16 q + j -- is that lane's own position v.  One matrix
+// instruction (16 cycles of a unit that idles here) per four positions and pair, no vector instruction, no exchange between
+// lanes, and delta -- the core's largest tensor, 308 MB written and read at 96 x 56 x 56, batch 128 -- never exists; the sums stay
+// in fp32 where dt_proj rounds them to 16 bits.  96 x 56 x 56, batch 128, bf16: 170 + 67 us of dt_proj -> 176 (three pairs, 16
+// positions per lane); the ranks come from L2, 2.5 times the lines of before, in runs of 1 KB (as x_proj's plain rows, 64 bytes from
+// lane to lane: 216).
+template <typename in_t, bool kSoftplus, int kGran, bool kVecDelta, bool kWide, int kWpd = 1, int kPairs = 0>
+__global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGran, kWide, kPairs>())) void ss2d_core_kernel(const CoreArgs p, FastDiv divL, FastDiv divW, FastDiv divD, FastDiv divTiles,
                                                            FastDiv divWt) {
     extern __shared__ __align__(16) float core_smem[];
     static_assert(kWpd == 1 || kWide, "several wavefronts per direction: the 16-positions-per-lane variant only");
@@ -124,8 +142,10 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
     in_t *xR = reinterpret_cast<in_t *>(planeB + plane_ext);
     in_t *xT = xR + map_ext;
 
+    static_assert(kPairs == 0 || (kSoftplus && core_flat_maps<in_t, kGran>()), "dt_proj folded in: 16-bit maps walked in blocks of 8");
     uint32_t bt, d;
-    divmod(blockIdx.x, divD, bt, d);                     // neighbouring workgroups share B / C rows (same images)
+    // neighbouring workgroups share B / C rows (same images) and the step's ranks, several times their bytes: one XCD each
+    divmod(kPairs > 0 ? xcd_contiguous_id(blockIdx.x, gridDim.x) : blockIdx.x, divD, bt, d);
     const int b0 = (int)bt * p.CB;
     const int nb = min(p.CB, p.B - b0);
     const int n_el = nb * L;
@@ -161,6 +181,92 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
     divmod((uint32_t)(lane * kIt + half * kPassLen), divL, next_img, next_j);
     divmod((uint32_t)(kStride * kPassLen), divL, step_img, step_j);
     next_img *= (uint32_t)L; step_img *= (uint32_t)L;
+    // ---- the step's ranks and their weights (kPairs > 0) ----------------------------------------------------------
+    constexpr int kPieces = kPairs > 0 ? kIt / 4 : 1, kP = kPairs > 0 ? kPairs : 1;
+    u32x4_t ranks[kP][kPieces];
+    uint32_t w_pair[kP];
+    if constexpr (kPairs > 0) {
+        const uint16_t *w = p.Wdt + (int64_t)kd * p.rank;
+#pragma unroll
+        for (int q = 0; q < kPairs; ++q) {
+            const uint32_t lo = 2 * q < p.rank ? w[2 * q] : 2 * q == p.rank ? p.pad_weight : 0u;
+            const uint32_t hi = 2 * q + 1 < p.rank ? w[2 * q + 1] : 2 * q + 1 == p.rank ? p.pad_weight : 0u;
+            w_pair[q] = lo | hi << 16;
+        }
+    }
+    u32x4_t w_frag[kP];
+    const int w_slot = (lane >> 4) == ((lane & 15) >> 2) ? lane & 3 : -1;     // which of A's four dwords of this lane is the pair
+    // The pieces of a pass's lanes lie side by side (DtsLayout): a load of a wavefront is 1 KB in one run.  Lanes past the end of
+    // the stream read its last lane's: finite where the stream is.  All but the lane's 16 bytes is in scalar registers.
+    const __amdgpu_buffer_rsrc_t dts_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t *>(p.dts), 0, (int)p.dts_span_bytes, kBufferRsrcWord3);
+    const uint32_t dts_first = (uint32_t)(dir * p.dts_ks + (int64_t)b0 * L) * 4u;
+    auto rank_lanes = [&](int pass) { return min(kWave, (n_el - pass * kPassLen) / kIt); };      // (whole lanes: kIt divides L)
+    auto rank_piece = [&](int pass, int q, int g, int lanes, int of_lane) {
+        const uint32_t first = dts_first + (uint32_t)(q * p.dts_ps + pass * kPassLen) * 4u + (uint32_t)(g * lanes) * 16u;
+        return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(dts_rsrc, min(of_lane, lanes - 1) * 16, (int)first, 0));
+    };
+    auto weights_at = [&](uint32_t w) { return u32x4_t{w_slot == 0 ? w : 0u, w_slot == 1 ? w : 0u, w_slot == 2 ? w : 0u, w_slot == 3 ? w : 0u}; };
+    if constexpr (kPairs > 0 && !kWide) {
+#pragma unroll
+        for (int q = 0; q < kPairs; ++q) {
+            w_frag[q] = weights_at(w_pair[q]);
+            asm volatile("" : "+v"(w_frag[q]));          // kept, not put together again
+        }
+    }
+    auto issue_ranks = [&](int pass) {
+        const int lanes = rank_lanes(pass);
+#pragma unroll
+        for (int q = 0; q < kPairs; ++q)
+#pragma unroll
+            for (int g = 0; g < kPieces; ++g) ranks[q][g] = rank_piece(pass, q, g, lanes, lane);
+    };
+    auto project = [&](float (&raw)[kIt]) {
+        if constexpr (kPairs > 0) {
+            floatx4_t acc[kPieces];
+#pragma unroll
+            for (int g = 0; g < kPieces; ++g) acc[g] = floatx4_t{0, 0, 0, 0};
+#pragma unroll
+            for (int q = 0; q < kPairs; ++q) {
+                u32x4_t frag = w_frag[q];
+                if constexpr (kWide) {                   // put together in every pass: there are no registers to keep it in
+                    uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)w_pair[q]);
+                    asm volatile("" : "+s"(w));
+                    frag = weights_at(w);
+                }
+#pragma unroll
+                for (int g = 0; g < kPieces; ++g) acc[g] = mfma_16x16x32(in_t{}, frag, ranks[q][g], acc[g]);
+            }
+#pragma unroll
+            for (int i = 0; i < kIt; ++i) raw[i] = acc[i / 4][i % 4];
+        }
+    };
+    auto project_one = [&](uint32_t pair, uint32_t w, float sum) {
+        if constexpr (sizeof(in_t) == 2)
+            return fmaf(unpack_hi<in_t>(pair), unpack_hi<in_t>(w), fmaf(unpack_lo<in_t>(pair), unpack_lo<in_t>(w), sum));
+        else return sum;
+    };
+    // The same sums within the lane: in the matrix product a rank that is infinite or NaN meets the zero weights of the other
+    // positions of its column and makes NaN of them.  For the images in which x_proj has found one.
+    bool in_lane = false;                                // uniform
+    if constexpr (kPairs > 0) {
+        int found = 0;
+        for (int i = lane; i < nb * p.flags_per_image; i += kWave) found |= p.dts_flags[(int64_t)b0 * p.flags_per_image + i];
+        in_lane = __any(found != 0);
+    }
+    auto project_in_lane = [&](int pass, float (&raw)[kIt]) {
+#pragma unroll
+        for (int g = 0; g < kPieces; ++g) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) raw[(4 * g + v) % kIt] = 0.0f;
+#pragma unroll
+            for (int q = 0; q < kPairs; ++q) {
+                const u32x4_t t = rank_piece(pass, q, g, rank_lanes(pass), lane);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) raw[(4 * g + v) % kIt] = project_one(t[v], w_pair[q], raw[(4 * g + v) % kIt]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
     auto issue = [&](int pass, Loads &r) {
         const int e0 = pass * kPassLen + lane * kIt;
 #pragma unroll
@@ -207,9 +313,27 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
 
     // the first passes' loads fly while the maps are staged
     Loads regs[kCoreBurst];
+    // kPairs > 0: B (and the pass's place in its image) with the ranks, C by itself; the rows of an image follow one another
+    auto issue_ranks_B = [&](int pass) {
+        issue_ranks(pass);
+        regs[0].img = next_img; regs[0].j0 = next_j;
+        next_img += step_img; next_j += step_j;
+        if (next_j >= (uint32_t)L) { next_j -= (uint32_t)L; next_img += (uint32_t)L; }
 #pragma unroll
-    for (int q = 0; q < kCoreBurst; ++q)
-        if (kStride * q + half < n_pass) issue(kStride * q + half, regs[q]);
+        for (int gi = 0; gi < kGroups; ++gi)
+            gather_group_raw<in_t, kGran>(B_rsrc, (uint32_t)(pass * kPassLen + lane * kIt + gi * kGran), B_soff, regs[0].b[gi]);
+    };
+    auto issue_C = [&](int pass) {
+#pragma unroll
+        for (int gi = 0; gi < kGroups; ++gi)
+            gather_group_raw<in_t, kGran>(C_rsrc, (uint32_t)(pass * kPassLen + lane * kIt + gi * kGran), C_soff, regs[0].c[gi]);
+    };
+    if constexpr (kPairs > 0) {
+    } else {
+#pragma unroll
+        for (int q = 0; q < kCoreBurst; ++q)
+            if (kStride * q + half < n_pass) issue(kStride * q + half, regs[q]);
+    }
 
     // ---- stage: copy the maps into xR / xT ------------------------------------------------------------------------
     const in_t *xin = reinterpret_cast<const in_t *>(p.x);
@@ -273,6 +397,9 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
     } else {
         stage_elements();
     }
+    if constexpr (kPairs > 0) {
+        if (half < n_pass) { issue_ranks_B(half); issue_C(half); }
+    }
     // the merge planes start at zero (every entry is then updated by plain read-add-write, 0 + y being exact), and so
     // does the block behind the maps
     {
@@ -301,8 +428,9 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
     // kDefer (kPair): stops before the incoming state is needed -- yv receives the lane's running products, hv its states
     // from a zero start, ex the wavefront scan's (a_ex, h_ex, a_tot, h_tot) -- and apply_carry finishes the pass.
     struct WaveScan { float a_ex, h_ex, a_tot, h_tot; };
+    // raw: kPairs > 0: the projected steps, before bias and softplus.
     auto compute = [&](bool reverse, int pass, const Loads &r, float &h_carry, float (&yv)[kIt], GroupSlot (&slot)[kGroups], auto defer_tag,
-                       float (&hv)[kIt], WaveScan &ex) {
+                       float (&hv)[kIt], WaveScan &ex, const float (&raw)[kIt]) {
         constexpr bool kDefer = decltype(defer_tag)::value;
         const int e0 = pass * kPassLen + lane * kIt;
         const int j0 = (int)r.j0;
@@ -312,7 +440,12 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
 #pragma unroll
         for (int blk = 0; blk < kBlocks; ++blk) {
             float raw8[kItems], bias8[kItems], dl8[kItems];
-            unpack_raw<in_t>(r.dl[blk], raw8);
+            if constexpr (kPairs > 0) {
+#pragma unroll
+                for (int i = 0; i < kItems; ++i) raw8[i] = raw[blk * kItems + i];
+            } else {
+                unpack_raw<in_t>(r.dl[blk], raw8);
+            }
             if constexpr (kBits) {
 #pragma unroll
                 for (int i = 0; i < kItems; ++i) dl8[i] = softplus_over_ln2(fmaf(raw8[i], kLog2e, bias * kLog2e));
@@ -436,7 +569,14 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
         const int base = reverse ? (int)(i * L) + L - 1 - (int)jj : e;      // this direction's index of the position
         float raw = 0.0f, Bv = 0.0f, Cv = 0.0f, u = 0.0f;
         if (valid) {
-            raw = to_f32(dl_base[e]);
+            if constexpr (kPairs > 0) {
+#pragma unroll
+                for (int q = 0; q < kPairs; ++q)
+                    raw = project_one(p.dts[(dts_first >> 2) + q * p.dts_ps + n_pass * kPassLen + (lane % kIt / 4 * rank_lanes(n_pass) + lane / kIt) * 4 + lane % 4],
+                                      w_pair[q], raw);
+            } else {
+                raw = to_f32(dl_base[e]);
+            }
             Bv = gather_elem<in_t>(B_rsrc, B_soff + i * (uint32_t)p.B_bs + jj);
             Cv = gather_elem<in_t>(C_rsrc, C_soff + i * (uint32_t)p.C_bs + jj);
             u = to_f32(xs[map_index<kEs, kFlat>(base)]);
@@ -458,6 +598,40 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
         __syncthreads();
     };
 
+    // A pass up to its states (kPairs > 0), from ranks, B and C that have been issued.  The next pass's ranks and B go out behind
+    // it, its C once the plane update is through with this one's: the update, the barriers and the other wavefronts cover their way.
+    auto projected_pass = [&](int pass, float &h_carry, float (&yv)[kIt], GroupSlot (&slot)[kGroups], auto defer_tag, float (&hv)[kIt],
+                              WaveScan &ex) {
+        float raw[kIt];
+        if (in_lane) project_in_lane(pass, raw);
+        else project(raw);
+        compute(reverse, pass, regs[0], h_carry, yv, slot, defer_tag, hv, ex, raw);
+        // (C has come before anything else is asked for: the wait for it would be one for all of that)
+#pragma unroll
+        for (int gi = 0; gi < kGroups; ++gi)
+#pragma unroll
+            for (int w = 0; w < Loads::kWords; ++w) asm volatile("" : "+v"(regs[0].c[gi][w]));
+        if (pass + kStride < n_pass) issue_ranks_B(pass + kStride);
+    };
+    auto next_C = [&](int pass) {
+        if (pass + kStride < n_pass) issue_C(pass + kStride);
+    };
+
+    auto projected_passes = [&]() {
+        float h_carry = 0.0f;
+        for (int pass = 0; pass < n_pass; ++pass) {  // uniform over the workgroup
+            float yv[kIt];
+            GroupSlot slot[kGroups];
+            WaveScan unused;
+            projected_pass(pass, h_carry, yv, slot, std::false_type{}, yv, unused);
+            if (!reverse) { update_plane(false, regs[0], yv, slot); next_C(pass); }
+            __syncthreads();
+            if (reverse) { update_plane(true, regs[0], yv, slot); next_C(pass); }
+            __syncthreads();
+        }
+        if (short_tail) short_pass(reverse, h_carry, true);
+    };
+    auto rounds = [&]() {
     if constexpr (!kPair) {
         float h_carry = 0.0f;
         for (int pass0 = 0; pass0 < n_pass; pass0 += kCoreBurst) {
@@ -468,7 +642,7 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
                     float yv[kIt];
                     GroupSlot slot[kGroups];
                     WaveScan unused;
-                    compute(reverse, pass, regs[q], h_carry, yv, slot, std::false_type{}, yv, unused);
+                    compute(reverse, pass, regs[q], h_carry, yv, slot, std::false_type{}, yv, unused, yv);
                     if (!reverse) update_plane(false, regs[q], yv, slot);
                     __syncthreads();
                     if (reverse) update_plane(true, regs[q], yv, slot);
@@ -485,6 +659,7 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
 #pragma unroll
             for (int q = 0; q < kCoreBurst; ++q) {
                 const int round = r0 + q;
+                Loads &rq = regs[kPairs > 0 ? 0 : q];
                 if (round < n_round) {               // uniform over the workgroup
                     const int pass = kWpd * round + half;
                     const bool active = pass < n_pass;                          // uniform over the wavefront
@@ -494,23 +669,29 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_min_waves<in_t,
                     WaveScan ex;
                     float unused = 0.0f;
                     if (active) {
-                        compute(reverse, pass, regs[q], unused, yv, slot, std::true_type{}, hv, ex);
+                        if constexpr (kPairs > 0) projected_pass(pass, unused, yv, slot, std::true_type{}, hv, ex);
+                        else compute(reverse, pass, rq, unused, yv, slot, std::true_type{}, hv, ex, yv);
                         if (lane == 0 && half < kWpd - 1) s_agg[dir][half] = make_float2(ex.a_tot, ex.h_tot);
                     }
                     __syncthreads();                 // aggregates of this round, state and plane updates of the round before
                     float h_out = 0.0f;
                     if (active) h_out = apply_carry(yv, hv, ex);
-                    if (active && !reverse) update_plane(false, regs[q], yv, slot);
+                    if (active && !reverse) update_plane(false, rq, yv, slot);
+                    if (kPairs > 0 && !reverse) next_C(pass);
                     __syncthreads();
-                    if (active && reverse) update_plane(true, regs[q], yv, slot);
+                    if (active && reverse) update_plane(true, rq, yv, slot);
+                    if (kPairs > 0 && reverse) next_C(pass);
                     if (last && lane == 0) s_carry[dir] = h_out;               // (everyone has read the old one before the barrier above)
-                    if (active && pass + kWpd * kCoreBurst < n_pass) issue(pass + kWpd * kCoreBurst, regs[q]);
+                    if (kPairs == 0 && active && pass + kWpd * kCoreBurst < n_pass) issue(pass + kWpd * kCoreBurst, rq);
                 }
             }
         }
         __syncthreads();                             // the last state and the last plane updates are in place
         if (short_tail) short_pass(reverse, s_carry[dir], half == 0);
     }
+    };
+    if constexpr (kPairs > 0 && !kPair) projected_passes();
+    else rounds();
 
     // ---- merge: out[r] = (A[r] + B[t(r)]) + (D0 + D1 + D2 + D3) * x[r] ---------------------------------------------
     float Dsum = 0.0f;
@@ -638,14 +819,14 @@ static bool core_fits_lds(const CoreArgs &a) {
     return lds_bytes_of<in_t>(a.L, flat) <= kCoreMaxLds;
 }
 
+// How a problem is cut: 16 positions per lane or 8, and the images per workgroup; the LDS bytes that takes.
 template <typename in_t>
-static int launch_core(CoreArgs a, hipStream_t stream) {
+static size_t core_cut(const CoreArgs &a, int64_t g, bool &wide, int64_t &CB) {
     const int64_t L = a.L;
-    const int64_t g = core_granularity<in_t>(a);
     const bool flat = sizeof(in_t) == 2 && g == kItems;       // core_flat_maps
     // 16 positions per lane and pass where one image alone takes more LDS than a sixth of a CU (the tile cannot be
     // shortened, six workgroups per CU are out of reach anyway); else 8, with tiles that let six workgroups share a CU
-    const bool wide = flat && a.dl_bs == L && lds_bytes_of<in_t>(L, true) > kCoreSixPerCu;
+    wide = flat && a.dl_bs == L && lds_bytes_of<in_t>(L, true) > (a.rank > 0 && dts_planes(a.rank, a.pad_weight != 0) > kCoreWidePairs ? kCoreMaxLds : kCoreSixPerCu);
     const int64_t pass_len = wide ? 2 * kPass : kPass;         // core_items * 64
     const size_t lds_cap = wide ? 40 * 1024 : kCoreSixPerCu;
     // Images per workgroup.  A workgroup walks its CB images as one stream in passes of 512 positions, so the last
@@ -659,7 +840,7 @@ static int launch_core(CoreArgs a, hipStream_t stream) {
         const int64_t n = images * L, rem = n % pass_len;
         return 10 * (n / pass_len) + (rem == 0 ? 0 : rem <= kWave ? 3 : 10);
     };
-    int64_t CB = 1;
+    CB = 1;
     if (a.dl_bs == L) {                                       // adjacent delta rows need the batch-innermost layout
         int64_t best = -1;
         for (int64_t cb = align_rows; cb < a.B && lds_bytes(cb) <= lds_cap; cb += align_rows) {
@@ -668,7 +849,17 @@ static int launch_core(CoreArgs a, hipStream_t stream) {
         }
         if (lds_bytes(a.B) <= lds_cap && (best < 0 || passes(a.B) <= best)) CB = a.B;   // a single tile starts at image 0
     }
-    const size_t smem = lds_bytes(CB);
+    return lds_bytes(CB);
+}
+
+template <typename in_t>
+static int launch_core(CoreArgs a, hipStream_t stream) {
+    const int64_t L = a.L;
+    const int64_t g = core_granularity<in_t>(a);
+    const bool flat = sizeof(in_t) == 2 && g == kItems;       // core_flat_maps
+    bool wide;
+    int64_t CB;
+    const size_t smem = core_cut<in_t>(a, g, wide, CB);
     if (smem > kCoreMaxLds) return SS2D_ENOTSUP;
     a.CB = (int)CB;
     // 16-byte loads of the delta stream need every (direction, channel, first image of a workgroup) start aligned;
@@ -688,6 +879,32 @@ static int launch_core(CoreArgs a, hipStream_t stream) {
     const FastDiv dT = make_fastdiv((uint32_t)(tiled ? (a.H / 4) * (a.W / 4) : 1)), dWt = make_fastdiv((uint32_t)(tiled ? a.W / 4 : 1));
     // several wavefronts per direction where the arrays leave a CU two workgroups (two each) or one (four)
     const int wpd = !(wide && smem > kCorePairLds) ? 1 : smem > kCoreQuadLds ? 4 : 2;
+    if (a.dts) {
+        if constexpr (sizeof(in_t) == 2) {
+#define SS2D_CORE_LAUNCH_D(W16, WPD, P)                                                                                               \
+    hipLaunchKernelGGL((ss2d_core_kernel<in_t, true, kItems, true, W16, WPD, P>), dim3((uint32_t)n_wg), dim3(WPD * kBlock), smem, stream, a, dL, dW, dD, dT, dWt)
+#define SS2D_CORE_LAUNCH_P(P)                                                                                                         \
+    do {                                                                                                                            \
+        if constexpr (P <= 2) {                                                                                                     \
+            if (wpd == 4) { SS2D_CORE_LAUNCH_D(true, 4, P); break; }                                                                 \
+            if (wpd == 2) { SS2D_CORE_LAUNCH_D(true, 2, P); break; }                                                                 \
+        }                                                                                                                           \
+        if constexpr (P <= kCoreWidePairs) {                                                                                        \
+            if (wide) { SS2D_CORE_LAUNCH_D(true, 1, P); break; }                                                                     \
+        }                                                                                                                           \
+        SS2D_CORE_LAUNCH_D(false, 1, P);                                                                                            \
+    } while (0)
+            const int planes = dts_planes(a.rank, a.pad_weight != 0);
+            if (g != kItems || a.dl_bs != L || !a.softplus || planes < 2 || planes > kCoreMostPairs) return SS2D_ENOTSUP;
+            if (planes == 2) SS2D_CORE_LAUNCH_P(2);
+            else if (planes == 3) SS2D_CORE_LAUNCH_P(3);
+            else SS2D_CORE_LAUNCH_P(4);
+            return launch_status();
+#undef SS2D_CORE_LAUNCH_D
+#undef SS2D_CORE_LAUNCH_P
+        }
+        return SS2D_ENOTSUP;
+    }
 #define SS2D_CORE_LAUNCH_W(SP, G, V, W16)                                                                                         \
     hipLaunchKernelGGL((ss2d_core_kernel<in_t, SP, G, V, W16>), dim3((uint32_t)n_wg), dim3(kBlock), smem, stream, a, dL, dW, dD, dT, dWt)
 #define SS2D_CORE_LAUNCH_P(SP, G, V, WPD)                                                                                         \
@@ -742,6 +959,7 @@ static int core_args(const ss2d_core_params *q, CoreArgs &a) {
     if (B_span >= 0x7fffffffll || C_span >= 0x7fffffffll) return SS2D_ENOTSUP;
     a.B_span_bytes = (uint32_t)B_span; a.C_span_bytes = (uint32_t)C_span;
     a.CB = 1; a.vec_ok = 0; a.vec_out = 0; a.stage_tiles = 0; a.tile_merge = 0;
+    a.dts = nullptr; a.Wdt = nullptr; a.dts_flags = nullptr; a.flags_per_image = 0; a.dts_ks = a.dts_ps = 0; a.rank = 0; a.pad_weight = 0;
     return SS2D_OK;
 }
 
@@ -757,6 +975,42 @@ static int core_launch_single(const CoreArgs &a, int in_dtype, hipStream_t s) {
     if (in_dtype == SS2D_F32) return launch_core<float>(a, s);
     if (in_dtype == SS2D_BF16) return launch_core<bf16_t>(a, s);
     return launch_core<f16_t>(a, s);
+}
+
+bool core_dts_takes(const ss2d_core_params *q, int rank, bool padded, DtsLayout &layout) {
+    CoreArgs a;
+    if (core_args(q, a) != SS2D_OK || q->in_dtype == SS2D_F32 || !a.softplus || a.dl_bs != a.L || a.B_bs != a.L || a.C_bs != a.L) return false;
+    const int planes = dts_planes(rank, padded);
+    if (planes < 2 || planes > kCoreMostPairs || core_small_eligible(a, q->in_dtype) || !core_fits_lds<bf16_t>(a) ||
+        core_granularity<bf16_t>(a) != kItems) return false;
+    bool wide;
+    int64_t CB;
+    a.rank = rank; a.pad_weight = padded;
+    const size_t smem = core_cut<bf16_t>(a, kItems, wide, CB);
+    layout = {wide ? 2 * kItems : kItems, (int32_t)CB};
+    // Several wavefronts per direction hold two pairs of ranks in their registers and spill with three, which takes all that the
+    // fold gives (16 bf16 maps of 96 x 96: 64 channels 225 -> 177 us, 96 channels 222 -> 223); 8 positions per lane have no such variant.
+    return a.L % layout.per_lane == 0 && (smem <= kCorePairLds || (wide && planes <= 2));
+}
+
+// bytes from the first of the ranks' dwords to behind the last
+static int64_t dts_span(const CoreDts &t, const ss2d_core_params *q) {
+    return 4 * (3 * t.dir_stride + (dts_planes(t.rank, t.pad_weight != 0) - 1) * t.pair_stride + (int64_t)q->batch * q->height * q->width);
+}
+
+int core_dts_fwd(const ss2d_core_params *q, const CoreDts &t, hipStream_t stream) {
+    DtsLayout layout;
+    if (!core_dts_takes(q, t.rank, t.pad_weight != 0, layout)) return SS2D_ENOTSUP;
+    if (dts_span(t, q) >= 0x7fffffff) return SS2D_ENOTSUP;
+    if (!t.dts || !t.weight || !t.flags || reinterpret_cast<uintptr_t>(t.dts) % 16 != 0 || t.dir_stride % 4 != 0 || t.pair_stride % 4 != 0) return SS2D_EINVAL;
+    CoreArgs a;
+    const int rc = core_args(q, a);
+    if (rc != SS2D_OK) return rc;
+    a.dts = (const uint32_t *)t.dts; a.Wdt = (const uint16_t *)t.weight;
+    a.dts_flags = t.flags; a.flags_per_image = t.flags_per_image;
+    a.dts_span_bytes = (uint32_t)dts_span(t, q);
+    a.dts_ks = t.dir_stride; a.dts_ps = t.pair_stride; a.rank = t.rank; a.pad_weight = t.pad_weight;
+    return q->in_dtype == SS2D_BF16 ? launch_core<bf16_t>(a, stream) : launch_core<f16_t>(a, stream);
 }
 
 }  // namespace ss2d

@@ -29,21 +29,15 @@ struct XProjArgs {
     void *out;
     int32_t D, C, H, Wd, Hp, Wp;         // map H x Wd, written as Hp x Wp (padded at the bottom / right)
     int32_t mask_row;                    // -1: none
+    int32_t rank, planes, pair_mask;     // planes > 0: the first `rank` rows leave in pairs (x_proj_pairs)
+    int32_t *flags;
+    DtsLayout layout;
+    int32_t B, real_h, real_w;           // the map's size before rows and columns were added to it
     int32_t n_dirs, Ce;                  // directions per workgroup (1, 2, 4); C rounded up to even: rows per direction in LDS
     int32_t Th, Tw, tiles_h, tiles_w, pitch, k_steps, k_split, v_row, v_col;
     int64_t ks, cs, bs;
     uint32_t total;
 };
-
-typedef float floatx4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ floatx4_t mfma_16x16x32(bf16_t, u32x4_t a, u32x4_t b, floatx4_t c) {
-    typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ floatx4_t mfma_16x16x32(f16_t, u32x4_t a, u32x4_t b, floatx4_t c) {
-    typedef _Float16 halfx8_t __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8_t, a), __builtin_bit_cast(halfx8_t, b), c, 0, 0, 0);
-}
 
 // q = x / d, r = x % d for 0 <= x < 2^23, inv = 1 / d
 __device__ __forceinline__ void small_divmod(int x, int d, float inv, int &q, int &r) {
@@ -53,12 +47,14 @@ __device__ __forceinline__ void small_divmod(int x, int d, float inv, int &q, in
     if (r >= d) { ++q; r -= d; }
 }
 
-template <typename T, int kMt>
+// kPaired: the ranks of the step leave in pairs (x_proj_pairs).
+template <typename T, int kMt, bool kPaired>
 __global__ __launch_bounds__(kBlock, kMt == 1 ? 4 : kMt <= 3 ? 3 : 2) void x_proj_kernel(const XProjArgs p) {
     extern __shared__ __align__(16) uint16_t xp_smem[];         // [tile positions][pitch], then the split channels' sums
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     uint32_t id = xcd_contiguous_id(blockIdx.x, p.total);
+    const uint32_t wg = id;
     const int n_sets = 4 / p.n_dirs, k_first = (int)(id % (uint32_t)n_sets) * p.n_dirs;
     id /= (uint32_t)n_sets;
     const int tw = (int)(id % (uint32_t)p.tiles_w); id /= (uint32_t)p.tiles_w;
@@ -228,86 +224,178 @@ __global__ __launch_bounds__(kBlock, kMt == 1 ? 4 : kMt <= 3 ? 3 : 2) void x_pro
     const int rows_p = (last_h ? p.Hp : h1) - h0, cols_p = (last_w ? p.Wp : w1) - w0;
     const int n_out = rows_p * cols_p, rows_in = h1 - h0;
     const int64_t L = (int64_t)p.Hp * p.Wp;
-    // kV consecutive scan positions of rows 2 c2 and 2 c2 + 1 per lane (one dword per position: the tile's pitch is an odd
-    // number of dwords, so that lanes 8 positions apart meet in few banks), kC row pairs side by side in a wavefront
-    auto emit = [&](int dir, auto v_tag) {
-        const int k = k_first + dir;
-        const bool by_cols = k & 1, mirrored = k >= 2;
-        const int run = by_cols ? rows_p : cols_p;               // positions per line of the scan inside the tile
-        uint16_t *out = reinterpret_cast<uint16_t *>(p.out) + k * p.ks + b * p.bs;
-        const uint32_t *tile = reinterpret_cast<const uint32_t *>(xp_smem + dir * p.Ce);
-        constexpr int kV = decltype(v_tag)::value;
-        constexpr int kC = kV > 1 ? 4 : 1;
-        const int n_groups = n_out / kV, pairs = (p.C + 1) / 2;
-        const float inv_run = 1.0f / (float)run, inv_block = 1.0f / (float)(n_groups * kC);
-        auto store = [&](int row, int64_t j, const uint32_t (&e)[kV]) {       // e: 16 bits each
-            uint16_t *dst = out + row * p.cs + (mirrored ? L - kV - j : j);
-            if constexpr (kV == 1) {
-                *dst = (uint16_t)e[0];
-            } else {
-                uint32_t wds[kV / 2];
+    if constexpr (kPaired) {
+        // x_proj_pairs: the position-major tile holds rows 2 c and 2 c + 1 in one dword already; kV positions of a plane per lane,
+        // and in the place of one more plane the rows B and C
+        uint32_t exponents = 0;                                      // bits 15 and 31: an exponent of all ones was among the ranks
+        auto emit_pairs = [&](int dir, auto v_tag) {
+            const int k = k_first + dir;
+            const bool by_cols = k & 1, mirrored = k >= 2;
+            const int run = by_cols ? rows_p : cols_p;
+            uint16_t *out = reinterpret_cast<uint16_t *>(p.out) + k * p.ks;
+            const uint32_t *tile = reinterpret_cast<const uint32_t *>(xp_smem + dir * p.Ce);
+            constexpr int kV = decltype(v_tag)::value;
+            constexpr int kC = 4;
+            const int n_groups = n_out / kV, units = p.planes + 1;
+            const float inv_run = 1.0f / (float)run, inv_block = 1.0f / (float)(n_groups * kC);
+            const uint32_t one = from_f32<T>(1.0f).bits, per_lane_log2 = p.layout.per_lane == 16 ? 4 : 3;
+            const int64_t stream = (b - b % p.layout.images) * L;    // of this image: its first position, its length, the image's place in it
+            const uint32_t stream_len = (uint32_t)min((int64_t)p.layout.images * L, p.B * L - stream), in_stream = (uint32_t)(b % p.layout.images * L);
+            const int n_items = (units + kC - 1) / kC * n_groups * kC;
+            for (int item = threadIdx.x; item < n_items; item += kBlock) {
+                int block, idx, line, i;
+                small_divmod(item, n_groups * kC, inv_block, block, idx);
+                const int unit = block * kC + idx % kC;
+                if (unit >= units) continue;
+                small_divmod(idx / kC * kV, run, inv_run, line, i);
+                const int64_t j = by_cols ? (int64_t)(w0 + line) * p.Hp + h0 + i : (int64_t)(h0 + line) * p.Wp + w0 + i;
+                const int64_t at = mirrored ? L - kV - j : j;
+                const bool bc = unit == p.planes;
+                const int c = bc ? p.rank : 2 * unit;                // row in the low half (bc: B)
+                const uint32_t keep = bc ? 0xffffffffu : (c < p.rank ? 0xffffu : 0u) | (c + 1 < p.rank ? 0xffff0000u : 0u);
+                const uint32_t added = bc || !p.pair_mask ? 0u : c == p.rank ? one : c + 1 == p.rank ? one << 16 : 0u;
+                uint32_t e[kV];
 #pragma unroll
-                for (int q = 0; q < kV / 2; ++q)
-                    wds[q] = mirrored ? e[kV - 1 - 2 * q] | e[kV - 2 - 2 * q] << 16 : e[2 * q] | e[2 * q + 1] << 16;
-                if constexpr (kV == 8) *reinterpret_cast<uint4 *>(dst) = make_uint4(wds[0], wds[1], wds[2], wds[3]);
-                else *reinterpret_cast<uint2 *>(dst) = make_uint2(wds[0], wds[1]);
+                for (int q = 0; q < kV; ++q) {
+                    const int h = by_cols ? i : line, w = by_cols ? line : i;
+                    e[q] = added;
+                    if (h0 + h < p.real_h && w0 + w < p.real_w) {
+                        const uint32_t *at_pos = tile + (h * n_cols + w) * (p.pitch / 2) + c / 2;
+                        e[q] = bc && c % 2 ? at_pos[0] >> 16 | at_pos[1] << 16 : at_pos[0] & keep;
+                    }
+                    if (++i == run) { i = 0; ++line; }
+                }
+                if (!bc) {
+                    constexpr uint32_t kExp = std::is_same<T, bf16_t>::value ? 0x7f80u : 0x7c00u, kUlp = kExp & ~(kExp << 1);
+#pragma unroll
+                    for (int q = 0; q < kV; ++q) exponents |= (e[q] & (kExp | kExp << 16)) + (kUlp | kUlp << 16);
+                    // the place of the stream's position s: DtsLayout
+                    const uint32_t s = in_stream + (uint32_t)at, pass_len = kWave << per_lane_log2;
+                    const uint32_t first = s & ~(pass_len - 1), lane_of = (s - first) >> per_lane_log2, g = (s & ((1u << per_lane_log2) - 1)) / 4;
+                    const uint32_t lanes = min(pass_len, stream_len - first) >> per_lane_log2;
+                    uint32_t *dst = reinterpret_cast<uint32_t *>(out + 2 * unit * p.cs) + stream + first;
+                    if constexpr (kV == 1) {
+                        dst[(g * lanes + lane_of) * 4 + s % 4] = e[0];
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < kV / 4; ++q)
+                            reinterpret_cast<uint4 *>(dst)[(g + q) * lanes + lane_of] = mirrored ? make_uint4(e[kV - 1 - 4 * q], e[kV - 2 - 4 * q], e[kV - 3 - 4 * q], e[kV - 4 - 4 * q])
+                                                                         : make_uint4(e[4 * q], e[4 * q + 1], e[4 * q + 2], e[4 * q + 3]);
+                    }
+                    continue;
+                }
+#pragma unroll
+                for (int row = 0; row < 2; ++row) {
+                    uint16_t *dst = out + (2 * p.planes + row) * p.cs + b * L + at;
+                    if constexpr (kV == 1) {
+                        *dst = (uint16_t)(row ? e[0] >> 16 : e[0]);
+                    } else {
+                        uint32_t wds[kV / 2];
+#pragma unroll
+                        for (int q = 0; q < kV / 2; ++q) {
+                            const uint32_t lo = mirrored ? e[kV - 1 - 2 * q] : e[2 * q], hi = mirrored ? e[kV - 2 - 2 * q] : e[2 * q + 1];
+                            wds[q] = __builtin_amdgcn_perm(hi, lo, row ? 0x07060302u : 0x05040100u);
+                        }
+                        if constexpr (kV == 8) *reinterpret_cast<uint4 *>(dst) = make_uint4(wds[0], wds[1], wds[2], wds[3]);
+                        else *reinterpret_cast<uint2 *>(dst) = make_uint2(wds[0], wds[1]);
+                    }
+                }
             }
         };
-        auto scan_index = [&](int line, int i) {
-            return by_cols ? (int64_t)(w0 + line) * p.Hp + h0 + i : (int64_t)(h0 + line) * p.Wp + w0 + i;
+        for (int dir = 0; dir < p.n_dirs; ++dir) {
+            const int v = (k_first + dir) & 1 ? p.v_col : p.v_row;
+            if (v == 8) emit_pairs(dir, std::integral_constant<int, 8>{});
+            else if (v == 4) emit_pairs(dir, std::integral_constant<int, 4>{});
+            else emit_pairs(dir, std::integral_constant<int, 1>{});
+        }
+        const int found = __syncthreads_or((int)(exponents & 0x80008000u));
+        if (threadIdx.x == 0) p.flags[wg] = found;
+    } else {
+        // kV consecutive scan positions of rows 2 c2 and 2 c2 + 1 per lane (one dword per position: the tile's pitch is an odd
+        // number of dwords, so that lanes 8 positions apart meet in few banks), kC row pairs side by side in a wavefront
+        auto emit = [&](int dir, auto v_tag) {
+            const int k = k_first + dir;
+            const bool by_cols = k & 1, mirrored = k >= 2;
+            const int run = by_cols ? rows_p : cols_p;               // positions per line of the scan inside the tile
+            uint16_t *out = reinterpret_cast<uint16_t *>(p.out) + k * p.ks + b * p.bs;
+            const uint32_t *tile = reinterpret_cast<const uint32_t *>(xp_smem + dir * p.Ce);
+            constexpr int kV = decltype(v_tag)::value;
+            constexpr int kC = kV > 1 ? 4 : 1;
+            const int n_groups = n_out / kV, pairs = (p.C + 1) / 2;
+            const float inv_run = 1.0f / (float)run, inv_block = 1.0f / (float)(n_groups * kC);
+            auto store = [&](int row, int64_t j, const uint32_t (&e)[kV]) {       // e: 16 bits each
+                uint16_t *dst = out + row * p.cs + (mirrored ? L - kV - j : j);
+                if constexpr (kV == 1) {
+                    *dst = (uint16_t)e[0];
+                } else {
+                    uint32_t wds[kV / 2];
+#pragma unroll
+                    for (int q = 0; q < kV / 2; ++q)
+                        wds[q] = mirrored ? e[kV - 1 - 2 * q] | e[kV - 2 - 2 * q] << 16 : e[2 * q] | e[2 * q + 1] << 16;
+                    if constexpr (kV == 8) *reinterpret_cast<uint4 *>(dst) = make_uint4(wds[0], wds[1], wds[2], wds[3]);
+                    else *reinterpret_cast<uint2 *>(dst) = make_uint2(wds[0], wds[1]);
+                }
+            };
+            auto scan_index = [&](int line, int i) {
+                return by_cols ? (int64_t)(w0 + line) * p.Hp + h0 + i : (int64_t)(h0 + line) * p.Wp + w0 + i;
+            };
+            const int n_items = (pairs + kC - 1) / kC * n_groups * kC;
+            for (int item = threadIdx.x; item < n_items; item += kBlock) {
+                int block, idx, line, i;
+                small_divmod(item, n_groups * kC, inv_block, block, idx);
+                const int c2 = block * kC + idx % kC;
+                if (c2 >= pairs) continue;
+                small_divmod(idx / kC * kV, run, inv_run, line, i);
+                const int64_t j = scan_index(line, i);
+                uint32_t e[kV];
+#pragma unroll
+                for (int q = 0; q < kV; ++q) {
+                    const int h = by_cols ? i : line, w = by_cols ? line : i;
+                    e[q] = h < rows_in && w < n_cols ? tile[(h * n_cols + w) * (p.pitch / 2) + c2] : 0u;
+                    if (++i == run) { i = 0; ++line; }
+                }
+                uint32_t half[kV];
+                const int c = 2 * c2, shift = p.mask_row >= 0 ? p.mask_row : p.C;      // rows from the mask row on move up by one
+#pragma unroll
+                for (int q = 0; q < kV; ++q) half[q] = e[q] & 0xffffu;
+                store(c + (c >= shift), j, half);
+                if (c + 1 < p.C) {
+#pragma unroll
+                    for (int q = 0; q < kV; ++q) half[q] = e[q] >> 16;
+                    store(c + 1 + (c + 1 >= shift), j, half);
+                }
+            }
+            if (p.mask_row < 0) return;
+            for (int idx = threadIdx.x; idx < n_groups; idx += kBlock) {
+                int line, i;
+                small_divmod(idx * kV, run, inv_run, line, i);
+                const int64_t j = scan_index(line, i);
+                uint32_t e[kV];
+#pragma unroll
+                for (int q = 0; q < kV; ++q) {
+                    const int h = by_cols ? i : line, w = by_cols ? line : i;
+                    e[q] = h < rows_in && w < n_cols ? 0u : from_f32<T>(1.0f).bits;
+                    if (++i == run) { i = 0; ++line; }
+                }
+                store(p.mask_row, j, e);
+            }
         };
-        const int n_items = (pairs + kC - 1) / kC * n_groups * kC;
-        for (int item = threadIdx.x; item < n_items; item += kBlock) {
-            int block, idx, line, i;
-            small_divmod(item, n_groups * kC, inv_block, block, idx);
-            const int c2 = block * kC + idx % kC;
-            if (c2 >= pairs) continue;
-            small_divmod(idx / kC * kV, run, inv_run, line, i);
-            const int64_t j = scan_index(line, i);
-            uint32_t e[kV];
-#pragma unroll
-            for (int q = 0; q < kV; ++q) {
-                const int h = by_cols ? i : line, w = by_cols ? line : i;
-                e[q] = h < rows_in && w < n_cols ? tile[(h * n_cols + w) * (p.pitch / 2) + c2] : 0u;
-                if (++i == run) { i = 0; ++line; }
-            }
-            uint32_t half[kV];
-            const int c = 2 * c2, shift = p.mask_row >= 0 ? p.mask_row : p.C;      // rows from the mask row on move up by one
-#pragma unroll
-            for (int q = 0; q < kV; ++q) half[q] = e[q] & 0xffffu;
-            store(c + (c >= shift), j, half);
-            if (c + 1 < p.C) {
-#pragma unroll
-                for (int q = 0; q < kV; ++q) half[q] = e[q] >> 16;
-                store(c + 1 + (c + 1 >= shift), j, half);
-            }
+        for (int dir = 0; dir < p.n_dirs; ++dir) {
+            const int v = (k_first + dir) & 1 ? p.v_col : p.v_row;
+            if (v == 8) emit(dir, std::integral_constant<int, 8>{});
+            else if (v == 4) emit(dir, std::integral_constant<int, 4>{});
+            else emit(dir, std::integral_constant<int, 1>{});
         }
-        if (p.mask_row < 0) return;
-        for (int idx = threadIdx.x; idx < n_groups; idx += kBlock) {
-            int line, i;
-            small_divmod(idx * kV, run, inv_run, line, i);
-            const int64_t j = scan_index(line, i);
-            uint32_t e[kV];
-#pragma unroll
-            for (int q = 0; q < kV; ++q) {
-                const int h = by_cols ? i : line, w = by_cols ? line : i;
-                e[q] = h < rows_in && w < n_cols ? 0u : from_f32<T>(1.0f).bits;
-                if (++i == run) { i = 0; ++line; }
-            }
-            store(p.mask_row, j, e);
-        }
-    };
-    for (int dir = 0; dir < p.n_dirs; ++dir) {
-        const int v = (k_first + dir) & 1 ? p.v_col : p.v_row;
-        if (v == 8) emit(dir, std::integral_constant<int, 8>{});
-        else if (v == 4) emit(dir, std::integral_constant<int, 4>{});
-        else emit(dir, std::integral_constant<int, 1>{});
     }
 }
 
 template <typename T>
 static int launch_x_proj(const XProjArgs &a, size_t smem, int m_tiles, hipStream_t s) {
-#define SS2D_XP_LAUNCH(M) hipLaunchKernelGGL((x_proj_kernel<T, M>), dim3(a.total), dim3(kBlock), smem, s, a)
+#define SS2D_XP_LAUNCH(M) \
+    do {                                                                                                            \
+        if (a.planes > 0) hipLaunchKernelGGL((x_proj_kernel<T, M, true>), dim3(a.total), dim3(kBlock), smem, s, a);    \
+        else hipLaunchKernelGGL((x_proj_kernel<T, M, false>), dim3(a.total), dim3(kBlock), smem, s, a);                \
+    } while (0)
     if (m_tiles == 1) SS2D_XP_LAUNCH(1);
     else if (m_tiles == 2) SS2D_XP_LAUNCH(2);
     else if (m_tiles == 3) SS2D_XP_LAUNCH(3);
@@ -391,6 +479,49 @@ static int x_proj_plan(int B, int D, int C, int H, int W, int Hp, int Wp, int dt
     return SS2D_OK;
 }
 
+// The pointers, the output's strides and the stores' width, and the launch.
+static int x_proj_run(XProjArgs &a, const void *x, const void *weight, void *out, int Hp, int Wp, int64_t ks, int64_t cs, int64_t bs,
+                      size_t smem, int m_tiles, int dtype, hipStream_t s) {
+    if (reinterpret_cast<uintptr_t>(weight) % 16 != 0) return SS2D_ENOTSUP;
+    a.x = x; a.W = weight; a.out = out;
+    a.ks = ks; a.cs = cs; a.bs = bs;
+    // elements per store: what divides every row base, the scan's length and the starts of the tiles' lines
+    const int64_t L = (int64_t)Hp * Wp;
+    int64_t g = xp_gcd(xp_gcd(8, a.ks), xp_gcd(a.cs, a.bs));
+    g = xp_gcd(g, xp_gcd(L, (int64_t)(reinterpret_cast<uintptr_t>(out) % 16 / 2)));
+    if (reinterpret_cast<uintptr_t>(out) % 2 != 0) return SS2D_EINVAL;
+    const int64_t row_start = a.tiles_w == 1 ? (int64_t)a.Th * Wp : xp_gcd(Wp, a.Tw), col_start = a.tiles_h == 1 ? (int64_t)a.Tw * Hp : xp_gcd(Hp, a.Th);
+    const int64_t vr = xp_gcd(g, row_start), vc = xp_gcd(g, col_start);
+    a.v_row = (int)(vr == 2 ? 1 : vr);
+    a.v_col = (int)(vc == 2 ? 1 : vc);
+    return dtype == SS2D_BF16 ? launch_x_proj<bf16_t>(a, smem, m_tiles, s) : launch_x_proj<f16_t>(a, smem, m_tiles, s);
+}
+
+int x_proj_pairs_workgroups(int B, int D, int R, int H, int W, int dtype) {
+    XProjArgs a;
+    int m_tiles;
+    size_t smem;
+    if (R < 1 || B < 1 || x_proj_plan(B, D, R + 2, H, W, H, W, dtype, a, m_tiles, smem) != SS2D_OK) return 0;
+    return (int)(a.total / (uint32_t)B);
+}
+
+int x_proj_pairs(const void *x, const void *weight, void *out, int32_t *flags, int B, int D, int R, int H, int W, int real_h, int real_w, int64_t dir_stride,
+                 int64_t row_stride, const DtsLayout &layout, int dtype, void *stream) {
+    XProjArgs a;
+    int m_tiles;
+    size_t smem;
+    const int rc = x_proj_plan(B, D, R + 2, H, W, H, W, dtype, a, m_tiles, smem);
+    if (rc != SS2D_OK) return rc;
+    const int64_t L = (int64_t)H * W;
+    if (reinterpret_cast<uintptr_t>(out) % 16 != 0 || (dir_stride | row_stride) % 8 != 0 || (layout.per_lane != 8 && layout.per_lane != 16) ||
+        L % layout.per_lane != 0 || layout.images < 1 || layout.images * L > 0x7fffffff) return SS2D_EINVAL;
+    a.layout = layout; a.B = B;
+    a.mask_row = -1;
+    a.real_h = real_h; a.real_w = real_w;
+    a.flags = flags; a.rank = R; a.pair_mask = real_h != H || real_w != W; a.planes = dts_planes(R, a.pair_mask);
+    return x_proj_run(a, x, weight, out, H, W, dir_stride, row_stride, L, smem, m_tiles, dtype, (hipStream_t)stream);
+}
+
 }  // namespace ss2d
 
 extern "C" int ss2d_x_proj_applies(int B, int D, int C, int H, int W, int dtype) {
@@ -417,19 +548,9 @@ extern "C" int ss2d_x_proj(const void *x, const void *weight, void *out, int B, 
     size_t smem;
     const int rc = x_proj_plan(B, D, C, H, W, Hp, Wp, dtype, a, m_tiles, smem);
     if (rc != SS2D_OK) return rc;
-    if (reinterpret_cast<uintptr_t>(weight) % 16 != 0) return SS2D_ENOTSUP;
-    a.x = x; a.W = weight; a.out = out;
     a.mask_row = mask_row < 0 ? -1 : mask_row;
-    a.ks = out_dir_stride; a.cs = out_chan_stride; a.bs = out_batch_stride;
-    // elements per store: what divides every row base, the scan's length and the starts of the tiles' lines
-    const int64_t L = (int64_t)Hp * Wp;
-    int64_t g = xp_gcd(xp_gcd(8, a.ks), xp_gcd(a.cs, a.bs));
-    g = xp_gcd(g, xp_gcd(L, (int64_t)(reinterpret_cast<uintptr_t>(out) % 16 / 2)));
-    if (reinterpret_cast<uintptr_t>(out) % 2 != 0) return SS2D_EINVAL;
-    const int64_t row_start = a.tiles_w == 1 ? (int64_t)a.Th * Wp : xp_gcd(Wp, a.Tw), col_start = a.tiles_h == 1 ? (int64_t)a.Tw * Hp : xp_gcd(Hp, a.Th);
-    const int64_t vr = xp_gcd(g, row_start), vc = xp_gcd(g, col_start);
-    a.v_row = (int)(vr == 2 ? 1 : vr);
-    a.v_col = (int)(vc == 2 ? 1 : vc);
-    hipStream_t s = (hipStream_t)stream;
-    return dtype == SS2D_BF16 ? launch_x_proj<bf16_t>(a, smem, m_tiles, s) : launch_x_proj<f16_t>(a, smem, m_tiles, s);
+    a.rank = a.planes = a.pair_mask = 0;
+    a.flags = nullptr;
+    a.layout = {8, 1}; a.B = B; a.real_h = H; a.real_w = W;
+    return x_proj_run(a, x, weight, out, Hp, Wp, out_dir_stride, out_chan_stride, out_batch_stride, smem, m_tiles, dtype, (hipStream_t)stream);
 }
