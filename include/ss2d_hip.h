@@ -535,6 +535,18 @@ int ss2d_linear_cl(const void *x, const void *ln_weight, const void *ln_bias, fl
                    const void *bias, const void *residual, void *out, int64_t M, int K, int N, int dtype, void *stream);
 
 /*
+ * A channel-last projection of few positions with its neighbours folded in:  out = [GELU]([LayerNorm](x) W^T + bias) + residual.
+ * Stands, in a VSS block, for in_proj with the LayerNorm before it, out_proj with the residual add, and the MLP's layers with the
+ * LayerNorm, the GELU and the add around them (classification/models/vmamba.py:1225-1229, :648-650, :662, :1116-1131).
+ *   x (M, K), residual (M, N) or NULL, out (M, N) contiguous;  weight (N, K);  bias (N) or NULL;
+ *   ln_weight (K) or NULL = no LayerNorm, ln_bias (K) or NULL, eps;  gelu: 0, or not 0 for the exact (erf) GELU;
+ *   all SS2D_BF16 or all SS2D_F16, 16-byte aligned.  out may be residual, but not x.
+ * K a multiple of 16 up to 3072 (768 with a LayerNorm), N a multiple of 8; anything else, and SS2D_F32, returns SS2D_ENOTSUP.
+ */
+int ss2d_linear_rows(const void *x, const void *ln_weight, const void *ln_bias, float eps, const void *weight, const void *bias,
+                     const void *residual, void *out, int64_t M, int K, int N, int gelu, int dtype, void *stream);
+
+/*
  * The same projection fed by the SS2D core: x is the fp32 channel-first map (B, K, L) that ss2d_core_fwd (or
  * CrossMerge) leaves, the LayerNorm is the block's out_norm over the K channels of each position, computed from the
  * fp32 values and rounded to dtype as the separate operator does (classification/models/vmamba.py:641-646), and

@@ -9,7 +9,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .norm import observed
+from .norm import LayerNorm, needs_grad, observed
 
 _DTYPE_CODE = {torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 FUSED_SHAPES = ((96, 96),)            # (in_features, out_features)
@@ -41,6 +41,73 @@ def linear_cl_hip(x, weight, bias=None, residual=None, ln_weight=None, ln_bias=N
     rc = _lib.launch(x, _lib.lib().ss2d_linear_cl, x.data_ptr(), ptr(small[0]), ptr(small[1]), float(eps), keep[0].data_ptr(),
                      ptr(small[2]), ptr(keep[1]), out.data_ptr(), x.numel() // K, K, N, _DTYPE_CODE[x.dtype])
     _lib.check(rc, "ss2d_linear_cl")
+    return out
+
+
+def _rows_params(x, *params):
+    return all(t is None or (t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0) for t in params)
+
+
+def linear_rows_takes(layer, x):
+    """True when ss2d_linear_rows stands for this layer at inference on rows of x's type and device: a plain nn.Linear that nothing
+    observes, its parameters of x's own 16-bit dtype."""
+    if type(layer) is not nn.Linear or not x.is_cuda or x.dtype not in _DTYPE_CODE:
+        return False
+    N, K = layer.weight.shape
+    return (K % 16 == 0 and 0 < K <= 3072 and N % 8 == 0 and _rows_params(x, layer.weight, layer.bias)
+            and not needs_grad(x, layer.weight, layer.bias) and not observed(layer) and not torch.is_autocast_enabled())
+
+
+def linear_rows_fusable(x, layer, norm=None):
+    """True when ss2d_linear_rows takes ``layer(x)`` -- ``layer(norm(x))`` with a norm of this package -- and has few enough
+    positions to be the faster one (linear_rows_pays)."""
+    K = x.shape[-1]
+    if not (linear_rows_takes(layer, x) and layer.weight.shape[1] == K and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and linear_rows_pays(x.numel() // K, layer.weight.shape[0], K)):
+        return False
+    return norm is None or (type(norm) is LayerNorm and norm.normalized_shape == (K,) and K <= 768 and norm.weight is not None
+                            and _rows_params(x, norm.weight, norm.bias) and not needs_grad(norm.weight, norm.bias) and not observed(norm))
+
+
+def linear_rows_pays(M, N, K):
+    """True up to the number of positions where ss2d_linear_rows falls behind what else takes this product.  Its time is 3-5 us for
+    the launch and then grows with M N K, every 32 x 32 tile reading its operands from the L2.  Replayed from graphs, us, in bf16,
+    with LayerNorm or residual on both sides: 96 -> 96 at 12 544 positions 5.0 against ss2d_linear_cl's 8.0; 192 -> 192 at 3136
+    6.0 against the library's 8.6, at 12 544 14.3 / 12.0; 384 -> 384 at 784 6.5 / 9.0, at 1568 8.9 / 9.8, at 3136 13.3 / 11.5;
+    768 -> 768 at 196 7.2 / 9.8, at 400 10.6 / 10.2.  The MLP (fc1 is asked for, four outputs per input) has fewer passes around it
+    to win back: 384 at 400 17.6 / 23.7, at 784 27.5 / 27.5, at 1568 43 / 35; 768 at 49 20.6 / 24.9, at 196 30.2 / 26.4, where the
+    host's share (two launches for four library calls of 24 us and two of the package's) still decides.  Widths 96 and 192 have
+    ss2d_mlp_fused, whose 128 positions per workgroup leave the chip idle below: 192 at 784 12.1 / 45.2, at 3136 27.2 / 45.5, at
+    6272 44.6 / 45.8; 96 at 6272 15.5 / 17.8, at 12 544 25.3 / 18.0."""
+    if N >= 4 * K:
+        return 0 < M <= 6144 if K <= 192 else 0 < M * N * K <= 480 << 20
+    return 0 < M * N * K <= 192 << 20
+
+
+def linear_rows_hip(x, weight, bias=None, residual=None, ln_weight=None, ln_bias=None, eps=1e-5, gelu=False):
+    """x (..., K) channel-last, weight (N, K), one 16-bit dtype: [gelu]([layer_norm(x)] @ weight.T + bias) + residual, shape
+    (..., N), for few positions (ss2d_linear_rows)."""
+    if not x.is_cuda:
+        raise NotImplementedError("linear_rows_hip: vmamba_amd runs on the GPU only")
+    if x.dtype not in _DTYPE_CODE:
+        raise TypeError(f"linear_rows_hip: unsupported dtype {x.dtype}")
+    K = x.shape[-1]
+    if weight.dim() != 2 or weight.shape[1] != K:
+        raise ValueError(f"linear_rows_hip: weight must be (N, {K}), got {tuple(weight.shape)}")
+    N = weight.shape[0]
+    for t, n in ((weight, N * K), (bias, N), (ln_weight, K), (ln_bias, K)):
+        if t is not None and (t.dtype != x.dtype or t.device != x.device or t.numel() != n or not t.is_contiguous()):
+            raise ValueError("linear_rows_hip: contiguous parameters of x's dtype on its device")
+    x = x.contiguous()
+    out = x.new_empty(x.shape[:-1] + (N,))
+    if residual is not None:
+        if residual.shape != out.shape or residual.dtype != x.dtype or residual.device != x.device:
+            raise ValueError("linear_rows_hip: residual must have the shape, dtype and device of the result")
+        residual = residual.contiguous()
+    ptr = lambda t: None if t is None else t.data_ptr()
+    rc = _lib.launch(x, _lib.lib().ss2d_linear_rows, x.data_ptr(), ptr(ln_weight), ptr(ln_bias), float(eps), weight.data_ptr(),
+                     ptr(bias), ptr(residual), out.data_ptr(), x.numel() // K, K, N, int(gelu), _DTYPE_CODE[x.dtype])
+    _lib.check(rc, "ss2d_linear_rows")
     return out
 
 

@@ -18,9 +18,10 @@ from collections import OrderedDict
 import torch
 import torch.nn as nn
 
+from .linear import linear_rows_fusable, linear_rows_hip, linear_rows_takes
 from .mlp import mlp_fusable, mlp_fused_hip
 from .norm import LayerNorm as HipLayerNorm
-from .norm import add_layer_norm_fusable, add_layer_norm_hip, bias_layer_norm_fusable, bias_layer_norm_hip, needs_grad
+from .norm import add_layer_norm_fusable, add_layer_norm_hip, bias_layer_norm_fusable, bias_layer_norm_hip, needs_grad, observed
 from .ss2d import SS2D, HipLayers, Linear2d
 from .pool import GlobalAvgPool2d
 from .stem import stem2_fusable, stem_conv2_ln_hip, stem_conv_ln_gelu_hip, stem_fusable
@@ -95,15 +96,27 @@ class Mlp(nn.Module):
         self.act = nn.GELU()
         self.fc2 = Linear(hidden, dim)
 
-    def takes_norm(self, x):
-        """True when forward runs the fused kernel for x (which then takes the preceding LayerNorm as a prologue)."""
+    def takes_norm(self, x, norm=None):
+        """True when forward runs a fused kernel for x, which then takes the preceding LayerNorm (``norm``) as a prologue."""
+        if norm is not None and self._rows(x, norm):
+            return True
         return (self.fused and not self.channel_first and mlp_fusable(x, self.fc1, self.fc2)
                 and not needs_grad(x, self.fc1.weight, self.fc2.weight, self.fc1.bias, self.fc2.bias))
+
+    def _rows(self, x, norm):
+        """True when two launches of ss2d_linear_rows stand for norm, fc1, act, fc2 and the add on x: few positions."""
+        return (self.fused and not self.channel_first and linear_rows_fusable(x, self.fc1, norm) and type(self.act) is nn.GELU
+                and self.act.approximate == "none" and not observed(self.act) and self.fc2.in_features == self.fc1.out_features
+                and linear_rows_takes(self.fc2, x))
 
     def forward(self, x, residual=None, pre_norm=None):
         """fc2(GELU(fc1(h))) (+ residual), h = x or pre_norm(x) (the block's second LayerNorm, vmamba.py:1229).
         Channel-last 16-bit inference at widths 96 / 192 runs as one HIP kernel that normalises the rows on the way
-        in and keeps the hidden activations in registers; everything else on the torch operators."""
+        in and keeps the hidden activations in registers; few positions behind a norm as two launches of ss2d_linear_rows at
+        any width; everything else on the torch operators."""
+        if pre_norm is not None and self._rows(x, pre_norm):
+            h = linear_rows_hip(x, self.fc1.weight, self.fc1.bias, None, pre_norm.weight, pre_norm.bias, pre_norm.eps, gelu=True)
+            return linear_rows_hip(h, self.fc2.weight, self.fc2.bias, residual)
         if (self.fused and not self.channel_first and mlp_fusable(x, self.fc1, self.fc2)
                 and not needs_grad(x, self.fc1.weight, self.fc2.weight, self.fc1.bias, self.fc2.bias)):
             if pre_norm is None:
@@ -145,7 +158,7 @@ class VSSBlock(nn.Module):
                 pre = None
             else:
                 x = inp = x + pending
-        if self.mlp.takes_norm(x):                    # the fused MLP kernel normalises its input itself
+        if self.mlp.takes_norm(x, self.norm2):        # the fused MLP kernels normalise their input themselves
             x = self.op(inp, residual=x, pre_norm=pre)
             return self.mlp(x, residual=x, pre_norm=self.norm2), None
         x, h = self.op(inp, residual=x, pre_norm=pre, post_norm=self.norm2)
