@@ -1,0 +1,75 @@
+"""A block of few positions as one call (ss2d_block_fwd): the bits of the separate calls, and who is left to them."""
+import pytest
+import torch
+
+from vmamba_amd import vssm
+from vmamba_amd.block import vss_block_hip
+from vmamba_amd.vssm import Mlp, VSSBlock, VSSM
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def make(dim, B, H, W, dtype, **kwargs):
+    torch.manual_seed(dim + H)
+    return (VSSBlock(dim, channel_first=False, **kwargs).to(DEV, dtype).eval(), torch.randn(B, H, W, dim, device=DEV, dtype=dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("dim,B,H,W,kwargs", [
+    (96, 1, 56, 56, {}), (96, 1, 14, 14, {}), (192, 2, 28, 28, {}), (384, 1, 14, 14, {}), (384, 2, 10, 12, {}), (768, 1, 7, 7, {}), (48, 3, 8, 8, {}),
+    (192, 1, 12, 12, dict(ssm_ratio=2.0, mlp_ratio=2.0)), (96, 1, 16, 16, dict(bias=True, conv_bias=True))])
+def test_same_bits(dim, B, H, W, kwargs, dtype, monkeypatch):
+    print("CASE vss_block", dim, B, H, W, kwargs, dtype, flush=True)
+    block, x = make(dim, B, H, W, dtype, **kwargs)
+    kept = x.clone()
+    with torch.no_grad():
+        assert vss_block_hip(block, Mlp, x) is not None
+        got = block(x)
+        monkeypatch.setattr(vssm, "vss_block_hip", lambda *a: None)
+        want = block(x)
+    assert torch.equal(got, want) and torch.equal(x, kept) and got.isfinite().all()
+
+
+def test_who_is_left_to_the_modules():
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    takes = lambda b=block, t=x: vss_block_hip(b, Mlp, t) is not None
+    assert not takes()                                               # autograd
+    with torch.no_grad():
+        assert takes() and not takes(t=x.permute(0, 2, 1, 3)) and not takes(t=x.float()) and not takes(t=x[:, :10, :13].contiguous())
+        assert not takes(t=x.expand(64, 14, 14, 384).contiguous())   # many positions
+        for module in (block.op, block.op.conv2d, block.op.out_norm, block.mlp, block.mlp.fc2, block.norm):
+            handle = module.register_forward_hook(lambda *a: None)
+            assert not takes()
+            handle.remove()
+        block.op.finish_core = lambda *a: None
+        assert not takes()
+        del block.op.finish_core
+        block.mlp.act.approximate = "tanh"
+        assert not takes()
+        block.mlp.act.approximate = "none"
+        with torch.autocast("cuda", torch.bfloat16):
+            assert not takes()
+        assert takes()
+        gated, _ = make(384, 1, 14, 14, torch.bfloat16, disable_z=False)
+        assert not takes(gated)
+
+
+def test_model_replayed_from_a_graph():
+    """Three replays with the program's own work between them, each against the eager call."""
+    torch.manual_seed(1)
+    model = VSSM(depths=(1, 1, 1, 1), channel_first=False, num_classes=16).to(DEV, torch.bfloat16).eval()
+    x = torch.randn(1, 3, 224, 224, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        for _ in range(2):
+            model(x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = model(x)
+        for i in range(3):
+            x.copy_(torch.randn(1, 3, 224, 224, device=DEV))
+            want = model(x)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), i

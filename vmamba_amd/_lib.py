@@ -24,7 +24,7 @@ EXPORTS = ("ss2d_abi_version", "ss2d_strerror", "ss2d_cross_scan", "ss2d_cross_m
            "ss2d_selective_scan_kernel", "ss2d_selective_scan_fwd_maps",
            "ss2d_layer_norm", "ss2d_add_layer_norm", "ss2d_bias_layer_norm", "ss2d_layer_norm_cf", "ss2d_layer_norm_cf_crop", "ss2d_dwconv3x3_silu",
            "ss2d_dwconv3x3_silu_f32", "ss2d_dwconv3x3_silu_bwd", "ss2d_dwconv3x3_silu_bwd_workspace_bytes", "ss2d_cross_scan_1b1", "ss2d_core_fwd",
-           "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_forward_core", "ss2d_forward_core_workspace_bytes", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
+           "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_forward_core", "ss2d_forward_core_workspace_bytes", "ss2d_block_fwd", "ss2d_block_workspace_bytes", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
            "ss2d_x_proj", "ss2d_x_proj_applies", "ss2d_x_proj_f32", "ss2d_dt_proj", "ss2d_dt_proj_f32", "ss2d_dt_proj_masked", "ss2d_cross_scan_flex", "ss2d_cross_scan_flex_ws", "ss2d_cross_scan_flex_static", "ss2d_cross_merge_flex",
            "ss2d_selective_scan_bwd", "ss2d_clear", "ss2d_round_pair", "ss2d_transpose_bcl", "ss2d_mlp_fused", "ss2d_linear_cl", "ss2d_linear_rows", "ss2d_linear_dw_f32", "ss2d_linear_dw_f32_workspace_bytes", "ss2d_linear_cf_ln", "ss2d_stem_conv_ln_gelu", "ss2d_stem_conv2_ln", "ss2d_mean_pool_cl")
 
@@ -76,6 +76,17 @@ class ForwardCoreParams(ctypes.Structure):
         + [("eps", ctypes.c_float)]
         + [(n, ctypes.c_void_p) for n in ("x", "x_proj_weight", "dt_proj_weight", "A", "D", "delta_bias", "norm_weight",
                                           "norm_bias", "pad_mask", "out")]
+    )
+
+
+class BlockParams(ctypes.Structure):
+    """struct ss2d_block_params (include/ss2d_hip.h)."""
+    _fields_ = (
+        [("core", ForwardCoreParams)] + [(n, ctypes.c_int32) for n in ("d_model", "hidden")]
+        + [(n, ctypes.c_float) for n in ("norm_eps", "norm2_eps")]
+        + [(n, ctypes.c_void_p) for n in ("x", "norm_weight", "norm_bias", "in_proj_weight", "in_proj_bias", "conv_weight", "conv_bias",
+                                          "out_proj_weight", "out_proj_bias", "norm2_weight", "norm2_bias", "fc1_weight", "fc1_bias",
+                                          "fc2_weight", "fc2_bias", "out")]
     )
 
 
@@ -152,6 +163,10 @@ def lib():
         L.ss2d_forward_core_workspace_bytes.argtypes = [ctypes.POINTER(ForwardCoreParams)]
         L.ss2d_forward_core.restype = ctypes.c_int
         L.ss2d_forward_core.argtypes = [ctypes.POINTER(ForwardCoreParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+        L.ss2d_block_workspace_bytes.restype = ctypes.c_int64
+        L.ss2d_block_workspace_bytes.argtypes = [ctypes.POINTER(BlockParams)]
+        L.ss2d_block_fwd.restype = ctypes.c_int
+        L.ss2d_block_fwd.argtypes = [ctypes.POINTER(BlockParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
         L.ss2d_core_embed_maps.restype = ctypes.c_int
         L.ss2d_core_embed_maps.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_int,
                                            ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]

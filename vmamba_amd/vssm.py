@@ -18,6 +18,7 @@ from collections import OrderedDict
 import torch
 import torch.nn as nn
 
+from .block import vss_block_hip
 from .linear import linear_rows_fusable, linear_rows_hip, linear_rows_takes
 from .mlp import mlp_fusable, mlp_fused_hip
 from .norm import LayerNorm as HipLayerNorm
@@ -151,6 +152,10 @@ class VSSBlock(nn.Module):
         yet; returns (x, pending) in the same sense.  Deferring the MLP's residual add lets the next block do it
         together with its first LayerNorm in one kernel (ss2d_add_layer_norm); it is only deferred where that kernel
         exists (channel-last 16-bit inference)."""
+        if pending is None:
+            out = vss_block_hip(self, Mlp, x)         # few positions: the whole block as one call
+            if out is not None:
+                return out, None
         inp, pre = x, self.norm
         if pending is not None:
             if self._fusable_add_norm(x, pending, self.norm):
