@@ -381,7 +381,8 @@ int ss2d_forward_core(const ss2d_forward_core_params *params, void *workspace, i
  *   s = x + out_proj(forward_core(silu(conv(in_proj(norm(x))))));   out = s + fc2(GELU(fc1(norm2(s)))).
  * core: the block's core as in ss2d_forward_core, dim the inner width, dtype SS2D_BF16 or SS2D_F16 for all tensors but A, D and
  * delta_bias, norm_* the out_norm; its x, out, normalise and out_channel_last are not looked at, and the map is not padded.
- * x, out (batch, height, width, d_model) contiguous, out not x; in_proj (dim, d_model), conv (dim, 1, 3, 3), out_proj (d_model, dim),
+ * norm_weight NULL: x is norm(x) already, and residual -- otherwise x if NULL -- the block's input.  fc1_weight NULL: out = s.
+ * x, residual, out (batch, height, width, d_model) contiguous, out neither of the others; in_proj (dim, d_model), conv (dim, 1, 3, 3), out_proj (d_model, dim),
  * fc1 (hidden, d_model), fc2 (d_model, hidden); biases NULL or there; 16-byte aligned.  The sizes are those ss2d_linear_rows
  * takes; SS2D_ENOTSUP, also from the size, where one of the kernels has no variant.
  */
@@ -389,7 +390,7 @@ typedef struct ss2d_block_params {
     ss2d_forward_core_params core;
     int32_t d_model, hidden;
     float norm_eps, norm2_eps;
-    const void *x, *norm_weight, *norm_bias, *in_proj_weight, *in_proj_bias, *conv_weight, *conv_bias, *out_proj_weight, *out_proj_bias;
+    const void *x, *residual, *norm_weight, *norm_bias, *in_proj_weight, *in_proj_bias, *conv_weight, *conv_bias, *out_proj_weight, *out_proj_bias;
     const void *norm2_weight, *norm2_bias, *fc1_weight, *fc1_bias, *fc2_weight, *fc2_bias;
     void *out;
 } ss2d_block_params;

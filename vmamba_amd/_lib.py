@@ -84,7 +84,7 @@ class BlockParams(ctypes.Structure):
     _fields_ = (
         [("core", ForwardCoreParams)] + [(n, ctypes.c_int32) for n in ("d_model", "hidden")]
         + [(n, ctypes.c_float) for n in ("norm_eps", "norm2_eps")]
-        + [(n, ctypes.c_void_p) for n in ("x", "norm_weight", "norm_bias", "in_proj_weight", "in_proj_bias", "conv_weight", "conv_bias",
+        + [(n, ctypes.c_void_p) for n in ("x", "residual", "norm_weight", "norm_bias", "in_proj_weight", "in_proj_bias", "conv_weight", "conv_bias",
                                           "out_proj_weight", "out_proj_bias", "norm2_weight", "norm2_bias", "fc1_weight", "fc1_bias",
                                           "fc2_weight", "fc2_bias", "out")]
     )

@@ -1,5 +1,5 @@
 """A channel-last VSS block of few positions as one call into the library (ss2d_block_fwd): LayerNorm + in_proj, depthwise
-convolution + SiLU, forward_core, out_proj + add, LayerNorm + fc1 + GELU, fc2 + add (classification/models/vmamba.py:1225-1229).
+convolution + SiLU, forward_core, out_proj + add, and with fewer still LayerNorm + fc1 + GELU, fc2 + add (classification/models/vmamba.py:1225-1229).
 
 The kernels and results are those of the separate calls; the host's share of a block goes from 100-120 us to about 40, which is what a
 model on a few images waits for.
@@ -9,7 +9,7 @@ import torch.nn as nn
 
 from . import _lib
 from .core import core_fits, padded_map_size
-from .linear import _DTYPE_CODE, linear_rows_pays
+from .linear import _DTYPE_CODE, LINEAR_ROWS_MOST, linear_rows_pays
 from .norm import LayerNorm
 from .ss2d import SS2D, HipLayers
 
@@ -27,8 +27,9 @@ def _plain(module, cls):
     return "forward" not in own and not any(own[name] for name in _HOOKS)
 
 
-def vss_block_hip(block, mlp_cls, x):
-    """``block`` on x (B, H, W, C) as one call, or None where that does not stand for its modules: autograd or autocast, layers
+def vss_block_hip(block, mlp_cls, x, residual=None):
+    """``block`` on x (B, H, W, C) as one call: (block(x), True), or (x + op(norm(x)), False) where the MLP has too many positions for
+    it; with ``residual``, x is norm(residual) already.  None where that does not stand for its modules: autograd or autocast, layers
     of other kinds, types, sizes or memory, too many positions (linear_rows_pays), a map that has to be padded."""
     code = _DTYPE_CODE.get(x.dtype)
     if (code is None or torch.is_grad_enabled() or not x.is_cuda or x.dim() != 4 or not x.is_contiguous() or torch.is_autocast_enabled()
@@ -36,7 +37,7 @@ def vss_block_hip(block, mlp_cls, x):
         return None
     B, H, W, C = x.shape
     M = B * H * W
-    if not linear_rows_pays(M, 4 * C, C):                            # (before the modules are looked at: large batches pay for this line alone)
+    if not 0 < M * C * C <= LINEAR_ROWS_MOST:
         return None
     mods = block._modules
     op, mlp, norm, norm2 = mods["op"], mods["mlp"], mods["norm"], mods["norm2"]
@@ -56,7 +57,9 @@ def vss_block_hip(block, mlp_cls, x):
     own = op._parameters
     x_proj, dt_proj = own["x_proj_weight"], own["dt_projs_weight"]
     index = x.get_device()
-    for t in (x, x_proj, dt_proj, *weight):
+    if residual is not None and residual.shape != x.shape:
+        return None
+    for t in (x, x if residual is None else residual, x_proj, dt_proj, *weight):
         if t is None or t.dtype != x.dtype or t.get_device() != index or not t.is_contiguous() or t.data_ptr() % 16:
             return None
     for t in bias:
@@ -69,10 +72,10 @@ def vss_block_hip(block, mlp_cls, x):
             or tuple(w_c.shape) != (D, 1, 3, 3) or tuple(x_proj.shape) != (4, R + 2, D) or tuple(dt_proj.shape) != (4, D, R) or R == 0
             or conv.padding != (1, 1) or conv.stride != (1, 1) or conv.dilation != (1, 1) or conv.padding_mode != "zeros"):
         return None
-    if (C % 16 or D % 16 or hidden % 16 or C > 768 or D > 3072 or hidden > 3072 or not linear_rows_pays(M, D, C)
-            or not linear_rows_pays(M, C, D) or not linear_rows_pays(M, hidden, C)
+    if (C % 16 or D % 16 or hidden % 16 or C > 768 or D > 3072 or hidden > 3072 or M * D * C > LINEAR_ROWS_MOST
             or not core_fits(H, W, x.dtype) or padded_map_size(H, W, x.dtype) is not None):
         return None
+    whole = linear_rows_pays(M, hidden, C)
     consts = op._inference_constants(0)
     As, Ds, dt_bias = consts["As"], consts["Ds"], consts["dt_bias"]
     for t in (As, Ds, dt_bias):
@@ -83,8 +86,10 @@ def vss_block_hip(block, mlp_cls, x):
     p = _lib.BlockParams(
         _lib.ForwardCoreParams(B, D, H, W, R, H, W, code, code, 1, 1, out_norm.eps, None, x_proj.data_ptr(), dt_proj.data_ptr(), As.data_ptr(),
                                Ds.data_ptr(), dt_bias.data_ptr(), w_on.data_ptr(), ptr[6], None, None),
-        C, hidden, norm.eps, norm2.eps, x.data_ptr(), w_n1.data_ptr(), ptr[4], w_in.data_ptr(), ptr[0], w_c.data_ptr(), ptr[7],
-        w_out.data_ptr(), ptr[1], w_n2.data_ptr(), ptr[5], w_1.data_ptr(), ptr[2], w_2.data_ptr(), ptr[3], out.data_ptr())
+        C, hidden, norm.eps, norm2.eps, x.data_ptr(), None if residual is None else residual.data_ptr(),
+        w_n1.data_ptr() if residual is None else None, ptr[4] if residual is None else None, w_in.data_ptr(), ptr[0], w_c.data_ptr(), ptr[7],
+        w_out.data_ptr(), ptr[1], w_n2.data_ptr(), ptr[5], w_1.data_ptr() if whole else None,
+        ptr[2], w_2.data_ptr() if whole else None, ptr[3], out.data_ptr())
     L = _lib.lib()
     need = L.ss2d_block_workspace_bytes(p)
     if need == _lib.SS2D_ENOTSUP:
@@ -95,4 +100,4 @@ def vss_block_hip(block, mlp_cls, x):
     if rc == _lib.SS2D_ENOTSUP:
         return None
     _lib.check(rc, "ss2d_block_fwd")
-    return out
+    return out, whole

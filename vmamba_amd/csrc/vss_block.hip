@@ -1,5 +1,6 @@
 // A block of few positions as one call (classification/models/vmamba.py:1225-1229): LayerNorm + in_proj, the depthwise convolution,
-// forward_core, out_proj + add, LayerNorm + fc1 + GELU, fc2 + add, enqueued back to back.  The kernels are those of the separate
+// forward_core, out_proj + add, and where the positions are few enough LayerNorm + fc1 + GELU and
+// fc2 + add, enqueued back to back.  The kernels are those of the separate
 // entry points and so are the results; what this saves is the host's share: six calls with their checks, tensors and views took
 // 100-120 us a block from Python, on one image twice the time of the kernels.
 #include "ss2d_common.h"
@@ -8,6 +9,7 @@ namespace ss2d {
 
 struct BlockPlan {
     ss2d_forward_core_params core;
+    bool mlp;                                                        // fc1 and fc2 are there
     bool narrow;                                                     // out_norm + out_proj + add in one kernel (ss2d_linear_cf_ln)
     int64_t proj, conv, mixed, sum, hidden, core_ws, core_bytes, total;   // byte offsets in the workspace; bytes
 };
@@ -17,9 +19,12 @@ static int block_plan(const ss2d_block_params *q, char *base, BlockPlan &p) {
     p.core = q->core;
     if (p.core.dtype != SS2D_BF16 && p.core.dtype != SS2D_F16) return p.core.dtype == SS2D_F32 ? SS2D_ENOTSUP : SS2D_EINVAL;
     if (p.core.batch <= 0 || p.core.height <= 0 || p.core.width <= 0 || p.core.dim <= 0 || q->d_model <= 0 || q->hidden <= 0) return SS2D_EINVAL;
-    if (!q->x || !q->out || !q->norm_weight || !q->in_proj_weight || !q->conv_weight || !q->out_proj_weight || !q->norm2_weight ||
-        !q->fc1_weight || !q->fc2_weight || !p.core.norm_weight)
+    if (!q->x || !q->out || !q->in_proj_weight || !q->conv_weight || !q->out_proj_weight ||
+        !p.core.norm_weight)
         return SS2D_EINVAL;
+    p.mlp = q->fc1_weight != nullptr;
+    if (p.mlp && (!q->fc2_weight || !q->norm2_weight)) return SS2D_EINVAL;
+    if (!q->norm_weight && !q->residual) return SS2D_EINVAL;         // (a normalised x is not the residual stream)
     const int64_t M = (int64_t)p.core.batch * p.core.height * p.core.width, D = p.core.dim;
     auto align = [](int64_t v) { return (v + 255) & ~(int64_t)255; };
     const int64_t L = (int64_t)p.core.height * p.core.width;
@@ -28,8 +33,8 @@ static int block_plan(const ss2d_block_params *q, char *base, BlockPlan &p) {
     p.conv = align(p.proj + M * D * 2);
     p.mixed = align(p.conv + M * D * 2);
     p.sum = align(p.mixed + M * D * (p.narrow ? 4 : 2));
-    p.hidden = align(p.sum + M * q->d_model * 2);
-    p.core_ws = align(p.hidden + M * q->hidden * 2);
+    p.hidden = align(p.sum + (p.mlp ? M * q->d_model * 2 : 0));
+    p.core_ws = align(p.hidden + (p.mlp ? M * q->hidden * 2 : 0));
     char *const at = base ? base : reinterpret_cast<char *>(256);    // (only the size is asked for: stand-ins of the same alignment)
     p.core.x = at + p.conv;
     p.core.out = at + p.mixed;
@@ -60,18 +65,24 @@ extern "C" int ss2d_block_fwd(const ss2d_block_params *q, void *workspace, int64
     const ss2d_forward_core_params &c = p.core;
     const int C = q->d_model, D = c.dim, dt = c.dtype;
     const int64_t M = (int64_t)c.batch * c.height * c.width;
-    rc = ss2d_linear_rows(q->x, q->norm_weight, q->norm_bias, q->norm_eps, q->in_proj_weight, q->in_proj_bias, nullptr, base + p.proj, M, C, D, 0, dt,
-                          stream);
+    const void *residual = q->residual ? q->residual : q->x;
+    void *sum = p.mlp ? base + p.sum : q->out;
+    // 96 -> 96 of many positions: the kernel that holds the weights and walks over tiles (12 544: 8.0 us against 5.0, 25 088: 8.2 / 8.2)
+    if (C == 96 && D == 96 && M > 24576)
+        rc = ss2d_linear_cl(q->x, q->norm_weight, q->norm_bias, q->norm_eps, q->in_proj_weight, q->in_proj_bias, nullptr, base + p.proj, M, C, D, dt, stream);
+    else
+        rc = ss2d_linear_rows(q->x, q->norm_weight, q->norm_bias, q->norm_eps, q->in_proj_weight, q->in_proj_bias, nullptr, base + p.proj, M, C, D, 0, dt,
+                              stream);
     if (rc == SS2D_OK) rc = ss2d_dwconv3x3_silu(base + p.proj, q->conv_weight, q->conv_bias, base + p.conv, c.batch, D, c.height, c.width, dt, 1, 1, stream);
     if (rc == SS2D_OK) rc = ss2d_forward_core(&p.core, base + p.core_ws, p.core_bytes, stream);
     if (rc == SS2D_OK && p.narrow)
-        rc = ss2d_linear_cf_ln(base + p.mixed, c.norm_weight, c.norm_bias, c.eps, q->out_proj_weight, q->out_proj_bias, q->x, base + p.sum, c.batch,
+        rc = ss2d_linear_cf_ln(base + p.mixed, c.norm_weight, c.norm_bias, c.eps, q->out_proj_weight, q->out_proj_bias, residual, sum, c.batch,
                                c.height * c.width, D, C, dt, stream);
     else if (rc == SS2D_OK)
-        rc = ss2d_linear_rows(base + p.mixed, nullptr, nullptr, 0.0f, q->out_proj_weight, q->out_proj_bias, q->x, base + p.sum, M, D, C, 0, dt, stream);
-    if (rc == SS2D_OK)
-        rc = ss2d_linear_rows(base + p.sum, q->norm2_weight, q->norm2_bias, q->norm2_eps, q->fc1_weight, q->fc1_bias, nullptr, base + p.hidden, M, C,
-                              q->hidden, 1, dt, stream);
+        rc = ss2d_linear_rows(base + p.mixed, nullptr, nullptr, 0.0f, q->out_proj_weight, q->out_proj_bias, residual, sum, M, D, C, 0, dt, stream);
+    if (rc != SS2D_OK || !p.mlp) return rc;
+    rc = ss2d_linear_rows(base + p.sum, q->norm2_weight, q->norm2_bias, q->norm2_eps, q->fc1_weight, q->fc1_bias, nullptr, base + p.hidden, M, C,
+                          q->hidden, 1, dt, stream);
     if (rc == SS2D_OK)
         rc = ss2d_linear_rows(base + p.hidden, nullptr, nullptr, 0.0f, q->fc2_weight, q->fc2_bias, base + p.sum, q->out, M, q->hidden, C, 0, dt, stream);
     return rc;

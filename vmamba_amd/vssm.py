@@ -19,7 +19,7 @@ import torch
 import torch.nn as nn
 
 from .block import vss_block_hip
-from .linear import linear_rows_fusable, linear_rows_hip, linear_rows_takes
+from .linear import few_positions, linear_rows_fusable, linear_rows_hip, linear_rows_takes
 from .mlp import mlp_fusable, mlp_fused_hip
 from .norm import LayerNorm as HipLayerNorm
 from .norm import add_layer_norm_fusable, add_layer_norm_hip, bias_layer_norm_fusable, bias_layer_norm_hip, needs_grad, observed
@@ -99,7 +99,7 @@ class Mlp(nn.Module):
 
     def takes_norm(self, x, norm=None):
         """True when forward runs a fused kernel for x, which then takes the preceding LayerNorm (``norm``) as a prologue."""
-        if norm is not None and self._rows(x, norm):
+        if norm is not None and few_positions(x) and self._rows(x, norm):
             return True
         return (self.fused and not self.channel_first and mlp_fusable(x, self.fc1, self.fc2)
                 and not needs_grad(x, self.fc1.weight, self.fc2.weight, self.fc1.bias, self.fc2.bias))
@@ -115,7 +115,7 @@ class Mlp(nn.Module):
         Channel-last 16-bit inference at widths 96 / 192 runs as one HIP kernel that normalises the rows on the way
         in and keeps the hidden activations in registers; few positions behind a norm as two launches of ss2d_linear_rows at
         any width; everything else on the torch operators."""
-        if pre_norm is not None and self._rows(x, pre_norm):
+        if pre_norm is not None and few_positions(x) and self._rows(x, pre_norm):
             h = linear_rows_hip(x, self.fc1.weight, self.fc1.bias, None, pre_norm.weight, pre_norm.bias, pre_norm.eps, gelu=True)
             return linear_rows_hip(h, self.fc2.weight, self.fc2.bias, residual)
         if (self.fused and not self.channel_first and mlp_fusable(x, self.fc1, self.fc2)
@@ -152,10 +152,6 @@ class VSSBlock(nn.Module):
         yet; returns (x, pending) in the same sense.  Deferring the MLP's residual add lets the next block do it
         together with its first LayerNorm in one kernel (ss2d_add_layer_norm); it is only deferred where that kernel
         exists (channel-last 16-bit inference)."""
-        if pending is None:
-            out = vss_block_hip(self, Mlp, x)         # few positions: the whole block as one call
-            if out is not None:
-                return out, None
         inp, pre = x, self.norm
         if pending is not None:
             if self._fusable_add_norm(x, pending, self.norm):
@@ -163,10 +159,21 @@ class VSSBlock(nn.Module):
                 pre = None
             else:
                 x = inp = x + pending
+        native = vss_block_hip(self, Mlp, inp, x if pre is None else None) if few_positions(x) else None       # as one call
+        if native is not None:
+            x, whole = native
+            if whole:
+                return x, None
+            if self.mlp.takes_norm(x, self.norm2):
+                return self.mlp(x, residual=x, pre_norm=self.norm2), None
+            return self._pending_mlp(x, self.norm2(x))
         if self.mlp.takes_norm(x, self.norm2):        # the fused MLP kernels normalise their input themselves
             x = self.op(inp, residual=x, pre_norm=pre)
             return self.mlp(x, residual=x, pre_norm=self.norm2), None
         x, h = self.op(inp, residual=x, pre_norm=pre, post_norm=self.norm2)
+        return self._pending_mlp(x, h)
+
+    def _pending_mlp(self, x, h):
         m = self.mlp(h)
         if self._fusable_add_norm(x, m, self.norm):
             return x, m
