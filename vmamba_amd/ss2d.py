@@ -116,6 +116,7 @@ def _pad_mask(H0, W0, H, W, n_images, device):
     return mask
 
 
+_CORE_PARAMS = ("A_logs", "Ds", "dt_projs_bias", "x_proj_weight", "dt_projs_weight")
 _CORE_STEPS = ("forward_core_fused", "finish_core", "_inference_constants")      # what SS2D._forward_core_native stands for
 
 
@@ -166,11 +167,12 @@ class SS2D(nn.Module):
         missing during a capture is computed inside the graph (its memory then belongs to the graph and is rewritten by
         every replay) and is not kept.  Pinned entries are copies of the parameter values at capture time: whoever
         replays the graph must not do so after an in-place parameter update (ConcurrentGraphRunner.replay checks)."""
-        params = (self.A_logs, self.Ds, self.dt_projs_bias, self.x_proj_weight, self.dt_projs_weight)
+        own = self._parameters                 # (the names themselves go through Module.__getattr__, five times a call)
+        params = [own[n] if n in own else getattr(self, n) for n in _CORE_PARAMS]
         key = (batch, torch.is_grad_enabled(), tuple((p._version, p.data_ptr(), p.dtype, p.device) for p in params))
         cache = self.__dict__.setdefault("_const_cache", {})
         pinned = self.__dict__.setdefault("_pinned_consts", {})
-        capturing = self.A_logs.is_cuda and torch.cuda.is_current_stream_capturing()
+        capturing = params[0].is_cuda and torch.cuda.is_current_stream_capturing()
         if key in pinned:
             return pinned[key]
         if key in cache:
