@@ -221,3 +221,19 @@ def test_forward_core_says_what_it_takes():
         assert bytes_of(**kw) > 0, kw
     for kw in refused:
         assert bytes_of(**kw) == _lib.SS2D_ENOTSUP, kw
+
+
+def test_forward_core_of_more_positions_than_the_folded_step_takes():
+    """Ranks beyond 32-bit offsets of the core with dt_proj folded in: the plan takes the separate kernels, whose room includes delta
+    (4 x 48 channels), instead of finding out behind x_proj."""
+    p = _lib.ForwardCoreParams(batch=0, dim=48, height=56, width=56, rank=6, padded_height=56, padded_width=56, dtype=_lib.SS2D_BF16,
+                               norm_dtype=_lib.SS2D_BF16, normalise=1, eps=1e-5)
+    for name in ("x", "x_proj_weight", "dt_proj_weight", "A", "D", "delta_bias", "norm_weight", "norm_bias", "out"):
+        setattr(p, name, 4096)
+    most = (2 ** 31 - 1) // (4 * 15 * 56 * 56)               # 3 directions of 4 planes' room, two planes and the positions of one
+    for batch, folded in ((most, True), (most + 1, False)):
+        p.batch = batch
+        positions = batch * 56 * 56
+        need, plain = _lib.lib().ss2d_forward_core_workspace_bytes(p), positions * (4 * 8 * 2 + 48 * 4)    # projections, y
+        delta = positions * 4 * 48 * 2
+        assert plain <= need < plain + delta // 4 if folded else need >= plain + delta, (batch, need)

@@ -71,7 +71,7 @@ static int forward_core_plan(const ss2d_forward_core_params *q, char *base, Forw
         const int planes = dts_planes(q->rank, p.padded);
         rows(2 * planes + 2);
         p.flags_per_image = x_proj_pairs_workgroups(q->batch, q->dim, q->rank, q->padded_height, q->padded_width, q->dtype);
-        if (p.flags_per_image > 0 && core_dts_takes(&c, q->rank, p.padded, p.layout)) p.planes = planes;
+        if (p.flags_per_image > 0 && core_dts_takes(&c, q->rank, p.padded, (planes + 1) * p.pitch, p.pitch, p.layout)) p.planes = planes;
     }
     if (p.planes > 0) {
         p.delta = align256(p.flags + (int64_t)q->batch * p.flags_per_image * 4);

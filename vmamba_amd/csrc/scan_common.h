@@ -69,7 +69,7 @@ int64_t core_tiled_workspace_bytes(const CoreArgs &a);
 int launch_core_tiled(const CoreArgs &a, int in_dtype, void *workspace, hipStream_t stream);
 
 // ss2d_core.hip: the core with dt_proj folded in.  Rows of `dts` (x_proj_pairs) in place of delta; `delta` in q is not read.
-// core_dts_takes: from sizes, types and the alignment of B and C alone.
+// core_dts_takes: from sizes, strides (of the rows, in dwords), types and the alignment of B and C alone.
 struct CoreDts {
     const void *dts, *weight;
     int64_t dir_stride, pair_stride;    // dwords
@@ -78,7 +78,7 @@ struct CoreDts {
     const int32_t *flags;
     int32_t flags_per_image;
 };
-bool core_dts_takes(const ss2d_core_params *q, int rank, bool padded, DtsLayout &layout);
+bool core_dts_takes(const ss2d_core_params *q, int rank, bool padded, int64_t dir_stride, int64_t pair_stride, DtsLayout &layout);
 int core_dts_fwd(const ss2d_core_params *q, const CoreDts &t, hipStream_t stream);
 
 // ---- 8-wide loads / stores ------------------------------------------------------------

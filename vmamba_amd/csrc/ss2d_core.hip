@@ -977,10 +977,16 @@ static int core_launch_single(const CoreArgs &a, int in_dtype, hipStream_t s) {
     return launch_core<f16_t>(a, s);
 }
 
-bool core_dts_takes(const ss2d_core_params *q, int rank, bool padded, DtsLayout &layout) {
+// bytes from the first of the ranks' dwords to behind the last
+static int64_t dts_span(const ss2d_core_params *q, int planes, int64_t dir_stride, int64_t pair_stride) {
+    return 4 * (3 * dir_stride + (planes - 1) * pair_stride + (int64_t)q->batch * q->height * q->width);
+}
+
+bool core_dts_takes(const ss2d_core_params *q, int rank, bool padded, int64_t dir_stride, int64_t pair_stride, DtsLayout &layout) {
     CoreArgs a;
     if (core_args(q, a) != SS2D_OK || q->in_dtype == SS2D_F32 || !a.softplus || a.dl_bs != a.L || a.B_bs != a.L || a.C_bs != a.L) return false;
     const int planes = dts_planes(rank, padded);
+    if (dts_span(q, planes, dir_stride, pair_stride) >= 0x7fffffff) return false;      // (32-bit offsets in the kernel)
     if (planes < 2 || planes > kCoreMostPairs || core_small_eligible(a, q->in_dtype) || !core_fits_lds<bf16_t>(a) ||
         core_granularity<bf16_t>(a) != kItems) return false;
     bool wide;
@@ -993,22 +999,16 @@ bool core_dts_takes(const ss2d_core_params *q, int rank, bool padded, DtsLayout 
     return a.L % layout.per_lane == 0 && (smem <= kCorePairLds || (wide && planes <= 2));
 }
 
-// bytes from the first of the ranks' dwords to behind the last
-static int64_t dts_span(const CoreDts &t, const ss2d_core_params *q) {
-    return 4 * (3 * t.dir_stride + (dts_planes(t.rank, t.pad_weight != 0) - 1) * t.pair_stride + (int64_t)q->batch * q->height * q->width);
-}
-
 int core_dts_fwd(const ss2d_core_params *q, const CoreDts &t, hipStream_t stream) {
     DtsLayout layout;
-    if (!core_dts_takes(q, t.rank, t.pad_weight != 0, layout)) return SS2D_ENOTSUP;
-    if (dts_span(t, q) >= 0x7fffffff) return SS2D_ENOTSUP;
+    if (!core_dts_takes(q, t.rank, t.pad_weight != 0, t.dir_stride, t.pair_stride, layout)) return SS2D_ENOTSUP;
     if (!t.dts || !t.weight || !t.flags || reinterpret_cast<uintptr_t>(t.dts) % 16 != 0 || t.dir_stride % 4 != 0 || t.pair_stride % 4 != 0) return SS2D_EINVAL;
     CoreArgs a;
     const int rc = core_args(q, a);
     if (rc != SS2D_OK) return rc;
     a.dts = (const uint32_t *)t.dts; a.Wdt = (const uint16_t *)t.weight;
     a.dts_flags = t.flags; a.flags_per_image = t.flags_per_image;
-    a.dts_span_bytes = (uint32_t)dts_span(t, q);
+    a.dts_span_bytes = (uint32_t)dts_span(q, dts_planes(t.rank, t.pad_weight != 0), t.dir_stride, t.pair_stride);
     a.dts_ks = t.dir_stride; a.dts_ps = t.pair_stride; a.rank = t.rank; a.pad_weight = t.pad_weight;
     return q->in_dtype == SS2D_BF16 ? launch_core<bf16_t>(a, stream) : launch_core<f16_t>(a, stream);
 }
