@@ -96,3 +96,41 @@ def test_model_replayed_from_a_graph():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want), i
+
+
+class Seen(torch.Tensor):
+    """A weight that sees the operators it is in, as quantised and sharded ones do."""
+    functions = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.functions.append(getattr(func, "__name__", ""))
+        with torch._C.DisableTorchFunctionSubclass():
+            return func(*args, **(kwargs or {}))
+
+
+def test_weights_of_other_kinds_are_left_to_torch():
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    with torch.no_grad():
+        want = block(x)
+        own = block.op.in_proj._parameters
+        own["weight"] = own["weight"].detach().as_subclass(Seen)
+        assert vss_block_hip(block, Mlp, x) is None
+        got = block(x)
+        assert "linear" in Seen.functions
+        # in_proj's sum is the library's on one side: 16 u, as in test_same_bits
+        assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 16 * 2.0 ** -8
+
+
+@pytest.mark.parametrize("layer", ["fc1", "fc2"])
+def test_bias_that_torch_broadcasts(layer):
+    """One element in the place of a row: the kernels read a row."""
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    mod = getattr(block.mlp, layer)
+    with torch.no_grad():
+        mod.bias = torch.nn.Parameter(torch.full((mod.out_features,), 0.5, device=DEV, dtype=torch.bfloat16))
+        want = block(x)
+        mod.bias = torch.nn.Parameter(torch.full((1,), 0.5, device=DEV, dtype=torch.bfloat16))
+        assert vss_block_hip(block, Mlp, x) is None
+        got = block(x)
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 16 * 2.0 ** -8

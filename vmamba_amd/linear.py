@@ -44,17 +44,23 @@ def linear_cl_hip(x, weight, bias=None, residual=None, ln_weight=None, ln_bias=N
     return out
 
 
+# Other kinds of tensors (quantised or sharded weights, subclasses that see the calls they are in) are left to torch's operators.
+_TENSORS = (torch.Tensor, nn.Parameter)
+
+
 def _rows_params(x, *params):
-    return all(t is None or (t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0) for t in params)
+    """True for (tensor or None, elements) whose memory the kernels can read as it is; a bias that torch would broadcast is not."""
+    return all(t is None or (type(t) in _TENSORS and t.dtype == x.dtype and t.device == x.device and t.numel() == n and t.is_contiguous()
+                             and t.data_ptr() % 16 == 0) for t, n in params)
 
 
 def linear_rows_takes(layer, x):
     """True when ss2d_linear_rows stands for this layer at inference on rows of x's type and device: a plain nn.Linear that nothing
     observes, its parameters of x's own 16-bit dtype."""
-    if type(layer) is not nn.Linear or not x.is_cuda or x.dtype not in _DTYPE_CODE:
+    if type(layer) is not nn.Linear or type(x) not in _TENSORS or not x.is_cuda or x.dtype not in _DTYPE_CODE:
         return False
     N, K = layer.weight.shape
-    return (K % 16 == 0 and 0 < K <= 3072 and N % 8 == 0 and _rows_params(x, layer.weight, layer.bias)
+    return (K % 16 == 0 and 0 < K <= 3072 and N % 8 == 0 and _rows_params(x, (layer.weight, N * K), (layer.bias, N))
             and not needs_grad(x, layer.weight, layer.bias) and not observed(layer) and not torch.is_autocast_enabled())
 
 
@@ -67,7 +73,7 @@ def linear_rows_fusable(x, layer, norm=None):
     if not (linear_rows_takes(layer, x) and tuple(layer.weight.shape) == (layer.out_features, K) and x.is_contiguous() and x.data_ptr() % 16 == 0):
         return False
     return norm is None or (type(norm) is LayerNorm and norm.normalized_shape == (K,) and K <= 768 and norm.weight is not None
-                            and _rows_params(x, norm.weight, norm.bias) and not needs_grad(norm.weight, norm.bias) and not observed(norm))
+                            and _rows_params(x, (norm.weight, K), (norm.bias, K)) and not needs_grad(norm.weight, norm.bias) and not observed(norm))
 
 
 LINEAR_ROWS_MOST = 448 << 20             # M N K of a projection
