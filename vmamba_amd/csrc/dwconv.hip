@@ -318,7 +318,7 @@ __global__ __launch_bounds__(kBlock) void dwconv3x3_rows_kernel(const T *__restr
 }
 
 // Plane variant of the channel-last kernel: the layout change happens on the way INTO LDS instead of on the way out.
-// A workgroup owns TH full rows x kCh channels (32 or 64, i.e. runs of 64 or 128 bytes per position).  The input rows
+// A workgroup owns TH full rows x kCh channels (32 or 64, i.e. runs of 64 or 128 bytes per position; 8 for few images).  The input rows
 // (with halo) are fetched as 16-byte channel vectors, two neighbouring positions per lane, and written into one LDS plane
 // per channel as dwords holding TWO NEIGHBOURING POSITIONS of that channel (one byte permute per channel and pair):
 // a plane is the zero-padded image rows of one channel, [TH + 2][pitch], padded column 0 = image column -1.
@@ -708,13 +708,25 @@ static int launch_dwconv(const void *x, const void *w, const void *bias, void *y
         // (channel-first input takes the same kernel with element-wise staging: no alignment asked of x)
         if (D % 32 == 0 && (W <= 120 || seg_t > 0) && (al16(x) || !in_channel_last) && al16(y) &&
             (int64_t)H * W * D * 2 < 0x7ffffff0ll) {
-            const int kch = D % 64 == 0 ? 64 : 32, lpc = kBlock / kch;
+            int kch = D % 64 == 0 ? 64 : 32, lpc = kBlock / kch;
             const int TW = seg_t > 0 ? 8 * seg_t : W, col_tiles = seg_t > 0 ? W / TW : 1;
             const int nseg = (TW + 7) / 8, pitch = 8 * nseg + 4;
+            const int flat_out = W % 4 != 0;
             int TH = (7 * lpc) / nseg;
             TH = TH > H ? H : TH;
+            // Few images: 6 workgroups of 64 channels for 384 x 14 x 14, each lane with seven segments one after the other.  Tiles of 8
+            // channels and one segment per lane instead, the same sums; 16 bytes of a position's channels per workgroup are fetched
+            // from the L2 then, which loses once the chip is full.  us, standard split -> this one, bf16, in a graph: 96 x 56 x 56
+            // 1 image 6.2 -> 3.1, 4 images (84 workgroups) 6.5 -> 4.4, 8 (168) 6.8 -> 7.3; 192 x 28 x 28 8 images (96) 6.8 -> 4.3,
+            // 16 (192) 7.3 -> 8.4; 384 x 14 x 14 1 image 7.5 -> 3.5, 16 (96) 7.9 -> 4.9, 32 (192) 8.4 -> 9.1; with no more than two
+            // segments per lane there is less to win: 768 x 7 x 7 1 image 4.1 -> 3.5, 4 (48) 4.2 -> 4.1, 8 (96) 4.2 -> 4.4.
+            if (TH >= 1 && in_channel_last && col_tiles == 1 && (!flat_out || TH == H) &&
+                (int64_t)B * ((H + TH - 1) / TH) * (D / kch) < (TH * nseg > 2 * lpc ? 128 : 64)) {
+                kch = 8; lpc = kBlock / kch;
+                TH = (flat_out ? 7 * lpc : lpc) / nseg;           // whole images, or rows for one segment per lane
+                TH = TH > H ? H : TH;
+            }
             const int row_tiles = TH >= 1 ? (H + TH - 1) / TH : 0, ch_tiles = D / kch;
-            const int flat_out = W % 4 != 0;
             const int n_it = TH >= 1 ? (TH * nseg + lpc - 1) / lpc : 0;
             int plane_dw = (TH + 2) * pitch / 2;
             const int want = kch == 64 ? 1 : 2;                    // see plane_at
@@ -728,7 +740,8 @@ static int launch_dwconv(const void *x, const void *w, const void *bias, void *y
                        (const T *)w, (const T *)bias, (T *)y, D, H, W, TH, row_tiles, ch_tiles, col_tiles, TW, pitch, plane_dw,  \
                        nseg, n_it, flat_out, in_channel_last ? 0 : 1, make_fastdiv((uint32_t)(pitch / 2)),                     \
                        make_fastdiv((uint32_t)nseg), make_fastdiv((uint32_t)((TH + 2) * (pitch / 2))))
-                if (kch == 64) { if (apply_silu) SS2D_DW_PLANES(true, 64); else SS2D_DW_PLANES(false, 64); }
+                if (kch == 8) { if (apply_silu) SS2D_DW_PLANES(true, 8); else SS2D_DW_PLANES(false, 8); }
+                else if (kch == 64) { if (apply_silu) SS2D_DW_PLANES(true, 64); else SS2D_DW_PLANES(false, 64); }
                 else { if (apply_silu) SS2D_DW_PLANES(true, 32); else SS2D_DW_PLANES(false, 32); }
 #undef SS2D_DW_PLANES
                 return launch_status();
