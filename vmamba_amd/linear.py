@@ -80,8 +80,8 @@ LINEAR_ROWS_MOST = 448 << 20             # M N K of a projection
 
 
 def few_positions(x):
-    """False where no square product of x's width can be linear_rows': asked first, so that large batches pay for nothing else."""
-    return x.numel() * x.shape[-1] <= LINEAR_ROWS_MOST
+    """False where no square product of x's type and width can be linear_rows': asked first, so that others pay for nothing else."""
+    return x.dtype in _DTYPE_CODE and x.numel() * x.shape[-1] <= LINEAR_ROWS_MOST
 
 
 def linear_rows_pays(M, N, K):
