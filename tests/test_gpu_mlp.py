@@ -9,6 +9,7 @@ import torch.nn.functional as F
 
 from vmamba_amd import _lib
 from vmamba_amd.mlp import mlp_fused_hip
+from vmamba_amd.norm import LayerNorm
 from vmamba_amd.vssm import Mlp
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +100,36 @@ def test_mlp_fused_rejections():
     assert L.ss2d_mlp_fused(x.data_ptr(), None, b2.data_ptr(), 1e-5, w1.data_ptr(), None, w2.data_ptr(), None, None, x.data_ptr(), 8, 96,
                             _lib.SS2D_BF16, None) == _lib.SS2D_EINVAL          # LayerNorm bias without weight
     assert mlp_fused_hip(x[:0], w1, b1, w2, b2, res[:0]).shape == (0, 96)
+
+
+class Seen(torch.Tensor):
+    """A tensor of a kind of its own."""
+
+
+@pytest.mark.parametrize("C", [96, 192, 384])
+@pytest.mark.parametrize("with_norm", [False, True])
+@pytest.mark.parametrize("kind", ["gradient", "single precision", "one row", "between 16-byte boundaries", "subclass"])
+def test_residuals_that_the_kernels_cannot_add(C, with_norm, kind):
+    """They are added by torch behind the kernels, as ``residual + y`` says: the same bits as that sum, and the gradient."""
+    print("CASE mlp residual", C, with_norm, kind, flush=True)
+    torch.manual_seed(C)
+    m = Mlp(C, 4 * C, channel_first=False).to(DEV).bfloat16().eval().requires_grad_(False)
+    norm = LayerNorm(C).to(DEV).bfloat16().requires_grad_(False) if with_norm else None
+    x = torch.randn(2, 5, 7, C, device=DEV).bfloat16()
+    r = torch.randn_like(x)
+    if kind == "gradient":
+        r.requires_grad_(True)
+    elif kind == "single precision":
+        r = r.float()
+    elif kind == "one row":
+        r = r[0, 0, 0].clone()
+    elif kind == "subclass":
+        r = r.as_subclass(Seen)
+    else:
+        r = torch.cat([r.new_zeros(1), r.flatten()])[1:].view(x.shape)
+    got, want = m(x, residual=r, pre_norm=norm), r + m(x, pre_norm=norm)
+    assert got.dtype == want.dtype and torch.equal(got, want) and type(got) is type(want)
+    assert got.requires_grad == (kind == "gradient")
+    if got.requires_grad:
+        got.float().sum().backward()
+        assert torch.equal(r.grad, torch.ones_like(r))

@@ -9,7 +9,7 @@ import torch.nn as nn
 
 from . import _lib
 from .core import core_fits, padded_map_size
-from .linear import _DTYPE_CODE, _TENSORS, LINEAR_ROWS_MOST, linear_rows_pays
+from .linear import _DTYPE_CODE, TENSOR_KINDS, LINEAR_ROWS_MOST, linear_rows_pays
 from .norm import LayerNorm
 from .ss2d import SS2D, HipLayers
 
@@ -60,12 +60,12 @@ def vss_block_hip(block, mlp_cls, x, residual=None):
     if residual is not None and residual.shape != x.shape:
         return None
     for t in (x, x if residual is None else residual, x_proj, dt_proj, *weight):
-        if t is None or type(t) not in _TENSORS or t.dtype != x.dtype or t.get_device() != index or not t.is_contiguous() or t.data_ptr() % 16:
+        if t is None or type(t) not in TENSOR_KINDS or t.dtype != x.dtype or t.get_device() != index or not t.is_contiguous() or t.data_ptr() % 16:
             return None
     w_in, w_out, w_1, w_2, w_n1, w_n2, w_on, w_c = weight
     D, hidden, R = w_in.shape[0], w_1.shape[0], dt_proj.shape[2]
     for t, n in zip(bias, (D, C, hidden, C, C, C, D, D)):           # (torch would broadcast one of another size)
-        if t is not None and (type(t) not in _TENSORS or t.numel() != n or t.dtype != x.dtype or t.get_device() != index
+        if t is not None and (type(t) not in TENSOR_KINDS or t.numel() != n or t.dtype != x.dtype or t.get_device() != index
                               or not t.is_contiguous() or t.data_ptr() % 16):
             return None
     if (tuple(w_in.shape) != (D, C) or tuple(w_out.shape) != (C, D) or tuple(w_1.shape) != (hidden, C) or tuple(w_2.shape) != (C, hidden)

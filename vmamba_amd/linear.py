@@ -45,19 +45,19 @@ def linear_cl_hip(x, weight, bias=None, residual=None, ln_weight=None, ln_bias=N
 
 
 # Other kinds of tensors (quantised or sharded weights, subclasses that see the calls they are in) are left to torch's operators.
-_TENSORS = (torch.Tensor, nn.Parameter)
+TENSOR_KINDS = (torch.Tensor, nn.Parameter)
 
 
 def _rows_params(x, *params):
     """True for (tensor or None, elements) whose memory the kernels can read as it is; a bias that torch would broadcast is not."""
-    return all(t is None or (type(t) in _TENSORS and t.dtype == x.dtype and t.device == x.device and t.numel() == n and t.is_contiguous()
+    return all(t is None or (type(t) in TENSOR_KINDS and t.dtype == x.dtype and t.device == x.device and t.numel() == n and t.is_contiguous()
                              and t.data_ptr() % 16 == 0) for t, n in params)
 
 
 def linear_rows_takes(layer, x):
     """True when ss2d_linear_rows stands for this layer at inference on rows of x's type and device: a plain nn.Linear that nothing
     observes, its parameters of x's own 16-bit dtype."""
-    if type(layer) is not nn.Linear or type(x) not in _TENSORS or not x.is_cuda or x.dtype not in _DTYPE_CODE:
+    if type(layer) is not nn.Linear or type(x) not in TENSOR_KINDS or not x.is_cuda or x.dtype not in _DTYPE_CODE:
         return False
     N, K = layer.weight.shape
     return (K % 16 == 0 and 0 < K <= 3072 and N % 8 == 0 and _rows_params(x, (layer.weight, N * K), (layer.bias, N))

@@ -19,7 +19,7 @@ import torch
 import torch.nn as nn
 
 from .block import vss_block_hip
-from .linear import few_positions, linear_rows_fusable, linear_rows_hip, linear_rows_takes
+from .linear import TENSOR_KINDS, few_positions, linear_rows_fusable, linear_rows_hip, linear_rows_takes
 from .mlp import mlp_fusable, mlp_fused_hip
 from .norm import LayerNorm as HipLayerNorm
 from .norm import add_layer_norm_fusable, add_layer_norm_hip, bias_layer_norm_fusable, bias_layer_norm_hip, needs_grad, observed
@@ -114,22 +114,31 @@ class Mlp(nn.Module):
         """fc2(GELU(fc1(h))) (+ residual), h = x or pre_norm(x) (the block's second LayerNorm, vmamba.py:1229).
         Channel-last 16-bit inference at widths 96 / 192 runs as one HIP kernel that normalises the rows on the way
         in and keeps the hidden activations in registers; few positions behind a norm as two launches of ss2d_linear_rows at
-        any width; everything else on the torch operators."""
-        if pre_norm is not None and few_positions(x) and self._rows(x, pre_norm):
+        any width; everything else on the torch operators.  A residual that the kernels cannot add -- one that autograd has to
+        see, of another shape, type, device or kind -- is added by torch behind them."""
+        rows = pre_norm is not None and few_positions(x) and self._rows(x, pre_norm)
+        one = (not rows and self.fused and not self.channel_first and mlp_fusable(x, self.fc1, self.fc2)
+               and not needs_grad(x, self.fc1.weight, self.fc2.weight, self.fc1.bias, self.fc2.bias)
+               and (pre_norm is None or (isinstance(pre_norm, nn.LayerNorm) and pre_norm.elementwise_affine
+                                         and not needs_grad(pre_norm.weight, pre_norm.bias))))
+        if (rows or one) and residual is not None and residual is not x and not self._adds(x, residual):
+            return residual + self.forward(x, None, pre_norm)
+        if rows:
             h = linear_rows_hip(x, self.fc1.weight, self.fc1.bias, None, pre_norm.weight, pre_norm.bias, pre_norm.eps, gelu=True)
             return linear_rows_hip(h, self.fc2.weight, self.fc2.bias, residual)
-        if (self.fused and not self.channel_first and mlp_fusable(x, self.fc1, self.fc2)
-                and not needs_grad(x, self.fc1.weight, self.fc2.weight, self.fc1.bias, self.fc2.bias)):
-            if pre_norm is None:
-                return mlp_fused_hip(x, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias, residual)
-            if (isinstance(pre_norm, nn.LayerNorm) and pre_norm.elementwise_affine
-                    and not needs_grad(pre_norm.weight, pre_norm.bias)):
-                return mlp_fused_hip(x, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias, residual,
-                                     pre_norm.weight, pre_norm.bias, pre_norm.eps)
+        if one:
+            norm = () if pre_norm is None else (pre_norm.weight, pre_norm.bias, pre_norm.eps)
+            return mlp_fused_hip(x, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias, residual, *norm)
         if pre_norm is not None:
             x = pre_norm(x)
         y = self.fc2(self.act(self.fc1(x)))
         return y if residual is None else residual + y
+
+    @staticmethod
+    def _adds(x, residual):
+        """True when the kernels' own addition stands for ``residual + y``, y of x's shape and type."""
+        return (type(residual) in TENSOR_KINDS and residual.shape == x.shape and residual.dtype == x.dtype and residual.device == x.device
+                and not needs_grad(residual) and (residual.data_ptr() % 16 == 0 or not residual.is_contiguous()))
 
 
 class VSSBlock(nn.Module):
