@@ -128,3 +128,17 @@ def test_block_of_few_positions_under_capture():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want), i
+
+
+@pytest.mark.parametrize("layer", ["fc1", "act", "fc2"])
+def test_layers_of_another_kind(layer):
+    """A layer wrapped in a module that has nothing of nn.Linear's is called: the block gives what the layers give."""
+    torch.manual_seed(11)
+    block = VSSBlock(384, channel_first=False).to(DEV, torch.bfloat16).eval()
+    x = torch.randn(1, 14, 14, 384, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        want = block(x)
+        setattr(block.mlp, layer, torch.nn.Sequential(getattr(block.mlp, layer), torch.nn.Dropout(0.5).eval()))
+        got = block(x)
+    # the layers are the library's on one side: 16 u, as in test_block_of_few_positions
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 16 * U[torch.bfloat16]

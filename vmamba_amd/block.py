@@ -40,15 +40,15 @@ def vss_block_hip(block, mlp_cls, x, residual=None):
     if not 0 < M * C * C <= LINEAR_ROWS_MOST:
         return None
     mods = block._modules
-    op, mlp, norm, norm2 = mods["op"], mods["mlp"], mods["norm"], mods["norm2"]
+    op, mlp, norm, norm2 = (mods.get(name) for name in ("op", "mlp", "norm", "norm2"))
     if not (_plain(op, SS2D) and _plain(mlp, mlp_cls) and _plain(norm, LayerNorm) and _plain(norm2, LayerNorm)):
         return None
     if (op.layers is not HipLayers or op.channel_first or mlp.channel_first or not mlp.fused or not op.fused_core or not op.disable_z
             or op.d_state != 1 or not vars(op).keys().isdisjoint(_STEPS) or tuple(getattr(SS2D, name) for name in _STEPS) != _CLASS_STEPS):
         return None
     inner = op._modules
-    in_proj, conv, out_norm, out_proj = inner["in_proj"], inner.get("conv2d"), inner["out_norm"], inner["out_proj"]
-    fc1, act, fc2 = (mlp._modules[name] for name in ("fc1", "act", "fc2"))
+    in_proj, conv, out_norm, out_proj = (inner.get(name) for name in ("in_proj", "conv2d", "out_norm", "out_proj"))
+    fc1, act, fc2 = (mlp._modules.get(name) for name in ("fc1", "act", "fc2"))
     if not (all(_plain(layer, nn.Linear) for layer in (in_proj, out_proj, fc1, fc2)) and _plain(conv, nn.Conv2d) and _plain(out_norm, LayerNorm)
             and _plain(act, nn.GELU) and act.approximate == "none"):
         return None

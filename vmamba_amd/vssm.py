@@ -107,8 +107,8 @@ class Mlp(nn.Module):
     def _rows(self, x, norm):
         """True when two launches of ss2d_linear_rows stand for norm, fc1, act, fc2 and the add on x: few positions."""
         return (self.fused and not self.channel_first and linear_rows_fusable(x, self.fc1, norm) and type(self.act) is nn.GELU
-                and self.act.approximate == "none" and not observed(self.act) and self.fc2.in_features == self.fc1.out_features
-                and linear_rows_takes(self.fc2, x))
+                and self.act.approximate == "none" and not observed(self.act) and linear_rows_takes(self.fc2, x)
+                and self.fc2.weight.shape[1] == self.fc1.out_features)
 
     def forward(self, x, residual=None, pre_norm=None):
         """fc2(GELU(fc1(h))) (+ residual), h = x or pre_norm(x) (the block's second LayerNorm, vmamba.py:1229).
