@@ -1,9 +1,13 @@
 """A block of few positions as one call (ss2d_block_fwd): the bits of the separate calls, and who is left to them."""
 import pytest
 import torch
+from torch.autograd import forward_ad
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from vmamba_amd import vssm
 from vmamba_amd.block import vss_block_hip
+from vmamba_amd.norm import LayerNorm
 from vmamba_amd.vssm import Mlp, VSSBlock, VSSM
 
 pytestmark = pytest.mark.gpu
@@ -134,3 +138,66 @@ def test_bias_that_torch_broadcasts(layer):
         assert vss_block_hip(block, Mlp, x) is None
         got = block(x)
     assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 16 * 2.0 ** -8
+
+
+class Functions(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(getattr(func, "__name__", ""))
+        return func(*args, **(kwargs or {}))
+
+
+class Operators(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(func.overloadpacket.__name__)
+        return func(*args, **(kwargs or {}))
+
+
+def test_modes_see_the_products_of_few_positions():
+    """Flop counters and loggers see the library's calls at widths whose layers are plain torch ones; the mode behind torch.device does
+    not look at them and changes nothing."""
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    with torch.no_grad():
+        want = block(x)
+        with Functions() as functions:
+            got = block(x)
+        assert functions.names.count("linear") == 4 and "gelu" in functions.names
+        with Operators() as operators:
+            again = block(x)
+        assert sum(name in ("mm", "addmm", "linear") for name in operators.names) >= 4 and "gelu" in operators.names
+        assert torch.equal(got, again)
+        with torch.device(DEV):
+            assert vss_block_hip(block, Mlp, x) is not None and torch.equal(block(x), want)
+    # in_proj, out_proj and the MLP are the library's on one side: 16 u, as in test_same_bits
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 16 * 2.0 ** -8
+
+
+@pytest.mark.parametrize("cls", [torch.nn.Linear, torch.nn.GELU, LayerNorm])
+def test_forward_replaced_on_a_class(cls, monkeypatch):
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    calls, forward = [], cls.forward
+    monkeypatch.setattr(cls, "forward", lambda self, *a: calls.append(self) or forward(self, *a))
+    with torch.no_grad():
+        block(x)
+    layers = {torch.nn.Linear: (block.op.in_proj, block.mlp.fc1, block.mlp.fc2), torch.nn.GELU: (block.mlp.act,),
+              LayerNorm: (block.norm,)}[cls]                 # (norm2 is in the add's kernel, as at every number of positions)
+    assert all(any(call is layer for call in calls) for layer in layers)
+
+
+def test_forward_mode_derivatives_of_the_mlp():
+    """A tangent of fc2's weight goes through torch's product."""
+    mlp = Mlp(384, 1536, channel_first=False).to(DEV, torch.bfloat16).eval()
+    norm = LayerNorm(384).to(DEV, torch.bfloat16)
+    x = torch.randn(1, 14, 14, 384, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad(), forward_ad.dual_level():
+        own = mlp.fc2._parameters
+        own["weight"] = forward_ad.make_dual(own["weight"].detach(), torch.ones_like(own["weight"]))
+        tangent = forward_ad.unpack_dual(mlp(x, pre_norm=norm)).tangent
+    assert tangent is not None and tangent.isfinite().all() and tangent.any()

@@ -262,3 +262,35 @@ def test_single_call_core_leaves_steps_of_an_instance_alone(monkeypatch):
             setattr(op, step, getattr(op, step))
             assert op._forward_core_native(x, True) is None
             delattr(op, step)
+
+
+def test_operators_seen():
+    """What may see or replace the operators that modules call, and what does not."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    from vmamba_amd.norm import operators_seen
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert not operators_seen()
+    for context in (Functions(), FlopCounterMode(display=False), forward_ad.dual_level()):
+        with context:
+            assert operators_seen()
+    with torch.device("cpu"):
+        assert not operators_seen()
+        with Functions():
+            assert operators_seen()
+    seen = []
+    for transform in (torch.func.vmap(lambda t: seen.append(operators_seen()) or t), torch.func.grad(lambda t: seen.append(operators_seen()) or t.sum())):
+        transform(torch.ones(2))
+    assert seen == [True, True]
+    forward = torch.nn.Linear.forward
+    try:
+        torch.nn.Linear.forward = lambda self, x: forward(self, x)
+        assert operators_seen()
+    finally:
+        torch.nn.Linear.forward = forward
+    assert not operators_seen()

@@ -10,7 +10,7 @@ import torch.nn as nn
 from . import _lib
 from .core import core_fits, padded_map_size
 from .linear import _DTYPE_CODE, TENSOR_KINDS, LINEAR_ROWS_MOST, linear_rows_pays
-from .norm import LayerNorm
+from .norm import LayerNorm, operators_seen
 from .ss2d import SS2D, HipLayers
 
 # what the call stands for: replaced on the class or the instance, they are called instead
@@ -29,11 +29,11 @@ def _plain(module, cls):
 
 def vss_block_hip(block, mlp_cls, x, residual=None):
     """``block`` on x (B, H, W, C) as one call: (block(x), True), or (x + op(norm(x)), False) where the MLP has too many positions for
-    it; with ``residual``, x is norm(residual) already.  None where that does not stand for its modules: autograd or autocast, layers
-    of other kinds, types, sizes or memory, too many positions (linear_rows_pays), a map that has to be padded."""
+    it; with ``residual``, x is norm(residual) already.  None where that does not stand for its modules: autograd, autocast or operators
+    that something sees, layers of other kinds, types, sizes or memory, too many positions (linear_rows_pays), a map that has to be padded."""
     code = _DTYPE_CODE.get(x.dtype)
     if (code is None or torch.is_grad_enabled() or not x.is_cuda or x.dim() != 4 or not x.is_contiguous() or torch.is_autocast_enabled()
-            or nn.modules.module._has_any_global_hook()):
+            or nn.modules.module._has_any_global_hook() or operators_seen()):
         return None
     B, H, W, C = x.shape
     M = B * H * W

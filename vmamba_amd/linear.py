@@ -9,7 +9,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .norm import LayerNorm, needs_grad, observed
+from .norm import LayerNorm, needs_grad, observed, operators_seen
 
 _DTYPE_CODE = {torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 FUSED_SHAPES = ((96, 96),)            # (in_features, out_features)
@@ -56,8 +56,8 @@ def _rows_params(x, *params):
 
 def linear_rows_takes(layer, x):
     """True when ss2d_linear_rows stands for this layer at inference on rows of x's type and device: a plain nn.Linear that nothing
-    observes, its parameters of x's own 16-bit dtype."""
-    if type(layer) is not nn.Linear or type(x) not in TENSOR_KINDS or not x.is_cuda or x.dtype not in _DTYPE_CODE:
+    observes, its parameters of x's own 16-bit dtype, and operators that nothing sees."""
+    if type(layer) is not nn.Linear or type(x) not in TENSOR_KINDS or not x.is_cuda or x.dtype not in _DTYPE_CODE or operators_seen():
         return False
     N, K = layer.weight.shape
     return (K % 16 == 0 and 0 < K <= 3072 and N % 8 == 0 and _rows_params(x, (layer.weight, N * K), (layer.bias, N))

@@ -7,6 +7,8 @@ torch modules, so state_dicts are interchangeable.  GPU tensors only: there is n
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -139,3 +141,21 @@ class LayerNorm2d(nn.LayerNorm):
         if needs_grad(x, self.weight, self.bias):          # vmamba.py:52-57
             return F.layer_norm(x.permute(0, 2, 3, 1), self.normalized_shape, self.weight, self.bias, self.eps).permute(0, 3, 1, 2)
         return layer_norm_cf_hip(x, self.weight, self.bias, self.eps, out_channel_last=False)
+
+
+_MODES = torch._C._len_torch_dispatch_stack, torch._C._functorch.peek_interpreter_stack, torch._C._len_torch_function_stack
+_CALLS = (nn.Linear.forward, nn.GELU.forward, LayerNorm.forward, F.linear, F.gelu)
+
+
+def operators_seen():
+    """True when the operators that modules call may be seen or replaced, so that a kernel standing for library calls would go past
+    it: an active TorchDispatchMode or TorchFunctionMode (flop counters, loggers; not the one behind torch.device and
+    set_default_device, which only looks at factories), forward-mode derivatives, torch.func's transforms, or another forward or
+    function in the place of torch's or this package's own."""
+    dispatch, transforms, functions = _MODES
+    if dispatch() or forward_ad._current_level >= 0 or transforms() is not None:
+        return True
+    modes = functions()
+    if modes and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes)):
+        return True
+    return (nn.Linear.forward, nn.GELU.forward, LayerNorm.forward, F.linear, F.gelu) != _CALLS
