@@ -203,3 +203,53 @@ def test_forward_mode_derivatives_of_the_mlp():
         own["weight"] = forward_ad.make_dual(own["weight"].detach(), torch.ones_like(own["weight"]))
         tangent = forward_ad.unpack_dual(mlp(x, pre_norm=norm)).tangent
     assert tangent is not None and tangent.isfinite().all() and tangent.any()
+
+
+class FormerMlp(Mlp):
+    """Knows neither a norm to ask for nor one to take."""
+
+    def takes_norm(self, x):
+        return False
+
+    def forward(self, x):
+        self.seen = x
+        return super().forward(x)
+
+
+def test_mlp_of_another_kind_is_called_with_the_normalised_rows():
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    with torch.no_grad():
+        want = block(x)
+        former = FormerMlp(384, 1536, channel_first=False).to(DEV, torch.bfloat16).eval()
+        former.load_state_dict(block.mlp.state_dict())
+        block.mlp = former
+        got = block(x)
+    # norm2's result: centred rows
+    assert former.seen.shape == x.shape and former.seen.float().mean(-1).abs().max() < 1e-2
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 16 * 2.0 ** -8          # as in test_same_bits
+
+
+@pytest.mark.parametrize("how", ["hook", "class"])
+def test_calls_of_the_mlp_are_the_same_with_few_positions(how, monkeypatch):
+    """What sees or replaces the MLP's calls gets norm2's result and nothing else, as it does with many positions."""
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    seen, forward = [], Mlp.forward
+    if how == "hook":
+        block.mlp.register_forward_pre_hook(lambda module, args, kwargs: seen.append((args, kwargs)), with_kwargs=True)
+    else:
+        monkeypatch.setattr(Mlp, "forward", lambda self, *a, **k: seen.append((a, k)) or forward(self, *a, **k))
+    with torch.no_grad():
+        block(x)
+        block(x.expand(32, 14, 14, 384).contiguous())
+    assert [(len(args), list(kwargs)) for args, kwargs in seen] == [(1, []), (1, [])]
+    assert all(args[0].float().mean(-1).abs().max() < 1e-2 for args, _ in seen)
+
+
+def test_hooks_of_op_get_what_they_get_with_many_positions():
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    seen = []
+    block.op.register_forward_hook(lambda module, args, out: seen.append(type(out)))
+    with torch.no_grad():
+        block(x)
+        block(x.expand(32, 14, 14, 384).contiguous())
+    assert seen == [tuple, tuple]
