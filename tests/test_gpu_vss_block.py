@@ -253,3 +253,13 @@ def test_hooks_of_op_get_what_they_get_with_many_positions():
         block(x)
         block(x.expand(32, 14, 14, 384).contiguous())
     assert seen == [tuple, tuple]
+
+
+def test_residual_of_another_kind_is_added_by_torch():
+    block, x = make(384, 1, 14, 14, torch.bfloat16)
+    Seen.functions.clear()
+    with torch.no_grad():
+        want, got = block.op(x, residual=x), block.op(x, residual=x.as_subclass(Seen))
+    assert "reshape" in Seen.functions                               # into torch's addmm
+    # two orders of one projection's sum, each rounded once
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 2 * 2.0 ** -8

@@ -27,7 +27,7 @@ from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_fits, core_mask_
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
 from .conv import DwConv3x3SiLU, dwconv3x3_silu_hip, dwconv_silu_trainable
-from .linear import LinearDw, few_positions, linear_cf_ln_fusable, linear_cf_ln_hip, linear_cl_hip, linear_dw_pays, linear_fusable, linear_rows_fusable, linear_rows_hip
+from .linear import TENSOR_KINDS, LinearDw, few_positions, linear_cf_ln_fusable, linear_cf_ln_hip, linear_cl_hip, linear_dw_pays, linear_fusable, linear_rows_fusable, linear_rows_hip
 from .norm import (LayerNorm, LayerNorm2d, add_layer_norm_fusable, add_layer_norm_hip, layer_norm_cf_hip,
                    needs_grad)
 
@@ -435,7 +435,7 @@ class SS2D(nn.Module):
         y = self.forward_core(x)
         if z is not None:
             y = y * z
-        if (few and residual is not None and not self.channel_first and residual.dtype == y.dtype and residual.device == y.device
+        if (few and residual is not None and not self.channel_first and type(residual) in TENSOR_KINDS and residual.dtype == y.dtype and residual.device == y.device
                 and residual.shape == y.shape[:-1] + (self.out_proj.out_features,)
                 and residual.data_ptr() % 16 == 0 and not needs_grad(residual) and linear_rows_fusable(y, self.out_proj)):
             return linear_rows_hip(y, self.out_proj.weight, self.out_proj.bias, residual)
