@@ -237,3 +237,40 @@ def test_forward_core_of_more_positions_than_the_folded_step_takes():
         need, plain = _lib.lib().ss2d_forward_core_workspace_bytes(p), positions * (4 * 8 * 2 + 48 * 4)    # projections, y
         delta = positions * 4 * 48 * 2
         assert plain <= need < plain + delta // 4 if folded else need >= plain + delta, (batch, need)
+
+
+def test_block_says_what_it_takes():
+    """Whatever one of the block's kernels refuses, the workspace query and the call refuse before anything is launched."""
+    L = _lib.lib()
+    BF16 = _lib.SS2D_BF16
+
+    def both(core={}, **kw):
+        p = _lib.BlockParams(core=_lib.ForwardCoreParams(batch=2, dim=64, height=8, width=8, rank=4, padded_height=8, padded_width=8, dtype=BF16,
+                                                         norm_dtype=BF16, eps=1e-5), d_model=64, hidden=256, norm_eps=1e-5, norm2_eps=1e-5)
+        for name in ("x_proj_weight", "dt_proj_weight", "A", "D", "delta_bias", "norm_weight", "norm_bias"):
+            setattr(p.core, name, 4096)
+        for name, kind in p._fields_:
+            if kind is ctypes.c_void_p and name != "residual":
+                setattr(p, name, 4096)
+        for name, value in core.items():
+            setattr(p.core, name, value)
+        for name, value in kw.items():
+            setattr(p, name, value)
+        # (no room: a call that is taken ends with SS2D_ENOMEM, before any launch)
+        return L.ss2d_block_workspace_bytes(p), L.ss2d_block_fwd(p, 4096, 0, None)
+
+    taken = [{}, dict(d_model=768, hidden=3072), dict(fc1_weight=None, hidden=4096), dict(hidden=272), dict(norm_bias=None, fc2_bias=None),
+             dict(norm_weight=None, norm_bias=None, residual=4096, d_model=784, fc1_weight=None), dict(core=dict(dtype=_lib.SS2D_F16, norm_dtype=_lib.SS2D_F16))]
+    refused = [dict(d_model=100), dict(d_model=392), dict(d_model=784), dict(d_model=8), dict(hidden=100), dict(hidden=264), dict(hidden=3088), dict(hidden=4096),
+               dict(core=dict(dim=72)), dict(core=dict(dim=3088)), dict(core=dict(rank=49)), dict(core=dict(dtype=_lib.SS2D_F32)),
+               dict(core=dict(norm_weight=4104)), *(dict([(name, 4104)]) for name in ("x", "residual", "in_proj_weight", "in_proj_bias", "out_proj_weight",
+                                                                                      "norm2_bias", "fc1_weight", "fc2_weight", "fc2_bias", "out"))]
+    wrong = [dict(x=None), dict(out=None), dict(fc2_weight=None), dict(norm2_weight=None), dict(norm_weight=None, norm_bias=None), dict(d_model=0), dict(hidden=-1),
+             dict(norm_weight=None, residual=4096), dict(core=dict(batch=0)), dict(core=dict(norm_weight=None))]
+    for kw in taken:
+        need, rc = both(**kw)
+        assert need > 0 and rc == _lib.SS2D_ENOMEM, kw
+    for kw in refused:
+        assert both(**kw) == (_lib.SS2D_ENOTSUP, _lib.SS2D_ENOTSUP), kw
+    for kw in wrong:
+        assert both(**kw) == (_lib.SS2D_EINVAL, _lib.SS2D_EINVAL), kw

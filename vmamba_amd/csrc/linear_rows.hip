@@ -159,10 +159,11 @@ static void launch_rows(const RowsArgs &a, bool gelu, uint32_t n_wg, hipStream_t
                 : launch_rows_ln<T, kPer, kMaxThreads, false, false>(a, gelu, n_wg, stream);
 }
 
+static int64_t rows_grid(int64_t M, int N) { return (M + kRowsTile - 1) / kRowsTile * ((N + kRowsTile - 1) / kRowsTile); }
+
 template <typename T>
 static int launch_rows_for(const RowsArgs &a, bool gelu, hipStream_t stream) {
-    const int64_t n_wg = (a.M + kRowsTile - 1) / kRowsTile * a.n_tiles;
-    if (n_wg > 0x7fffffff) return SS2D_ENOTSUP;
+    const int64_t n_wg = rows_grid(a.M, a.N);
     const int steps = a.K / 16;
     // up to 4 wavefronts of 3 steps, 8 or 16 of 6, 16 of 12: the shares a wavefront holds in registers at once
     if (steps <= 12) launch_rows<T, 3, 256, true>(a, gelu, (uint32_t)n_wg, stream);
@@ -170,6 +171,11 @@ static int launch_rows_for(const RowsArgs &a, bool gelu, hipStream_t stream) {
     else if (steps <= 96) launch_rows<T, 6, 1024, false>(a, gelu, (uint32_t)n_wg, stream);
     else launch_rows<T, 12, 1024, false>(a, gelu, (uint32_t)n_wg, stream);
     return launch_status();
+}
+
+bool linear_rows_takes(int64_t M, int K, int N, bool layer_norm, int dtype) {
+    return dtype != SS2D_F32 && K % 16 == 0 && K <= 3072 && N % 8 == 0 && (!layer_norm || K <= 16 * 6 * kRowsMaxLnWaves) &&
+           rows_grid(M, N) <= 0x7fffffff;
 }
 
 }  // namespace ss2d
@@ -181,7 +187,7 @@ extern "C" int ss2d_linear_rows(const void *x, const void *ln_weight, const void
     if (dtype != SS2D_F32 && dtype != SS2D_BF16 && dtype != SS2D_F16) return SS2D_EINVAL;
     if (M == 0) return SS2D_OK;
     if (!x || !weight || !out || (ln_bias && !ln_weight)) return SS2D_EINVAL;
-    if (dtype == SS2D_F32 || K % 16 != 0 || K > 3072 || N % 8 != 0 || (ln_weight && K > 16 * 6 * kRowsMaxLnWaves)) return SS2D_ENOTSUP;
+    if (!linear_rows_takes(M, K, N, ln_weight != nullptr, dtype)) return SS2D_ENOTSUP;
     const void *ptrs[] = {x, ln_weight, ln_bias, weight, bias, residual, out};
     for (const void *q : ptrs)
         if (q && (reinterpret_cast<uintptr_t>(q) & 15u) != 0) return SS2D_ENOTSUP;

@@ -221,10 +221,11 @@ __device__ __forceinline__ void layer_norm_tile_rows(uint16_t *tile, int pitch, 
 }
 
 // What the entry points of other files take, from the sizes and types alone (ss2d_dt_proj_masked, ss2d_dt_proj_f32,
-// ss2d_layer_norm_cf): for callers that launch several kernels and have to know before the first.
+// ss2d_layer_norm_cf, ss2d_linear_rows): for callers that launch several kernels and have to know before the first.
 bool dt_proj_takes(int D, int R, int64_t N, int64_t x_rank_stride, int dtype);
 bool dt_proj_f32_takes(int R);
 bool layer_norm_cf_takes(int C, int in_dtype, int w_dtype, int out_dtype);
+bool linear_rows_takes(int64_t M, int K, int N, bool layer_norm, int dtype);
 
 // ss2d_x_proj for one state per channel with the step's ranks in pairs, as the core with dt_proj folded in reads them
 // (core_dts_fwd): per direction ceil((R + padded) / 2) planes of dwords, low half rank 2 p, high half rank 2 p + 1 -- zero where

@@ -14,6 +14,19 @@ struct BlockPlan {
     int64_t proj, conv, mixed, sum, hidden, core_ws, core_bytes, total;   // byte offsets in the workspace; bytes
 };
 
+// What a kernel of the block refuses is found here, before a caller has allocated or launched anything.
+static bool block_kernels_take(const ss2d_block_params *q, int64_t M) {
+    const int C = q->d_model, D = q->core.dim, hidden = q->hidden, dt = q->core.dtype;
+    const void *const ptrs[] = {q->x, q->residual, q->norm_weight, q->norm_bias, q->in_proj_weight, q->in_proj_bias, q->core.norm_weight, q->core.norm_bias,
+                                q->out_proj_weight, q->out_proj_bias, q->norm2_weight, q->norm2_bias, q->fc1_weight, q->fc1_bias, q->fc2_weight,
+                                q->fc2_bias, q->out};
+    for (const void *at : ptrs)
+        if (reinterpret_cast<uintptr_t>(at) % 16 != 0) return false;
+    if ((int64_t)q->core.height * q->core.width > 0x3fffffff) return false;                       // the convolution's
+    return linear_rows_takes(M, C, D, q->norm_weight != nullptr, dt) && linear_rows_takes(M, D, C, false, dt) &&
+           (!q->fc1_weight || (linear_rows_takes(M, C, hidden, true, dt) && linear_rows_takes(M, hidden, C, false, dt)));
+}
+
 static int block_plan(const ss2d_block_params *q, char *base, BlockPlan &p) {
     if (!q) return SS2D_EINVAL;
     p.core = q->core;
@@ -25,7 +38,9 @@ static int block_plan(const ss2d_block_params *q, char *base, BlockPlan &p) {
     p.mlp = q->fc1_weight != nullptr;
     if (p.mlp && (!q->fc2_weight || !q->norm2_weight)) return SS2D_EINVAL;
     if (!q->norm_weight && !q->residual) return SS2D_EINVAL;         // (a normalised x is not the residual stream)
+    if (q->norm_bias && !q->norm_weight) return SS2D_EINVAL;
     const int64_t M = (int64_t)p.core.batch * p.core.height * p.core.width, D = p.core.dim;
+    if (!block_kernels_take(q, M)) return SS2D_ENOTSUP;
     auto align = [](int64_t v) { return (v + 255) & ~(int64_t)255; };
     const int64_t L = (int64_t)p.core.height * p.core.width;
     p.narrow = q->d_model == 96 && D == 96 && L % 32 == 0 && p.core.norm_dtype == p.core.dtype;
