@@ -7,22 +7,53 @@ from torch.utils._python_dispatch import TorchDispatchMode
 
 from vmamba_amd import vssm
 from vmamba_amd.block import vss_block_hip
-from vmamba_amd.norm import LayerNorm
+from vmamba_amd.conv import dwconv3x3_silu_hip
+from vmamba_amd.linear import linear_cf_ln_hip, linear_cl_hip, linear_rows_hip
+from vmamba_amd.norm import LayerNorm, add_layer_norm_hip
 from vmamba_amd.vssm import Mlp, VSSBlock, VSSM
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def make(dim, B, H, W, dtype, **kwargs):
+def unlike_norms(block, biases=True):
+    """Norms that cannot stand in for one another, nor be applied twice: weights, biases and eps of their own."""
+    with torch.no_grad():
+        for norm, eps in ((block.norm, 1e-5), (block.norm2, 3e-2), (block.op.out_norm, 4e-1)):
+            norm.eps = eps
+            norm.weight.uniform_(0.5, 1.5)
+            norm.bias.uniform_(-0.5, 0.5)
+            if not biases:
+                norm.bias = None
+    return block
+
+
+def make(dim, B, H, W, dtype, norm_biases=True, **kwargs):
     torch.manual_seed(dim + H)
-    return (VSSBlock(dim, channel_first=False, **kwargs).to(DEV, dtype).eval(), torch.randn(B, H, W, dim, device=DEV, dtype=dtype))
+    block = VSSBlock(dim, channel_first=False, **kwargs).to(DEV, dtype).eval()
+    return unlike_norms(block, norm_biases), torch.randn(B, H, W, dim, device=DEV, dtype=dtype)
+
+
+def one_by_one(block, x, residual=None):
+    """What the call gives without the MLP -- x + op(norm(x)), or residual + op(x) with x normalised already -- from its kernels."""
+    op, norm = block.op, block.norm
+    ln = (norm.weight, norm.bias, norm.eps) if residual is None else ()
+    walk = x.shape[-1] == op.d_inner == 96 and x.numel() > 24576 * 96
+    project = linear_cl_hip if walk else linear_rows_hip
+    h = project(x, op.in_proj.weight, op.in_proj.bias, None, *ln)
+    h = dwconv3x3_silu_hip(h, op.conv2d.weight, op.conv2d.bias, in_channel_last=True, apply_silu=True)
+    add, out = x if residual is None else residual, op.out_proj
+    if x.shape[-1] == op.d_inner == 96 and x.shape[1] * x.shape[2] % 32 == 0:
+        y = op._forward_core_native(h, False)
+        return linear_cf_ln_hip(y, op.out_norm.weight, op.out_norm.bias, op.out_norm.eps, out.weight, out.bias, add).view(x.shape)
+    return project(op.forward_core(h), out.weight, out.bias, add)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("dim,B,H,W,kwargs", [
     (96, 1, 56, 56, {}), (96, 1, 14, 14, {}), (192, 2, 28, 28, {}), (384, 1, 14, 14, {}), (384, 2, 10, 12, {}), (768, 1, 7, 7, {}), (48, 3, 8, 8, {}),
-    (384, 8, 14, 14, {}), (768, 8, 7, 7, {}), (96, 8, 56, 56, {}), (96, 8, 60, 62, {}), (192, 8, 28, 28, {}), (192, 1, 12, 12, dict(ssm_ratio=2.0, mlp_ratio=2.0)), (96, 1, 16, 16, dict(bias=True, conv_bias=True))])
+    (384, 8, 14, 14, {}), (768, 8, 7, 7, {}), (96, 8, 56, 56, {}), (96, 8, 60, 62, {}), (192, 8, 28, 28, {}), (192, 1, 12, 12, dict(ssm_ratio=2.0, mlp_ratio=2.0)), (96, 1, 16, 16, dict(bias=True, conv_bias=True)),
+    (96, 1, 14, 14, dict(norm_biases=False)), (384, 1, 14, 14, dict(norm_biases=False)), (384, 8, 14, 14, dict(bias=True, norm_biases=False))])
 def test_same_bits(dim, B, H, W, kwargs, dtype, monkeypatch):
     print("CASE vss_block", dim, B, H, W, kwargs, dtype, flush=True)
     block, x = make(dim, B, H, W, dtype, **kwargs)
@@ -32,7 +63,16 @@ def test_same_bits(dim, B, H, W, kwargs, dtype, monkeypatch):
         got = block(x)
         monkeypatch.setattr(vssm, "vss_block_hip", lambda *a: None)
         want = block(x)
-        whole = vss_block_hip(block, Mlp, x)[1]
+        native, whole = vss_block_hip(block, Mlp, x)
+        if not whole:
+            assert torch.equal(native, one_by_one(block, x))
+        normalised, stream = torch.randn_like(x), torch.randn_like(x)
+        beside = vss_block_hip(block, Mlp, normalised, stream)
+        if not whole:
+            assert torch.equal(beside[0], one_by_one(block, normalised, stream))
+        else:
+            s = one_by_one(block, normalised, stream)
+            assert torch.equal(beside[0], block.mlp(s, residual=s, pre_norm=block.norm2))
     assert torch.equal(x, kept) and got.isfinite().all()
     if whole or dim <= 192:
         assert torch.equal(got, want)
@@ -43,19 +83,27 @@ def test_same_bits(dim, B, H, W, kwargs, dtype, monkeypatch):
 
 @pytest.mark.parametrize("dim,B,side", [(384, 8, 14), (768, 6, 7)])
 def test_blocks_with_the_mlp_left_to_the_library(dim, B, side, monkeypatch):
-    """The first block leaves its MLP's sum to the second's LayerNorm, whose result the call takes beside the residual stream."""
+    """The first block leaves its MLP's sum to the second's LayerNorm, whose result the call takes beside the residual stream: the
+    bits of the kernels and the library's MLPs one by one."""
     torch.manual_seed(dim)
     stage = vssm.BlockSequence(*[VSSBlock(dim, channel_first=False) for _ in range(3)]).to(DEV, torch.bfloat16).eval()
+    for block in stage:
+        unlike_norms(block)
     x = torch.randn(B, side, side, dim, device=DEV, dtype=torch.bfloat16)
     calls = []
     with torch.no_grad():
         monkeypatch.setattr(vssm, "vss_block_hip", lambda *a: calls.append(vss_block_hip(*a)) or calls[-1])
         got = stage(x)
         assert len(calls) == 3 and all(c is not None and not c[1] for c in calls)
-        monkeypatch.setattr(vssm, "vss_block_hip", lambda *a: None)
-        want = stage(x)
-    # three blocks whose residual stream may round the other way at each of their six sums and products: 16 u each at most
-    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 3 * 16 * 2.0 ** -8
+        stream, term = x, None
+        for block in stage:
+            if term is None:
+                stream = one_by_one(block, stream)
+            else:
+                total, h = add_layer_norm_hip(term, stream, block.norm.weight, block.norm.bias, block.norm.eps)
+                stream = one_by_one(block, h, total)
+            term = block.mlp(block.norm2(stream))
+    assert torch.equal(got, stream + term)
 
 
 def test_who_is_left_to_the_modules():
@@ -218,6 +266,8 @@ class FormerMlp(Mlp):
 
 def test_mlp_of_another_kind_is_called_with_the_normalised_rows():
     block, x = make(384, 1, 14, 14, torch.bfloat16)
+    torch.nn.init.zeros_(block.norm2.bias)
+    torch.nn.init.ones_(block.norm2.weight)
     with torch.no_grad():
         want = block(x)
         former = FormerMlp(384, 1536, channel_first=False).to(DEV, torch.bfloat16).eval()
@@ -233,6 +283,8 @@ def test_mlp_of_another_kind_is_called_with_the_normalised_rows():
 def test_calls_of_the_mlp_are_the_same_with_few_positions(how, monkeypatch):
     """What sees or replaces the MLP's calls gets norm2's result and nothing else, as it does with many positions."""
     block, x = make(384, 1, 14, 14, torch.bfloat16)
+    torch.nn.init.zeros_(block.norm2.bias)
+    torch.nn.init.ones_(block.norm2.weight)
     seen, forward = [], Mlp.forward
     if how == "hook":
         block.mlp.register_forward_pre_hook(lambda module, args, kwargs: seen.append((args, kwargs)), with_kwargs=True)
