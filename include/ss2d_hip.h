@@ -355,11 +355,13 @@ int ss2d_core_fwd_ws(const ss2d_core_params *params, void *workspace, int64_t wo
 /*
  * SS2Dv2.forward_corev2 of a one-state block (classification/models/vmamba.py:603-646) in one call: ss2d_x_proj, ss2d_dt_proj,
  * ss2d_core_fwd_ws and -- with `normalise` -- ss2d_layer_norm_cf as out_norm, enqueued on `stream` (fp32: the _f32 projections).
+ * 16-bit maps of 2^19 elements or more and up to 8 ranks (7 padded) may take dt_proj into the core instead, where the step's sums stay in fp32.
  *   x (B,D,H,W); x_proj_weight (4, rank + 2, D); dt_proj_weight (4, D, rank), all of `dtype`; A, D, delta_bias (4*D) fp32
  *   out   normalise: (B,D,L), or (B,L,D) if out_channel_last, of `dtype`; else the merged map (B,D,L) fp32
  *   norm_weight, norm_bias (D) of norm_dtype or NULL
  *   padded_height, padded_width   the map's own size, or a larger one to embed it in (ss2d_core_embed_maps; 16-bit types), with
- *         pad_mask as ss2d_dt_proj_masked takes it for the (4, batch * padded positions) in scan order; the result is cropped
+ *         pad_mask as ss2d_dt_proj_masked takes it for the (4, batch * padded positions) in scan order (asked for also where dt_proj
+ *         is in the core, which does not read it); the result is cropped
  * Everything contiguous.  workspace: ss2d_forward_core_workspace_bytes(params) bytes, 16-byte aligned, contents irrelevant;
  * workspace_bytes depends on the sizes and types, and on the pointers' alignment.  Either function returns SS2D_ENOTSUP where
  * one of the kernels has no variant for the problem.

@@ -29,8 +29,9 @@ static bool forward_core_kernels_take(const ss2d_forward_core_params *q, int64_t
 
 // Elements of the map from which dt_proj is folded into the core where the core takes that (core_dts_takes): 96 x 56 x 56, batch 128,
 // bf16 292 -> 234 us, 64 x 96 x 96, batch 33 225 -> 177, 48 x 96 maps of 57 x 58, fp16 159 -> 150, 54 x 128 x 8 x 9 (0.5 Mi elements)
-// 26 -> 22.  Below it, where a call is bound by its launches (0.1 Mi elements, in a graph: 18.4 -> 16.2), the separate kernels keep
-// one result with the calls that take them one by one.
+// 26 -> 22.  Below it a call is bound by its launches and the host, there is less to win (0.1 Mi elements, in a graph: 18.4 -> 16.2),
+// and small calls keep the bits of the kernels one by one.  The line is one of rounding too: above it the step is the fp32 sum over its
+// ranks, below it that sum rounded to 16 bits, so an image alone and the same image in a large batch differ by that rounding.
 constexpr int64_t kFoldFrom = 1 << 19;
 
 static int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }

@@ -73,7 +73,8 @@ template <bool kWide> constexpr int core_items() { return kWide ? 2 * kItems : k
 // a few values that only live before and after the pass loop are then parked in scratch memory), four otherwise.
 template <typename in_t, int kGran, bool kWide> constexpr int core_min_waves() { return sizeof(in_t) == 2 && kGran >= 4 && !kWide ? 6 : 4; }
 
-// With dt_proj folded in the ranks of a pass take more registers than its delta did: four.
+// With dt_proj folded in the ranks of a pass take more registers than its delta did: four.  Three pairs with 16 positions per lane
+// (kCoreWidePairs) take all 128 registers and park four values (fp16: three) in scratch memory before the pass loop; none inside it.
 template <typename in_t, int kGran, bool kWide, int kPairs> constexpr int core_waves() {
     return kPairs > 0 && !kWide ? 4 : core_min_waves<in_t, kGran, kWide>();
 }
