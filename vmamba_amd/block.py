@@ -4,6 +4,8 @@ convolution + SiLU, forward_core, out_proj + add, and with fewer still LayerNorm
 The kernels and results are those of the separate calls; the host's share of a block goes from 100-120 us to about 40, which is what a
 model on a few images waits for.
 """
+from operator import attrgetter
+
 import torch
 import torch.nn as nn
 
@@ -15,7 +17,8 @@ from .ss2d import SS2D, HipLayers
 
 # what the call stands for: replaced on the class or the instance, they are called instead
 _STEPS = ("forward", "forward_core", "forward_core_fused", "finish_core", "_inference_constants", "_forward_core_native")
-_CLASS_STEPS = tuple(getattr(SS2D, name) for name in _STEPS)
+_class_steps = attrgetter(*_STEPS)
+_CLASS_STEPS = _class_steps(SS2D)
 _HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
 
 
@@ -39,16 +42,17 @@ def vss_block_hip(block, mlp_cls, x, residual=None):
     M = B * H * W
     if not 0 < M * C * C <= LINEAR_ROWS_MOST:
         return None
-    mods = block._modules
-    op, mlp, norm, norm2 = (mods.get(name) for name in ("op", "mlp", "norm", "norm2"))
+    get = block._modules.get
+    op, mlp, norm, norm2 = get("op"), get("mlp"), get("norm"), get("norm2")
     if not (_plain(op, SS2D) and _plain(mlp, mlp_cls) and _plain(norm, LayerNorm) and _plain(norm2, LayerNorm)):
         return None
     if (op.layers is not HipLayers or op.channel_first or mlp.channel_first or not mlp.fused or not op.fused_core or not op.disable_z
-            or op.d_state != 1 or not vars(op).keys().isdisjoint(_STEPS) or tuple(getattr(SS2D, name) for name in _STEPS) != _CLASS_STEPS):
+            or op.d_state != 1 or not vars(op).keys().isdisjoint(_STEPS) or _class_steps(SS2D) != _CLASS_STEPS):
         return None
-    inner = op._modules
-    in_proj, conv, out_norm, out_proj = (inner.get(name) for name in ("in_proj", "conv2d", "out_norm", "out_proj"))
-    fc1, act, fc2 = (mlp._modules.get(name) for name in ("fc1", "act", "fc2"))
+    get = op._modules.get
+    in_proj, conv, out_norm, out_proj = get("in_proj"), get("conv2d"), get("out_norm"), get("out_proj")
+    get = mlp._modules.get
+    fc1, act, fc2 = get("fc1"), get("act"), get("fc2")
     if not (all(_plain(layer, nn.Linear) for layer in (in_proj, out_proj, fc1, fc2)) and _plain(conv, nn.Conv2d) and _plain(out_norm, LayerNorm)
             and _plain(act, nn.GELU) and act.approximate == "none"):
         return None

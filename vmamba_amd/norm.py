@@ -144,7 +144,13 @@ class LayerNorm2d(nn.LayerNorm):
 
 
 _MODES = torch._C._len_torch_dispatch_stack, torch._C._functorch.peek_interpreter_stack, torch._C._len_torch_function_stack
-_CALLS = (nn.Linear.forward, nn.GELU.forward, LayerNorm.forward, F.linear, F.gelu)
+
+
+def _calls():
+    return nn.Linear.forward, nn.GELU.forward, LayerNorm.forward, F.linear, F.gelu
+
+
+_CALLS = _calls()
 
 
 def operators_seen():
@@ -153,9 +159,7 @@ def operators_seen():
     set_default_device, which only looks at factories), forward-mode derivatives, torch.func's transforms, or another forward or
     function in the place of torch's or this package's own."""
     dispatch, transforms, functions = _MODES
-    if dispatch() or forward_ad._current_level >= 0 or transforms() is not None:
+    if dispatch() or forward_ad._current_level >= 0 or transforms() is not None or _calls() != _CALLS:
         return True
     modes = functions()
-    if modes and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes)):
-        return True
-    return (nn.Linear.forward, nn.GELU.forward, LayerNorm.forward, F.linear, F.gelu) != _CALLS
+    return modes > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))

@@ -171,7 +171,7 @@ class VSSBlock(nn.Module):
                 pre = None
             else:
                 x = inp = x + pending
-        few = few_positions(x) and self._steps_as_written()
+        few = few_positions(x) and Mlp.forward is _STEPS[1]
         native = vss_block_hip(self, Mlp, inp, x if pre is None else None) if few else None       # as one call
         if native is not None:
             x, whole = native
@@ -181,7 +181,7 @@ class VSSBlock(nn.Module):
                 return self.mlp(x, residual=x, pre_norm=self.norm2), None
             return self._pending_mlp(x, self.norm2(x))
         # the fused MLP kernels normalise their input themselves
-        if self.mlp.takes_norm(x, self.norm2) if few else self.mlp.takes_norm(x):
+        if self.mlp.takes_norm(x, self.norm2) if few and self._steps_as_written() else self.mlp.takes_norm(x):
             x = self.op(inp, residual=x, pre_norm=pre)
             return self.mlp(x, residual=x, pre_norm=self.norm2), None
         x, h = self.op(inp, residual=x, pre_norm=pre, post_norm=self.norm2)
