@@ -38,21 +38,20 @@ def one_by_one(block, x, residual=None):
     """What the call gives without the MLP -- x + op(norm(x)), or residual + op(x) with x normalised already -- from its kernels."""
     op, norm = block.op, block.norm
     ln = (norm.weight, norm.bias, norm.eps) if residual is None else ()
-    walk = x.shape[-1] == op.d_inner == 96 and x.numel() > 24576 * 96
-    project = linear_cl_hip if walk else linear_rows_hip
-    h = project(x, op.in_proj.weight, op.in_proj.bias, None, *ln)
+    narrow, M = x.shape[-1] == op.d_inner == 96, x.numel() // x.shape[-1]
+    h = (linear_cl_hip if narrow and M > 24576 else linear_rows_hip)(x, op.in_proj.weight, op.in_proj.bias, None, *ln)
     h = dwconv3x3_silu_hip(h, op.conv2d.weight, op.conv2d.bias, in_channel_last=True, apply_silu=True)
     add, out = x if residual is None else residual, op.out_proj
-    if x.shape[-1] == op.d_inner == 96 and x.shape[1] * x.shape[2] % 32 == 0:
+    if narrow and x.shape[1] * x.shape[2] % 32 == 0:
         y = op._forward_core_native(h, False)
         return linear_cf_ln_hip(y, op.out_norm.weight, op.out_norm.bias, op.out_norm.eps, out.weight, out.bias, add).view(x.shape)
-    return project(op.forward_core(h), out.weight, out.bias, add)
+    return linear_rows_hip(op.forward_core(h), out.weight, out.bias, add)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("dim,B,H,W,kwargs", [
     (96, 1, 56, 56, {}), (96, 1, 14, 14, {}), (192, 2, 28, 28, {}), (384, 1, 14, 14, {}), (384, 2, 10, 12, {}), (768, 1, 7, 7, {}), (48, 3, 8, 8, {}),
-    (384, 8, 14, 14, {}), (768, 8, 7, 7, {}), (96, 8, 56, 56, {}), (96, 8, 60, 62, {}), (192, 8, 28, 28, {}), (192, 1, 12, 12, dict(ssm_ratio=2.0, mlp_ratio=2.0)), (96, 1, 16, 16, dict(bias=True, conv_bias=True)),
+    (384, 8, 14, 14, {}), (768, 8, 7, 7, {}), (96, 8, 56, 56, {}), (192, 8, 28, 28, {}), (192, 1, 12, 12, dict(ssm_ratio=2.0, mlp_ratio=2.0)), (96, 1, 16, 16, dict(bias=True, conv_bias=True)),
     (96, 1, 14, 14, dict(norm_biases=False)), (384, 1, 14, 14, dict(norm_biases=False)), (384, 8, 14, 14, dict(bias=True, norm_biases=False))])
 def test_same_bits(dim, B, H, W, kwargs, dtype, monkeypatch):
     print("CASE vss_block", dim, B, H, W, kwargs, dtype, flush=True)
@@ -79,6 +78,15 @@ def test_same_bits(dim, B, H, W, kwargs, dtype, monkeypatch):
     else:                      # out_proj's sum and the MLP are the library's on the other side: 16 u, as any two such blocks
         u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
         assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 16 * u
+
+
+@pytest.mark.parametrize("B", [6, 8, 12])
+def test_projections_of_many_positions(B):
+    """22 320, 29 760 and 44 640 positions of width 96, their maps no multiple of 32: either side of in_proj's line, out_proj's kernel."""
+    block, x = make(96, B, 60, 62, torch.bfloat16)
+    with torch.no_grad():
+        got, whole = vss_block_hip(block, Mlp, x)
+        assert not whole and torch.equal(got, one_by_one(block, x))
 
 
 @pytest.mark.parametrize("dim,B,side", [(384, 8, 14), (768, 6, 7)])

@@ -1,7 +1,8 @@
 """A channel-last VSS block of few positions as one call into the library (ss2d_block_fwd): LayerNorm + in_proj, depthwise
 convolution + SiLU, forward_core, out_proj + add, and with fewer still LayerNorm + fc1 + GELU, fc2 + add (classification/models/vmamba.py:1225-1229).
 
-The kernels and results are those of the separate calls; the host's share of a block goes from 100-120 us to about 40, which is what a
+The kernels and results are those of the separate calls, but for out_proj at width 96 on more than 24 576 positions
+of maps that are no multiple of 32 (ss2d_linear_rows here, ss2d_linear_cl there); the host's share of a block goes from 100-120 us to about 40, which is what a
 model on a few images waits for.
 """
 from operator import attrgetter

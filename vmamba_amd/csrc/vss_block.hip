@@ -82,9 +82,12 @@ extern "C" int ss2d_block_fwd(const ss2d_block_params *q, void *workspace, int64
     const int64_t M = (int64_t)c.batch * c.height * c.width;
     const void *residual = q->residual ? q->residual : q->x;
     void *sum = p.mlp ? base + p.sum : q->out;
-    // 96 -> 96 of many positions: the kernel that holds the weights and walks over tiles (12 544: 8.0 us against 5.0, 25 088: 8.2 / 8.2)
-    const bool walk = C == 96 && D == 96 && M > 24576;
-    if (walk)
+    // 96 -> 96 of many positions: the kernel that holds the weights and walks over tiles.  bf16, in a graph, ss2d_linear_rows against it in
+    // us: with the LayerNorm 12 544 positions 4.9 / 8.0, 25 088 7.0 / 8.3, 31 360 8.8 / 8.5, 43 904 10.9 / 8.9 (the line is the separate
+    // calls', linear_rows_pays).  out_proj with its residual crosses later, 29 760 7.3 / 8.5, 37 632 9.0 / 9.4, 43 904 10.0 / 9.1, and in
+    // the block, behind the norm that has just written its operand, no earlier than its most positions (two blocks of 8 x 60 x 62
+    // 192 / 198, of 12 x 60 x 62 244 / 244): ss2d_linear_rows throughout.
+    if (C == 96 && D == 96 && M > 24576)
         rc = ss2d_linear_cl(q->x, q->norm_weight, q->norm_bias, q->norm_eps, q->in_proj_weight, q->in_proj_bias, nullptr, base + p.proj, M, C, D, dt, stream);
     else
         rc = ss2d_linear_rows(q->x, q->norm_weight, q->norm_bias, q->norm_eps, q->in_proj_weight, q->in_proj_bias, nullptr, base + p.proj, M, C, D, 0, dt,
@@ -94,8 +97,6 @@ extern "C" int ss2d_block_fwd(const ss2d_block_params *q, void *workspace, int64
     if (rc == SS2D_OK && p.narrow)
         rc = ss2d_linear_cf_ln(base + p.mixed, c.norm_weight, c.norm_bias, c.eps, q->out_proj_weight, q->out_proj_bias, residual, sum, c.batch,
                                c.height * c.width, D, C, dt, stream);
-    else if (rc == SS2D_OK && walk)
-        rc = ss2d_linear_cl(base + p.mixed, nullptr, nullptr, 0.0f, q->out_proj_weight, q->out_proj_bias, residual, sum, M, D, C, dt, stream);
     else if (rc == SS2D_OK)
         rc = ss2d_linear_rows(base + p.mixed, nullptr, nullptr, 0.0f, q->out_proj_weight, q->out_proj_bias, residual, sum, M, D, C, 0, dt, stream);
     if (rc != SS2D_OK || !p.mlp) return rc;
