@@ -111,7 +111,7 @@ struct CorePassLoads {
 // piece and zero elsewhere, so that D[4 q + v][j] -- accumulator v of lane 16 q + j -- is that lane's own position v.  One matrix
 // instruction (16 cycles of a unit that idles here) per four positions and pair, no vector instruction, no exchange between
 // lanes, and delta -- the core's largest tensor, 308 MB written and read at 96 x 56 x 56, batch 128 -- never exists; the sums stay
-// in fp32 where dt_proj rounds them to 16 bits.  96 x 56 x 56, batch 128, bf16: 170 + 67 us of dt_proj -> 176 (three pairs, 16
+// in fp32 where dt_proj rounds them to 16 bits.  96 x 56 x 56, batch 128, bf16: 170 + 67 us of dt_proj -> 176-186 by card (three pairs, 16
 // positions per lane); the ranks come from L2, 2.5 times the lines of before, in runs of 1 KB (as x_proj's plain rows, 64 bytes from
 // lane to lane: 216).
 template <typename in_t, bool kSoftplus, int kGran, bool kVecDelta, bool kWide, int kWpd = 1, int kPairs = 0>

@@ -90,14 +90,16 @@ def linear_rows_pays(M, N, K):
     with LayerNorm or residual on both sides: 96 -> 96 at 12 544 positions 5.0 against ss2d_linear_cl's 8.0; 192 -> 192 at 3136
     6.0 against the library's 8.6, at 12 544 14.3 / 12.0; 384 -> 384 at 784 6.5 / 9.0, at 1568 8.9 / 9.8, at 3136 13.3 / 11.5;
     768 -> 768 at 196 7.2 / 9.8, at 400 10.6 / 10.2, at 784 15.3 / 11.4.  The rule lies up to 4 us a product beyond the crossing:
-    the library's call takes 24 us on the host, and a model on up to 16 images waits for that (3090 us a pass whose kernels run for 1700).  The MLP (fc1 is asked for, four outputs per input) has fewer passes around it
-    to win back: 384 at 400 17.6 / 23.7, at 784 27.5 / 27.5, at 1568 43 / 35; 768 at 49 20.6 / 24.9, at 196 30.2 / 26.4, where the
+    the library's call takes 24 us on the host, and a model on up to 16 images waits for that (3090 us a pass whose kernels run for 1700).
+    Replayed from a graph nothing waits, and the rule is the same there, so that a replay has the eager call's bits: two blocks of
+    768 x 7 x 7 214 -> 219 at 16 images (eager 405 -> 271), 200 -> 199 at 12.  The MLP (fc1 is asked for, four outputs per input) has fewer
+    passes around it to win back: 384 at 400 17.6 / 23.7, at 784 27.5 / 27.5, at 1568 43 / 35; 768 at 49 20.6 / 24.9, at 196 30.2 / 26.4, where the
     host's share (two launches for four library calls of 24 us and two of the package's) still decides.  Widths 96 and 192 have
     ss2d_mlp_fused, whose 128 positions per workgroup leave the chip idle below: 192 at 784 12.1 / 45.2, at 3136 27.2 / 45.5, at
     6272 44.6 / 45.8; 96 at 6272 15.5 / 17.8, at 12 544 25.3 / 18.0."""
     if N >= 4 * K:
         return 0 < M <= 6144 if K <= 192 else 0 < M * N * K <= 480 << 20
-    if N == K == 96:                     # ss2d_linear_cl's: 8.2 / 8.2 at 25 088
+    if N == K == 96:                     # ss2d_linear_cl's: with the LayerNorm 7.0 / 8.3 at 25 088, 8.8 / 8.5 at 31 360
         return 0 < M <= 24576
     return 0 < M * N * K <= LINEAR_ROWS_MOST
 
