@@ -133,3 +133,18 @@ def test_residuals_that_the_kernels_cannot_add(C, with_norm, kind):
     if got.requires_grad:
         got.float().sum().backward()
         assert torch.equal(r.grad, torch.ones_like(r))
+
+
+class Doubled(Mlp):
+    def forward(self, x, residual=None, pre_norm=None):
+        return 2 * super().forward(x, residual, pre_norm)
+
+
+@pytest.mark.parametrize("C", [96, 384])
+def test_residual_added_by_torch_behind_a_subclass(C):
+    """The subclass's own step happens once."""
+    m = Doubled(C, 4 * C, channel_first=False).to(DEV).bfloat16().eval().requires_grad_(False)
+    norm = LayerNorm(C).to(DEV).bfloat16().requires_grad_(False)
+    x = torch.randn(2, 5, 7, C, device=DEV).bfloat16()
+    r = torch.randn_like(x).requires_grad_(True)
+    assert torch.equal(m(x, residual=r, pre_norm=norm), 2 * (r + Mlp.forward(m, x, None, norm)))

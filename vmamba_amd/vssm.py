@@ -121,18 +121,16 @@ class Mlp(nn.Module):
                and not needs_grad(x, self.fc1.weight, self.fc2.weight, self.fc1.bias, self.fc2.bias)
                and (pre_norm is None or (isinstance(pre_norm, nn.LayerNorm) and pre_norm.elementwise_affine
                                          and not needs_grad(pre_norm.weight, pre_norm.bias))))
-        if (rows or one) and residual is not None and residual is not x and not self._adds(x, residual):
-            return residual + self.forward(x, None, pre_norm)
+        add = residual if (rows or one) and residual is not None and (residual is x or self._adds(x, residual)) else None       # by the kernel
         if rows:
             h = linear_rows_hip(x, self.fc1.weight, self.fc1.bias, None, pre_norm.weight, pre_norm.bias, pre_norm.eps, gelu=True)
-            return linear_rows_hip(h, self.fc2.weight, self.fc2.bias, residual)
-        if one:
+            y = linear_rows_hip(h, self.fc2.weight, self.fc2.bias, add)
+        elif one:
             norm = () if pre_norm is None else (pre_norm.weight, pre_norm.bias, pre_norm.eps)
-            return mlp_fused_hip(x, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias, residual, *norm)
-        if pre_norm is not None:
-            x = pre_norm(x)
-        y = self.fc2(self.act(self.fc1(x)))
-        return y if residual is None else residual + y
+            y = mlp_fused_hip(x, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias, add, *norm)
+        else:
+            y = self.fc2(self.act(self.fc1(x if pre_norm is None else pre_norm(x))))
+        return y if residual is None or add is not None else residual + y
 
     @staticmethod
     def _adds(x, residual):
@@ -191,7 +189,7 @@ class VSSBlock(nn.Module):
         """True when nothing sees or replaces the calls of op and mlp, whose arguments and results with few positions are others than
         with many: an MLP of another kind is called with norm2's result, as everywhere beyond widths 96 and 192."""
         op, mlp = self.op, self.mlp
-        return (isinstance(mlp, Mlp) and (type(op).forward, type(mlp).forward, type(mlp).takes_norm) == _STEPS
+        return (isinstance(mlp, Mlp) and (getattr(type(op), "forward", None), type(mlp).forward, type(mlp).takes_norm) == _STEPS
                 and not observed(op) and not observed(mlp))
 
     def _pending_mlp(self, x, h):
