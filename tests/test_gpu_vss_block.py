@@ -1,6 +1,7 @@
 """A block of few positions as one call (ss2d_block_fwd): the bits of the separate calls, and who is left to them."""
 import pytest
 import torch
+import torch.nn.functional as F
 from torch.autograd import forward_ad
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -329,3 +330,46 @@ def test_residual_of_another_kind_is_added_by_torch():
     assert "reshape" in Seen.functions                               # into torch's addmm
     # two orders of one projection's sum, each rounded once
     assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 2 * 2.0 ** -8
+
+
+def block_f64(block, x):
+    """The block in float64 from its 16-bit parameters and input (classification/models/vmamba.py:603-663, 1225-1229)."""
+    op, mlp = block.op, block.mlp
+    d = lambda t: None if t is None else t.double()
+    ln = lambda n, t: F.layer_norm(t, n.normalized_shape, d(n.weight), d(n.bias), n.eps)
+    x = x.double()
+    B, H, W, _ = x.shape
+    h = F.linear(ln(block.norm, x), d(op.in_proj.weight), d(op.in_proj.bias)).permute(0, 3, 1, 2)
+    h = F.silu(F.conv2d(h, d(op.conv2d.weight), d(op.conv2d.bias), padding=1, groups=h.shape[1]))
+    D, L, R = h.shape[1], H * W, op.dt_rank
+    rows, cols = h.flatten(2), h.transpose(2, 3).flatten(2)
+    u = torch.stack([rows, cols, rows.flip(-1), cols.flip(-1)])                              # (4, B, D, L)
+    proj = torch.einsum("kcd,kbdl->kbcl", d(op.x_proj_weight), u)
+    step = F.softplus(torch.einsum("kdr,kbrl->kbdl", d(op.dt_projs_weight), proj[:, :, :R]) + d(op.dt_projs_bias).view(4, 1, D, 1))
+    decay, state = torch.exp(-step * d(op.A_logs).exp().view(4, 1, D, 1)), step * u * proj[:, :, R, None]
+    for j in range(1, L):
+        state[..., j] += decay[..., j] * state[..., j - 1]
+    y = state * proj[:, :, R + 1, None] + d(op.Ds).view(4, 1, D, 1) * u
+    down = (y[1] + y[3].flip(-1)).view(B, D, W, H).transpose(2, 3).flatten(2)
+    y = (y[0] + y[2].flip(-1) + down).view(B, D, H, W).permute(0, 2, 3, 1)
+    x = x + F.linear(ln(op.out_norm, y), d(op.out_proj.weight), d(op.out_proj.bias))
+    return x + F.linear(F.gelu(F.linear(ln(block.norm2, x), d(mlp.fc1.weight), d(mlp.fc1.bias))), d(mlp.fc2.weight), d(mlp.fc2.bias))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("dim,B,H,W", [(96, 1, 28, 28), (192, 1, 28, 20), (384, 1, 14, 14), (384, 8, 14, 14), (768, 1, 7, 7)])
+def test_no_further_from_float64_than_the_modules(dim, B, H, W, dtype):
+    """The call rounds where the modules do, but for out_proj's and fc2's sums, which are rounded once with the residual instead of
+    before and behind it: its error's 2-norm over the result is the modules' or less.  Both are sums over 37 632 independent roundings or
+    more, whose ratio strays by about 1 / sqrt(37 632); 2 % is four times that."""
+    print("CASE vss_block f64", dim, B, H, W, dtype, flush=True)
+    block, x = make(dim, B, H, W, dtype)
+    with torch.no_grad():
+        assert vss_block_hip(block, Mlp, x) is not None
+        got = block(x)
+        with Functions():                       # products and GELU are the library's
+            modules = block(x)
+        want = block_f64(block, x)
+    off = lambda t: ((t.double() - want).norm() / want.norm()).item()
+    print("  off float64 by", off(got), "modules", off(modules), flush=True)
+    assert off(got) <= 1.02 * off(modules)
