@@ -362,6 +362,7 @@ int ss2d_core_fwd_ws(const ss2d_core_params *params, void *workspace, int64_t wo
  *   padded_height, padded_width   the map's own size, or a larger one to embed it in (ss2d_core_embed_maps; 16-bit types), with
  *         pad_mask as ss2d_dt_proj_masked takes it for the (4, batch * padded positions) in scan order (asked for also where dt_proj
  *         is in the core, which does not read it); the result is cropped
+ * A few short maps in their own size take ss2d_x_proj_few and ss2d_core_few instead (where ss2d_few_applies says so).
  * Everything contiguous.  workspace: ss2d_forward_core_workspace_bytes(params) bytes, 16-byte aligned, contents irrelevant;
  * workspace_bytes depends on the sizes and types, and on the pointers' alignment.  Either function returns SS2D_ENOTSUP where
  * one of the kernels has no variant for the problem.
@@ -377,6 +378,21 @@ typedef struct ss2d_forward_core_params {
 
 int64_t ss2d_forward_core_workspace_bytes(const ss2d_forward_core_params *params);
 int ss2d_forward_core(const ss2d_forward_core_params *params, void *workspace, int64_t workspace_bytes, void *stream);
+
+/*
+ * x_proj, and dt_proj with the core, of a few short one-state maps (classification/models/vmamba.py:603-638):
+ *   ss2d_x_proj_few   x (B,D,H,W), weight (4, rank + 2, D), 16-byte aligned, of one dtype -> rows: ss2d_few_rows_bytes bytes, 16-byte aligned,
+ *                     every position's four directions side by side in the map's own order, a layout for ss2d_core_few alone
+ *   ss2d_core_few     x, those rows, dt_weight (4, D, rank) of the same dtype; A, D_skip, delta_bias (4*D) fp32, the last two or NULL
+ *                     -> y (B,D,L) fp32, the merged map; softplus on, the step's sum over its ranks kept in fp32
+ * ss2d_few_rows_bytes: SS2D_ENOTSUP where the kernels have no variant (maps of more than 256 positions or fewer than 4, ranks
+ * beyond 48, dim no multiple of 8).  ss2d_few_applies: SS2D_OK where they are also the faster ones, SS2D_ENOTSUP elsewhere.
+ */
+int64_t ss2d_few_rows_bytes(int batch, int dim, int rank, int height, int width, int dtype);
+int ss2d_few_applies(int batch, int dim, int rank, int height, int width, int dtype);
+int ss2d_x_proj_few(const void *x, const void *weight, void *rows, int batch, int dim, int rank, int height, int width, int dtype, void *stream);
+int ss2d_core_few(const void *x, const void *rows, const void *dt_weight, const float *A, const float *D_skip, const float *delta_bias, float *y,
+                  int batch, int dim, int rank, int height, int width, int dtype, void *stream);
 
 /*
  * A channel-last block of few positions as one call (classification/models/vmamba.py:1225-1229):

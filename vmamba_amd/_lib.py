@@ -163,6 +163,14 @@ def lib():
         L.ss2d_forward_core_workspace_bytes.argtypes = [ctypes.POINTER(ForwardCoreParams)]
         L.ss2d_forward_core.restype = ctypes.c_int
         L.ss2d_forward_core.argtypes = [ctypes.POINTER(ForwardCoreParams), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+        L.ss2d_few_rows_bytes.restype = ctypes.c_int64
+        L.ss2d_few_rows_bytes.argtypes = [ctypes.c_int] * 6
+        L.ss2d_few_applies.restype = ctypes.c_int
+        L.ss2d_few_applies.argtypes = [ctypes.c_int] * 6
+        L.ss2d_x_proj_few.restype = ctypes.c_int
+        L.ss2d_x_proj_few.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_int] * 6 + [ctypes.c_void_p]
+        L.ss2d_core_few.restype = ctypes.c_int
+        L.ss2d_core_few.argtypes = [ctypes.c_void_p] * 7 + [ctypes.c_int] * 6 + [ctypes.c_void_p]
         L.ss2d_block_workspace_bytes.restype = ctypes.c_int64
         L.ss2d_block_workspace_bytes.argtypes = [ctypes.POINTER(BlockParams)]
         L.ss2d_block_fwd.restype = ctypes.c_int

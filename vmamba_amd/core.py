@@ -164,7 +164,7 @@ def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=Non
     if (code is None or x.numel() == 0 or R == 0 or tuple(x_proj_weight.shape) != (4, R + 2, D) or tuple(dt_proj_weight.shape) != (4, D, R)
             or not As.numel() == Ds.numel() == dt_bias.numel() == 4 * D):
         return None
-    padded = padded_map_size(H, W, x.dtype)
+    padded = None if few_applies(B, D, H, W, R, x.dtype) and x_proj_weight.data_ptr() % 16 == 0 else padded_map_size(H, W, x.dtype)
     if padded is not None and (pad_mask is None or R > DT_PROJ_MAX_RANK):
         return None
     index = x.get_device()
@@ -209,6 +209,40 @@ def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=Non
         return None
     _lib.check(rc, "ss2d_forward_core")
     return out
+
+
+def few_applies(B, D, H, W, rank, dtype):
+    """True when the two kernels for a few short maps (B, D, H, W) are the faster way from the map to its merged map, one state per
+    channel and ``rank`` ranks per direction (ss2d_few_applies)."""
+    code = _DTYPE_CODE.get(dtype)
+    return (code is not None and H * W <= FEW_MOST_POSITIONS
+            and _lib.lib().ss2d_few_applies(B, D, rank, H, W, code) == _lib.SS2D_OK)
+
+
+FEW_MOST_POSITIONS = 256             # of a map; a first look that costs nothing
+
+
+def core_few_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias):
+    """x (B, D, H, W), x_proj_weight (4, R + 2, D), dt_proj_weight (4, D, R) of one dtype, As, Ds, dt_bias (4 * D) fp32: the merged
+    map (B, D, L) in fp32 of a few short maps (ss2d_x_proj_few, ss2d_core_few)."""
+    _check(x.is_cuda and x.dim() == 4 and x.dtype in _DTYPE_CODE, "core_few: a (B, D, H, W) map on the GPU")
+    B, D, H, W = x.shape
+    R = dt_proj_weight.shape[2]
+    _check(tuple(x_proj_weight.shape) == (4, R + 2, D) and tuple(dt_proj_weight.shape) == (4, D, R), "core_few: weights (4, R + 2, D) and (4, D, R)")
+    for t in (x_proj_weight, dt_proj_weight):
+        _check(t.dtype == x.dtype and t.device == x.device, "core_few: weights of x's dtype on its device")
+    for t in (As, Ds, dt_bias):
+        _check(t.dtype == torch.float32 and t.device == x.device and t.numel() == 4 * D and t.is_contiguous(), "core_few: A, D and the bias (4 * D) float32")
+    x, x_proj_weight, dt_proj_weight = x.contiguous(), x_proj_weight.contiguous(), dt_proj_weight.contiguous()
+    code, L = _DTYPE_CODE[x.dtype], _lib.lib()
+    need = L.ss2d_few_rows_bytes(B, D, R, H, W, code)
+    _lib.check(min(need, 0), "ss2d_few_rows_bytes")
+    rows = torch.empty(need, dtype=torch.uint8, device=x.device)
+    y = torch.empty((B, D, H * W), device=x.device, dtype=torch.float32)
+    _lib.check(_lib.launch(x, L.ss2d_x_proj_few, x.data_ptr(), x_proj_weight.data_ptr(), rows.data_ptr(), B, D, R, H, W, code), "ss2d_x_proj_few")
+    _lib.check(_lib.launch(x, L.ss2d_core_few, x.data_ptr(), rows.data_ptr(), dt_proj_weight.data_ptr(), As.data_ptr(), Ds.data_ptr(),
+                           dt_bias.data_ptr(), y.data_ptr(), B, D, R, H, W, code), "ss2d_core_few")
+    return y
 
 
 def x_proj_fits(x, weight):

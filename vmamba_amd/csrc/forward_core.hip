@@ -9,7 +9,7 @@
 namespace ss2d {
 
 struct ForwardCorePlan {
-    bool padded;
+    bool padded, few;                                                // few: core_few.hip's two kernels
     DtsLayout layout;
     int planes, flags_per_image;                                     // planes > 0: dt_proj folded into the core
     int64_t pitch, x, x_dbl, flags, delta, y, out, scratch, total;   // row pitch in elements; byte offsets; bytes
@@ -51,6 +51,15 @@ static int forward_core_plan(const ss2d_forward_core_params *q, char *base, Forw
     p.pitch = (q->batch * L + vec - 1) / vec * vec;
     // on a padded map delta has to start every image where its mask does
     if (p.padded && p.pitch != q->batch * L) return SS2D_ENOTSUP;
+    p.few = !p.padded && few_pays(q->batch, q->dim, q->rank, q->height, q->width, q->dtype) && reinterpret_cast<uintptr_t>(q->x_proj_weight) % 16 == 0;
+    if (p.few) {
+        if (q->dtype == SS2D_F32 && !dt_proj_f32_takes(q->rank)) return SS2D_ENOTSUP;
+        if (q->normalise && !layer_norm_cf_takes(q->dim, SS2D_F32, q->norm_dtype, q->dtype)) return SS2D_ENOTSUP;
+        p.x_dbl = 0;
+        p.y = align256(few_rows_bytes(q->batch, q->rank, L, q->dtype));
+        p.total = align256(p.y + (q->normalise ? q->batch * D * L * 4 : 0));
+        return SS2D_OK;
+    }
     if (!forward_core_kernels_take(q, p.pitch)) return SS2D_ENOTSUP;
     p.x = 0;
     p.x_dbl = p.padded ? align256(p.x + q->batch * D * L * es) : 0;
@@ -111,6 +120,14 @@ extern "C" int ss2d_forward_core(const ss2d_forward_core_params *q, void *worksp
     const int B = q->batch, D = q->dim, H = q->padded_height, W = q->padded_width, R = q->rank, C = R + 2;
     const int64_t L = (int64_t)H * W, ks = C * p.pitch;
     const int es = q->dtype == SS2D_F32 ? 4 : 2;
+    if (p.few) {
+        float *y = q->normalise ? (float *)(base + p.y) : (float *)q->out;
+        rc = ss2d_x_proj_few(q->x, q->x_proj_weight, base + p.x_dbl, B, D, R, H, W, q->dtype, stream);
+        if (rc == SS2D_OK) rc = ss2d_core_few(q->x, base + p.x_dbl, q->dt_proj_weight, (const float *)q->A, (const float *)q->D, (const float *)q->delta_bias, y, B, D, R, H, W, q->dtype, stream);
+        if (rc == SS2D_OK && q->normalise)
+            rc = ss2d_layer_norm_cf(y, q->norm_weight, q->norm_bias, q->out, B, D, (int)L, q->eps, SS2D_F32, q->norm_dtype, q->dtype, q->out_channel_last, stream);
+        return rc;
+    }
     void *x_dbl = base + p.x_dbl, *delta = base + p.delta;
     if (p.padded) rc = ss2d_core_embed_maps(q->x, base + p.x, (int64_t)B * D, q->height, q->width, H, W, es, stream);
     const void *x = p.core.x;

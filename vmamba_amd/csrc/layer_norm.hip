@@ -853,16 +853,16 @@ static int ln_cf_crop(const void *x, const void *w, const void *b, void *y, int 
     return launch_ln_cf_crop<w_t, out_t, 4, 64, 12>(x, w, b, y, B, C, L, eps, crop, s);
 }
 
-// Few short images of an odd length: a wavefront per position, its channels C / 64 to a lane, all in registers.  The image
-// kernel keeps such an image on one workgroup (its vectors straddle channel rows), which is the whole time where one CU's
-// loads are all there is in flight.  One image of 768 x 7 x 7 into bf16, channel-last: 10.5 -> 6.2 us; 384 x 13 x 13: 16.0 -> 4.3.
+// Few short images: a wavefront per position, its channels C / 64 to a lane, all in registers.  The image kernel keeps such an image on
+// one workgroup where its vectors straddle channel rows, and on a few otherwise, which is the whole time where those CUs' loads are
+// all there is in flight.  One image of 768 x 7 x 7 into bf16, channel-last: 10.5 -> 6.2 us; 384 x 13 x 13: 16.0 -> 4.3.
 template <typename in_t, typename w_t, typename out_t, bool kOutChannelLast>
 __global__ __launch_bounds__(kBlock) void layer_norm_cf_position_kernel(const in_t *__restrict__ x, const w_t *__restrict__ weight,
                                                                         const w_t *__restrict__ bias, out_t *__restrict__ y, int C, int L,
                                                                         int n_pos, float eps, FastDiv by_image) {
     constexpr int kPer = 16;                         // channels per lane at most
     const int lane = threadIdx.x & (kWave - 1);
-    const int pos = (int)(blockIdx.x * (kBlock / kWave)) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int pos = (int)(blockIdx.x * (blockDim.x / kWave)) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (pos >= n_pos) return;
     uint32_t b, l;
     divmod((uint32_t)pos, by_image, b, l);
@@ -894,20 +894,24 @@ __global__ __launch_bounds__(kBlock) void layer_norm_cf_position_kernel(const in
 }
 
 // Most positions of a call that takes it.  A load instruction touches 64 cache lines, and a channel-first store as many: 16 images
-// of 768 x 7 x 7 channel-first are level (10.4 us against 10.6; channel-last 6.5 against 10.9), 20 behind (11.4 against 10.7).
-constexpr int kLnPositions = 800;
+// of 768 x 7 x 7 channel-first are level (10.4 us against 10.6; channel-last 6.5 against 10.9), 20 behind (11.4 against 10.7).  Where
+// the image kernel splits an image -- L a multiple of 4 --, channel-first output falls behind earlier: 384 x 14 x 14 channel-last / first
+// one image 6.2 / 5.2 -> 3.9 / 4.5, four 6.3 / 5.4 -> 4.3 / 6.5 (one line for both layouts, which hold the same bits).
+constexpr int kLnPositionsOdd = 800, kLnPositions = 256;
 
 template <typename in_t, typename w_t, typename out_t>
 static int launch_ln_cf_position(const void *x, const void *w, const void *b, void *y, int B, int C, int L, float eps,
                                  int out_channel_last, hipStream_t stream) {
     const int n_pos = B * L;
-    const dim3 grid((uint32_t)((n_pos + kBlock / kWave - 1) / (kBlock / kWave)));
+    // a wavefront per workgroup while that spreads the positions over more CUs: 768 x 7 x 7 6.1 -> 5.4 us, 16 of 8 x 8 the other way, 6.9 -> 7.4
+    const int waves = n_pos <= 256 ? 1 : kBlock / kWave;
+    const dim3 grid((uint32_t)((n_pos + waves - 1) / waves)), block(waves * kWave);
     const FastDiv by_image = make_fastdiv((uint32_t)L);
     if (out_channel_last)
-        hipLaunchKernelGGL((layer_norm_cf_position_kernel<in_t, w_t, out_t, true>), grid, dim3(kBlock), 0, stream, (const in_t *)x,
+        hipLaunchKernelGGL((layer_norm_cf_position_kernel<in_t, w_t, out_t, true>), grid, block, 0, stream, (const in_t *)x,
                            (const w_t *)w, (const w_t *)b, (out_t *)y, C, L, n_pos, eps, by_image);
     else
-        hipLaunchKernelGGL((layer_norm_cf_position_kernel<in_t, w_t, out_t, false>), grid, dim3(kBlock), 0, stream, (const in_t *)x,
+        hipLaunchKernelGGL((layer_norm_cf_position_kernel<in_t, w_t, out_t, false>), grid, block, 0, stream, (const in_t *)x,
                            (const w_t *)w, (const w_t *)b, (out_t *)y, C, L, n_pos, eps, by_image);
     return launch_status();
 }
@@ -983,7 +987,7 @@ constexpr int kLnCfMaxChannels = 156 * 1024 / (5 * (int)sizeof(float));
 template <typename in_t, typename w_t, typename out_t>
 static int launch_ln_cf(const void *x, const void *w, const void *b, void *y, int B, int C, int L, float eps,
                         int out_channel_last, hipStream_t stream) {
-    if (L % 4 != 0 && C <= 1024 && (int64_t)B * L <= kLnPositions)
+    if (C <= 1024 && (int64_t)B * L <= (L % 4 != 0 ? kLnPositionsOdd : kLnPositions))
         return launch_ln_cf_position<in_t, w_t, out_t>(x, w, b, y, B, C, L, eps, out_channel_last, stream);
     {
         // short images: a whole image, or an even share of one, per workgroup

@@ -28,17 +28,6 @@ namespace ss2d {
 
 constexpr int kMlpChunk = 32;      // hidden units per chunk = one MFMA tile
 
-// One global_load_lds_dwordx4: every lane fetches 16 bytes from its own address, the wavefront's 1 KB lands at
-// lds_base + 16 * lane (lds_base wave-uniform).  Written as assembly so that the compiler does not order every later
-// LDS read behind the outstanding load (it cannot tell the double buffers apart and waits for vmcnt(0) at the first
-// LDS access after the issue, which puts the whole L2 latency on the critical path of every chunk); the waits are
-// placed by hand instead: wait_loads_to_lds() before the barrier that publishes a buffer.
-__device__ __forceinline__ void load_to_lds_16(const void *src, const void *lds_base) {
-    const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)lds_base);
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(base) : "memory", "m0");
-}
-__device__ __forceinline__ void wait_loads_to_lds() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
-
 struct MlpArgs {
     const void *x, *ln_w, *ln_b, *w1, *b1, *w2, *b2, *residual;
     void *out;

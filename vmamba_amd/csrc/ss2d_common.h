@@ -122,6 +122,18 @@ template <typename U> __device__ __forceinline__ void store_streaming(U *p, U v)
     __builtin_nontemporal_store(__builtin_bit_cast(W, v), reinterpret_cast<W *>(p));
 }
 
+// ---- global memory to LDS ---------------------------------------------------------------------------------------
+// One global_load_lds_dwordx4: every lane fetches 16 bytes from its own address, the wavefront's 1 KB lands at
+// lds_base + 16 * lane (lds_base wave-uniform).  Written as assembly so that the compiler does not order every later
+// LDS read behind the outstanding load (it cannot tell the double buffers apart and waits for vmcnt(0) at the first
+// LDS access after the issue, which puts the whole L2 latency on the critical path of every chunk); the waits are
+// placed by hand instead: wait_loads_to_lds() before the barrier that publishes a buffer.
+__device__ __forceinline__ void load_to_lds_16(const void *src, const void *lds_base) {
+    const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)lds_base);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void wait_loads_to_lds() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
+
 // ---- matrix cores -------------------------------------------------------------------------------------------
 // v_mfma_f32_32x32x8 (bf16 / f16 operands, fp32 accumulate): D (32 x 32) += A (32 x 8) * B (8 x 32).  Lane l supplies
 // A[l % 32][4*(l/32) .. +3] and B[4*(l/32) .. +3][l % 32] as two dwords of packed 16-bit values, and holds
@@ -226,6 +238,10 @@ bool dt_proj_takes(int D, int R, int64_t N, int64_t x_rank_stride, int dtype);
 bool dt_proj_f32_takes(int R);
 bool layer_norm_cf_takes(int C, int in_dtype, int w_dtype, int out_dtype);
 bool linear_rows_takes(int64_t M, int K, int N, bool layer_norm, int dtype);
+
+// The two kernels of core_few.hip: where they are the faster ones, and what ss2d_x_proj_few writes.
+bool few_pays(int B, int D, int R, int H, int W, int dtype);
+int64_t few_rows_bytes(int B, int R, int64_t L, int dtype);
 
 // ss2d_x_proj for one state per channel with the step's ranks in pairs, as the core with dt_proj folded in reads them
 // (core_dts_fwd): per direction ceil((R + padded) / 2) planes of dwords, low half rank 2 p, high half rank 2 p + 1 -- zero where

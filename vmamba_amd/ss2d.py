@@ -21,8 +21,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ._lib import SS2D_ENOTSUP, Ss2dError
-from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_fits, core_mask_pads_hip, dt_proj_f32_hip, dt_proj_hip,
-                   embed_maps_hip, forward_core_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_f32_pays,
+from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_few_hip, core_fits, core_mask_pads_hip, dt_proj_f32_hip, dt_proj_hip,
+                   embed_maps_hip, few_applies, forward_core_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_f32_pays,
                    x_proj_fits, x_proj_hip, x_proj_pays)
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
@@ -253,6 +253,9 @@ class SS2D(nn.Module):
         B, D, H0, W0 = x.shape
         K, R = self.k_group, self.dt_rank
         C = R + 2
+        if x.is_cuda and few_applies(B, D, H0, W0, R, x.dtype) and self.x_proj_weight.data_ptr() % 16 == 0:
+            y = core_few_hip(x, self.x_proj_weight, self.dt_projs_weight, consts["As"].view(-1), consts["Ds"], consts["dt_bias"])
+            return y if crop else (y, (H0, W0))
         # Maps the kernel would walk element by element (sides like 57 x 58, 75, 19: a number of positions that is not a
         # multiple of 4) are embedded in a slightly larger map: zeros on the added rows / columns, the projections
         # computed on the padded map, and the step of the added positions set to 0 (delta = -inf), which makes them
