@@ -24,7 +24,7 @@ EXPORTS = ("ss2d_abi_version", "ss2d_strerror", "ss2d_cross_scan", "ss2d_cross_m
            "ss2d_selective_scan_kernel", "ss2d_selective_scan_fwd_maps",
            "ss2d_layer_norm", "ss2d_add_layer_norm", "ss2d_bias_layer_norm", "ss2d_layer_norm_cf", "ss2d_layer_norm_cf_crop", "ss2d_dwconv3x3_silu",
            "ss2d_dwconv3x3_silu_f32", "ss2d_dwconv3x3_silu_bwd", "ss2d_dwconv3x3_silu_bwd_workspace_bytes", "ss2d_cross_scan_1b1", "ss2d_core_fwd",
-           "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_forward_core", "ss2d_forward_core_workspace_bytes", "ss2d_block_fwd", "ss2d_block_workspace_bytes", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
+           "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_forward_core", "ss2d_forward_core_workspace_bytes", "ss2d_block_fwd", "ss2d_block_workspace_bytes", "ss2d_few_rows_bytes", "ss2d_few_applies", "ss2d_x_proj_few", "ss2d_core_few", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
            "ss2d_x_proj", "ss2d_x_proj_applies", "ss2d_x_proj_f32", "ss2d_dt_proj", "ss2d_dt_proj_f32", "ss2d_dt_proj_masked", "ss2d_cross_scan_flex", "ss2d_cross_scan_flex_ws", "ss2d_cross_scan_flex_static", "ss2d_cross_merge_flex",
            "ss2d_selective_scan_bwd", "ss2d_clear", "ss2d_round_pair", "ss2d_transpose_bcl", "ss2d_mlp_fused", "ss2d_linear_cl", "ss2d_linear_rows", "ss2d_linear_dw_f32", "ss2d_linear_dw_f32_workspace_bytes", "ss2d_linear_cf_ln", "ss2d_stem_conv_ln_gelu", "ss2d_stem_conv2_ln", "ss2d_mean_pool_cl")
 
@@ -234,6 +234,22 @@ def lib():
             raise ImportError(f"{LIB_PATH}: ABI version {L.ss2d_abi_version()} != expected {ABI_VERSION}; rebuild")
         _lib = L
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The extension behind forward_core_hip and vss_block_hip (csrc/host_ext.cpp)."""
+    global _host
+    if _host is None:
+        lib()                                # (the same libss2d_hip.so, its version checked)
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise ImportError(f"vmamba_amd._host is missing or does not load: build it first (python -m vmamba_amd.build): {e}") from e
+        _host = module
+    return _host
 
 
 def launch(tensor, fn, *args):

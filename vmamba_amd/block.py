@@ -57,54 +57,25 @@ def vss_block_hip(block, mlp_cls, x, residual=None):
     if not (all(_plain(layer, nn.Linear) for layer in (in_proj, out_proj, fc1, fc2)) and _plain(conv, nn.Conv2d) and _plain(out_norm, LayerNorm)
             and _plain(act, nn.GELU) and act.approximate == "none"):
         return None
-    weight = [layer._parameters.get("weight") for layer in (in_proj, out_proj, fc1, fc2, norm, norm2, out_norm, conv)]
-    bias = [layer._parameters.get("bias") for layer in (in_proj, out_proj, fc1, fc2, norm, norm2, out_norm, conv)]
+    layers = (in_proj, out_proj, fc1, fc2, norm, norm2, out_norm, conv)
+    weight = tuple([layer._parameters.get("weight") for layer in layers])
+    bias = tuple([layer._parameters.get("bias") for layer in layers])
     own = op._parameters
     x_proj, dt_proj = own.get("x_proj_weight"), own.get("dt_projs_weight")
-    index = x.get_device()
-    if residual is not None and residual.shape != x.shape:
+    if weight[0] is None or weight[2] is None or dt_proj is None:
         return None
-    for t in (x, x if residual is None else residual, x_proj, dt_proj, *weight):
-        if t is None or type(t) not in TENSOR_KINDS or t.dtype != x.dtype or t.get_device() != index or not t.is_contiguous() or t.data_ptr() % 16:
-            return None
-    w_in, w_out, w_1, w_2, w_n1, w_n2, w_on, w_c = weight
-    D, hidden, R = w_in.shape[0], w_1.shape[0], dt_proj.shape[2]
-    for t, n in zip(bias, (D, C, hidden, C, C, C, D, D)):           # (torch would broadcast one of another size)
-        if t is not None and (type(t) not in TENSOR_KINDS or t.numel() != n or t.dtype != x.dtype or t.get_device() != index
-                              or not t.is_contiguous() or t.data_ptr() % 16):
-            return None
-    if (tuple(w_in.shape) != (D, C) or tuple(w_out.shape) != (C, D) or tuple(w_1.shape) != (hidden, C) or tuple(w_2.shape) != (C, hidden)
-            or norm.normalized_shape != (C,) or norm2.normalized_shape != (C,) or out_norm.normalized_shape != (D,)
-            or w_n1.numel() != C or w_n2.numel() != C or w_on.numel() != D
-            or tuple(w_c.shape) != (D, 1, 3, 3) or tuple(x_proj.shape) != (4, R + 2, D) or tuple(dt_proj.shape) != (4, D, R) or R == 0
-            or conv.padding != (1, 1) or conv.stride != (1, 1) or conv.dilation != (1, 1) or conv.padding_mode != "zeros"):
-        return None
-    if (C % 16 or D % 16 or hidden % 16 or C > 768 or D > 3072 or hidden > 3072 or M * D * C > LINEAR_ROWS_MOST
+    D, hidden = weight[0].shape[0], weight[2].shape[0]
+    if (norm.normalized_shape != (C,) or norm2.normalized_shape != (C,) or out_norm.normalized_shape != (D,)
+            or conv.padding != (1, 1) or conv.stride != (1, 1) or conv.dilation != (1, 1) or conv.padding_mode != "zeros"
+            or C % 16 or D % 16 or hidden % 16 or C > 768 or D > 3072 or hidden > 3072 or M * D * C > LINEAR_ROWS_MOST
             or not core_fits(H, W, x.dtype) or padded_map_size(H, W, x.dtype) is not None):
         return None
     whole = linear_rows_pays(M, hidden, C)
     consts = op._inference_constants(0)
-    As, Ds, dt_bias = consts["As"], consts["Ds"], consts["dt_bias"]
-    for t in (As, Ds, dt_bias):
-        if t.get_device() != index or t.numel() != 4 * D or not t.is_contiguous():
-            return None
-    out = torch.empty_like(x)
-    ptr = [None if t is None else t.data_ptr() for t in bias]
-    p = _lib.BlockParams(
-        _lib.ForwardCoreParams(B, D, H, W, R, H, W, code, code, 1, 1, out_norm.eps, None, x_proj.data_ptr(), dt_proj.data_ptr(), As.data_ptr(),
-                               Ds.data_ptr(), dt_bias.data_ptr(), w_on.data_ptr(), ptr[6], None, None),
-        C, hidden, norm.eps, norm2.eps, x.data_ptr(), None if residual is None else residual.data_ptr(),
-        w_n1.data_ptr() if residual is None else None, ptr[4] if residual is None else None, w_in.data_ptr(), ptr[0], w_c.data_ptr(), ptr[7],
-        w_out.data_ptr(), ptr[1], w_n2.data_ptr(), ptr[5], w_1.data_ptr() if whole else None,
-        ptr[2], w_2.data_ptr() if whole else None, ptr[3], out.data_ptr())
-    L = _lib.lib()
-    need = L.ss2d_block_workspace_bytes(p)
-    if need == _lib.SS2D_ENOTSUP:
+    out = _lib.host().block(TENSOR_KINDS, x, residual, weight, bias, x_proj, dt_proj, consts["As"], consts["Ds"], consts["dt_bias"],
+                            (norm.eps, norm2.eps, out_norm.eps), whole)
+    if out is None:
         return None
-    _lib.check(min(need, 0), "ss2d_block_workspace_bytes")
-    workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
-    rc = _lib.launch(x, L.ss2d_block_fwd, p, workspace.data_ptr(), need)
-    if rc == _lib.SS2D_ENOTSUP:
-        return None
-    _lib.check(rc, "ss2d_block_fwd")
+    if type(out) is int:
+        _lib.check(out, "ss2d_block_fwd")
     return out, whole

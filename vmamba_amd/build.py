@@ -1,6 +1,7 @@
 """Builds the native pieces in-tree with hipcc / g++ (no GPU needed: gfx950 is cross-compiled).
 
   libss2d_hip.so                  HIP kernels + C ABI (include/ss2d_hip.h)
+  _host*.so                       the host's share of forward_core and of a block of few positions, over the C ABI
   selective_scan_cuda_oflex*.so   thin PyTorch C++ extension over the C ABI, importable under the
                                   name the reference probes for (classification/models/csms6s.py:9-14)
 
@@ -48,23 +49,26 @@ def build_hip(verbose=True, jobs=None):
     return LIB
 
 
+def ext_path(name):
+    return os.path.join(PKG, name + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
+
+
 def torch_ext_path():
-    suffix = sysconfig.get_config_var("EXT_SUFFIX") or ".so"
-    return os.path.join(PKG, "selective_scan_cuda_oflex" + suffix)
+    return ext_path("selective_scan_cuda_oflex")
 
 
-def build_torch_ext():
+def _build_ext(name, source):
     import torch
     from torch.utils import cpp_extension
 
-    out = torch_ext_path()
+    out = ext_path(name)
     tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
     inc = cpp_extension.include_paths() + [os.path.join(ROCM, "include"), sysconfig.get_paths()["include"]]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           "-DTORCH_EXTENSION_NAME=selective_scan_cuda_oflex", "-DTORCH_API_INCLUDE_EXTENSION_H",
+           f"-DTORCH_EXTENSION_NAME={name}", "-DTORCH_API_INCLUDE_EXTENSION_H",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-deprecated-declarations"]
     cmd += [f"-I{p}" for p in inc]
-    cmd += [os.path.join(CSRC, "torch_ext.cpp"), "-o", out,
+    cmd += [os.path.join(CSRC, source), "-o", out,
             f"-L{tlib}", "-lc10", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10_hip", "-ltorch_hip",
             f"-L{PKG}", "-lss2d_hip", f"-L{os.path.join(ROCM, 'lib')}", "-lamdhip64",
             "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{tlib}", f"-Wl,-rpath,{os.path.join(ROCM, 'lib')}"]
@@ -72,8 +76,17 @@ def build_torch_ext():
     return out
 
 
+def build_host_ext():
+    return _build_ext("_host", "host_ext.cpp")
+
+
+def build_torch_ext():
+    return _build_ext("selective_scan_cuda_oflex", "torch_ext.cpp")
+
+
 def build_all(torch_ext=True):
     build_hip()
+    build_host_ext()
     if torch_ext and os.path.exists(os.path.join(CSRC, "torch_ext.cpp")):
         build_torch_ext()
 

@@ -160,54 +160,20 @@ def forward_core_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, norm=Non
     _check(x.is_cuda, "forward_core: vmamba_amd runs on the GPU only")
     B, D, H, W = x.shape
     R = dt_proj_weight.shape[2]
-    code = _DTYPE_CODE.get(x.dtype)
-    if (code is None or x.numel() == 0 or R == 0 or tuple(x_proj_weight.shape) != (4, R + 2, D) or tuple(dt_proj_weight.shape) != (4, D, R)
-            or not As.numel() == Ds.numel() == dt_bias.numel() == 4 * D):
-        return None
-    padded = None if few_applies(B, D, H, W, R, x.dtype) and x_proj_weight.data_ptr() % 16 == 0 else padded_map_size(H, W, x.dtype)
-    if padded is not None and (pad_mask is None or R > DT_PROJ_MAX_RANK):
-        return None
-    index = x.get_device()
-    for t in (x_proj_weight, dt_proj_weight):
-        if t.dtype != x.dtype or t.get_device() != index or not t.is_contiguous():
-            return None
-    for t in (As, Ds, dt_bias):
-        if t.dtype != torch.float32 or t.get_device() != index or not t.is_contiguous():
-            return None
-    x = x.contiguous()
-    p = _lib.ForwardCoreParams(B, D, H, W, R, *(padded or (H, W)), code)
+    dtype = x.dtype
+    padded = None if few_applies(B, D, H, W, R, dtype) and x_proj_weight.data_ptr() % 16 == 0 else padded_map_size(H, W, dtype)
+    mask = None
     if padded is not None:
-        mask = pad_mask(H, W, *padded, B, x.device)
-        _check(mask.get_device() == index and mask.dtype == torch.int16 and mask.is_contiguous()
-               and tuple(mask.shape) == (4, B * padded[0] * padded[1]), "pad_mask: (4, B * L) int16")
-        p.pad_mask = mask.data_ptr()
-    if norm is not None:
-        weight, bias = norm.weight, norm.bias
-        for t in (weight, bias):
-            if t is not None and (t.get_device() != index or not t.is_contiguous() or t.numel() != D or t.dtype not in _DTYPE_CODE):
-                return None
-        if weight is not None and bias is not None and weight.dtype != bias.dtype:
+        if pad_mask is None or R > DT_PROJ_MAX_RANK or dtype not in _DTYPE_CODE or x.numel() == 0:
             return None
-        p.normalise, p.out_channel_last, p.eps = 1, int(out_channel_last), norm.eps
-        if weight is not None:
-            p.norm_weight, p.norm_dtype = weight.data_ptr(), _DTYPE_CODE[weight.dtype]
-        if bias is not None:
-            p.norm_bias, p.norm_dtype = bias.data_ptr(), _DTYPE_CODE[bias.dtype]
-        out = x.new_empty((B, H, W, D) if out_channel_last else (B, D, H, W))
-    else:
-        out = torch.empty((B, D, H * W), device=x.device, dtype=torch.float32)
-    p.x, p.x_proj_weight, p.dt_proj_weight = x.data_ptr(), x_proj_weight.data_ptr(), dt_proj_weight.data_ptr()
-    p.A, p.D, p.delta_bias, p.out = As.data_ptr(), Ds.data_ptr(), dt_bias.data_ptr(), out.data_ptr()
-    L = _lib.lib()
-    need = L.ss2d_forward_core_workspace_bytes(p)
-    if need == _lib.SS2D_ENOTSUP:
-        return None
-    _lib.check(min(need, 0), "ss2d_forward_core_workspace_bytes")
-    workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
-    rc = _lib.launch(x, L.ss2d_forward_core, p, workspace.data_ptr(), need)
-    if rc == _lib.SS2D_ENOTSUP:
-        return None
-    _lib.check(rc, "ss2d_forward_core")
+        mask = pad_mask(H, W, *padded, B, x.device)
+        _check(mask.get_device() == x.get_device() and mask.dtype == torch.int16 and mask.is_contiguous()
+               and tuple(mask.shape) == (4, B * padded[0] * padded[1]), "pad_mask: (4, B * L) int16")
+        H, W = padded
+    weight, bias, eps = (None, None, 0.0) if norm is None else (norm.weight, norm.bias, norm.eps)
+    out = _lib.host().forward_core(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias, weight, bias, eps, norm is not None, out_channel_last, H, W, mask)
+    if type(out) is int:
+        _lib.check(out, "ss2d_forward_core")
     return out
 
 
