@@ -604,6 +604,19 @@ int ss2d_linear_cf_ln(const void *x, const void *ln_weight, const void *ln_bias,
  */
 int ss2d_mean_pool_cl(const void *x, void *y, int B, int L, int C, int dtype, void *stream);
 
+/*
+ * A product in single precision on the bf16 matrix cores (each value as the sum of three bf16 ones, six products, fp32 sums; the error is
+ * that of a product in fp32): out (M, N) with out[m][n] = sum over K of A(m, k) B(n, k), A stored (M, K) or by columns (K, M), B (N, K) or (K, N).
+ *   mode 0: + bias (N) + other (M, N), either or both NULL.  mode 1: out = sum + bias, out2 = GELU(out).
+ *   mode 2: out = (sum + bias) GELU'(other), other the pre-activation.
+ * The fp32 Linear layers of a block and their gradients (classification/models/vmamba.py:648-662, :1116-1131).  Contiguous, 16-byte
+ * aligned, rows in multiples of 4 elements (SS2D_ENOTSUP otherwise); out none of the operands.  workspace:
+ * ss2d_product_f32_workspace_bytes(...) bytes, 16-byte aligned; no atomics, the same bits every time.
+ */
+int64_t ss2d_product_f32_workspace_bytes(int64_t M, int N, int64_t K, int a_by_columns, int b_by_columns);
+int ss2d_product_f32(const float *a, const float *b, const float *bias, const float *other, float *out, float *out2, int64_t M, int N, int64_t K,
+                     int a_by_columns, int b_by_columns, int mode, void *workspace, int64_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

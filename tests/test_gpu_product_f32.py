@@ -1,0 +1,144 @@
+"""ss2d_product_f32 against float64: the edges of its tiles, steps and shares, both ways either operand may be stored, and what stands
+behind the sum; MlpF32 and its derivatives.
+
+An output is a sum of six products a term, added in fp32: it stays within 6 K 2^-24 of the sum of the terms' magnitudes whatever the order
+(the terms left out and the rest of a value behind its third part are below 2^-25 of a term)."""
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from vmamba_amd import _lib
+from vmamba_amd.linear import PRODUCT_GELU, PRODUCT_GELU_GRAD, LinearDw, MlpF32, mlp_f32_pays, product_f32_hip, product_pays
+from vmamba_amd.vssm import Mlp
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def make(M, N, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    a, b = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    return (a * torch.exp2(torch.randint(-20, 20, (M, 1), generator=g).float())).to(DEV), b.to(DEV)
+
+
+def stored(t, by_columns):
+    return t.t().contiguous() if by_columns else t
+
+
+@pytest.mark.parametrize("a_cols,b_cols", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(4, 4, 4), (128, 64, 32), (124, 68, 36), (132, 132, 60), (260, 60, 512), (64, 192, 4100), (1000, 1028, 100), (12544, 128, 96)])
+def test_product(M, N, K, a_cols, b_cols):
+    print("CASE product_f32", M, N, K, a_cols, b_cols, flush=True)
+    a, b = make(M, N, K, M + K)
+    got = product_f32_hip(stored(a, a_cols), stored(b, b_cols), a_cols, b_cols).double()
+    want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    assert bool(((got - want).abs() <= 6 * K * 2.0 ** -24 * size).all())
+    lib = (a @ b.t()).double()
+    scale = want.norm(dim=1, keepdim=True)
+    assert ((got - want) / scale).norm().item() <= 1.1 * ((lib - want) / scale).norm().item() + 1e-7
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 132, 64), (200, 68, 2048)])       # one share, and several added by the second kernel
+def test_what_stands_behind_the_sum(M, N, K):
+    print("CASE product_f32 epilogue", M, N, K, flush=True)
+    assert (_lib.lib().ss2d_product_f32_workspace_bytes(M, N, K, 0, 0) > 0) == (K > 1000)
+    g = torch.Generator().manual_seed(K)
+    a, b = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV) / K ** 0.5
+    bias, other = torch.randn(N, generator=g).to(DEV), torch.randn(M, N, generator=g).to(DEV)
+    z = a.double() @ b.double().t()
+    close = lambda got, want: torch.allclose(got.double(), want, rtol=1e-5, atol=1e-5)        # sums of unit size, 2^-24 a rounding
+    assert close(product_f32_hip(a, b, bias=bias, other=other), z + bias.double() + other.double())
+    pre, act = product_f32_hip(a, b, bias=bias, mode=PRODUCT_GELU)
+    assert close(pre, z + bias.double()) and close(act, F.gelu(z + bias.double()))
+    x = other.double().requires_grad_()
+    slope = torch.autograd.grad(F.gelu(x).sum(), x)[0]
+    assert close(product_f32_hip(a, b, other=other, mode=PRODUCT_GELU_GRAD), z * slope)
+
+
+@pytest.mark.parametrize("a_cols,b_cols", [(False, False), (True, True)])
+def test_infinities_and_nan(a_cols, b_cols):
+    """The same outputs are infinite and NaN as in the library's product, and values near fp32's largest, which round beyond bf16's, count."""
+    a, b = make(300, 132, 384, 3)
+    a, b = a / a.abs().amax(1, keepdim=True), b * 0.01
+    a[5, 7], a[9, 3], a[200, 1], a[201, 1], b[77, 11] = float("inf"), float("nan"), 3.4e38, -3.402e38, -float("inf")
+    got, want = product_f32_hip(stored(a, a_cols), stored(b, b_cols), a_cols, b_cols), a @ b.t()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())
+    ok = want.isfinite()
+    assert torch.allclose(got[ok], want[ok], rtol=1e-4, atol=1e-6)
+
+
+def test_refused():
+    a = torch.zeros(8, 8, device=DEV)
+    with pytest.raises(ValueError):
+        product_f32_hip(a, a[:, :4])
+    with pytest.raises(ValueError):
+        product_f32_hip(a, a.half())
+    for args in ((torch.zeros(8, 6, device=DEV), torch.zeros(8, 6, device=DEV)), (a, torch.zeros(6, 8, device=DEV)),
+                 (torch.zeros(65, device=DEV)[1:].view(8, 8), a)):
+        with pytest.raises(_lib.Ss2dError):
+            product_f32_hip(*args)
+
+
+@pytest.mark.parametrize("bias", [True, False])
+def test_mlp_autograd(bias):
+    """Both derivatives against float64: relative errors of a few hundred roundings of 2^-24."""
+    torch.manual_seed(0)
+    mlp = Mlp(96, 384, channel_first=False).to(DEV)
+    if not bias:
+        mlp.fc1.bias = mlp.fc2.bias = None
+    x = torch.randn(4, 56, 56, 96, device=DEV, requires_grad=True)
+    dy = torch.randn_like(x)
+    assert mlp_f32_pays(x, mlp.fc1, mlp.act, mlp.fc2)
+    params = [x] + list(mlp.parameters())
+    exact = [t.detach().double().requires_grad_() for t in params]
+    e = iter(exact[1:])
+    xd = exact[0]
+    w1, b1, w2, b2 = next(e), next(e) if bias else None, next(e), next(e) if bias else None
+    y, want_y = mlp(x), F.linear(F.gelu(F.linear(xd, w1, b1)), w2, b2)
+    assert y.grad_fn.name().startswith("MlpF32")
+    got, want = torch.autograd.grad(y, params, dy), torch.autograd.grad(want_y, exact, dy.double(), create_graph=True)
+    for g, w in zip((y,) + got, (want_y,) + want):
+        assert ((g.double() - w).norm() / w.norm()).item() < 2e-6
+    # a second backward, through the torch operators
+    dx = torch.autograd.grad(mlp(x), x, dy, create_graph=True)[0]
+    got, want = torch.autograd.grad(dx.square().sum(), params[:2]), torch.autograd.grad(want[0].square().sum(), exact[:2])
+    for g, w in zip(got, want):
+        assert ((g.double() - w).norm() / w.norm()).item() < 1e-5
+
+
+def test_who_is_left_to_the_operators():
+    mlp = Mlp(96, 384, channel_first=False).to(DEV)
+    x = torch.randn(12544, 96, device=DEV)
+    takes = lambda t=x: mlp_f32_pays(t, mlp.fc1, mlp.act, mlp.fc2)
+    assert takes() and not takes(x[:784]) and not takes(x.half())
+    with torch.no_grad():
+        assert not takes()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not takes()
+    seen = []
+    handle = mlp.act.register_forward_hook(lambda *a: seen.append(1))
+    mlp(x)
+    assert seen and not takes()
+    handle.remove()
+    with torch.autograd.forward_ad.dual_level():
+        assert not takes()
+    assert torch.func.grad(lambda t: mlp(t).sum())(x).shape == x.shape
+    mlp.act.approximate = "tanh"
+    assert not takes()
+    mlp.act.approximate = "none"
+    mlp.fc1.weight = nn.Parameter(torch.randn(96, 384, device=DEV).t())
+    assert not takes()
+    # both sides of the line
+    assert product_pays(12544, 1536, 384) and not product_pays(784, 1536, 384) and product_pays(1536, 384, 4096, True) and not product_pays(1536, 384, 4095, True)
+
+
+def test_projection_with_residual():
+    layer = nn.Linear(768, 512, bias=False).to(DEV)
+    x, r = torch.randn(7000, 768, device=DEV, requires_grad=True), torch.randn(7000, 512, device=DEV)
+    dy = torch.randn(7000, 512, device=DEV)
+    y = LinearDw.apply(x, layer.weight, r)
+    got = (y,) + torch.autograd.grad(y, (x, layer.weight), dy)
+    w, xd = layer.weight.double(), x.double()
+    for g, want in zip(got, (r.double() + xd @ w.t(), dy.double() @ w, dy.double().t() @ xd)):
+        assert ((g.double() - want).norm() / want.norm()).item() < 2e-6

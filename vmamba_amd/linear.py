@@ -2,8 +2,8 @@
 
 Stands in, in a channel-last VSS block of width 96, for norm + in_proj and for out_proj + the residual add
 (classification/models/vmamba.py:1225-1228, :648-650, :662) at inference in bf16 / fp16; other widths and fp32
-stay on the PyTorch-ROCm operators.  In single-precision training the weight gradient of these projections is a HIP kernel
-(ss2d_linear_dw_f32) where that is the faster one.
+stay on the PyTorch-ROCm operators.  In single-precision training the products of these projections and of the MLP, and their gradients,
+are HIP kernels (ss2d_product_f32, ss2d_linear_dw_f32) where those are the faster ones.
 """
 import torch
 import torch.nn as nn
@@ -180,41 +180,155 @@ def linear_dw_hip(x, dy):
     return dw
 
 
+# ss2d_product_f32: what stands behind the sum
+PRODUCT_PLAIN, PRODUCT_GELU, PRODUCT_GELU_GRAD = range(3)
+
+
+def product_f32_hip(a, b, a_by_columns=False, b_by_columns=False, bias=None, other=None, mode=PRODUCT_PLAIN):
+    """sum_k A(m, k) B(n, k) in float32 on the bf16 matrix cores (ss2d_product_f32): a (M, K), or (K, M) by columns, b (N, K) or (K, N),
+    contiguous; + bias (N) + other (M, N); PRODUCT_GELU: (the sum with the bias, its GELU); PRODUCT_GELU_GRAD: times GELU'(other)."""
+    M, K = a.shape[::-1] if a_by_columns else a.shape
+    N = b.shape[1] if b_by_columns else b.shape[0]
+    if not a.is_cuda or b.shape[0 if b_by_columns else 1] != K:
+        raise ValueError("product_f32_hip: a (M, K) and b (N, K) on one GPU, either stored by columns")
+    if any(t is not None and (t.dtype != torch.float32 or t.device != a.device or not t.is_contiguous()) for t in (a, b, bias, other)):
+        raise ValueError("product_f32_hip: contiguous float32 tensors on one GPU")
+    if (bias is not None and bias.numel() != N) or (other is not None and tuple(other.shape) != (M, N)):
+        raise ValueError("product_f32_hip: bias (N), other (M, N)")
+    out = a.new_empty((M, N))
+    out2 = torch.empty_like(out) if mode == PRODUCT_GELU else None
+    L = _lib.lib()
+    need = L.ss2d_product_f32_workspace_bytes(M, N, K, a_by_columns, b_by_columns)
+    _lib.check(min(need, 0), "ss2d_product_f32_workspace_bytes")
+    workspace = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+    ptr = lambda t: None if t is None else t.data_ptr()
+    rc = _lib.launch(a, L.ss2d_product_f32, a.data_ptr(), b.data_ptr(), ptr(bias), ptr(other), out.data_ptr(), ptr(out2), M, N, K,
+                     a_by_columns, b_by_columns, mode, ptr(workspace), need)
+    _lib.check(rc, "ss2d_product_f32")
+    return out if out2 is None else (out, out2)
+
+
+def product_pays(M, N, K, gradient=False):
+    """True where ss2d_product_f32 is ahead of the library's fp32 product, whose rate is 90-100 TFLOP/s at best.  The kernel needs
+    workgroups: 384 tiles of 128 x 64 outputs, or shares of a long sum (``gradient``: both operands by columns, K the positions), or 6 G
+    products in any cut.  us, library / kernel: 12 544 x 1536 x 384 159 / 109, x 384 x 1536 157 / 120, x 384 x 384 49 / 35 (588 tiles); 50 176 x 96 x 96
+    29 / 19; 1176 x 2048 x 512 37 / 33 (320 tiles, left), 4181 x 384 x 384 16 / 20 (198), 3136 x 768 x 192 14 / 16 (300); 9408 x 512 x 2048 191 / 151
+    (592 tiles), 3136 x 512 x 2048 57 / 61 (3.3 G), 2090 x 768 x 3072 82 / 83 (4.9 G).  Gradients: 1536 x 384 over 12 544 positions 144 / 91, 384 x 96 over
+    50 176 256 / 75, 256 x 1024 over 6272 39 / 39, 768 x 192 over 3136 22 / 28."""
+    if gradient:
+        return K >= 4096
+    return -(-M // 128) * -(-N // 64) >= 384 or M * N * K >= 6 << 30
+
+
+def _product(a, b, a_by_columns=False, b_by_columns=False, bias=None, other=None, mode=PRODUCT_PLAIN):
+    """product_f32_hip where it stands for the library's product, which is taken under a second backward (the kernel has no gradient of its
+    own), for views that start between 16-byte boundaries and where it is the faster one."""
+    M, K = a.shape[::-1] if a_by_columns else a.shape
+    N = b.shape[1] if b_by_columns else b.shape[0]
+    rows = (M if a_by_columns else K, N if b_by_columns else K, N)
+    if not torch.is_grad_enabled() and all(n % 4 == 0 for n in rows) and M * N * K > 0 and product_pays(M, N, K, a_by_columns and b_by_columns):
+        a, b = a.contiguous(), b.contiguous()
+        other = None if other is None else other.contiguous()
+        if all(t is None or t.data_ptr() % 16 == 0 for t in (a, b, bias, other)):
+            return product_f32_hip(a, b, a_by_columns, b_by_columns, bias, other, mode)
+    a, b = a.t() if a_by_columns else a, b if b_by_columns else b.t()
+    if mode == PRODUCT_GELU_GRAD:
+        return torch.ops.aten.gelu_backward(torch.mm(a, b), other)
+    term = bias if other is None else other if bias is None else other + bias
+    y = torch.mm(a, b) if term is None else torch.addmm(term, a, b)
+    return y if mode == PRODUCT_PLAIN else (y, nn.functional.gelu(y))
+
+
+def _weight_gradient(dy, x):
+    """dy^T x, dy (M, N) and x (M, K)."""
+    N, K = dy.shape[1], x.shape[1]
+    if N * K <= 384 * 384 and x.shape[0] >= 4096 and N % 4 == 0 and K % 4 == 0 and not torch.is_grad_enabled():
+        x, dy = x.contiguous(), dy.contiguous()
+        if (x.data_ptr() | dy.data_ptr()) % 16 == 0:
+            return linear_dw_hip(x, dy)
+    return _product(dy, x, True, True)
+
+
+def calls_unseen():
+    """True when nothing but autograd follows the operators that are called: no mode or transform (operators_seen), no compiler or tracer."""
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or operators_seen() or torch.is_autocast_enabled())
+
+
+def _plain_f32(x, *tensors):
+    return all(t is None or (type(t) in TENSOR_KINDS and t.dtype == torch.float32 and t.device == x.device) for t in tensors)
+
+
 def linear_dw_pays(layer, x):
     """True when LinearDw stands for ``layer(x)`` in training: a plain nn.Linear without bias, hooks or autocast, on float32
-    positions many enough and with outputs few enough that the library leaves most of the chip idle.  12 544 positions, library
-    against kernel in us: 384 x 384 outputs 77 against 54; 576 x 576 104 against 106.  96 x 96 over 200 704: 443 against 141;
-    384 x 384 over 3136: 25 against 28."""
+    positions many enough and with outputs few enough that the library leaves most of the chip idle, or where ss2d_product_f32 is ahead
+    of it.  12 544 positions, weight gradient, library against kernel in us: 384 x 384 outputs 77 against 54.
+    96 x 96 over 200 704: 443 against 141; 384 x 384 over 3136: 25 against 28."""
     if not (type(layer) is nn.Linear and layer.bias is None and x.is_cuda and x.dim() >= 2 and x.dtype == torch.float32):
         return False
     weight = layer.weight
     N, K = weight.shape
     return (torch.is_grad_enabled() and weight.requires_grad and weight.dtype == x.dtype and weight.device == x.device
-            and x.shape[-1] == K and N % 4 == 0 and K % 4 == 0 and 0 < N * K <= 384 * 384 and x.numel() >= 4096 * K
-            and not observed(layer) and not torch.is_autocast_enabled())
+            and x.shape[-1] == K and N % 4 == 0 and K % 4 == 0 and N * K > 0 and x.numel() >= 4096 * K
+            and (N * K <= 384 * 384 or product_pays(x.numel() // K, N, K)) and not observed(layer) and calls_unseen())
 
 
 class LinearDw(torch.autograd.Function):
-    """x W^T, plus ``residual`` if one is given, with dW = dy^T x on ss2d_linear_dw_f32."""
+    """x W^T, plus ``residual`` if one is given; dW = dy^T x on ss2d_linear_dw_f32, and ss2d_product_f32 for what it is faster at."""
 
     @staticmethod
     def forward(ctx, x, weight, residual):
         ctx.save_for_backward(x, weight)
-        if residual is None:
-            return nn.functional.linear(x, weight)
-        return torch.addmm(residual.reshape(-1, weight.shape[0]), x.reshape(-1, weight.shape[1]), weight.t()).view(residual.shape)
+        N, K = weight.shape
+        y = _product(x.reshape(-1, K), weight, other=None if residual is None else residual.reshape(-1, N))
+        return y.view(x.shape[:-1] + (N,) if residual is None else residual.shape)
 
     @staticmethod
     def backward(ctx, dy):
         x, weight = ctx.saved_tensors
         N, K = weight.shape
         dy2, x2 = dy.reshape(-1, N), x.reshape(-1, K)
-        dx = torch.mm(dy2, weight).view(x.shape) if ctx.needs_input_grad[0] else None
-        dw = None
-        if ctx.needs_input_grad[1]:
-            # the library's product where the kernel does not stand for it: under a second backward (it has no gradient of its
-            # own), and for views that start between 16-byte boundaries, which contiguous() leaves where they are
-            x2, dy2 = x2.contiguous(), dy2.contiguous()
-            kernel = not torch.is_grad_enabled() and (x2.data_ptr() | dy2.data_ptr()) % 16 == 0
-            dw = linear_dw_hip(x2, dy2) if kernel else torch.mm(dy2.t(), x2)
+        dx = _product(dy2, weight, b_by_columns=True).view(x.shape) if ctx.needs_input_grad[0] else None
+        dw = _weight_gradient(dy2, x2) if ctx.needs_input_grad[1] else None
         return dx, dw, dy if ctx.needs_input_grad[2] else None
+
+
+def mlp_f32_pays(x, fc1, act, fc2):
+    """True when MlpF32 stands for ``fc2(act(fc1(x)))`` in training: plain nn.Linear layers and exact GELU that nothing observes, contiguous
+    float32 parameters, and a first product that ss2d_product_f32 is ahead in."""
+    if not (type(x) in TENSOR_KINDS and x.is_cuda and x.dtype == torch.float32 and x.dim() >= 2 and type(fc1) is type(fc2) is nn.Linear
+            and type(act) is nn.GELU and act.approximate == "none"):
+        return False
+    N, K = fc1.weight.shape
+    params = (fc1.weight, fc1.bias, fc2.weight, fc2.bias)
+    return (needs_grad(x, *params) and x.shape[-1] == K and tuple(fc2.weight.shape)[1:] == (N,) and N % 4 == 0 and K % 4 == 0 and N * K > 0
+            and product_pays(x.numel() // K, N, K) and _plain_f32(x, *params) and all(t is None or t.is_contiguous() for t in params)
+            and (fc1.bias is None or fc1.bias.numel() == N) and (fc2.bias is None or fc2.bias.numel() == fc2.weight.shape[0])
+            and not any(observed(m) for m in (fc1, act, fc2)) and calls_unseen())
+
+
+class MlpF32(torch.autograd.Function):
+    """fc2(GELU(fc1(x))) in single precision: GELU behind the first product, its derivative behind the second one's input gradient."""
+
+    @staticmethod
+    def forward(ctx, x, w1, b1, w2, b2):
+        pre, act = _product(x.reshape(-1, x.shape[-1]), w1, bias=b1, mode=PRODUCT_GELU)
+        ctx.save_for_backward(x, w1, b1, w2, pre, act)
+        return _product(act, w2, bias=b2).view(x.shape[:-1] + (w2.shape[0],))
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w1, b1, w2, pre, act = ctx.saved_tensors
+        x2, dy2 = x.reshape(-1, x.shape[-1]), dy.reshape(-1, dy.shape[-1])
+        if torch.is_grad_enabled():                                  # a second backward goes through what stands between, not only through x
+            pre = nn.functional.linear(x2, w1, b1)
+            act = nn.functional.gelu(pre)
+        wants = ctx.needs_input_grad
+        dw2 = _weight_gradient(dy2, act) if wants[3] else None
+        db2 = dy2.sum(0) if wants[4] else None
+        if not any(wants[:3]):
+            return None, None, None, dw2, db2
+        dpre = _product(dy2, w2, b_by_columns=True, other=pre, mode=PRODUCT_GELU_GRAD)
+        dw1 = _weight_gradient(dpre, x2) if wants[1] else None
+        db1 = dpre.sum(0) if wants[2] else None
+        dx = _product(dpre, w1, b_by_columns=True).view(x.shape) if wants[0] else None
+        return dx, dw1, db1, dw2, db2

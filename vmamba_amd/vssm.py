@@ -19,7 +19,7 @@ import torch
 import torch.nn as nn
 
 from .block import vss_block_hip
-from .linear import TENSOR_KINDS, few_positions, linear_rows_fusable, linear_rows_hip, linear_rows_takes
+from .linear import TENSOR_KINDS, MlpF32, few_positions, linear_rows_fusable, linear_rows_hip, linear_rows_takes, mlp_f32_pays
 from .mlp import mlp_fusable, mlp_fused_hip
 from .norm import LayerNorm as HipLayerNorm
 from .norm import add_layer_norm_fusable, add_layer_norm_hip, bias_layer_norm_fusable, bias_layer_norm_hip, needs_grad, observed
@@ -114,7 +114,8 @@ class Mlp(nn.Module):
         """fc2(GELU(fc1(h))) (+ residual), h = x or pre_norm(x) (the block's second LayerNorm, vmamba.py:1229).
         Channel-last 16-bit inference at widths 96 / 192 runs as one HIP kernel that normalises the rows on the way
         in and keeps the hidden activations in registers; few positions behind a norm as two launches of ss2d_linear_rows at
-        any width; everything else on the torch operators.  A residual that the kernels cannot add -- one that autograd has to
+        any width; single-precision training on the products of ss2d_product_f32 where those are the faster ones (MlpF32); everything else
+        on the torch operators.  A residual that the kernels cannot add -- one that autograd has to
         see, of another shape, type, device or kind -- is added by torch behind them."""
         rows = pre_norm is not None and few_positions(x) and self._rows(x, pre_norm)
         one = (not rows and self.fused and not self.channel_first and mlp_fusable(x, self.fc1, self.fc2)
@@ -129,7 +130,11 @@ class Mlp(nn.Module):
             norm = () if pre_norm is None else (pre_norm.weight, pre_norm.bias, pre_norm.eps)
             y = mlp_fused_hip(x, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias, add, *norm)
         else:
-            y = self.fc2(self.act(self.fc1(x if pre_norm is None else pre_norm(x))))
+            h = x if pre_norm is None else pre_norm(x)
+            if self.fused and not self.channel_first and mlp_f32_pays(h, self.fc1, self.act, self.fc2):
+                y = MlpF32.apply(h, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias)
+            else:
+                y = self.fc2(self.act(self.fc1(h)))
         return y if residual is None or add is not None else residual + y
 
     @staticmethod
