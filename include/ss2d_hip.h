@@ -605,6 +605,17 @@ int ss2d_linear_cf_ln(const void *x, const void *ln_weight, const void *ln_bias,
 int ss2d_mean_pool_cl(const void *x, void *y, int B, int L, int C, int dtype, void *stream);
 
 /*
+ * Channel-last products of many positions (a block's projections and MLP, classification/models/vmamba.py:648-662, :1116-1131):
+ *   out (M, N) = [GELU](x (M, K) weight (N, K)^T + bias (N)) + residual (M, N); bias and residual may be NULL, the residual also with `gelu` must be.
+ * and the convolution between two stages (vmamba.py:1430-1437), 3 x 3, stride 2, padding 1, without a separate im2col:
+ *   x (B, H, W, C), weight (N, 3, 3, C), out (B, (H + 1) / 2, (W + 1) / 2, N).
+ * One 16-bit dtype, contiguous, 16-byte aligned; K (C) a multiple of 32, N of 8, SS2D_ENOTSUP otherwise; out neither operand, the residual may be it.
+ */
+int ss2d_linear_tiles(const void *x, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int K, int N, int gelu, int dtype,
+                      void *stream);
+int ss2d_conv3x3s2_cl(const void *x, const void *weight, const void *bias, void *out, int B, int H, int W, int C, int N, int dtype, void *stream);
+
+/*
  * A product in single precision on the bf16 matrix cores (each value as the sum of three bf16 ones, six products, fp32 sums; the error is
  * that of a product in fp32): out (M, N) with out[m][n] = sum over K of A(m, k) B(n, k), A stored (M, K) or by columns (K, M), B (N, K) or (K, N).
  *   mode 0: + bias (N) + other (M, N), either or both NULL.  mode 1: out = sum + bias, out2 = GELU(out).

@@ -131,6 +131,57 @@ def linear_rows_hip(x, weight, bias=None, residual=None, ln_weight=None, ln_bias
     return out
 
 
+def linear_tiles_fusable(x, layer, act=None):
+    """True when ss2d_linear_tiles stands for ``layer(x)`` -- ``act(layer(x))``, act exact GELU that nothing observes -- at inference on
+    contiguous rows of x and is the faster one (linear_tiles_pays)."""
+    if type(layer) is not nn.Linear or type(x) not in TENSOR_KINDS or x.dtype not in _DTYPE_CODE:
+        return False
+    if act is not None and not (type(act) is nn.GELU and act.approximate == "none" and not observed(act)):
+        return False
+    N, K = layer.weight.shape
+    return (x.shape[-1] == K and K % 32 == 0 and K > 0 and linear_tiles_pays(x.numel() // K, N, K, act is not None) and linear_rows_takes(layer, x)
+            and calls_unseen() and x.is_contiguous() and x.data_ptr() % 16 == 0)
+
+
+def linear_tiles_pays(M, N, K, gelu):
+    """True where ss2d_linear_tiles is ahead of the library.  With the GELU, which is a pass over the result there: us in bf16, library
+    product and GELU / kernel, four outputs per input: 384 at 3136 positions 21 / 16, at 25 088 91 / 63, at 100 352 354 / 264; 96 at 3136 10 / 11,
+    at 12 544 19 / 12; 256 at 3136 16 / 14; 512 at 6272 33 / 36, at 12 544 75 / 54, at 50 176 276 / 174; 640 at 12 544 67 / 70; 768 at 6272 65 / 55, at 12 544
+    89 / 92.  Without, the library's larger tiles are ahead but where the contraction is short and the outputs fill tiles of 192: 384 x 384 at
+    12 544 positions 11 / 12, at 25 088 25 / 18, at 50 176 41 / 30; 320 x 320 at 25 088 19 / 16; 192 x 192 at 25 088 10 / 10, at 100 352 26 / 23; 256 x 256 at
+    50 176 15 / 23; 512 x 512 at 25 088 20 / 28."""
+    if gelu:
+        return K <= 512 and M >= (12544 if K > 384 else 3136 if K >= 192 else 6272)
+    return K <= 384 and (N % 192 == 0 or N % 192 >= 128) and M * N >= 8 << 20
+
+
+def linear_tiles_hip(x, weight, bias=None, residual=None, gelu=False):
+    """x (..., K) channel-last, weight (N, K), one 16-bit dtype: [gelu](x @ weight.T + bias) + residual, shape (..., N), for many positions
+    (ss2d_linear_tiles); no residual behind a GELU."""
+    if not x.is_cuda:
+        raise NotImplementedError("linear_tiles_hip: vmamba_amd runs on the GPU only")
+    if x.dtype not in _DTYPE_CODE:
+        raise TypeError(f"linear_tiles_hip: unsupported dtype {x.dtype}")
+    K = x.shape[-1]
+    if weight.dim() != 2 or weight.shape[1] != K:
+        raise ValueError(f"linear_tiles_hip: weight must be (N, {K}), got {tuple(weight.shape)}")
+    N = weight.shape[0]
+    for t, n in ((weight, N * K), (bias, N)):
+        if t is not None and (t.dtype != x.dtype or t.device != x.device or t.numel() != n or not t.is_contiguous()):
+            raise ValueError("linear_tiles_hip: contiguous parameters of x's dtype on its device")
+    x = x.contiguous()
+    out = x.new_empty(x.shape[:-1] + (N,))
+    if residual is not None:
+        if residual.shape != out.shape or residual.dtype != x.dtype or residual.device != x.device:
+            raise ValueError("linear_tiles_hip: residual must have the shape, dtype and device of the result")
+        residual = residual.contiguous()
+    ptr = lambda t: None if t is None else t.data_ptr()
+    rc = _lib.launch(x, _lib.lib().ss2d_linear_tiles, x.data_ptr(), weight.data_ptr(), ptr(bias), ptr(residual), out.data_ptr(), x.numel() // K, K, N,
+                     int(gelu), _DTYPE_CODE[x.dtype])
+    _lib.check(rc, "ss2d_linear_tiles")
+    return out
+
+
 def linear_cf_ln_fusable(K, weight, L):
     """True when ss2d_linear_cf_ln takes an fp32 channel-first map (B, K, L) with this 16-bit GPU weight (N, K)."""
     return (weight.is_cuda and weight.dtype in _DTYPE_CODE and weight.dim() == 2 and weight.shape[1] == K

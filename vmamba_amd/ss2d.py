@@ -27,7 +27,7 @@ from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_few_hip, core_fi
 from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
 from .conv import DwConv3x3SiLU, dwconv3x3_silu_hip, dwconv_silu_trainable
-from .linear import TENSOR_KINDS, LinearDw, few_positions, linear_cf_ln_fusable, linear_cf_ln_hip, linear_cl_hip, linear_dw_pays, linear_fusable, linear_rows_fusable, linear_rows_hip
+from .linear import TENSOR_KINDS, LinearDw, few_positions, linear_cf_ln_fusable, linear_cf_ln_hip, linear_cl_hip, linear_dw_pays, linear_fusable, linear_rows_fusable, linear_rows_hip, linear_tiles_fusable, linear_tiles_hip
 from .norm import (LayerNorm, LayerNorm2d, add_layer_norm_fusable, add_layer_norm_hip, layer_norm_cf_hip,
                    needs_grad)
 
@@ -415,7 +415,12 @@ class SS2D(nn.Module):
             x = linear_cl_hip(x, self.in_proj.weight, self.in_proj.bias, None, pre_norm.weight, pre_norm.bias, pre_norm.eps)
         else:
             x = x if pre_norm is None else pre_norm(x)
-            x = LinearDw.apply(x, self.in_proj.weight, None) if self.layers is HipLayers and linear_dw_pays(self.in_proj, x) else self.in_proj(x)
+            if self.layers is HipLayers and linear_dw_pays(self.in_proj, x):
+                x = LinearDw.apply(x, self.in_proj.weight, None)
+            elif self.layers is HipLayers and not self.channel_first and linear_tiles_fusable(x, self.in_proj):
+                x = linear_tiles_hip(x, self.in_proj.weight, self.in_proj.bias)
+            else:
+                x = self.in_proj(x)
         z = None
         if not self.disable_z:
             x, z = x.chunk(2, dim=(1 if self.channel_first else -1))
@@ -448,6 +453,8 @@ class SS2D(nn.Module):
         if trains:
             return LinearDw.apply(y, self.out_proj.weight, residual)
         if residual is None:
+            if self.layers is HipLayers and not self.channel_first and linear_tiles_fusable(y, self.out_proj):
+                return linear_tiles_hip(y, self.out_proj.weight, self.out_proj.bias)
             return self.out_proj(y)
         if self.channel_first or self.out_proj.bias is not None:
             return residual + self.out_proj(y)

@@ -19,13 +19,13 @@ import torch
 import torch.nn as nn
 
 from .block import vss_block_hip
-from .linear import TENSOR_KINDS, MlpF32, few_positions, linear_rows_fusable, linear_rows_hip, linear_rows_takes, mlp_f32_pays
+from .linear import TENSOR_KINDS, MlpF32, few_positions, linear_rows_fusable, linear_rows_hip, linear_rows_takes, linear_tiles_fusable, linear_tiles_hip, mlp_f32_pays
 from .mlp import mlp_fusable, mlp_fused_hip
 from .norm import LayerNorm as HipLayerNorm
 from .norm import add_layer_norm_fusable, add_layer_norm_hip, bias_layer_norm_fusable, bias_layer_norm_hip, needs_grad, observed
 from .ss2d import SS2D, HipLayers, Linear2d
 from .pool import GlobalAvgPool2d
-from .stem import stem2_fusable, stem_conv2_ln_hip, stem_conv_ln_gelu_hip, stem_fusable
+from .stem import conv_tiles_fusable, conv_tiles_hip, stem2_fusable, stem_conv2_ln_hip, stem_conv_ln_gelu_hip, stem_fusable
 
 
 class Permute(nn.Module):
@@ -65,7 +65,10 @@ class ConvNormSequence(nn.Sequential):
                     x = stem_conv2_ln_hip(x.permute(0, 2, 3, 1), conv.weight, conv.bias, norm.weight, norm.bias, norm.eps)
                     i += 3
                     continue
-                x = conv._conv_forward(x, conv.weight, None).permute(0, 2, 3, 1)
+                if conv_tiles_fusable(x, conv):
+                    x = conv_tiles_hip(x.permute(0, 2, 3, 1), conv.weight)
+                else:
+                    x = conv._conv_forward(x, conv.weight, None).permute(0, 2, 3, 1)
                 x = bias_layer_norm_hip(x, conv.bias, norm.weight, norm.bias, norm.eps)
                 i += 3
             else:
@@ -114,7 +117,7 @@ class Mlp(nn.Module):
         """fc2(GELU(fc1(h))) (+ residual), h = x or pre_norm(x) (the block's second LayerNorm, vmamba.py:1229).
         Channel-last 16-bit inference at widths 96 / 192 runs as one HIP kernel that normalises the rows on the way
         in and keeps the hidden activations in registers; few positions behind a norm as two launches of ss2d_linear_rows at
-        any width; single-precision training on the products of ss2d_product_f32 where those are the faster ones (MlpF32); everything else
+        any width; many positions of a wider layer with the GELU behind fc1's product (ss2d_linear_tiles); single-precision training on the products of ss2d_product_f32 where those are the faster ones (MlpF32); everything else
         on the torch operators.  A residual that the kernels cannot add -- one that autograd has to
         see, of another shape, type, device or kind -- is added by torch behind them."""
         rows = pre_norm is not None and few_positions(x) and self._rows(x, pre_norm)
@@ -133,6 +136,8 @@ class Mlp(nn.Module):
             h = x if pre_norm is None else pre_norm(x)
             if self.fused and not self.channel_first and mlp_f32_pays(h, self.fc1, self.act, self.fc2):
                 y = MlpF32.apply(h, self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias)
+            elif self.fused and not self.channel_first and linear_tiles_fusable(h, self.fc1, self.act):
+                y = self.fc2(linear_tiles_hip(h, self.fc1.weight, self.fc1.bias, gelu=True))
             else:
                 y = self.fc2(self.act(self.fc1(h)))
         return y if residual is None or add is not None else residual + y
