@@ -616,6 +616,18 @@ int ss2d_linear_tiles(const void *x, const void *weight, const void *bias, const
 int ss2d_conv3x3s2_cl(const void *x, const void *weight, const void *bias, void *out, int B, int H, int W, int C, int N, int dtype, void *stream);
 
 /*
+ * Backward of ss2d_layer_norm on fp32 rows (rows, C): x, dy and weight (C, or NULL for 1) -> dx (rows, C), dweight (C), dbias (C), any of them
+ * NULL where it is not wanted; the statistics are computed again from x.  And out[n] = sum over the rows of x[row][n], a bias gradient.
+ * Contiguous, 16-byte aligned, C a multiple of 4 up to 1024, N of 4 (SS2D_ENOTSUP otherwise, and without rows); dx neither x nor dy.
+ * workspace: ..._workspace_bytes(C or N) bytes (for dweight and dbias), 16-byte aligned.  No atomics: the same bits every time.
+ */
+int64_t ss2d_layer_norm_bwd_f32_workspace_bytes(int C);
+int ss2d_layer_norm_bwd_f32(const float *x, const float *dy, const float *weight, float eps, float *dx, float *dweight, float *dbias, int64_t rows, int C,
+                            void *workspace, int64_t workspace_bytes, void *stream);
+int64_t ss2d_column_sums_f32_workspace_bytes(int N);
+int ss2d_column_sums_f32(const float *x, float *out, int64_t rows, int N, void *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * A product in single precision on the bf16 matrix cores (each value as the sum of three bf16 ones, six products, fp32 sums; the error is
  * that of a product in fp32): out (M, N) with out[m][n] = sum over K of A(m, k) B(n, k), A stored (M, K) or by columns (K, M), B (N, K) or (K, N).
  *   mode 0: + bias (N) + other (M, N), either or both NULL.  mode 1: out = sum + bias, out2 = GELU(out).

@@ -50,6 +50,18 @@ def transpose_bcl_hip(x):
     return y
 
 
+class TransposeBCL(torch.autograd.Function):
+    """transpose_bcl_hip, and its own adjoint."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return transpose_bcl_hip(x)
+
+    @staticmethod
+    def backward(ctx, dy):
+        return TransposeBCL.apply(dy)
+
+
 def cross_scan_flex_hip(x, in_channel_first=True, out_channel_first=True, one_by_one=False, scans=0):
     """Any layout / mode of CrossScan; bit-exact for any 1/2/4/8-byte dtype.  Mixed layouts go through
     ss2d_cross_scan_flex_ws, which first brings x (the small side) to the layout of y with one tiled transpose into a

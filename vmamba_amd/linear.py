@@ -9,7 +9,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .norm import LayerNorm, needs_grad, observed, operators_seen
+from .norm import TENSOR_KINDS, LayerNorm, calls_unseen, column_sums, needs_grad, observed, operators_seen
 
 _DTYPE_CODE = {torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 FUSED_SHAPES = ((96, 96),)            # (in_features, out_features)
@@ -42,10 +42,6 @@ def linear_cl_hip(x, weight, bias=None, residual=None, ln_weight=None, ln_bias=N
                      ptr(small[2]), ptr(keep[1]), out.data_ptr(), x.numel() // K, K, N, _DTYPE_CODE[x.dtype])
     _lib.check(rc, "ss2d_linear_cl")
     return out
-
-
-# Other kinds of tensors (quantised or sharded weights, subclasses that see the calls they are in) are left to torch's operators.
-TENSOR_KINDS = (torch.Tensor, nn.Parameter)
 
 
 def _rows_params(x, *params):
@@ -300,11 +296,6 @@ def _weight_gradient(dy, x):
     return _product(dy, x, True, True)
 
 
-def calls_unseen():
-    """True when nothing but autograd follows the operators that are called: no mode or transform (operators_seen), no compiler or tracer."""
-    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or operators_seen() or torch.is_autocast_enabled())
-
-
 def _plain_f32(x, *tensors):
     return all(t is None or (type(t) in TENSOR_KINDS and t.dtype == torch.float32 and t.device == x.device) for t in tensors)
 
@@ -375,11 +366,11 @@ class MlpF32(torch.autograd.Function):
             act = nn.functional.gelu(pre)
         wants = ctx.needs_input_grad
         dw2 = _weight_gradient(dy2, act) if wants[3] else None
-        db2 = dy2.sum(0) if wants[4] else None
+        db2 = column_sums(dy2) if wants[4] else None
         if not any(wants[:3]):
             return None, None, None, dw2, db2
         dpre = _product(dy2, w2, b_by_columns=True, other=pre, mode=PRODUCT_GELU_GRAD)
         dw1 = _weight_gradient(dpre, x2) if wants[1] else None
-        db1 = dpre.sum(0) if wants[2] else None
+        db1 = column_sums(dpre) if wants[2] else None
         dx = _product(dpre, w1, b_by_columns=True).view(x.shape) if wants[0] else None
         return dx, dw1, db1, dw2, db2

@@ -122,6 +122,69 @@ def observed(layer):
     return any(hooks) or nn.modules.module._has_any_global_hook() or "forward" in vars(layer)
 
 
+# Other kinds of tensors (quantised or sharded weights, subclasses that see the calls they are in) are left to torch's operators.
+TENSOR_KINDS = (torch.Tensor, nn.Parameter)
+
+
+def layer_norm_trains(x, normalized_shape, weight, bias, C=None):
+    """True when LayerNormF32 stands for F.layer_norm over the C channels of x (default: its last axis) in training: float32 on the GPU, a
+    multiple of 4 channels up to 1024, and operators that nothing sees."""
+    if C is None:
+        C = x.shape[-1] if x.dim() else 0
+    return (type(x) in TENSOR_KINDS and x.is_cuda and x.dtype == torch.float32 and x.numel() > 0 and tuple(normalized_shape) == (C,) and C % 4 == 0
+            and C <= 1024 and all(t is None or (type(t) in TENSOR_KINDS and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
+                                                and t.data_ptr() % 16 == 0) for t in (weight, bias)) and calls_unseen())
+
+
+class LayerNormF32(torch.autograd.Function):
+    """F.layer_norm over the last axis with its backward on ss2d_layer_norm_bwd_f32, which computes the statistics again from x."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, eps):
+        ctx.save_for_backward(x, weight)
+        ctx.eps = eps
+        return layer_norm_hip(x, weight, bias, eps)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        wants = ctx.needs_input_grad
+        C = x.shape[-1]
+        if torch.is_grad_enabled():                                  # a second backward goes through the torch operators
+            mean = x.mean(-1, keepdim=True)
+            centred = x - mean
+            rstd = (centred.square().mean(-1, keepdim=True) + ctx.eps).rsqrt()
+            xhat, g = centred * rstd, dy if weight is None else dy * weight
+            dx = rstd * (g - g.mean(-1, keepdim=True) - xhat * (g * xhat).mean(-1, keepdim=True)) if wants[0] else None
+            return dx, (dy * xhat).reshape(-1, C).sum(0) if wants[1] else None, dy.reshape(-1, C).sum(0) if wants[2] else None, None
+        x, dy = x.contiguous(), dy.contiguous()
+        if (x.data_ptr() | dy.data_ptr()) % 16:                      # (views between 16-byte boundaries)
+            x, dy = x.clone(), dy.clone()
+        dx = torch.empty_like(x) if wants[0] else None
+        dw, db = (torch.empty(C, dtype=x.dtype, device=x.device) if want else None for want in wants[1:3])
+        L = _lib.lib()
+        need = L.ss2d_layer_norm_bwd_f32_workspace_bytes(C)
+        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+        ptr = lambda t: None if t is None else t.data_ptr()
+        rc = _lib.launch(x, L.ss2d_layer_norm_bwd_f32, x.data_ptr(), dy.data_ptr(), ptr(weight), ctx.eps, ptr(dx), ptr(dw), ptr(db), x.numel() // C, C,
+                         workspace.data_ptr(), need)
+        _lib.check(rc, "ss2d_layer_norm_bwd_f32")
+        return dx, dw, db, None
+
+
+def column_sums(x):
+    """x.sum(0) of a float32 matrix (ss2d_column_sums_f32; the library's where autograd follows or the kernel has no variant)."""
+    if torch.is_grad_enabled() or x.dtype != torch.float32 or not x.is_contiguous() or x.numel() == 0 or x.shape[1] % 4 or x.data_ptr() % 16:
+        return x.sum(0)
+    rows, N = x.shape
+    out = torch.empty(N, dtype=x.dtype, device=x.device)
+    L = _lib.lib()
+    need = L.ss2d_column_sums_f32_workspace_bytes(N)
+    workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+    _lib.check(_lib.launch(x, L.ss2d_column_sums_f32, x.data_ptr(), out.data_ptr(), rows, N, workspace.data_ptr(), need), "ss2d_column_sums_f32")
+    return out
+
+
 def _gpu_only(x, what):
     if not x.is_cuda:
         raise NotImplementedError(f"{what}: vmamba_amd runs on the GPU only (got a {x.device.type} tensor)")
@@ -131,6 +194,8 @@ class LayerNorm(nn.LayerNorm):
     def forward(self, x):
         _gpu_only(x, "LayerNorm")
         if needs_grad(x, self.weight, self.bias):
+            if layer_norm_trains(x, self.normalized_shape, self.weight, self.bias):
+                return LayerNormF32.apply(x, self.weight, self.bias, self.eps)
             return F.layer_norm(x, self.normalized_shape, self.weight, self.bias, self.eps)
         return layer_norm_hip(x, self.weight, self.bias, self.eps)
 
@@ -163,3 +228,8 @@ def operators_seen():
         return True
     modes = functions()
     return modes > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))
+
+
+def calls_unseen():
+    """True when nothing but autograd follows the operators that are called: no mode or transform (operators_seen), no compiler or tracer."""
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or operators_seen() or torch.is_autocast_enabled())

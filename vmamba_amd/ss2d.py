@@ -24,12 +24,12 @@ from ._lib import SS2D_ENOTSUP, Ss2dError
 from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_few_hip, core_fits, core_mask_pads_hip, dt_proj_f32_hip, dt_proj_hip,
                    embed_maps_hip, few_applies, forward_core_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_f32_pays,
                    x_proj_fits, x_proj_hip, x_proj_pays)
-from .csm import cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
+from .csm import TransposeBCL, cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
 from .conv import DwConv3x3SiLU, dwconv3x3_silu_hip, dwconv_silu_trainable
 from .linear import TENSOR_KINDS, LinearDw, few_positions, linear_cf_ln_fusable, linear_cf_ln_hip, linear_cl_hip, linear_dw_pays, linear_fusable, linear_rows_fusable, linear_rows_hip, linear_tiles_fusable, linear_tiles_hip
-from .norm import (LayerNorm, LayerNorm2d, add_layer_norm_fusable, add_layer_norm_hip, layer_norm_cf_hip,
-                   needs_grad)
+from .norm import (LayerNorm, LayerNorm2d, LayerNormF32, add_layer_norm_fusable, add_layer_norm_hip, layer_norm_cf_hip,
+                   layer_norm_trains, needs_grad)
 
 
 class Linear2d(nn.Linear):
@@ -56,6 +56,10 @@ class HipLayers:
         layout and dtype: one kernel reads (B, D, L) and writes the normalised (B, D, L) or (B, L, D).  Under
         autograd: the reference's own torch operators (vmamba.py:641-646)."""
         if needs_grad(y, norm.weight, norm.bias):
+            B, D, H, W = y.shape
+            if not channel_first and y.is_contiguous() and layer_norm_trains(y, norm.normalized_shape, norm.weight, norm.bias, D):
+                rows = TransposeBCL.apply(y.view(B, D, H * W)).view(B, H, W, D)
+                return LayerNormF32.apply(rows, norm.weight, norm.bias, norm.eps).to(dtype)
             out = F.layer_norm(y.permute(0, 2, 3, 1), norm.normalized_shape, norm.weight, norm.bias, norm.eps)
             return (out.permute(0, 3, 1, 2) if channel_first else out).to(dtype)
         return layer_norm_cf_hip(y, norm.weight, norm.bias, norm.eps, out_channel_last=not channel_first, out_dtype=dtype)
