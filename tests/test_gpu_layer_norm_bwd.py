@@ -53,18 +53,19 @@ def test_column_sums(rows, N):
 
 
 def test_who_takes_it():
-    norm, x = LayerNorm(96).to(DEV), torch.randn(10, 96, device=DEV, requires_grad=True)
+    norm, x = LayerNorm(96).to(DEV), torch.randn(22000, 96, device=DEV, requires_grad=True)
     takes = lambda t=x, n=norm: layer_norm_trains(t, n.normalized_shape, n.weight, n.bias)
-    assert takes() and not takes(x.half()) and not takes(x[:0]) and not takes(x[:, :48]) and norm(x).grad_fn.name().startswith("LayerNormF32")
-    assert not takes(n=LayerNorm(96).to(DEV).half()) and not takes(torch.randn(4, 1028, device=DEV), LayerNorm(1028).to(DEV))
+    assert takes() and not takes(x.half()) and not takes(x[:21000]) and not takes(x[:, :48]) and norm(x).grad_fn.name().startswith("LayerNormF32")
+    assert not takes(n=LayerNorm(96).to(DEV).half()) and not takes(torch.randn(2100, 1028, device=DEV), LayerNorm(1028).to(DEV))
     with torch.autocast("cuda", torch.bfloat16):
         assert not takes()
     with torch.autograd.forward_ad.dual_level():
         assert not takes()
     assert torch.func.grad(lambda t: norm(t).square().sum())(x).shape == x.shape
     # a non-contiguous gradient and views between 16-byte boundaries
-    shifted = torch.randn(961, device=DEV)[1:].view(10, 96).requires_grad_()
-    for t, dy in ((x, torch.randn(96, 10, device=DEV).t()), (shifted, torch.randn(961, device=DEV)[1:].view(10, 96))):
+    off = lambda: torch.randn(22000 * 96 + 1, device=DEV)[1:].view(22000, 96)
+    shifted = off().requires_grad_()
+    for t, dy in ((x, torch.randn(96, 22000, device=DEV).t()), (shifted, off())):
         got, want = (torch.autograd.grad(f(t), t, dy)[0] for f in (norm, lambda t: F.layer_norm(t, (96,), norm.weight, norm.bias)))
         assert torch.allclose(got, want, rtol=1e-4, atol=1e-5)
 
@@ -75,10 +76,11 @@ def test_out_norm_of_a_map():
     op = SS2D(d_model=64, channel_first=False).to(DEV)
     with torch.no_grad():
         op.out_norm.weight.uniform_(0.5, 1.5)
-    y = torch.randn(3, 64, 9, 7, device=DEV, requires_grad=True)
-    dy = torch.randn(3, 9, 7, 64, device=DEV)
-    got = op.finish_core(y.view(3, 64, 63), 3, 64, 9, 7, torch.float32)
+    y = torch.randn(600, 64, 9, 7, device=DEV, requires_grad=True)
+    dy = torch.randn(600, 9, 7, 64, device=DEV)
+    got = op.finish_core(y.view(600, 64, 63), 600, 64, 9, 7, torch.float32)
+    assert got.grad_fn.name().startswith("LayerNormF32")
     want = F.layer_norm(y.permute(0, 2, 3, 1), (64,), op.out_norm.weight, op.out_norm.bias)
     assert torch.allclose(got, want, rtol=1e-5, atol=1e-5)
     for a, b in zip(torch.autograd.grad(got, [y, op.out_norm.weight], dy), torch.autograd.grad(want, [y, op.out_norm.weight], dy)):
-        assert torch.allclose(a, b, rtol=1e-4, atol=1e-5)
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-5 * max(1.0, b.abs().max().item()))

@@ -87,7 +87,7 @@ def test_mlp_autograd(bias):
     mlp = Mlp(96, 384, channel_first=False).to(DEV)
     if not bias:
         mlp.fc1.bias = mlp.fc2.bias = None
-    x = torch.randn(4, 56, 56, 96, device=DEV, requires_grad=True)
+    x = torch.randn(7, 56, 56, 96, device=DEV, requires_grad=True)
     dy = torch.randn_like(x)
     assert mlp_f32_pays(x, mlp.fc1, mlp.act, mlp.fc2)
     params = [x] + list(mlp.parameters())
@@ -109,9 +109,9 @@ def test_mlp_autograd(bias):
 
 def test_who_is_left_to_the_operators():
     mlp = Mlp(96, 384, channel_first=False).to(DEV)
-    x = torch.randn(12544, 96, device=DEV)
+    x = torch.randn(22000, 96, device=DEV)
     takes = lambda t=x: mlp_f32_pays(t, mlp.fc1, mlp.act, mlp.fc2)
-    assert takes() and not takes(x[:784]) and not takes(x.half())
+    assert takes() and not takes(x[:21000]) and not takes(x.half())
     with torch.no_grad():
         assert not takes()
     with torch.autocast("cuda", dtype=torch.bfloat16):
@@ -142,3 +142,34 @@ def test_projection_with_residual():
     w, xd = layer.weight.double(), x.double()
     for g, want in zip(got, (r.double() + xd @ w.t(), dy.double() @ w, dy.double().t() @ xd)):
         assert ((g.double() - want).norm() / want.norm()).item() < 2e-6
+
+
+def test_projections_of_the_core_in_training():
+    """x_proj and dt_proj of forward_core on the kernels, their gradients against the operators they stand for (sums of 96 and 21 952 terms)."""
+    from vmamba_amd import ss2d
+    torch.manual_seed(0)
+    op = ss2d.SS2D(d_model=96, channel_first=False).to(DEV)
+    x = torch.randn(28, 96, 28, 28, device=DEV, requires_grad=True)
+    dy = torch.randn(28, 28, 28, 96, device=DEV)
+    wanted = [x] + [p for n, p in op.named_parameters() if n.split(".")[0] in ("x_proj_weight", "dt_projs_weight", "A_logs", "Ds", "dt_projs_bias")]
+    def run():
+        y = op.forward_core(x)
+        return (y.detach(),) + torch.autograd.grad(y, wanted, dy)
+    calls, apply = [], ss2d.XProjF32.apply
+    ss2d.XProjF32.apply = lambda *a: calls.append(1) or apply(*a)
+    try:
+        got = run()
+    finally:
+        ss2d.XProjF32.apply = apply
+    assert calls
+    takes, ss2d.projections_train = ss2d.projections_train, lambda *a: False
+    try:
+        want = run()
+    finally:
+        ss2d.projections_train = takes
+    for g, w in zip(got, want):
+        assert ((g - w).norm() / w.norm()).item() < 1e-5
+    # a second backward through the projections
+    rows = ss2d.XProjF32.apply(x, op.x_proj_weight)
+    dx = torch.autograd.grad(rows.square().sum(), x, create_graph=True)[0]
+    assert torch.autograd.grad(dx.sum(), op.x_proj_weight)[0].isfinite().all()

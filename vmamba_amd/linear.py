@@ -9,7 +9,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .norm import TENSOR_KINDS, LayerNorm, calls_unseen, column_sums, needs_grad, observed, operators_seen
+from .norm import TENSOR_KINDS, TRAIN_FROM, LayerNorm, calls_unseen, column_sums, needs_grad, observed, operators_seen
 
 _DTYPE_CODE = {torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 FUSED_SHAPES = ((96, 96),)            # (in_features, out_features)
@@ -272,8 +272,8 @@ def _product(a, b, a_by_columns=False, b_by_columns=False, bias=None, other=None
     own), for views that start between 16-byte boundaries and where it is the faster one."""
     M, K = a.shape[::-1] if a_by_columns else a.shape
     N = b.shape[1] if b_by_columns else b.shape[0]
-    rows = (M if a_by_columns else K, N if b_by_columns else K, N)
-    if not torch.is_grad_enabled() and all(n % 4 == 0 for n in rows) and M * N * K > 0 and product_pays(M, N, K, a_by_columns and b_by_columns):
+    if (product_pays(M, N, K, a_by_columns and b_by_columns) and not torch.is_grad_enabled() and N % 4 == 0 and (M if a_by_columns else K) % 4 == 0
+            and (b_by_columns or K % 4 == 0) and M * N * K > 0):
         a, b = a.contiguous(), b.contiguous()
         other = None if other is None else other.contiguous()
         if all(t is None or t.data_ptr() % 16 == 0 for t in (a, b, bias, other)):
@@ -311,7 +311,7 @@ def linear_dw_pays(layer, x):
     N, K = weight.shape
     return (torch.is_grad_enabled() and weight.requires_grad and weight.dtype == x.dtype and weight.device == x.device
             and x.shape[-1] == K and N % 4 == 0 and K % 4 == 0 and N * K > 0 and x.numel() >= 4096 * K
-            and (N * K <= 384 * 384 or product_pays(x.numel() // K, N, K)) and not observed(layer) and calls_unseen())
+            and (N * K <= 384 * 384 or (x.numel() >= TRAIN_FROM and product_pays(x.numel() // K, N, K))) and not observed(layer) and calls_unseen())
 
 
 class LinearDw(torch.autograd.Function):
@@ -336,8 +336,8 @@ class LinearDw(torch.autograd.Function):
 
 def mlp_f32_pays(x, fc1, act, fc2):
     """True when MlpF32 stands for ``fc2(act(fc1(x)))`` in training: plain nn.Linear layers and exact GELU that nothing observes, contiguous
-    float32 parameters, and a first product that ss2d_product_f32 is ahead in."""
-    if not (type(x) in TENSOR_KINDS and x.is_cuda and x.dtype == torch.float32 and x.dim() >= 2 and type(fc1) is type(fc2) is nn.Linear
+    float32 parameters, TRAIN_FROM elements, and a first product that ss2d_product_f32 is ahead in."""
+    if not (x.dtype == torch.float32 and x.numel() >= TRAIN_FROM and type(x) in TENSOR_KINDS and x.is_cuda and x.dim() >= 2 and type(fc1) is type(fc2) is nn.Linear
             and type(act) is nn.GELU and act.approximate == "none"):
         return False
     N, K = fc1.weight.shape

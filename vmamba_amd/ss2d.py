@@ -21,8 +21,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ._lib import SS2D_ENOTSUP, Ss2dError
-from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, core_few_hip, core_fits, core_mask_pads_hip, dt_proj_f32_hip, dt_proj_hip,
-                   embed_maps_hip, few_applies, forward_core_hip, padded_map_size, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_f32_pays,
+from .core import (DT_PROJ_F32_MAX_RANK, DT_PROJ_MAX_RANK, DtProjF32, XProjF32, core_few_hip, core_fits, core_mask_pads_hip, dt_proj_f32_hip, dt_proj_hip,
+                   embed_maps_hip, few_applies, forward_core_hip, padded_map_size, projections_train, ss2d_core_hip, x_proj_f32_fits, x_proj_f32_hip, x_proj_f32_pays,
                    x_proj_fits, x_proj_hip, x_proj_pays)
 from .csm import TransposeBCL, cross_merge_fn, cross_scan_1b1_hip, cross_scan_fn
 from .csms6s import selective_scan_fn, selective_scan_from_map
@@ -227,7 +227,10 @@ class SS2D(nn.Module):
         direction's rows in that direction's order.  x_proj then reads the map once instead of its four copies."""
         B, D, H, W = x.shape
         K, L, R, N = self.k_group, H * W, self.dt_rank, self.d_state
-        if x_proj_pays(x, self.x_proj_weight) and x_proj_fits(x, self.x_proj_weight) and not needs_grad(x, self.x_proj_weight):
+        trains = "Wx_all" not in consts              # forward_core's: the kernels take the weights as they are
+        if trains:
+            x_dbl = XProjF32.apply(x, self.x_proj_weight)
+        elif x_proj_pays(x, self.x_proj_weight) and x_proj_fits(x, self.x_proj_weight) and not needs_grad(x, self.x_proj_weight):
             x_dbl = x_proj_hip(x, self.x_proj_weight, x.new_empty((B, K, R + 2 * N, L)))
         elif (x_proj_f32_fits(x, self.x_proj_weight) and x_proj_f32_pays(x, self.x_proj_weight)
               and not needs_grad(x, self.x_proj_weight)):
@@ -237,7 +240,9 @@ class SS2D(nn.Module):
             x_dbl = cross_scan_fn(proj, in_channel_first=True, out_channel_first=True, one_by_one=True, scans=0)   # (B, K, R+2N, L)
         dts, Bs, Cs = torch.split(x_dbl, [R, N, N], dim=2)
         dts = dts.reshape(B * K, R, L)
-        if dts.dtype != torch.float32 and R <= DT_PROJ_MAX_RANK and not needs_grad(dts, self.dt_projs_weight):
+        if trains:
+            dts = DtProjF32.apply(dts, self.dt_projs_weight.unsqueeze(0).expand(B, -1, -1, -1).reshape(B * K, D, R))
+        elif dts.dtype != torch.float32 and R <= DT_PROJ_MAX_RANK and not needs_grad(dts, self.dt_projs_weight):
             dts = dt_proj_hip(dts, consts["Wdt"])                     # one (image, direction) problem per weight copy
         elif dts.dtype == torch.float32 and dts.is_cuda and R <= DT_PROJ_F32_MAX_RANK and not needs_grad(dts, self.dt_projs_weight):
             dts = dt_proj_f32_hip(dts, consts["Wdt"])
@@ -337,8 +342,9 @@ class SS2D(nn.Module):
             return out
         B, D, H, W = x.shape
         K, L = self.k_group, H * W
-        consts = self._inference_constants(B)
-        if self._fused_core_applies(x):
+        trains = needs_grad(x, self.x_proj_weight, self.dt_projs_weight) and projections_train(x, self.x_proj_weight, self.dt_projs_weight)
+        consts = self._inference_constants(0 if trains else B)
+        if not trains and self._fused_core_applies(x):
             try:
                 # out_norm runs on the map the kernel ran on (a padded map has rows the norm's vector paths like as
                 # well) and the added rows / columns are cut off its 16-bit result, half the bytes of the fp32 map
