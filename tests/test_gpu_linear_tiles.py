@@ -39,6 +39,21 @@ def test_linear(M, K, N, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N", [(128 * 1024, 32, 8), (128 * 1024 + 1, 32, 8), (128 * 1024 + 127, 64, 16), (128 * 512 + 5, 96, 200), (43 * 128 - 3, 160, 192 * 24 - 8)])
+def test_linear_of_many_tiles(M, K, N, dtype):
+    """The GELU on both sides of 1024 workgroups, from where on the ring has two buffers: one step and several, edges in both directions."""
+    print("CASE linear_tiles many", M, K, N, dtype, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, w = torch.randn(M, K, generator=g, device=DEV).to(dtype), (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).to(dtype)
+    b = torch.randn(N, generator=g, device=DEV).to(dtype)
+    z = x.double() @ w.double().t() + b.double()
+    terms = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+    pre = linear_tiles_hip(x, w, b)
+    assert near(pre, z, terms, dtype)
+    assert near(linear_tiles_hip(x, w, b, gelu=True), F.gelu(pre.double()), 2e-7, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,H,W,C,N", [(1, 1, 1, 32, 8), (2, 2, 3, 32, 192), (3, 7, 9, 64, 200), (1, 16, 15, 96, 192), (2, 23, 1, 32, 40), (5, 14, 14, 192, 384)])
 def test_convolution(B, H, W, C, N, dtype):
     print("CASE conv_tiles", B, H, W, C, N, dtype, flush=True)

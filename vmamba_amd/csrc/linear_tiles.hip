@@ -3,8 +3,8 @@
 //     out[m][n] = [GELU](sum_k x[m][k] w[n][k] + bias[n]) + residual[m][n]
 // and, for a convolution, x[m][k] = the input pixel and channel that term k = (kh, kw, c) of output pixel m meets, 0 outside the image.
 //   * a workgroup of four wavefronts owns kBM x kBN outputs, a wavefront a quarter of them in tiles of 32 x 32; 32 terms a step.  Operands
-//     go from memory straight into LDS (global_load_lds, 16 bytes a lane), two steps ahead in a ring of three buffers: one barrier a
-//     step, and a wait that leaves the newer step's loads in flight;
+//     go from memory straight into LDS (global_load_lds, 16 bytes a lane), two steps ahead in a ring of three buffers -- one barrier a
+//     step, and a wait that leaves the newer step's loads in flight --, or one step ahead in a ring of two (kTlThreePerCu);
 //   * a row of a step is 64 bytes of LDS, its four 16-byte pieces in an order that differs from row to row, so that lanes with a row each read
 //     all banks once; the order is made by the addresses the lanes load from, the LDS side being linear;
 //   * a lane's accumulators are runs of four outputs of one position.  They go through LDS into rows, which leave 16 bytes a lane with the
@@ -26,13 +26,13 @@ struct TilesArgs {
     FastDiv div_image, div_wo;                                       // Ho * Wo, Wo
 };
 
-constexpr int kTlDepth = 32, kTlStages = 3;
+constexpr int kTlDepth = 32;
 
-template <typename T, int kBM, int kBN, bool kGelu> struct TilesLayout {
+template <typename T, int kBM, int kBN, bool kGelu, int kStages> struct TilesLayout {
     static constexpr int kStage = (kBM + kBN) * kTlDepth;            // elements
     static constexpr int kPitch = kBN + 8;                           // of the outputs' rows
     static constexpr bool kTable = kGelu && ElemTraits<T>::dtype == SS2D_BF16;
-    static constexpr int kElems = kTlStages * kStage > 64 * kPitch ? kTlStages * kStage : 64 * kPitch;
+    static constexpr int kElems = kStages * kStage > 64 * kPitch ? kStages * kStage : 64 * kPitch;
     static constexpr size_t kBytes = (size_t)kElems * 2 + (kTable ? kGeluEntries * sizeof(float) : 0);
 };
 
@@ -46,9 +46,9 @@ template <int kNewer> __device__ __forceinline__ void tl_wait_and_meet() {
 
 __device__ const uint4 kTlZeros = {0u, 0u, 0u, 0u};                     // what a pixel outside the image is loaded from
 
-template <typename T, int kBM, int kBN, bool kGelu, bool kConv>
-__global__ __launch_bounds__(kBlock, 2) void linear_tiles_kernel(const TilesArgs p) {
-    using Lay = TilesLayout<T, kBM, kBN, kGelu>;
+template <typename T, int kBM, int kBN, bool kGelu, bool kConv, int kStages>
+__global__ __launch_bounds__(kBlock, kStages == 2 ? 3 : 2) void linear_tiles_kernel(const TilesArgs p) {
+    using Lay = TilesLayout<T, kBM, kBN, kGelu, kStages>;
     constexpr int kI = kBM / 64, kE = kBN / 64;                       // a wavefront's 32 x 32 tiles along positions and outputs
     constexpr int kLoadsA = kBM / 64, kLoadsB = kBN / 64;             // of a wavefront a step: 16 rows each
     extern __shared__ __align__(16) uint16_t tl_smem[];
@@ -124,13 +124,13 @@ __global__ __launch_bounds__(kBlock, 2) void linear_tiles_kernel(const TilesArgs
             reinterpret_cast<uint4 *>(tbl)[i] = reinterpret_cast<const uint4 *>(kGeluHalfErfBits)[i];
     const int wm = (wave & 1) * (kBM / 2), wn = (wave >> 1) * (kBN / 2);
     fetch(0, 0);
-    if (steps > 1) fetch(1, 1);
+    if (kStages > 2 && steps > 1) fetch(1, 1);
     int buffer = 0;
     for (int step = 0; step < steps; ++step) {
-        if (step + 1 < steps) tl_wait_and_meet<kLoadsA + kLoadsB>();
+        if (kStages > 2 && step + 1 < steps) tl_wait_and_meet<kLoadsA + kLoadsB>();
         else tl_wait_and_meet<0>();
         // (the buffer filled here was read in the step before this one, which every wavefront has left)
-        if (step + 2 < steps) fetch(step + 2, buffer == 0 ? 2 : buffer - 1);
+        if (step + kStages - 1 < steps) fetch(step + kStages - 1, buffer == 0 ? kStages - 1 : buffer - 1);
         const uint16_t *sa = tl_smem + buffer * Lay::kStage, *sb = sa + kBM * kTlDepth;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kBlock, 2) void linear_tiles_kernel(const TilesArgs
 #pragma unroll
                 for (int e = 0; e < kE; ++e) acc[i][e] = mfma_32x32x16(T{}, fb[e], fa[i], acc[i][e]);
         }
-        buffer = buffer == 2 ? 0 : buffer + 1;
+        buffer = buffer == kStages - 1 ? 0 : buffer + 1;
     }
     // ---- out, 64 positions at a time through the ring's room: a lane holds, of position wm + 32 i + j, outputs wn + 32 e + 8 g + 4 kh + t
     // in accumulator 4 g + t
@@ -189,23 +189,32 @@ __global__ __launch_bounds__(kBlock, 2) void linear_tiles_kernel(const TilesArgs
     }
 }
 
-template <typename T, int kBM, int kBN, bool kGelu, bool kConv>
+template <typename T, int kBM, int kBN, bool kGelu, bool kConv, int kStages>
 static int launch_tiles(TilesArgs a, hipStream_t s) {
     a.tiles_n = (a.N + kBN - 1) / kBN;
     const int64_t total = (a.M + kBM - 1) / kBM * a.tiles_n;
     if (total > 0x7fffffff) return SS2D_ENOTSUP;
     a.total = (uint32_t)total;
-    auto kern = linear_tiles_kernel<T, kBM, kBN, kGelu, kConv>;
-    constexpr size_t smem = TilesLayout<T, kBM, kBN, kGelu>::kBytes;
+    auto kern = linear_tiles_kernel<T, kBM, kBN, kGelu, kConv, kStages>;
+    constexpr size_t smem = TilesLayout<T, kBM, kBN, kGelu, kStages>::kBytes;
     if (smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
         return SS2D_ELAUNCH;
     hipLaunchKernelGGL(kern, dim3(a.total), dim3(kBlock), smem, s, a);
     return launch_status();
 }
 
+// With the GELU a workgroup's time is two parts, the product and what stands behind it (a gather of the table and a pass through LDS), that only
+// other workgroups of the CU overlap.  A ring of two buffers leaves room for three of them (50 KB of LDS; the loads one step ahead, which the other
+// two cover) where a ring of three leaves two.  us, three buffers / two, bf16 and fp16: 384 -> 1536 at 25 088 positions (1568 workgroups)
+// 65 / 61 and 74 / 67, at 50 176 115 / 104 and 130 / 117, at 100 352 261 / 229 and 285 / 259; 512 -> 2048 at 12 544 (1078) 55 / 48 and 60 / 56.
+// About as many workgroups as places, or fewer, gain nothing: 384 -> 1536 at 12 544 (784) 38 / 39 and 43 / 42, 256 -> 1024 at 17 000 (798) 31.5 / 32.3 and 38 / 36.
+constexpr int64_t kTlThreePerCu = 1024;
+
 template <typename T> static int launch_linear_tiles(const TilesArgs &a, bool gelu, hipStream_t s) {
-    if (gelu) return launch_tiles<T, 128, 192, true, false>(a, s);
-    return launch_tiles<T, 128, 192, false, false>(a, s);
+    const int64_t total = (a.M + 127) / 128 * ((a.N + 191) / 192);
+    if (gelu && total > kTlThreePerCu) return launch_tiles<T, 128, 192, true, false, 2>(a, s);
+    if (gelu) return launch_tiles<T, 128, 192, true, false, 3>(a, s);
+    return launch_tiles<T, 128, 192, false, false, 3>(a, s);
 }
 
 }  // namespace ss2d
@@ -241,6 +250,6 @@ extern "C" int ss2d_conv3x3s2_cl(const void *x, const void *weight, const void *
     TilesArgs a = {};
     a.x = x; a.w = weight; a.bias = bias; a.out = out; a.M = M; a.K = 9 * C; a.N = N; a.H = H; a.W = W; a.C = C;
     a.div_image = make_fastdiv((uint32_t)(Ho * Wo)); a.div_wo = make_fastdiv((uint32_t)Wo);
-    if (dtype == SS2D_BF16) return launch_tiles<bf16_t, 128, 192, false, true>(a, (hipStream_t)stream);
-    return launch_tiles<f16_t, 128, 192, false, true>(a, (hipStream_t)stream);
+    if (dtype == SS2D_BF16) return launch_tiles<bf16_t, 128, 192, false, true, 3>(a, (hipStream_t)stream);
+    return launch_tiles<f16_t, 128, 192, false, true, 3>(a, (hipStream_t)stream);
 }
