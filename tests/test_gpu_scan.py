@@ -166,6 +166,51 @@ def test_scan_channel_per_lane_kernel_matches_oracle(batch, dim, G, N, L, dtype)
     check_states(x, xw)
 
 
+# Few workgroups: the rows are cut into segments.  The fewest and shortest of them (3 of 128), one position group less (whole), a last
+# segment that would be too short for its state (joined to the one before), many segments, 2048 inside one and at the end of one,
+# both sides of 64 workgroups (400 positions) and of four segments (512 and 504 positions, 96 workgroups).
+SEGMENTS = [(1, 64, 1, 32, 384), (1, 64, 1, 32, 376), (1, 48, 1, 32, 520), (1, 96, 1, 16, 4112), (1, 64, 1, 4, 4096), (1, 33, 1, 8, 9000),
+            (64, 64, 1, 16, 400), (65, 64, 1, 16, 400), (96, 64, 1, 4, 512), (96, 64, 1, 4, 504)]
+
+
+@pytest.mark.parametrize("batch,dim,G,N,L", SEGMENTS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_rows_cut_into_segments(batch, dim, G, N, L, dtype):
+    """Against the oracle, with the chunk states and without, and in the input's own dtype (whose rows hold the segments' states)."""
+    _announce("scan-segments", batch, dim, G, N, L, dtype)
+    args = make_inputs(33, batch, dim, G, N, L, dtype, ss2d_like=True)
+    assert kernel_of(*args[:5], want_x=False) == "chan"
+    want, xw = orc.selective_scan(*args, True, out_float=True, return_x=True)
+    got, x = run_gpu(*args, True, True, want_x=True)
+    assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
+    check_states(x, xw, TOL32)
+    assert torch.equal(run_gpu(*args, True, True, want_x=False)[0], got)
+    if dtype != torch.float32:
+        small, _ = run_gpu(*args, True, False, want_x=False)
+        assert torch.equal(small, got.to(dtype))
+
+
+def test_scan_segments_hold_what_a_whole_row_does():
+    """A state of 0 enters a segment whose decays multiply to infinity, as it would position by position; NaN and infinity go on
+    through the segments behind them and stay out of the ones before."""
+    batch, dim, N, L = 1, 64, 16, 2048
+    u, delta, A, B, C, D, bias = make_inputs(34, batch, dim, 1, N, L, torch.float32, ss2d_like=True)
+    A = torch.full_like(A, 0.5)                                      # growing: 2048 steps of about 1.3
+    delta = torch.full_like(delta, 1.0)
+    u[:, :, :1800] = 0.0
+    want = orc.selective_scan(u, delta, A, B, C, D, bias, True, out_float=True, return_x=True)[0]
+    got, _ = run_gpu(u, delta, A, B, C, D, bias, True, True, want_x=False)
+    assert torch.equal(got[:, :, :1800], want[:, :, :1800]) and not bool(got[:, :, :1800].isnan().any())
+    assert torch.equal(got.isfinite(), want.isfinite())
+    u, delta, A, B, C, D, bias = make_inputs(35, batch, dim, 1, N, L, torch.float32, ss2d_like=True)
+    u[0, 3, 700], delta[0, 5, 900] = float("nan"), float("inf")
+    want = orc.selective_scan(u, delta, A, B, C, D, bias, True, out_float=True, return_x=True)[0]
+    got, _ = run_gpu(u, delta, A, B, C, D, bias, True, True, want_x=False)
+    assert torch.equal(got.isnan(), want.isnan()) and bool(got[0, 3, 700:].isnan().all()) and not bool(got[0, 3, :700].isnan().any())
+    ok = want.isfinite()
+    assert torch.allclose(got[ok], want[ok], **TOL32)
+
+
 @pytest.mark.parametrize("batch,Dm,H,W,N", [(2, 32, 8, 8, 16), (1, 64, 14, 12, 4), (2, 48, 7, 8, 8), (1, 96, 56, 56, 16), (3, 40, 4, 6, 32)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_scan_reading_the_map_through_the_cross_scan_routes(batch, Dm, H, W, N, dtype):

@@ -17,6 +17,10 @@
 //   compute  twice 16 positions: every lane reads its channel's dl / du (16-byte LDS reads), runs its wavefront's
 //            states over them and leaves 16 partial outputs in LDS;
 //   combine  thread (r, q) adds the four partials and the skip term for 4 positions and stores them (16 bytes of fp32).
+//
+// Few workgroups (small batches) leave the chip idle behind that serial chain.  Their rows are cut into segments that run side by side
+// in two launches of the same kernel, with one between them that walks the segments (ChanPhase, chan_segments): what a segment leaves
+// from state 0 and its sum of dl; what enters each, h_in' = exp2(A sum dl) h_in + h; the outputs from there.
 #include "scan_common.h"
 
 namespace ss2d {
@@ -124,7 +128,12 @@ __device__ __forceinline__ void store4(out_t *__restrict__ dst, const float (&v)
 struct ChanGeom {
     int32_t n_cb;            // channel blocks of 64 per group
     FastDiv div_cb, div_groups;
+    int32_t seg_len, n_segs;                 // of a row cut into segments (kLocal, kRest)
+    FastDiv div_segs;                        // segments of a row that this launch walks
 };
+
+// A row as a whole, or cut into segments: what a segment leaves from state 0, then its outputs from the state that enters it.
+enum ChanPhase { kWhole, kLocal, kRest };
 
 // kX: the chunk-end states are written as well -- x[row][chunk][2n] = product of a_n since the row's start,
 // x[..][2n + 1] = h_n, after every 2048 positions and at the row's end.  h is what the lane holds; the product is
@@ -149,7 +158,7 @@ __device__ __forceinline__ Raw4<in_t> reverse4(const Raw4<in_t> &r) {
     return o;
 }
 
-template <typename in_t, typename out_t, int kSpw, bool kSoftplus, bool kX, bool kMaps = false>
+template <typename in_t, typename out_t, int kSpw, bool kSoftplus, bool kX, bool kMaps = false, int kPhase = kWhole>
 __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restrict__ u_all, const in_t *__restrict__ dl_all,
                                                            const in_t *__restrict__ B_all, const in_t *__restrict__ C_all,
                                                            const float *__restrict__ A_all, out_t *__restrict__ o_all,
@@ -158,18 +167,21 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
     __shared__ __align__(16) float s_dl[kChanBlock * kChanTilePitch];
     __shared__ __align__(16) float s_du[kChanBlock * kChanTilePitch];
     __shared__ __align__(16) float s_y[kWavesPerWg * kChanBlock * kChanSubPitch];
-    __shared__ float s_sum[kX ? kWavesPerWg * kChanBlock : 1];
+    __shared__ float s_sum[kX || kPhase == kLocal ? kWavesPerWg * kChanBlock : 1];
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     // neighbouring workgroups are the channel blocks of one (image, group) and read the same B / C rows: keep them
     // on one XCD (one L2)
-    const uint32_t wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
-    uint32_t bg, cb, b, grp;
+    uint32_t wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
+    uint32_t bg, cb, b, grp, seg = 0;
+    if constexpr (kPhase != kWhole) divmod(wg, geo.div_segs, wg, seg);
     divmod(wg, geo.div_cb, bg, cb);
     divmod(bg, geo.div_groups, b, grp);
     const int L = p.L, dpg = p.dim_per_group;
+    const int begin = kPhase == kWhole ? 0 : (int)seg * geo.seg_len;           // (a multiple of kChanTile)
+    const int stop = kPhase == kWhole || (int)seg + 1 == geo.n_segs ? L : begin + geo.seg_len;
 
     // ---- staging / combine role: row r, quarter q -----------------------------------------------------------------
     const int r = tid >> 2, q = tid & 3;
@@ -215,7 +227,9 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
         h[j] = 0.0f;
     }
     const in_t *B_wave = B_all + (int64_t)b * p.B_bs + (int64_t)grp * p.B_gs + (int64_t)(wave * kSpw) * p.B_ns;
-    const in_t *C_wave = C_all + (int64_t)b * p.C_bs + (int64_t)grp * p.C_gs + (int64_t)(wave * kSpw) * p.C_ns;
+    // (kLocal has no use for C: the same lines of B twice)
+    const in_t *C_wave = kPhase == kLocal ? B_wave : C_all + (int64_t)b * p.C_bs + (int64_t)grp * p.C_gs + (int64_t)(wave * kSpw) * p.C_ns;
+    const int64_t C_ns = kPhase == kLocal ? p.B_ns : p.C_ns;
     const float *my_dl = s_dl + lane * kChanTilePitch, *my_du = s_du + lane * kChanTilePitch;
     float *my_y = s_y + (wave * kChanBlock + lane) * kChanSubPitch;
     const float *sum_y = s_y + r * kChanSubPitch + 4 * q;
@@ -223,21 +237,30 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
     const bool chan_ok = (int)cb * kChanBlock + lane < dpg;
     float *x_lane = kX ? p.x + ((int64_t)b * p.dim + dc) * p.n_chunks * 2 * p.N + 2 * (wave * kSpw) : nullptr;
 
+    // a segment's states, its sum of dl and (from the carry kernel) that of all before it, where its outputs will be
+    uint8_t *seg_state = reinterpret_cast<uint8_t *>(o_all + (int64_t)b * p.o_bs + (int64_t)dc * p.o_ds + begin);
+    if constexpr (kPhase == kRest) {
+        if (seg > 0) {
+            __builtin_memcpy(h, seg_state + sizeof(float) * (wave * kSpw), sizeof(h));
+            if (kX && wave == 0) __builtin_memcpy(&dl_sum, seg_state + sizeof(float) * (p.N + 1), sizeof(dl_sum));
+        }
+    }
+
     constexpr float kFill = delta_fill<kSoftplus>();
     Raw4<in_t> ru[2], rd[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-        ru[s] = load_u(s * kChanSub + 4 * q);
-        rd[s] = load_raw4<in_t>(dl_row, s * kChanSub + 4 * q, L, kFill);
+        ru[s] = load_u(begin + s * kChanSub + 4 * q);
+        rd[s] = load_raw4<in_t>(dl_row, begin + s * kChanSub + 4 * q, L, kFill);
     }
     // B / C of the (round, state) processed next are always one step ahead in scalar registers: requested before the
     // arithmetic of the current state starts, they have arrived when it ends.  Rows are multiples of 8 positions, so
     // the second half of a round lies entirely inside or entirely outside the row; outside, the first half is read
     // again (du is 0 there, nothing of it is stored), and a round past the row's end reads the row's start.
     UniRaw<in_t> next_bc;
-    load_uniform<in_t>(B_wave, C_wave, 0, 8 < L ? 8 : 0, next_bc);
+    load_uniform<in_t>(B_wave, C_wave, begin, begin + 8 < L ? begin + 8 : begin, next_bc);
 
-    for (int t0 = 0; t0 < L; t0 += kChanTile) {
+    for (int t0 = begin; t0 < stop; t0 += kChanTile) {
         // ---- stage: dl, du into LDS; the skip term stays with this thread for the combine ---------------------------
         float skip[2][4];
 #pragma unroll
@@ -257,7 +280,7 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
             *reinterpret_cast<float4 *>(st_du + s * kChanSub) = make_float4(du[0], du[1], du[2], du[3]);
         }
         // the next step's inputs travel while this step computes
-        if (t0 + kChanTile < L) {
+        if (t0 + kChanTile < stop) {
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 ru[s] = load_u(t0 + kChanTile + s * kChanSub + 4 * q);
@@ -281,7 +304,7 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
                 }
 #pragma unroll
                 for (int i = 0; i < kChanSub; ++i) y[i] = 0.0f;
-                if constexpr (kX) {
+                if constexpr (kX || kPhase == kLocal) {
                     const float4 q4 = *reinterpret_cast<const float4 *>(my_dl + s * kChanSub + 4 * wave);
                     dl_sum += (q4.x + q4.y) + (q4.z + q4.w);  // (dl is 0 past the row's end)
                 }
@@ -298,7 +321,7 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
                         int pn = j + 1 < kSpw ? ps : ps + kChanSub;
                         pn = pn < L ? pn : 0;
                         const int pn1 = pn + 8 < L ? pn + 8 : pn;
-                        load_uniform<in_t>(B_wave + (int64_t)jn * p.B_ns, C_wave + (int64_t)jn * p.C_ns, pn, pn1, next_bc);
+                        load_uniform<in_t>(B_wave + (int64_t)jn * p.B_ns, C_wave + (int64_t)jn * C_ns, pn, pn1, next_bc);
                     }
                     __builtin_amdgcn_sched_barrier(0);      // the requests above are issued before the arithmetic below
                     float Bv[kChanSub], Cv[kChanSub];
@@ -311,14 +334,18 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
 #pragma unroll
                     for (int i = 0; i < kChanSub; ++i) {
                         hj = fmaf(a[i], hj, Bv[i] * du[i]);
-                        y[i] = fmaf(Cv[i], hj, y[i]);
+                        if constexpr (kPhase != kLocal) y[i] = fmaf(Cv[i], hj, y[i]);
                     }
                     h[j] = hj;
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int v = 0; v < kChanSub / 4; ++v)
+                for (int v = 0; v < kChanSub / 4 && kPhase != kLocal; ++v)
                     *reinterpret_cast<float4 *>(my_y + 4 * v) = make_float4(y[4 * v], y[4 * v + 1], y[4 * v + 2], y[4 * v + 3]);
+            }
+            if constexpr (kPhase == kLocal) {
+                if (s == 1) __syncthreads();                // dl / du read before the next step's are written
+                continue;
             }
             __syncthreads();                                // the four partial sums of this round are in place
             if (ps < L) {
@@ -352,6 +379,54 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
             }
         }
     }
+    if constexpr (kPhase == kLocal) {
+        s_sum[wave * kChanBlock + lane] = dl_sum;
+        __syncthreads();
+        if (!chan_ok) return;
+        __builtin_memcpy(seg_state + sizeof(float) * (wave * kSpw), h, sizeof(h));
+        if (wave == 0) {
+            const float total = (s_sum[lane] + s_sum[kChanBlock + lane]) + (s_sum[2 * kChanBlock + lane] + s_sum[3 * kChanBlock + lane]);
+            __builtin_memcpy(seg_state + sizeof(float) * p.N, &total, sizeof(total));
+        }
+    }
+}
+
+// What enters every segment but the first, in the place of what the segment left: a thread per (row, state).
+template <typename out_t>
+__global__ __launch_bounds__(kBlock) void scan_chan_carry_kernel(const float *__restrict__ A_all, out_t *o_all, const ScanArgs p, int seg_len, int n_segs,
+                                                                 uint32_t n_items, FastDiv div_n, FastDiv div_dim) {
+    const uint32_t item = blockIdx.x * kBlock + threadIdx.x;
+    if (item >= n_items) return;
+    uint32_t row, n, b, d;
+    divmod(item, div_n, row, n);
+    divmod(row, div_dim, b, d);
+    const float A2 = A_all[(int64_t)d * p.A_ds + (int64_t)n * p.A_ns] * kLog2e;
+    uint8_t *state = reinterpret_cast<uint8_t *>(o_all + (int64_t)b * p.o_bs + (int64_t)d * p.o_ds);
+    const int64_t pitch = (int64_t)seg_len * sizeof(out_t);
+    float carry = 0.0f, before = 0.0f;
+    constexpr int kFly = 8;
+    for (int first = 0; first < n_segs; first += kFly) {
+        float left[kFly], sum[kFly];
+#pragma unroll
+        for (int i = 0; i < kFly; ++i) {                    // (past the last but one segment: that one again, not used)
+            const uint8_t *from = state + min(first + i, n_segs - 2) * pitch;
+            __builtin_memcpy(&left[i], from + sizeof(float) * n, sizeof(float));
+            __builtin_memcpy(&sum[i], from + sizeof(float) * p.N, sizeof(float));
+        }
+#pragma unroll
+        for (int i = 0; i < kFly; ++i) {
+            const int s = first + i;
+            if (s >= n_segs) break;
+            if (s > 0) {
+                __builtin_memcpy(state + s * pitch + sizeof(float) * n, &carry, sizeof(float));
+                if (n == 0) __builtin_memcpy(state + s * pitch + sizeof(float) * (p.N + 1), &before, sizeof(float));
+            }
+            before += sum[i];
+            // the product of the segment's a in two halves, so that neither leaves fp32's range before the state would; none of 0
+            const float half = __builtin_amdgcn_exp2f(0.5f * A2 * sum[i]);
+            carry = carry == 0.0f ? left[i] : fmaf(carry * half, half, left[i]);
+        }
+    }
 }
 
 bool scan_chan_eligible(const ScanArgs &a) {
@@ -359,9 +434,33 @@ bool scan_chan_eligible(const ScanArgs &a) {
     return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.L % 8 == 0 && a.dim_per_group >= 32;
 }
 
+// The number of segments of a row (1: not cut) and the length of all but the last, which has at least 72 positions: a segment's N + 2
+// floats lie where its outputs will be.
+//
+// A workgroup takes 1.7 us per 16 positions of 16 states however few there are (1.0 of 4 states, 2.7 of 32).  Cut rows run the recurrence
+// twice (the first time without C), in three launches, and are ahead where the segments find room beside one another: three
+// workgroups per CU, segments of 128 positions or more.  us, whole / cut, workgroups of whole rows in front: 16 states in bf16, 4: 16 384
+// positions 1699 / 58; 8: 3136 331 / 42; 12: 784 86 / 39, 400 46 / 38; 48: 784 87 / 39, 400 47 / 38; 96: 784 89 / 51, 512 59 / 43; 192: 3136 388 / 265; in fp32, 8: 3136
+// 310 / 39; 96: 784 83 / 53; 4 states, 8: 3136 173 / 28; 48: 400 25.2 / 23.8; 32 states in fp16, 8: 3136 528 / 63; 48: 400 72 / 58.  Left whole: few segments
+// of many workgroups, 192: 784 positions 89 / 83 in bf16, 86 / 90 in fp32, 138 / 156 of 32 states; 96: 400 47 / 44, 43.5 / 43.6, 72 / 74.
+constexpr int64_t kSegPlaces = 768, kSegLeast = 128;
+
+static int64_t chan_segments(const ScanArgs &a, int64_t n_wg, int32_t &seg_len) {
+    if (a.out == a.u || a.out == a.delta || (int64_t)a.batch * a.dim * a.N > 0x7fffffff) return 1;
+    const int64_t fewest = n_wg <= 64 ? 3 : n_wg <= 128 || a.L >= 2048 ? 4 : kSegPlaces;
+    int64_t n = kSegPlaces / n_wg;
+    if (n > a.L / kSegLeast) n = a.L / kSegLeast;
+    if (n < fewest) return 1;
+    const int64_t len = ((a.L + n - 1) / n + kChanTile - 1) / kChanTile * kChanTile;
+    n = (a.L + len - 1) / len;
+    if (a.L - (n - 1) * len < 72) --n;
+    seg_len = (int32_t)len;
+    return n;
+}
+
 template <typename in_t, typename out_t>
 static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stream) {
-    ChanGeom geo;
+    ChanGeom geo = {};
     geo.n_cb = (a.dim_per_group + kChanBlock - 1) / kChanBlock;
     const int groups = a.dim / a.dim_per_group;
     geo.div_cb = make_fastdiv((uint32_t)geo.n_cb);
@@ -381,12 +480,43 @@ static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stre
     }
 #define SS2D_LAUNCH_CHAN_X(SP, M) \
     if (a.x) { SS2D_LAUNCH_CHAN_N(SP, true, M) } else { SS2D_LAUNCH_CHAN_N(SP, false, M) }
+#define SS2D_LAUNCH_CHAN_SPLIT(SPW, X, M)                                                                                   \
+    do {                                                                                                                   \
+        geo.div_segs = make_fastdiv((uint32_t)segs - 1);                                                                    \
+        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, false, M, kLocal>), dim3((uint32_t)(n_wg * (segs - 1))), dim3(kBlock), 0, stream, \
+                           (const in_t *)a.u, (const in_t *)a.delta, (const in_t *)a.B, (const in_t *)a.C, a.A, (out_t *)a.out, a, geo, (const in_t *)xt); \
+        hipLaunchKernelGGL((scan_chan_carry_kernel<out_t>), dim3((n_items + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, a.A, (out_t *)a.out, a, \
+                           geo.seg_len, geo.n_segs, n_items, make_fastdiv((uint32_t)a.N), make_fastdiv((uint32_t)a.dim));   \
+        geo.div_segs = make_fastdiv((uint32_t)segs);                                                                        \
+        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, X, M, kRest>), dim3((uint32_t)(n_wg * segs)), dim3(kBlock), 0, stream, \
+                           (const in_t *)a.u, (const in_t *)a.delta, (const in_t *)a.B, (const in_t *)a.C, a.A, (out_t *)a.out, a, geo, (const in_t *)xt); \
+    } while (0)
+#define SS2D_LAUNCH_CHAN_SPLIT_N(X, M)                          \
+    switch (a.N) {                                              \
+        case 4: SS2D_LAUNCH_CHAN_SPLIT(1, X, M); break;         \
+        case 8: SS2D_LAUNCH_CHAN_SPLIT(2, X, M); break;         \
+        case 16: SS2D_LAUNCH_CHAN_SPLIT(4, X, M); break;        \
+        default: SS2D_LAUNCH_CHAN_SPLIT(8, X, M); break;        \
+    }
+    const int64_t segs = a.softplus ? chan_segments(a, n_wg, geo.seg_len) : 1;
+    if (segs > 1) {
+        geo.n_segs = (int32_t)segs;
+        const uint32_t n_items = (uint32_t)((int64_t)a.batch * a.dim * a.N);
+        if (a.x) {
+            if (xt) { SS2D_LAUNCH_CHAN_SPLIT_N(true, true) } else { SS2D_LAUNCH_CHAN_SPLIT_N(true, false) }
+        } else {
+            if (xt) { SS2D_LAUNCH_CHAN_SPLIT_N(false, true) } else { SS2D_LAUNCH_CHAN_SPLIT_N(false, false) }
+        }
+        return launch_status();
+    }
     if (xt) {
         if (a.softplus) { SS2D_LAUNCH_CHAN_X(true, true) } else { SS2D_LAUNCH_CHAN_X(false, true) }
     } else {
         if (a.softplus) { SS2D_LAUNCH_CHAN_X(true, false) } else { SS2D_LAUNCH_CHAN_X(false, false) }
     }
 #undef SS2D_LAUNCH_CHAN_X
+#undef SS2D_LAUNCH_CHAN_SPLIT_N
+#undef SS2D_LAUNCH_CHAN_SPLIT
 #undef SS2D_LAUNCH_CHAN_N
 #undef SS2D_LAUNCH_CHAN
     return launch_status();
