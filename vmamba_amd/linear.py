@@ -141,8 +141,8 @@ def linear_tiles_fusable(x, layer, act=None):
 
 def linear_tiles_pays(M, N, K, gelu):
     """True where ss2d_linear_tiles is ahead of the library.  With the GELU, which is a pass over the result there: us in bf16, library
-    product and GELU / kernel, four outputs per input: 384 at 3136 positions 21 / 16, at 25 088 91 / 63, at 100 352 354 / 264; 96 at 3136 10 / 11,
-    at 12 544 19 / 12; 256 at 3136 16 / 14; 512 at 6272 33 / 36, at 12 544 75 / 54, at 50 176 276 / 174; 640 at 12 544 67 / 70; 768 at 6272 65 / 55, at 12 544
+    product and GELU / kernel, four outputs per input: 384 at 3136 positions 21 / 16, at 25 088 91 / 61, at 100 352 354 / 229; 96 at 3136 10 / 11,
+    at 12 544 19 / 12; 256 at 3136 16 / 14; 512 at 6272 33 / 36, at 12 544 75 / 48, at 50 176 276 / 159; 640 at 12 544 67 / 70; 768 at 6272 65 / 55, at 12 544
     89 / 92.  Without, the library's larger tiles are ahead but where the contraction is short and the outputs fill tiles of 192: 384 x 384 at
     12 544 positions 11 / 12, at 25 088 25 / 18, at 50 176 41 / 30; 320 x 320 at 25 088 19 / 16; 192 x 192 at 25 088 10 / 10, at 100 352 26 / 23; 256 x 256 at
     50 176 15 / 23; 512 x 512 at 25 088 20 / 28."""
