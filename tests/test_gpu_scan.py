@@ -211,6 +211,28 @@ def test_scan_segments_hold_what_a_whole_row_does():
     assert torch.allclose(got[ok], want[ok], **TOL32)
 
 
+def test_scan_segments_in_a_graph():
+    """Captured once, replayed with eager calls on other inputs between: every replay gives the eager call's bits."""
+    args = [t.to(DEV) for t in make_inputs(36, 1, 64, 1, 16, 1024, torch.bfloat16, ss2d_like=True)]
+    other = [t.to(DEV) for t in make_inputs(37, 1, 64, 1, 16, 1024, torch.bfloat16, ss2d_like=True)]
+    call = lambda a: va.selective_scan_fwd(*a, True, 1, True, want_x=False)[0]
+    want = call(args)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        call(args)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = call(args)
+    torch.cuda.synchronize()
+    for _ in range(4):
+        out.zero_()
+        call(other)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("batch,Dm,H,W,N", [(2, 32, 8, 8, 16), (1, 64, 14, 12, 4), (2, 48, 7, 8, 8), (1, 96, 56, 56, 16), (3, 40, 4, 6, 32)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_scan_reading_the_map_through_the_cross_scan_routes(batch, Dm, H, W, N, dtype):
