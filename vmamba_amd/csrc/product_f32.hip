@@ -20,7 +20,7 @@
 // split's instructions between them.  One accumulator for all six, three workgroups per CU: 93, and the bias above.  Against 64 bits the error
 // is 1.1e-7 (library 3.5e-7), of the gradient 1.6e-7 (2.0e-6).  Two fp16 parts and three products would be twice as fast and hold less
 // than fp32's range.
-#include "ss2d_common.h"
+#include "normal_cdf.h"
 
 namespace ss2d {
 
@@ -139,35 +139,16 @@ template <bool kByCols, int kRows> struct PfTile {
     }
 };
 
-// exp(-x^2 / 2) and the normal distribution at -|x|, which is half of erfc(z) = exp(-z^2) erfcx(z), z = |x| / sqrt 2: erfcx as a polynomial
-// in 1 / (1 + z / 2), a least-squares fit of degree 9 with weights driven to the even error of 3e-8 over 0 <= z <= 9.5 (beyond, exp(-z^2)
-// is 0).  GELU comes out 3.9e-8 from float64 (rms over a normal x; 0.5 x (1 + erff) 3.7e-8) and keeps its relative error for large
-// negative x.  erff, two branches of some thirty instructions each, made the two kernels 144 and 148 us at 12 544 x 1536 x 384; with this they are 134 and 139 (108 without, and without their second tensor of 77 MB).
-__device__ __forceinline__ void normal_tail(float x, float &e, float &tail) {
-    const float z = fabsf(x) * 0.70710678118654752f;
-    const float t = __builtin_amdgcn_rcpf(fmaf(0.5f, z, 1.0f));
-    e = __builtin_amdgcn_exp2f(z * z * -1.4426950408889634f);
-    float y = -0.0541273268f;
-    y = fmaf(y, t, 0.259068346f);
-    y = fmaf(y, t, -0.430575281f);
-    y = fmaf(y, t, 0.207323139f);
-    y = fmaf(y, t, 0.0280119366f);
-    y = fmaf(y, t, 0.175724077f);
-    y = fmaf(y, t, 0.25157837f);
-    y = fmaf(y, t, 0.280743992f);
-    y = fmaf(y, t, 0.282260565f);
-    y = fmaf(y, t, -7.84717933e-06f);
-    tail = 0.5f * (e * y);
-}
+// 12 544 x 1536 x 384, us: 129 with GELU and 124 with its derivative, 103 without and without their second tensor of 77 MB.  One fit of degree 9 took 125 and
+// 120 and lost accuracy (normal_cdf.h); erff, two branches of some thirty instructions each, ten more than that.
 __device__ __forceinline__ float gelu_f32(float x) {
-    float e, tail;
-    normal_tail(x, e, tail);
-    return x * (x < 0.0f ? tail : 1.0f - tail);
+    float e;
+    return x * normal_cdf(x, e);
 }
 __device__ __forceinline__ float gelu_grad_f32(float x) {
-    float e, tail;
-    normal_tail(x, e, tail);
-    return fmaf(x * 0.39894228040143268f, e, x < 0.0f ? tail : 1.0f - tail);
+    float e;
+    const float cdf = normal_cdf(x, e);
+    return fmaf(x * 0.39894228040143268f, e, cdf);
 }
 
 // What stands behind the sum: outputs n .. n + 3 of a row, at `at`
