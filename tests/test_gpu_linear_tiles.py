@@ -126,3 +126,25 @@ def test_model_no_further_from_float64(monkeypatch):
         before = half(x).double()
     error = lambda y: ((y - want).norm() / want.norm()).item()
     assert error(got) <= 1.1 * error(before)
+
+
+@pytest.mark.parametrize("lo,hi", [(-8, -4), (-4, -3), (-3, -2), (-2, -1), (-1, 0), (0, 1), (1, 2), (2, 4), (4, 65504)])
+def test_fp16_gelu_rounds_no_worse_than_erff(lo, hi):
+    """Every fp16 argument in (lo, hi], as a bias behind a product of zeros: no more results than the library's erff form gives are another
+    neighbour than the exact value's -- one of the 15 360 on either side of 0, where x = 0.0013 has an exact value 4.2e-8 of itself from the middle of two
+    neighbours, less than a rounding in fp32 --, and none is further off than its furthest or 0.502 of a unit."""
+    from vmamba_amd.linear import linear_rows_hip
+    every = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    every = every[every.isfinite() & (every > lo) & (every <= hi)]
+    n = every.numel() // 8 * 8
+    x = every[:n].to(DEV)
+    exact = F.gelu(x.double())
+    nearest = exact.to(torch.float16)
+    unit = (torch.nextafter(nearest.abs(), torch.full_like(nearest, float("inf"))) - nearest.abs()).double()
+    zero, weight = torch.zeros(8, 32, device=DEV, dtype=torch.float16), torch.zeros(n, 32, device=DEV, dtype=torch.float16)
+    lib = F.gelu(x)
+    off = lambda y: ((y.double() - exact).abs() / unit).max().item()
+    for kernel in (linear_tiles_hip, linear_rows_hip):
+        got = kernel(zero, weight, x, gelu=True)[0]
+        print("fp16 gelu", lo, hi, n, "other neighbours %d / %d, furthest %.3f / %.3f" % ((got != nearest).sum(), (lib != nearest).sum(), off(got), off(lib)), flush=True)
+        assert (got != nearest).sum() <= (lib != nearest).sum() + (n > 15000 and abs(lo + hi) == 1) and off(got) <= max(off(lib), 0.502)

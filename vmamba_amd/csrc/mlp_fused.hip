@@ -21,7 +21,7 @@
 //   * bf16: the pre-activation is a bf16 value, so gelu(x) = 0.5 x + |x| E(|x|), E(x) = 0.5 erf(x / sqrt 2), with E read
 //     from a 2176-entry fp32 table in LDS indexed by the bf16 bit pattern clamped to [2^-14, 8) (below, |x| E is under
 //     1e-4 of 0.5 |x|; above, E is 0.5 to fp32 precision).  The table is generated in double precision at build time;
-//   * fp16: erf from Abramowitz-Stegun 7.1.26 (absolute error 1.5e-7, far below 16-bit rounding).
+//   * fp16: the normal distribution function by a polynomial in fp32 whose relative error is far below 16-bit rounding (gelu.h).
 #include "gelu.h"
 
 namespace ss2d {
