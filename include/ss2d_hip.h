@@ -629,7 +629,7 @@ int ss2d_column_sums_f32(const float *x, float *out, int64_t rows, int N, void *
 
 /*
  * A product in single precision on the bf16 matrix cores (each value as the sum of three bf16 ones, six products, fp32 sums; the error is
- * that of a product in fp32): out (M, N) with out[m][n] = sum over K of A(m, k) B(n, k), A stored (M, K) or by columns (K, M), B (N, K) or (K, N).
+ * that of a product in fp32 over its whole range): out (M, N) with out[m][n] = sum over K of A(m, k) B(n, k), A stored (M, K) or by columns (K, M), B (N, K) or (K, N).
  *   mode 0: + bias (N) + other (M, N), either or both NULL.  mode 1: out = sum + bias, out2 = GELU(out).
  *   mode 2: out = (sum + bias) GELU'(other), other the pre-activation.
  * The fp32 Linear layers of a block and their gradients (classification/models/vmamba.py:648-662, :1116-1131).  Contiguous, 16-byte

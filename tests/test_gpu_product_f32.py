@@ -68,6 +68,28 @@ def test_infinities_and_nan(a_cols, b_cols):
     assert torch.allclose(got[ok], want[ok], rtol=1e-4, atol=1e-6)
 
 
+@pytest.mark.parametrize("a_cols,b_cols", [(False, False), (False, True), (True, True)])
+@pytest.mark.parametrize("down,M,N,K", [((100, 0), 132, 68, 96), ((116, 0), 132, 68, 96), ((0, 116), 132, 68, 96), ((58, 58), 132, 68, 96), ((120, -100), 64, 64, 4096)])
+def test_small_operands_lose_nothing(down, M, N, K, a_cols, b_cols):
+    """Operands times powers of two give the same digits, as long as the results are fp32 normals (a share's of a long sum too)."""
+    print("CASE product_f32 small", down, M, N, K, a_cols, b_cols, flush=True)
+    g = torch.Generator().manual_seed(K)
+    a, b = torch.randn(M, K, generator=g).to(DEV) * 2.0 ** -down[0], torch.randn(N, K, generator=g).to(DEV) * 2.0 ** -down[1]      # (some subnormal)
+    small = product_f32_hip(stored(a, a_cols), stored(b, b_cols), a_cols, b_cols)
+    one = product_f32_hip(stored(a * 2.0 ** down[0], a_cols), stored(b * 2.0 ** down[1], b_cols), a_cols, b_cols)
+    normal = one.abs() * 2.0 ** -sum(down) > 2.0 ** -125
+    assert normal.float().mean() > 0.99 and torch.equal((small * 2.0 ** sum(down))[normal], one[normal])
+
+
+def test_subnormal_operands():
+    """Subnormal fp32 values, exact as integers of 2^-149, against float64: an error of a product in fp32."""
+    g = torch.Generator().manual_seed(0)
+    a = (torch.randint(-2 ** 23, 2 ** 23, (132, 64), generator=g).double() * 2.0 ** -149).float().to(DEV)
+    b = torch.randn(68, 64, generator=g).to(DEV) * 2.0 ** 60
+    got, want = product_f32_hip(a, b).double(), a.double() @ b.double().t()
+    assert bool((a.abs() < 2.0 ** -126).all()) and ((got - want).norm() / want.norm()).item() < 2.0 ** -22
+
+
 def test_refused():
     a = torch.zeros(8, 8, device=DEV)
     with pytest.raises(ValueError):

@@ -13,8 +13,11 @@
 //     while this one's are multiplied; they are split on the way into LDS, [row][term] in three planes whichever way they were
 //     stored, the 16-byte pieces of a row in an order of its own, so that neither side of LDS meets itself in a bank.
 //   * few outputs and a long sum (a weight gradient) are cut into shares of the terms, added by a second kernel in a fixed order.
-//   * infinities and NaN, and values that round beyond bf16's largest, leave a NaN or an infinity in the sums: a wavefront that finds one
-//     computes its outputs again on the fp32 matrix cores, from memory.
+//   * a third part of a value v lies down to 2^-24 v, and bf16 ends at 2^-126: values are multiplied by 2^24 on the way into their parts and the sums
+//     by 2^-48 behind the last term, exactly, so that every fp32 value, the subnormal ones too, is the sum of its parts, and products of them do
+//     not vanish that count in fp32.  (Without it a value of 2^-116 is off by 3e-6 of itself; 1 to 3 % of the time.)
+//   * infinities and NaN, and values that round beyond bf16's largest or sums beyond fp32's (from 2^104 and 2^80 on), leave a NaN or an infinity in the
+//     sums: a wavefront that finds one computes its outputs again on the fp32 matrix cores, from memory.
 // 12 544 x 1536 x 384: 148 us as the library's product (100 TFLOP/s), 108 here (137); 384 x 1536 outputs over 12 544 positions, both by columns,
 // 144 -> 105.  What bounds it is the matrix cores' rate under load, 1.2 PFLOP/s in bf16 on this card, a sixth of it here: 200; then the
 // split's instructions between them.  One accumulator for all six, three workgroups per CU: 93, and the bias above.  Against 64 bits the error
@@ -38,8 +41,11 @@ struct ProductArgs {
 
 enum { kPfPlain = 0, kPfGelu = 1, kPfGeluGrad = 2 };
 
-// Two floats as three packed bf16 pairs: rounded, the rounded remainder, the remainder of both (exact for what 24 bits hold)
+constexpr float kPfScale = 0x1p24f, kPfUnscale = 0x1p-48f;           // of a value, of a sum of products
+
+// Two floats times kPfScale as three packed bf16 pairs: rounded, the rounded remainder, the remainder of both (exact for what 24 bits hold)
 __device__ __forceinline__ void split3(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
+    a *= kPfScale; b *= kPfScale;
     h = pack2_from_f32<bf16_t>(a, b);
     a -= unpack_lo<bf16_t>(h); b -= unpack_hi<bf16_t>(h);
     m = pack2_from_f32<bf16_t>(a, b);
@@ -244,6 +250,7 @@ __global__ __launch_bounds__(kBlock, kTileN == 128 ? 2 : 3) void product_f32_ker
             for (int v = 0; v < 16; ++v) {
                 acc[i][e][v] += low[i][e][v];
                 odd |= !(fabsf(acc[i][e][v]) <= 3.4028235e38f);
+                acc[i][e][v] *= kPfUnscale;
             }
     if (__any(odd)) {
         int64_t ra[2], rb[kE];
