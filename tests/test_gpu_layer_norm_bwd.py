@@ -5,9 +5,12 @@ dx is a handful of fp32 operations on values of unit size behind sums of C terms
 import pytest
 import torch
 import torch.nn.functional as F
+from torch.utils._python_dispatch import TorchDispatchMode
 
+from vmamba_amd.linear import LinearDw
 from vmamba_amd.norm import LayerNorm, LayerNormF32, column_sums, layer_norm_trains
 from vmamba_amd.ss2d import SS2D
+from vmamba_amd.vssm import Mlp
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -84,3 +87,42 @@ def test_out_norm_of_a_map():
     assert torch.allclose(got, want, rtol=1e-5, atol=1e-5)
     for a, b in zip(torch.autograd.grad(got, [y, op.out_norm.weight], dy), torch.autograd.grad(want, [y, op.out_norm.weight], dy)):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-5 * max(1.0, b.abs().max().item()))
+
+
+class Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.calls = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.calls.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("what", ["norm", "out_norm", "mlp", "linear"])
+def test_gradients_whose_memory_is_not_theirs(what):
+    """A batch of gradients (is_grads_batched, a vectorised jacobian) and a mode around the backward alone: both go through torch's operators,
+    as they do where those stand in the forward, and give the gradients of the separate calls (sums of up to 35 000 terms in fp32)."""
+    torch.manual_seed(0)
+    if what == "out_norm":
+        op = SS2D(d_model=64, channel_first=False).to(DEV)
+        x = torch.randn(600, 64, 9, 7, device=DEV, requires_grad=True)
+        y, wanted = op.finish_core(x.view(600, 64, 63), 600, 64, 9, 7, torch.float32), [x, op.out_norm.weight, op.out_norm.bias]
+    else:
+        x = torch.randn(22000, 96, device=DEV, requires_grad=True)
+        if what == "linear":
+            layer = torch.nn.Linear(96, 96, bias=False).to(DEV)
+            y, wanted = LinearDw.apply(x, layer.weight, None), [x, layer.weight]
+        else:
+            layer = LayerNorm(96).to(DEV) if what == "norm" else Mlp(96, 384, channel_first=False).to(DEV)
+            y, wanted = layer(x), [x] + list(layer.parameters())
+    assert y.grad_fn.name().split("Backward")[0] in ("LayerNormF32", "MlpF32", "LinearDw")
+    dys = torch.randn(3, *y.shape, device=DEV)
+    singly = [torch.autograd.grad(y, wanted, dy, retain_graph=True) for dy in dys]
+    near = lambda a, b: ((a - b).norm() / b.norm()).item() < 1e-5
+    batched = torch.autograd.grad(y, wanted, dys, is_grads_batched=True, retain_graph=True)
+    assert all(near(many, torch.stack(few)) for many, few in zip(batched, zip(*singly)))
+    with Seen() as mode:
+        seen = torch.autograd.grad(y, wanted, dys[0])
+    assert all(near(a, b) for a, b in zip(seen, singly[0]))
+    assert any(("mm" if what in ("mlp", "linear") else "rsqrt") in call for call in mode.calls)

@@ -294,3 +294,14 @@ def test_operators_seen():
     finally:
         torch.nn.Linear.forward = forward
     assert not operators_seen()
+
+
+def test_mlp_backward_of_a_batch_of_gradients():
+    """MlpF32's backward takes torch's operators for gradients without memory of their own (sizes the kernels are not asked for)."""
+    from vmamba_amd.linear import MlpF32
+    torch.manual_seed(0)
+    x, w1, b1, w2, b2 = wanted = [torch.randn(*s, requires_grad=True) for s in ((5, 8), (12, 8), (12,), (8, 12), (8,))]
+    dys = torch.randn(3, 5, 8)
+    want = torch.nn.functional.linear(torch.nn.functional.gelu(torch.nn.functional.linear(x, w1, b1)), w2, b2)
+    for got, ref in zip(torch.autograd.grad(MlpF32.apply(*wanted), wanted, dys, is_grads_batched=True), torch.autograd.grad(want, wanted, dys, is_grads_batched=True)):
+        assert torch.allclose(got, ref, rtol=1e-5, atol=1e-5)

@@ -13,6 +13,7 @@ supported with the same two kernels.
 import torch
 
 from . import _lib
+from .norm import memory_readable
 
 _DTYPE_CODE = {torch.float32: _lib.SS2D_F32, torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 
@@ -59,7 +60,7 @@ class TransposeBCL(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        return TransposeBCL.apply(dy)
+        return TransposeBCL.apply(dy) if memory_readable(dy) else dy.transpose(1, 2).contiguous()
 
 
 def cross_scan_flex_hip(x, in_channel_first=True, out_channel_first=True, one_by_one=False, scans=0):

@@ -9,7 +9,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .norm import TENSOR_KINDS, TRAIN_FROM, LayerNorm, calls_unseen, column_sums, needs_grad, observed, operators_seen
+from .norm import TENSOR_KINDS, TRAIN_FROM, LayerNorm, calls_unseen, column_sums, memory_readable, needs_grad, observed, operators_seen
 
 _DTYPE_CODE = {torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 FUSED_SHAPES = ((96, 96),)            # (in_features, out_features)
@@ -269,11 +269,11 @@ def product_pays(M, N, K, gradient=False):
 
 def _product(a, b, a_by_columns=False, b_by_columns=False, bias=None, other=None, mode=PRODUCT_PLAIN):
     """product_f32_hip where it stands for the library's product, which is taken under a second backward (the kernel has no gradient of its
-    own), for views that start between 16-byte boundaries and where it is the faster one."""
+    own), for tensors whose memory is not theirs (memory_readable), for views that start between 16-byte boundaries and where it is the faster one."""
     M, K = a.shape[::-1] if a_by_columns else a.shape
     N = b.shape[1] if b_by_columns else b.shape[0]
     if (product_pays(M, N, K, a_by_columns and b_by_columns) and not torch.is_grad_enabled() and N % 4 == 0 and (M if a_by_columns else K) % 4 == 0
-            and (b_by_columns or K % 4 == 0) and M * N * K > 0):
+            and (b_by_columns or K % 4 == 0) and M * N * K > 0 and memory_readable(a, b, bias, other)):
         a, b = a.contiguous(), b.contiguous()
         other = None if other is None else other.contiguous()
         if all(t is None or t.data_ptr() % 16 == 0 for t in (a, b, bias, other)):
@@ -289,7 +289,7 @@ def _product(a, b, a_by_columns=False, b_by_columns=False, bias=None, other=None
 def _weight_gradient(dy, x):
     """dy^T x, dy (M, N) and x (M, K)."""
     N, K = dy.shape[1], x.shape[1]
-    if N * K <= 384 * 384 and x.shape[0] >= 4096 and N % 4 == 0 and K % 4 == 0 and not torch.is_grad_enabled():
+    if N * K <= 384 * 384 and x.shape[0] >= 4096 and N % 4 == 0 and K % 4 == 0 and not torch.is_grad_enabled() and memory_readable(x, dy):
         x, dy = x.contiguous(), dy.contiguous()
         if (x.data_ptr() | dy.data_ptr()) % 16 == 0:
             return linear_dw_hip(x, dy)

@@ -142,6 +142,13 @@ def layer_norm_trains(x, normalized_shape, weight, bias, C=None):
                                                 and t.data_ptr() % 16 == 0) for t in (weight, bias)) and calls_unseen())
 
 
+def memory_readable(*tensors):
+    """True where a backward may hand these tensors (or None) to a kernel by their addresses: memory of their own -- a batch of gradients under
+    is_grads_batched or a vectorised jacobian has none, nor does another kind of tensor, and a negated view's is another -- and operators that
+    nothing sees now, whatever saw them in the forward."""
+    return not operators_seen() and all(t is None or (type(t) in TENSOR_KINDS and torch._C._has_storage(t) and not t.is_neg()) for t in tensors)
+
+
 class LayerNormF32(torch.autograd.Function):
     """F.layer_norm over the last axis with its backward on ss2d_layer_norm_bwd_f32, which computes the statistics again from x."""
 
@@ -156,7 +163,7 @@ class LayerNormF32(torch.autograd.Function):
         x, weight = ctx.saved_tensors
         wants = ctx.needs_input_grad
         C = x.shape[-1]
-        if torch.is_grad_enabled():                                  # a second backward goes through the torch operators
+        if torch.is_grad_enabled() or not memory_readable(x, weight, dy):          # a second backward goes through the torch operators
             mean = x.mean(-1, keepdim=True)
             centred = x - mean
             rstd = (centred.square().mean(-1, keepdim=True) + ctx.eps).rsqrt()
@@ -179,8 +186,8 @@ class LayerNormF32(torch.autograd.Function):
 
 
 def column_sums(x):
-    """x.sum(0) of a float32 matrix (ss2d_column_sums_f32; the library's where autograd follows or the kernel has no variant)."""
-    if torch.is_grad_enabled() or x.dtype != torch.float32 or not x.is_contiguous() or x.numel() == 0 or x.shape[1] % 4 or x.data_ptr() % 16:
+    """x.sum(0) of a float32 matrix (ss2d_column_sums_f32; the library's where autograd or something else follows or the kernel has no variant)."""
+    if torch.is_grad_enabled() or not memory_readable(x) or x.dtype != torch.float32 or not x.is_contiguous() or x.numel() == 0 or x.shape[1] % 4 or x.data_ptr() % 16:
         return x.sum(0)
     rows, N = x.shape
     out = torch.empty(N, dtype=x.dtype, device=x.device)
