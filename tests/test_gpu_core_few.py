@@ -79,6 +79,23 @@ def test_nan_stays_where_it_is(H, W, dtype):
     assert torch.equal(got[[0, 2]], clean[[0, 2]]) and torch.equal(got.isnan(), want.isnan())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("names", [("Ds",), ("dt_projs_bias",), ("A_logs",), ("x_proj_weight", "dt_projs_weight"), ("Ds", "dt_projs_bias", "A_logs", "x_proj_weight", "dt_projs_weight")])
+def test_strided_parameters(names, dtype):
+    """Parameters that are every other element of a larger tensor: forward_core's bits of the same values side by side."""
+    op, x = make(64, 5, dtype, 3), torch.randn(2, 64, 7, 9, device=DEV).to(dtype)
+    assert few_applies(2, 64, 7, 9, 5, dtype)
+    with torch.no_grad():
+        want = op.forward_core(x)
+        for name in names:
+            p = getattr(op, name)
+            wide = torch.empty(p.shape + (2,), device=DEV, dtype=p.dtype)
+            wide[..., 0].copy_(p)
+            setattr(op, name, torch.nn.Parameter(wide[..., 0]))
+            assert not getattr(op, name).is_contiguous()
+        assert torch.equal(op.forward_core(x), want)
+
+
 def test_rule():
     """Both sides of the line in one map's sizes, and what has no variant."""
     assert few_applies(1, 768, 7, 7, 48, torch.bfloat16) and few_applies(27, 768, 7, 7, 48, torch.bfloat16)

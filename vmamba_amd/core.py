@@ -200,8 +200,8 @@ def core_few_hip(x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias):
     for t in (x_proj_weight, dt_proj_weight):
         _check(t.dtype == x.dtype and t.device == x.device, "core_few: weights of x's dtype on its device")
     for t in (As, Ds, dt_bias):
-        _check(t.dtype == torch.float32 and t.device == x.device and t.numel() == 4 * D and t.is_contiguous(), "core_few: A, D and the bias (4 * D) float32")
-    x, x_proj_weight, dt_proj_weight = x.contiguous(), x_proj_weight.contiguous(), dt_proj_weight.contiguous()
+        _check(t.dtype == torch.float32 and t.device == x.device and t.numel() == 4 * D, "core_few: A, D and the bias (4 * D) float32")
+    x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias = (t.contiguous() for t in (x, x_proj_weight, dt_proj_weight, As, Ds, dt_bias))
     code, L = _DTYPE_CODE[x.dtype], _lib.lib()
     need = L.ss2d_few_rows_bytes(B, D, R, H, W, code)
     _lib.check(min(need, 0), "ss2d_few_rows_bytes")
