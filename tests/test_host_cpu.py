@@ -305,3 +305,13 @@ def test_mlp_backward_of_a_batch_of_gradients():
     want = torch.nn.functional.linear(torch.nn.functional.gelu(torch.nn.functional.linear(x, w1, b1)), w2, b2)
     for got, ref in zip(torch.autograd.grad(MlpF32.apply(*wanted), wanted, dys, is_grads_batched=True), torch.autograd.grad(want, wanted, dys, is_grads_batched=True)):
         assert torch.allclose(got, ref, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("name", ["linear", "gelu", "layer_norm"])
+def test_replaced_functions_are_not_passed_by(name, monkeypatch):
+    """What LayerNorm and the MLP call in training, replaced by the user: no kernel stands for it."""
+    from vmamba_amd.norm import calls_unseen
+    function = getattr(torch.nn.functional, name)
+    assert calls_unseen()
+    monkeypatch.setattr(torch.nn.functional, name, lambda *a, **k: function(*a, **k))
+    assert not calls_unseen()

@@ -225,7 +225,7 @@ _MODES = torch._C._len_torch_dispatch_stack, torch._C._functorch.peek_interprete
 
 
 def _calls():
-    return nn.Linear.forward, nn.GELU.forward, LayerNorm.forward, F.linear, F.gelu
+    return nn.Linear.forward, nn.GELU.forward, LayerNorm.forward, F.linear, F.gelu, F.layer_norm
 
 
 _CALLS = _calls()
