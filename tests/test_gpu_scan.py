@@ -211,6 +211,30 @@ def test_scan_segments_hold_what_a_whole_row_does():
     assert torch.allclose(got[ok], want[ok], **TOL32)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N", [4, 32])
+@pytest.mark.parametrize("step", [0.5, 30.0])
+def test_scan_segments_keep_an_infinite_state(N, dtype, step):
+    """A state that overflowed stays infinite, of its sign, through segments whose decays multiply to less than fp32's smallest, as it would
+    position by position; one decay of 0 on the way makes it NaN from there on.  B and C of one sign: the outputs' sum over the states too."""
+    _announce("scan-infinite-state", N, dtype, step)
+    dim, L = 64, 2048
+    u, delta = torch.ones(1, dim, L), torch.full((1, dim, L), 0.5)       # softplus: 0.97, decays of 2^-22, 128 of them 2^-2900
+    u[0, :32, 200], u[0, 32:, 200] = 3e38, -3e38
+    u[0, 5, 200] = 1.0                                                   # stays finite
+    delta[0, 7, 1001], delta[0, 9, 130] = step, step                     # 30: a decay of 0, behind the overflow and before it
+    A, B, C = torch.full((dim, N), -16.0), torch.full((1, 1, N, L), 4.0), torch.full((1, 1, N, L), 0.5)
+    args = [t.to(dtype) for t in (u, delta)] + [A, B.to(dtype), C.to(dtype), torch.ones(dim), torch.zeros(dim)]
+    assert kernel_of(*args[:5], want_x=False) == "chan"
+    want = orc.selective_scan(*args, True, out_float=True, return_x=True)[0]
+    got = run_gpu(*args, True, True, want_x=False)[0]
+    for test in (torch.isposinf, torch.isneginf, torch.isnan):
+        assert torch.equal(test(got), test(want))
+    assert want[0, 0, 200:].isposinf().all() and want[0, 40, 200:].isneginf().all() and bool(want[0, 7, 1001:].isnan().all()) == (step > 1)
+    finite = want.isfinite()
+    assert torch.allclose(got[finite], want[finite], **TOL32)
+
+
 def test_scan_segments_in_a_graph():
     """Captured once, replayed with eager calls on other inputs between: every replay gives the eager call's bits."""
     args = [t.to(DEV) for t in make_inputs(36, 1, 64, 1, 16, 1024, torch.bfloat16, ss2d_like=True)]

@@ -20,7 +20,7 @@
 //
 // Few workgroups (small batches) leave the chip idle behind that serial chain.  Their rows are cut into segments that run side by side
 // in two launches of the same kernel, with one between them that walks the segments (ChanPhase, chan_segments): what a segment leaves
-// from state 0 and its sum of dl; what enters each, h_in' = exp2(A sum dl) h_in + h; the outputs from there.
+// from state 0, its sum of dl and its largest dl; what enters each, h_in' = exp2(A sum dl) h_in + h; the outputs from there.
 #include "scan_common.h"
 
 namespace ss2d {
@@ -168,6 +168,7 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
     __shared__ __align__(16) float s_du[kChanBlock * kChanTilePitch];
     __shared__ __align__(16) float s_y[kWavesPerWg * kChanBlock * kChanSubPitch];
     __shared__ float s_sum[kX || kPhase == kLocal ? kWavesPerWg * kChanBlock : 1];
+    __shared__ float s_max[kPhase == kLocal ? kWavesPerWg * kChanBlock : 1];
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -234,10 +235,11 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
     float *my_y = s_y + (wave * kChanBlock + lane) * kChanSubPitch;
     const float *sum_y = s_y + r * kChanSubPitch + 4 * q;
     float dl_sum = 0.0f;                                    // kX: this wavefront's quarter of the channel's sum of dl
+    float dl_max = 0.0f;                                    // kLocal: its largest
     const bool chan_ok = (int)cb * kChanBlock + lane < dpg;
     float *x_lane = kX ? p.x + ((int64_t)b * p.dim + dc) * p.n_chunks * 2 * p.N + 2 * (wave * kSpw) : nullptr;
 
-    // a segment's states, its sum of dl and (from the carry kernel) that of all before it, where its outputs will be
+    // a segment's states, its sum of dl, (from the carry kernel) that of all before it and its largest dl, where its outputs will be
     uint8_t *seg_state = reinterpret_cast<uint8_t *>(o_all + (int64_t)b * p.o_bs + (int64_t)dc * p.o_ds + begin);
     if constexpr (kPhase == kRest) {
         if (seg > 0) {
@@ -307,6 +309,7 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
                 if constexpr (kX || kPhase == kLocal) {
                     const float4 q4 = *reinterpret_cast<const float4 *>(my_dl + s * kChanSub + 4 * wave);
                     dl_sum += (q4.x + q4.y) + (q4.z + q4.w);  // (dl is 0 past the row's end)
+                    if constexpr (kPhase == kLocal) dl_max = fmaxf(fmaxf(dl_max, fmaxf(q4.x, q4.y)), fmaxf(q4.z, q4.w));
                 }
                 // the LDS reads above have landed before the first scalar request below is made (one wait covers both
                 // kinds of traffic, so a request issued earlier would be waited for at once)
@@ -381,12 +384,15 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
     }
     if constexpr (kPhase == kLocal) {
         s_sum[wave * kChanBlock + lane] = dl_sum;
+        s_max[wave * kChanBlock + lane] = dl_max;
         __syncthreads();
         if (!chan_ok) return;
         __builtin_memcpy(seg_state + sizeof(float) * (wave * kSpw), h, sizeof(h));
         if (wave == 0) {
             const float total = (s_sum[lane] + s_sum[kChanBlock + lane]) + (s_sum[2 * kChanBlock + lane] + s_sum[3 * kChanBlock + lane]);
+            const float most = fmaxf(fmaxf(s_max[lane], s_max[kChanBlock + lane]), fmaxf(s_max[2 * kChanBlock + lane], s_max[3 * kChanBlock + lane]));
             __builtin_memcpy(seg_state + sizeof(float) * p.N, &total, sizeof(total));
+            __builtin_memcpy(seg_state + sizeof(float) * (p.N + 2), &most, sizeof(most));
         }
     }
 }
@@ -406,12 +412,13 @@ __global__ __launch_bounds__(kBlock) void scan_chan_carry_kernel(const float *__
     float carry = 0.0f, before = 0.0f;
     constexpr int kFly = 8;
     for (int first = 0; first < n_segs; first += kFly) {
-        float left[kFly], sum[kFly];
+        float left[kFly], sum[kFly], most[kFly];
 #pragma unroll
         for (int i = 0; i < kFly; ++i) {                    // (past the last but one segment: that one again, not used)
             const uint8_t *from = state + min(first + i, n_segs - 2) * pitch;
             __builtin_memcpy(&left[i], from + sizeof(float) * n, sizeof(float));
             __builtin_memcpy(&sum[i], from + sizeof(float) * p.N, sizeof(float));
+            __builtin_memcpy(&most[i], from + sizeof(float) * (p.N + 2), sizeof(float));
         }
 #pragma unroll
         for (int i = 0; i < kFly; ++i) {
@@ -422,9 +429,11 @@ __global__ __launch_bounds__(kBlock) void scan_chan_carry_kernel(const float *__
                 if (n == 0) __builtin_memcpy(state + s * pitch + sizeof(float) * (p.N + 1), &before, sizeof(float));
             }
             before += sum[i];
-            // the product of the segment's a in two halves, so that neither leaves fp32's range before the state would; none of 0
+            // the product of the segment's a in two halves, so that neither leaves fp32's range before the state would; none of 0, and none of an
+            // infinite state: it stays infinite unless one of the a is 0 (the one of the largest dl, where A is negative), which leaves NaN
             const float half = __builtin_amdgcn_exp2f(0.5f * A2 * sum[i]);
-            carry = carry == 0.0f ? left[i] : fmaf(carry * half, half, left[i]);
+            if (fabsf(carry) == __builtin_inff()) carry = __builtin_amdgcn_exp2f(A2 * most[i]) > 0.0f ? carry + left[i] : __builtin_nanf("");
+            else carry = carry == 0.0f ? left[i] : fmaf(carry * half, half, left[i]);
         }
     }
 }
@@ -434,8 +443,8 @@ bool scan_chan_eligible(const ScanArgs &a) {
     return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.L % 8 == 0 && a.dim_per_group >= 32;
 }
 
-// The number of segments of a row (1: not cut) and the length of all but the last, which has at least 72 positions: a segment's N + 2
-// floats lie where its outputs will be.
+// The number of segments of a row (1: not cut) and the length of all but the last, which has at least 72 positions: a segment's N + 3
+// floats (the last one's N + 2) lie where its outputs will be.
 //
 // A workgroup takes 1.7 us per 16 positions of 16 states however few there are (1.0 of 4 states, 2.7 of 32).  Cut rows run the recurrence
 // twice (the first time without C), in three launches, and are ahead where the segments find room beside one another: three
