@@ -96,6 +96,34 @@ def test_strided_parameters(names, dtype):
         assert torch.equal(op.forward_core(x), want)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,W", [(7, 7), (8, 8), (9, 12)])
+@pytest.mark.parametrize("bad", range(4))
+def test_directions_and_channels_keep_to_themselves(H, W, dtype, bad):
+    """One direction's state of one channel overflows on the way, through a step of that direction alone (2^126, no decay): the merged map is
+    infinite nowhere but from there on in that direction's order, and the other channels have the bits they had."""
+    op, x = make(64, 5, dtype, 4), torch.rand(2, 64, H, W, device=DEV).add(0.5).to(dtype)
+    with torch.no_grad():
+        op.x_proj_weight.abs_()
+        op.x_proj_weight[:, 5:].div_(16)                             # B and C positive, below 1
+        c = op._inference_constants(0)
+        c = {"As": c["As"].view(-1).clone(), "Ds": c["Ds"].clone(), "dt_bias": c["dt_bias"].clone()}
+        call = lambda: core_few_hip(x, op.x_proj_weight, op.dt_projs_weight, c["As"], c["Ds"], c["dt_bias"])
+        clean = call()
+        c["As"][bad * 64 + 3], c["dt_bias"][bad * 64 + 3] = 0.0, 2.0 ** 126
+        got = call()
+        others = [d for d in range(64) if d != 3]
+        assert torch.equal(got[:, others], clean[:, others])
+        # the state in units of the step, which swallows its ranks; where the sum of two lanes' shares would overflow their outputs may still not
+        rows = torch.einsum("cd,bdl->bcl", op.x_proj_weight[bad].double(), routes(x.double())[bad]).to(dtype).double()
+        state = torch.cumsum(routes(x.double())[bad][:, 3] * rows[:, 5], -1)
+        value = torch.stack([state, 2.0 ** 126 * state * rows[:, 6]])
+        value = value.flip(-1) if bad >= 2 else value
+        state, value = value.view(2, 2, W, H).transpose(2, 3).flatten(2) if bad % 2 else value
+    over, near = state > 3.99, torch.isclose(got[:, 3].double(), value, rtol=1e-4 if dtype == torch.float32 else 2.0 ** -7)
+    assert 0 < over.sum() < over.numel() and bool((near | over & got[:, 3].isposinf()).all()) and bool(got[:, 3].isposinf().any())
+
+
 def test_rule():
     """Both sides of the line in one map's sizes, and what has no variant."""
     assert few_applies(1, 768, 7, 7, 48, torch.bfloat16) and few_applies(27, 768, 7, 7, 48, torch.bfloat16)

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(kFewThreads) void core_few_kernel(const FewCoreArgs
     }
     const T *my_rows = s_rows + dir * p.row, *my_x = s_x + chan * L;
     float2 *my_y = s_y + (chan * 4 + dir) * L;
-    float prod = t0 == 0 ? 0.0f : 1.0f, h = 0.0f;                                // (nothing enters a scan from the lanes before its first)
+    float prod = t0 == 0 ? 0.0f : 1.0f, h = 0.0f;                                // (nothing enters a scan's first position)
     for (int t = t0; t < t1; ++t) {
         const T *r = my_rows + pos * p.pitch;
         float z[2] = {bias, 0.0f};
@@ -261,7 +261,7 @@ __global__ __launch_bounds__(kFewThreads) void core_few_kernel(const FewCoreArgs
         pos += end ? wrap : step;
         left = end ? p.H - 1 : left - 1;
     }
-    const float h_in = row_scan_state_in<false>(prod, h);
+    const float h_in = kG == 8 ? octet_scan_state_in(prod, h) : row_scan_state_in<false>(prod, h);      // (of the direction's lanes)
     __shared__ float s_in[kFewThreads];
     s_in[threadIdx.x] = h_in;
     wave_lds_sync();

@@ -491,6 +491,22 @@ __device__ __forceinline__ float row_scan_state_in(float a, float h, float *a_in
     return hx;
 }
 
+// The same among groups of 8 lanes, two to a row: a lane takes nothing from the group below it -- not even times 0, which an infinite or NaN
+// state there would turn into NaN here.
+__device__ __forceinline__ float octet_scan_state_in(float a, float h) {
+    const int i = threadIdx.x & 7;
+#define SS2D_OCTET_STEP(N)                                                                                                            \
+    {                                                                                                                                 \
+        const float a_up = dpp_move<0x110 + N>(0.0f, a), h_up = dpp_move<0x110 + N>(0.0f, h);      /* row_shr:N */                 \
+        h = i >= N ? fmaf(a, h_up, h) : h;                                                                                            \
+        a = i >= N ? a * a_up : a;                                                                                                    \
+    }
+    SS2D_OCTET_STEP(1) SS2D_OCTET_STEP(2) SS2D_OCTET_STEP(4)
+#undef SS2D_OCTET_STEP
+    const float h_up = dpp_move<0x111>(0.0f, h);
+    return i >= 1 ? h_up : 0.0f;
+}
+
 // kS consecutive 16-bit elements of an LDS tile, packed two to a register as they sit there; item() widens element j.
 // Even kS: the run starts at an even element offset (4-byte reads).  Odd kS: it may start anywhere -- the dwords that
 // cover it are read and funnel-shifted into place (one more LDS element than the run is touched when it starts at an
