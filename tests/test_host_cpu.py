@@ -315,3 +315,24 @@ def test_replaced_functions_are_not_passed_by(name, monkeypatch):
     assert calls_unseen()
     monkeypatch.setattr(torch.nn.functional, name, lambda *a, **k: function(*a, **k))
     assert not calls_unseen()
+
+
+@pytest.mark.parametrize("on", ["class", "instance"])
+def test_replaced_projections_get_the_constants_they_had(on, monkeypatch):
+    """project_from_map of a subclass, or set on the instance, is called in training with the weights repeated over the images, as at any size."""
+    from vmamba_amd import ss2d
+    monkeypatch.setattr(ss2d, "projections_train", lambda *args: True)
+
+    class Called(Exception):
+        pass
+
+    def project_from_map(self, x, consts):
+        raise Called(sorted(consts))
+
+    kind = type("Own", (SS2D,), {"project_from_map": project_from_map}) if on == "class" else SS2D
+    op = kind(d_model=16)
+    if on == "instance":
+        op.project_from_map = lambda x, consts: project_from_map(op, x, consts)
+    with pytest.raises(Called) as called:
+        op.forward_core(torch.zeros(1, 16, 4, 4))
+    assert {"Wx_all", "Wx", "Wdt"} <= set(called.value.args[0])

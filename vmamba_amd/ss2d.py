@@ -122,6 +122,7 @@ def _pad_mask(H0, W0, H, W, n_images, device):
 
 _CORE_PARAMS = ("A_logs", "Ds", "dt_projs_bias", "x_proj_weight", "dt_projs_weight")
 _CORE_STEPS = ("forward_core_fused", "finish_core", "_inference_constants")      # what SS2D._forward_core_native stands for
+_PROJECTION_STEPS = ("project_from_map", "_inference_constants")                 # what knows the constants without repeated weights
 
 
 class SS2D(nn.Module):
@@ -342,7 +343,8 @@ class SS2D(nn.Module):
             return out
         B, D, H, W = x.shape
         K, L = self.k_group, H * W
-        trains = needs_grad(x, self.x_proj_weight, self.dt_projs_weight) and projections_train(x, self.x_proj_weight, self.dt_projs_weight)
+        trains = (needs_grad(x, self.x_proj_weight, self.dt_projs_weight) and projections_train(x, self.x_proj_weight, self.dt_projs_weight)
+                  and all(getattr(type(self), n) is getattr(SS2D, n) for n in _PROJECTION_STEPS) and vars(self).keys().isdisjoint(_PROJECTION_STEPS))
         consts = self._inference_constants(0 if trains else B)
         if not trains and self._fused_core_applies(x):
             try:
