@@ -336,3 +336,17 @@ def test_replaced_projections_get_the_constants_they_had(on, monkeypatch):
     with pytest.raises(Called) as called:
         op.forward_core(torch.zeros(1, 16, 4, 4))
     assert {"Wx_all", "Wx", "Wdt"} <= set(called.value.args[0])
+
+
+def test_weights_of_another_kind_are_left_to_their_layer():
+    """A weight that is another kind of tensor answers the layer's own call in training: LinearDw would read its memory."""
+    from vmamba_amd.linear import linear_dw_pays
+
+    class Kind(torch.Tensor):
+        pass
+
+    layer, rows = torch.nn.Linear(8, 8, bias=False), _OnGpu(torch.zeros(4096, 8))
+    rows.device = torch.device("cpu")                                # the weight's own
+    assert linear_dw_pays(layer, rows)
+    layer.weight = torch.nn.Parameter(layer.weight.detach().as_subclass(Kind))
+    assert type(layer.weight) is Kind and not linear_dw_pays(layer, rows)

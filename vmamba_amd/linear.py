@@ -309,7 +309,7 @@ def linear_dw_pays(layer, x):
         return False
     weight = layer.weight
     N, K = weight.shape
-    return (torch.is_grad_enabled() and weight.requires_grad and weight.dtype == x.dtype and weight.device == x.device
+    return (torch.is_grad_enabled() and type(weight) in TENSOR_KINDS and weight.requires_grad and weight.dtype == x.dtype and weight.device == x.device
             and x.shape[-1] == K and N % 4 == 0 and K % 4 == 0 and N * K > 0 and x.numel() >= 4096 * K
             and (N * K <= 384 * 384 or (x.numel() >= TRAIN_FROM and product_pays(x.numel() // K, N, K))) and not observed(layer) and calls_unseen())
 
