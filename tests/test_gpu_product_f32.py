@@ -191,10 +191,37 @@ def test_projections_of_the_core_in_training():
         ss2d.projections_train = takes
     for g, w in zip(got, want):
         assert ((g - w).norm() / w.norm()).item() < 1e-5
-    # a second backward through the projections
-    rows = ss2d.XProjF32.apply(x, op.x_proj_weight)
-    dx = torch.autograd.grad(rows.square().sum(), x, create_graph=True)[0]
-    assert torch.autograd.grad(dx.sum(), op.x_proj_weight)[0].isfinite().all()
+
+
+def routes(x):
+    """(B, D, H, W) -> (B, 4, D, L) in the directions' scan orders."""
+    rows, cols = x.flatten(2), x.transpose(2, 3).flatten(2)
+    return torch.stack([rows, cols, rows.flip(-1), cols.flip(-1)], 1)
+
+
+@pytest.mark.parametrize("what", ["x_proj", "dt_proj", "transpose"])
+def test_second_derivatives_of_the_projections(what):
+    """Both derivatives of the cubes' sum, every input, against the same expression in float64: sums of up to 1000 terms in fp32."""
+    from vmamba_amd.core import DtProjF32, XProjF32
+    from vmamba_amd.csm import TransposeBCL
+    g = torch.Generator().manual_seed(3)
+    make = lambda *s: torch.randn(*s, generator=g).to(DEV).requires_grad_()
+    if what == "x_proj":
+        wanted = [make(2, 32, 6, 9), make(4, 5, 32)]
+        call, exact = XProjF32.apply, lambda x, w: torch.matmul(w, routes(x))
+    elif what == "dt_proj":
+        wanted = [make(4, 6, 200), make(4, 24, 6)]
+        call, exact = DtProjF32.apply, lambda rows, w: torch.matmul(w, rows)
+    else:
+        wanted = [make(3, 20, 33)]
+        call, exact = TransposeBCL.apply, lambda x: x.transpose(1, 2)
+
+    def derivatives(f, inputs):
+        y = f(*inputs)
+        first = torch.autograd.grad((y ** 3).sum(), inputs, create_graph=True)
+        return [y.detach()] + [t.detach() for t in first] + list(torch.autograd.grad(sum((t ** 2).sum() for t in first), inputs))
+    for got, want in zip(derivatives(call, wanted), derivatives(exact, [t.detach().double().requires_grad_() for t in wanted])):
+        assert got.shape == want.shape and ((got.double() - want).norm() / want.norm()).item() < 1e-5
 
 
 GELU_RANGES = [(-0.01, 0.01), (-0.5, 0.0), (0.0, 0.5), (-1.0, -0.5), (0.5, 1.0), (-1.5, -1.0), (1.0, 1.5), (-2.0, -1.5), (1.5, 2.0), (-3.0, -2.0), (2.0, 3.0),
