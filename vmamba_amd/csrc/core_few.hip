@@ -10,7 +10,7 @@
 //     the LDS copy all eight wavefronts share.  The step is the fp32 sum over the ranks, two to an instruction, never rounded to 16
 //     bits and never in memory.  Outputs meet in LDS planes, one per direction, and leave as (y0 + y2) + (y1 + y3) + (D0 + .. + D3) x.
 // What bounds such a call is a trip to memory per launch and the instructions, which every launch fetches anew (see core_few_kernel):
-// the three launches of one image of 768 x 7 x 7 now take 6.1, 6.7 and 5.4 us.  Whole calls: few_pays.
+// the three launches of one image of 768 x 7 x 7 now take 6.1, 6.7 and 6.5 us (17.9 in a graph).  Whole calls: few_pays.
 #include "scan_common.h"
 
 namespace ss2d {

@@ -903,7 +903,8 @@ template <typename in_t, typename w_t, typename out_t>
 static int launch_ln_cf_position(const void *x, const void *w, const void *b, void *y, int B, int C, int L, float eps,
                                  int out_channel_last, hipStream_t stream) {
     const int n_pos = B * L;
-    // a wavefront per workgroup while that spreads the positions over more CUs: 768 x 7 x 7 6.1 -> 5.4 us, 16 of 8 x 8 the other way, 6.9 -> 7.4
+    // a wavefront per workgroup while that spreads the positions over more CUs (twenty in a graph, us each): 768 x 7 x 7 6.5 -> 5.7, 8 x 8 7.0 -> 5.7;
+    // 16 of 8 x 8 the other way, 6.9 -> 7.4
     const int waves = n_pos <= 256 ? 1 : kBlock / kWave;
     const dim3 grid((uint32_t)((n_pos + waves - 1) / waves)), block(waves * kWave);
     const FastDiv by_image = make_fastdiv((uint32_t)L);

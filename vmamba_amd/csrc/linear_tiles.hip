@@ -7,8 +7,8 @@
 //     step, and a wait that leaves the newer step's loads in flight --, or one step ahead in a ring of two (kTlThreePerCu);
 //   * a row of a step is 64 bytes of LDS, its four 16-byte pieces in an order that differs from row to row, so that lanes with a row each read
 //     all banks once; the order is made by the addresses the lanes load from, the LDS side being linear;
-//   * a lane's accumulators are runs of four outputs of one position.  They go through LDS into rows, which leave 16 bytes a lane with the
-//     residual read the same way.
+//   * a lane's accumulators are runs of four outputs of one position, where a residual is added, 8 bytes a lane.  They go through LDS into rows,
+//     which leave 16 bytes a lane.
 // Rounding follows the separate operators: the product with its bias is rounded to T, GELU of that once more; a residual is added before the
 // rounding, as the library's addmm does it.
 #include "gelu.h"

@@ -18,9 +18,9 @@
 //     not vanish that count in fp32.  (Without it a value of 2^-116 is off by 3e-6 of itself; 1 to 3 % of the time.)
 //   * infinities and NaN, and values that round beyond bf16's largest or sums beyond fp32's (from 2^104 and 2^80 on), leave a NaN or an infinity in the
 //     sums: a wavefront that finds one computes its outputs again on the fp32 matrix cores, from memory.
-// 12 544 x 1536 x 384: 148 us as the library's product (100 TFLOP/s), 108 here (137); 384 x 1536 outputs over 12 544 positions, both by columns,
-// 144 -> 105.  What bounds it is the matrix cores' rate under load, 1.2 PFLOP/s in bf16 on this card, a sixth of it here: 200; then the
-// split's instructions between them.  One accumulator for all six, three workgroups per CU: 93, and the bias above.  Against 64 bits the error
+// 12 544 x 1536 x 384: 146 us as the library's product (101 TFLOP/s), 104 here (142); 384 x 1536 outputs over 12 544 positions, both by columns,
+// 142 -> 91.  What bounds it is the matrix cores' rate under load, 1.2 PFLOP/s in bf16 on this card, a sixth of it here: 200; then the
+// split's instructions between them.  One accumulator for all six, three workgroups per CU: 93 where two took 108, and the bias above.  Against 64 bits the error
 // is 1.1e-7 (library 3.5e-7), of the gradient 1.6e-7 (2.0e-6).  Two fp16 parts and three products would be twice as fast and hold less
 // than fp32's range.
 #include "normal_cdf.h"
@@ -306,9 +306,10 @@ __global__ __launch_bounds__(kBlock) void product_f32_sum_kernel(const ProductAr
 }
 
 // How a product is cut.  Tiles of 128 x 128, two workgroups per CU, where there are several rounds of them and for gradients, whose long sum
-// is cut into shares until they fill the chip; else 128 x 64, three per CU: 12 544 positions, us, 1536 x 384 108 (128 x 64: 115); gradient of 1536 x 384
-// 105 (109); 384 x 1536 127 in two shares, 112 with 128 x 64; 384 x 384 36, 33.  Shares of eight steps at least: fewer terms and the
-// second kernel costs more than the workgroups give.
+// is cut into shares until they fill the chip; else 128 x 64, three per CU.  us, 128 x 128 / 128 x 64, over 12 544 positions: 1536 x 384
+// 104 / 110, 384 x 1536 (two shares of the larger tiles) 126 / 113, 384 x 384 37 / 33; gradients: 1536 x 384 91 / 109; up to 384 x 384 outputs the smaller tiles
+// are ahead, 384 x 384 43 / 42, 256 x 256 35 / 32, 96 x 96 over 200 704 158 / 137 (a block's own of that size are ss2d_linear_dw_f32's).  Shares of
+// eight steps at least: fewer terms and the second kernel costs more than the workgroups give.
 static int product_plan(int64_t M, int N, int64_t K, bool a_cols, bool b_cols, ProductArgs &a, int64_t &shares) {
     if (M <= 0 || N <= 0 || K <= 0 || N % 4 != 0 || (a_cols ? M % 4 != 0 : K % 4 != 0) || (!b_cols && K % 4 != 0)) return SS2D_ENOTSUP;
     const int64_t tiles_m = (M + kPfTile - 1) / kPfTile, most = K / (8 * kPfDepth);

@@ -258,10 +258,10 @@ def product_f32_hip(a, b, a_by_columns=False, b_by_columns=False, bias=None, oth
 def product_pays(M, N, K, gradient=False):
     """True where ss2d_product_f32 is ahead of the library's fp32 product, whose rate is 90-100 TFLOP/s at best.  The kernel needs
     workgroups: 384 tiles of 128 x 64 outputs, or shares of a long sum (``gradient``: both operands by columns, K the positions), or 6 G
-    products in any cut.  us, library / kernel: 12 544 x 1536 x 384 159 / 109, x 384 x 1536 157 / 120, x 384 x 384 49 / 35 (588 tiles); 50 176 x 96 x 96
-    29 / 19; 1176 x 2048 x 512 37 / 33 (320 tiles, left), 4181 x 384 x 384 16 / 20 (198), 3136 x 768 x 192 14 / 16 (300); 9408 x 512 x 2048 191 / 151
-    (592 tiles), 3136 x 512 x 2048 57 / 61 (3.3 G), 2090 x 768 x 3072 82 / 83 (4.9 G).  Gradients: 1536 x 384 over 12 544 positions 144 / 91, 384 x 96 over
-    50 176 256 / 75, 256 x 1024 over 6272 39 / 39, 768 x 192 over 3136 22 / 28."""
+    products in any cut.  us in a graph, library / kernel: 12 544 x 1536 x 384 146 / 104, x 384 x 1536 147 / 114, x 384 x 384 48 / 34 (588 tiles);
+    50 176 x 96 x 96 28 / 18; 1176 x 2048 x 512 38 / 34 (320 tiles, left), 4181 x 384 x 384 16 / 22 (198), 3136 x 768 x 192 13 / 15 (300);
+    9408 x 512 x 2048 188 / 148 (592 tiles), 3136 x 512 x 2048 55 / 61 (3.3 G), 2090 x 768 x 3072 79 / 83 (4.9 G).  Gradients: 1536 x 384 over
+    12 544 positions 142 / 91, over 4096 50 / 42, 384 x 96 over 50 176 253 / 74, 256 x 1024 over 6272 42 / 38, 768 x 192 over 3136 22 / 28."""
     if gradient:
         return K >= 4096
     return -(-M // 128) * -(-N // 64) >= 384 or M * N * K >= 6 << 30
@@ -287,7 +287,8 @@ def _product(a, b, a_by_columns=False, b_by_columns=False, bias=None, other=None
 
 
 def _weight_gradient(dy, x):
-    """dy^T x, dy (M, N) and x (M, K)."""
+    """dy^T x, dy (M, N) and x (M, K).  Up to 384 x 384 outputs ss2d_linear_dw_f32 has the longest sums and ss2d_product_f32, in graphs, some of
+    the others: 96 x 96 over 200 704 positions 136 / 158 us, over 50 176 87 / 68, 192 x 192 over 50 176 70 / 72, 384 x 384 over 12 544 51 / 43, 256 x 256 44 / 35."""
     N, K = dy.shape[1], x.shape[1]
     if N * K <= 384 * 384 and x.shape[0] >= 4096 and N % 4 == 0 and K % 4 == 0 and not torch.is_grad_enabled() and memory_readable(x, dy):
         x, dy = x.contiguous(), dy.contiguous()
@@ -303,8 +304,8 @@ def _plain_f32(x, *tensors):
 def linear_dw_pays(layer, x):
     """True when LinearDw stands for ``layer(x)`` in training: a plain nn.Linear without bias, hooks or autocast, on float32
     positions many enough and with outputs few enough that the library leaves most of the chip idle, or where ss2d_product_f32 is ahead
-    of it.  12 544 positions, weight gradient, library against kernel in us: 384 x 384 outputs 77 against 54.
-    96 x 96 over 200 704: 443 against 141; 384 x 384 over 3136: 25 against 28."""
+    of it.  12 544 positions, weight gradient, library against kernel in us: 384 x 384 outputs 72 against 51.
+    96 x 96 over 200 704: 435 against 136; 384 x 384 over 6272: 36 against 36, over 4096: 25 against 31."""
     if not (type(layer) is nn.Linear and layer.bias is None and x.is_cuda and x.dim() >= 2 and x.dtype == torch.float32):
         return False
     weight = layer.weight

@@ -128,7 +128,9 @@ TENSOR_KINDS = (torch.Tensor, nn.Parameter)
 
 # Elements of the activation from which training in single precision takes this package's own autograd functions for LayerNorm, the MLP and
 # the core's projections.  They are Python on the host, up to 10 us a call more than torch's, and a block of fewer elements waits for the host
-# -- 1.35 ms a step, whatever runs --: 736 x 16 x 16, two images (0.4 Mi) 1355 us, with them 1464; 576 x 51 x 38, three images (3.3 Mi) 2068 -> 1715.
+# -- 1.3 to 1.7 ms a step by box, whatever runs.  A block's step without / with them, us, from 2.1 Mi elements on: 192 x 28 x 28, 16 images (2.3 Mi) 1678 / 1590,
+# 384 x 14 x 14, 30 (2.15) 1689 / 1618, 576 x 51 x 38, two (2.13) 1474 / 1392, 736 x 16 x 16, 12 (2.16) 1667 / 1520, 96 x 56 x 56, 8 (2.3) 1713 / 1514; below it goes either way:
+# 768 x 7 x 7, 52 (1.87) 1644 / 1698, 736 x 16 x 16, 8 (1.44) 1331 / 1374, 384 x 14 x 14, 20 (1.44) 1653 / 1652, 192 x 28 x 28, 12 (1.72) 1674 / 1595, 576 x 51 x 38, one (1.06) 1285 / 1320.
 TRAIN_FROM = 2 << 20
 
 
