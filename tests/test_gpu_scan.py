@@ -129,10 +129,8 @@ def test_scan_matches_oracle(batch, dim, G, N, L, dtype):
     check(*make_inputs(21, batch, dim, G, N, L, dtype), True)
 
 
-# Several states per channel with enough channels per group: the channel-per-lane kernel (64 channels of one group per
-# workgroup, the four wavefronts splitting the states).  Groups of exactly one block, of 1.5 blocks (a half-filled
-# second block), of 48 channels (lanes idle); rows of one round, of whole steps, ending mid-step and mid-round;
-# 4 / 8 / 16 / 32 states.
+# Several states per channel with enough channels per group: the channel-per-lane kernel.  Groups of 64, 96 and 48
+# channels; rows of one round, of whole steps, ending mid-step and mid-round; 4 / 8 / 16 / 32 states.
 CHAN_GRID = [
     (2, 128, 2, 16, 520), (1, 96, 1, 16, 200), (2, 192, 4, 8, 72), (1, 64, 1, 4, 1000), (1, 128, 2, 32, 136),
     (3, 64, 2, 16, 8), (1, 256, 1, 16, 3136), (2, 96, 2, 16, 48), (1, 80, 2, 8, 2056),
@@ -166,9 +164,8 @@ def test_scan_channel_per_lane_kernel_matches_oracle(batch, dim, G, N, L, dtype)
     check_states(x, xw)
 
 
-# Few workgroups: the rows are cut into segments.  The fewest and shortest of them (3 of 128), one position group less (whole), a last
-# segment that would be too short for its state (joined to the one before), many segments, 2048 inside one and at the end of one,
-# both sides of 64 workgroups (400 positions) and of four segments (512 and 504 positions, 96 workgroups).
+# Few wavefronts: the rows are cut into segments.  Few and short ones, a last segment that would be too short for its state (joined to
+# the one before), many segments, 2048 inside one and at the end of one, and more wavefronts with rows of 400 to 512 positions.
 SEGMENTS = [(1, 64, 1, 32, 384), (1, 64, 1, 32, 376), (1, 48, 1, 32, 520), (1, 96, 1, 16, 4112), (1, 64, 1, 4, 4096), (1, 33, 1, 8, 9000),
             (64, 64, 1, 16, 400), (65, 64, 1, 16, 400), (96, 64, 1, 4, 512), (96, 64, 1, 4, 504)]
 
@@ -188,6 +185,26 @@ def test_scan_rows_cut_into_segments(batch, dim, G, N, L, dtype):
     if dtype != torch.float32:
         small, _ = run_gpu(*args, True, False, want_x=False)
         assert torch.equal(small, got.to(dtype))
+
+
+# Blocks of 16 channels and steps of 32 positions: groups that leave 1, 15 and 14 channels to the last block, one to four blocks to the
+# last workgroup; rows of half a round, of a round and a half, of a step and half a round; 576 and 580 wavefronts of rows that would be
+# cut, 192 and 204 of three segments.
+BLOCKS = [(1, 33, 1, 16, 8), (2, 47, 1, 8, 24), (1, 186, 3, 32, 40), (1, 51, 1, 4, 56), (3, 35, 1, 16, 72),
+          (144, 64, 1, 4, 512), (145, 64, 1, 4, 512), (64, 48, 1, 16, 384), (68, 48, 1, 16, 384)]
+
+
+@pytest.mark.parametrize("batch,dim,G,N,L", BLOCKS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_blocks_of_channels(batch, dim, G, N, L, dtype):
+    _announce("scan-blocks", batch, dim, G, N, L, dtype)
+    args = make_inputs(36, batch, dim, G, N, L, dtype, ss2d_like=True)
+    assert kernel_of(*args[:5], want_x=False) == "chan"
+    want, xw = orc.selective_scan(*args, True, out_float=True, return_x=True)
+    got, x = run_gpu(*args, True, True, want_x=True)
+    assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
+    check_states(x, xw, TOL32)
+    assert torch.equal(run_gpu(*args, True, True, want_x=False)[0], got)
 
 
 def test_scan_segments_hold_what_a_whole_row_does():

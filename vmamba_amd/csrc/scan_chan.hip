@@ -2,23 +2,25 @@
 // serially along the sequence.
 //
 // With N states the work per position is N recurrences  h_n = a_n h_n + B_n du,  y += C_n h_n.  The wavefront-scan
-// kernels (selective_scan.hip) pay a 64-lane DPP scan per (512 positions, state) and fetch B / C per lane.  Here the
-// 64 lanes of a wavefront are 64 channels of one (image, group): all of them meet the same B_n,t and C_n,t, so these
-// are wave-uniform values that ride in scalar registers (the loads below have uniform addresses), the recurrence is a
-// plain serial chain per lane -- multiply, exp2, multiply, two fused multiply-adds per (position, state) -- and no
-// scan, no carry logic and no per-lane B / C traffic remain.
+// kernels (selective_scan.hip) pay a 64-lane DPP scan per (512 positions, state).  Here a lane is one channel of one (image, group)
+// and a quarter of its states, and the recurrence is a plain serial chain per lane -- multiply, exp2, multiply, two fused multiply-adds
+// per (position, state) -- with no scan and no carry logic.
 //
-// Parallelism: a workgroup owns 64 channels; its four wavefronts split the STATES (N/4 each), so each keeps N/4
-// independent chains in flight, and their partial sums over n meet in LDS.  Per step of 32 positions:
-//   stage    thread (row r = tid/4, quarter q) loads 2 x 4 positions of u and delta of channel r (the next step's loads
-//            are issued before this step's arithmetic), computes dl = softplus(delta + bias), du = dl u and the skip
-//            term D u, and writes dl / du into LDS tiles [channel][position] -- the transposition that lets global
-//            accesses run along the sequence while the compute phase reads along channels;
-//   compute  twice 16 positions: every lane reads its channel's dl / du (16-byte LDS reads), runs its wavefront's
-//            states over them and leaves 16 partial outputs in LDS;
-//   combine  thread (r, q) adds the four partials and the skip term for 4 positions and stores them (16 bytes of fp32).
+// A wavefront owns 16 channels: lane = channel % 4 + 4 set + 16 (channel / 4), the four sets sharing out the states.  It meets no other
+// wavefront: its LDS tiles are its own and there is no workgroup barrier.  Per step of 32 positions:
+//   stage    lane (row r = lane / 4, quarter q) loads 2 x 4 positions of u and delta of channel r (requested a step ahead), computes
+//            dl = softplus(delta + bias), du = dl u and the skip term D u, and writes dl / du into LDS tiles [channel][position] -- the
+//            transposition that lets global accesses run along the sequence while the compute phase reads along channels;
+//   compute  twice 16 positions: B and C of all states go to LDS as fp32 (requested 32 positions ahead) and are read back as 16-byte
+//            broadcasts; the four sets' sums meet in DPP additions that leave 4 positions with each set (sum_over_sets);
+//   output   through the dl tile back to lane (r, q), which adds the skip term and stores.
+// What bounds it: vector issue.  64 maps of 192 x 56 x 56 as four directions, 16 states: 624 us, 98 % of it issuing, at 4.8 cycles per vector
+// instruction and 1.9 GHz; 6.5 instructions per (position, state) of which the recurrence is 5 with one exp2 at 8 cycles.  A workgroup of 64
+// channels whose wavefronts share out the states and meet at four barriers per step, B and C in scalar registers (a fused multiply-add
+// with a scalar operand takes twice the cycles): 641; 16 images of 192 x 28 x 28: 90, now 68, as there are four times as many wavefronts
+// as blocks of 64 channels and each is done on its own.
 //
-// Few workgroups (small batches) leave the chip idle behind that serial chain.  Their rows are cut into segments that run side by side
+// Few wavefronts (small batches) leave the chip idle behind that serial chain.  Their rows are cut into segments that run side by side
 // in two launches of the same kernel, with one between them that walks the segments (ChanPhase, chan_segments): what a segment leaves
 // from state 0, its sum of dl and its largest dl; what enters each, h_in' = exp2(A sum dl) h_in + h; the outputs from there.
 #include "scan_common.h"
@@ -29,78 +31,25 @@ constexpr int kChanTile = 32;                     // positions staged per step
 constexpr int kChanSub = 16;                      // positions per compute / combine round
 constexpr int kChanTilePitch = kChanTile + 4;     // floats; + 4 spreads the 16-byte reads of 8 lanes over all banks
 constexpr int kChanSubPitch = kChanSub + 4;
-constexpr int kChanBlock = 64;                    // channels per workgroup
-
-// The B and C values of one state for one round of 16 positions, as loaded: two halves of 8 positions, each at a
-// wave-uniform, 16-byte aligned address.  The addresses are uniform and the memory is read-only for the kernel, so these
-// are scalar loads and the widening to fp32 is scalar ALU work.
-template <typename in_t> struct UniRaw {
-    static constexpr int kVecs = (int)sizeof(in_t);      // 16-byte pieces per 16 elements
-    uint4 b[kVecs], c[kVecs];
-};
-
-template <typename in_t>
-__device__ __forceinline__ void load_uniform(const in_t *__restrict__ Brow, const in_t *__restrict__ Crow, int half0, int half1,
-                                             UniRaw<in_t> &r) {
-    constexpr int kHalfVecs = UniRaw<in_t>::kVecs / 2;  // 1 (16-bit) or 2 (fp32) pieces per 8 elements
-    constexpr int kPer = 16 / (int)sizeof(in_t);
-#pragma unroll
-    for (int v = 0; v < kHalfVecs; ++v) {
-        r.b[v] = *reinterpret_cast<const uint4 *>(Brow + half0 + v * kPer);
-        r.b[kHalfVecs + v] = *reinterpret_cast<const uint4 *>(Brow + half1 + v * kPer);
-        r.c[v] = *reinterpret_cast<const uint4 *>(Crow + half0 + v * kPer);
-        r.c[kHalfVecs + v] = *reinterpret_cast<const uint4 *>(Crow + half1 + v * kPer);
-    }
-}
-
-// Makes the compiler wait here until every dword of r has arrived (it places its wait before the first use of a loaded
-// register, and scalar loads complete out of order, so that wait is for all outstanding ones): put in front of the
-// NEXT set of requests, it keeps them out of the wait for this set.
-template <typename in_t>
-__device__ __forceinline__ void arrived(const UniRaw<in_t> &r) {
-#pragma unroll
-    for (int v = 0; v < UniRaw<in_t>::kVecs; ++v)
-        asm volatile("" ::"s"(r.b[v].x), "s"(r.b[v].y), "s"(r.b[v].z), "s"(r.b[v].w), "s"(r.c[v].x), "s"(r.c[v].y), "s"(r.c[v].z),
-                     "s"(r.c[v].w));
-}
-
-template <typename in_t>
-__device__ __forceinline__ void widen16(const uint4 (&w)[UniRaw<in_t>::kVecs], float (&v)[16]) {
-    if constexpr (sizeof(in_t) == 2) {
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const uint32_t ww[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                v[8 * k + 2 * i] = to_f32(in_t{(uint16_t)(ww[i] & 0xffffu)});
-                v[8 * k + 2 * i + 1] = to_f32(in_t{(uint16_t)(ww[i] >> 16)});
-            }
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            v[4 * k] = bits_to_f32(w[k].x); v[4 * k + 1] = bits_to_f32(w[k].y);
-            v[4 * k + 2] = bits_to_f32(w[k].z); v[4 * k + 3] = bits_to_f32(w[k].w);
-        }
-    }
-}
+constexpr int kChanBlock = 16;                    // channels per wavefront
+constexpr int kChanSets = 4;                      // lanes per channel, each with a quarter of the states
 
 // Four consecutive elements of a row as loaded (8 bytes of 16-bit values or 16 bytes of fp32).
 template <typename in_t> struct Raw4 { uint32_t w[sizeof(in_t)]; };
 
+// From byte offset `off` of a buffer whose end the hardware checks: past it (kNowhere) the elements are 0.  No branch: the
+// wait for a load behind one would be at its end, not where the elements are used.
+constexpr uint32_t kNowhere = 0xfffffff0u;
+
 template <typename in_t>
-__device__ __forceinline__ Raw4<in_t> load_raw4(const in_t *__restrict__ row, int pos, int L, float fill) {
+__device__ __forceinline__ Raw4<in_t> load_raw4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off) {
     Raw4<in_t> r;
     if constexpr (sizeof(in_t) == 2) {
-        const uint32_t f2 = (uint32_t)from_f32<in_t>(fill).bits * 0x10001u;
-        uint2 v = make_uint2(f2, f2);
-        if (pos < L) v = *reinterpret_cast<const uint2 *>(row + pos);
-        r.w[0] = v.x; r.w[1] = v.y;
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)off, 0, 0);
+        r.w[0] = v[0]; r.w[1] = v[1];
     } else {
-        const uint32_t f = f32_to_bits(fill);
-        uint4 v = make_uint4(f, f, f, f);
-        if (pos < L) v = *reinterpret_cast<const uint4 *>(row + pos);
-        r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0);
+        r.w[0] = v[0]; r.w[1] = v[1]; r.w[2] = v[2]; r.w[3] = v[3];
     }
     return r;
 }
@@ -117,16 +66,27 @@ __device__ __forceinline__ void unpack_raw4(const Raw4<in_t> &r, float (&v)[4]) 
 }
 
 template <typename out_t>
-__device__ __forceinline__ void store4(out_t *__restrict__ dst, const float (&v)[4]) {
+__device__ __forceinline__ void store4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, const float (&v)[4]) {
+    typedef uint32_t words4_t __attribute__((ext_vector_type(4)));
+    typedef uint32_t words2_t __attribute__((ext_vector_type(2)));
     if constexpr (sizeof(out_t) == 4) {
-        *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+        const words4_t w = {f32_to_bits(v[0]), f32_to_bits(v[1]), f32_to_bits(v[2]), f32_to_bits(v[3])};
+        __builtin_amdgcn_raw_buffer_store_b128(w, rsrc, (int)off, 0, 0);
     } else {
-        *reinterpret_cast<uint2 *>(dst) = make_uint2(pack2_from_f32<out_t>(v[0], v[1]), pack2_from_f32<out_t>(v[2], v[3]));
+        const words2_t w = {pack2_from_f32<out_t>(v[0], v[1]), pack2_from_f32<out_t>(v[2], v[3])};
+        __builtin_amdgcn_raw_buffer_store_b64(w, rsrc, (int)off, 0, 0);
     }
 }
 
+// `rows` rows of L elements, `stride` apart
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const T *first, int rows, int64_t stride, int L) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(first), 0, (int)(((rows - 1) * stride + L) * (int)sizeof(T)), kBufferRsrcWord3);
+}
+
 struct ChanGeom {
-    int32_t n_cb;            // channel blocks of 64 per group
+    uint32_t n_units;        // wavefronts
+    int32_t n_cb;            // channel blocks per group
     FastDiv div_cb, div_groups;
     int32_t seg_len, n_segs;                 // of a row cut into segments (kLocal, kRest)
     FastDiv div_segs;                        // segments of a row that this launch walks
@@ -137,9 +97,8 @@ enum ChanPhase { kWhole, kLocal, kRest };
 
 // kX: the chunk-end states are written as well -- x[row][chunk][2n] = product of a_n since the row's start,
 // x[..][2n + 1] = h_n, after every 2048 positions and at the row's end.  h is what the lane holds; the product is
-// exp2(A_n log2e * sum dl), and the sum is per CHANNEL, not per state: each of the four wavefronts adds up a quarter of
-// every round's positions for its lane's channel (one LDS read, four adds per 16 positions) and the quarters meet in LDS
-// when a chunk ends.
+// exp2(A_n log2e * sum dl), and the sum is per CHANNEL, not per state: each of a channel's four lanes adds up a quarter of
+// every round's positions (one LDS read, four adds per 16 positions) and the quarters meet when a chunk ends.
 //
 // kMaps: CrossScan folded in.  u is not the (batch, 4 D, L) tensor of the four scan-ordered copies but the map itself,
 // x (batch, D, L), plus its transpose xt (batch, D, L: every H x W map stored as W x H): direction k = the channel's
@@ -158,219 +117,255 @@ __device__ __forceinline__ Raw4<in_t> reverse4(const Raw4<in_t> &r) {
     return o;
 }
 
+// y[i] summed over the four sets of lanes (the banks of four lanes in a row of 16) for every position i of 16: afterwards
+// y[0 .. 3] are positions 4 set .. 4 set + 3.  Two DPP additions, each with its own banks, put two positions into one register:
+// half the additions of a sum that every lane gets, and no selects.
+__device__ __forceinline__ void sum_over_sets(float (&y)[16]) {
+#define SS2D_ADD(R, S, CTRL) "v_add_f32_dpp %" #R ", %" #S ", %" #S " " CTRL "\n\t"
+#define SS2D_ALL(R) SS2D_ADD(R, R, "row_ror:8 row_mask:0xf bank_mask:0xf")
+#define SS2D_UPPER(R, S) SS2D_ADD(R, S, "row_ror:8 row_mask:0xf bank_mask:0xc")
+#define SS2D_EVEN(R) SS2D_ADD(R, R, "row_shl:4 row_mask:0xf bank_mask:0x5")
+#define SS2D_ODD(R, S) SS2D_ADD(R, S, "row_shr:4 row_mask:0xf bank_mask:0xa")
+    asm("s_nop 1\n\t"
+        SS2D_ALL(0) SS2D_ALL(1) SS2D_ALL(2) SS2D_ALL(3) SS2D_ALL(4) SS2D_ALL(5) SS2D_ALL(6) SS2D_ALL(7)
+        SS2D_UPPER(0, 8) SS2D_UPPER(1, 9) SS2D_UPPER(2, 10) SS2D_UPPER(3, 11)
+        SS2D_UPPER(4, 12) SS2D_UPPER(5, 13) SS2D_UPPER(6, 14) SS2D_UPPER(7, 15)
+        SS2D_EVEN(0) SS2D_EVEN(1) SS2D_EVEN(2) SS2D_EVEN(3)
+        SS2D_ODD(0, 4) SS2D_ODD(1, 5) SS2D_ODD(2, 6) SS2D_ODD(3, 7)
+        "s_nop 1"
+        : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(y[4]), "+v"(y[5]), "+v"(y[6]), "+v"(y[7])
+        : "v"(y[8]), "v"(y[9]), "v"(y[10]), "v"(y[11]), "v"(y[12]), "v"(y[13]), "v"(y[14]), "v"(y[15]));
+#undef SS2D_ADD
+#undef SS2D_ALL
+#undef SS2D_UPPER
+#undef SS2D_EVEN
+#undef SS2D_ODD
+}
+
 template <typename in_t, typename out_t, int kSpw, bool kSoftplus, bool kX, bool kMaps = false, int kPhase = kWhole>
-__global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restrict__ u_all, const in_t *__restrict__ dl_all,
+__global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void scan_chan_kernel(const in_t *__restrict__ u_all, const in_t *__restrict__ dl_all,
                                                            const in_t *__restrict__ B_all, const in_t *__restrict__ C_all,
                                                            const float *__restrict__ A_all, out_t *__restrict__ o_all,
                                                            const ScanArgs p, const ChanGeom geo,
                                                            const in_t *__restrict__ ut_all = nullptr) {
-    __shared__ __align__(16) float s_dl[kChanBlock * kChanTilePitch];
-    __shared__ __align__(16) float s_du[kChanBlock * kChanTilePitch];
-    __shared__ __align__(16) float s_y[kWavesPerWg * kChanBlock * kChanSubPitch];
-    __shared__ float s_sum[kX || kPhase == kLocal ? kWavesPerWg * kChanBlock : 1];
-    __shared__ float s_max[kPhase == kLocal ? kWavesPerWg * kChanBlock : 1];
+    constexpr int kBcRows = 2 * kChanSets * kSpw;                                       // [B, C][state of the lane][set]
+    __shared__ __align__(16) float s_dl_all[kWavesPerWg * kChanBlock * kChanTilePitch]; // later: the outputs
+    __shared__ __align__(16) float s_du_all[kWavesPerWg * kChanBlock * kChanTilePitch];
+    __shared__ __align__(16) float s_bc_all[kWavesPerWg * kBcRows * kChanSubPitch];
 
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    // neighbouring workgroups are the channel blocks of one (image, group) and read the same B / C rows: keep them
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    float *s_dl = s_dl_all + wave * kChanBlock * kChanTilePitch, *s_du = s_du_all + wave * kChanBlock * kChanTilePitch;
+    float *s_bc = s_bc_all + wave * kBcRows * kChanSubPitch;
+    // neighbouring wavefronts are the channel blocks of one (image, group) and read the same B / C rows: keep them
     // on one XCD (one L2)
-    uint32_t wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
+    uint32_t unit = xcd_contiguous_id(blockIdx.x, gridDim.x) * kWavesPerWg + wave;
+    if (unit >= geo.n_units) return;                        // whole wavefronts; no workgroup barrier in this kernel
     uint32_t bg, cb, b, grp, seg = 0;
-    if constexpr (kPhase != kWhole) divmod(wg, geo.div_segs, wg, seg);
-    divmod(wg, geo.div_cb, bg, cb);
+    if constexpr (kPhase != kWhole) divmod(unit, geo.div_segs, unit, seg);
+    divmod(unit, geo.div_cb, bg, cb);
     divmod(bg, geo.div_groups, b, grp);
     const int L = p.L, dpg = p.dim_per_group;
     const int begin = kPhase == kWhole ? 0 : (int)seg * geo.seg_len;           // (a multiple of kChanTile)
     const int stop = kPhase == kWhole || (int)seg + 1 == geo.n_segs ? L : begin + geo.seg_len;
 
-    // ---- staging / combine role: row r, quarter q -----------------------------------------------------------------
-    const int r = tid >> 2, q = tid & 3;
-    const int cs = (int)cb * kChanBlock + r;
-    const bool row_ok = cs < dpg;
-    const int ds = (int)grp * dpg + min(cs, dpg - 1);
-    const int dgs = ds / p.dim_per_delta;
-    const in_t *u_row = u_all + (int64_t)b * p.u_bs + (int64_t)ds * p.u_ds;
-    bool u_rev = false;                                     // kMaps: uniform over the workgroup (one group = one direction)
+    // ---- staging / output role: row r, quarter q -------------------------------------------------------------------
+    const int r = lane >> 2, q = lane & 3;
+    const int c_first = (int)cb * kChanBlock, n_chan = min(kChanBlock, dpg - c_first);
+    const int d_first = (int)grp * dpg + c_first, ds = d_first + min(r, n_chan - 1);
+    const int dg_first = d_first / p.dim_per_delta, dgs = ds / p.dim_per_delta;
+    const in_t *u_first = u_all + (int64_t)b * p.u_bs + (int64_t)d_first * p.u_ds;
+    bool u_rev = false;                                     // kMaps: uniform over the wavefront (one group = one direction)
     if constexpr (kMaps) {
-        const int Dm = p.dim >> 2, k = ds / Dm;
-        u_row = ((k & 1) ? ut_all : u_all) + (int64_t)b * p.u_bs + (int64_t)(ds - k * Dm) * p.u_ds;
+        const int Dm = p.dim >> 2, k = d_first / Dm;
+        u_first = ((k & 1) ? ut_all : u_all) + (int64_t)b * p.u_bs + (int64_t)(d_first - k * Dm) * p.u_ds;
         u_rev = k >= 2;
     }
+    const auto u_buf = rows_buffer(u_first, n_chan, p.u_ds, L);
+    const auto dl_buf = rows_buffer(dl_all + (int64_t)b * p.dl_bs + (int64_t)dg_first * p.dl_ds, (d_first + n_chan - 1) / p.dim_per_delta - dg_first + 1, p.dl_ds, L);
+    const auto o_buf = rows_buffer(o_all + (int64_t)b * p.o_bs + (int64_t)d_first * p.o_ds, n_chan, p.o_ds, L);
+    const uint32_t u_off = (uint32_t)((ds - d_first) * p.u_ds), dl_off = (uint32_t)((dgs - dg_first) * p.dl_ds), o_off = (uint32_t)((ds - d_first) * p.o_ds);
     // four positions of u from position pos of the scan on, as they lie in memory: backwards these are the four elements
     // that end at L - 1 - pos, and they are put in scan order where they are widened (in_scan_order) -- not here, which
     // would make the wavefront wait for a load it has just issued for the NEXT step
     auto load_u = [&](int pos) {
-        if constexpr (kMaps) {
-            if (u_rev) return load_raw4<in_t>(u_row, pos < L ? L - 4 - pos : L, L, 0.0f);
-        }
-        return load_raw4<in_t>(u_row, pos, L, 0.0f);
+        const int at = kMaps && u_rev ? L - 4 - pos : pos;
+        return load_raw4<in_t>(u_buf, pos < L ? (u_off + (uint32_t)at) * (uint32_t)sizeof(in_t) : kNowhere);
     };
+    auto load_dl = [&](int pos) { return load_raw4<in_t>(dl_buf, pos < L ? (dl_off + (uint32_t)pos) * (uint32_t)sizeof(in_t) : kNowhere); };
     auto in_scan_order = [&](const Raw4<in_t> &r) {
         if constexpr (kMaps) {
             if (u_rev) return reverse4<in_t>(r);
         }
         return r;
     };
-    const in_t *dl_row = dl_all + (int64_t)b * p.dl_bs + (int64_t)dgs * p.dl_ds;
-    out_t *o_row = o_all + (int64_t)b * p.o_bs + (int64_t)ds * p.o_ds;
     const float bias_s = p.bias ? p.bias[dgs] : 0.0f;
     const float D_s = p.D ? p.D[ds] : 0.0f;
     float *st_dl = s_dl + r * kChanTilePitch + 4 * q;
     float *st_du = s_du + r * kChanTilePitch + 4 * q;
+    // B / C: four positions of a row per lane and piece, rows [B, C][state of the lane][set]
+    constexpr int kBcPieces = kSpw > 4 ? kSpw / 4 : 1;      // of each
+    const bool bc_mine = kSpw >= 4 || lane < 16 * kSpw;
+    const auto B_buf = rows_buffer(B_all + (int64_t)b * p.B_bs + (int64_t)grp * p.B_gs, kChanSets * kSpw, p.B_ns, L);
+    const auto C_buf = rows_buffer(C_all + (int64_t)b * p.C_bs + (int64_t)grp * p.C_gs, kChanSets * kSpw, p.C_ns, L);
+    uint32_t B_off[kBcPieces], C_off[kBcPieces];
+#pragma unroll
+    for (int k = 0; k < kBcPieces; ++k) {
+        const int n = (r & 3) * kSpw + (r >> 2) + 4 * k;    // row r + 16 k of the array: state r / 4 + 4 k of set r % 4
+        B_off[k] = (uint32_t)(n * p.B_ns + 4 * q);
+        C_off[k] = (uint32_t)(n * p.C_ns + 4 * q);
+    }
+    auto load_bc = [&](int t, Raw4<in_t> (&raw)[2 * kBcPieces]) {
+        const bool ok = bc_mine && t + 4 * q < L;
+#pragma unroll
+        for (int k = 0; k < kBcPieces; ++k) {
+            raw[k] = load_raw4<in_t>(B_buf, ok ? (B_off[k] + (uint32_t)t) * (uint32_t)sizeof(in_t) : kNowhere);
+            if constexpr (kPhase != kLocal) raw[kBcPieces + k] = load_raw4<in_t>(C_buf, ok ? (C_off[k] + (uint32_t)t) * (uint32_t)sizeof(in_t) : kNowhere);
+        }
+    };
+    float *st_bc = s_bc + r * kChanSubPitch + 4 * q;
 
-    // ---- compute role: channel = lane, states wave*kSpw .. + kSpw ---------------------------------------------------
-    const int dc = (int)grp * dpg + min((int)cb * kChanBlock + lane, dpg - 1);
+    // ---- compute role: a channel, states set * kSpw .. + kSpw ------------------------------------------------
+    const int ch = (lane >> 4) * 4 + (lane & 3), set = (lane >> 2) & 3;
+    const int dc = d_first + min(ch, n_chan - 1);
     float A2[kSpw], h[kSpw];
 #pragma unroll
     for (int j = 0; j < kSpw; ++j) {
-        A2[j] = A_all[(int64_t)dc * p.A_ds + (int64_t)(wave * kSpw + j) * p.A_ns] * kLog2e;
+        A2[j] = A_all[(int64_t)dc * p.A_ds + (int64_t)(set * kSpw + j) * p.A_ns] * kLog2e;
         h[j] = 0.0f;
     }
-    const in_t *B_wave = B_all + (int64_t)b * p.B_bs + (int64_t)grp * p.B_gs + (int64_t)(wave * kSpw) * p.B_ns;
-    // (kLocal has no use for C: the same lines of B twice)
-    const in_t *C_wave = kPhase == kLocal ? B_wave : C_all + (int64_t)b * p.C_bs + (int64_t)grp * p.C_gs + (int64_t)(wave * kSpw) * p.C_ns;
-    const int64_t C_ns = kPhase == kLocal ? p.B_ns : p.C_ns;
-    const float *my_dl = s_dl + lane * kChanTilePitch, *my_du = s_du + lane * kChanTilePitch;
-    float *my_y = s_y + (wave * kChanBlock + lane) * kChanSubPitch;
-    const float *sum_y = s_y + r * kChanSubPitch + 4 * q;
-    float dl_sum = 0.0f;                                    // kX: this wavefront's quarter of the channel's sum of dl
+    const float *my_bc = s_bc + set * kChanSubPitch;
+    float *my_dl = s_dl + ch * kChanTilePitch;
+    const float *my_du = s_du + ch * kChanTilePitch;
+    float dl_sum = 0.0f;                                    // kX: this lane's quarter of the channel's sum of dl
     float dl_max = 0.0f;                                    // kLocal: its largest
-    const bool chan_ok = (int)cb * kChanBlock + lane < dpg;
-    float *x_lane = kX ? p.x + ((int64_t)b * p.dim + dc) * p.n_chunks * 2 * p.N + 2 * (wave * kSpw) : nullptr;
+    const bool chan_ok = ch < n_chan;
+    float *x_lane = kX ? p.x + ((int64_t)b * p.dim + dc) * p.n_chunks * 2 * p.N + 2 * (set * kSpw) : nullptr;
+    auto over_sets = [&](float v) { v += __shfl_xor(v, 4, kWave); return v + __shfl_xor(v, 8, kWave); };
 
     // a segment's states, its sum of dl, (from the carry kernel) that of all before it and its largest dl, where its outputs will be
     uint8_t *seg_state = reinterpret_cast<uint8_t *>(o_all + (int64_t)b * p.o_bs + (int64_t)dc * p.o_ds + begin);
     if constexpr (kPhase == kRest) {
         if (seg > 0) {
-            __builtin_memcpy(h, seg_state + sizeof(float) * (wave * kSpw), sizeof(h));
-            if (kX && wave == 0) __builtin_memcpy(&dl_sum, seg_state + sizeof(float) * (p.N + 1), sizeof(dl_sum));
+            __builtin_memcpy(h, seg_state + sizeof(float) * (set * kSpw), sizeof(h));
+            if (kX && set == 0) __builtin_memcpy(&dl_sum, seg_state + sizeof(float) * (p.N + 1), sizeof(dl_sum));
         }
     }
-
-    constexpr float kFill = delta_fill<kSoftplus>();
-    Raw4<in_t> ru[2], rd[2];
+    Raw4<in_t> ru[2], rd[2], rbc[2][2 * kBcPieces];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         ru[s] = load_u(begin + s * kChanSub + 4 * q);
-        rd[s] = load_raw4<in_t>(dl_row, begin + s * kChanSub + 4 * q, L, kFill);
+        rd[s] = load_dl(begin + s * kChanSub + 4 * q);
     }
-    // B / C of the (round, state) processed next are always one step ahead in scalar registers: requested before the
-    // arithmetic of the current state starts, they have arrived when it ends.  Rows are multiples of 8 positions, so
-    // the second half of a round lies entirely inside or entirely outside the row; outside, the first half is read
-    // again (du is 0 there, nothing of it is stored), and a round past the row's end reads the row's start.
-    UniRaw<in_t> next_bc;
-    load_uniform<in_t>(B_wave, C_wave, begin, begin + 8 < L ? begin + 8 : begin, next_bc);
+    // requested in the order in which a step does: what the compiler waits for is then a count of younger requests, not all
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) load_bc(begin + s * kChanSub, rbc[s]);
+    __builtin_amdgcn_sched_barrier(0);
 
     for (int t0 = begin; t0 < stop; t0 += kChanTile) {
-        // ---- stage: dl, du into LDS; the skip term stays with this thread for the combine ---------------------------
+        // ---- stage: dl, du into LDS; the skip term stays with this lane -----------------------------------------------
         float skip[2][4];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             float uv[4], raw[4], dl[4], du[4];
             unpack_raw4<in_t>(in_scan_order(ru[s]), uv);
             unpack_raw4<in_t>(rd[s], raw);
-            const bool in_row = t0 + s * kChanSub + 4 * q < L;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                if constexpr (kSoftplus) dl[i] = softplus_log2(fmaf(raw[i], kLog2e, bias_s * kLog2e));   // fill -inf: 0
-                else dl[i] = in_row ? raw[i] + bias_s : 0.0f;
+                dl[i] = kSoftplus ? softplus_log2(fmaf(raw[i], kLog2e, bias_s * kLog2e)) : raw[i] + bias_s;
+            }
+            if (t0 + kChanTile > L) {                       // uniform; past the row's end 0, the identity of the recurrence
+                const bool in_row = t0 + s * kChanSub + 4 * q < L;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dl[i] = in_row ? dl[i] : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
                 du[i] = dl[i] * uv[i];
                 skip[s][i] = D_s * uv[i];
             }
             *reinterpret_cast<float4 *>(st_dl + s * kChanSub) = make_float4(dl[0], dl[1], dl[2], dl[3]);
             *reinterpret_cast<float4 *>(st_du + s * kChanSub) = make_float4(du[0], du[1], du[2], du[3]);
         }
-        // the next step's inputs travel while this step computes
-        if (t0 + kChanTile < stop) {
+        // the next step's inputs travel while this step computes (after the last step of a segment: not used)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                ru[s] = load_u(t0 + kChanTile + s * kChanSub + 4 * q);
-                rd[s] = load_raw4<in_t>(dl_row, t0 + kChanTile + s * kChanSub + 4 * q, L, kFill);
-            }
+        for (int s = 0; s < 2; ++s) {
+            ru[s] = load_u(t0 + kChanTile + s * kChanSub + 4 * q);
+            rd[s] = load_dl(t0 + kChanTile + s * kChanSub + 4 * q);
         }
-        __syncthreads();                                    // dl / du of this step are in place
-
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int ps = t0 + s * kChanSub;
-            if (ps < L) {                                   // uniform over the workgroup
-                // ---- compute: 16 positions, this wavefront's states -------------------------------------------------
-                float dl[kChanSub], du[kChanSub], y[kChanSub];
+            // ---- compute: 16 positions of every lane's states -----------------------------------------------------------
+#pragma unroll
+            for (int k = 0; k < (kPhase == kLocal ? 1 : 2) * kBcPieces; ++k) {
+                float v[4];
+                unpack_raw4<in_t>(rbc[s][k], v);
+                const int at = (k / kBcPieces) * kChanSets * kSpw + (k % kBcPieces) * 16;
+                if (bc_mine) *reinterpret_cast<float4 *>(st_bc + at * kChanSubPitch) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+            load_bc(ps + kChanTile, rbc[s]);
+            __builtin_amdgcn_sched_barrier(0);
+            wave_lds_sync();                                // dl / du of this step, B / C of this round are in place
+            if (s > 0 && ps >= L) break;                    // uniform; no memory request is behind it
+            float dl[kChanSub], du[kChanSub], y[kChanSub];
+#pragma unroll
+            for (int v = 0; v < kChanSub / 4; ++v) {
+                const float4 a4 = *reinterpret_cast<const float4 *>(my_dl + s * kChanSub + 4 * v);
+                const float4 b4 = *reinterpret_cast<const float4 *>(my_du + s * kChanSub + 4 * v);
+                dl[4 * v] = a4.x; dl[4 * v + 1] = a4.y; dl[4 * v + 2] = a4.z; dl[4 * v + 3] = a4.w;
+                du[4 * v] = b4.x; du[4 * v + 1] = b4.y; du[4 * v + 2] = b4.z; du[4 * v + 3] = b4.w;
+            }
+#pragma unroll
+            for (int i = 0; i < kChanSub; ++i) y[i] = 0.0f;
+            if constexpr (kX || kPhase == kLocal) {
+                const float4 q4 = *reinterpret_cast<const float4 *>(my_dl + s * kChanSub + 4 * set);
+                dl_sum += (q4.x + q4.y) + (q4.z + q4.w);      // (dl is 0 past the row's end)
+                if constexpr (kPhase == kLocal) dl_max = fmaxf(fmaxf(dl_max, fmaxf(q4.x, q4.y)), fmaxf(q4.z, q4.w));
+            }
+#pragma unroll
+            for (int j = 0; j < kSpw; ++j) {
+                float Bv[kChanSub], Cv[kChanSub];
 #pragma unroll
                 for (int v = 0; v < kChanSub / 4; ++v) {
-                    const float4 a4 = *reinterpret_cast<const float4 *>(my_dl + s * kChanSub + 4 * v);
-                    const float4 b4 = *reinterpret_cast<const float4 *>(my_du + s * kChanSub + 4 * v);
-                    dl[4 * v] = a4.x; dl[4 * v + 1] = a4.y; dl[4 * v + 2] = a4.z; dl[4 * v + 3] = a4.w;
-                    du[4 * v] = b4.x; du[4 * v + 1] = b4.y; du[4 * v + 2] = b4.z; du[4 * v + 3] = b4.w;
+                    const float4 b4 = *reinterpret_cast<const float4 *>(my_bc + j * kChanSets * kChanSubPitch + 4 * v);
+                    const float4 c4 = *reinterpret_cast<const float4 *>(my_bc + (kSpw + j) * kChanSets * kChanSubPitch + 4 * v);
+                    Bv[4 * v] = b4.x; Bv[4 * v + 1] = b4.y; Bv[4 * v + 2] = b4.z; Bv[4 * v + 3] = b4.w;
+                    Cv[4 * v] = c4.x; Cv[4 * v + 1] = c4.y; Cv[4 * v + 2] = c4.z; Cv[4 * v + 3] = c4.w;
                 }
+                float hj = h[j];
 #pragma unroll
-                for (int i = 0; i < kChanSub; ++i) y[i] = 0.0f;
-                if constexpr (kX || kPhase == kLocal) {
-                    const float4 q4 = *reinterpret_cast<const float4 *>(my_dl + s * kChanSub + 4 * wave);
-                    dl_sum += (q4.x + q4.y) + (q4.z + q4.w);  // (dl is 0 past the row's end)
-                    if constexpr (kPhase == kLocal) dl_max = fmaxf(fmaxf(dl_max, fmaxf(q4.x, q4.y)), fmaxf(q4.z, q4.w));
+                for (int i = 0; i < kChanSub; ++i) {
+                    hj = fmaf(__builtin_amdgcn_exp2f(dl[i] * A2[j]), hj, Bv[i] * du[i]);
+                    if constexpr (kPhase != kLocal) y[i] = fmaf(Cv[i], hj, y[i]);
                 }
-                // the LDS reads above have landed before the first scalar request below is made (one wait covers both
-                // kinds of traffic, so a request issued earlier would be waited for at once)
-                asm volatile("" ::"v"(dl[0]), "v"(dl[4]), "v"(dl[8]), "v"(dl[12]), "v"(du[0]), "v"(du[4]), "v"(du[8]), "v"(du[12]));
-#pragma unroll
-                for (int j = 0; j < kSpw; ++j) {
-                    const UniRaw<in_t> cur_bc = next_bc;
-                    arrived<in_t>(cur_bc);
-                    {
-                        // what comes next: the following state of this round, or the first state of the next round
-                        const int jn = j + 1 < kSpw ? j + 1 : 0;
-                        int pn = j + 1 < kSpw ? ps : ps + kChanSub;
-                        pn = pn < L ? pn : 0;
-                        const int pn1 = pn + 8 < L ? pn + 8 : pn;
-                        load_uniform<in_t>(B_wave + (int64_t)jn * p.B_ns, C_wave + (int64_t)jn * C_ns, pn, pn1, next_bc);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);      // the requests above are issued before the arithmetic below
-                    float Bv[kChanSub], Cv[kChanSub];
-                    widen16<in_t>(cur_bc.b, Bv);
-                    widen16<in_t>(cur_bc.c, Cv);
-                    float a[kChanSub];
-#pragma unroll
-                    for (int i = 0; i < kChanSub; ++i) a[i] = __builtin_amdgcn_exp2f(dl[i] * A2[j]);
-                    float hj = h[j];
-#pragma unroll
-                    for (int i = 0; i < kChanSub; ++i) {
-                        hj = fmaf(a[i], hj, Bv[i] * du[i]);
-                        if constexpr (kPhase != kLocal) y[i] = fmaf(Cv[i], hj, y[i]);
-                    }
-                    h[j] = hj;
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (int v = 0; v < kChanSub / 4 && kPhase != kLocal; ++v)
-                    *reinterpret_cast<float4 *>(my_y + 4 * v) = make_float4(y[4 * v], y[4 * v + 1], y[4 * v + 2], y[4 * v + 3]);
+                h[j] = hj;
             }
-            if constexpr (kPhase == kLocal) {
-                if (s == 1) __syncthreads();                // dl / du read before the next step's are written
-                continue;
+            wave_lds_sync();                                // dl / du, B / C of this round are read
+            if constexpr (kPhase != kLocal) {
+                // the four sets' sums: positions 4 set .. + 4 of the lane's channel, into the place of the dl read above
+                sum_over_sets(y);
+                *reinterpret_cast<float4 *>(my_dl + s * kChanSub + 4 * set) = make_float4(y[0], y[1], y[2], y[3]);
             }
-            __syncthreads();                                // the four partial sums of this round are in place
-            if (ps < L) {
-                // ---- combine: 4 positions of row r ---------------------------------------------------------------
-                float acc[4] = {skip[s][0], skip[s][1], skip[s][2], skip[s][3]};
+        }
+        if constexpr (kPhase != kLocal) {
+            // ---- output: 4 positions of row r, twice -----------------------------------------------------------------
+            wave_lds_sync();
 #pragma unroll
-                for (int w = 0; w < kWavesPerWg; ++w) {
-                    const float4 part = *reinterpret_cast<const float4 *>(sum_y + w * kChanBlock * kChanSubPitch);
-                    acc[0] += part.x; acc[1] += part.y; acc[2] += part.z; acc[3] += part.w;
-                }
-                if (row_ok && ps + 4 * q < L) store4<out_t>(o_row + ps + 4 * q, acc);
+            for (int s = 0; s < 2; ++s) {
+                const float4 part = *reinterpret_cast<const float4 *>(st_dl + s * kChanSub);
+                const float acc[4] = {skip[s][0] + part.x, skip[s][1] + part.y, skip[s][2] + part.z, skip[s][3] + part.w};
+                const int pos = t0 + s * kChanSub + 4 * q;
+                store4<out_t>(o_buf, r < n_chan && pos < L ? (o_off + (uint32_t)pos) * (uint32_t)sizeof(out_t) : kNowhere, acc);
             }
-            if (s == 0) __syncthreads();                    // partials read before the next round overwrites them
-            // (after the second round the barrier at the top of the next step does this: its staging writes touch
-            //  dl / du only, which every wavefront has finished reading by then)
+            wave_lds_sync();
         }
         if constexpr (kX) {
             const int t_end = t0 + kChanTile;
-            if (t_end % SS2D_SCAN_CHUNK == 0 || t_end >= L) {   // uniform over the workgroup; at least 64 steps apart
-                s_sum[wave * kChanBlock + lane] = dl_sum;
-                __syncthreads();
-                const float total = (s_sum[lane] + s_sum[kChanBlock + lane]) + (s_sum[2 * kChanBlock + lane] + s_sum[3 * kChanBlock + lane]);
+            if (t_end % SS2D_SCAN_CHUNK == 0 || t_end >= L) {   // uniform; at least 64 steps apart
+                const float total = over_sets(dl_sum);
                 if (chan_ok) {
                     float *xo = x_lane + (int64_t)((min(t_end, L) - 1) / SS2D_SCAN_CHUNK) * 2 * p.N;
 #pragma unroll
@@ -383,14 +378,11 @@ __global__ __launch_bounds__(kBlock) void scan_chan_kernel(const in_t *__restric
         }
     }
     if constexpr (kPhase == kLocal) {
-        s_sum[wave * kChanBlock + lane] = dl_sum;
-        s_max[wave * kChanBlock + lane] = dl_max;
-        __syncthreads();
+        const float total = over_sets(dl_sum);
+        const float pair = fmaxf(dl_max, __shfl_xor(dl_max, 4, kWave)), most = fmaxf(pair, __shfl_xor(pair, 8, kWave));
         if (!chan_ok) return;
-        __builtin_memcpy(seg_state + sizeof(float) * (wave * kSpw), h, sizeof(h));
-        if (wave == 0) {
-            const float total = (s_sum[lane] + s_sum[kChanBlock + lane]) + (s_sum[2 * kChanBlock + lane] + s_sum[3 * kChanBlock + lane]);
-            const float most = fmaxf(fmaxf(s_max[lane], s_max[kChanBlock + lane]), fmaxf(s_max[2 * kChanBlock + lane], s_max[3 * kChanBlock + lane]));
+        __builtin_memcpy(seg_state + sizeof(float) * (set * kSpw), h, sizeof(h));
+        if (set == 0) {
             __builtin_memcpy(seg_state + sizeof(float) * p.N, &total, sizeof(total));
             __builtin_memcpy(seg_state + sizeof(float) * (p.N + 2), &most, sizeof(most));
         }
@@ -439,27 +431,32 @@ __global__ __launch_bounds__(kBlock) void scan_chan_carry_kernel(const float *__
 }
 
 bool scan_chan_eligible(const ScanArgs &a) {
-    // N/4 states per wavefront; rows in whole 8-position vectors; at least half a wavefront of channels per group
+    // N/4 states per lane; rows in whole 8-position vectors; at least two blocks of channels per group; a block's rows within 32-bit
+    // byte offsets
+    for (int64_t s : {a.u_ds, a.dl_ds, a.o_ds})
+        if (s < 0 || (kChanBlock - 1) * s + a.L > kNowhere / 2 / 4) return false;
+    for (int64_t s : {a.B_ns, a.C_ns})
+        if (s < 0 || (a.N - 1) * s + a.L > kNowhere / 2 / 4) return false;
     return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.L % 8 == 0 && a.dim_per_group >= 32;
 }
 
 // The number of segments of a row (1: not cut) and the length of all but the last, which has at least 72 positions: a segment's N + 3
 // floats (the last one's N + 2) lie where its outputs will be.
 //
-// A workgroup takes 1.7 us per 16 positions of 16 states however few there are (1.0 of 4 states, 2.7 of 32).  Cut rows run the recurrence
-// twice (the first time without C), in three launches, and are ahead where the segments find room beside one another: three
-// workgroups per CU, segments of 128 positions or more.  us, whole / cut, workgroups of whole rows in front: 16 states in bf16, 4: 16 384
-// positions 1699 / 58; 8: 3136 331 / 42; 12: 784 86 / 39, 400 46 / 38; 48: 784 87 / 39, 400 47 / 38; 96: 784 89 / 51, 512 59 / 43; 192: 3136 388 / 265; in fp32, 8: 3136
-// 310 / 39; 96: 784 83 / 53; 4 states, 8: 3136 173 / 28; 48: 400 25.2 / 23.8; 32 states in fp16, 8: 3136 528 / 63; 48: 400 72 / 58.  Left whole: few segments
-// of many workgroups, 192: 784 positions 89 / 83 in bf16, 86 / 90 in fp32, 138 / 156 of 32 states; 96: 400 47 / 44, 43.5 / 43.6, 72 / 74.
-constexpr int64_t kSegPlaces = 768, kSegLeast = 128;
+// A wavefront takes 1.3 us per 16 positions of 16 states while it has its SIMD to itself (0.65 of 4 states, 2.1 of 32).  Cut rows run the
+// recurrence twice (the first time without C), in three launches, and are ahead while there are not nearly as many wavefronts as SIMDs (1024).
+// us, whole / cut, wavefronts of whole rows in front: 16 states in bf16, 16: 3136 positions 249 / 34, 784 65 / 28, 400 35 / 27; 192: 3136 251 / 78,
+// 784 66 / 33, 400 35 / 31; 384: 3136 243 / 133, 784 66 / 48, 400 (three segments) 36 / 38; 768: 3136 246 / 245, 784 66 / 72; in fp32, 384: 3136 231 / 139; 4 states,
+// 16: 400 18.2 / 17.0; 384: 784 35 / 28, 400 19 / 21; 768: 1568 63 / 68; 32 states in fp16, 384: 784 108 / 74; 768: 784 107 / 115.  More segments than
+// kSegPlaces are no faster (384: 3136 positions in 12: 140, in 24: 137), nor are shorter ones than kSegLeast where many run (192: 784 in 6: 33, in 8: 35).
+constexpr int64_t kSegPlaces = 4608, kSegUnits = 576, kSegLeast = 128;
 
-static int64_t chan_segments(const ScanArgs &a, int64_t n_wg, int32_t &seg_len) {
-    if (a.out == a.u || a.out == a.delta || (int64_t)a.batch * a.dim * a.N > 0x7fffffff) return 1;
-    const int64_t fewest = n_wg <= 64 ? 3 : n_wg <= 128 || a.L >= 2048 ? 4 : kSegPlaces;
-    int64_t n = kSegPlaces / n_wg;
-    if (n > a.L / kSegLeast) n = a.L / kSegLeast;
-    if (n < fewest) return 1;
+static int64_t chan_segments(const ScanArgs &a, int64_t n_units, int32_t &seg_len) {
+    if (a.out == a.u || a.out == a.delta || (int64_t)a.batch * a.dim * a.N > 0x7fffffff || n_units > kSegUnits) return 1;
+    const int64_t least = n_units <= 64 ? 96 : kSegLeast;
+    int64_t n = kSegPlaces / n_units;
+    if (n > a.L / least) n = a.L / least;
+    if (n < (n_units <= 192 ? 3 : 4)) return 1;
     const int64_t len = ((a.L + n - 1) / n + kChanTile - 1) / kChanTile * kChanTile;
     n = (a.L + len - 1) / len;
     if (a.L - (n - 1) * len < 72) --n;
@@ -474,10 +471,12 @@ static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stre
     const int groups = a.dim / a.dim_per_group;
     geo.div_cb = make_fastdiv((uint32_t)geo.n_cb);
     geo.div_groups = make_fastdiv((uint32_t)groups);
-    const int64_t n_wg = (int64_t)a.batch * groups * geo.n_cb;
-    if (n_wg > 0x7fffffff) return SS2D_ENOTSUP;
+    const int64_t n_rows = (int64_t)a.batch * groups * geo.n_cb;
+    if (n_rows > 0x7fffffff) return SS2D_ENOTSUP;
+    geo.n_units = (uint32_t)n_rows;
+    auto n_wg = [&] { return dim3((geo.n_units + kWavesPerWg - 1) / kWavesPerWg); };
 #define SS2D_LAUNCH_CHAN(SPW, SP, X, M)                                                                                    \
-    hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, SP, X, M>), dim3((uint32_t)n_wg), dim3(kBlock), 0, stream,       \
+    hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, SP, X, M>), n_wg(), dim3(kBlock), 0, stream,       \
                        (const in_t *)a.u, (const in_t *)a.delta, (const in_t *)a.B, (const in_t *)a.C, a.A, (out_t *)a.out, a, geo, \
                        (const in_t *)xt)
 #define SS2D_LAUNCH_CHAN_N(SP, X, M)                            \
@@ -492,12 +491,14 @@ static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stre
 #define SS2D_LAUNCH_CHAN_SPLIT(SPW, X, M)                                                                                   \
     do {                                                                                                                   \
         geo.div_segs = make_fastdiv((uint32_t)segs - 1);                                                                    \
-        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, false, M, kLocal>), dim3((uint32_t)(n_wg * (segs - 1))), dim3(kBlock), 0, stream, \
+        geo.n_units = (uint32_t)(n_rows * (segs - 1));                                                                      \
+        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, false, M, kLocal>), n_wg(), dim3(kBlock), 0, stream, \
                            (const in_t *)a.u, (const in_t *)a.delta, (const in_t *)a.B, (const in_t *)a.C, a.A, (out_t *)a.out, a, geo, (const in_t *)xt); \
         hipLaunchKernelGGL((scan_chan_carry_kernel<out_t>), dim3((n_items + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, a.A, (out_t *)a.out, a, \
                            geo.seg_len, geo.n_segs, n_items, make_fastdiv((uint32_t)a.N), make_fastdiv((uint32_t)a.dim));   \
         geo.div_segs = make_fastdiv((uint32_t)segs);                                                                        \
-        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, X, M, kRest>), dim3((uint32_t)(n_wg * segs)), dim3(kBlock), 0, stream, \
+        geo.n_units = (uint32_t)(n_rows * segs);                                                                            \
+        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, X, M, kRest>), n_wg(), dim3(kBlock), 0, stream, \
                            (const in_t *)a.u, (const in_t *)a.delta, (const in_t *)a.B, (const in_t *)a.C, a.A, (out_t *)a.out, a, geo, (const in_t *)xt); \
     } while (0)
 #define SS2D_LAUNCH_CHAN_SPLIT_N(X, M)                          \
@@ -507,7 +508,7 @@ static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stre
         case 16: SS2D_LAUNCH_CHAN_SPLIT(4, X, M); break;        \
         default: SS2D_LAUNCH_CHAN_SPLIT(8, X, M); break;        \
     }
-    const int64_t segs = a.softplus ? chan_segments(a, n_wg, geo.seg_len) : 1;
+    const int64_t segs = a.softplus ? chan_segments(a, n_rows, geo.seg_len) : 1;
     if (segs > 1) {
         geo.n_segs = (int32_t)segs;
         const uint32_t n_items = (uint32_t)((int64_t)a.batch * a.dim * a.N);
