@@ -109,6 +109,66 @@ def test_scan_bwd_16bit_row_lengths(N, L, dtype, dout_float):
     compare(got, want, 3e-2, "16-bit")
 
 
+# A channel per lane (scan_bwd_chan.hip): rows of one segment (up to 72 positions, many of them), of two, and of many; the last chunk of 8 positions with
+# 1, 3, 7 and 8 of them; 16, 33, 50 and 51 channels per group (1 and 2 in the last wavefront, idle wavefronts); 4, 8 and 16 states; delta rows
+# shared; rows off the dword grid.  Bound in single precision: sums of up to 1030 terms and 51 channels, each term good to a few 2^-23 -- 1e-4 of the largest gradient.
+CHANNEL_CASES = [
+    (64, 64, 1, 16, 72, None, True), (64, 64, 1, 16, 73, None, True), (64, 66, 2, 8, 33, None, True), (64, 64, 1, 8, 7, None, False), (128, 64, 1, 4, 57, None, True),
+    (64, 64, 1, 16, 128, None, True), (1, 96, 2, 16, 512, None, True), (1, 50, 1, 8, 515, 10, True), (1, 16, 1, 4, 1030, None, True), (2, 51, 1, 16, 779, 17, True),
+    (1, 33, 1, 16, 600, None, False), (1, 80, 1, 16, 1000, None, True),
+]
+
+
+@pytest.mark.parametrize("case", CHANNEL_CASES, ids=lambda c: "x".join(str(v) for v in c))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_bwd_channel_per_lane(case, dtype):
+    batch, dim, G, N, L, delta_dim, softplus = case
+    print("CASE scan-bwd-chan", case, dtype, flush=True)
+    u, delta, A, B, C, D, bias, dout = make(sum(map(int, case[:5])), batch, dim, G, N, L, dtype, delta_dim, softplus)
+    dout = dout.to(dtype) if L % 3 == 0 else dout
+    want = torch_ref.selective_scan_grads(u.float(), delta.float(), A, B.float(), C.float(), D, bias, dout.float(), softplus)
+    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, softplus, 1)
+    compare(got, want, 1e-4 if dtype == torch.float32 else 3e-2, "channel per lane")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_scan_bwd_channel_per_lane_strided_views(dtype):
+    """Rows at odd distances and from odd elements on, B and C views of one projection: the bits of the contiguous call, but for the atomics' order."""
+    print("CASE scan-bwd-chan-views", dtype, flush=True)
+    batch, dim, N, L = 2, 50, 16, 600
+    u, delta, A, B, C, D, bias, dout = [t.to(DEV) for t in make(3, batch, dim, 1, N, L, dtype)]
+    want = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
+
+    def view(t, pitch):
+        rows = t.reshape(-1, t.shape[-1])
+        store = torch.full((rows.shape[0] * pitch + 1,), float("nan"), device=DEV, dtype=t.dtype)
+        out = store[1:].view(rows.shape[0], pitch)[:, :L]
+        out.copy_(rows)
+        return out.unflatten(0, t.shape[:-1])
+
+    proj = torch.cat([B, C], 2).contiguous()
+    args = (view(u, L + 5), view(delta, L + 1), A, proj[:, :, :N], view(C, L + 3), D, bias, view(dout, L + 7))
+    got = va.selective_scan_bwd(*args, None, True, 1)
+    for name, g, w in zip(NAMES, got, want):
+        if name in ("du", "ddelta"):
+            assert torch.equal(g, w), name
+        else:
+            assert torch.allclose(g.float(), w.float(), rtol=1e-2 if dtype == torch.bfloat16 else 1e-5, atol=1e-5 * w.float().abs().max().item()), name
+
+
+def test_scan_bwd_channel_per_lane_keeps_channels_apart():
+    """A NaN of one channel reaches that channel's rows and the sums over channels, not the other channels' rows: lanes without a channel, which read the
+    last one's constants, included."""
+    batch, dim, N, L = 1, 50, 16, 600
+    u, delta, A, B, C, D, bias, dout = [t.to(DEV) for t in make(4, batch, dim, 1, N, L, torch.float32)]
+    want = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
+    u[0, 49, 300] = float("nan")
+    got = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
+    for i in (0, 1):
+        assert torch.equal(got[i][:, :49], want[i][:, :49])
+    assert bool(got[1][0, 49, :301].isnan().any()) and bool(got[2][:49].isfinite().all())
+
+
 def test_selective_scan_fn_trains():
     """autograd through selective_scan_fn (csms6s.py:112-126): gradients reach every input."""
     print("CASE scan-autograd", flush=True)

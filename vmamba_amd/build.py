@@ -17,7 +17,7 @@ CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libss2d_hip.so")
 HIP_SOURCES = ["cross_scan.hip", "cross_merge.hip", "selective_scan.hip", "scan_chan.hip", "scan_small.hip", "layer_norm.hip", "layer_norm_bwd.hip", "dwconv.hip", "dwconv_bwd.hip",
                "ss2d_core.hip", "ss2d_core_small.hip", "ss2d_core_tiled.hip", "core_pads.hip", "core_few.hip", "forward_core.hip", "vss_block.hip", "x_proj.hip", "dt_proj.hip", "proj_f32.hip", "cross_flex.hip",
-               "selective_scan_bwd.hip", "scan_bwd_io.hip", "mlp_fused.hip", "linear_cl.hip", "linear_rows.hip", "linear_tiles.hip", "linear_dw.hip", "product_f32.hip", "stem_conv.hip", "stem_conv2.hip", "mean_pool.hip"]
+               "selective_scan_bwd.hip", "scan_bwd_chan.hip", "scan_bwd_io.hip", "mlp_fused.hip", "linear_cl.hip", "linear_rows.hip", "linear_tiles.hip", "linear_dw.hip", "product_f32.hip", "stem_conv.hip", "stem_conv2.hip", "mean_pool.hip"]
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 

@@ -33,6 +33,20 @@ bool scan_chan_eligible(const ScanArgs &a);
 // xt != nullptr: a.u is the map x (batch, dim / 4, L) and xt its transpose, read through CrossScan's routes (group = direction)
 int launch_scan_chan(const ScanArgs &a, int in_dtype, int out_dtype, hipStream_t stream, const void *xt = nullptr);
 
+struct ScanBwdArgs {
+    const void *u, *delta, *B, *C, *dout;
+    const float *A, *D, *bias;
+    void *du, *ddelta;
+    float *dA, *dB, *dC, *dD, *dbias;
+    int32_t batch, dim, L, N, dim_per_group, dim_per_delta, softplus, vec_ok, rows, n_pass;
+    int64_t u_bs, u_ds, dl_bs, dl_ds, A_ds, A_ns, B_bs, B_gs, B_ns, C_bs, C_gs, C_ns, do_bs, do_ds;
+    int64_t g_bs, g_gs, g_ns;      // strides of dB / dC (contiguous (batch, groups, N, L))
+};
+
+// scan_bwd_chan.hip: the backward with a channel per lane.  SS2D_ENOTSUP: nothing launched.
+bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size);
+int launch_scan_bwd_chan(const ScanBwdArgs &a, int in_dtype, int dout_dtype, hipStream_t stream);
+
 // Arguments of the fused core kernels (ss2d_core.hip, ss2d_core_small.hip): the C ABI's ss2d_core_params with derived
 // fields.  Strides in elements.
 struct CoreArgs {
@@ -281,6 +295,12 @@ __device__ __forceinline__ float softplus_log2(float z) {
 __device__ __forceinline__ float softplus_over_ln2(float z) {
     const float t = __builtin_amdgcn_exp2f(-__builtin_fabsf(z));
     return __builtin_fmaxf(z, 0.0f) + __builtin_amdgcn_logf(1.0f + t);
+}
+
+// d softplus / dz at z = raw + bias
+__device__ __forceinline__ float bwd_sigmoid(float raw, float bias) {
+    const float t = __builtin_amdgcn_exp2f(-fmaf(raw, kLog2e, bias * kLog2e));
+    return __builtin_amdgcn_rcpf(1.0f + t);
 }
 
 template <bool kSoftplus>

@@ -24,22 +24,13 @@
 //   * scan_bwd_one_kernel     one state: a wavefront owns channels, the four wavefronts' sums meet in LDS once per pass;
 //   * scan_bwd_states_kernel  2 .. 32 states: a wavefront owns four STATES and walks every channel of the workgroup, the
 //                             wavefronts' S and T meet in LDS once per channel and pass;
+//   * scan_bwd_chan.hip       4, 8 or 16 states and rows enough, or long ones: a lane is a channel and a quarter of its states;
 //   * scan_bwd_kernel         more states: a wavefront per row, atomics per channel.
 #include <type_traits>
 
 #include "scan_common.h"
 
 namespace ss2d {
-
-struct ScanBwdArgs {
-    const void *u, *delta, *B, *C, *dout;
-    const float *A, *D, *bias;
-    void *du, *ddelta;
-    float *dA, *dB, *dC, *dD, *dbias;
-    int32_t batch, dim, L, N, dim_per_group, dim_per_delta, softplus, vec_ok, rows, n_pass;
-    int64_t u_bs, u_ds, dl_bs, dl_ds, A_ds, A_ns, B_bs, B_gs, B_ns, C_bs, C_gs, C_ns, do_bs, do_ds;
-    int64_t g_bs, g_gs, g_ns;      // strides of dB / dC (contiguous (batch, groups, N, L))
-};
 
 __device__ __forceinline__ float lane_reverse(float v, int lane) { return __shfl(v, kWave - 1 - lane, kWave); }
 
@@ -335,12 +326,6 @@ __device__ __forceinline__ void bwd_step(const RawN<in_t, kI> &raw, float bias, 
     }
 }
 
-// d softplus / dz at z = raw + bias
-template <typename in_t> __device__ __forceinline__ float bwd_sigmoid(float raw, float bias) {
-    const float t = __builtin_amdgcn_exp2f(-fmaf(raw, kLog2e, bias * kLog2e));
-    return __builtin_amdgcn_rcpf(1.0f + t);
-}
-
 // The rows and constants of channel d of image b; kN states from n_first on, of which ns exist.
 template <typename in_t, typename dy_t, int kN> struct BwdRows {
     __amdgpu_buffer_rsrc_t u, dl, dy, du, dd;
@@ -512,7 +497,7 @@ __global__ __launch_bounds__(kBlock, 3) void scan_bwd_one_kernel(const ScanBwdAr
             }
             if (softplus) {
 #pragma unroll
-                for (int i = 0; i < kI; ++i) dd[i] *= bwd_sigmoid<in_t>(raw[i], rn.bias);
+                for (int i = 0; i < kI; ++i) dd[i] *= bwd_sigmoid(raw[i], rn.bias);
             }
 #pragma unroll
             for (int i = 0; i < kI; ++i) db_acc += dd[i];
@@ -788,7 +773,7 @@ __global__ __launch_bounds__(512, 2) void scan_bwd_states_kernel(const ScanBwdAr
                     }
                     if (softplus) {
 #pragma unroll
-                        for (int j = 0; j < kG; ++j) dd[j] *= bwd_sigmoid<in_t>(raw[q * kG + j], rn.bias);
+                        for (int j = 0; j < kG; ++j) dd[j] *= bwd_sigmoid(raw[q * kG + j], rn.bias);
                     }
 #pragma unroll
                     for (int j = 0; j < kG; ++j) db_acc += dd[j];
@@ -878,6 +863,11 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
             if (st % in_vec != 0) return false;
         return a.do_bs % dy_vec == 0 && a.do_ds % dy_vec == 0;
     };
+    // several states and enough channels per group: one channel per lane
+    if (scan_bwd_chan_takes(a, in_size, dy_size)) {
+        const int rc = launch_scan_bwd_chan(a, q->in_dtype, q->dout_dtype, s);
+        if (rc != SS2D_ENOTSUP) return rc;                  // (before any launch)
+    }
     if (a.N <= 8 * kStates && (int64_t)a.L * 4 < 0x7fffffff) {
         const bool one = a.N == 1;
         // Positions per lane (measured with the others, us): 8 where rows are long, as the wavefront scans are paid per pass
