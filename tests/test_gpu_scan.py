@@ -207,6 +207,41 @@ def test_scan_blocks_of_channels(batch, dim, G, N, L, dtype):
     assert torch.equal(run_gpu(*args, True, True, want_x=False)[0], got)
 
 
+# Rows of no whole 16-byte pieces in the same kernel: a row shorter than a group of four, one that ends 1, 2 and 3 positions into a group, rows on odd
+# elements, cut rows, 4 to 32 states; what the rule leaves to the other kernels beside it.
+ODD_ROWS = [(2, 64, 2, 16, 3, "chan"), (1, 33, 1, 16, 9, "chan"), (2, 47, 1, 8, 49, "chan"), (1, 40, 1, 32, 62, "chan"), (2, 96, 2, 16, 225, "chan"),
+            (1, 48, 1, 16, 1003, "chan"), (3, 35, 1, 4, 331, "chan"), (1, 48, 1, 16, 3306, "chan"), (1, 64, 1, 4, 225, "row"), (1, 64, 1, 4, 3307, "row4")]
+
+
+@pytest.mark.parametrize("batch,dim,G,N,L,kernel", ODD_ROWS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_odd_rows_channel_per_lane(batch, dim, G, N, L, kernel, dtype):
+    _announce("scan-odd-rows", batch, dim, G, N, L, dtype)
+    args = make_inputs(37, batch, dim, G, N, L, dtype, ss2d_like=True)
+    assert kernel_of(*args[:5], want_x=False) == kernel
+    want, xw = orc.selective_scan(*args, True, out_float=True, return_x=True)
+    got, x = run_gpu(*args, True, True, want_x=True)
+    assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
+    check_states(x, xw, TOL32)
+    if dtype != torch.float32 and kernel == "chan":
+        assert torch.equal(run_gpu(*args, True, False, want_x=False)[0], got.to(dtype))
+
+
+@pytest.mark.parametrize("batch,Dm,H,W,N", [(2, 32, 7, 9, 16), (1, 48, 5, 5, 16), (3, 33, 3, 1, 16), (1, 64, 15, 19, 8), (1, 48, 57, 58, 16), (2, 40, 6, 6, 32)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_reading_odd_maps_through_the_cross_scan_routes(batch, Dm, H, W, N, dtype):
+    """The bits of CrossScan and the scan behind it, for maps whose rows end inside a group of four positions, forwards and backwards."""
+    from vmamba_amd.csms6s import selective_scan_from_map
+    _announce("scan-odd-maps", batch, Dm, H, W, N, dtype)
+    L = H * W
+    _, delta, A, B, C, D, bias = [t.to("cuda") for t in make_inputs(38, batch, 4 * Dm, 4, N, L, dtype, ss2d_like=True)]
+    x = torch.randn(batch, Dm, H, W, generator=torch.Generator().manual_seed(39)).to("cuda", dtype)
+    xs = va.cross_scan_fn(x).view(batch, 4 * Dm, L)
+    assert kernel_of(xs, delta, A, B, C, want_x=False) == "chan"
+    want = va.selective_scan_fwd(xs, delta, A, B, C, D, bias, True, 1, True, want_x=False)[0]
+    assert torch.equal(selective_scan_from_map(x, delta, A, B, C, D, bias), want)
+
+
 def test_scan_segments_hold_what_a_whole_row_does():
     """A state of 0 enters a segment whose decays multiply to infinity, as it would position by position; NaN and infinity go on
     through the segments behind them and stay out of the ones before."""

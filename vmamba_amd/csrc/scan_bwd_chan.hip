@@ -27,56 +27,11 @@ constexpr int kBcSub = 8;                         // positions per chunk
 constexpr int kBcPitch = kBcSub + 4;              // floats of an LDS row of a chunk; 16-byte pieces, 8 rows over all banks
 constexpr int kBcChunks = 9;                      // chunks per segment at most
 constexpr int kBcSeg = kBcChunks * kBcSub;
-constexpr uint32_t kNowhere = 0xfffffff0u;        // a byte offset past the end of every buffer: loads 0, stores nothing
 
 struct BwdChanGeom {
     int32_t n_cb, n_segs, seg_len;                // blocks of 64 channels per group; segments per row, all but the last of seg_len positions
     FastDiv div_cb, div_groups, div_segs;
 };
-
-// Rows in a buffer whose base is rounded down to a dword: kI elements from `pos` of the row at element `row` (counted from that base)
-// as whole dwords; what lies past the buffer's last dword, or past the row's end as a whole, is 0, and the callers mask a group that
-// straddles the row's end.  kDwords: rows start on dwords (always so in single precision); otherwise a dword more is loaded and the
-// elements, if they start in the upper half of one, are shifted down.
-template <int kN> __device__ __forceinline__ void load_dwords(__amdgpu_buffer_rsrc_t buf, uint32_t off, uint32_t (&w)[kN]) {
-    if constexpr (kN == 1) {
-        w[0] = __builtin_amdgcn_raw_buffer_load_b32(buf, (int)off, 0, 0);
-    } else if constexpr (kN == 2) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(buf, (int)off, 0, 0);
-        w[0] = v[0]; w[1] = v[1];
-    } else if constexpr (kN == 3) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b96(buf, (int)off, 0, 0);
-        w[0] = v[0]; w[1] = v[1]; w[2] = v[2];
-    } else {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(buf, (int)off, 0, 0);
-        w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
-    }
-}
-
-template <typename T, int kI, bool kDwords> struct RawGroup { uint32_t w[kI * (int)sizeof(T) / 4 + (kDwords ? 0 : 1)]; };
-
-template <typename T, int kI, bool kDwords>
-__device__ __forceinline__ RawGroup<T, kI, kDwords> load_at(__amdgpu_buffer_rsrc_t buf, uint32_t row, int pos, int L, bool ok = true) {
-    RawGroup<T, kI, kDwords> r;
-    const uint32_t off = (row + (uint32_t)pos) * (uint32_t)sizeof(T);
-    load_dwords(buf, ok && pos < L ? (kDwords ? off : off & ~3u) : kNowhere, r.w);
-    return r;
-}
-
-// the elements of a group (of a row at element `row`) as fp32; pos is a multiple of 2
-template <typename T, int kI, bool kDwords> __device__ __forceinline__ void widen(const RawGroup<T, kI, kDwords> &r, uint32_t row, float (&v)[kI]) {
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int i = 0; i < kI; ++i) v[i] = bits_to_f32(r.w[i]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < kI / 2; ++i) {
-            const uint32_t w = kDwords ? r.w[i] : __builtin_amdgcn_alignbit(r.w[i + (kDwords ? 0 : 1)], r.w[i], (row & 1) * 16);
-            v[2 * i] = unpack_lo<T>(w);
-            v[2 * i + 1] = unpack_hi<T>(w);
-        }
-    }
-}
 
 // Two elements from an even `pos` of a row that a plain (not rounded) base and element `row` give.
 template <typename T, bool kDwords>
@@ -98,21 +53,6 @@ __device__ __forceinline__ void store2_at(__amdgpu_buffer_rsrc_t buf, uint32_t r
         __builtin_amdgcn_raw_buffer_store_b32(f32_to_bits(v0), buf, off0, 0, 0);
         __builtin_amdgcn_raw_buffer_store_b32(f32_to_bits(v1), buf, off1, 0, 0);
     }
-}
-
-// `rows` rows of L elements, `stride` apart, from element `first` on
-template <typename T>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_of(const void *base, int64_t first, int rows, int64_t stride, int L) {
-    T *at = const_cast<T *>(reinterpret_cast<const T *>(base)) + first;
-    return __builtin_amdgcn_make_buffer_rsrc(at, 0, (int)(((rows - 1) * stride + L) * (int)sizeof(T)), kBufferRsrcWord3);
-}
-// ... for loads: whole dwords, the first element at `skew` (0 or 1) of the buffer
-template <typename T>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t dwords_of(const void *base, int64_t first, int rows, int64_t stride, int L, uint32_t &skew) {
-    const uintptr_t at = reinterpret_cast<uintptr_t>(reinterpret_cast<const T *>(base) + first);
-    skew = (uint32_t)(at & 3) / (uint32_t)sizeof(T);
-    const uint32_t bytes = (uint32_t)(((rows - 1) * stride + L) * (int)sizeof(T)) + (uint32_t)(at & 3);
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(at & ~(uintptr_t)3), 0, (int)((bytes + 3) & ~3u), kBufferRsrcWord3);
 }
 
 // v[i] summed over the 16 channels (lane / 4) for every i of 16, entry 8 (lane bit 3) + 4 (bit 2) + 2 (bit 5) + (bit 4) left with each

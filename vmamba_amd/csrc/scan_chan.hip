@@ -34,54 +34,28 @@ constexpr int kChanSubPitch = kChanSub + 4;
 constexpr int kChanBlock = 16;                    // channels per wavefront
 constexpr int kChanSets = 4;                      // lanes per channel, each with a quarter of the states
 
-// Four consecutive elements of a row as loaded (8 bytes of 16-bit values or 16 bytes of fp32).
-template <typename in_t> struct Raw4 { uint32_t w[sizeof(in_t)]; };
-
-// From byte offset `off` of a buffer whose end the hardware checks: past it (kNowhere) the elements are 0.  No branch: the
-// wait for a load behind one would be at its end, not where the elements are used.
-constexpr uint32_t kNowhere = 0xfffffff0u;
-
-template <typename in_t>
-__device__ __forceinline__ Raw4<in_t> load_raw4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off) {
-    Raw4<in_t> r;
-    if constexpr (sizeof(in_t) == 2) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)off, 0, 0);
-        r.w[0] = v[0]; r.w[1] = v[1];
-    } else {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0);
-        r.w[0] = v[0]; r.w[1] = v[1]; r.w[2] = v[2]; r.w[3] = v[3];
-    }
-    return r;
-}
-
-template <typename in_t>
-__device__ __forceinline__ void unpack_raw4(const Raw4<in_t> &r, float (&v)[4]) {
-    if constexpr (sizeof(in_t) == 2) {
-        v[0] = to_f32(in_t{(uint16_t)(r.w[0] & 0xffffu)}); v[1] = to_f32(in_t{(uint16_t)(r.w[0] >> 16)});
-        v[2] = to_f32(in_t{(uint16_t)(r.w[1] & 0xffffu)}); v[3] = to_f32(in_t{(uint16_t)(r.w[1] >> 16)});
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = bits_to_f32(r.w[i]);
-    }
-}
-
-template <typename out_t>
-__device__ __forceinline__ void store4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, const float (&v)[4]) {
+// Four elements from byte offset `off` on (a dword's, kDwords), the first n of them where not all lie inside the row.
+template <typename out_t, bool kDwords>
+__device__ __forceinline__ void store4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, bool whole, int n, const float (&v)[4]) {
     typedef uint32_t words4_t __attribute__((ext_vector_type(4)));
     typedef uint32_t words2_t __attribute__((ext_vector_type(2)));
-    if constexpr (sizeof(out_t) == 4) {
-        const words4_t w = {f32_to_bits(v[0]), f32_to_bits(v[1]), f32_to_bits(v[2]), f32_to_bits(v[3])};
-        __builtin_amdgcn_raw_buffer_store_b128(w, rsrc, (int)off, 0, 0);
+    if (whole && (kDwords || sizeof(out_t) == 4)) {
+        const int at = (int)(n > 0 ? off : kNowhere);
+        if constexpr (sizeof(out_t) == 4) {
+            const words4_t w = {f32_to_bits(v[0]), f32_to_bits(v[1]), f32_to_bits(v[2]), f32_to_bits(v[3])};
+            __builtin_amdgcn_raw_buffer_store_b128(w, rsrc, at, 0, 0);
+        } else {
+            const words2_t w = {pack2_from_f32<out_t>(v[0], v[1]), pack2_from_f32<out_t>(v[2], v[3])};
+            __builtin_amdgcn_raw_buffer_store_b64(w, rsrc, at, 0, 0);
+        }
     } else {
-        const words2_t w = {pack2_from_f32<out_t>(v[0], v[1]), pack2_from_f32<out_t>(v[2], v[3])};
-        __builtin_amdgcn_raw_buffer_store_b64(w, rsrc, (int)off, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int at = (int)(i < n ? off + i * (uint32_t)sizeof(out_t) : kNowhere);
+            if constexpr (sizeof(out_t) == 4) __builtin_amdgcn_raw_buffer_store_b32(f32_to_bits(v[i]), rsrc, at, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(pack2_from_f32<out_t>(v[i & ~1], v[i | 1]) >> (i & 1) * 16), rsrc, at, 0, 0);
+        }
     }
-}
-
-// `rows` rows of L elements, `stride` apart
-template <typename T>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const T *first, int rows, int64_t stride, int L) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(first), 0, (int)(((rows - 1) * stride + L) * (int)sizeof(T)), kBufferRsrcWord3);
 }
 
 struct ChanGeom {
@@ -103,20 +77,10 @@ enum ChanPhase { kWhole, kLocal, kRest };
 // kMaps: CrossScan folded in.  u is not the (batch, 4 D, L) tensor of the four scan-ordered copies but the map itself,
 // x (batch, D, L), plus its transpose xt (batch, D, L: every H x W map stored as W x H): direction k = the channel's
 // group reads x (k = 0, 2) or xt (k = 1, 3), forwards (k < 2) or backwards -- position t of the scan is element t or
-// L - 1 - t of that row (cross_scan_fwd, classification/models/csm_triton.py:22-29).  A thread's four positions are then
-// the four elements that END at L - 1 - t, taken in reverse.
-template <typename in_t>
-__device__ __forceinline__ Raw4<in_t> reverse4(const Raw4<in_t> &r) {
-    Raw4<in_t> o;
-    if constexpr (sizeof(in_t) == 2) {
-        o.w[0] = __builtin_amdgcn_alignbit(r.w[1], r.w[1], 16);      // halves of a dword exchanged
-        o.w[1] = __builtin_amdgcn_alignbit(r.w[0], r.w[0], 16);
-    } else {
-        o.w[0] = r.w[3]; o.w[1] = r.w[2]; o.w[2] = r.w[1]; o.w[3] = r.w[0];
-    }
-    return o;
-}
-
+// L - 1 - t of that row (cross_scan_fwd, classification/models/csm_triton.py:22-29).  A lane's four positions are then
+// the four elements that END at L - 1 - t, taken in reverse; where fewer are left, the row's first four.
+//
+// kDwords: the rows of 16-bit inputs start on dwords (RawGroup).
 // y[i] summed over the four sets of lanes (the banks of four lanes in a row of 16) for every position i of 16: afterwards
 // y[0 .. 3] are positions 4 set .. 4 set + 3.  Two DPP additions, each with its own banks, put two positions into one register:
 // half the additions of a sum that every lane gets, and no selects.
@@ -142,7 +106,7 @@ __device__ __forceinline__ void sum_over_sets(float (&y)[16]) {
 #undef SS2D_ODD
 }
 
-template <typename in_t, typename out_t, int kSpw, bool kSoftplus, bool kX, bool kMaps = false, int kPhase = kWhole>
+template <typename in_t, typename out_t, int kSpw, bool kSoftplus, bool kX, bool kMaps, int kPhase, bool kDwords>
 __global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void scan_chan_kernel(const in_t *__restrict__ u_all, const in_t *__restrict__ dl_all,
                                                            const in_t *__restrict__ B_all, const in_t *__restrict__ C_all,
                                                            const float *__restrict__ A_all, out_t *__restrict__ o_all,
@@ -181,23 +145,41 @@ __global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void sca
         u_first = ((k & 1) ? ut_all : u_all) + (int64_t)b * p.u_bs + (int64_t)(d_first - k * Dm) * p.u_ds;
         u_rev = k >= 2;
     }
-    const auto u_buf = rows_buffer(u_first, n_chan, p.u_ds, L);
-    const auto dl_buf = rows_buffer(dl_all + (int64_t)b * p.dl_bs + (int64_t)dg_first * p.dl_ds, (d_first + n_chan - 1) / p.dim_per_delta - dg_first + 1, p.dl_ds, L);
-    const auto o_buf = rows_buffer(o_all + (int64_t)b * p.o_bs + (int64_t)d_first * p.o_ds, n_chan, p.o_ds, L);
-    const uint32_t u_off = (uint32_t)((ds - d_first) * p.u_ds), dl_off = (uint32_t)((dgs - dg_first) * p.dl_ds), o_off = (uint32_t)((ds - d_first) * p.o_ds);
+    uint32_t u_row, dl_row, B_row, C_row;                   // the element a lane's row starts at
+    const auto u_buf = dwords_of<in_t>(u_first, 0, n_chan, p.u_ds, L, u_row);
+    const auto dl_buf = dwords_of<in_t>(dl_all, (int64_t)b * p.dl_bs + (int64_t)dg_first * p.dl_ds, (d_first + n_chan - 1) / p.dim_per_delta - dg_first + 1, p.dl_ds, L, dl_row);
+    const auto o_buf = rows_of<out_t>(o_all, (int64_t)b * p.o_bs + (int64_t)d_first * p.o_ds, n_chan, p.o_ds, L);
+    const uint32_t o_row = (uint32_t)((ds - d_first) * p.o_ds);
+    u_row += (uint32_t)((ds - d_first) * p.u_ds);
+    dl_row += (uint32_t)((dgs - dg_first) * p.dl_ds);
+    using Four = RawGroup<in_t, 4, kDwords>;
     // four positions of u from position pos of the scan on, as they lie in memory: backwards these are the four elements
-    // that end at L - 1 - pos, and they are put in scan order where they are widened (in_scan_order) -- not here, which
+    // that end at L - 1 - pos, and they are put in scan order where they are widened (unpack_u) -- not here, which
     // would make the wavefront wait for a load it has just issued for the NEXT step
-    auto load_u = [&](int pos) {
-        const int at = kMaps && u_rev ? L - 4 - pos : pos;
-        return load_raw4<in_t>(u_buf, pos < L ? (u_off + (uint32_t)at) * (uint32_t)sizeof(in_t) : kNowhere);
-    };
-    auto load_dl = [&](int pos) { return load_raw4<in_t>(dl_buf, pos < L ? (dl_off + (uint32_t)pos) * (uint32_t)sizeof(in_t) : kNowhere); };
-    auto in_scan_order = [&](const Raw4<in_t> &r) {
+    auto first_of = [&](int pos) { return kMaps && u_rev ? max(L - 4 - pos, 0) : pos; };
+    auto load_u = [&](int pos) { return load_at<in_t, 4, kDwords>(u_buf, u_row, first_of(pos), L, pos < L); };
+    auto load_dl = [&](int pos) { return load_at<in_t, 4, kDwords>(dl_buf, dl_row, pos, L); };
+    auto unpack_u = [&](const Four &raw, int pos, float (&v)[4]) {
+        float m[4];
+        widen<in_t, 4, kDwords>(raw, u_row + (uint32_t)first_of(pos), m);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = m[i];
         if constexpr (kMaps) {
-            if (u_rev) return reverse4<in_t>(r);
+            if (u_rev) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = m[3 - i];
+                if (L % 4 != 0 && pos + 4 > L) {            // the row's first elements, of which fewer are left
+                    const int skip = pos + 4 - L;
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        float at = v[i];
+#pragma unroll
+                        for (int k = 1; k < 4 - i; ++k) at = skip == k ? m[3 - i - k] : at;
+                        v[i] = at;
+                    }
+                }
+            }
         }
-        return r;
     };
     const float bias_s = p.bias ? p.bias[dgs] : 0.0f;
     const float D_s = p.D ? p.D[ds] : 0.0f;
@@ -206,21 +188,20 @@ __global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void sca
     // B / C: four positions of a row per lane and piece, rows [B, C][state of the lane][set]
     constexpr int kBcPieces = kSpw > 4 ? kSpw / 4 : 1;      // of each
     const bool bc_mine = kSpw >= 4 || lane < 16 * kSpw;
-    const auto B_buf = rows_buffer(B_all + (int64_t)b * p.B_bs + (int64_t)grp * p.B_gs, kChanSets * kSpw, p.B_ns, L);
-    const auto C_buf = rows_buffer(C_all + (int64_t)b * p.C_bs + (int64_t)grp * p.C_gs, kChanSets * kSpw, p.C_ns, L);
-    uint32_t B_off[kBcPieces], C_off[kBcPieces];
+    const auto B_buf = dwords_of<in_t>(B_all, (int64_t)b * p.B_bs + (int64_t)grp * p.B_gs, kChanSets * kSpw, p.B_ns, L, B_row);
+    const auto C_buf = dwords_of<in_t>(C_all, (int64_t)b * p.C_bs + (int64_t)grp * p.C_gs, kChanSets * kSpw, p.C_ns, L, C_row);
+    uint32_t B_rows[kBcPieces], C_rows[kBcPieces];
 #pragma unroll
     for (int k = 0; k < kBcPieces; ++k) {
         const int n = (r & 3) * kSpw + (r >> 2) + 4 * k;    // row r + 16 k of the array: state r / 4 + 4 k of set r % 4
-        B_off[k] = (uint32_t)(n * p.B_ns + 4 * q);
-        C_off[k] = (uint32_t)(n * p.C_ns + 4 * q);
+        B_rows[k] = B_row + (uint32_t)(n * p.B_ns);
+        C_rows[k] = C_row + (uint32_t)(n * p.C_ns);
     }
-    auto load_bc = [&](int t, Raw4<in_t> (&raw)[2 * kBcPieces]) {
-        const bool ok = bc_mine && t + 4 * q < L;
+    auto load_bc = [&](int t, Four (&raw)[2 * kBcPieces]) {
 #pragma unroll
         for (int k = 0; k < kBcPieces; ++k) {
-            raw[k] = load_raw4<in_t>(B_buf, ok ? (B_off[k] + (uint32_t)t) * (uint32_t)sizeof(in_t) : kNowhere);
-            if constexpr (kPhase != kLocal) raw[kBcPieces + k] = load_raw4<in_t>(C_buf, ok ? (C_off[k] + (uint32_t)t) * (uint32_t)sizeof(in_t) : kNowhere);
+            raw[k] = load_at<in_t, 4, kDwords>(B_buf, B_rows[k], t + 4 * q, L, bc_mine);
+            if constexpr (kPhase != kLocal) raw[kBcPieces + k] = load_at<in_t, 4, kDwords>(C_buf, C_rows[k], t + 4 * q, L, bc_mine);
         }
     };
     float *st_bc = s_bc + r * kChanSubPitch + 4 * q;
@@ -251,7 +232,7 @@ __global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void sca
             if (kX && set == 0) __builtin_memcpy(&dl_sum, seg_state + sizeof(float) * (p.N + 1), sizeof(dl_sum));
         }
     }
-    Raw4<in_t> ru[2], rd[2], rbc[2][2 * kBcPieces];
+    Four ru[2], rd[2], rbc[2][2 * kBcPieces];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         ru[s] = load_u(begin + s * kChanSub + 4 * q);
@@ -269,16 +250,19 @@ __global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void sca
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             float uv[4], raw[4], dl[4], du[4];
-            unpack_raw4<in_t>(in_scan_order(ru[s]), uv);
-            unpack_raw4<in_t>(rd[s], raw);
+            unpack_u(ru[s], t0 + s * kChanSub + 4 * q, uv);
+            widen<in_t, 4, kDwords>(rd[s], dl_row, raw);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 dl[i] = kSoftplus ? softplus_log2(fmaf(raw[i], kLog2e, bias_s * kLog2e)) : raw[i] + bias_s;
             }
             if (t0 + kChanTile > L) {                       // uniform; past the row's end 0, the identity of the recurrence
-                const bool in_row = t0 + s * kChanSub + 4 * q < L;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) dl[i] = in_row ? dl[i] : 0.0f;
+                for (int i = 0; i < 4; ++i) {
+                    const bool in_row = t0 + s * kChanSub + 4 * q + i < L;
+                    dl[i] = in_row ? dl[i] : 0.0f;
+                    uv[i] = in_row ? uv[i] : 0.0f;
+                }
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -302,7 +286,11 @@ __global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void sca
 #pragma unroll
             for (int k = 0; k < (kPhase == kLocal ? 1 : 2) * kBcPieces; ++k) {
                 float v[4];
-                unpack_raw4<in_t>(rbc[s][k], v);
+                widen<in_t, 4, kDwords>(rbc[s][k], k < kBcPieces ? B_rows[k % kBcPieces] : C_rows[k % kBcPieces], v);
+                if (L % 4 != 0 && ps + kChanSub > L) {      // uniform; four elements that the row's end divides
+#pragma unroll
+                    for (int i = 1; i < 4; ++i) v[i] = ps + 4 * q + i < L ? v[i] : 0.0f;
+                }
                 const int at = (k / kBcPieces) * kChanSets * kSpw + (k % kBcPieces) * 16;
                 if (bc_mine) *reinterpret_cast<float4 *>(st_bc + at * kChanSubPitch) = make_float4(v[0], v[1], v[2], v[3]);
             }
@@ -358,7 +346,7 @@ __global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void sca
                 const float4 part = *reinterpret_cast<const float4 *>(st_dl + s * kChanSub);
                 const float acc[4] = {skip[s][0] + part.x, skip[s][1] + part.y, skip[s][2] + part.z, skip[s][3] + part.w};
                 const int pos = t0 + s * kChanSub + 4 * q;
-                store4<out_t>(o_buf, r < n_chan && pos < L ? (o_off + (uint32_t)pos) * (uint32_t)sizeof(out_t) : kNowhere, acc);
+                store4<out_t, kDwords>(o_buf, (o_row + (uint32_t)pos) * (uint32_t)sizeof(out_t), L % 4 == 0 || t0 + kChanTile <= L, r < n_chan ? L - pos : 0, acc);
             }
             wave_lds_sync();
         }
@@ -430,14 +418,27 @@ __global__ __launch_bounds__(kBlock) void scan_chan_carry_kernel(const float *__
     }
 }
 
-bool scan_chan_eligible(const ScanArgs &a) {
-    // N/4 states per lane; rows in whole 8-position vectors; at least two blocks of channels per group; a block's rows within 32-bit
-    // byte offsets
+// Rows of whole 16-byte pieces and 8 positions are this kernel's at any size.  Others would take the kernels with positions in lanes, whose 16 states
+// of odd rows (49 positions, 64 x 96 maps in bf16: 191 us, here 24; 225: 281 / 55; 3306, 16 x 192: 1369 / 263) and larger calls of 4, 8 and 32 are far behind;
+// left to them are few wavefronts, each alone with its row: 4 states, 12 of them, 225 positions 9.0 / 12.4, 3306 21 / 24; 8 states, 225 14.2 / 15.4; 32 in
+// single precision 37 / 41; single precision of an odd number of fours, which they read in whole pieces: 4 states, 192: 1764 positions 34 / 55, 768: 90 / 83.
+static bool chan_pays(const ScanArgs &a, bool vec, int in_size) {
+    if (vec && a.L % 8 == 0) return true;
+    const int64_t units = (int64_t)a.batch * (a.dim / a.dim_per_group) * ((a.dim_per_group + kChanBlock - 1) / kChanBlock);
+    if (vec && a.N < 16) return units >= (a.L < 512 ? 192 : 768);
+    if (vec) return a.L < 512 || units >= 768 || units <= 48;
+    if (a.N == 4 && a.L > 2048 && units < 48) return false;
+    if (a.L > 64 && a.L <= 256 && units < 192) return a.N == 16 || (a.N == 32 && in_size == 2);
+    return true;
+}
+
+bool scan_chan_eligible(const ScanArgs &a, bool vec, int in_size) {
+    // N/4 states per lane; at least two blocks of channels per group; a block's rows within 32-bit byte offsets
     for (int64_t s : {a.u_ds, a.dl_ds, a.o_ds})
         if (s < 0 || (kChanBlock - 1) * s + a.L > kNowhere / 2 / 4) return false;
     for (int64_t s : {a.B_ns, a.C_ns})
         if (s < 0 || (a.N - 1) * s + a.L > kNowhere / 2 / 4) return false;
-    return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.L % 8 == 0 && a.dim_per_group >= 32;
+    return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.dim_per_group >= 32 && chan_pays(a, vec, in_size);
 }
 
 // The number of segments of a row (1: not cut) and the length of all but the last, which has at least 72 positions: a segment's N + 3
@@ -464,7 +465,7 @@ static int64_t chan_segments(const ScanArgs &a, int64_t n_units, int32_t &seg_le
     return n;
 }
 
-template <typename in_t, typename out_t>
+template <typename in_t, typename out_t, bool kDwords>
 static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stream) {
     ChanGeom geo = {};
     geo.n_cb = (a.dim_per_group + kChanBlock - 1) / kChanBlock;
@@ -476,7 +477,7 @@ static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stre
     geo.n_units = (uint32_t)n_rows;
     auto n_wg = [&] { return dim3((geo.n_units + kWavesPerWg - 1) / kWavesPerWg); };
 #define SS2D_LAUNCH_CHAN(SPW, SP, X, M)                                                                                    \
-    hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, SP, X, M>), n_wg(), dim3(kBlock), 0, stream,       \
+    hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, SP, X, M, kWhole, kDwords>), n_wg(), dim3(kBlock), 0, stream,       \
                        (const in_t *)a.u, (const in_t *)a.delta, (const in_t *)a.B, (const in_t *)a.C, a.A, (out_t *)a.out, a, geo, \
                        (const in_t *)xt)
 #define SS2D_LAUNCH_CHAN_N(SP, X, M)                            \
@@ -492,13 +493,13 @@ static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stre
     do {                                                                                                                   \
         geo.div_segs = make_fastdiv((uint32_t)segs - 1);                                                                    \
         geo.n_units = (uint32_t)(n_rows * (segs - 1));                                                                      \
-        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, false, M, kLocal>), n_wg(), dim3(kBlock), 0, stream, \
+        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, false, M, kLocal, kDwords>), n_wg(), dim3(kBlock), 0, stream, \
                            (const in_t *)a.u, (const in_t *)a.delta, (const in_t *)a.B, (const in_t *)a.C, a.A, (out_t *)a.out, a, geo, (const in_t *)xt); \
         hipLaunchKernelGGL((scan_chan_carry_kernel<out_t>), dim3((n_items + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, a.A, (out_t *)a.out, a, \
                            geo.seg_len, geo.n_segs, n_items, make_fastdiv((uint32_t)a.N), make_fastdiv((uint32_t)a.dim));   \
         geo.div_segs = make_fastdiv((uint32_t)segs);                                                                        \
         geo.n_units = (uint32_t)(n_rows * segs);                                                                            \
-        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, X, M, kRest>), n_wg(), dim3(kBlock), 0, stream, \
+        hipLaunchKernelGGL((scan_chan_kernel<in_t, out_t, SPW, true, X, M, kRest, kDwords>), n_wg(), dim3(kBlock), 0, stream, \
                            (const in_t *)a.u, (const in_t *)a.delta, (const in_t *)a.B, (const in_t *)a.C, a.A, (out_t *)a.out, a, geo, (const in_t *)xt); \
     } while (0)
 #define SS2D_LAUNCH_CHAN_SPLIT_N(X, M)                          \
@@ -533,11 +534,19 @@ static int launch_chan_typed(const ScanArgs &a, const void *xt, hipStream_t stre
 }
 
 int launch_scan_chan(const ScanArgs &a, int in_dtype, int out_dtype, hipStream_t stream, const void *xt) {
-    if (in_dtype == SS2D_F32) return launch_chan_typed<float, float>(a, xt, stream);
-    if (in_dtype == SS2D_BF16) {
-        return out_dtype == SS2D_F32 ? launch_chan_typed<bf16_t, float>(a, xt, stream) : launch_chan_typed<bf16_t, bf16_t>(a, xt, stream);
-    }
-    return out_dtype == SS2D_F32 ? launch_chan_typed<f16_t, float>(a, xt, stream) : launch_chan_typed<f16_t, f16_t>(a, xt, stream);
+    if (in_dtype == SS2D_F32) return launch_chan_typed<float, float, true>(a, xt, stream);
+    bool dwords = a.L % 2 == 0;                             // every row starts on a dword
+    for (const void *ptr : {a.u, a.delta, a.B, a.C, xt}) dwords = dwords && reinterpret_cast<uintptr_t>(ptr) % 4 == 0;
+    for (int64_t s : {a.u_bs, a.u_ds, a.dl_bs, a.dl_ds, a.B_bs, a.B_gs, a.B_ns, a.C_bs, a.C_gs, a.C_ns}) dwords = dwords && s % 2 == 0;
+    if (out_dtype != SS2D_F32) dwords = dwords && reinterpret_cast<uintptr_t>(a.out) % 4 == 0 && a.o_bs % 2 == 0 && a.o_ds % 2 == 0;
+#define SS2D_CHAN(T)                                                                                                                          \
+    do {                                                                                                                                      \
+        if (out_dtype == SS2D_F32) return dwords ? launch_chan_typed<T, float, true>(a, xt, stream) : launch_chan_typed<T, float, false>(a, xt, stream); \
+        return dwords ? launch_chan_typed<T, T, true>(a, xt, stream) : launch_chan_typed<T, T, false>(a, xt, stream);                          \
+    } while (0)
+    if (in_dtype == SS2D_BF16) SS2D_CHAN(bf16_t);
+    SS2D_CHAN(f16_t);
+#undef SS2D_CHAN
 }
 
 }  // namespace ss2d

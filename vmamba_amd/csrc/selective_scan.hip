@@ -762,7 +762,7 @@ static int plan_scan(const ss2d_scan_params *q, ScanArgs &a, bool &vec) {
     // rows of 49 / 196 positions, one state, rows adjacent in memory: one segment of a row per lane
     if (scan_small_eligible(a, q->in_dtype, q->u, q->delta, q->out)) return SS2D_SCAN_KERNEL_SMALL;
     // several states per channel and enough channels per group to fill wavefronts: one channel per lane
-    if (vec && scan_chan_eligible(a)) return SS2D_SCAN_KERNEL_CHAN;
+    if (scan_chan_eligible(a, vec, (int)in_bytes)) return SS2D_SCAN_KERNEL_CHAN;
     // A pass of the flat kernel costs about 1.4x a pass of the row kernel (measured), so the flat kernel wins
     // when the row kernel would leave more than ~30 % of its lanes idle, or cannot use vector I/O at all.
     const int64_t row_slots = ((int64_t)q->seqlen + kPass - 1) / kPass * kPass;
