@@ -2,6 +2,8 @@
 // buffer-descriptor gathers, the delta transform (bias + softplus) and the wavefront scan of (a, b) pairs.
 #pragma once
 
+#include <type_traits>
+
 #include "ss2d_common.h"
 
 namespace ss2d {
@@ -240,6 +242,68 @@ __device__ __forceinline__ void store_items_buffer(__amdgpu_buffer_rsrc_t rsrc, 
         __builtin_amdgcn_raw_buffer_store_b128(hi, rsrc, byte_off + 16, 0, 0);
     }
 }
+
+// the 16-bit type a row's fill is rounded to
+template <typename T> using bits_of = std::conditional_t<sizeof(T) == 2, T, bf16_t>;
+
+// Eight elements of a row from any multiple of 8 on, for rows of any length and alignment (RowReader).
+template <typename T> struct Raw8Any { uint32_t w[sizeof(T) == 2 ? 5 : 8]; };
+
+// A row, read eight elements a lane: in aligned 16-byte pieces (kVec), or as whole dwords from a base rounded down to one (the
+// hardware checks every dword against the row's end), elements that start in the upper half of a dword shifted down when they are
+// used (settle) and those past the row's end replaced.  The row is the same for the whole wavefront.
+template <typename T, bool kVec> struct RowReader {
+    using Raw = std::conditional_t<kVec, Raw8<T>, Raw8Any<T>>;
+    const T *row;
+    int L;
+
+    __device__ __forceinline__ RowReader(const T *row_, int L_) : row(row_), L(L_) {}
+    // of the first element in its dword, in bits
+    __device__ __forceinline__ uint32_t shift() const { return (uint32_t)(reinterpret_cast<uintptr_t>(row) & 3) * 8; }
+    // positions first + lane_pos .. + 7; first: uniform over the wavefront, a multiple of 8
+    template <bool kStream = false> __device__ __forceinline__ Raw load(int first, int lane_pos, float fill = 0.0f) const {
+        if constexpr (kVec) {
+            return load_raw<T, true, kStream>(row, first + lane_pos, L, fill);
+        } else {
+            // (a buffer of its own from `first` on: offsets stay small whatever the row's length)
+            constexpr int kAux = kStream ? 2 : 0;
+            const int off = lane_pos * (int)sizeof(T);
+            const uintptr_t at = reinterpret_cast<uintptr_t>(row + first);
+            const int64_t bytes = max((int64_t)(L - first), (int64_t)0) * (int)sizeof(T) + (int)(at & 3) + 3;
+            const auto buf = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(at & ~(uintptr_t)3), 0, L > first ? (int)min(bytes & ~(int64_t)3, (int64_t)1 << 20) : 0, kBufferRsrcWord3);
+            Raw r;
+            const auto a = __builtin_amdgcn_raw_buffer_load_b128(buf, off, 0, kAux);
+            r.w[0] = a[0]; r.w[1] = a[1]; r.w[2] = a[2]; r.w[3] = a[3];
+            if constexpr (sizeof(T) == 2) {
+                r.w[4] = __builtin_amdgcn_raw_buffer_load_b32(buf, off + 16, 0, kAux);
+            } else {
+                const auto b = __builtin_amdgcn_raw_buffer_load_b128(buf, off + 16, 0, kAux);
+                r.w[4] = b[0]; r.w[5] = b[1]; r.w[6] = b[2]; r.w[7] = b[3];
+            }
+            return r;
+        }
+    }
+    __device__ __forceinline__ Raw8<T> settle(const Raw &r, int pos, float fill = 0.0f) const {
+        if constexpr (kVec) {
+            return r;
+        } else {
+            Raw8<T> o;
+#pragma unroll
+            for (int i = 0; i < (int)sizeof(T) * 2; ++i) o.w[i] = sizeof(T) == 2 ? __builtin_amdgcn_alignbit(r.w[i + (sizeof(T) == 2)], r.w[i], shift()) : r.w[i];
+            if (pos + kItems > L) {                // (the one lane where the row ends, and those behind it)
+                const uint32_t f = sizeof(T) == 2 ? (uint32_t)from_f32<bits_of<T>>(fill).bits : 0u;
+#pragma unroll
+                for (int i = 0; i < kItems; ++i) {
+                    const bool in = pos + i < L;
+                    if constexpr (sizeof(T) == 4) o.w[i] = in ? o.w[i] : f32_to_bits(fill);
+                    else if (i % 2) o.w[i / 2] = in ? o.w[i / 2] : (o.w[i / 2] & 0xffffu) | f << 16;
+                    else o.w[i / 2] = in ? o.w[i / 2] : (o.w[i / 2] & 0xffff0000u) | f;
+                }
+            }
+            return o;
+        }
+    }
+};
 
 // A pass's outputs, 8 consecutive positions per lane, stored as fp32 so that each store instruction writes 1 KB of
 // consecutive addresses: at 32 bytes per lane an instruction would write every other 16 bytes of a 2 KB span, and

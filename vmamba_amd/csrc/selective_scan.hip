@@ -15,7 +15,8 @@
 //                2048-position chunk of one row and exchange their totals through LDS.
 //
 // I/O is 16-byte vectors per lane whenever pointers, strides and the row length allow
-// (kVec); otherwise element-wise with bounds checks.  Positions past the end of a row are fed
+// (kVec); otherwise whole dwords from a base rounded down to one (RowReader; one state, 4096 rows of 3249 positions in fp16: 107 us element by
+// element, 35 so).  Positions past the end of a row are fed
 // as dl = 0, u = 0, i.e. the identity pair (1, 0), so the state at the end of the last pass is
 // the state at the last real position.
 #include "scan_common.h"
@@ -85,19 +86,21 @@ __global__ __launch_bounds__(kBlock) void scan_row_kernel(const ScanArgs p) {
     const bool short_tail = kShortTail;
     const int n_pass = short_tail ? L / kPass : (L + kPass - 1) / kPass;
     const int L_body = short_tail ? n_pass * kPass : L;              // what the 8-per-lane passes cover
-    constexpr bool kTiledStore = kVec && sizeof(out_t) == 4;     // fp32 out as whole 1 KB runs (store_pass_f32)
+    constexpr bool kTiledStore = sizeof(out_t) == 4;             // fp32 out as whole 1 KB runs (store_pass_f32)
     __shared__ __align__(16) float y_tile[kTiledStore ? kWavesPerWg : 1][kTiledStore ? kPass : 4];
-    const __amdgpu_buffer_rsrc_t o_buf = row_buffer(o_row, kTiledStore ? L_body : 0);
+    const __amdgpu_buffer_rsrc_t o_buf = row_buffer(o_row, kTiledStore && kVec ? L_body : 0);
+    using Reader = RowReader<in_t, kVec>;
+    const Reader u_in(u_row, L_body), dl_in(dl_row, L_body), B_in(B_row, L_body), C_in(C_row, L_body);
     for (int pass0 = 0; pass0 < n_pass; pass0 += kBurst) {
-        Raw8<in_t> u_burst[kBurst], dl_burst[kBurst], B_burst[kBurst], C_burst[kBurst];
+        typename Reader::Raw u_burst[kBurst], dl_burst[kBurst], B_burst[kBurst], C_burst[kBurst];
 #pragma unroll
         for (int s = 0; s < kBurst; ++s) {
-            const int pos_s = (pass0 + s) * kPass + lane * kItems;
-            u_burst[s] = load_raw<in_t, kVec, true>(u_row, pos_s, L_body);
-            dl_burst[s] = load_raw<in_t, kVec, true>(dl_row, pos_s, L_body, delta_fill<kSoftplus>());
+            const int first = (pass0 + s) * kPass, mine = lane * kItems;
+            u_burst[s] = u_in.template load<true>(first, mine);
+            dl_burst[s] = dl_in.template load<true>(first, mine, delta_fill<kSoftplus>());
             if constexpr (kBurstBC) {
-                B_burst[s] = load_raw<in_t, kVec>(B_row, pos_s, L_body);
-                C_burst[s] = load_raw<in_t, kVec>(C_row, pos_s, L_body);
+                B_burst[s] = B_in.load(first, mine);
+                C_burst[s] = C_in.load(first, mine);
             }
         }
 #pragma unroll
@@ -105,9 +108,9 @@ __global__ __launch_bounds__(kBlock) void scan_row_kernel(const ScanArgs p) {
         const int pass = pass0 + s;
         if (pass >= n_pass) break;
         const int pos = pass * kPass + lane * kItems;
-        const Raw8<in_t> u_raw = u_burst[s], dl_raw = dl_burst[s];
+        const Raw8<in_t> u_raw = u_in.settle(u_burst[s], pos), dl_raw = dl_in.settle(dl_burst[s], pos, delta_fill<kSoftplus>());
         Raw8<in_t> B_raw, C_raw;
-        if constexpr (kBurstBC) { B_raw = B_burst[s]; C_raw = C_burst[s]; }
+        if constexpr (kBurstBC) { B_raw = B_in.settle(B_burst[s], pos); C_raw = C_in.settle(C_burst[s], pos); }
         float dl[kItems], du[kItems], y[kItems];
         prepare_delta_u<in_t, kSoftplus>(u_raw, dl_raw, L_body - pos, bias, Dv, dl, du, y);
         const bool chunk_end = x_row && ((pass + 1) % kPassesPerChunk == 0 || (pass == n_pass - 1 && !short_tail));
@@ -121,8 +124,10 @@ __global__ __launch_bounds__(kBlock) void scan_row_kernel(const ScanArgs p) {
                     unpack_raw<in_t>(B_raw, Bv);
                     unpack_raw<in_t>(C_raw, Cv);
                 } else {
-                    load_items<in_t, kVec>(B_row + n * p.B_ns, pos, L, Bv);
-                    load_items<in_t, kVec>(C_row + n * p.C_ns, pos, L, Cv);
+                    const Reader Bn(B_row + n * p.B_ns, L), Cn(C_row + n * p.C_ns, L);
+                    const auto b_raw = Bn.load(pass * kPass, lane * kItems), c_raw = Cn.load(pass * kPass, lane * kItems);
+                    unpack_raw<in_t>(Bn.settle(b_raw, pos), Bv);
+                    unpack_raw<in_t>(Cn.settle(c_raw, pos), Cv);
                 }
                 scan_state_pass(dl, du, Bv, Cv, A_reg[n], h_reg[n], y, a_tot, h_tot);
                 h_reg[n] = fmaf(a_tot, h_reg[n], h_tot);
@@ -148,8 +153,10 @@ __global__ __launch_bounds__(kBlock) void scan_row_kernel(const ScanArgs p) {
                         for (int i = 0; i < kHalf; ++i) { Bv[hv * kHalf + i] = bh[i]; Cv[hv * kHalf + i] = ch[i]; }
                     }
                 } else {
-                    load_items<in_t, kVec>(B_row + n * p.B_ns, pos, L, Bv);
-                    load_items<in_t, kVec>(C_row + n * p.C_ns, pos, L, Cv);
+                    const Reader Bn(B_row + n * p.B_ns, L), Cn(C_row + n * p.C_ns, L);
+                    const auto b_raw = Bn.load(pass * kPass, lane * kItems), c_raw = Cn.load(pass * kPass, lane * kItems);
+                    unpack_raw<in_t>(Bn.settle(b_raw, pos), Bv);
+                    unpack_raw<in_t>(Cn.settle(c_raw, pos), Cv);
                 }
                 const float ap = st[2 * n], h0 = st[2 * n + 1];
                 scan_state_pass(dl, du, Bv, Cv, A_row[n * p.A_ns] * kLog2e, h0, y, a_tot, h_tot);
@@ -160,7 +167,8 @@ __global__ __launch_bounds__(kBlock) void scan_row_kernel(const ScanArgs p) {
                 }
             }
         }
-        if constexpr (kVec && sizeof(out_t) == 4) store_pass_f32(y_tile[wave], o_buf, pass * kPass, lane, y);
+        if constexpr (kTiledStore && kVec) store_pass_f32(y_tile[wave], o_buf, pass * kPass, lane, y);
+        else if constexpr (kTiledStore) store_pass_f32(y_tile[wave], row_buffer(o_row + (int64_t)pass * kPass, min(kPass, L_body - pass * kPass)), 0, lane, y);
         else store_items<out_t, kVec>(o_row, pos, L_body, y);
         }
     }
@@ -405,26 +413,28 @@ __global__ __launch_bounds__(kBlock) void scan_row4_kernel(const ScanArgs p) {
     const float bias = p.bias ? p.bias[dg] : 0.0f;
     const int L = p.L;
 
-    constexpr bool kTiledStore = kVec && sizeof(out_t) == 4;     // fp32 out as whole 1 KB runs (store_pass_f32)
+    constexpr bool kTiledStore = sizeof(out_t) == 4;             // fp32 out as whole 1 KB runs (store_pass_f32)
     __shared__ __align__(16) float y_tile[kTiledStore ? kWavesPerWg : 1][kTiledStore ? kPass : 4];
-    const __amdgpu_buffer_rsrc_t o_buf = row_buffer(o_row, kTiledStore ? L : 0);
+    const __amdgpu_buffer_rsrc_t o_buf = row_buffer(o_row, kTiledStore && kVec ? L : 0);
     const int n_chunks = (L + SS2D_SCAN_CHUNK - 1) / SS2D_SCAN_CHUNK;
     // the next chunk's u / delta (and B / C of the first state) are requested before this chunk's arithmetic and its
     // barriers: a wavefront always has a chunk of loads in flight (positions past the row's end come back as the fill)
     const int pos_first = wave * kPass + lane * kItems;
-    Raw8<in_t> u_nx = load_raw<in_t, kVec, true>(u_row, pos_first, L);
-    Raw8<in_t> dl_nx = load_raw<in_t, kVec, true>(dl_row, pos_first, L, delta_fill<kSoftplus>());
-    Raw8<in_t> B_nx = load_raw<in_t, kVec>(B_row, pos_first, L), C_nx = load_raw<in_t, kVec>(C_row, pos_first, L);
+    using Reader = RowReader<in_t, kVec>;
+    const Reader u_in(u_row, L), dl_in(dl_row, L), B_in(B_row, L), C_in(C_row, L);
+    auto u_nx = u_in.template load<true>(0, pos_first), dl_nx = dl_in.template load<true>(0, pos_first, delta_fill<kSoftplus>());
+    auto B_nx = B_in.load(0, pos_first), C_nx = C_in.load(0, pos_first);
     for (int chunk = 0; chunk < n_chunks; ++chunk) {
         const int par = chunk & 1;
         const int pos = chunk * SS2D_SCAN_CHUNK + pos_first;
-        const Raw8<in_t> u_raw = u_nx, dl_raw = dl_nx, B_raw = B_nx, C_raw = C_nx;
+        const Raw8<in_t> u_raw = u_in.settle(u_nx, pos), dl_raw = dl_in.settle(dl_nx, pos, delta_fill<kSoftplus>());
+        const Raw8<in_t> B_raw = B_in.settle(B_nx, pos), C_raw = C_in.settle(C_nx, pos);
         if (chunk + 1 < n_chunks) {
-            const int pos_nx = pos + SS2D_SCAN_CHUNK;
-            u_nx = load_raw<in_t, kVec, true>(u_row, pos_nx, L);
-            dl_nx = load_raw<in_t, kVec, true>(dl_row, pos_nx, L, delta_fill<kSoftplus>());
-            B_nx = load_raw<in_t, kVec>(B_row, pos_nx, L);
-            C_nx = load_raw<in_t, kVec>(C_row, pos_nx, L);
+            const int next = (chunk + 1) * SS2D_SCAN_CHUNK;
+            u_nx = u_in.template load<true>(next, pos_first);
+            dl_nx = dl_in.template load<true>(next, pos_first, delta_fill<kSoftplus>());
+            B_nx = B_in.load(next, pos_first);
+            C_nx = C_in.load(next, pos_first);
         }
         float dl[kItems], du[kItems], y[kItems];
         prepare_delta_u<in_t, kSoftplus>(u_raw, dl_raw, L - pos, bias, Dv, dl, du, y);
@@ -434,8 +444,10 @@ __global__ __launch_bounds__(kBlock) void scan_row4_kernel(const ScanArgs p) {
                 unpack_raw<in_t>(B_raw, Bv);
                 unpack_raw<in_t>(C_raw, Cv);
             } else {
-                load_items<in_t, kVec>(B_row + n * p.B_ns, pos, L, Bv);
-                load_items<in_t, kVec>(C_row + n * p.C_ns, pos, L, Cv);
+                const Reader Bn(B_row + n * p.B_ns, L), Cn(C_row + n * p.C_ns, L);
+                const auto b_raw = Bn.load(chunk * SS2D_SCAN_CHUNK, pos_first), c_raw = Cn.load(chunk * SS2D_SCAN_CHUNK, pos_first);
+                unpack_raw<in_t>(Bn.settle(b_raw, pos), Bv);
+                unpack_raw<in_t>(Cn.settle(c_raw, pos), Cv);
             }
             const float A_log2e = A_row[n * p.A_ns] * kLog2e;
             float ac[kItems], hh[kItems];
@@ -471,7 +483,12 @@ __global__ __launch_bounds__(kBlock) void scan_row4_kernel(const ScanArgs p) {
                 }
             }
         }
-        if constexpr (kTiledStore) store_pass_f32(y_tile[wave], o_buf, chunk * SS2D_SCAN_CHUNK + wave * kPass, lane, y);
+        if constexpr (kTiledStore && kVec) {
+            store_pass_f32(y_tile[wave], o_buf, chunk * SS2D_SCAN_CHUNK + wave * kPass, lane, y);
+        } else if constexpr (kTiledStore) {
+            const int first = chunk * SS2D_SCAN_CHUNK + wave * kPass;
+            store_pass_f32(y_tile[wave], row_buffer(o_row + first, max(0, min(kPass, L - first))), 0, lane, y);
+        }
         else store_items<out_t, kVec>(o_row, pos, L, y);
     }
 }
@@ -602,14 +619,30 @@ static bool span_fits_u32(const ScanArgs &a, int64_t elem_bytes) {
 // per channel, rows of at least one lane vector, and dstate 1 or 16.
 static bool flat_eligible(const ScanArgs &a, const ss2d_scan_params *q) {
     const int64_t L = a.L, KD = a.dim;
-    // rows of four passes and more only where the row kernel would fall back to element-wise accesses (the caller
-    // checks that) and there are rows enough to fill the chip eight to a wavefront (measured, unaligned bf16 rows of
-    // 5625 positions: 27 264 rows 515 us against 1112, 6144 rows 191 against 241, 3072 rows 153 against 114)
+    // (many rows of four passes and more keep this kernel's id; dispatch_vec)
     const bool length_ok = L < 4 * kPass || (L <= (1 << 24) && a.N == 1 && a.rows >= 6144);
     return L >= kItems && length_ok && (a.N == 1 || a.N == 16) && q->delta_dim == q->dim &&
            a.u_ds == L && a.dl_ds == L && a.o_ds == L && a.u_bs == KD * L && a.dl_bs == KD * L && a.o_bs == KD * L &&
            aligned16(q->u) && aligned16(q->delta) && aligned16(q->out) &&
            span_fits_u32(a, q->in_dtype == SS2D_F32 ? 4 : 2);
+}
+
+static int flat_granularity(const ScanArgs &a, int64_t elem_bytes);
+
+// Several rows to a wavefront, or one.  A wavefront of the flat kernel walks eight rows or more behind one another, so few rows leave the
+// chip idle: a wavefront per row is ahead at any length (one state, us, flat / row; 192 rows: 56 positions 13.4 / 4.4, 225 21 / 5.5, 1353 34 / 5.7;
+// 3072: 56 11.6 / 4.0, 225 20 / 6.9, 576 16 / 8.3, 1353 44 / 14).  Many rows: a pass of the flat kernel costs about 1.4x a pass of the row kernel with
+// groups of two elements or more, and more with single ones, so it is ahead where the row kernel would leave more than 30 % of its lanes idle
+// (12 288 rows: 601 of 1024 positions 42 / 32 with single elements; 24 576: 418 of 512 in pairs 44 / 50, 601 72 / 77, 1003 124 / 104,
+// 1353 176 / 138) and, reading pairs or fours, on rows that are no whole 16-byte pieces (24 576 of 484: 38 / 46).
+static bool flat_pays(const ScanArgs &a, bool vec, int in_size) {
+    if (a.L >= 4 * kPass) return !vec;                     // long rows off the 16-byte grid: dispatch_vec
+    const bool half_full = 10 * (int64_t)a.L < 7 * (((int64_t)a.L + kPass - 1) / kPass * kPass);
+    if (a.rows <= 8192 || (vec && in_size == 2 && a.L <= 336 && a.rows <= 12288)) return false;
+    if (vec) return half_full;
+    const int gran = flat_granularity(a, in_size);
+    if (a.rows <= 16384) return gran == 1 ? a.L < 64 : 4 * (int64_t)a.L < 3 * (((int64_t)a.L + kPass - 1) / kPass * kPass);
+    return gran > 1 || half_full;
 }
 
 static int gcd_i64(int64_t a, int64_t b) { while (b) { const int64_t t = a % b; a = b; b = t; } return (int)(a < 0 ? -a : a); }
@@ -703,7 +736,9 @@ static int launch_scan(const ScanArgs &a, bool split_rows, hipStream_t stream) {
 
 template <typename in_t, typename out_t>
 static int dispatch_vec(const ScanArgs &a, bool vec, int kernel, hipStream_t stream) {
-    if (kernel == SS2D_SCAN_KERNEL_FLAT) return launch_flat<in_t, out_t>(a, stream);
+    // long rows under the flat kernel's id are a wavefront's each all the same: eight to a wavefront as one stream gather B and C element by
+    // element (one state, us, stream / row: 6144 rows of 2051 positions in bf16 64 / 31, 24 576 119 / 108, 24 576 of 5625 389 / 267; in fp32 227 / 142, 585 / 371)
+    if (kernel == SS2D_SCAN_KERNEL_FLAT && a.L < 4 * kPass) return launch_flat<in_t, out_t>(a, stream);
     const bool split_rows = kernel == SS2D_SCAN_KERNEL_ROW4;
     return vec ? launch_scan<in_t, out_t, true>(a, split_rows, stream) : launch_scan<in_t, out_t, false>(a, split_rows, stream);
 }
@@ -763,10 +798,7 @@ static int plan_scan(const ss2d_scan_params *q, ScanArgs &a, bool &vec) {
     if (scan_small_eligible(a, q->in_dtype, q->u, q->delta, q->out)) return SS2D_SCAN_KERNEL_SMALL;
     // several states per channel and enough channels per group to fill wavefronts: one channel per lane
     if (scan_chan_eligible(a, vec, (int)in_bytes)) return SS2D_SCAN_KERNEL_CHAN;
-    // A pass of the flat kernel costs about 1.4x a pass of the row kernel (measured), so the flat kernel wins
-    // when the row kernel would leave more than ~30 % of its lanes idle, or cannot use vector I/O at all.
-    const int64_t row_slots = ((int64_t)q->seqlen + kPass - 1) / kPass * kPass;
-    if (flat_eligible(a, q) && (!vec || 10 * (int64_t)q->seqlen < 7 * row_slots)) return SS2D_SCAN_KERNEL_FLAT;
+    if (flat_eligible(a, q) && flat_pays(a, vec, (int)in_bytes)) return SS2D_SCAN_KERNEL_FLAT;
     // few long rows: every row split over the four wavefronts of a workgroup (3072 rows and more: a wavefront per row is faster)
     if (a.L > SS2D_SCAN_CHUNK && a.rows < 2048) return SS2D_SCAN_KERNEL_ROW4;
     return SS2D_SCAN_KERNEL_ROW;
