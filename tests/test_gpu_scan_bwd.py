@@ -109,6 +109,19 @@ def test_scan_bwd_16bit_row_lengths(N, L, dtype, dout_float):
     compare(got, want, 3e-2, "16-bit")
 
 
+# Rows that are no whole 16-byte pieces, read as dwords: one, two and three elements into a group of four and of eight, rows on odd elements and on
+# even ones, one state and three; float64 as above.
+@pytest.mark.parametrize("dtype,dout_float", [(torch.float32, True), (torch.bfloat16, True), (torch.bfloat16, False), (torch.float16, True)])
+@pytest.mark.parametrize("N,L", [(1, 65), (1, 254), (1, 255), (1, 257), (1, 331), (1, 1030), (3, 67), (3, 301)])
+def test_scan_bwd_odd_rows(N, L, dtype, dout_float):
+    print("CASE scan-bwd-odd-rows", N, L, dtype, dout_float, flush=True)
+    u, delta, A, B, C, D, bias, dout = make(N + L, 2, 10, 2, N, L, dtype)
+    dout = dout if dout_float else dout.to(dtype)
+    want = torch_ref.selective_scan_grads(u.float(), delta.float(), A, B.float(), C.float(), D, bias, dout.float(), True)
+    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, True, 1)
+    compare(got, want, 1e-4 if dtype == torch.float32 else 3e-2, "odd rows")
+
+
 # A channel per lane (scan_bwd_chan.hip): rows of one segment (up to 72 positions, many of them), of two, and of many; the last chunk of 8 positions with
 # 1, 3, 7 and 8 of them; 16, 33, 50 and 51 channels per group (1 and 2 in the last wavefront, idle wavefronts); 4, 8 and 16 states; delta rows
 # shared; rows off the dword grid.  Bound in single precision: sums of up to 1030 terms and 51 channels, each term good to a few 2^-23 -- 1e-4 of the largest gradient.

@@ -209,25 +209,57 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_kernel(const ScanBwdArgs p) {
 
 // ---- pieces of the two register-summing kernels -------------------------------------------------------------------
 // kI consecutive elements of a row seen through a buffer descriptor: a load past the row's end returns 0, a store there
-// is dropped.  kVec: rows start on kI-element boundaries and hold a whole number of such groups.
+// is dropped, dword by dword.  kVec: rows are whole dwords (single precision always); otherwise
+// the descriptor's base is rounded down to a dword, a dword more is loaded, and settle shifts the elements down.
 template <typename T, int kI> struct RawN { uint32_t w[gather_words<T, kI>()]; };
+template <typename T, int kI, bool kVec> struct LoadN { uint32_t w[gather_words<T, kI>() + (!kVec && sizeof(T) == 2 && kI > 1)]; };
 
 template <typename T, int kI, bool kVec>
-__device__ __forceinline__ RawN<T, kI> load_group(__amdgpu_buffer_rsrc_t rsrc, int pos) {
-    RawN<T, kI> r;
-    if constexpr (kVec || kI == 1) {
+__device__ __forceinline__ LoadN<T, kI, kVec> load_group(__amdgpu_buffer_rsrc_t rsrc, int pos) {
+    LoadN<T, kI, kVec> r;
+    if constexpr (kVec || kI == 1 || sizeof(T) == 4) {
         gather_group_raw<T, kI>(rsrc, (uint32_t)pos, 0, r.w);
+    } else if constexpr (kI == 4) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b96(rsrc, pos * 2, 0, 0);
+        r.w[0] = v[0]; r.w[1] = v[1]; r.w[2] = v[2];
     } else {
-        uint32_t e[kI][1];
-#pragma unroll
-        for (int i = 0; i < kI; ++i) gather_group_raw<T, 1>(rsrc, (uint32_t)(pos + i), 0, e[i]);
-#pragma unroll
-        for (int i = 0; i < gather_words<T, kI>(); ++i) {
-            if constexpr (sizeof(T) == 2) r.w[i] = e[2 * i][0] | (e[2 * i + 1][0] << 16);
-            else r.w[i] = e[i][0];
-        }
+        static_assert(kI == 8, "groups of 1, 4 or 8");
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, pos * 2, 0, 0);
+        r.w[0] = v[0]; r.w[1] = v[1]; r.w[2] = v[2]; r.w[3] = v[3];
+        r.w[4] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, pos * 2 + 16, 0, 0);
     }
     return r;
+}
+
+// The elements as they arrived; `shift`: bits before the row's first element in its dword, n_valid: elements inside the row.
+template <typename T, int kI, bool kVec>
+__device__ __forceinline__ RawN<T, kI> settle(const LoadN<T, kI, kVec> &r, uint32_t shift, int n_valid) {
+    RawN<T, kI> o;
+    if constexpr (kVec || kI == 1 || sizeof(T) == 4) {
+#pragma unroll
+        for (int i = 0; i < gather_words<T, kI>(); ++i) o.w[i] = r.w[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < kI / 2; ++i) o.w[i] = __builtin_amdgcn_alignbit(r.w[i + 1], r.w[i], shift);
+        if (n_valid < kI) {                                     // (the dword that the row's end divides holds another row's element)
+#pragma unroll
+            for (int i = 0; i < kI / 2; ++i) o.w[i] &= (2 * i < n_valid ? 0xffffu : 0u) | (2 * i + 1 < n_valid ? 0xffff0000u : 0u);
+        }
+    }
+    return o;
+}
+
+// A row's buffer for load_group, and its shift.
+template <typename T, bool kVec>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t load_buffer(const T *row, int L, uint32_t &shift) {
+    if constexpr (kVec || sizeof(T) == 4) {
+        shift = 0;
+        return row_buffer(row, L);
+    } else {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(row);
+        shift = (uint32_t)(at & 2) * 8;
+        return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(at & ~(uintptr_t)3), 0, (2 * L + (int)(at & 2) + 3) & ~3, kBufferRsrcWord3);
+    }
 }
 
 template <typename T, int kI, bool kVec>
@@ -235,7 +267,7 @@ __device__ __forceinline__ void store_group(__amdgpu_buffer_rsrc_t rsrc, int pos
     typedef uint32_t words4_t __attribute__((ext_vector_type(4)));
     typedef uint32_t words2_t __attribute__((ext_vector_type(2)));
     const int off = pos * (int)sizeof(T);
-    if constexpr (!kVec || kI == 1) {
+    if constexpr ((!kVec && sizeof(T) == 2) || kI == 1) {
 #pragma unroll
         for (int i = 0; i < kI; ++i) {
             if constexpr (sizeof(T) == 2) __builtin_amdgcn_raw_buffer_store_b16(from_f32<T>(v[i]).bits, rsrc, off + 2 * i, 0, 0);
@@ -327,14 +359,15 @@ __device__ __forceinline__ void bwd_step(const RawN<in_t, kI> &raw, float bias, 
 }
 
 // The rows and constants of channel d of image b; kN states from n_first on, of which ns exist.
-template <typename in_t, typename dy_t, int kN> struct BwdRows {
+template <typename in_t, typename dy_t, int kN, bool kVec> struct BwdRows {
     __amdgpu_buffer_rsrc_t u, dl, dy, du, dd;
+    uint32_t u_shift, dl_shift, dy_shift;
     float bias, Dv, A[kN];
     __device__ __forceinline__ void set(const ScanBwdArgs &p, int b, int d, int n_first = 0, int ns = kN) {
         const int dg = d / p.dim_per_delta;
-        u = row_buffer(reinterpret_cast<const in_t *>(p.u) + b * p.u_bs + d * p.u_ds, p.L);
-        dl = row_buffer(reinterpret_cast<const in_t *>(p.delta) + b * p.dl_bs + dg * p.dl_ds, p.L);
-        dy = row_buffer(reinterpret_cast<const dy_t *>(p.dout) + b * p.do_bs + d * p.do_ds, p.L);
+        u = load_buffer<in_t, kVec>(reinterpret_cast<const in_t *>(p.u) + b * p.u_bs + d * p.u_ds, p.L, u_shift);
+        dl = load_buffer<in_t, kVec>(reinterpret_cast<const in_t *>(p.delta) + b * p.dl_bs + dg * p.dl_ds, p.L, dl_shift);
+        dy = load_buffer<dy_t, kVec>(reinterpret_cast<const dy_t *>(p.dout) + b * p.do_bs + d * p.do_ds, p.L, dy_shift);
         du = row_buffer(reinterpret_cast<const in_t *>(p.du) + ((size_t)b * p.dim + d) * p.L, p.L);
         dd = row_buffer(reinterpret_cast<const in_t *>(p.ddelta) + ((size_t)b * p.dim + d) * p.L, p.L);
         bias = p.bias ? p.bias[dg] : 0.0f;
@@ -368,24 +401,25 @@ __global__ __launch_bounds__(kBlock, 3) void scan_bwd_one_kernel(const ScanBwdAr
     const int nc = c_first < c_end ? (c_end - c_first + kWavesPerWg - 1) / kWavesPerWg : 0;
     const int d_first = grp * p.dim_per_group + c_first;
     const bool softplus = p.softplus != 0;
-    const auto B_buf = row_buffer(reinterpret_cast<const in_t *>(p.B) + b * p.B_bs + grp * p.B_gs, L);
-    const auto C_buf = row_buffer(reinterpret_cast<const in_t *>(p.C) + b * p.C_bs + grp * p.C_gs, L);
-    using Rows = BwdRows<in_t, dy_t, 1>;
+    uint32_t B_shift, C_shift;
+    const auto B_buf = load_buffer<in_t, kVec>(reinterpret_cast<const in_t *>(p.B) + b * p.B_bs + grp * p.B_gs, L, B_shift);
+    const auto C_buf = load_buffer<in_t, kVec>(reinterpret_cast<const in_t *>(p.C) + b * p.C_bs + grp * p.C_gs, L, C_shift);
+    using Rows = BwdRows<in_t, dy_t, 1, kVec>;
 
     // ---- sweep 1: the state entering every pass, for every channel of this wavefront ------------------------------
     for (int i = lane; i < nc; i += kWave) h_in[i * P] = 0.0f;
     if (nc > 0 && P > 1) {
         Rows r;
         r.set(p, b, d_first);
-        RawN<in_t, kI> u_raw = load_group<in_t, kI, kVec>(r.u, lane * kI), dl_raw = load_group<in_t, kI, kVec>(r.dl, lane * kI);
+        LoadN<in_t, kI, kVec> u_raw = load_group<in_t, kI, kVec>(r.u, lane * kI), dl_raw = load_group<in_t, kI, kVec>(r.dl, lane * kI);
         for (int pass = 0; pass + 1 < P; ++pass) {
             const int pos = pass * kLen + lane * kI;
-            const RawN<in_t, kI> B_raw = load_group<in_t, kI, kVec>(B_buf, pos);
+            const RawN<in_t, kI> B_raw = settle<in_t, kI, kVec>(load_group<in_t, kI, kVec>(B_buf, pos), B_shift, kI);
             float Bv[kI];
             unpack_group<in_t, kI>(B_raw.w, Bv);
             for (int ci = 0; ci < nc; ++ci) {
                 const float bias = r.bias, A_log2e = r.A[0] * kLog2e;
-                const RawN<in_t, kI> u_now = u_raw, dl_now = dl_raw;
+                const RawN<in_t, kI> u_now = settle<in_t, kI, kVec>(u_raw, r.u_shift, kI), dl_now = settle<in_t, kI, kVec>(dl_raw, r.dl_shift, kI);
                 // the next channel, or the first one of the next pass
                 const bool wrap = ci + 1 == nc;
                 const int pos_next = wrap ? pos + kLen : pos;
@@ -413,8 +447,8 @@ __global__ __launch_bounds__(kBlock, 3) void scan_bwd_one_kernel(const ScanBwdAr
     // ---- sweep 2: passes in reverse, channels inside ------------------------------------------------------------------
     float g_carry = 0.0f, a_next = 1.0f, dA_sum = 0.0f, dD_sum = 0.0f, db_sum = 0.0f;      // lane i: channel i
     Rows r;
-    RawN<in_t, kI> u_raw, dl_raw;
-    RawN<dy_t, kI> dy_raw;
+    LoadN<in_t, kI, kVec> u_raw, dl_raw;
+    LoadN<dy_t, kI, kVec> dy_raw;
     if (nc > 0) {
         const int pos = (P - 1) * kLen + lane * kI;
         r.set(p, b, d_first);
@@ -427,7 +461,8 @@ __global__ __launch_bounds__(kBlock, 3) void scan_bwd_one_kernel(const ScanBwdAr
         const int n_valid = pass + 1 < P ? kI : L - pos;
         float Bv[kI], Cv[kI], sumB[kI], sumC[kI];
         {
-            const RawN<in_t, kI> B_raw = load_group<in_t, kI, kVec>(B_buf, pos), C_raw = load_group<in_t, kI, kVec>(C_buf, pos);
+            const auto B_in = load_group<in_t, kI, kVec>(B_buf, pos), C_in = load_group<in_t, kI, kVec>(C_buf, pos);
+            const RawN<in_t, kI> B_raw = settle<in_t, kI, kVec>(B_in, B_shift, n_valid), C_raw = settle<in_t, kI, kVec>(C_in, C_shift, n_valid);
             unpack_group<in_t, kI>(B_raw.w, Bv);
             unpack_group<in_t, kI>(C_raw.w, Cv);
         }
@@ -435,8 +470,8 @@ __global__ __launch_bounds__(kBlock, 3) void scan_bwd_one_kernel(const ScanBwdAr
         for (int i = 0; i < kI; ++i) { sumB[i] = 0.0f; sumC[i] = 0.0f; }
         for (int ci = 0; ci < nc; ++ci) {
             const Rows rn = r;
-            const RawN<in_t, kI> u_now = u_raw, dl_now = dl_raw;
-            const RawN<dy_t, kI> dy_now = dy_raw;
+            const RawN<in_t, kI> u_now = settle<in_t, kI, kVec>(u_raw, rn.u_shift, n_valid), dl_now = settle<in_t, kI, kVec>(dl_raw, rn.dl_shift, n_valid);
+            const RawN<dy_t, kI> dy_now = settle<dy_t, kI, kVec>(dy_raw, rn.dy_shift, n_valid);
             const bool wrap = ci + 1 == nc;
             const int pos_next = wrap && pass > 0 ? pos - kLen : pos;      // (after the last one: read again, not used)
             r.set(p, b, d_first + (wrap ? 0 : ci + 1) * kWavesPerWg);
@@ -563,11 +598,12 @@ __global__ __launch_bounds__(512, 2) void scan_bwd_states_kernel(const ScanBwdAr
     const bool softplus = p.softplus != 0;
     const in_t *B_rows = reinterpret_cast<const in_t *>(p.B) + b * p.B_bs + grp * p.B_gs + n_first * p.B_ns;
     const in_t *C_rows = reinterpret_cast<const in_t *>(p.C) + b * p.C_bs + grp * p.C_gs + n_first * p.C_ns;
-    using Rows = BwdRows<in_t, dy_t, kStates>;
-    auto load_states = [&](const in_t *rows, int64_t stride, int pos, RawN<in_t, kI> (&raw)[kStates]) {
+    using Rows = BwdRows<in_t, dy_t, kStates, kVec>;
+    auto load_states = [&](const in_t *rows, int64_t stride, int pos, int n_valid, RawN<in_t, kI> (&raw)[kStates]) {
 #pragma unroll
         for (int s = 0; s < kStates; ++s) {
-            if (s < ns) raw[s] = load_group<in_t, kI, kVec>(row_buffer(rows + s * stride, L), pos);
+            uint32_t shift;
+            if (s < ns) raw[s] = settle<in_t, kI, kVec>(load_group<in_t, kI, kVec>(load_buffer<in_t, kVec>(rows + s * stride, L, shift), pos), shift, n_valid);
             else raw[s] = RawN<in_t, kI>{};                      // states past N: B = C = 0, they stay 0
         }
     };
@@ -577,14 +613,14 @@ __global__ __launch_bounds__(512, 2) void scan_bwd_states_kernel(const ScanBwdAr
     if (P > 1) {
         Rows r;
         r.set(p, b, d_first, n_first, ns);
-        RawN<in_t, kI> u_raw = load_group<in_t, kI, kVec>(r.u, lane * kI), dl_raw = load_group<in_t, kI, kVec>(r.dl, lane * kI);
+        LoadN<in_t, kI, kVec> u_raw = load_group<in_t, kI, kVec>(r.u, lane * kI), dl_raw = load_group<in_t, kI, kVec>(r.dl, lane * kI);
         for (int pass = 0; pass + 1 < P; ++pass) {
             const int pos = pass * kLen + lane * kI;
             RawN<in_t, kI> B_raw[kStates];
-            load_states(B_rows, p.B_ns, pos, B_raw);
+            load_states(B_rows, p.B_ns, pos, kI, B_raw);
             for (int ci = 0; ci < nc; ++ci) {
                 const Rows rn = r;
-                const RawN<in_t, kI> u_now = u_raw, dl_now = dl_raw;
+                const RawN<in_t, kI> u_now = settle<in_t, kI, kVec>(u_raw, rn.u_shift, kI), dl_now = settle<in_t, kI, kVec>(dl_raw, rn.dl_shift, kI);
                 const bool wrap = ci + 1 == nc;
                 const int pos_next = wrap ? pos + kLen : pos;
                 r.set(p, b, d_first + (wrap ? 0 : ci + 1), n_first, ns);
@@ -625,8 +661,8 @@ __global__ __launch_bounds__(512, 2) void scan_bwd_states_kernel(const ScanBwdAr
     Rows r;
     r.set(p, b, d_first, n_first, ns);
     int buffer = 0;
-    RawN<in_t, kI> u_raw, dl_raw;
-    RawN<dy_t, kI> dy_raw;
+    LoadN<in_t, kI, kVec> u_raw, dl_raw;
+    LoadN<dy_t, kI, kVec> dy_raw;
     {
         const int pos = (P - 1) * kLen + lane * kI;
         u_raw = load_group<in_t, kI, kVec>(r.u, pos);
@@ -637,8 +673,8 @@ __global__ __launch_bounds__(512, 2) void scan_bwd_states_kernel(const ScanBwdAr
         const int pos = pass * kLen + lane * kI;
         const int n_valid = pass + 1 < P ? kI : L - pos;
         RawN<in_t, kI> B_raw[kStates], C_raw[kStates];
-        load_states(B_rows, p.B_ns, pos, B_raw);
-        load_states(C_rows, p.C_ns, pos, C_raw);
+        load_states(B_rows, p.B_ns, pos, n_valid, B_raw);
+        load_states(C_rows, p.C_ns, pos, n_valid, C_raw);
         float sumB[kStates][kI], sumC[kStates][kI];
 #pragma unroll
         for (int s = 0; s < kStates; ++s)
@@ -647,8 +683,8 @@ __global__ __launch_bounds__(512, 2) void scan_bwd_states_kernel(const ScanBwdAr
 
         for (int ci = 0; ci < nc; ++ci) {
             const Rows rn = r;
-            const RawN<in_t, kI> u_now = u_raw, dl_now = dl_raw;
-            const RawN<dy_t, kI> dy_now = dy_raw;
+            const RawN<in_t, kI> u_now = settle<in_t, kI, kVec>(u_raw, rn.u_shift, n_valid), dl_now = settle<in_t, kI, kVec>(dl_raw, rn.dl_shift, n_valid);
+            const RawN<dy_t, kI> dy_now = settle<dy_t, kI, kVec>(dy_raw, rn.dy_shift, n_valid);
             const bool wrap = ci + 1 == nc;
             const int pos_next = wrap && pass > 0 ? pos - kLen : pos;      // (after the last one: read again, not used)
             r.set(p, b, d_first + (wrap ? 0 : ci + 1), n_first, ns);
@@ -853,6 +889,7 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
     // whether rows can be read and written in groups of `items` elements: 16-byte pieces at most, so the group's alignment
     // is that of its piece
     const int in_size = q->in_dtype == SS2D_F32 ? 4 : 2, dy_size = q->dout_dtype == SS2D_F32 ? 4 : 2;
+    // (of the element-wise kernel; the others need dwords only, and single precision nothing)
     auto groups_ok = [&](int items) {
         const int64_t in_vec = items * in_size > 16 ? 16 / in_size : items, dy_vec = items * dy_size > 16 ? 16 / dy_size : items;
         auto aligned = [](const void *ptr, int64_t bytes) { return (reinterpret_cast<uintptr_t>(ptr) & (uintptr_t)(bytes - 1)) == 0; };
@@ -868,6 +905,18 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
         const int rc = launch_scan_bwd_chan(a, q->in_dtype, q->dout_dtype, s);
         if (rc != SS2D_ENOTSUP) return rc;                  // (before any launch)
     }
+    auto dwords_ok = [&](int items) {                            // rows of whole dwords (with one position per lane elements are read)
+        if (items == 1) return true;
+        auto odd = [](const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 3) != 0; };
+        if (in_size == 2) {
+            for (const void *ptr : {q->u, q->delta, q->B, q->C, (const void *)q->du, (const void *)q->ddelta})
+                if (odd(ptr)) return false;
+            for (int64_t st : {a.u_bs, a.u_ds, a.dl_bs, a.dl_ds, a.B_bs, a.B_gs, a.B_ns, a.C_bs, a.C_gs, a.C_ns})
+                if (st % 2 != 0) return false;
+            if (q->seqlen % 2 != 0) return false;
+        }
+        return dy_size == 4 || (!odd(q->dout) && a.do_bs % 2 == 0 && a.do_ds % 2 == 0 && q->seqlen % 2 == 0);
+    };
     if (a.N <= 8 * kStates && (int64_t)a.L * 4 < 0x7fffffff) {
         const bool one = a.N == 1;
         // Positions per lane (measured with the others, us): 8 where rows are long, as the wavefront scans are paid per pass
@@ -875,8 +924,8 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
         // with 1: 166) and with several states, whose B, C and sums fill the registers; 1 for rows that fit 64 lanes
         // (768 x 7 x 7: 70; with 4: 144).
         const int items = a.L <= kWave ? 1 : a.L <= 4 * kWave || !one ? 4 : 8;
-        const bool vec = groups_ok(items);
-        const int kI = items == 8 && !vec ? 4 : items;           // element by element, 4 at a time are enough in flight
+        const bool vec = dwords_ok(items);
+        const int kI = items;
         const int n_pass = (a.L + kWave * kI - 1) / (kWave * kI);
         const int n_waves = one ? kWavesPerWg : (a.N + kStates - 1) / kStates;
         // Channels per workgroup: more of them mean fewer atomics on dB / dC (one per entry and workgroup), fewer mean more
@@ -911,10 +960,11 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
     } while (0)
 #define SS2D_BWD_ITEMS(IN, DY)                                                                                                  \
     do {                                                                                                                        \
-        if (kI == 8) SS2D_BWD_LAUNCH(IN, DY, 8, true);                                                                          \
+        if (kI == 8 && vec) SS2D_BWD_LAUNCH(IN, DY, 8, true);                                                                   \
+        else if (kI == 8) SS2D_BWD_LAUNCH(IN, DY, 8, sizeof(IN) == 4);                                                              \
         else if (kI == 1) SS2D_BWD_LAUNCH(IN, DY, 1, true);                                                                     \
-        else if (vec && items == 4) SS2D_BWD_LAUNCH(IN, DY, 4, true);                                                           \
-        else SS2D_BWD_LAUNCH(IN, DY, 4, false);                                                                                 \
+        else if (vec) SS2D_BWD_LAUNCH(IN, DY, 4, true);                                                                         \
+        else SS2D_BWD_LAUNCH(IN, DY, 4, sizeof(IN) == 4);                                                                                 \
     } while (0)
             if (q->in_dtype == SS2D_F32) SS2D_BWD_ITEMS(float, float);
             else if (q->in_dtype == SS2D_BF16) { if (q->dout_dtype == SS2D_F32) SS2D_BWD_ITEMS(bf16_t, float); else SS2D_BWD_ITEMS(bf16_t, bf16_t); }
