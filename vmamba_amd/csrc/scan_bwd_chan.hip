@@ -468,10 +468,10 @@ static int bwd_chan_segments(int L, int N, int size, int32_t &seg_len) {
 
 // Where a channel per lane is ahead of positions in lanes (scan_bwd_states_kernel).  That one works in passes of 256 positions, and a few
 // images of one or two passes are done before two more kernels have been launched here; many of them or longer rows fill the chip either way,
-// and this kernel has half the instructions per (position, state).  us, positions / channels in lanes, wavefronts of whole rows in front, bf16: 16 states, 12: 196 positions 22 / 46,
-// 400 46 / 57, 576 66 / 59, 3136 200 / 55; 192: 56 29 / 26, 196 41 / 48, 400 72 / 67, 784 135 / 96; 768: 56 78 / 28, 196 108 / 66, 784 411 / 228; 8 states, 1536: 196 102 / 95, 255
-// 115 / 127; 512 of two wavefronts per workgroup (32 channels), in fp32: 130 86 / 89, 1225 396 / 421.  Of 4 states a lane has one, and the work per position is as much as that per state: 192: 784 73 / 49;
-// 768: 56 29 / 18, 196 41 / 46, 784 131 / 133; 1536: 784 226 / 269.
+// and this kernel has half the instructions per (position, state).  us, positions / channels in lanes, wavefronts of whole rows in front, bf16: 16 states, 12: 196 positions 20 / 44,
+// 400 36 / 46, 576 51 / 46, 3136 202 / 65; 192: 56 31 / 25, 196 44 / 48, 400 74 / 70, 784 140 / 110; 768: 56 76 / 27, 196 109 / 83, 784 422 / 224; 8 states, 1536: 196 99 / 87, 255
+// 110 / 106; 512 of two wavefronts per workgroup (32 channels), in fp32: 130 48 / 45, 1225 209 / 227.  Of 4 states a lane has one, and the work per position is as much as that per state: 192: 784 73 / 51;
+// 768: 56 28 / 17, 196 41 / 46, 784 132 / 133; 1536: 400 114 / 127.
 static bool bwd_chan_pays(const ScanBwdArgs &a) {
     const int64_t units = (int64_t)a.batch * (a.dim / a.dim_per_group) * ((a.dim_per_group + kBcChan - 1) / kBcChan);
     if (a.N == 4) return a.L > 256 ? units <= 192 : a.L <= 96 && units >= 512;

@@ -419,9 +419,9 @@ __global__ __launch_bounds__(kBlock) void scan_chan_carry_kernel(const float *__
 }
 
 // Rows of whole 16-byte pieces and 8 positions are this kernel's at any size.  Others would take the kernels with positions in lanes, whose 16 states
-// of odd rows (49 positions, 64 x 96 maps in bf16: 191 us, here 24; 225: 281 / 55; 3306, 16 x 192: 1369 / 263) and larger calls of 4, 8 and 32 are far behind;
-// left to them are few wavefronts, each alone with its row: 4 states, 12 of them, 225 positions 9.0 / 12.4, 3306 21 / 24; 8 states, 225 14.2 / 15.4; 32 in
-// single precision 37 / 41; single precision of an odd number of fours, which they read in whole pieces: 4 states, 192: 1764 positions 34 / 55, 768: 90 / 83.
+// of odd rows (64 x 96 maps in bf16, before, and as they are now: 49 positions 93 / 81 us, here 12.5; 225 182 / 87, 37; 16 x 192 of 3306 1390 / 323, 266) and larger calls of 4, 8 and 32 are far behind;
+// left to them are few wavefronts, each alone with its row: 4 states, 12 of them, 225 positions 5.7 / 13.5, 3306 10.9 / 22.9; 8 states, 225 7.9 / 16.6; 32 in
+// single precision 18.5 / 34.3; single precision of an odd number of fours, which they read in whole pieces: 4 states, 192: 1764 positions 24.9 / 40.0, 768: 86.6 / 81.9.
 static bool chan_pays(const ScanArgs &a, bool vec, int in_size) {
     if (vec && a.L % 8 == 0) return true;
     const int64_t units = (int64_t)a.batch * (a.dim / a.dim_per_group) * ((a.dim_per_group + kChanBlock - 1) / kChanBlock);

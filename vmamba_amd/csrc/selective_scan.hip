@@ -15,8 +15,8 @@
 //                2048-position chunk of one row and exchange their totals through LDS.
 //
 // I/O is 16-byte vectors per lane whenever pointers, strides and the row length allow
-// (kVec); otherwise whole dwords from a base rounded down to one (RowReader; one state, 4096 rows of 3249 positions in fp16: 107 us element by
-// element, 35 so).  Positions past the end of a row are fed
+// (kVec); otherwise whole dwords from a base rounded down to one (RowReader; one state, 4096 rows of 3249 positions in fp16: 111 us element by
+// element, 29 so).  Positions past the end of a row are fed
 // as dl = 0, u = 0, i.e. the identity pair (1, 0), so the state at the end of the last pass is
 // the state at the last real position.
 #include "scan_common.h"
@@ -619,7 +619,6 @@ static bool span_fits_u32(const ScanArgs &a, int64_t elem_bytes) {
 // per channel, rows of at least one lane vector, and dstate 1 or 16.
 static bool flat_eligible(const ScanArgs &a, const ss2d_scan_params *q) {
     const int64_t L = a.L, KD = a.dim;
-    // (many rows of four passes and more keep this kernel's id; dispatch_vec)
     const bool length_ok = L < 4 * kPass || (L <= (1 << 24) && a.N == 1 && a.rows >= 6144);
     return L >= kItems && length_ok && (a.N == 1 || a.N == 16) && q->delta_dim == q->dim &&
            a.u_ds == L && a.dl_ds == L && a.o_ds == L && a.u_bs == KD * L && a.dl_bs == KD * L && a.o_bs == KD * L &&
@@ -629,14 +628,21 @@ static bool flat_eligible(const ScanArgs &a, const ss2d_scan_params *q) {
 
 static int flat_granularity(const ScanArgs &a, int64_t elem_bytes);
 
-// Several rows to a wavefront, or one.  A wavefront of the flat kernel walks eight rows or more behind one another, so few rows leave the
-// chip idle: a wavefront per row is ahead at any length (one state, us, flat / row; 192 rows: 56 positions 13.4 / 4.4, 225 21 / 5.5, 1353 34 / 5.7;
-// 3072: 56 11.6 / 4.0, 225 20 / 6.9, 576 16 / 8.3, 1353 44 / 14).  Many rows: a pass of the flat kernel costs about 1.4x a pass of the row kernel with
+// Rows that the row kernel reads off the 16-byte grid or with more than 30 % of its lanes idle.
+static bool flat_class(const ScanArgs &a, bool vec) {
+    return !vec || 10 * (int64_t)a.L < 7 * (((int64_t)a.L + kPass - 1) / kPass * kPass);
+}
+
+// Several of those to a wavefront, or one.  A wavefront of the flat kernel walks eight rows or more behind one another, so few rows leave the
+// chip idle: a wavefront per row is ahead at any length (one state in bf16, us, flat / row; 192 rows: 56 positions 10.6 / 3.7, 225 20.4 / 4.7, 1353 36.4 / 6.0;
+// 3072: 56 11.6 / 4.0, 225 21.0 / 7.1, 576 11.5 / 5.7, 1353 37.5 / 11.3).  Many rows: a pass of the flat kernel costs about 1.4x a pass of the row kernel with
 // groups of two elements or more, and more with single ones, so it is ahead where the row kernel would leave more than 30 % of its lanes idle
-// (12 288 rows: 601 of 1024 positions 42 / 32 with single elements; 24 576: 418 of 512 in pairs 44 / 50, 601 72 / 77, 1003 124 / 104,
-// 1353 176 / 138) and, reading pairs or fours, on rows that are no whole 16-byte pieces (24 576 of 484: 38 / 46).
+// (12 288 rows: 601 of 1024 positions 29.7 / 23.2 with single elements; 24 576: 418 of 512 in pairs 31.0 / 35.9, 601 40.4 / 42.1, 1003 61.2 / 52.2,
+// 1353 81.0 / 63.9) and, reading pairs or fours, on rows that are no whole 16-byte pieces (24 576 of 484: 30.7 / 37.3).
+// Long ones are a wavefront's each: eight to a wavefront as one stream gather B and C element by element (before and now: 6144 rows of 2051 positions 62.9 / 30.4,
+// 24 576 118 / 107, 24 576 of 5625 389 / 262).
 static bool flat_pays(const ScanArgs &a, bool vec, int in_size) {
-    if (a.L >= 4 * kPass) return !vec;                     // long rows off the 16-byte grid: dispatch_vec
+    if (a.L >= 4 * kPass) return false;
     const bool half_full = 10 * (int64_t)a.L < 7 * (((int64_t)a.L + kPass - 1) / kPass * kPass);
     if (a.rows <= 8192 || (vec && in_size == 2 && a.L <= 336 && a.rows <= 12288)) return false;
     if (vec) return half_full;
@@ -736,9 +742,7 @@ static int launch_scan(const ScanArgs &a, bool split_rows, hipStream_t stream) {
 
 template <typename in_t, typename out_t>
 static int dispatch_vec(const ScanArgs &a, bool vec, int kernel, hipStream_t stream) {
-    // long rows under the flat kernel's id are a wavefront's each all the same: eight to a wavefront as one stream gather B and C element by
-    // element (one state, us, stream / row: 6144 rows of 2051 positions in bf16 64 / 31, 24 576 119 / 108, 24 576 of 5625 389 / 267; in fp32 227 / 142, 585 / 371)
-    if (kernel == SS2D_SCAN_KERNEL_FLAT && a.L < 4 * kPass) return launch_flat<in_t, out_t>(a, stream);
+    if (kernel == SS2D_SCAN_KERNEL_FLAT && flat_pays(a, vec, (int)sizeof(in_t))) return launch_flat<in_t, out_t>(a, stream);
     const bool split_rows = kernel == SS2D_SCAN_KERNEL_ROW4;
     return vec ? launch_scan<in_t, out_t, true>(a, split_rows, stream) : launch_scan<in_t, out_t, false>(a, split_rows, stream);
 }
@@ -798,7 +802,7 @@ static int plan_scan(const ss2d_scan_params *q, ScanArgs &a, bool &vec) {
     if (scan_small_eligible(a, q->in_dtype, q->u, q->delta, q->out)) return SS2D_SCAN_KERNEL_SMALL;
     // several states per channel and enough channels per group to fill wavefronts: one channel per lane
     if (scan_chan_eligible(a, vec, (int)in_bytes)) return SS2D_SCAN_KERNEL_CHAN;
-    if (flat_eligible(a, q) && flat_pays(a, vec, (int)in_bytes)) return SS2D_SCAN_KERNEL_FLAT;
+    if (flat_eligible(a, q) && flat_class(a, vec)) return SS2D_SCAN_KERNEL_FLAT;
     // few long rows: every row split over the four wavefronts of a workgroup (3072 rows and more: a wavefront per row is faster)
     if (a.L > SS2D_SCAN_CHUNK && a.rows < 2048) return SS2D_SCAN_KERNEL_ROW4;
     return SS2D_SCAN_KERNEL_ROW;
