@@ -177,6 +177,16 @@ def core_workspace_bytes(B, D, H, W, dtype=torch.bfloat16):
     return _lib.lib().ss2d_core_workspace_bytes(p)
 
 
+# Tiles of 8, 16, 24, 32 and 40 positions at the edges (runs of 1, 2, 4 and 8 lanes), on either side and on both, in one row or column of tiles too.
+TILED_EDGES = [(1, 3, 136, 144), (2, 2, 152, 136), (1, 2, 160, 168), (1, 1, 8, 1680), (1, 1, 1672, 24), (1, 2, 40, 392), (1, 1, 144, 152)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", TILED_EDGES, ids=lambda s: "x".join(map(str, s)))
+def test_core_tiles_at_the_edges(shape, dtype):
+    test_core_large_maps_in_tiles_match_oracle_composition(shape, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("shape", TILED_SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_core_large_maps_in_tiles_match_oracle_composition(shape, dtype):

@@ -22,7 +22,11 @@
 //
 // A run of 64 positions occupies 8 lanes (half a DPP row).  The lane-local scan of 8 items is followed by a scan over
 // the 8 lanes with DPP row shifts; the run's first lane (in the direction's order) takes the carry in and passes on a
-// decay of zero, which also stops anything from the other run that shares its DPP row.
+// decay of zero, which also stops anything from the other runs that share its DPP row.
+//
+// The tiles at a map's right and lower edges are often far smaller than 64 x 64 (144 = 64 + 64 + 16).  The runs across such a side take 4, 2 or 1
+// lanes, and as many more of them go into a pass; passes without lines are not computed: a 16 x 64 tile has 4 passes instead of 16.
+// (Two passes per wavefront of 8-lane runs whatever the tile: 4 x 192 maps of 136 x 136 207 us for the call, so 183; 16 x 48 of 224 x 224 543 and 532.)
 // Semantics: as ss2d_core_fwd (classification/models/vmamba.py:604, 625-633, 638; cross_merge_fwd's pairing,
 // classification/models/csm_triton.py:56-62).
 #include <type_traits>
@@ -67,19 +71,13 @@ __device__ __forceinline__ float run_scan(float a, float &h) {
     return hx;
 }
 
-// Product of v over the 8 lanes of a run, delivered in the run's last lane in scan order.
+// Product of v over the 2^log_lanes lanes of a run (uniform), delivered in the run's last lane in scan order.
 template <bool kReverse>
-__device__ __forceinline__ float run_product(float v) {
-    if constexpr (!kReverse) {
-        v *= dpp_move<kDppRowShr1>(1.0f, v);
-        v *= dpp_move<kDppRowShr2>(1.0f, v);
-        v *= dpp_move<kDppRowShr4>(1.0f, v);
-    } else {
-        constexpr int kShl1 = 0x101, kShl2 = 0x102, kShl4 = 0x104;
-        v *= dpp_move<kShl1>(1.0f, v);
-        v *= dpp_move<kShl2>(1.0f, v);
-        v *= dpp_move<kShl4>(1.0f, v);
-    }
+__device__ __forceinline__ float run_product(float v, int log_lanes) {
+    constexpr int kShl1 = 0x101, kShl2 = 0x102, kShl4 = 0x104;
+    if (log_lanes > 0) v *= dpp_move<kReverse ? kShl1 : kDppRowShr1>(1.0f, v);
+    if (log_lanes > 1) v *= dpp_move<kReverse ? kShl2 : kDppRowShr2>(1.0f, v);
+    if (log_lanes > 2) v *= dpp_move<kReverse ? kShl4 : kDppRowShr4>(1.0f, v);
     return v;
 }
 
@@ -91,26 +89,39 @@ struct TilePassLoads {
     uint32_t u[kCol ? 8 : 4];              // column runs: one 16-bit value per register, as gathered
     float carry[kOut ? 2 : 1];
     int32_t run, p;                        // run index of the pair's forward direction; first stream position of the lane
+    int32_t line;                          // of the tile
     bool valid, line_ok;
 };
 
-template <typename in_t, bool kSoftplus, bool kOut>
+// kEdges: a side of the map is no multiple of 64.
+template <typename in_t, bool kSoftplus, bool kOut, bool kEdges>
 __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, const TiledGeom g, float2 *__restrict__ agg,
                                                             const float *__restrict__ carry) {
     static_assert(sizeof(in_t) == 2, "16-bit streams");
     __shared__ float s_plane[kOut ? kTile * kTilePitch : 1];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    // neighbours in the grid are the channels of one tile of one image: they read the same B / C pieces, so each XCD
-    // (one L2) gets a contiguous range of them
+    // Each XCD (one L2) gets a contiguous range of the grid.  Neighbours in it are the channels of one tile, which read the same B / C pieces; where the sides
+    // are no multiples of 64 the tiles of one map: their runs end inside 128-byte lines whose rest is the next tile's (2 x 736 maps of 144 x 144, passes A and B:
+    // channels 189 + 241 us, tiles 129 + 173; 4 x 192 of 136 x 136, whole call: 230, 183; 4 x 96 of 256 x 256 277, 279).
     const uint32_t wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
-    uint32_t bt, d, b, tile, tr, tc;
-    divmod(wg, g.div_D, bt, d);
-    divmod(bt, g.div_tiles, b, tile);
+    uint32_t plane, d, b, tile, tr, tc;
+    if constexpr (kEdges) {
+        divmod(wg, g.div_tiles, plane, tile);
+        divmod(plane, g.div_D, b, d);
+    } else {
+        divmod(wg, g.div_D, plane, d);
+        divmod(plane, g.div_tiles, b, tile);
+    }
     divmod(tile, g.div_ntc, tr, tc);
     const int H = p.H, W = p.W, L = p.L;
     const int h0 = (int)tr * kTile, w0 = (int)tc * kTile;
-    const int seg = lane & 7, sub = lane >> 3;               // piece of the run; run of the pass
+    // lanes of a run (log2) down the tile's columns and along its rows
+    auto lanes_of = [](int positions) { return positions > 32 ? 3 : positions > 16 ? 2 : positions > 8 ? 1 : 0; };
+    const int lg_col = kEdges ? lanes_of(H - h0) : 3, lg_row = kEdges ? lanes_of(W - w0) : 3;
+    // pass j of a wavefront: its first line; none of the map's (uniform): not computed
+    auto first_line = [&](int lg, int j) { return kEdges ? (j * kWavesPerWg + wave) << (6 - lg) : 8 * (2 * wave + j); };
+    auto pass_pays = [&](int lg, int j, int lines) { return !kEdges || first_line(lg, j) < min(lines, kTile); };
     const in_t *x_map = reinterpret_cast<const in_t *>(p.x) + ((int64_t)b * p.D + d) * L;
     const in_t *dl_bd = reinterpret_cast<const in_t *>(p.delta) + (int64_t)d * p.dl_ds + (int64_t)b * p.dl_bs;
     const in_t *B_b = reinterpret_cast<const in_t *>(p.Bm) + (int64_t)b * p.B_bs;
@@ -125,10 +136,12 @@ __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, co
         bias[k] = p.bias ? p.bias[k * p.D + (int)d] : 0.0f;
     }
 
-    // ---- one pass: 8 runs of the tile (rows h0 + line, or columns w0 + line), 8 positions per lane -------------------
+    // ---- one pass: 8 runs of the tile or more (rows h0 + line, or columns w0 + line), 8 positions per lane -------------------
     auto issue = [&](auto col_tag, int pass, auto &r) {
         constexpr bool kCol = decltype(col_tag)::value;
-        const int line = wave * 16 + pass * 8 + sub;
+        const int lg = kCol ? lg_col : lg_row, seg = lane & ((1 << lg) - 1);
+        const int line = first_line(lg, pass) + (lane >> lg);
+        r.line = line;
         const int n_lines = kCol ? W : H, n_along = kCol ? H : W;
         const int line_abs = (kCol ? w0 : h0) + line, along = (kCol ? h0 : w0) + 8 * seg;
         r.line_ok = line < kTile && line_abs < n_lines;
@@ -160,7 +173,7 @@ __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, co
 
     // One direction of a pass.  Items j = 0..7 are in the direction's order; position index i = j forwards, 7 - j
     // backwards.  kOut: acc[i] (by position) receives C * h; else the run's aggregate goes to agg.
-    auto direction = [&](auto rev_tag, auto first_tag, int k, const uint4 &dl_raw, const uint4 &b_raw, const uint4 &c_raw,
+    auto direction = [&](auto rev_tag, auto first_tag, int k, const uint4 &dl_raw, const uint4 &b_raw, const uint4 &c_raw, int lg,
                          const float (&uf)[kItems], float carry_in, bool valid, bool line_ok, int run, float (&acc)[kItems]) {
         constexpr bool kRev = decltype(rev_tag)::value, kFirstOfPair = decltype(first_tag)::value;
         const uint32_t dw[4] = {dl_raw.x, dl_raw.y, dl_raw.z, dl_raw.w}, bw[4] = {b_raw.x, b_raw.y, b_raw.z, b_raw.w};
@@ -179,7 +192,8 @@ __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, co
         }
         // lanes without positions are the identity; the run's first lane takes the carry in and cuts the chain
         const float a_lane = valid ? ac[kItems - 1] : 1.0f, h_lane = valid ? hh[kItems - 1] : 0.0f;
-        const bool first = kRev ? seg == 7 : seg == 0;
+        const int ends = (1 << lg) - 1, seg = lane & ends;
+        const bool first = seg == (kRev ? ends : 0);
         const float c_in = kOut ? carry_in : 0.0f;
         float h_run = first ? fmaf(a_lane, c_in, h_lane) : h_lane;
         const float h_before = run_scan<kRev>(first ? 0.0f : a_lane, h_run);
@@ -194,8 +208,8 @@ __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, co
                 acc[i] = kFirstOfPair ? Cv * h : fmaf(Cv, h, acc[i]);
             }
         } else {
-            const float prod = run_product<kRev>(a_lane);
-            const bool last = kRev ? seg == 0 : seg == 7;
+            const float prod = run_product<kRev>(a_lane, lg);
+            const bool last = seg == (kRev ? 0 : ends);
             if (last && line_ok) agg[(k * BD + bd) * g.nr_max + run] = make_float2(prod, h_run);
         }
     };
@@ -203,6 +217,7 @@ __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, co
     auto compute = [&](auto col_tag, const auto &r, float (&acc)[kItems], float (&uf)[kItems]) {
         constexpr bool kCol = decltype(col_tag)::value;
         constexpr int kf = kCol ? 1 : 0, kb = kf + 2;
+        const int lg = kCol ? lg_col : lg_row;
         if constexpr (kCol) {
 #pragma unroll
             for (int i = 0; i < kItems; ++i) uf[i] = to_f32(in_t{(uint16_t)r.u[i]});
@@ -210,8 +225,8 @@ __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, co
 #pragma unroll
             for (int i = 0; i < kItems; ++i) uf[i] = (i & 1) ? unpack_hi<in_t>(r.u[i / 2]) : unpack_lo<in_t>(r.u[i / 2]);
         }
-        direction(std::false_type{}, std::true_type{}, kf, r.dl[0], r.bq[0], r.cq[0], uf, r.carry[0], r.valid, r.line_ok, r.run, acc);
-        direction(std::true_type{}, std::false_type{}, kb, r.dl[1], r.bq[1], r.cq[kOut ? 1 : 0], uf, r.carry[kOut ? 1 : 0], r.valid,
+        direction(std::false_type{}, std::true_type{}, kf, r.dl[0], r.bq[0], r.cq[0], lg, uf, r.carry[0], r.valid, r.line_ok, r.run, acc);
+        direction(std::true_type{}, std::false_type{}, kb, r.dl[1], r.bq[1], r.cq[kOut ? 1 : 0], lg, uf, r.carry[kOut ? 1 : 0], r.valid,
                   r.line_ok, r.run, acc);
     };
 
@@ -225,9 +240,10 @@ __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, co
 
     // ---- column runs: directions 1 + 3; the sums go into the transposition tile, [column][row] ---------------------
     auto column_pass = [&](int pass, const ColLoads &r) {
+        if (!pass_pays(lg_col, pass, W - w0)) return;
         compute(std::true_type{}, r, acc, uf);
         if constexpr (kOut) {
-            float *dst = s_plane + (wave * 16 + pass * 8 + sub) * kTilePitch + 8 * seg;
+            float *dst = s_plane + r.line * kTilePitch + 8 * (lane & ((1 << lg_col) - 1));
 #pragma unroll
             for (int i = 0; i < kItems; ++i) dst[i] = acc[i];
         }
@@ -242,10 +258,10 @@ __global__ __launch_bounds__(kBlock) void core_tiled_kernel(const CoreArgs p, co
     float Dsum = 0.0f;
     if (kOut && p.Dv) Dsum = (p.Dv[d] + p.Dv[2 * p.D + (int)d]) + (p.Dv[p.D + (int)d] + p.Dv[3 * p.D + (int)d]);
     auto row_pass = [&](int pass, const RowLoads &r) {
+        if (!pass_pays(lg_row, pass, H - h0)) return;
         compute(std::false_type{}, r, acc, uf);
         if constexpr (kOut) {
-            const int line = wave * 16 + pass * 8 + sub;
-            const float *src = s_plane + (8 * seg) * kTilePitch + line;
+            const float *src = s_plane + 8 * (lane & ((1 << lg_row) - 1)) * kTilePitch + r.line;
             float o[kItems];
 #pragma unroll
             for (int i = 0; i < kItems; ++i) {
@@ -352,12 +368,16 @@ static int launch_core_tiled_typed(const CoreArgs &a, void *workspace, hipStream
     float *carry = reinterpret_cast<float *>(agg + rows * g.nr_max);
     const uint32_t n_wg = (uint32_t)((int64_t)a.B * a.D * g.ntr * g.ntc);
     const uint32_t carry_wg = (uint32_t)rows;                // one workgroup per (direction, image, channel)
-#define SS2D_TILED_LAUNCH(SP)                                                                                                      \
-    hipLaunchKernelGGL((core_tiled_kernel<in_t, SP, false>), dim3(n_wg), dim3(kBlock), 0, stream, a, g, agg, (const float *)carry); \
+#define SS2D_TILED_LAUNCH(SP, E)                                                                                                   \
+    hipLaunchKernelGGL((core_tiled_kernel<in_t, SP, false, E>), dim3(n_wg), dim3(kBlock), 0, stream, a, g, agg, (const float *)carry); \
     hipLaunchKernelGGL(core_carry_kernel, dim3(carry_wg), dim3(kBlock), 0, stream, (const float2 *)agg, carry, (int)rows,           \
                        a.B * a.D, g.nr02, g.nr13, g.nr_max);                                                                        \
-    hipLaunchKernelGGL((core_tiled_kernel<in_t, SP, true>), dim3(n_wg), dim3(kBlock), 0, stream, a, g, agg, (const float *)carry)
-    if (a.softplus) { SS2D_TILED_LAUNCH(true); } else { SS2D_TILED_LAUNCH(false); }
+    hipLaunchKernelGGL((core_tiled_kernel<in_t, SP, true, E>), dim3(n_wg), dim3(kBlock), 0, stream, a, g, agg, (const float *)carry)
+    if (a.H % kTile != 0 || a.W % kTile != 0) {
+        if (a.softplus) { SS2D_TILED_LAUNCH(true, true); } else { SS2D_TILED_LAUNCH(false, true); }
+    } else {
+        if (a.softplus) { SS2D_TILED_LAUNCH(true, false); } else { SS2D_TILED_LAUNCH(false, false); }
+    }
 #undef SS2D_TILED_LAUNCH
     return launch_status();
 }
