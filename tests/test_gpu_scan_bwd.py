@@ -227,3 +227,62 @@ def test_cleared_accumulators_and_rounded_pair():
                                _lib.SS2D_BF16 if dtype == torch.bfloat16 else _lib.SS2D_F16) == _lib.SS2D_OK
             assert torch.equal(x[:n0], a.to(dtype)) and torch.equal(y[:n1], b[:n1].to(dtype))
             assert bool((x[n0:] == 7).all()) and bool((y[n1:] == 7).all())
+
+
+class _Watching(torch.overrides.TorchFunctionMode):
+    """Sees the operators that are called: the Python route makes the tensors."""
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def _same(got, want):
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        assert a is None or (a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride() and torch.equal(a, b))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,delta_dim,has_D,has_bias", [(1, 24, True, True), (16, 24, False, True), (2, 24, True, False), (1, 6, False, False)])
+def test_operators_made_in_the_extension_equal_those_made_from_python(N, delta_dim, has_D, has_bias, dtype):
+    """The three operators forwards and backwards on dense, strided and transposed tensors: the same bits, sizes, strides and types.   (dA, dB, dC and the
+    two vectors are sums of atomics over few positions: one wavefront's order.)"""
+    from vmamba_amd.csms6s import selective_scan_bwd, selective_scan_fwd
+    g = torch.Generator().manual_seed(71)
+    rand = lambda *s: torch.randn(*s, generator=g).to("cuda", dtype)
+    u, B, C, dout = rand(2, 30, 60)[:, 3:27, 8:58], rand(2, 4, N, 50), rand(2, 4, N + 1, 50)[:, :, :N], rand(2, 24, 50)
+    delta, A = rand(2, delta_dim, 50) * 0.3, -torch.rand(24, N, generator=g).cuda()
+    D, bias = (torch.rand(24, generator=g).cuda() if has_D else None), (torch.rand(delta_dim, generator=g).cuda() if has_bias else None)
+    x, ys = rand(2, 6, 5, 10), rand(2, 4, 6, 5, 10)
+    calls = [lambda: selective_scan_fwd(u, delta, A, B, C, D, bias, True, 1, True, True), lambda: selective_scan_fwd(u, delta, A, B, C, D, bias, False, 1, False, False),
+             lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True)[:2], lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout.float(), None, False)[:2],
+             lambda: [va.cross_scan_fn(x)], lambda: [va.cross_scan_fn(x.transpose(2, 3))], lambda: [va.cross_merge_fn(ys)], lambda: [va.cross_merge_fn(ys.transpose(3, 4))]]
+    for call in calls:
+        got = call()
+        with _Watching():
+            _same(got, call())
+    sums = lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True)[2:]
+    got = sums()
+    with _Watching():
+        want = sums()
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None) and (a is None or (a.dtype == b.dtype and a.shape == b.shape and torch.allclose(a.float(), b.float(), rtol=2e-2, atol=1e-4 * b.abs().max().item())))
+
+
+def test_operators_made_in_the_extension_refuse_what_python_refuses():
+    from vmamba_amd.csms6s import selective_scan_bwd, selective_scan_fwd
+    u, A, B = torch.zeros(1, 8, 16, device="cuda"), torch.zeros(8, 1, device="cuda"), torch.zeros(1, 2, 1, 16, device="cuda")
+    bad = [(u, u[:, :, :15], A, B, B), (u, u.half(), A, B, B), (u, u, A.half(), B, B), (u, u, A, B[:, :, :, ::2], B), (u.transpose(1, 2), u, A, B, B), (u, u, A, B, B.cpu()),
+           (u, u, A, B, B, torch.zeros(7, device="cuda")), (u, u, A, B, B, None, torch.zeros(8, device="cuda", dtype=torch.half))]
+    for args in bad:
+        args = args + (None,) * (7 - len(args))
+        with pytest.raises(RuntimeError):
+            selective_scan_fwd(*args, True)
+        with pytest.raises(RuntimeError):
+            selective_scan_bwd(*args, u, None, True)
+    with pytest.raises(RuntimeError):
+        selective_scan_bwd(u, u, A, B, B, None, None, u.half()[:, :, :8], None, True)
+    with pytest.raises(ValueError):
+        va.cross_scan_fn(u)
+    with pytest.raises(TypeError):
+        va.cross_merge_fn(torch.zeros(1, 4, 2, 3, 3, device="cuda", dtype=torch.float64))

@@ -279,6 +279,13 @@ def launch(tensor, fn, *args):
         return fn(*args, torch._C._cuda_getCurrentRawStream(index))
 
 
+def result(value, what):
+    """What a function of host() has made, or its status raised."""
+    if type(value) is int:
+        check(value, what)
+    return value
+
+
 def strerror(code):
     return lib().ss2d_strerror(int(code)).decode()
 

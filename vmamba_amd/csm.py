@@ -13,7 +13,7 @@ supported with the same two kernels.
 import torch
 
 from . import _lib
-from .norm import memory_readable
+from .norm import TENSOR_KINDS, memory_readable, native_stands
 
 _DTYPE_CODE = {torch.float32: _lib.SS2D_F32, torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 
@@ -116,6 +116,10 @@ def cross_merge_flex_hip(y, in_channel_first=True, out_channel_first=True, one_b
 
 def cross_scan_hip(x):
     """x (B,C,H,W) -> (B,4,C,H*W), any 1/2/4/8-byte dtype, bit-exact permutation."""
+    if native_stands(x):
+        y = _lib.host().cross_scan(TENSOR_KINDS, x)
+        if y is not None:
+            return _lib.result(y, "ss2d_cross_scan")
     _require_gpu(x, "cross_scan")
     if x.dim() != 4:
         raise ValueError(f"cross_scan expects (B,C,H,W), got {tuple(x.shape)}")
@@ -151,6 +155,10 @@ def cross_scan_1b1_hip(x, out=None):
 
 def cross_merge_hip(ys, order=_lib.MERGE_PAIRWISE):
     """ys (B,4,C,H,W) -> (B,C,H*W); adds rounded to ys.dtype in the order of cross_merge_fwd."""
+    if order == _lib.MERGE_PAIRWISE and native_stands(ys):
+        out = _lib.host().cross_merge(TENSOR_KINDS, ys)
+        if out is not None:
+            return _lib.result(out, "ss2d_cross_merge")
     _require_gpu(ys, "cross_merge")
     if ys.dim() != 5 or ys.shape[1] != 4:
         raise ValueError(f"cross_merge expects (B,4,C,H,W), got {tuple(ys.shape)}")

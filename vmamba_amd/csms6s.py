@@ -13,6 +13,7 @@ import ctypes
 import torch
 
 from . import _lib
+from .norm import TENSOR_KINDS, native_stands
 
 _DTYPE_CODE = {torch.float32: _lib.SS2D_F32, torch.bfloat16: _lib.SS2D_BF16, torch.float16: _lib.SS2D_F16}
 MAX_DSTATE = 256
@@ -60,6 +61,10 @@ def selective_scan_fwd(u, delta, A, B, C, D=None, delta_bias=None, delta_softplu
     holds the chunk-end states (None when ``want_x`` is False).  ``nrows`` is accepted and
     ignored, as in the reference (selective_scan_oflex.cpp:224-226).
     """
+    if native_stands(u):
+        native = _lib.host().scan_fwd(TENSOR_KINDS, u, delta, A, B, C, D, delta_bias, bool(delta_softplus), bool(out_float), bool(want_x))
+        if native is not None:
+            return _lib.result(native, "ss2d_selective_scan_fwd")
     _check(u.dtype in _DTYPE_CODE, f"selective_scan_fwd not implemented for input type '{u.dtype}'")
     _check(A.dtype == torch.float32, "A must be float32")
     _check(delta.dtype == u.dtype and B.dtype == u.dtype and C.dtype == u.dtype, "delta, B, C must have u's dtype")
@@ -137,6 +142,10 @@ def selective_scan_bwd(u, delta, A, B, C, D, delta_bias, dout, x=None, delta_sof
     """Python twin of ``selective_scan_cuda_oflex.bwd``: returns [du, ddelta, dA, dB, dC, dD, ddelta_bias]
     (selective_scan_oflex.cpp:233-355).  ``x`` (the forward's chunk states) and ``nrows`` are accepted and unused:
     the kernel recomputes the states it needs."""
+    if native_stands(u):
+        native = _lib.host().scan_bwd(TENSOR_KINDS, u, delta, A, B, C, D, delta_bias, dout, bool(delta_softplus))
+        if native is not None:
+            return _lib.result(native, "ss2d_selective_scan_bwd")
     _check(u.dtype in _DTYPE_CODE, f"selective_scan_bwd not implemented for input type '{u.dtype}'")
     _check(A.dtype == torch.float32, "A must be float32")
     _check(dout.dtype in (u.dtype, torch.float32), "dout must have u's dtype or be float32")

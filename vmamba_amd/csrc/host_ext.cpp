@@ -1,6 +1,7 @@
-// The host's share of forward_core and of a block of few positions, in C++: the checks of their tensors, the outputs and workspaces and
-// the one call into the C ABI.  Through ctypes and torch's Python interface that took 14 us of a forward_core whose three kernels
-// run for 18, and 20 us of a block; no kernel lives here, and what is checked is what the Python callers (core.py, block.py) checked.
+// The host's share of forward_core, of a block of few positions and of the three operators, in C++: the checks of their tensors, the outputs and
+// workspaces and the calls into the C ABI.  Through ctypes and torch's Python interface that took 14 us of a forward_core whose three kernels
+// run for 18, 20 us of a block, and most of what the three operators take on a few small maps (2 x 96 of 14 x 14: inference 38 us, so 24;
+// forward and backward 161, 98; with 16 states forward_core 113, 75).  No kernel lives here, and what is checked is what the Python callers (core.py, block.py, csm.py, csms6s.py) checked.
 #include <ATen/hip/HIPContext.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -146,7 +147,142 @@ static py::object block(const py::tuple &kinds, const py::object &x_in, const py
     return rc != SS2D_OK ? py::object(py::int_(rc)) : py::cast(out);
 }
 
+// The scan's tensors, forward and backward: the caller's, as far as a kernel may have their addresses.
+struct ScanTensors {
+    at::Tensor u, delta, A, B, C, D, bias;
+    int64_t batch, dim, L, N, groups, delta_dim;
+    int code;
+
+    // False for whatever csms6s.py refuses or has to look at itself.
+    bool read(const py::tuple &kinds, const py::object &u_in, const py::object &delta_in, const py::object &A_in, const py::object &B_in,
+              const py::object &C_in, const py::object &D_in, const py::object &bias_in) {
+        bool ok = true;
+        u = exactly(u_in, kinds, ok); delta = exactly(delta_in, kinds, ok); A = exactly(A_in, kinds, ok); B = exactly(B_in, kinds, ok);
+        C = exactly(C_in, kinds, ok); D = exactly(D_in, kinds, ok); bias = exactly(bias_in, kinds, ok);
+        if (!ok) return false;
+        for (const at::Tensor *t : {&u, &delta, &A, &B, &C})
+            if (!t->defined() || !plain(*t) || !on(*t, u) || t->numel() == 0) return false;
+        code = dtype_code(u.scalar_type());
+        if (code < 0 || u.dim() != 3 || delta.dim() != 3 || A.dim() != 2 || B.dim() != 4 || C.dim() != 4 || A.scalar_type() != at::kFloat) return false;
+        batch = u.size(0); dim = u.size(1); L = u.size(2); N = A.size(1); groups = B.size(1); delta_dim = delta.size(1);
+        for (const at::Tensor *t : {&u, &delta, &B, &C})
+            if (t->scalar_type() != u.scalar_type() || !(t->stride(-1) == 1 || t->size(-1) == 1)) return false;
+        if (dim % groups != 0 || dim % delta_dim != 0 || N > 256 || batch > INT32_MAX || dim > INT32_MAX || L > INT32_MAX) return false;
+        if (!has_shape(delta, {batch, delta_dim, L}) || !has_shape(A, {dim, N}) || !has_shape(B, {batch, groups, N, L}) || !has_shape(C, {batch, groups, N, L}))
+            return false;
+        if (D.defined() && (D.scalar_type() != at::kFloat || !on(D, u) || !plain(D) || !has_shape(D, {dim}) || !D.is_contiguous())) return false;
+        return !bias.defined() || (bias.scalar_type() == at::kFloat && on(bias, u) && plain(bias) && has_shape(bias, {delta_dim}) && bias.is_contiguous());
+    }
+
+    template <typename P> void describe(P &p, bool softplus) const {
+        p.batch = (int)batch; p.dim = (int)dim; p.seqlen = (int)L; p.dstate = (int)N; p.n_groups = (int)groups; p.delta_dim = (int)delta_dim;
+        p.in_dtype = code; p.delta_softplus = softplus ? 1 : 0;
+        p.u = u.data_ptr(); p.delta = delta.data_ptr(); p.A = A.data_ptr(); p.B = B.data_ptr(); p.C = C.data_ptr();
+        p.D = ptr_of(D); p.delta_bias = ptr_of(bias);
+        p.u_batch_stride = u.stride(0); p.u_d_stride = u.stride(1);
+        p.delta_batch_stride = delta.stride(0); p.delta_d_stride = delta.stride(1);
+        p.A_d_stride = A.stride(0); p.A_dstate_stride = A.stride(1);
+        p.B_batch_stride = B.stride(0); p.B_group_stride = B.stride(1); p.B_dstate_stride = B.stride(2);
+        p.C_batch_stride = C.stride(0); p.C_group_stride = C.stride(1); p.C_dstate_stride = C.stride(2);
+    }
+};
+
+// csms6s.py:selective_scan_fwd -- [out, x], None where its own checks have to speak, or the status of a failed call.
+static py::object scan_fwd(const py::tuple &kinds, const py::object &u, const py::object &delta, const py::object &A, const py::object &B, const py::object &C,
+                           const py::object &D, const py::object &bias, bool softplus, bool out_float, bool want_x) {
+    ScanTensors t;
+    if (!t.read(kinds, u, delta, A, B, C, D, bias)) return py::none();
+    const auto f32 = t.u.options().dtype(at::kFloat);
+    at::Tensor out = at::empty({t.batch, t.dim, t.L}, out_float ? f32 : t.u.options()), x;
+    if (want_x) x = at::empty({t.batch, t.dim, (t.L + SS2D_SCAN_CHUNK - 1) / SS2D_SCAN_CHUNK, 2 * t.N}, f32);
+    ss2d_scan_params p = {};
+    t.describe(p, softplus);
+    p.out_dtype = out_float ? SS2D_F32 : t.code;
+    p.out = out.data_ptr(); p.x = want_x ? x.data_ptr() : nullptr;
+    p.out_batch_stride = out.stride(0); p.out_d_stride = out.stride(1);
+    const int rc = enqueue(t.u, [&](void *stream) { return ss2d_selective_scan_fwd(&p, stream); });
+    if (rc != SS2D_OK) return py::int_(rc);
+    py::list result(2);
+    result[0] = py::cast(out);
+    result[1] = want_x ? py::cast(x) : py::none();
+    return result;
+}
+
+// csms6s.py:selective_scan_bwd, a delta row per channel -- the seven gradients (None for one that is not asked for), None or a status as above.
+static py::object scan_bwd(const py::tuple &kinds, const py::object &u, const py::object &delta, const py::object &A, const py::object &B, const py::object &C,
+                           const py::object &D, const py::object &bias, const py::object &dout_in, bool softplus) {
+    ScanTensors t;
+    bool ok = true;
+    const at::Tensor dout = exactly(dout_in, kinds, ok);
+    if (!ok || !dout.defined() || !t.read(kinds, u, delta, A, B, C, D, bias) || t.delta_dim != t.dim) return py::none();
+    if (!plain(dout) || !on(dout, t.u) || !has_shape(dout, {t.batch, t.dim, t.L}) || !(dout.stride(-1) == 1 || t.L == 1) ||
+        (dout.scalar_type() != t.u.scalar_type() && dout.scalar_type() != at::kFloat))
+        return py::none();
+    const auto f32 = t.u.options().dtype(at::kFloat);
+    at::Tensor du = at::empty({t.batch, t.dim, t.L}, t.u.options()), ddelta = at::empty({t.batch, t.dim, t.L}, t.u.options());
+    // sums, cleared in one launch
+    at::Tensor sums[5] = {at::empty({t.dim, t.N}, f32), at::empty({t.batch, t.groups, t.N, t.L}, f32), at::empty({t.batch, t.groups, t.N, t.L}, f32)};
+    if (t.D.defined()) sums[3] = at::empty({t.dim}, f32);
+    if (t.bias.defined()) sums[4] = at::empty({t.dim}, f32);
+    at::Tensor &dA = sums[0], dB = sums[1], dC = sums[2];
+    void *ptrs[5];
+    int64_t bytes[5];
+    int n = 0;
+    for (const at::Tensor &s : sums)
+        if (s.defined()) { ptrs[n] = s.data_ptr(); bytes[n++] = 4 * s.numel(); }
+    if (t.code != SS2D_F32) { dB = at::empty(sums[1].sizes(), t.u.options()); dC = at::empty(sums[2].sizes(), t.u.options()); }
+    ss2d_scan_bwd_params p = {};
+    t.describe(p, softplus);
+    p.dout_dtype = dtype_code(dout.scalar_type());
+    p.dout = dout.data_ptr(); p.dout_batch_stride = dout.stride(0); p.dout_d_stride = dout.stride(1);
+    p.du = du.data_ptr(); p.ddelta = ddelta.data_ptr(); p.dA = dA.data_ptr(); p.dB = sums[1].data_ptr(); p.dC = sums[2].data_ptr();
+    p.dD = sums[3].defined() ? sums[3].data_ptr() : nullptr;
+    p.ddelta_bias = sums[4].defined() ? sums[4].data_ptr() : nullptr;
+    const int rc = enqueue(t.u, [&](void *stream) {
+        int status = ss2d_clear(ptrs, bytes, n, stream);
+        if (status == SS2D_OK) status = ss2d_selective_scan_bwd(&p, stream);
+        if (status == SS2D_OK && t.code != SS2D_F32)
+            status = ss2d_round_pair((const float *)p.dB, dB.data_ptr(), dB.numel(), (const float *)p.dC, dC.data_ptr(), dC.numel(), t.code, stream);
+        return status;
+    });
+    if (rc != SS2D_OK) return py::int_(rc);
+    py::list result(7);
+    const at::Tensor grads[7] = {du, ddelta, dA, dB, dC, sums[3], sums[4]};
+    for (size_t i = 0; i < 7; ++i) result[i] = grads[i].defined() ? py::cast(grads[i]) : py::none();
+    return result;
+}
+
+// csm.py:cross_scan_hip and cross_merge_hip (pairwise): the result, None or a status as above.
+static py::object cross_scan(const py::tuple &kinds, const py::object &x_in) {
+    bool ok = true;
+    const at::Tensor x = exactly(x_in, kinds, ok);
+    if (!ok || !x.defined() || x.dim() != 4 || x.numel() == 0 || !x.is_cuda() || !plain(x) || !x.is_contiguous()) return py::none();
+    const int64_t B = x.size(0), C = x.size(1), H = x.size(2), W = x.size(3);
+    if (B > INT32_MAX || C > INT32_MAX || H > INT32_MAX || W > INT32_MAX) return py::none();
+    at::Tensor y = at::empty({B, 4, C, H * W}, x.options());
+    const int rc = enqueue(x, [&](void *stream) { return ss2d_cross_scan(x.data_ptr(), y.data_ptr(), (int)B, (int)C, (int)H, (int)W, (int)x.element_size(), stream); });
+    return rc != SS2D_OK ? py::object(py::int_(rc)) : py::cast(y);
+}
+
+static py::object cross_merge(const py::tuple &kinds, const py::object &y_in) {
+    bool ok = true;
+    const at::Tensor y = exactly(y_in, kinds, ok);
+    if (!ok || !y.defined() || y.dim() != 5 || y.numel() == 0 || y.size(1) != 4 || !y.is_cuda() || !plain(y) || !y.is_contiguous()) return py::none();
+    const int64_t B = y.size(0), C = y.size(2), H = y.size(3), W = y.size(4);
+    const int code = dtype_code(y.scalar_type());
+    if (code < 0 || B > INT32_MAX || C > INT32_MAX || H > INT32_MAX || W > INT32_MAX) return py::none();
+    at::Tensor out = at::empty({B, C, H * W}, y.options());
+    const int rc = enqueue(y, [&](void *stream) {
+        return ss2d_cross_merge(y.data_ptr(), out.data_ptr(), (int)B, (int)C, (int)H, (int)W, code, SS2D_MERGE_PAIRWISE, stream);
+    });
+    return rc != SS2D_OK ? py::object(py::int_(rc)) : py::cast(out);
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("forward_core", &forward_core);
     m.def("block", &block);
+    m.def("scan_fwd", &scan_fwd);
+    m.def("scan_bwd", &scan_bwd);
+    m.def("cross_scan", &cross_scan);
+    m.def("cross_merge", &cross_merge);
 }

@@ -245,6 +245,11 @@ def operators_seen():
     return modes > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))
 
 
+def native_stands(x):
+    """True where an operator on x may make and look at its tensors in _lib.host(): nobody who follows its calls expects them from Python."""
+    return type(x) in TENSOR_KINDS and x.is_cuda and not torch.compiler.is_compiling() and not operators_seen()
+
+
 def calls_unseen():
     """True when nothing but autograd follows the operators that are called: no mode or transform (operators_seen), no compiler or tracer."""
     return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or operators_seen() or torch.is_autocast_enabled())
