@@ -177,6 +177,43 @@ def core_workspace_bytes(B, D, H, W, dtype=torch.bfloat16):
     return _lib.lib().ss2d_core_workspace_bytes(p)
 
 
+# fp32 maps of L % 8 = 1 .. 7 positions on either side of the length from which they are walked in groups, up to the largest; strides that are no
+# multiples of 4 with 8 positions to a group.
+RAGGED = [(1, 2, 209, 1), (2, 3, 15, 14), (3, 2, 21, 11), (1, 3, 13, 17), (2, 2, 14, 17), (5, 2, 9, 23), (2, 2, 31, 31), (2, 1, 63, 59), (1, 2, 97, 101), (1, 1, 2, 4899)]
+
+
+@pytest.mark.parametrize("softplus", [True, False])
+@pytest.mark.parametrize("shape", RAGGED, ids=lambda s: "x".join(map(str, s)))
+def test_core_fp32_maps_of_no_whole_groups(shape, softplus):
+    """Against the oracle; and what lies around an image's rows -- another image's infinities and NaN, in front of them and behind -- stays out of it."""
+    _announce("core ragged", shape, softplus)
+    args = list(make_core_inputs(sum(shape) + 1, *shape, torch.float32))
+    if not softplus:
+        args[1] = args[1].abs() * 0.1
+        args[6] = args[6].abs() * 0.1
+    want = oracle_core(*args, softplus)
+    got = run_core(*args, softplus)
+    assert torch.allclose(got, want, rtol=1e-3, atol=max(4e-4, 2e-5 * want.abs().max().item())), f"max abs err {(got - want).abs().max().item()}"
+    if shape[0] > 1 and shape[2] * shape[3] >= 208:           # (below, several images are one stream)
+        for k, bad in ((1, float("inf")), (2, float("nan")), (3, float("-inf"))):
+            args[k] = args[k].clone()
+            args[k][..., 1, :] = bad
+        again = run_core(*args, softplus)
+        keep = [b for b in range(shape[0]) if b != 1]
+        assert torch.equal(again[keep], got[keep])
+
+
+def test_core_fp32_rows_off_the_grid():
+    _announce("core ragged strides")
+    x, delta, Bs, Cs, A, Dv, bias = make_core_inputs(91, 2, 3, 16, 16, torch.float32)
+    wide = [torch.full(t.shape[:-1] + (259,), float("nan")) for t in (delta, Bs, Cs)]
+    for w, t in zip(wide, (delta, Bs, Cs)):
+        w[..., 2:258] = t
+    dev = lambda t: t.to(DEV)
+    got = ss2d_core_hip(dev(x), dev(wide[0])[..., 2:258], dev(wide[1])[..., 2:258], dev(wide[2])[..., 2:258], dev(A), dev(Dv), dev(bias), True).cpu()
+    assert torch.allclose(got, oracle_core(x, delta, Bs, Cs, A, Dv, bias), **TOL)
+
+
 # Tiles of 8, 16, 24, 32 and 40 positions at the edges (runs of 1, 2, 4 and 8 lanes), on either side and on both, in one row or column of tiles too.
 TILED_EDGES = [(1, 3, 136, 144), (2, 2, 152, 136), (1, 2, 160, 168), (1, 1, 8, 1680), (1, 1, 1672, 24), (1, 2, 40, 392), (1, 1, 144, 152)]
 

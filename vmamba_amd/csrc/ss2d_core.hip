@@ -114,7 +114,13 @@ struct CorePassLoads {
 // in fp32 where dt_proj rounds them to 16 bits.  96 x 56 x 56, batch 128, bf16: 170 + 67 us of dt_proj -> 176-186 by card (three pairs, 16
 // positions per lane); the ranks come from L2, 2.5 times the lines of before, in runs of 1 KB (as x_proj's plain rows, 64 bytes from
 // lane to lane: 216).
-template <typename in_t, bool kSoftplus, int kGran, bool kVecDelta, bool kWide, int kWpd = 1, int kPairs = 0>
+//
+// kRagged: one fp32 image per workgroup of any length and strides, in groups of 8 all the same.  fp32 rows start on dwords, which is all that the buffer
+// loads of 16 bytes ask for; what has to lie on blocks of 8 are the LDS arrays.  So the rows are walked as if they were rounded up to
+// Lp = a multiple of 8: the forward directions from position 0, with Lp - L items behind the row's end, the backward ones from position
+// L - Lp, with as many in front of it, which are made the identity (behind the row's end nothing valid follows); the maps are 0 there and
+// nobody reads the planes.  Single elements and groups worked out one by one before: 3 x 624 maps of 63 x 59 136 us, so 67 (64 x 60: 60); 20 x 128 of 31 x 31 62, 22.
+template <typename in_t, bool kSoftplus, int kGran, bool kVecDelta, bool kWide, int kWpd = 1, int kPairs = 0, bool kRagged = false>
 __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGran, kWide, kPairs>())) void ss2d_core_kernel(const CoreArgs p, FastDiv divL, FastDiv divW, FastDiv divD, FastDiv divTiles,
                                                            FastDiv divWt) {
     extern __shared__ __align__(16) float core_smem[];
@@ -136,7 +142,9 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGr
     constexpr bool kBits = kSoftplus && sizeof(in_t) == 2;
     using Loads = CorePassLoads<in_t, kGran, kWide>;
     const int L = p.L, H = p.H;
-    const int n_max = p.CB * L;
+    static_assert(!kRagged || (kEs == 4 && kGran == kItems && kVecDelta && kWpd == 1 && kPairs == 0), "whole groups of fp32");
+    const int Lp = kRagged ? core_zero_block(L) : L;
+    const int n_max = kRagged ? Lp : p.CB * L;
     const int plane_ext = lds_extent<4>(n_max), map_ext = core_map_extent<kEs, kFlat>(n_max);
     float *planeA = core_smem;                           // fl(y0 + y2), row-major index
     float *planeB = planeA + plane_ext;                  // fl(y1 + y3), column-major index
@@ -159,22 +167,24 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGr
     const in_t *xs = (dir & 1) ? xT : xR;
     float *plane = (dir & 1) ? planeB : planeA;
     const int kd = dir * p.D + (int)d;
-    const in_t *dl_base = reinterpret_cast<const in_t *>(p.delta) + dir * p.dl_ks + (int64_t)d * p.dl_ds + b0 * p.dl_bs;
-    const __amdgpu_buffer_rsrc_t dl_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<in_t *>(dl_base), 0, (n_el * kEs + 3) & ~3, kBufferRsrcWord3);
+    const bool reverse = dir >= 2;                       // uniform per wavefront
+    const int pad = kRagged && reverse ? Lp - L : 0;     // items in front of the row's first (there is memory in front: directions 0 and 1)
+    const in_t *dl_base = reinterpret_cast<const in_t *>(p.delta) + dir * p.dl_ks + (int64_t)d * p.dl_ds + b0 * p.dl_bs - pad;
+    const __amdgpu_buffer_rsrc_t dl_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<in_t *>(dl_base), 0, ((n_el + pad) * kEs + 3) & ~3, kBufferRsrcWord3);
     const __amdgpu_buffer_rsrc_t B_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.Bm), 0, (int)p.B_span_bytes, kBufferRsrcWord3);
     const __amdgpu_buffer_rsrc_t C_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.Cm), 0, (int)p.C_span_bytes, kBufferRsrcWord3);
-    const uint32_t B_soff = (uint32_t)(dir * p.B_ks + b0 * p.B_bs), C_soff = (uint32_t)(dir * p.C_ks + b0 * p.C_bs);
+    const uint32_t B_soff = (uint32_t)(dir * p.B_ks + b0 * p.B_bs - pad), C_soff = (uint32_t)(dir * p.C_ks + b0 * p.C_bs - pad);
     const float A_log2e = kBits ? p.A[kd] : p.A[kd] * kLog2e;
     const float bias = p.bias ? p.bias[kd] : 0.0f;
-    const bool reverse = dir >= 2;                       // uniform per wavefront
     const uint32_t u_sel = reverse ? 0x05040706u : 0x03020100u;
     // B / C rows of consecutive images adjacent in memory (what one x_proj GEMM per direction writes): a lane's offset
     // into them is its stream position
-    const bool bc_dense = p.B_bs == L && p.C_bs == L;
+    const bool bc_dense = kRagged || (p.B_bs == L && p.C_bs == L);
     // passes of 512 or 1024 positions; a remainder of at most 64 positions is walked one position per lane instead
-    const int tail_len = n_el % kPassLen;
-    const bool short_tail = tail_len > 0 && tail_len <= kWave;
-    const int n_pass = short_tail ? n_el / kPassLen : (n_el + kPassLen - 1) / kPassLen;
+    const int n_stream = kRagged ? Lp : n_el;
+    const int tail_len = n_stream % kPassLen;
+    const bool short_tail = !kRagged && tail_len > 0 && tail_len <= kWave;
+    const int n_pass = short_tail ? n_stream / kPassLen : (n_stream + kPassLen - 1) / kPassLen;
 
     // Image and position of this lane's first item in the pass issued next: passes are issued strictly in order, so
     // the pair just advances by 512 positions each time (no division in the loop).
@@ -288,6 +298,7 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGr
             }
         }
         r.img = next_img; r.j0 = next_j;
+        if constexpr (kRagged) { r.img = 0; r.j0 = (uint32_t)e0; }
         next_img += step_img; next_j += step_j;
         if (next_j >= (uint32_t)L) { next_j -= (uint32_t)L; next_img += (uint32_t)L; }
         if (bc_dense) {                                  // uniform
@@ -412,6 +423,9 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGr
         if (threadIdx.x < 2 * kItems) {
             in_t *m = threadIdx.x < kItems ? xR : xT;
             m[map_index<kEs, kFlat>(core_zero_block(n_max) + (int)(threadIdx.x % kItems))] = in_t{};
+            if constexpr (kRagged) {
+                if (L + (int)(threadIdx.x % kItems) < Lp) m[map_index<kEs, kFlat>(L + (int)(threadIdx.x % kItems))] = in_t{};
+            }
         }
     }
     __syncthreads();
@@ -472,8 +486,8 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGr
             // The group's kGran logical indices in this direction's order are consecutive and kGran-aligned (L and
             // every group start are multiples of kGran): forwards they are the stream positions e0 + gi*kGran + t,
             // backwards img*L + L-1 - (jg + t), i.e. the block starting at img*L + L - jg - kGran read downwards.
-            const bool valid = e0 + gi * kGran < n_el;
-            int base = reverse ? img_off + L - jg - kGran : e0 + gi * kGran;
+            const bool valid = e0 + gi * kGran < n_stream;
+            int base = reverse ? img_off + Lp - jg - kGran : e0 + gi * kGran;
             base = valid ? base : zero_block;                                // past the end: u = 0
             slot[gi].valid = valid;
             slot[gi].plane_idx = lds_index<4>(base);
@@ -506,8 +520,27 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGr
             float a = __builtin_amdgcn_exp2f(dl[i] * A_log2e);
             if (i % kGran == 0) a = first[i / kGran] ? 0.0f : a;
             const float bb = Bv[i] * (dl[i] * uv[i]);
-            ac[i] = i == 0 ? a : ac[i - 1] * a;
-            hh[i] = i == 0 ? bb : fmaf(a, hh[i - 1], bb);
+            if constexpr (kRagged) {                     // put together below
+                ac[i] = a; hh[i] = bb;
+            } else {
+                ac[i] = i == 0 ? a : ac[i - 1] * a;
+                hh[i] = i == 0 ? bb : fmaf(a, hh[i - 1], bb);
+            }
+        }
+        if constexpr (kRagged) {
+            if (pass == 0 && reverse) {                  // uniform
+                const int front = lane == 0 ? pad : -1;  // the items in front, and the state at the first behind them
+#pragma unroll
+                for (int i = 0; i < kIt; ++i) {
+                    ac[i] = i <= front ? 0.0f : ac[i];
+                    hh[i] = i < front ? 0.0f : hh[i];
+                }
+            }
+#pragma unroll
+            for (int i = 1; i < kIt; ++i) {
+                hh[i] = fmaf(ac[i], hh[i - 1], hh[i]);
+                ac[i] = ac[i - 1] * ac[i];
+            }
         }
         float a_ex, h_ex, a_tot, h_tot;
         wave_scan_pairs(ac[kIt - 1], hh[kIt - 1], a_ex, h_ex, a_tot, h_tot);
@@ -733,7 +766,7 @@ __global__ __launch_bounds__(kWpd * kBlock, (kWpd > 1 ? 4 : core_waves<in_t, kGr
         }
         return;
     }
-    if (kGran >= 4 && p.vec_out && p.W >= 4) {
+    if (kGran >= 4 && !kRagged && p.vec_out && p.W >= 4) {
         // four consecutive positions per lane (L is a multiple of kGran, so they share an image and, with W >= 4, span
         // at most two rows): one 16-byte store
         const int n_quad = n_el / 4;
@@ -862,6 +895,14 @@ static int launch_core(CoreArgs a, hipStream_t stream) {
     int64_t CB;
     const size_t smem = core_cut<in_t>(a, g, wide, CB);
     if (smem > kCoreMaxLds) return SS2D_ENOTSUP;
+    // fp32 rows that are no whole groups: by themselves once they fill two fifths of a pass (a group's items one by one take 2.5 times the instructions)
+    bool ragged = false;
+    size_t smem_ragged = 0;
+    if constexpr (sizeof(in_t) == 4) {
+        smem_ragged = lds_bytes_of<in_t>(core_zero_block(a.L), false);
+        ragged = g == 1 && L >= 208 && smem_ragged <= kCoreMaxLds && a.dl_ks >= kItems / 2 && a.B_ks >= kItems / 2 && a.C_ks >= kItems / 2;
+        if (ragged) CB = 1;
+    }
     a.CB = (int)CB;
     // 16-byte loads of the delta stream need every (direction, channel, first image of a workgroup) start aligned;
     // otherwise the kernel loads element-wise
@@ -878,6 +919,15 @@ static int launch_core(CoreArgs a, hipStream_t stream) {
     if (n_wg > 0x7fffffff) return SS2D_ENOTSUP;
     const FastDiv dL = make_fastdiv((uint32_t)L), dW = make_fastdiv((uint32_t)a.W), dD = make_fastdiv((uint32_t)a.D);
     const FastDiv dT = make_fastdiv((uint32_t)(tiled ? (a.H / 4) * (a.W / 4) : 1)), dWt = make_fastdiv((uint32_t)(tiled ? a.W / 4 : 1));
+    if constexpr (sizeof(in_t) == 4) {
+        if (ragged) {
+            if (a.softplus)
+                hipLaunchKernelGGL((ss2d_core_kernel<in_t, true, kItems, true, false, 1, 0, true>), dim3((uint32_t)n_wg), dim3(kBlock), smem_ragged, stream, a, dL, dW, dD, dT, dWt);
+            else
+                hipLaunchKernelGGL((ss2d_core_kernel<in_t, false, kItems, true, false, 1, 0, true>), dim3((uint32_t)n_wg), dim3(kBlock), smem_ragged, stream, a, dL, dW, dD, dT, dWt);
+            return launch_status();
+        }
+    }
     // several wavefronts per direction where the arrays leave a CU two workgroups (two each) or one (four)
     const int wpd = !(wide && smem > kCorePairLds) ? 1 : smem > kCoreQuadLds ? 4 : 2;
     if (a.dts) {
