@@ -139,6 +139,25 @@ def test_layer_norm_channel_first(B, C, H, W, in_dt, w_dt, out_dt, out_cl):
     assert torch.allclose(got.float(), want.float(), **_tol(out_dt))
 
 
+# fp32 rows that start on dwords only, in quads of positions: the four widths of the kernel, L % 4 = 1, 2 and 3, a last workgroup of one and of three positions.
+QUADS_OFF_THE_GRID = [(9, 96, 41, 77), (7, 72, 43, 75), (9, 192, 38, 43), (9, 384, 35, 51), (9, 768, 33, 49), (40, 40, 15, 15)]
+
+
+@pytest.mark.parametrize("B,C,H,W", QUADS_OFF_THE_GRID)
+@pytest.mark.parametrize("w_dt,out_dt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)])
+def test_layer_norm_channel_first_rows_off_the_grid(B, C, H, W, w_dt, out_dt):
+    """Neighbouring rows hold infinities at their ends: what a row's last quad reads of the next one stays out of it."""
+    print("CASE ln-cf-off-grid", B, C, H, W, out_dt, flush=True)
+    g = torch.Generator().manual_seed(47)
+    x = torch.randn(B, C, H, W, generator=g) * 2 - 0.3
+    w, b = (torch.randn(C, generator=g) + 1).to(w_dt), torch.randn(C, generator=g).to(w_dt)
+    want = torch_ref.layer_norm_cf(x, w, b, 1e-5, True, out_dt)
+    x[:, :, 0, 0] = float("inf")
+    got = layer_norm_cf_hip(_dev(x), _dev(w), _dev(b), 1e-5, out_channel_last=True, out_dtype=out_dt).cpu()
+    got, want = got.flatten(1, 2)[:, 1:], want.flatten(1, 2)[:, 1:]
+    assert torch.allclose(got.float(), want.float(), **_tol(out_dt))
+
+
 @pytest.mark.parametrize("B,C,H,W", [(128, 192, 28, 28), (128, 384, 14, 14), (128, 768, 7, 7), (64, 384, 14, 14), (300, 768, 7, 7)])
 def test_layer_norm_channel_first_benchmark_batches(B, C, H, W):
     """The out_norm shapes of the 224 x 224 model at the benchmark's batch (the split of an image over workgroups

@@ -402,7 +402,7 @@ __global__ __launch_bounds__(kBlock) void layer_norm_cf_quad_kernel(const in_t *
     const int q = threadIdx.x % kQ, g = threadIdx.x / kQ;
     const int wave = threadIdx.x / kWave;
     const int l = l0 + 4 * q;
-    const bool valid = l < L;                        // L % 4 == 0 (host-checked): a quad is inside or outside
+    const bool valid = l < L;                        // a quad is inside or outside, or (kOutChannelLast, fp32) what is behind the row's end is not stored
     const in_t *xb = x + (size_t)b * C * L;
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<in_t *>(xb), 0, C * L * (int)sizeof(in_t), 0x00020000);
 
@@ -997,8 +997,10 @@ static int launch_ln_cf(const void *x, const void *w, const void *b, void *y, in
             return launch_ln_cf_image<in_t, w_t, out_t>(plan, x, w, b, y, B, C, L, eps, out_channel_last, stream);
     }
     {
-        // quads of positions: 16-byte loads of fp32 input, 8-byte loads of 16-bit input (and 16-byte channel-last stores)
-        const bool quad_ok = L % 4 == 0 && ln_aligned16(x) && (int64_t)C * L * 4 < 0x7ffffff0ll && (int64_t)B * ((L + 15) / 16) <= 0x7fffffff &&
+        // quads of positions: 16-byte loads of fp32 input, 8-byte loads of 16-bit input (and 16-byte channel-last stores).  fp32 rows start on dwords, which
+        // the loads are content with; 16-bit ones and channel-first stores want whole quads.  (Maps of 63 x 59, 3 x 624 of them: 35 us a position per
+        // lane, so 20; 20 x 128 of 31 x 31 17, 9.5; 159 x 159, 432 of them: 53, 31.)
+        const bool quad_ok = (L % 4 == 0 || (sizeof(in_t) == 4 && out_channel_last)) && ln_aligned16(x) && (int64_t)C * L * 4 < 0x7ffffff0ll && (int64_t)B * ((L + 15) / 16) <= 0x7fffffff &&
                              (out_channel_last ? (C % (16 / (int)sizeof(out_t)) == 0 && ln_aligned16(y)) : ln_aligned16(y));
         if (quad_ok) {
             if (C <= 96) return launch_ln_cf_quad<in_t, w_t, out_t, 16, 16, 6>(x, w, b, y, B, C, L, eps, out_channel_last, stream);
