@@ -641,6 +641,25 @@ def test_dt_proj_masked_positions_take_the_fill_value(K, D, R, N, dtype, fill):
         dt_proj_hip(x, w, mask.to(torch.int32), fill)                  # wrong type
 
 
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+@pytest.mark.parametrize("D,R,N", [(33, 33, 72), (97, 1, 64), (35, 3, 200), (31, 7, 65), (40, 18, 130), (64, 39, 136), (37, 41, 8), (31, 47, 70), (100, 30, 20000), (200, 43, 9000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_dt_proj_weights_on_any_element(D, R, N, offset, dtype):
+    """Directions whose weights start in either half of a dword, ranks of 1 to 3 more than whole fours, one to three blocks per wavefront: what lies around the weights -- the
+    next row's, NaN before the first and behind the last -- stays out of the sums.  fp32 sums of R products, one rounding: half an ulp of the result and R ulps of fp32."""
+    _announce("dt_proj weights", D, R, N, offset, dtype)
+    g = torch.Generator().manual_seed(D + R)
+    x = torch.randn(4, R, N, generator=g).to(dtype)
+    w = torch.randn(4, D, R, generator=g).to(dtype)
+    room = torch.full((offset + w.numel() + 8,), float("nan"), dtype=dtype)
+    room[offset:offset + w.numel()] = w.flatten()
+    room = room.to(DEV)
+    got = va.core.dt_proj_hip(x.to(DEV), room[offset:offset + w.numel()].view(4, D, R)).double().cpu()
+    want, size = torch.matmul(w.double(), x.double()), torch.matmul(w.double().abs(), x.double().abs())
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert bool(((got - want).abs() <= ulp * want.abs() + (R + 1) * 2.0 ** -23 * size + 1e-7).all())
+
+
 def test_dt_proj_rejections():
     from vmamba_amd.core import dt_proj_hip
     with pytest.raises(RuntimeError):

@@ -63,7 +63,9 @@ __global__ __launch_bounds__(kBlock) void dt_proj_kernel(const DtArgs p) {
     const T *x = reinterpret_cast<const T *>(p.x) + (int64_t)k * p.x_ks;
     const T *W = reinterpret_cast<const T *>(p.W) + (int64_t)k * p.D * p.R;
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(x), 0, (int)p.x_span_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t W_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(W), 0, p.D * p.R * 2, 0x00020000);
+    // (W's from the dword that holds its first element: w_odd)
+    const int w_odd = (int)(reinterpret_cast<uintptr_t>(W) >> 1 & 1);
+    const __amdgpu_buffer_rsrc_t W_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(W - w_odd), 0, ((w_odd + p.D * p.R) * 2 + 3) & ~3, 0x00020000);
     T *out = reinterpret_cast<T *>(p.out) + (int64_t)k * p.D * p.N;
     const int d_base = dc * kDtGroups * kDtTile;
 
@@ -83,14 +85,15 @@ __global__ __launch_bounds__(kBlock) void dt_proj_kernel(const DtArgs p) {
                 wf[g][s][0] = t[0];
                 wf[g][s][1] = t[1];
             } else {
-                uint32_t e[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t off = (d < p.D && r0 + q < p.R) ? (uint32_t)(d * p.R + r0 + q) * 2u : kDtOutOfRange;
-                    e[q] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(W_rsrc, (int)off, 0, 0);
-                }
-                wf[g][s][0] = e[0] | (e[1] << 16);
-                wf[g][s][1] = e[2] | (e[3] << 16);
+                // three dwords hold the four ranks, from either half of the first on; what is past the last rank is the next row's.  (Element by
+                // element they were 72 loads of a wavefront with 33 to 48 ranks, more than all else it does: 528 channels, 33 ranks,
+                // 15 680 positions, bf16 32 us, so 25; with room for 40 ranks instead of 48 22.6.)
+                const uint32_t at = (uint32_t)(w_odd + d * p.R + r0);
+                const auto t = __builtin_amdgcn_raw_buffer_load_b96(W_rsrc, (int)(d < p.D && r0 < p.R ? at / 2 * 4 : kDtOutOfRange), 0, 0);
+                const int shift = (int)(at & 1) * 16, left = p.R - r0;
+                const uint32_t lo = __builtin_amdgcn_alignbit(t[1], t[0], shift), hi = __builtin_amdgcn_alignbit(t[2], t[1], shift);
+                wf[g][s][0] = left >= 2 ? lo : lo & 0xffffu;
+                wf[g][s][1] = left >= 4 ? hi : left == 3 ? hi & 0xffffu : 0u;
             }
         }
     }
@@ -231,6 +234,7 @@ static int launch_dt_proj(DtArgs a, hipStream_t stream) {
     else if (steps == 2) SS2D_DT_LAUNCH(2);
     else if (steps == 3) SS2D_DT_LAUNCH(3);
     else if (steps == 4) SS2D_DT_LAUNCH(4);
+    else if (steps == 5) SS2D_DT_LAUNCH(5);
     else SS2D_DT_LAUNCH(6);
 #undef SS2D_DT_LAUNCH
     return launch_status();
@@ -278,14 +282,27 @@ extern "C" int ss2d_dt_proj_masked(const void *x, const void *weight, const void
     a.K = K; a.D = D; a.R = R; a.N = N; a.x_ks = x_dir_stride; a.x_rs = x_rank_stride;
     a.d_chunks = (D + kDtGroups * kDtTile - 1) / (kDtGroups * kDtTile);
     a.n_blocks = (N + kDtBlock - 1) / kDtBlock;
-    // enough wavefronts to fill the chip several times over, yet several blocks each so the W fragments are reused
-    int64_t bpw = (int64_t)K * a.d_chunks * a.n_blocks / 8192;
-    bpw = bpw < 1 ? 1 : (bpw > 4 ? 4 : bpw);
+    a.w_vec = (R % 4 == 0) && (reinterpret_cast<uintptr_t>(weight) % 8 == 0);
+    // Blocks per wavefront.  The W fragments are loaded once per wavefront, a quarter of a block's time as quads and half of one as dwords; against that
+    // stand the rounds in which the wavefronts pass through the chip (registers: 4 on a SIMD up to 24 ranks, 3 beyond).  One, two or three blocks by
+    // the least of rounds times a wavefront's time.  us for 1 / 2 / 3, bf16: 304 channels of 20 000 positions 17.8 / 16.1 / 16.2, 464 of 28 224 29.6 / 27.1 / 27.7,
+    // 528 of 15 680 22.7 / 20.9 / 20.8, 656 of 20 800 35.2 / 33.2 / 30.9, 704 of 12 096 20.2 / 17.8 / 18.4.  Up to 16 ranks, and up to 24 as quads, there is little to load
+    // and rounds matter less than what the stores meet in memory: one block up to 16 384 of them, then up to four (1 / 2 / 3: 96 of 262 144 40.5 / 36.9 / -, 64 of 262 144
+    // 32 / 25 / -, 96 of 401 408 60.8 / 61.7 / 65.8, 112 of 144 500 31.0 / 37.7 / 36.6, 320 of 29 008 19.8 / 22.5 / 23.7).
+    const int steps = (R + 7) / 8;
+    const int64_t waves = (int64_t)K * a.d_chunks * a.n_blocks, resident = steps <= 3 ? 4096 : 3072;
+    int64_t bpw = waves / 8192 < 1 ? 1 : waves / 8192 > 4 ? 4 : waves / 8192;
+    if (steps > (a.w_vec ? 3 : 2)) {
+        int64_t least = INT64_MAX;
+        for (int64_t n = 1; n <= 3; ++n) {
+            const int64_t cost = (waves + n * resident - 1) / (n * resident) * (4 * n + (a.w_vec ? 1 : 2));
+            if (cost < least) { least = cost; bpw = n; }
+        }
+    }
     a.blocks_per_wave = (int)bpw;
     a.n_pos_chunks = (a.n_blocks + bpw - 1) / bpw;
     a.total_waves = (int64_t)K * a.d_chunks * a.n_pos_chunks;
     a.x_span_bytes = (uint32_t)dt_x_span(R, N, x_rank_stride);
-    a.w_vec = (R % 4 == 0) && (reinterpret_cast<uintptr_t>(weight) % 8 == 0);
     // 16-byte loads of x and stores of delta: rows and bases on 16-byte boundaries
     a.vec_ok = (N % 8 == 0) && (x_dir_stride % 8 == 0) && (x_rank_stride % 8 == 0) &&
                (reinterpret_cast<uintptr_t>(x) % 16 == 0) && (reinterpret_cast<uintptr_t>(delta) % 16 == 0) &&
