@@ -47,6 +47,16 @@ CASES = [
     (3, 16, 3, 5, 7, (8, 8), 3),           # mask row behind the last row
 ]
 
+# Plans by rounds of workgroups: four, two and one direction, tiles of 4, 8 and 12 rows, a last tile of 4 of 8 rows, pieces of a row, a padded map, 90 output rows.
+ROUNDS = [(12, 128, 10, 84, 84, None, -1), (15, 176, 13, 48, 48, None, -1), (3, 528, 45, 56, 56, None, -1), (5, 320, 22, 60, 28, None, -1), (2, 144, 29, 152, 152, None, -1),
+          (10, 136, 43, 52, 40, None, -1), (9, 208, 15, 92, 94, (92, 96), 14)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", ROUNDS, ids=lambda c: "x".join(map(str, c[:5])))
+def test_x_proj_plans_by_rounds(case, dtype):
+    test_x_proj(case, dtype)
+
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:5])))

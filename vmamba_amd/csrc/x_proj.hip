@@ -452,11 +452,36 @@ static int x_proj_plan(int B, int D, int C, int H, int W, int Hp, int Wp, int dt
     // wavefronts share the channels as well (k_split below).  One image, bf16: 768 x 56 x 56, C = 50 34.5 -> 12.9 us, 336 x 45 x 45,
     // C = 23 25.2 -> 8.2, 192 x 28 x 28, C = 14 9.3 -> 6.8.  From 160 workgroups on it costs more than it gives (at 192: 48 images
     // of 384 x 14 x 14, C = 32 11.9 -> 15.3).
+    const bool few = total < 160;
     while (total < 160 && Th > 1 && Th * a.Tw > kXpGroup) {
         int64_t t = (Th + 1) / 2;
         if (unit > 1 && t > 2) t = (t + 3) / 4 * 4;
         if (t >= Th) break;
         Th = t;
+        total = (int64_t)B * (4 / a.n_dirs) * a.tiles_w * ((H + Th - 1) / Th);
+    }
+    // A few hundred workgroups pass through the 256 compute units in two or three rounds, and a plan that fills the last of them is worth more than one that shares
+    // more of x: a workgroup's time is that of its steps of 32 channels, a turn of four column groups at a time, of the results it puts into order, and a part it has in
+    // any case; up to four rounds count whole.  The constants order 1700 measured plans of 60 sizes; a plan is left only for one that this
+    // puts a tenth ahead, and not where the channels are few or shared out (k_split), or the rows no multiple of 4, which it knows nothing of.  us, before / so: 20 x 208 maps of 96 x 96 38.9 / 28.6, 125 x 528 of 20 x 20 41.7 / 31.2, 2 x 480 of 84 x 112
+    // 22.4 / 18.7, 15 x 496 of 64 x 64 37.1 / 31.4; 90 other sizes 1.02 in the mean, the worst 52.7 / 53.6.
+    auto cost = [&](int dirs, int64_t t) {
+        const int64_t wgs = (int64_t)B * (4 / dirs) * a.tiles_w * ((H + t - 1) / t), pos = t * a.Tw, out_rows = dirs * a.Ce;
+        const double own = (double)((pos + 4 * kXpGroup - 1) / (4 * kXpGroup)) * a.k_steps + 0.003 * pos * out_rows + 2.0;
+        return own * (wgs <= 256 ? 1.1 : wgs <= 1024 ? (double)((wgs + 255) / 256) : wgs / 256.0 + 0.5);
+    };
+    if (!few && D >= 128 && H % 4 == 0 && Th * a.Tw > 2 * kXpGroup) {
+        double least = 0.9 * cost(a.n_dirs, Th);
+        for (int dirs = 4; dirs >= 1; dirs /= 2) {
+            const int out_rows = dirs * a.Ce, pitch = out_rows + (out_rows / 2 % 2 == 0 ? 2 : 0);
+            for (int64_t t = 4; out_rows <= 96 && t <= H && t * a.Tw * pitch * 2 <= 64 * 1024; t += 4) {
+                if (t * a.Tw <= 2 * kXpGroup || cost(dirs, t) >= least) continue;
+                least = cost(dirs, t);
+                a.n_dirs = dirs; a.pitch = pitch;
+                Th = t;
+            }
+        }
+        row_bytes = (int64_t)a.Tw * a.pitch * 2;
         total = (int64_t)B * (4 / a.n_dirs) * a.tiles_w * ((H + Th - 1) / Th);
     }
     // a row of a width that is no multiple of 4 is not cut: there is a widest one
