@@ -144,7 +144,8 @@ int ss2d_selective_scan_kernel(const ss2d_scan_params *params);
  * height x width map transposed (width x height).  n_groups must be 4 and group k is scan direction k: its channels
  * read x (k = 0, 2) or x_t (k = 1, 3), forwards (k < 2) or backwards (cross_scan_fwd, csm_triton.py:22-29).  Everything
  * else as ss2d_selective_scan_fwd.  Served by the channel-per-lane kernel only (dstate 4 / 8 / 16 / 32, dim / 4 >= 32,
- * 16-byte aligned x_t; ss2d_selective_scan_kernel tells for the same sizes): SS2D_ENOTSUP otherwise.
+ * 16-byte aligned x_t): where ss2d_selective_scan_kernel names it for the same sizes, and at 16 and 32 states for every
+ * size; SS2D_ENOTSUP otherwise.
  */
 int ss2d_selective_scan_fwd_maps(const ss2d_scan_params *params, const void *x_t, void *stream);
 

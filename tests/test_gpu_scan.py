@@ -229,8 +229,9 @@ def test_scan_odd_rows(batch, dim, G, N, L, dtype):
 
 # Rows of no whole 16-byte pieces in the same kernel: a row shorter than a group of four, one that ends 1, 2 and 3 positions into a group, rows on odd
 # elements, cut rows, 4 to 32 states; what the rule leaves to the other kernels beside it.
-ODD_ROWS = [(2, 64, 2, 16, 3, "chan"), (1, 33, 1, 16, 9, "chan"), (2, 47, 1, 8, 49, "chan"), (1, 40, 1, 32, 62, "chan"), (2, 96, 2, 16, 225, "chan"),
-            (1, 48, 1, 16, 1003, "chan"), (3, 35, 1, 4, 331, "chan"), (1, 48, 1, 16, 3306, "chan"), (1, 64, 1, 4, 225, "row"), (1, 64, 1, 4, 3307, "row4")]
+ODD_ROWS = [(2, 64, 2, 16, 3, "chan"), (1, 33, 1, 16, 9, "chan"), (2, 47, 1, 8, 49, "chan"), (1, 40, 1, 32, 62, "chan"), (26, 99, 1, 16, 135, "chan"), (25, 99, 1, 16, 135, "flat"), (2, 96, 2, 16, 225, "flat"),
+            (1, 48, 1, 16, 1225, "chan"), (1, 48, 1, 16, 1003, "flat"), (1, 40, 1, 32, 3306, "chan"), (1, 48, 1, 16, 3306, "row4"), (64, 48, 1, 8, 77, "chan"), (37, 33, 1, 4, 77, "row"),
+            (39, 33, 1, 4, 77, "chan"), (3, 35, 1, 4, 331, "row"), (1, 64, 1, 4, 3307, "row4")]
 
 
 @pytest.mark.parametrize("batch,dim,G,N,L,kernel", ODD_ROWS)
@@ -247,7 +248,8 @@ def test_scan_odd_rows_channel_per_lane(batch, dim, G, N, L, kernel, dtype):
         assert torch.equal(run_gpu(*args, True, False, want_x=False)[0], got.to(dtype))
 
 
-@pytest.mark.parametrize("batch,Dm,H,W,N", [(2, 32, 7, 9, 16), (1, 48, 5, 5, 16), (3, 33, 3, 1, 16), (1, 64, 15, 19, 8), (1, 48, 57, 58, 16), (2, 40, 6, 6, 32)])
+@pytest.mark.parametrize("batch,Dm,H,W,N", [(2, 32, 7, 9, 16), (1, 48, 5, 5, 16), (3, 33, 3, 1, 16), (1, 64, 9, 7, 8), (1, 48, 33, 41, 16), (1, 40, 61, 57, 32), (20, 48, 11, 11, 16),
+                                           (2, 40, 6, 6, 32)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_scan_reading_odd_maps_through_the_cross_scan_routes(batch, Dm, H, W, N, dtype):
     """The bits of CrossScan and the scan behind it, for maps whose rows end inside a group of four positions, forwards and backwards."""
@@ -260,6 +262,21 @@ def test_scan_reading_odd_maps_through_the_cross_scan_routes(batch, Dm, H, W, N,
     assert kernel_of(xs, delta, A, B, C, want_x=False) == "chan"
     want = va.selective_scan_fwd(xs, delta, A, B, C, D, bias, True, 1, True, want_x=False)[0]
     assert torch.equal(selective_scan_from_map(x, delta, A, B, C, D, bias), want)
+
+
+@pytest.mark.parametrize("batch,Dm,H,W,N", [(1, 48, 15, 15, 16), (2, 33, 21, 17, 32), (1, 40, 57, 58, 16)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_reading_few_odd_maps(batch, Dm, H, W, N, dtype):
+    """Where the scan of the four copies is another kernel's: the same recurrence in another order."""
+    from vmamba_amd.csms6s import selective_scan_from_map
+    _announce("scan-few-odd-maps", batch, Dm, H, W, N, dtype)
+    L = H * W
+    _, delta, A, B, C, D, bias = [t.to("cuda") for t in make_inputs(41, batch, 4 * Dm, 4, N, L, dtype, ss2d_like=True)]
+    x = torch.randn(batch, Dm, H, W, generator=torch.Generator().manual_seed(42)).to("cuda", dtype)
+    xs = va.cross_scan_fn(x).view(batch, 4 * Dm, L)
+    assert kernel_of(xs, delta, A, B, C, want_x=False) != "chan"
+    want = va.selective_scan_fwd(xs, delta, A, B, C, D, bias, True, 1, True, want_x=False)[0]
+    assert torch.allclose(selective_scan_from_map(x, delta, A, B, C, D, bias), want, **TOL32)
 
 
 def test_scan_segments_hold_what_a_whole_row_does():

@@ -418,27 +418,38 @@ __global__ __launch_bounds__(kBlock) void scan_chan_carry_kernel(const float *__
     }
 }
 
-// Rows of whole 16-byte pieces and 8 positions are this kernel's at any size.  Others would take the kernels with positions in lanes, whose 16 states
-// of odd rows (64 x 96 maps in bf16, before, and as they are now: 49 positions 93 / 81 us, here 12.5; 225 182 / 87, 37; 16 x 192 of 3306 1390 / 323, 266) and larger calls of 4, 8 and 32 are far behind;
-// left to them are few wavefronts, each alone with its row: 4 states, 12 of them, 225 positions 5.7 / 13.5, 3306 10.9 / 22.9; 8 states, 225 7.9 / 16.6; 32 in
-// single precision 18.5 / 34.3; single precision of an odd number of fours, which they read in whole pieces: 4 states, 192: 1764 positions 24.9 / 40.0, 768: 86.6 / 81.9.
+// Rows of whole 16-byte pieces and 8 positions are this kernel's at any size.  Others were the flat kernel's or element by element (16 states in bf16, 64 x 96 maps of
+// 49 positions 93 us, here 12.5; of 225 182, 37; 16 x 192 of 3306 1390, 266).  Of them, what the kernels with positions in lanes are ahead with is left to those: they do a row in
+// steps of 256 or 512 positions, each in the same time however few the rows, where a wavefront here walks its row serially.  So few wavefronts on 100 to 1000 positions, the more
+// the fewer the states (us, positions / channels in lanes, wavefronts of whole rows in front, bf16: 16 states, 12: 100 positions 12.0 / 12.3, 196 12.1 / 19.9, 324 12.1 / 32.5; 192: 100 17.9 / 12.7,
+// 196 18.4 / 20.5, 324 18.4 / 30.8; 384: 196 27.4 / 21.1, 324 27.9 / 31.3; 768: 324 48.2 / 32.6; 4 states, 192: 77 8.1 / 7.3, 196 8.6 / 12.6; 384: 196 11.9 / 13.0, 324 12.1 / 19.2; 768: 324
+// 21.0 / 20.1), and longer ones of 4 and 8 states (768: 1225 positions of 4 60.9 / 62.1; 12: 3306 of 4 10.9 / 23.1, 16 states 29.2 / 30.7; 96: 70.5 / 54.1); single precision of an odd number of fours
+// they read in whole pieces (16 states, 192: 1764 positions 0.86 of the time here, 768 1.16).
 static bool chan_pays(const ScanArgs &a, bool vec, int in_size) {
     if (vec && a.L % 8 == 0) return true;
     const int64_t units = (int64_t)a.batch * (a.dim / a.dim_per_group) * ((a.dim_per_group + kChanBlock - 1) / kChanBlock);
-    if (vec && a.N < 16) return units >= (a.L < 512 ? 192 : 768);
-    if (vec) return a.L < 512 || units >= 768 || units <= 48;
-    if (a.N == 4 && a.L > 2048 && units < 48) return false;
-    if (a.L > 64 && a.L <= 256 && units < 192) return a.N == 16 || (a.N == 32 && in_size == 2);
-    return true;
+    const int at = a.N == 4 ? 0 : a.N == 8 ? 1 : a.N == 16 ? 2 : 3;
+    constexpr int kAlways[4] = {56, 64, 104, 104};                // positions up to which a wavefront's walk is as short as a step
+    constexpr int kFrom[4] = {45, 55, 60, 60}, kPerTen[4] = {36, 27, 24, 19};      // wavefronts wanted per 10 positions behind the first ones, up to 512 positions
+    constexpr int kMedium[4] = {1024, 704, 576, 576};             // wavefronts wanted up to 1024 positions
+    if (a.L <= kAlways[at]) return true;
+    if (a.L <= 512) return 10 * units >= (int64_t)kPerTen[at] * (a.L - kFrom[at]);
+    if (a.L <= 1024) return units >= kMedium[at];
+    if (vec && units > 48 && units < 768) return false;
+    if (a.N == 4) return units >= (in_size == 4 ? 768 : 1024);
+    if (a.N == 8) return units >= 576;
+    return a.N == 32 || a.L <= 2048 || units >= 64;
 }
 
-bool scan_chan_eligible(const ScanArgs &a, bool vec, int in_size) {
+bool scan_chan_eligible(const ScanArgs &a, bool vec, int in_size, bool maps) {
+    // With CrossScan folded in the other kernels' lead on few wavefronts is not worth the four copies and another launch (forward_core of 4 x 128 maps of 19 x 19,
+    // 16 states in bf16, 87 us, 106 apart).
     // N/4 states per lane; at least two blocks of channels per group; a block's rows within 32-bit byte offsets
     for (int64_t s : {a.u_ds, a.dl_ds, a.o_ds})
         if (s < 0 || (kChanBlock - 1) * s + a.L > kNowhere / 2 / 4) return false;
     for (int64_t s : {a.B_ns, a.C_ns})
         if (s < 0 || (a.N - 1) * s + a.L > kNowhere / 2 / 4) return false;
-    return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.dim_per_group >= 32 && chan_pays(a, vec, in_size);
+    return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.dim_per_group >= 32 && ((maps && a.N >= 16) || chan_pays(a, vec, in_size));
 }
 
 // The number of segments of a row (1: not cut) and the length of all but the last, which has at least 72 positions: a segment's N + 3

@@ -31,7 +31,7 @@ struct ScanArgs {
 
 // scan_chan.hip: the channel-per-lane kernel for several states per channel.  True when it takes this problem
 // (vec: 16-byte vector I/O); launch returns an SS2D status.
-bool scan_chan_eligible(const ScanArgs &a, bool vec, int in_size);
+bool scan_chan_eligible(const ScanArgs &a, bool vec, int in_size, bool maps = false);
 // xt != nullptr: a.u is the map x (batch, dim / 4, L) and xt its transpose, read through CrossScan's routes (group = direction)
 int launch_scan_chan(const ScanArgs &a, int in_dtype, int out_dtype, hipStream_t stream, const void *xt = nullptr);
 

@@ -826,7 +826,7 @@ extern "C" int ss2d_selective_scan_fwd_maps(const ss2d_scan_params *q, const voi
     if (kernel < 0) return kernel;
     if (kernel == SS2D_SCAN_KERNEL_NONE) return SS2D_OK;
     // only the channel-per-lane kernel reads u through the routes
-    if (kernel != SS2D_SCAN_KERNEL_CHAN || !aligned16(x_t)) return SS2D_ENOTSUP;
+    if ((kernel != SS2D_SCAN_KERNEL_CHAN && !scan_chan_eligible(a, vec, q->in_dtype == SS2D_F32 ? 4 : 2, true)) || !aligned16(x_t)) return SS2D_ENOTSUP;
     return launch_scan_chan(a, q->in_dtype, q->out_dtype, (hipStream_t)stream, x_t);
 }
 
