@@ -182,6 +182,25 @@ def test_scan_bwd_channel_per_lane_keeps_channels_apart():
     assert bool(got[1][0, 49, :301].isnan().any()) and bool(got[2][:49].isfinite().all())
 
 
+@pytest.mark.parametrize("L", [600, 72])
+def test_scan_bwd_channel_per_lane_lanes_without_a_channel_add_nothing(L):
+    """33 channels per group: 15 lanes of the third wavefront have none.  The last channel's bias alone would let their decay overflow (softplus off,
+    exp(-20 * -30)), where its own steps are small; an infinite C makes g of a zero dout NaN.  dB and dC are the real channels' sums."""
+    print("CASE scan-bwd-chan-idle-lanes", L, flush=True)
+    batch, dim, N = 64 if L == 72 else 1, 33, 16
+    u, delta, A, B, C, D, bias, dout = make(6, batch, dim, 1, N, L, torch.float32, softplus=False)
+    A[32], bias[32] = -20.0, -30.0
+    delta[:, 32] += 30.0
+    want = torch_ref.selective_scan_grads(u, delta, A, B, C, D, bias, dout, False)
+    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)
+    compare(got[3:5], want[3:5], 1e-4, "overflowing decay")
+    u, delta, A, B, C, D, bias, dout = make(6, batch, dim, 1, N, L, torch.float32, softplus=False)
+    u, B, C, dout = [t.abs() + 0.1 for t in (u, B, C, dout)]
+    C[0, 0, 5, L - 1] = float("inf")
+    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)
+    assert bool((got[3][0, 0, 5] == float("inf")).all()) and bool(got[3][0, 0, :5].isfinite().all()) and bool(got[4].isfinite().all())
+
+
 def test_selective_scan_fn_trains():
     """autograd through selective_scan_fn (csms6s.py:112-126): gradients reach every input."""
     print("CASE scan-autograd", flush=True)

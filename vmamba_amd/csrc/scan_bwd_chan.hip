@@ -25,6 +25,8 @@ constexpr int kBcChan = 16;                       // channels per wavefront
 constexpr int kBcSets = 4;                        // lanes per channel
 constexpr int kBcSub = 8;                         // positions per chunk
 constexpr int kBcPitch = kBcSub + 4;              // floats of an LDS row of a chunk; 16-byte pieces, 8 rows over all banks
+constexpr int kBcGroup = kBcSets * kBcPitch + 4;  // floats of the sets' rows of B or C for one of a lane's states, and a row of zeros from the last pad on
+constexpr int kBcZeros = kBcSets * kBcPitch - 4;
 constexpr int kBcChunks = 9;                      // chunks per segment at most
 constexpr int kBcSeg = kBcChunks * kBcSub;
 
@@ -89,8 +91,8 @@ __device__ __forceinline__ float sum_over_channels(float (&v)[16]) {
 // kGrad: the gradients from the states that enter the segment (see the top); otherwise what the segment leaves on either side.
 template <typename in_t, typename dy_t, int kSpw, bool kDwords, bool kGrad>
 __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4) ? 2 : 3) void scan_bwd_chan_kernel(const ScanBwdArgs p, const BwdChanGeom geo) {
-    constexpr int kN = kBcSets * kSpw, kBcRows = 2 * kN;
-    constexpr int kTile = 3 * kBcChan * kBcPitch + kBcRows * kBcPitch;
+    constexpr int kN = kBcSets * kSpw;
+    constexpr int kTile = 3 * kBcChan * kBcPitch + 2 * kSpw * kBcGroup;
     constexpr int kScratch = kTile > kWave * kBcPitch ? kTile : kWave * kBcPitch;       // also S / T of all lanes
     __shared__ __align__(16) float s_all[kWavesPerWg * kScratch];
     constexpr int kChunk = kWave * kSpw + 4;                                            // (+ 4: the last sums' reads across chunks on other banks)
@@ -110,7 +112,7 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
 
     if (n_chan > 0) {                                       // uniform over the wavefront
         float *s_dl = s_all + wave * kScratch, *s_dlu = s_dl + kBcChan * kBcPitch, *s_dy = s_dlu + kBcChan * kBcPitch;
-        float *s_bc = s_dy + kBcChan * kBcPitch;            // rows [B, C][state of the lane][set]
+        float *s_bc = s_dy + kBcChan * kBcPitch;            // rows [B, C][state of the lane][set or zeros]
         float *s_h = s_h_all + wave * kBcChunks * kChunk;
         const int ch = lane >> 2, set = lane & 3;
         const bool chan_ok = ch < n_chan;
@@ -125,8 +127,9 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
         u_row += (uint32_t)((d - d_first) * p.u_ds);
         dl_row += (uint32_t)((dg - dg_first) * p.dl_ds);
         dy_row += (uint32_t)((d - d_first) * p.do_ds);
-        // staging: two positions of a channel's rows per lane (no channel: zeros, which add nothing to dB and dC), and four of a
-        // row of B and of C each
+        // staging: two positions of a channel's rows per lane (no channel: zeros), and four of a row of B and of C each, the lanes behind those of zeros.
+        // A lane without a channel reads the zeros for B and C and has a decay of 1, so that it adds nothing to dB and dC: with the last channel's A and bias
+        // its decay may overflow where that channel's does not, and B and C may be infinite.
         const int q2 = 2 * set;
         struct Raw {
             RawGroup<in_t, 2, kDwords> u, dl;
@@ -136,6 +139,7 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
         const int r2 = lane >> 1, p4 = 4 * (lane & 1);      // rows of B (and of C): r2 < N
         const bool bc_mine = r2 < kN;
         const int n_row = (r2 & 3) * kSpw + min(r2 >> 2, kSpw - 1);
+        float *st_bc = s_bc + (bc_mine ? (r2 >> 2) * kBcGroup + (r2 & 3) * kBcPitch : r2 % kSpw * kBcGroup + kBcZeros) + p4;
         B_row += (uint32_t)(n_row * p.B_ns);
         C_row += (uint32_t)(n_row * p.C_ns);
         auto load_rows = [&](int t, bool all, Raw &r) {
@@ -147,11 +151,11 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
                 r.C = load_at<in_t, 4, kDwords>(C_buf, C_row, t + p4, L, bc_mine);
             }
         };
-        const float bias = p.bias ? p.bias[dg] : 0.0f, Dv = p.D ? p.D[d] : 0.0f;
+        const float bias = p.bias && chan_ok ? p.bias[dg] : 0.0f, Dv = p.D ? p.D[d] : 0.0f;
         float A[kSpw], A2[kSpw];
 #pragma unroll
         for (int j = 0; j < kSpw; ++j) {
-            A[j] = p.A[(int64_t)d * p.A_ds + (int64_t)(set * kSpw + j) * p.A_ns];
+            A[j] = chan_ok ? p.A[(int64_t)d * p.A_ds + (int64_t)(set * kSpw + j) * p.A_ns] : 0.0f;
             A2[j] = A[j] * kLog2e;
         }
         // a chunk's dl, dl u (dy), B (C) into LDS; dl, u, dy, raw: this lane's own positions
@@ -184,19 +188,19 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
             const int at = ch * kBcPitch + q2;
             *reinterpret_cast<float2 *>(s_dl + at) = make_float2(dl[0], dl[1]);
             *reinterpret_cast<float2 *>(s_dlu + at) = make_float2(dl[0] * uv[0], dl[1] * uv[1]);
-            if (bc_mine) *reinterpret_cast<float4 *>(s_bc + r2 * kBcPitch + p4) = make_float4(Bv[0], Bv[1], Bv[2], Bv[3]);
+            *reinterpret_cast<float4 *>(st_bc) = make_float4(Bv[0], Bv[1], Bv[2], Bv[3]);
             if (all) {
                 *reinterpret_cast<float2 *>(s_dy + at) = make_float2(dy[0], dy[1]);
-                if (bc_mine) *reinterpret_cast<float4 *>(s_bc + (kN + r2) * kBcPitch + p4) = make_float4(Cv[0], Cv[1], Cv[2], Cv[3]);
+                *reinterpret_cast<float4 *>(st_bc + kSpw * kBcGroup) = make_float4(Cv[0], Cv[1], Cv[2], Cv[3]);
             }
         };
         auto read8 = [](const float *from, float (&v)[kBcSub]) {
             const float4 lo = *reinterpret_cast<const float4 *>(from), hi = *reinterpret_cast<const float4 *>(from + 4);
             v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
         };
-        const float *my_bc = s_bc + set * kBcPitch;
-        auto read_B = [&](int j, float (&v)[kBcSub]) { read8(my_bc + j * kBcSets * kBcPitch, v); };
-        auto read_C = [&](int j, float (&v)[kBcSub]) { read8(my_bc + (kSpw + j) * kBcSets * kBcPitch, v); };
+        const float *my_bc = s_bc + (chan_ok ? set * kBcPitch : kBcZeros);
+        auto read_B = [&](int j, float (&v)[kBcSub]) { read8(my_bc + j * kBcGroup, v); };
+        auto read_C = [&](int j, float (&v)[kBcSub]) { read8(my_bc + (kSpw + j) * kBcGroup, v); };
 
         // what enters (leaves) the segment, where its du and d delta will be: N states and the sum of dl; N adjoints
         uint8_t *h_state = reinterpret_cast<uint8_t *>(reinterpret_cast<in_t *>(p.du) + ((int64_t)b * p.dim + d) * L + begin);
