@@ -201,6 +201,30 @@ def test_scan_bwd_channel_per_lane_lanes_without_a_channel_add_nothing(L):
     assert bool((got[3][0, 0, 5] == float("inf")).all()) and bool(got[3][0, 0, :5].isfinite().all()) and bool(got[4].isfinite().all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,L", [(4, 680), (8, 1000), (16, 700)])
+def test_scan_bwd_channel_per_lane_infinite_states(N, L, dtype):
+    """An infinite state and an infinite adjoint go through segments whose decays multiply to 0, as they would position by position (every one of them is
+    above exp(-6)): infinities, not NaN, and only where they belong."""
+    print("CASE scan-bwd-chan-infinite", N, L, dtype, flush=True)
+    dim, inf, first, last = 16, float("inf"), 100, L - 90
+    u, delta, A, B, C, D, bias, dout = make(8, 1, dim, 1, N, L, dtype, softplus=False)
+    u, B, C, dout = [t.abs() + 0.125 for t in (u, B, C, dout)]                  # every sum is one of positive terms
+    A, delta, bias, D = torch.full_like(A, -1.0), 5.0 + delta.abs(), torch.zeros_like(bias), D.abs()
+    call = lambda: [t.double().cpu() for t in va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)]
+    u[0, 3, first] = inf
+    du, ddelta, dA, dB, dC = call()[:5]
+    assert bool((dC[0, 0, :, first:] == inf).all()) and bool(dC[0, 0, :, :first].isfinite().all())
+    assert bool((dB[0, 0, :, first] == inf).all()) and bool(dB[0, 0, :, :first].isfinite().all()) and bool(dB[0, 0, :, first + 1:].isfinite().all())
+    assert bool(du.isfinite().all()) and bool((ddelta[0, 3, first + 1:] == -inf).all()) and bool(ddelta[0, 3, :first].isfinite().all())
+    assert not bool(dA[3].isfinite().any()) and bool(dA[:3].isfinite().all()) and bool(ddelta[0, 4:].isfinite().all())
+    u[0, 3, first], dout[0, 5, last] = 1.0, inf
+    du, ddelta, dA, dB, dC = call()[:5]
+    assert bool((du[0, 5, :last + 1] == inf).all()) and bool(du[0, 5, last + 1:].isfinite().all()) and bool(du[0, :5].isfinite().all())
+    assert bool((dB[0, 0, :, :last + 1] == inf).all()) and bool(dB[0, 0, :, last + 1:].isfinite().all())
+    assert bool((dC[0, 0, :, last] == inf).all()) and bool(dC[0, 0, :, :last].isfinite().all()) and bool(ddelta[0, :5].isfinite().all())
+
+
 def test_selective_scan_fn_trains():
     """autograd through selective_scan_fn (csms6s.py:112-126): gradients reach every input."""
     print("CASE scan-autograd", flush=True)

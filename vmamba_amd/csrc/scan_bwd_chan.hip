@@ -9,7 +9,7 @@
 //
 // Rows are cut into segments of at most 72 positions, which run side by side in two passes with one between them:
 //   local   what a segment leaves from state 0 (h), what it hands to the positions before it with nothing behind it (a_t g_t of its
-//           first position), its sum of dl and its share of dD;
+//           first position), its sum of dl, its largest dl and its share of dD;
 //   carry   what enters every segment from either side; dD of all but the last segment, so that rounding does not add up over segments;
 //   grad    a forward sweep that keeps the state entering every chunk of 8 positions in LDS, and the reverse sweep with the gradients.
 // The states lie where the segment's du and d delta will be, so there is no workspace.
@@ -90,7 +90,7 @@ __device__ __forceinline__ float sum_over_channels(float (&v)[16]) {
 
 // kGrad: the gradients from the states that enter the segment (see the top); otherwise what the segment leaves on either side.
 template <typename in_t, typename dy_t, int kSpw, bool kDwords, bool kGrad>
-__global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4) ? 2 : 3) void scan_bwd_chan_kernel(const ScanBwdArgs p, const BwdChanGeom geo) {
+__global__ __launch_bounds__(kBlock, !kGrad ? (kSpw == 4 ? 4 : 5) : kSpw == 4 && (!kDwords || sizeof(in_t) == 4) ? 2 : 3) void scan_bwd_chan_kernel(const ScanBwdArgs p, const BwdChanGeom geo) {
     constexpr int kN = kBcSets * kSpw;
     constexpr int kTile = 3 * kBcChan * kBcPitch + 2 * kSpw * kBcGroup;
     constexpr int kScratch = kTile > kWave * kBcPitch ? kTile : kWave * kBcPitch;       // also S / T of all lanes
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
         auto read_B = [&](int j, float (&v)[kBcSub]) { read8(my_bc + j * kBcGroup, v); };
         auto read_C = [&](int j, float (&v)[kBcSub]) { read8(my_bc + (kSpw + j) * kBcGroup, v); };
 
-        // what enters (leaves) the segment, where its du and d delta will be: N states and the sum of dl; N adjoints
+        // what enters (leaves) the segment, where its du and d delta will be: N states, the sum of dl and the largest; N adjoints and a share of dD
         uint8_t *h_state = reinterpret_cast<uint8_t *>(reinterpret_cast<in_t *>(p.du) + ((int64_t)b * p.dim + d) * L + begin);
         uint8_t *g_state = reinterpret_cast<uint8_t *>(reinterpret_cast<in_t *>(p.ddelta) + ((int64_t)b * p.dim + d) * L + begin);
         float h[kSpw], g[kSpw];                             // g: a_t+1 g_t+1 of the position t that is next
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
 
         auto over_quad = [](float x) { x += __shfl_xor(x, 1, kWave); return x + __shfl_xor(x, 2, kWave); };
         if constexpr (!kGrad) {
-            float dl_sum = 0.0f, dD = 0.0f;
+            float dl_sum = 0.0f, dl_max = 0.0f, dD = 0.0f;
             Raw next;
             load_rows(begin, true, next);
             for (int t = begin; t < stop; t += kBcSub) {
@@ -238,8 +238,35 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
                     g[j] = gl == 0.0f ? g[j] : fmaf(__builtin_amdgcn_exp2f(A2[j] * dl_sum), gl, g[j]);
                 }
                 dD += fmaf(own_dy[0], own_u[0], own_dy[1] * own_u[1]);
+                dl_max = fmaxf(dl_max, fmaxf(fmaxf(fmaxf(dl[0], dl[1]), fmaxf(dl[2], dl[3])), fmaxf(fmaxf(dl[4], dl[5]), fmaxf(dl[6], dl[7]))));
                 dl_sum += ((dl[0] + dl[1]) + (dl[2] + dl[3])) + ((dl[4] + dl[5]) + (dl[6] + dl[7]));
                 wave_lds_sync();
+            }
+            // An infinite gl times a product of a that has left fp32's range is NaN, where it would pass every position unless one of their a is 0: walk the
+            // positions in their own order then.
+            bool walk = false;
+#pragma unroll
+            for (int j = 0; j < kSpw; ++j) walk = walk || g[j] != g[j];
+            if (__any(walk)) {                              // uniform
+#pragma unroll
+                for (int j = 0; j < kSpw; ++j) g[j] = 0.0f;
+                for (int t = begin + (n_chunks - 1) * kBcSub; t >= begin; t -= kBcSub) {
+                    float own_dl[2], own_u[2], own_dy[2], own_raw[2];
+                    load_rows(t, true, next);
+                    stage(next, t, true, own_dl, own_u, own_dy, own_raw);
+                    wave_lds_sync();
+                    float dl[kBcSub], dy[kBcSub];
+                    read8(s_dl + ch * kBcPitch, dl);
+                    read8(s_dy + ch * kBcPitch, dy);
+#pragma unroll
+                    for (int j = 0; j < kSpw; ++j) {
+                        float Cv[kBcSub];
+                        read_C(j, Cv);
+#pragma unroll
+                        for (int i = kBcSub - 1; i >= 0; --i) g[j] = fmaf(Cv[i], dy[i], g[j]) * __builtin_amdgcn_exp2f(dl[i] * A2[j]);
+                    }
+                    wave_lds_sync();
+                }
             }
             dD = over_quad(dD);
             if (chan_ok) {
@@ -247,6 +274,7 @@ __global__ __launch_bounds__(kBlock, kSpw == 4 && (!kDwords || sizeof(in_t) == 4
                 __builtin_memcpy(g_state + sizeof(float) * (set * kSpw), g, sizeof(g));
                 if (set == 0 && (int)seg + 1 < geo.n_segs) {
                     __builtin_memcpy(h_state + sizeof(float) * kN, &dl_sum, sizeof(float));
+                    __builtin_memcpy(h_state + sizeof(float) * (kN + 1), &dl_max, sizeof(float));
                     __builtin_memcpy(g_state + sizeof(float) * kN, &dD, sizeof(float));
                 }
             }
@@ -413,8 +441,14 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanB
         }
         unsafeAtomicAdd(p.dD + d, (float)dD);
     }
-    // carry through a segment: the product of its a in two halves, so that neither leaves fp32's range before the state would; none of a state of 0
-    auto through = [&](float carry, float sum, float left) {
+    // carry through a segment: the product of its a in two halves, so that neither leaves fp32's range before the state would; none of a state of 0, and
+    // none of an infinite one: it stays infinite unless one of the a is 0 (the one of the largest dl, where A is negative), which leaves NaN
+    auto through = [&](int s, float carry, float sum, float left) {
+        if (fabsf(carry) == __builtin_inff()) {
+            float most;
+            __builtin_memcpy(&most, sums + min(s, n_segs - 2) * pitch + sizeof(float), sizeof(float));
+            return __builtin_amdgcn_exp2f(A2 * most) > 0.0f ? carry + left : __builtin_nanf("");
+        }
         const float half = __builtin_amdgcn_exp2f(0.5f * A2 * sum);
         return carry == 0.0f ? left : fmaf(carry * half, half, left);
     };
@@ -434,7 +468,7 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanB
                 const int s = first + i;
                 if (s >= n_segs) break;
                 if (s > 0) __builtin_memcpy(h_state + s * pitch, &carry, sizeof(float));
-                carry = through(carry, sum[i], left[i]);
+                carry = through(s, carry, sum[i], left[i]);
             }
         }
         return;
@@ -452,7 +486,7 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanB
             const int s = first - i;
             if (s < 0) break;
             __builtin_memcpy(g_state + s * pitch, &carry, sizeof(float));
-            carry = through(carry, sum[i], left[i]);
+            carry = through(s, carry, sum[i], left[i]);
         }
     }
 }
@@ -465,7 +499,7 @@ static int bwd_chan_segments(int L, int N, int size, int32_t &seg_len) {
         seg_len = len;
         if (n == 1) return 1;
         const int last = L - (n - 1) * len;
-        if (last >= room && len >= room + 4 / size) return n;
+        if (last >= room && len >= room + 8 / size) return n;
     }
     return 0;
 }
