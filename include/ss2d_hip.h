@@ -181,6 +181,17 @@ typedef struct ss2d_scan_bwd_params {
 int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *params, void *stream);
 
 /*
+ * Which kernel ss2d_selective_scan_bwd launches for these params (>= 0), or the status of a call that launches none.  Nothing is
+ * launched; as ss2d_selective_scan_kernel.
+ */
+#define SS2D_SCAN_BWD_KERNEL_NONE 0   /* empty problem                                                            */
+#define SS2D_SCAN_BWD_KERNEL_ROWS 1   /* more than 32 states: one wavefront per (batch, channel) row               */
+#define SS2D_SCAN_BWD_KERNEL_ONE 2    /* one state: positions in lanes                                            */
+#define SS2D_SCAN_BWD_KERNEL_STATES 3 /* 2 to 32 states: positions in lanes, a wavefront per four states           */
+#define SS2D_SCAN_BWD_KERNEL_CHAN 4   /* 4, 8 or 16 states: a channel per lane, rows cut into segments             */
+int ss2d_selective_scan_bwd_kernel(const ss2d_scan_bwd_params *params);
+
+/*
  * Around it: up to SS2D_CLEAR_MAX buffers of 4-byte elements on 16-byte boundaries set to zero (the accumulators of the call
  * above, selective_scan_oflex.cpp:310-330), and two fp32 tensors rounded to bf16 / fp16 (dB and dC, :346), one launch each.
  */

@@ -126,6 +126,36 @@ def test_scan_kernel_choice_does_not_depend_on_the_chunk_state_output():
     assert len(_lib.SCAN_KERNEL_NAMES) == 6
 
 
+def _scan_bwd_plan(batch, dim, L, N, G, dtype=_lib.SS2D_BF16, base=1 << 32):
+    """ss2d_selective_scan_bwd_kernel for dense tensors of these sizes at made-up, 256-byte aligned addresses far apart."""
+    p = _lib.ScanBwdParams()
+    p.batch, p.dim, p.seqlen, p.dstate, p.n_groups, p.delta_dim = batch, dim, L, N, G, dim
+    p.in_dtype, p.dout_dtype, p.delta_softplus = dtype, _lib.SS2D_F32, 1
+    p.u, p.delta, p.A, p.B, p.C, p.dout, p.du, p.ddelta, p.dA, p.dB, p.dC = (base * k for k in range(1, 12))
+    p.u_batch_stride, p.u_d_stride = dim * L, L
+    p.delta_batch_stride, p.delta_d_stride = dim * L, L
+    p.dout_batch_stride, p.dout_d_stride = dim * L, L
+    p.A_d_stride, p.A_dstate_stride = N, 1
+    p.B_batch_stride, p.B_group_stride, p.B_dstate_stride = G * N * L, N * L, L
+    p.C_batch_stride, p.C_group_stride, p.C_dstate_stride = G * N * L, N * L, L
+    return _lib.lib().ss2d_selective_scan_bwd_kernel(p)
+
+
+def test_scan_bwd_kernel_choice():
+    """The query names the kernel that the call would launch, and the status of a call that would be refused."""
+    name = lambda *args: _lib.SCAN_BWD_KERNEL_NAMES[_scan_bwd_plan(*args)]
+    shapes = {  # batch, dim = 4 * d_inner, L, N -> kernel
+        (64, 384, 3136, 1): "one", (64, 768, 784, 1): "one", (16, 768, 784, 16): "chan", (16, 768, 196, 16): "chan", (1, 384, 196, 16): "states",
+        (16, 384, 784, 2): "states", (16, 48, 49, 16): "states", (1, 96, 3136, 16): "chan", (2, 16, 300, 40): "rows",
+    }
+    for (batch, dim, L, N), kernel in shapes.items():
+        assert name(batch, dim, L, N, 4) == kernel, (batch, dim, L, N)
+    assert name(0, 384, 3136, 1, 4) == "none"
+    assert _scan_bwd_plan(2, 384, 3136, 1, 5) == _lib.SS2D_EINVAL
+    assert _scan_bwd_plan(1, 16, 400_000, 40, 4) == _lib.SS2D_ENOTSUP
+    assert _lib.lib().ss2d_selective_scan_bwd_kernel(None) == _lib.SS2D_EINVAL
+
+
 def test_host_api_rejects_cpu_tensors_and_unsupported_modes():
     import torch
     import vmamba_amd as va

@@ -43,6 +43,13 @@ def compare(got, want, tol, what):
         assert err <= tol * scale + tol * 1e-3, f"{what} {name}: max err {err} vs scale {scale}"
 
 
+def bwd_kernel_of(u, delta, A, B, C, dout):
+    """Name of the kernel the library picks for these tensors once they sit on the GPU."""
+    from vmamba_amd.csms6s import scan_bwd_kernel_name
+    u, delta, A, B, C, dout = (t.to(DEV) for t in (u, delta, A, B, C, dout))
+    return scan_bwd_kernel_name(u, delta, A, B, C, dout, torch.empty(u.shape, device=DEV, dtype=u.dtype), torch.empty(u.shape, device=DEV, dtype=u.dtype))
+
+
 CASES = [
     # batch, dim, G, N, L, delta_dim, softplus
     (2, 4, 1, 1, 40, None, True),          # one short pass
@@ -139,6 +146,7 @@ def test_scan_bwd_channel_per_lane(case, dtype):
     print("CASE scan-bwd-chan", case, dtype, flush=True)
     u, delta, A, B, C, D, bias, dout = make(sum(map(int, case[:5])), batch, dim, G, N, L, dtype, delta_dim, softplus)
     dout = dout.to(dtype) if L % 3 == 0 else dout
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
     want = torch_ref.selective_scan_grads(u.float(), delta.float(), A, B.float(), C.float(), D, bias, dout.float(), softplus)
     got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, softplus, 1)
     compare(got, want, 1e-4 if dtype == torch.float32 else 3e-2, "channel per lane")
@@ -151,6 +159,7 @@ def test_scan_bwd_channel_per_lane_strided_views(dtype):
     batch, dim, N, L = 2, 50, 16, 600
     u, delta, A, B, C, D, bias, dout = [t.to(DEV) for t in make(3, batch, dim, 1, N, L, dtype)]
     want = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
 
     def view(t, pitch):
         rows = t.reshape(-1, t.shape[-1])
@@ -174,6 +183,7 @@ def test_scan_bwd_channel_per_lane_keeps_channels_apart():
     last one's constants, included."""
     batch, dim, N, L = 1, 50, 16, 600
     u, delta, A, B, C, D, bias, dout = [t.to(DEV) for t in make(4, batch, dim, 1, N, L, torch.float32)]
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
     want = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
     u[0, 49, 300] = float("nan")
     got = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
@@ -187,10 +197,11 @@ def test_scan_bwd_channel_per_lane_lanes_without_a_channel_add_nothing(L):
     """33 channels per group: 15 lanes of the third wavefront have none.  The last channel's bias alone would let their decay overflow (softplus off,
     exp(-20 * -30)), where its own steps are small; an infinite C makes g of a zero dout NaN.  dB and dC are the real channels' sums."""
     print("CASE scan-bwd-chan-idle-lanes", L, flush=True)
-    batch, dim, N = 64 if L == 72 else 1, 33, 16
+    batch, dim, N = 96 if L == 72 else 1, 33, 16
     u, delta, A, B, C, D, bias, dout = make(6, batch, dim, 1, N, L, torch.float32, softplus=False)
     A[32], bias[32] = -20.0, -30.0
     delta[:, 32] += 30.0
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
     want = torch_ref.selective_scan_grads(u, delta, A, B, C, D, bias, dout, False)
     got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)
     compare(got[3:5], want[3:5], 1e-4, "overflowing decay")
@@ -213,6 +224,7 @@ def test_scan_bwd_channel_per_lane_infinite_states(N, L, dtype):
     A, delta, bias, D = torch.full_like(A, -1.0), 5.0 + delta.abs(), torch.zeros_like(bias), D.abs()
     call = lambda: [t.double().cpu() for t in va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)]
     u[0, 3, first] = inf
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
     du, ddelta, dA, dB, dC = call()[:5]
     assert bool((dC[0, 0, :, first:] == inf).all()) and bool(dC[0, 0, :, :first].isfinite().all())
     assert bool((dB[0, 0, :, first] == inf).all()) and bool(dB[0, 0, :, :first].isfinite().all()) and bool(dB[0, 0, :, first + 1:].isfinite().all())

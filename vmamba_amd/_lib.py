@@ -19,6 +19,7 @@ ABI_VERSION = 1
 
 SCAN_KERNEL_NONE, SCAN_KERNEL_ROW, SCAN_KERNEL_ROW4, SCAN_KERNEL_FLAT, SCAN_KERNEL_SMALL, SCAN_KERNEL_CHAN = range(6)
 SCAN_KERNEL_NAMES = ("none", "row", "row4", "flat", "small", "chan")
+SCAN_BWD_KERNEL_NAMES = ("none", "rows", "one", "states", "chan")
 
 EXPORTS = ("ss2d_abi_version", "ss2d_strerror", "ss2d_cross_scan", "ss2d_cross_merge", "ss2d_selective_scan_fwd",
            "ss2d_selective_scan_kernel", "ss2d_selective_scan_fwd_maps",
@@ -26,7 +27,7 @@ EXPORTS = ("ss2d_abi_version", "ss2d_strerror", "ss2d_cross_scan", "ss2d_cross_m
            "ss2d_dwconv3x3_silu_f32", "ss2d_dwconv3x3_silu_bwd", "ss2d_dwconv3x3_silu_bwd_workspace_bytes", "ss2d_cross_scan_1b1", "ss2d_core_fwd",
            "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_forward_core", "ss2d_forward_core_workspace_bytes", "ss2d_block_fwd", "ss2d_block_workspace_bytes", "ss2d_few_rows_bytes", "ss2d_few_applies", "ss2d_x_proj_few", "ss2d_core_few", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
            "ss2d_x_proj", "ss2d_x_proj_applies", "ss2d_x_proj_f32", "ss2d_dt_proj", "ss2d_dt_proj_f32", "ss2d_dt_proj_masked", "ss2d_cross_scan_flex", "ss2d_cross_scan_flex_ws", "ss2d_cross_scan_flex_static", "ss2d_cross_merge_flex",
-           "ss2d_selective_scan_bwd", "ss2d_clear", "ss2d_round_pair", "ss2d_transpose_bcl", "ss2d_mlp_fused", "ss2d_linear_cl", "ss2d_linear_rows", "ss2d_linear_tiles", "ss2d_conv3x3s2_cl", "ss2d_linear_dw_f32", "ss2d_layer_norm_bwd_f32", "ss2d_layer_norm_bwd_f32_workspace_bytes", "ss2d_column_sums_f32", "ss2d_column_sums_f32_workspace_bytes", "ss2d_product_f32", "ss2d_product_f32_workspace_bytes", "ss2d_linear_dw_f32_workspace_bytes", "ss2d_linear_cf_ln", "ss2d_stem_conv_ln_gelu", "ss2d_stem_conv2_ln", "ss2d_mean_pool_cl")
+           "ss2d_selective_scan_bwd", "ss2d_selective_scan_bwd_kernel", "ss2d_clear", "ss2d_round_pair", "ss2d_transpose_bcl", "ss2d_mlp_fused", "ss2d_linear_cl", "ss2d_linear_rows", "ss2d_linear_tiles", "ss2d_conv3x3s2_cl", "ss2d_linear_dw_f32", "ss2d_layer_norm_bwd_f32", "ss2d_layer_norm_bwd_f32_workspace_bytes", "ss2d_column_sums_f32", "ss2d_column_sums_f32_workspace_bytes", "ss2d_product_f32", "ss2d_product_f32_workspace_bytes", "ss2d_linear_dw_f32_workspace_bytes", "ss2d_linear_cf_ln", "ss2d_stem_conv_ln_gelu", "ss2d_stem_conv2_ln", "ss2d_mean_pool_cl")
 
 
 class ScanParams(ctypes.Structure):
@@ -205,6 +206,8 @@ def lib():
         L.ss2d_cross_merge_flex.argtypes = [ctypes.c_void_p] * 2 + [ctypes.c_int] * 10 + [ctypes.c_void_p]
         L.ss2d_selective_scan_bwd.restype = ctypes.c_int
         L.ss2d_selective_scan_bwd.argtypes = [ctypes.POINTER(ScanBwdParams), ctypes.c_void_p]
+        L.ss2d_selective_scan_bwd_kernel.restype = ctypes.c_int
+        L.ss2d_selective_scan_bwd_kernel.argtypes = [ctypes.POINTER(ScanBwdParams)]
         L.ss2d_clear.restype = ctypes.c_int
         L.ss2d_clear.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_int64), ctypes.c_int, ctypes.c_void_p]
         L.ss2d_round_pair.restype = ctypes.c_int

@@ -138,6 +138,34 @@ def selective_scan_from_map(x, delta, A, B, C, D=None, delta_bias=None, delta_so
     return out
 
 
+def _scan_bwd_params(u, delta, A, B, C, D, delta_bias, dout, delta_softplus, du, ddelta, dA, dB, dC, dD, dbias):
+    """struct ss2d_scan_bwd_params of tensors that are what selective_scan_bwd checks them to be."""
+    ptr = lambda t: None if t is None else t.data_ptr()
+    p = _lib.ScanBwdParams()
+    p.batch, p.dim, p.seqlen = u.shape
+    p.dstate, p.n_groups, p.delta_dim = A.size(1), B.size(1), delta.size(1)
+    p.in_dtype, p.dout_dtype = _DTYPE_CODE[u.dtype], _DTYPE_CODE[dout.dtype]
+    p.delta_softplus = int(bool(delta_softplus))
+    p.u, p.delta, p.A, p.B, p.C, p.dout, p.D, p.delta_bias = (ptr(t) for t in (u, delta, A, B, C, dout, D, delta_bias))
+    p.du, p.ddelta, p.dA, p.dB, p.dC, p.dD, p.ddelta_bias = (ptr(t) for t in (du, ddelta, dA, dB, dC, dD, dbias))
+    p.u_batch_stride, p.u_d_stride = u.stride(0), u.stride(1)
+    p.delta_batch_stride, p.delta_d_stride = delta.stride(0), delta.stride(1)
+    p.A_d_stride, p.A_dstate_stride = A.stride(0), A.stride(1)
+    p.B_batch_stride, p.B_group_stride, p.B_dstate_stride = B.stride(0), B.stride(1), B.stride(2)
+    p.C_batch_stride, p.C_group_stride, p.C_dstate_stride = C.stride(0), C.stride(1), C.stride(2)
+    p.dout_batch_stride, p.dout_d_stride = dout.stride(0), dout.stride(1)
+    return p
+
+
+def scan_bwd_kernel_name(u, delta, A, B, C, dout, du, ddelta):
+    """Which kernel of the library makes the gradients of these (already allocated) tensors: one of _lib.SCAN_BWD_KERNEL_NAMES.
+    Nothing is launched (ss2d_selective_scan_bwd_kernel)."""
+    p = _scan_bwd_params(u, delta, A, B, C, None, None, dout, True, du, ddelta, A, B, C, None, None)     # (the sums' addresses play no part)
+    rc = _lib.lib().ss2d_selective_scan_bwd_kernel(p)
+    _lib.check(min(rc, 0), "ss2d_selective_scan_bwd_kernel")
+    return _lib.SCAN_BWD_KERNEL_NAMES[rc]
+
+
 def selective_scan_bwd(u, delta, A, B, C, D, delta_bias, dout, x=None, delta_softplus=False, nrows=1):
     """Python twin of ``selective_scan_cuda_oflex.bwd``: returns [du, ddelta, dA, dB, dC, dD, ddelta_bias]
     (selective_scan_oflex.cpp:233-355).  ``x`` (the forward's chunk states) and ``nrows`` are accepted and unused:
@@ -181,23 +209,7 @@ def selective_scan_bwd(u, delta, A, B, C, D, delta_bias, dout, x=None, delta_sof
     dD = zeroed[3] if D is not None else None
     dbias = zeroed[-1] if delta_bias is not None else None
 
-    p = _lib.ScanBwdParams()
-    p.batch, p.dim, p.seqlen, p.dstate, p.n_groups, p.delta_dim = batch, dim, seqlen, dstate, n_groups, delta_dim
-    p.in_dtype, p.dout_dtype = _DTYPE_CODE[u.dtype], _DTYPE_CODE[dout.dtype]
-    p.delta_softplus = int(bool(delta_softplus))
-    p.u, p.delta, p.A, p.B, p.C, p.dout = (u.data_ptr(), delta.data_ptr(), A.data_ptr(), B.data_ptr(), C.data_ptr(),
-                                           dout.data_ptr())
-    p.D = D.data_ptr() if D is not None else None
-    p.delta_bias = delta_bias.data_ptr() if delta_bias is not None else None
-    p.du, p.ddelta, p.dA, p.dB, p.dC = du.data_ptr(), ddelta.data_ptr(), dA.data_ptr(), dB.data_ptr(), dC.data_ptr()
-    p.dD = dD.data_ptr() if dD is not None else None
-    p.ddelta_bias = dbias.data_ptr() if dbias is not None else None
-    p.u_batch_stride, p.u_d_stride = u.stride(0), u.stride(1)
-    p.delta_batch_stride, p.delta_d_stride = delta.stride(0), delta.stride(1)
-    p.A_d_stride, p.A_dstate_stride = A.stride(0), A.stride(1)
-    p.B_batch_stride, p.B_group_stride, p.B_dstate_stride = B.stride(0), B.stride(1), B.stride(2)
-    p.C_batch_stride, p.C_group_stride, p.C_dstate_stride = C.stride(0), C.stride(1), C.stride(2)
-    p.dout_batch_stride, p.dout_d_stride = dout.stride(0), dout.stride(1)
+    p = _scan_bwd_params(u, delta, A, B, C, D, delta_bias, dout, delta_softplus, du, ddelta, dA, dB, dC, dD, dbias)
     if u.numel():
         rc = _lib.launch(u, _lib.lib().ss2d_selective_scan_bwd, p)
         _lib.check(rc, "ss2d_selective_scan_bwd")

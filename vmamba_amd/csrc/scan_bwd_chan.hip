@@ -518,8 +518,25 @@ static bool bwd_chan_pays(const ScanBwdArgs &a) {
     return units >= (a.L > 256 ? 192 : a.L > 128 ? 640 : 256) && (a.N == 16 || a.L <= 208 || a.L > 256);
 }
 
+// False: no grid for it.
+static bool bwd_chan_geom(const ScanBwdArgs &a, int in_size, BwdChanGeom &geo, uint32_t &n_wg) {
+    geo = {};
+    geo.n_segs = bwd_chan_segments(a.L, a.N, in_size, geo.seg_len);
+    const int64_t groups = a.dim / a.dim_per_group;
+    geo.n_cb = (a.dim_per_group + 63) / 64;
+    const int64_t n = (int64_t)a.batch * groups * geo.n_cb * geo.n_segs;
+    if (geo.n_segs == 0 || n > 0x7fffffff) return false;
+    geo.div_cb = make_fastdiv((uint32_t)geo.n_cb);
+    geo.div_groups = make_fastdiv((uint32_t)groups);
+    geo.div_segs = make_fastdiv((uint32_t)geo.n_segs);
+    n_wg = (uint32_t)n;
+    return true;
+}
+
 bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size) {
-    if ((a.N != 4 && a.N != 8 && a.N != 16) || a.dim_per_group < kBcChan || !bwd_chan_pays(a)) return false;
+    BwdChanGeom geo;
+    uint32_t n_wg;
+    if ((a.N != 4 && a.N != 8 && a.N != 16) || a.dim_per_group < kBcChan || !bwd_chan_pays(a) || !bwd_chan_geom(a, in_size, geo, n_wg)) return false;
     // the gradients' memory holds the segments' states between the passes
     auto apart = [&](const void *x, int64_t elems, int size) {
         const uintptr_t first = reinterpret_cast<uintptr_t>(x), last = first + (uintptr_t)(elems * size);
@@ -546,22 +563,16 @@ bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size) {
 
 template <typename in_t, typename dy_t, int kSpw, bool kDwords>
 static int launch_bwd_chan(const ScanBwdArgs &a, hipStream_t stream) {
-    BwdChanGeom geo = {};
-    geo.n_segs = bwd_chan_segments(a.L, a.N, (int)sizeof(in_t), geo.seg_len);
-    const int64_t groups = a.dim / a.dim_per_group;
-    geo.n_cb = (a.dim_per_group + 63) / 64;
-    const int64_t n = (int64_t)a.batch * groups * geo.n_cb * geo.n_segs;
-    if (geo.n_segs == 0 || n > 0x7fffffff) return SS2D_ENOTSUP;
-    geo.div_cb = make_fastdiv((uint32_t)geo.n_cb);
-    geo.div_groups = make_fastdiv((uint32_t)groups);
-    geo.div_segs = make_fastdiv((uint32_t)geo.n_segs);
+    BwdChanGeom geo;
+    uint32_t n;
+    if (!bwd_chan_geom(a, (int)sizeof(in_t), geo, n)) return SS2D_ENOTSUP;
     if (geo.n_segs > 1) {
         const uint32_t n_items = (uint32_t)((int64_t)a.batch * a.dim * a.N);
-        hipLaunchKernelGGL((scan_bwd_chan_kernel<in_t, dy_t, kSpw, kDwords, false>), dim3((uint32_t)n), dim3(kBlock), 0, stream, a, geo);
+        hipLaunchKernelGGL((scan_bwd_chan_kernel<in_t, dy_t, kSpw, kDwords, false>), dim3(n), dim3(kBlock), 0, stream, a, geo);
         hipLaunchKernelGGL((scan_bwd_chan_carry_kernel<in_t>), dim3((n_items + kBlock - 1) / kBlock, 2), dim3(kBlock), 0, stream, a, geo.seg_len, geo.n_segs, n_items,
                            make_fastdiv((uint32_t)a.N), make_fastdiv((uint32_t)a.dim));
     }
-    hipLaunchKernelGGL((scan_bwd_chan_kernel<in_t, dy_t, kSpw, kDwords, true>), dim3((uint32_t)n), dim3(kBlock), 0, stream, a, geo);
+    hipLaunchKernelGGL((scan_bwd_chan_kernel<in_t, dy_t, kSpw, kDwords, true>), dim3(n), dim3(kBlock), 0, stream, a, geo);
     return launch_status();
 }
 

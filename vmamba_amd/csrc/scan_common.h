@@ -45,7 +45,7 @@ struct ScanBwdArgs {
     int64_t g_bs, g_gs, g_ns;      // strides of dB / dC (contiguous (batch, groups, N, L))
 };
 
-// scan_bwd_chan.hip: the backward with a channel per lane.  SS2D_ENOTSUP: nothing launched.
+// scan_bwd_chan.hip: the backward with a channel per lane, for what scan_bwd_chan_takes.
 bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size);
 int launch_scan_bwd_chan(const ScanBwdArgs &a, int in_dtype, int dout_dtype, hipStream_t stream);
 

@@ -850,10 +850,19 @@ __global__ __launch_bounds__(512, 2) void scan_bwd_states_kernel(const ScanBwdAr
     }
 }
 
-}  // namespace ss2d
+// How the register-summing kernels walk a problem, and which kernel that is.
+struct BwdPlan {
+    int32_t kernel;             // SS2D_SCAN_BWD_KERNEL_*
+    int32_t items;              // positions per lane
+    bool vec;                   // rows of whole dwords
+    int32_t n_waves, chunk, cpg;            // wavefronts and channels per workgroup, workgroups per group
+    int64_t n_wg;
+    size_t smem;
+};
 
-extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stream) {
-    using namespace ss2d;
+// The arguments in the kernels' terms and the kernel for them; a status where none is launched (SS2D_OK: nothing to do).
+static int plan_scan_bwd(const ss2d_scan_bwd_params *q, ScanBwdArgs &a, BwdPlan &plan) {
+    plan = {};
     if (!q) return SS2D_EINVAL;
     if (q->batch < 0 || q->dim < 0 || q->seqlen < 0) return SS2D_EINVAL;
     if (q->dstate <= 0 || q->dstate > 256 || q->n_groups <= 0 || q->delta_dim <= 0) return SS2D_EINVAL;
@@ -867,7 +876,6 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
     if ((q->delta_bias == nullptr) != (q->ddelta_bias == nullptr)) return SS2D_EINVAL;
     if ((int64_t)q->batch * q->dim > 0x7fffffff - kWavesPerWg) return SS2D_ENOTSUP;
 
-    ScanBwdArgs a;
     a.u = q->u; a.delta = q->delta; a.B = q->B; a.C = q->C; a.dout = q->dout;
     a.A = (const float *)q->A; a.D = (const float *)q->D; a.bias = (const float *)q->delta_bias;
     a.du = q->du; a.ddelta = q->ddelta;
@@ -885,25 +893,11 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
     a.C_bs = q->C_batch_stride; a.C_gs = q->C_group_stride; a.C_ns = q->C_dstate_stride;
     a.do_bs = q->dout_batch_stride; a.do_ds = q->dout_d_stride;
     a.g_ns = q->seqlen; a.g_gs = (int64_t)q->dstate * q->seqlen; a.g_bs = (int64_t)q->n_groups * a.g_gs;
-    hipStream_t s = (hipStream_t)stream;
-    // whether rows can be read and written in groups of `items` elements: 16-byte pieces at most, so the group's alignment
-    // is that of its piece
     const int in_size = q->in_dtype == SS2D_F32 ? 4 : 2, dy_size = q->dout_dtype == SS2D_F32 ? 4 : 2;
-    // (of the element-wise kernel; the others need dwords only, and single precision nothing)
-    auto groups_ok = [&](int items) {
-        const int64_t in_vec = items * in_size > 16 ? 16 / in_size : items, dy_vec = items * dy_size > 16 ? 16 / dy_size : items;
-        auto aligned = [](const void *ptr, int64_t bytes) { return (reinterpret_cast<uintptr_t>(ptr) & (uintptr_t)(bytes - 1)) == 0; };
-        for (const void *ptr : {q->u, q->delta, q->B, q->C, (const void *)q->du, (const void *)q->ddelta})
-            if (!aligned(ptr, in_vec * in_size)) return false;
-        if (!aligned(q->dout, dy_vec * dy_size) || q->seqlen % in_vec != 0 || q->seqlen % dy_vec != 0) return false;
-        for (int64_t st : {a.u_bs, a.u_ds, a.dl_bs, a.dl_ds, a.B_bs, a.B_gs, a.B_ns, a.C_bs, a.C_gs, a.C_ns})
-            if (st % in_vec != 0) return false;
-        return a.do_bs % dy_vec == 0 && a.do_ds % dy_vec == 0;
-    };
     // several states and enough channels per group: one channel per lane
     if (scan_bwd_chan_takes(a, in_size, dy_size)) {
-        const int rc = launch_scan_bwd_chan(a, q->in_dtype, q->dout_dtype, s);
-        if (rc != SS2D_ENOTSUP) return rc;                  // (before any launch)
+        plan.kernel = SS2D_SCAN_BWD_KERNEL_CHAN;
+        return SS2D_OK;
     }
     auto dwords_ok = [&](int items) {                            // rows of whole dwords (with one position per lane elements are read)
         if (items == 1) return true;
@@ -924,9 +918,7 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
         // with 1: 166) and with several states, whose B, C and sums fill the registers; 1 for rows that fit 64 lanes
         // (768 x 7 x 7: 70; with 4: 144).
         const int items = a.L <= kWave ? 1 : a.L <= 4 * kWave || !one ? 4 : 8;
-        const bool vec = dwords_ok(items);
-        const int kI = items;
-        const int n_pass = (a.L + kWave * kI - 1) / (kWave * kI);
+        const int n_pass = (a.L + kWave * items - 1) / (kWave * items);
         const int n_waves = one ? kWavesPerWg : (a.N + kStates - 1) / kStates;
         // Channels per workgroup: more of them mean fewer atomics on dB / dC (one per entry and workgroup), fewer mean more
         // wavefronts.  The grid is filled first -- one state: 8 wavefronts per SIMD, as three at a time are resident (96 x 56 x 56,
@@ -941,7 +933,7 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
         int64_t chunk = a.dim_per_group * images / want_wg;
         chunk = chunk > 24 ? 24 : chunk < least ? least : chunk;
         if (chunk > a.dim_per_group) chunk = a.dim_per_group;
-        const size_t fixed = (size_t)(one ? 2 : 5) * n_waves * kWave * kI * sizeof(float);
+        const size_t fixed = (size_t)(one ? 2 : 5) * n_waves * kWave * items * sizeof(float);
         auto smem_of = [&](int64_t c) {
             const size_t per_wave = one ? (size_t)((c + kWavesPerWg - 1) / kWavesPerWg) * n_pass : (size_t)c * n_pass * 4;
             return fixed + n_waves * per_wave * sizeof(float);
@@ -951,37 +943,75 @@ extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stre
         chunk = (a.dim_per_group + cpg - 1) / cpg;               // even split
         const int64_t n = images * cpg;
         const size_t smem = smem_of(chunk);
+        plan.items = items; plan.vec = dwords_ok(items);
+        plan.n_waves = n_waves; plan.chunk = (int)chunk; plan.cpg = (int)cpg;
+        plan.n_wg = n; plan.smem = smem;
         if (n <= 0x7fffffff && smem <= 160 * 1024) {
-            const dim3 grid((uint32_t)n), block(n_waves * kWave);
+            plan.kernel = one ? SS2D_SCAN_BWD_KERNEL_ONE : SS2D_SCAN_BWD_KERNEL_STATES;
+            return SS2D_OK;
+        }
+    }
+    plan.smem = (size_t)kWavesPerWg * (a.n_pass + 2) * a.N * sizeof(float);
+    if (plan.smem > 48 * 1024) return SS2D_ENOTSUP;        // very long rows x many states: the per-pass states do not fit LDS
+    // Rows read and written in groups of 8 elements: 16-byte pieces at most, so a group's alignment is that of its piece.  (The kernels above need dwords
+    // only, and single precision nothing.)
+    const int64_t in_vec = 16 / in_size, dy_vec = 16 / dy_size;
+    auto aligned16 = [](const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
+    bool vec = q->seqlen % in_vec == 0 && q->seqlen % dy_vec == 0 && a.do_bs % dy_vec == 0 && a.do_ds % dy_vec == 0;
+    for (const void *ptr : {q->u, q->delta, q->B, q->C, q->dout, (const void *)q->du, (const void *)q->ddelta}) vec = vec && aligned16(ptr);
+    for (int64_t st : {a.u_bs, a.u_ds, a.dl_bs, a.dl_ds, a.B_bs, a.B_gs, a.B_ns, a.C_bs, a.C_gs, a.C_ns}) vec = vec && st % in_vec == 0;
+    a.vec_ok = vec ? 1 : 0;
+    plan.n_wg = (a.rows + kWavesPerWg - 1) / kWavesPerWg;
+    plan.kernel = SS2D_SCAN_BWD_KERNEL_ROWS;
+    return SS2D_OK;
+}
+
+}  // namespace ss2d
+
+extern "C" int ss2d_selective_scan_bwd_kernel(const ss2d_scan_bwd_params *q) {
+    using namespace ss2d;
+    ScanBwdArgs a;
+    BwdPlan plan;
+    const int rc = plan_scan_bwd(q, a, plan);
+    return rc != SS2D_OK ? rc : plan.kernel;
+}
+
+extern "C" int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *q, void *stream) {
+    using namespace ss2d;
+    ScanBwdArgs a;
+    BwdPlan plan;
+    const int rc = plan_scan_bwd(q, a, plan);
+    if (rc != SS2D_OK || plan.kernel == SS2D_SCAN_BWD_KERNEL_NONE) return rc;
+    hipStream_t s = (hipStream_t)stream;
+    if (plan.kernel == SS2D_SCAN_BWD_KERNEL_CHAN) return launch_scan_bwd_chan(a, q->in_dtype, q->dout_dtype, s);
+    const dim3 grid((uint32_t)plan.n_wg);
+    if (plan.kernel != SS2D_SCAN_BWD_KERNEL_ROWS) {
+        const bool one = plan.kernel == SS2D_SCAN_BWD_KERNEL_ONE;
+        const dim3 block(plan.n_waves * kWave);
 #define SS2D_BWD_LAUNCH(IN, DY, KI, VEC)                                                                                        \
     do {                                                                                                                        \
-        if (KI == 8 || one) hipLaunchKernelGGL((scan_bwd_one_kernel<IN, DY, KI, VEC>), grid, block, smem, s, a, (int)chunk, (int)cpg, q->n_groups); \
-        else hipLaunchKernelGGL((scan_bwd_states_kernel<IN, DY, KI == 8 ? 4 : KI, VEC>), grid, block, smem, s, a, (int)chunk, (int)cpg, q->n_groups);  \
+        if (KI == 8 || one) hipLaunchKernelGGL((scan_bwd_one_kernel<IN, DY, KI, VEC>), grid, block, plan.smem, s, a, plan.chunk, plan.cpg, q->n_groups); \
+        else hipLaunchKernelGGL((scan_bwd_states_kernel<IN, DY, KI == 8 ? 4 : KI, VEC>), grid, block, plan.smem, s, a, plan.chunk, plan.cpg, q->n_groups);  \
     } while (0)
 #define SS2D_BWD_ITEMS(IN, DY)                                                                                                  \
     do {                                                                                                                        \
-        if (kI == 8 && vec) SS2D_BWD_LAUNCH(IN, DY, 8, true);                                                                   \
-        else if (kI == 8) SS2D_BWD_LAUNCH(IN, DY, 8, sizeof(IN) == 4);                                                              \
-        else if (kI == 1) SS2D_BWD_LAUNCH(IN, DY, 1, true);                                                                     \
-        else if (vec) SS2D_BWD_LAUNCH(IN, DY, 4, true);                                                                         \
-        else SS2D_BWD_LAUNCH(IN, DY, 4, sizeof(IN) == 4);                                                                                 \
+        if (plan.items == 8 && plan.vec) SS2D_BWD_LAUNCH(IN, DY, 8, true);                                                      \
+        else if (plan.items == 8) SS2D_BWD_LAUNCH(IN, DY, 8, sizeof(IN) == 4);                                                  \
+        else if (plan.items == 1) SS2D_BWD_LAUNCH(IN, DY, 1, true);                                                             \
+        else if (plan.vec) SS2D_BWD_LAUNCH(IN, DY, 4, true);                                                                    \
+        else SS2D_BWD_LAUNCH(IN, DY, 4, sizeof(IN) == 4);                                                                       \
     } while (0)
-            if (q->in_dtype == SS2D_F32) SS2D_BWD_ITEMS(float, float);
-            else if (q->in_dtype == SS2D_BF16) { if (q->dout_dtype == SS2D_F32) SS2D_BWD_ITEMS(bf16_t, float); else SS2D_BWD_ITEMS(bf16_t, bf16_t); }
-            else { if (q->dout_dtype == SS2D_F32) SS2D_BWD_ITEMS(f16_t, float); else SS2D_BWD_ITEMS(f16_t, f16_t); }
+        if (q->in_dtype == SS2D_F32) SS2D_BWD_ITEMS(float, float);
+        else if (q->in_dtype == SS2D_BF16) { if (q->dout_dtype == SS2D_F32) SS2D_BWD_ITEMS(bf16_t, float); else SS2D_BWD_ITEMS(bf16_t, bf16_t); }
+        else { if (q->dout_dtype == SS2D_F32) SS2D_BWD_ITEMS(f16_t, float); else SS2D_BWD_ITEMS(f16_t, f16_t); }
 #undef SS2D_BWD_ITEMS
 #undef SS2D_BWD_LAUNCH
-            return launch_status();
-        }
+        return launch_status();
     }
-    const size_t smem = (size_t)kWavesPerWg * (a.n_pass + 2) * a.N * sizeof(float);
-    if (smem > 48 * 1024) return SS2D_ENOTSUP;        // very long rows x many states: the per-pass states do not fit LDS
-    a.vec_ok = groups_ok(8) ? 1 : 0;
-    const uint32_t n_wg = (uint32_t)((a.rows + kWavesPerWg - 1) / kWavesPerWg);
 #define SS2D_BWD_LAUNCH(IN, DY)                                                                                         \
     do {                                                                                                                \
-        if (a.softplus) hipLaunchKernelGGL((scan_bwd_kernel<IN, DY, true>), dim3(n_wg), dim3(kBlock), smem, s, a);      \
-        else hipLaunchKernelGGL((scan_bwd_kernel<IN, DY, false>), dim3(n_wg), dim3(kBlock), smem, s, a);                \
+        if (a.softplus) hipLaunchKernelGGL((scan_bwd_kernel<IN, DY, true>), grid, dim3(kBlock), plan.smem, s, a);       \
+        else hipLaunchKernelGGL((scan_bwd_kernel<IN, DY, false>), grid, dim3(kBlock), plan.smem, s, a);                 \
     } while (0)
     if (q->in_dtype == SS2D_F32) SS2D_BWD_LAUNCH(float, float);
     else if (q->in_dtype == SS2D_BF16) { if (q->dout_dtype == SS2D_F32) SS2D_BWD_LAUNCH(bf16_t, float); else SS2D_BWD_LAUNCH(bf16_t, bf16_t); }
