@@ -150,6 +150,8 @@ def test_scan_bwd_kernel_choice():
     }
     for (batch, dim, L, N), kernel in shapes.items():
         assert name(batch, dim, L, N, 4) == kernel, (batch, dim, L, N)
+    for L in list(range(512, 2600)) + [3025, 3481, 3844, 3969, 65537]:      # every length of the rule's range, not only those that equal segments fill
+        assert all(name(1, 256, L, N, 4, dtype) == "chan" for N in (8, 16) for dtype in (_lib.SS2D_BF16, _lib.SS2D_F32)), L
     assert name(0, 384, 3136, 1, 4) == "none"
     assert _scan_bwd_plan(2, 384, 3136, 1, 5) == _lib.SS2D_EINVAL
     assert _scan_bwd_plan(1, 16, 400_000, 40, 4) == _lib.SS2D_ENOTSUP

@@ -129,13 +129,15 @@ def test_scan_bwd_odd_rows(N, L, dtype, dout_float):
     compare(got, want, 1e-4 if dtype == torch.float32 else 3e-2, "odd rows")
 
 
-# A channel per lane (scan_bwd_chan.hip): rows of one segment (up to 72 positions, many of them), of two, and of many; the last chunk of 8 positions with
+# A channel per lane (scan_bwd_chan.hip): rows of one segment (up to 72 positions, many of them), of two, and of many, equal or not; the last chunk of 8 positions with
 # 1, 3, 7 and 8 of them; 16, 33, 50 and 51 channels per group (1 and 2 in the last wavefront, idle wavefronts); 4, 8 and 16 states; delta rows
 # shared; rows off the dword grid.  Bound in single precision: sums of up to 1030 terms and 51 channels, each term good to a few 2^-23 -- 1e-4 of the largest gradient.
 CHANNEL_CASES = [
     (64, 64, 1, 16, 72, None, True), (64, 64, 1, 16, 73, None, True), (64, 66, 2, 8, 33, None, True), (64, 64, 1, 8, 7, None, False), (128, 64, 1, 4, 57, None, True),
     (64, 64, 1, 16, 128, None, True), (1, 96, 2, 16, 512, None, True), (1, 50, 1, 8, 515, 10, True), (1, 16, 1, 4, 1030, None, True), (2, 51, 1, 16, 779, 17, True),
     (1, 33, 1, 16, 600, None, False), (1, 80, 1, 16, 1000, None, True),
+    # lengths that no equal segments fill: what is left for the last one would be shorter than its states
+    (1, 17, 1, 16, 529, None, True), (1, 32, 2, 16, 729, None, False), (1, 20, 1, 16, 961, 10, True), (1, 16, 1, 8, 585, None, True),
 ]
 
 

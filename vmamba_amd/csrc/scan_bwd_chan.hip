@@ -31,9 +31,14 @@ constexpr int kBcChunks = 9;                      // chunks per segment at most
 constexpr int kBcSeg = kBcChunks * kBcSub;
 
 struct BwdChanGeom {
-    int32_t n_cb, n_segs, seg_len;                // blocks of 64 channels per group; segments per row, all but the last of seg_len positions
+    int32_t n_cb, n_segs;                         // blocks of 64 channels per group; segments per row
+    int32_t seg_chunks, n_longer;                 // chunks of a segment; the first n_longer segments have one more
     FastDiv div_cb, div_groups, div_segs;
 };
+
+__host__ __device__ __forceinline__ int bwd_chan_begin(int seg, int seg_chunks, int n_longer) {
+    return (seg * seg_chunks + (seg < n_longer ? seg : n_longer)) * kBcSub;
+}
 
 // Two elements from an even `pos` of a row that a plain (not rounded) base and element `row` give.
 template <typename T, bool kDwords>
@@ -105,7 +110,8 @@ __global__ __launch_bounds__(kBlock, !kGrad ? (kSpw == 4 ? 4 : 5) : kSpw == 4 &&
     divmod(wg, geo.div_segs, wg, seg);
     divmod(wg, geo.div_cb, bg, cb);
     divmod(bg, geo.div_groups, b, grp);
-    const int L = p.L, begin = (int)seg * geo.seg_len, stop = (int)seg + 1 == geo.n_segs ? L : begin + geo.seg_len;
+    const int L = p.L, begin = bwd_chan_begin((int)seg, geo.seg_chunks, geo.n_longer);
+    const int stop = min(L, bwd_chan_begin((int)seg + 1, geo.seg_chunks, geo.n_longer));
     const int n_chunks = (stop - begin + kBcSub - 1) / kBcSub;
     const int c_first = (int)cb * 64 + wave * kBcChan, n_chan = min(kBcChan, p.dim_per_group - c_first);
     const bool softplus = p.softplus != 0;
@@ -421,7 +427,7 @@ __global__ __launch_bounds__(kBlock, !kGrad ? (kSpw == 4 ? 4 : 5) : kSpw == 4 &&
 
 // What enters every segment of a row from either side, in the place of what the segments left: a thread per (row, state) and side.
 template <typename in_t>
-__global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanBwdArgs p, int seg_len, int n_segs, uint32_t n_items, FastDiv div_n, FastDiv div_dim) {
+__global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanBwdArgs p, int seg_chunks, int n_longer, int n_segs, uint32_t n_items, FastDiv div_n, FastDiv div_dim) {
     const uint32_t item = blockIdx.x * kBlock + threadIdx.x;
     if (item >= n_items) return;
     uint32_t row, n, b, d;
@@ -431,12 +437,12 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanB
     uint8_t *h_state = reinterpret_cast<uint8_t *>(reinterpret_cast<in_t *>(p.du) + (int64_t)row * p.L) + sizeof(float) * n;
     uint8_t *g_state = reinterpret_cast<uint8_t *>(reinterpret_cast<in_t *>(p.ddelta) + (int64_t)row * p.L) + sizeof(float) * n;
     const uint8_t *sums = reinterpret_cast<const uint8_t *>(reinterpret_cast<const in_t *>(p.du) + (int64_t)row * p.L) + sizeof(float) * p.N;
-    const int64_t pitch = (int64_t)seg_len * sizeof(in_t);
+    auto place = [&](int s) { return (int64_t)bwd_chan_begin(s, seg_chunks, n_longer) * (int)sizeof(in_t); };
     if (n == 0 && blockIdx.y == 0 && p.dD) {
         double dD = 0.0;
         for (int s = 0; s + 1 < n_segs; ++s) {
             float part;
-            __builtin_memcpy(&part, g_state + s * pitch + sizeof(float) * p.N, sizeof(float));
+            __builtin_memcpy(&part, g_state + place(s) + sizeof(float) * p.N, sizeof(float));
             dD += part;
         }
         unsafeAtomicAdd(p.dD + d, (float)dD);
@@ -446,7 +452,7 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanB
     auto through = [&](int s, float carry, float sum, float left) {
         if (fabsf(carry) == __builtin_inff()) {
             float most;
-            __builtin_memcpy(&most, sums + min(s, n_segs - 2) * pitch + sizeof(float), sizeof(float));
+            __builtin_memcpy(&most, sums + place(min(s, n_segs - 2)) + sizeof(float), sizeof(float));
             return __builtin_amdgcn_exp2f(A2 * most) > 0.0f ? carry + left : __builtin_nanf("");
         }
         const float half = __builtin_amdgcn_exp2f(0.5f * A2 * sum);
@@ -459,7 +465,7 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanB
             float left[kFly], sum[kFly];
 #pragma unroll
             for (int i = 0; i < kFly; ++i) {                    // (past the last but one segment: that one again, not used)
-                const int64_t at = min(first + i, n_segs - 2) * pitch;
+                const int64_t at = place(min(first + i, n_segs - 2));
                 __builtin_memcpy(&left[i], h_state + at, sizeof(float));
                 __builtin_memcpy(&sum[i], sums + at, sizeof(float));
             }
@@ -467,7 +473,7 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanB
             for (int i = 0; i < kFly; ++i) {
                 const int s = first + i;
                 if (s >= n_segs) break;
-                if (s > 0) __builtin_memcpy(h_state + s * pitch, &carry, sizeof(float));
+                if (s > 0) __builtin_memcpy(h_state + place(s), &carry, sizeof(float));
                 carry = through(s, carry, sum[i], left[i]);
             }
         }
@@ -478,31 +484,28 @@ __global__ __launch_bounds__(kBlock) void scan_bwd_chan_carry_kernel(const ScanB
 #pragma unroll
         for (int i = 0; i < kFly; ++i) {                    // (the last segment's sum is not used: nothing enters it; before the first: that one again)
             const int s = max(first - i, 0);
-            __builtin_memcpy(&left[i], g_state + s * pitch, sizeof(float));
-            __builtin_memcpy(&sum[i], sums + min(s, n_segs - 2) * pitch, sizeof(float));
+            __builtin_memcpy(&left[i], g_state + place(s), sizeof(float));
+            __builtin_memcpy(&sum[i], sums + place(min(s, n_segs - 2)), sizeof(float));
         }
 #pragma unroll
         for (int i = 0; i < kFly; ++i) {
             const int s = first - i;
             if (s < 0) break;
-            __builtin_memcpy(g_state + s * pitch, &carry, sizeof(float));
+            __builtin_memcpy(g_state + place(s), &carry, sizeof(float));
             carry = through(s, carry, sum[i], left[i]);
         }
     }
 }
 
-// Segments of a row: the fewest whose last one has room for its states where its gradients will be.  0: none found.
-static int bwd_chan_segments(int L, int N, int size, int32_t &seg_len) {
-    const int n_least = (L + kBcSeg - 1) / kBcSeg, room = (N * 4 + size - 1) / size;
-    for (int n = n_least; n <= n_least + 8; ++n) {
-        const int len = ((L + n - 1) / n + kBcSub - 1) / kBcSub * kBcSub;
-        seg_len = len;
-        if (n == 1) return 1;
-        const int last = L - (n - 1) * len;
-        if (last >= room && len >= room + 8 / size) return n;
-    }
-    return 0;
+// A row's segments: as few as hold it, its chunks of 8 dealt out evenly, the longer ones first.  From 10 chunks on (the first row that is cut) that is 5
+// chunks at least: 33 positions in the last segment, room for its 16 states in 16 bits, 40 in the others, room for theirs and two sums.
+static void bwd_chan_segments(int L, BwdChanGeom &geo) {
+    const int n_chunks = (L + kBcSub - 1) / kBcSub;
+    geo.n_segs = (n_chunks + kBcChunks - 1) / kBcChunks;
+    geo.seg_chunks = n_chunks / geo.n_segs;
+    geo.n_longer = n_chunks % geo.n_segs;
 }
+static_assert(kBcSub * 4 + 1 >= 2 * 16 && kBcSub * 5 >= 2 * (16 + 2), "a segment's place");
 
 // Where a channel per lane is ahead of positions in lanes (scan_bwd_states_kernel).  That one works in passes of 256 positions, and a few
 // images of one or two passes are done before two more kernels have been launched here; many of them or longer rows fill the chip either way,
@@ -519,13 +522,13 @@ static bool bwd_chan_pays(const ScanBwdArgs &a) {
 }
 
 // False: no grid for it.
-static bool bwd_chan_geom(const ScanBwdArgs &a, int in_size, BwdChanGeom &geo, uint32_t &n_wg) {
+static bool bwd_chan_geom(const ScanBwdArgs &a, BwdChanGeom &geo, uint32_t &n_wg) {
     geo = {};
-    geo.n_segs = bwd_chan_segments(a.L, a.N, in_size, geo.seg_len);
+    bwd_chan_segments(a.L, geo);
     const int64_t groups = a.dim / a.dim_per_group;
     geo.n_cb = (a.dim_per_group + 63) / 64;
     const int64_t n = (int64_t)a.batch * groups * geo.n_cb * geo.n_segs;
-    if (geo.n_segs == 0 || n > 0x7fffffff) return false;
+    if (n > 0x7fffffff) return false;
     geo.div_cb = make_fastdiv((uint32_t)geo.n_cb);
     geo.div_groups = make_fastdiv((uint32_t)groups);
     geo.div_segs = make_fastdiv((uint32_t)geo.n_segs);
@@ -536,7 +539,7 @@ static bool bwd_chan_geom(const ScanBwdArgs &a, int in_size, BwdChanGeom &geo, u
 bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size) {
     BwdChanGeom geo;
     uint32_t n_wg;
-    if ((a.N != 4 && a.N != 8 && a.N != 16) || a.dim_per_group < kBcChan || !bwd_chan_pays(a) || !bwd_chan_geom(a, in_size, geo, n_wg)) return false;
+    if ((a.N != 4 && a.N != 8 && a.N != 16) || a.dim_per_group < kBcChan || !bwd_chan_pays(a) || !bwd_chan_geom(a, geo, n_wg)) return false;
     // the gradients' memory holds the segments' states between the passes
     auto apart = [&](const void *x, int64_t elems, int size) {
         const uintptr_t first = reinterpret_cast<uintptr_t>(x), last = first + (uintptr_t)(elems * size);
@@ -565,11 +568,11 @@ template <typename in_t, typename dy_t, int kSpw, bool kDwords>
 static int launch_bwd_chan(const ScanBwdArgs &a, hipStream_t stream) {
     BwdChanGeom geo;
     uint32_t n;
-    if (!bwd_chan_geom(a, (int)sizeof(in_t), geo, n)) return SS2D_ENOTSUP;
+    if (!bwd_chan_geom(a, geo, n)) return SS2D_ENOTSUP;
     if (geo.n_segs > 1) {
         const uint32_t n_items = (uint32_t)((int64_t)a.batch * a.dim * a.N);
         hipLaunchKernelGGL((scan_bwd_chan_kernel<in_t, dy_t, kSpw, kDwords, false>), dim3(n), dim3(kBlock), 0, stream, a, geo);
-        hipLaunchKernelGGL((scan_bwd_chan_carry_kernel<in_t>), dim3((n_items + kBlock - 1) / kBlock, 2), dim3(kBlock), 0, stream, a, geo.seg_len, geo.n_segs, n_items,
+        hipLaunchKernelGGL((scan_bwd_chan_carry_kernel<in_t>), dim3((n_items + kBlock - 1) / kBlock, 2), dim3(kBlock), 0, stream, a, geo.seg_chunks, geo.n_longer, geo.n_segs, n_items,
                            make_fastdiv((uint32_t)a.N), make_fastdiv((uint32_t)a.dim));
     }
     hipLaunchKernelGGL((scan_bwd_chan_kernel<in_t, dy_t, kSpw, kDwords, true>), dim3(n), dim3(kBlock), 0, stream, a, geo);
