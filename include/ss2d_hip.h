@@ -131,8 +131,8 @@ int ss2d_selective_scan_fwd(const ss2d_scan_params *params, void *stream);
 #define SS2D_SCAN_KERNEL_NONE 0  /* empty problem: nothing to launch                                           */
 #define SS2D_SCAN_KERNEL_ROW 1   /* one wavefront per (batch, channel) row                                       */
 #define SS2D_SCAN_KERNEL_ROW4 2  /* few long rows: the four wavefronts of a workgroup share a row                */
-#define SS2D_SCAN_KERNEL_FLAT 3  /* short rows and rows off the 16-byte grid: where there are many, several to
-                                    a wavefront as one stream; few, and long ones, a wavefront each             */
+#define SS2D_SCAN_KERNEL_FLAT 3  /* many short rows, or rows off the 16-byte grid: several to a wavefront as one
+                                    stream                                                                      */
 #define SS2D_SCAN_KERNEL_SMALL 4 /* rows of 49 / 196 positions, one state: a segment of a row per lane           */
 #define SS2D_SCAN_KERNEL_CHAN 5  /* several states per channel: one channel per lane, positions walked serially  */
 int ss2d_selective_scan_kernel(const ss2d_scan_params *params);

@@ -114,8 +114,9 @@ def test_scan_kernel_choice_does_not_depend_on_the_chunk_state_output():
         (128, 384, 3136, 1): _lib.SCAN_KERNEL_ROW, (128, 768, 784, 1): _lib.SCAN_KERNEL_ROW,
         (128, 1536, 196, 1): _lib.SCAN_KERNEL_SMALL, (128, 3072, 49, 1): _lib.SCAN_KERNEL_SMALL,
         (64, 768, 3136, 16): _lib.SCAN_KERNEL_CHAN, (4, 384, 65536, 1): _lib.SCAN_KERNEL_ROW4,
-        (4, 768, 16384, 1): _lib.SCAN_KERNEL_ROW, (48, 384, 3306, 1): _lib.SCAN_KERNEL_FLAT,
-        (16, 384, 100, 1): _lib.SCAN_KERNEL_FLAT,
+        (4, 768, 16384, 1): _lib.SCAN_KERNEL_ROW, (48, 384, 3306, 1): _lib.SCAN_KERNEL_ROW,
+        (16, 384, 100, 1): _lib.SCAN_KERNEL_ROW, (128, 384, 100, 1): _lib.SCAN_KERNEL_FLAT, (128, 768, 484, 1): _lib.SCAN_KERNEL_FLAT,
+        (128, 384, 3306, 1): _lib.SCAN_KERNEL_ROW, (1, 768, 3307, 1): _lib.SCAN_KERNEL_ROW4,
     }
     for (batch, dim, L, N), kernel in shapes.items():
         for with_x in (False, True):

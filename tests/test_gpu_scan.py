@@ -209,15 +209,17 @@ def test_scan_blocks_of_channels(batch, dim, G, N, L, dtype):
 
 # One state and three: rows of no whole 16-byte pieces read as dwords, a wavefront per row and four; both sides of the lines between a wavefront per
 # row and several rows to one (8192 rows; 16 384 and single elements; rows of two and four).
-ROW_READS = [(2, 8, 4, 1, 1), (2, 8, 4, 1, 57), (1, 12, 2, 1, 513), (1, 6, 2, 3, 335), (1, 8, 4, 1, 2051), (2, 6, 1, 3, 2309), (128, 64, 4, 1, 57), (129, 64, 4, 1, 57),
-             (129, 64, 4, 1, 65), (257, 64, 4, 1, 65), (257, 64, 4, 1, 363), (257, 64, 4, 1, 66), (129, 64, 4, 1, 390), (129, 64, 4, 1, 382)]
+ROW_READS = [(2, 8, 4, 1, 1, "row"), (2, 8, 4, 1, 57, "row"), (1, 12, 2, 1, 513, "row"), (1, 6, 2, 3, 335, "row"), (1, 8, 4, 1, 2051, "row4"), (2, 6, 1, 3, 2309, "row4"),
+             (128, 64, 4, 1, 57, "row"), (129, 64, 4, 1, 57, "flat"), (129, 64, 4, 1, 65, "row"), (257, 64, 4, 1, 65, "flat"), (257, 64, 4, 1, 363, "row"), (257, 64, 4, 1, 66, "flat"),
+             (129, 64, 4, 1, 390, "row"), (129, 64, 4, 1, 382, "flat")]
 
 
-@pytest.mark.parametrize("batch,dim,G,N,L", ROW_READS)
+@pytest.mark.parametrize("batch,dim,G,N,L,kernel", ROW_READS)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-def test_scan_odd_rows(batch, dim, G, N, L, dtype):
+def test_scan_odd_rows(batch, dim, G, N, L, kernel, dtype):
     _announce("scan-row-reads", batch, dim, G, N, L, dtype)
     args = make_inputs(40, batch, dim, G, N, L, dtype, ss2d_like=True)
+    assert kernel_of(*args[:5], want_x=False) == kernel_of(*args[:5], want_x=True) == kernel
     want, xw = orc.selective_scan(*args, True, out_float=True, return_x=True)
     got, x = run_gpu(*args, True, True, want_x=True)
     assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
@@ -229,8 +231,8 @@ def test_scan_odd_rows(batch, dim, G, N, L, dtype):
 
 # Rows of no whole 16-byte pieces in the same kernel: a row shorter than a group of four, one that ends 1, 2 and 3 positions into a group, rows on odd
 # elements, cut rows, 4 to 32 states; what the rule leaves to the other kernels beside it.
-ODD_ROWS = [(2, 64, 2, 16, 3, "chan"), (1, 33, 1, 16, 9, "chan"), (2, 47, 1, 8, 49, "chan"), (1, 40, 1, 32, 62, "chan"), (26, 99, 1, 16, 135, "chan"), (25, 99, 1, 16, 135, "flat"), (2, 96, 2, 16, 225, "flat"),
-            (1, 48, 1, 16, 1225, "chan"), (1, 48, 1, 16, 1003, "flat"), (1, 40, 1, 32, 3306, "chan"), (1, 48, 1, 16, 3306, "row4"), (64, 48, 1, 8, 77, "chan"), (37, 33, 1, 4, 77, "row"),
+ODD_ROWS = [(2, 64, 2, 16, 3, "chan"), (1, 33, 1, 16, 9, "chan"), (2, 47, 1, 8, 49, "chan"), (1, 40, 1, 32, 62, "chan"), (26, 99, 1, 16, 135, "chan"), (25, 99, 1, 16, 135, "row"), (2, 96, 2, 16, 225, "row"),
+            (1, 48, 1, 16, 1225, "chan"), (1, 48, 1, 16, 1003, "row"), (1, 40, 1, 32, 3306, "chan"), (1, 48, 1, 16, 3306, "row4"), (64, 48, 1, 8, 77, "chan"), (37, 33, 1, 4, 77, "row"),
             (39, 33, 1, 4, 77, "chan"), (3, 35, 1, 4, 331, "row"), (1, 64, 1, 4, 3307, "row4")]
 
 
@@ -553,11 +555,11 @@ def test_scan_errors_from_host_api():
 @pytest.mark.parametrize("batch,dim,G,L,dtype", [(16, 384, 4, 2051, torch.bfloat16), (24, 256, 4, 2307, torch.float32),
                                                  (13, 512, 2, 2049, torch.float16)])
 def test_many_long_rows_off_the_vector_grid(batch, dim, G, L, dtype):
-    """6144 rows and more of odd length (no row but the first starts on a 16-byte boundary): the library walks them eight
-    to a wavefront as one aligned stream.  Every row against the oracle, without and with the chunk states."""
+    """6144 rows and more of odd length (no row but the first starts on a 16-byte boundary), a wavefront each.  Every row against the oracle, without
+    and with the chunk states."""
     _announce("scan-long-unaligned", batch, dim, G, L, dtype)
     args = make_inputs(batch * 1000 + L, batch, dim, G, 1, L, dtype, ss2d_like=True)
-    assert kernel_of(*args[:5], want_x=False) == kernel_of(*args[:5], want_x=True) == "flat"
+    assert kernel_of(*args[:5], want_x=False) == kernel_of(*args[:5], want_x=True) == "row"
     want, xw = orc.selective_scan(*args, True, out_float=True, return_x=True)
     for want_x in (False, True):
         got, x = run_gpu(*args, True, True, want_x=want_x)
@@ -574,8 +576,7 @@ def test_full_size_properties(cfg):
     _announce("scan-full", cfg)
     batch, Dn, L, N = dict(stage1=(128, 96, 3136, 1), stage2=(128, 192, 784, 1), stage3=(128, 384, 196, 1),
                            stage4=(128, 768, 49, 1), n16=(64, 192, 3136, 16), hires=(4, 96, 65536, 1),
-                           # many long rows that do not start on 16-byte boundaries (the reference's 57 x 58 check size,
-                           # an odd map): walked eight rows to a wavefront as one aligned stream
+                           # many long rows that do not start on 16-byte boundaries (the reference's 57 x 58 check size, an odd map)
                            rows57x58=(48, 96, 3306, 1), rows75x75=(8, 192, 5625, 1))[cfg]
     K = 4
     g = torch.Generator(device=DEV).manual_seed(28)

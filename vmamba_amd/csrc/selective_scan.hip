@@ -219,11 +219,11 @@ __global__ __launch_bounds__(kBlock) void scan_row_kernel(const ScanArgs p) {
 // descriptors (their rows are shared by dim/n_groups channels and stay in L1/L2).  A lane
 // touches at most two rows (L >= 8); with kGran == 8 exactly one.
 //
-// kX: the chunk-end states are written too.  h at a chunk's (or row's) last position is what the scan yields there.  The
+// kX: the chunk-end states are written too.  A row here is shorter than a chunk: they are the states at its last position, which is what the scan yields there.  The
 // product of a since the row's start is a second recurrence on the SAME multipliers: with a forced to 0 at a row's
 // first position, g_t = a_t g_(t-1) + c_t with c = the true a at that first position and 0 elsewhere gives
-// g_t = a_start ... a_t, so it rides through the lane-local and the wavefront scan beside h (wave_scan_pairs2).  Chunk
-// and row ends fall on group boundaries (rows start at multiples of kGran in the stream, chunks at multiples of 8).
+// g_t = a_start ... a_t, so it rides through the lane-local and the wavefront scan beside h (wave_scan_pairs2).  Row ends
+// fall on group boundaries (rows start at multiples of kGran in the stream).
 template <typename in_t, typename out_t, int kN, bool kSoftplus, int kGran, bool kX>
 __global__ __launch_bounds__(kBlock) void scan_flat_kernel(const ScanArgs p, int rows_per_wave, FastDiv divL,
                                                            FastDiv divDim, FastDiv divDpg) {
@@ -305,17 +305,16 @@ __global__ __launch_bounds__(kBlock) void scan_flat_kernel(const ScanArgs p, int
         float du[kItems], y[kItems], bias_items[kItems];
         bool in_a[kGroups], first[kGroups];
         uint32_t boff[kGroups], coff[kGroups];
-        float *x_end[kX ? kGroups : 1];       // kX: where the group's last item puts its state (null: not a chunk end)
+        float *x_end[kX ? kGroups : 1];       // kX: where the group's last item puts its state (null: not a row's end)
 #pragma unroll
         for (int gi = 0; gi < kGroups; ++gi) {
             in_a[gi] = kGran == kItems ? true : gi * kGran < k;
             const uint32_t li = in_a[gi] ? l0 + gi * kGran : (uint32_t)(gi * kGran - k);
             first[gi] = li == 0;
             if constexpr (kX) {
-                const uint32_t l_end = li + kGran;
-                const bool ends = e0 + gi * kGran < n_el && (l_end == (uint32_t)L || l_end % SS2D_SCAN_CHUNK == 0);
+                const bool ends = e0 + gi * kGran < n_el && li + kGran == (uint32_t)L;
                 const int64_t row = r0 + rl + (in_a[gi] ? 0 : 1);
-                x_end[gi] = ends ? p.x + (row * p.n_chunks + (l_end - 1) / SS2D_SCAN_CHUNK) * 2 * kN : nullptr;
+                x_end[gi] = ends ? p.x + row * 2 * kN : nullptr;
             }
             boff[gi] = (in_a[gi] ? Boff_a : Boff_b) + li;
             coff[gi] = (in_a[gi] ? Coff_a : Coff_b) + li;
@@ -616,11 +615,11 @@ static bool span_fits_u32(const ScanArgs &a, int64_t elem_bytes) {
 }
 
 // The flat kernel needs dense u / delta / out (rows adjacent in memory, base 16-byte aligned), one delta row
-// per channel, rows of at least one lane vector, and dstate 1 or 16.
+// per channel, rows of at least one lane vector and shorter than a chunk (longer ones gather B and C element by element for nothing: 6144 rows of 2051
+// positions, one state in bf16, 62.9 us so and 30.4 a wavefront each, 24 576 of 5625 389 and 262), and dstate 1 or 16.
 static bool flat_eligible(const ScanArgs &a, const ss2d_scan_params *q) {
     const int64_t L = a.L, KD = a.dim;
-    const bool length_ok = L < 4 * kPass || (L <= (1 << 24) && a.N == 1 && a.rows >= 6144);
-    return L >= kItems && length_ok && (a.N == 1 || a.N == 16) && q->delta_dim == q->dim &&
+    return L >= kItems && L < 4 * kPass && (a.N == 1 || a.N == 16) && q->delta_dim == q->dim &&
            a.u_ds == L && a.dl_ds == L && a.o_ds == L && a.u_bs == KD * L && a.dl_bs == KD * L && a.o_bs == KD * L &&
            aligned16(q->u) && aligned16(q->delta) && aligned16(q->out) &&
            span_fits_u32(a, q->in_dtype == SS2D_F32 ? 4 : 2);
@@ -628,21 +627,13 @@ static bool flat_eligible(const ScanArgs &a, const ss2d_scan_params *q) {
 
 static int flat_granularity(const ScanArgs &a, int64_t elem_bytes);
 
-// Rows that the row kernel reads off the 16-byte grid or with more than 30 % of its lanes idle.
-static bool flat_class(const ScanArgs &a, bool vec) {
-    return !vec || 10 * (int64_t)a.L < 7 * (((int64_t)a.L + kPass - 1) / kPass * kPass);
-}
-
-// Several of those to a wavefront, or one.  A wavefront of the flat kernel walks eight rows or more behind one another, so few rows leave the
+// Several rows to a wavefront, or one.  A wavefront of the flat kernel walks eight rows or more behind one another, so few rows leave the
 // chip idle: a wavefront per row is ahead at any length (one state in bf16, us, flat / row; 192 rows: 56 positions 10.6 / 3.7, 225 20.4 / 4.7, 1353 36.4 / 6.0;
 // 3072: 56 11.6 / 4.0, 225 21.0 / 7.1, 576 11.5 / 5.7, 1353 37.5 / 11.3).  Many rows: a pass of the flat kernel costs about 1.4x a pass of the row kernel with
 // groups of two elements or more, and more with single ones, so it is ahead where the row kernel would leave more than 30 % of its lanes idle
 // (12 288 rows: 601 of 1024 positions 29.7 / 23.2 with single elements; 24 576: 418 of 512 in pairs 31.0 / 35.9, 601 40.4 / 42.1, 1003 61.2 / 52.2,
 // 1353 81.0 / 63.9) and, reading pairs or fours, on rows that are no whole 16-byte pieces (24 576 of 484: 30.7 / 37.3).
-// Long ones are a wavefront's each: eight to a wavefront as one stream gather B and C element by element (before and now: 6144 rows of 2051 positions 62.9 / 30.4,
-// 24 576 118 / 107, 24 576 of 5625 389 / 262).
 static bool flat_pays(const ScanArgs &a, bool vec, int in_size) {
-    if (a.L >= 4 * kPass) return false;
     const bool half_full = 10 * (int64_t)a.L < 7 * (((int64_t)a.L + kPass - 1) / kPass * kPass);
     if (a.rows <= 8192 || (vec && in_size == 2 && a.L <= 336 && a.rows <= 12288)) return false;
     if (vec) return half_full;
@@ -742,7 +733,7 @@ static int launch_scan(const ScanArgs &a, bool split_rows, hipStream_t stream) {
 
 template <typename in_t, typename out_t>
 static int dispatch_vec(const ScanArgs &a, bool vec, int kernel, hipStream_t stream) {
-    if (kernel == SS2D_SCAN_KERNEL_FLAT && flat_pays(a, vec, (int)sizeof(in_t))) return launch_flat<in_t, out_t>(a, stream);
+    if (kernel == SS2D_SCAN_KERNEL_FLAT) return launch_flat<in_t, out_t>(a, stream);
     const bool split_rows = kernel == SS2D_SCAN_KERNEL_ROW4;
     return vec ? launch_scan<in_t, out_t, true>(a, split_rows, stream) : launch_scan<in_t, out_t, false>(a, split_rows, stream);
 }
@@ -802,7 +793,7 @@ static int plan_scan(const ss2d_scan_params *q, ScanArgs &a, bool &vec) {
     if (scan_small_eligible(a, q->in_dtype, q->u, q->delta, q->out)) return SS2D_SCAN_KERNEL_SMALL;
     // several states per channel and enough channels per group to fill wavefronts: one channel per lane
     if (scan_chan_eligible(a, vec, (int)in_bytes)) return SS2D_SCAN_KERNEL_CHAN;
-    if (flat_eligible(a, q) && flat_class(a, vec)) return SS2D_SCAN_KERNEL_FLAT;
+    if (flat_eligible(a, q) && flat_pays(a, vec, (int)in_bytes)) return SS2D_SCAN_KERNEL_FLAT;
     // few long rows: every row split over the four wavefronts of a workgroup (3072 rows and more: a wavefront per row is faster)
     if (a.L > SS2D_SCAN_CHUNK && a.rows < 2048) return SS2D_SCAN_KERNEL_ROW4;
     return SS2D_SCAN_KERNEL_ROW;
