@@ -229,6 +229,30 @@ def test_scan_odd_rows(batch, dim, G, N, L, kernel, dtype):
         assert torch.allclose(small.float(), want.to(dtype).float(), **TOL16)
 
 
+# Several rows to a wavefront: groups of one, two, four and eight elements within a row, the last wavefront with fewer rows than the others, one state and
+# 16 (of groups of fewer than 32 channels), rows of the shortest and of nearly a chunk; what is on the other side of the rule's lines is a row's own wavefront's.
+MANY_ROWS = [(131, 64, 4, 1, 9, "flat"), (193, 64, 4, 1, 16, "flat"), (193, 64, 4, 1, 72, "flat"), (131, 64, 4, 1, 102, "flat"), (131, 64, 4, 1, 92, "flat"), (17, 1024, 8, 1, 1358, "flat"),
+             (9, 1024, 8, 1, 2044, "row"), (131, 128, 8, 16, 36, "flat"), (131, 128, 8, 16, 24, "flat"), (137, 120, 4, 16, 30, "flat"), (131, 128, 8, 16, 33, "row"), (128, 128, 8, 16, 36, "row"),
+             (131, 128, 8, 16, 212, "row"), (257, 160, 8, 16, 210, "flat")]
+
+
+@pytest.mark.parametrize("batch,dim,G,N,L,kernel", MANY_ROWS)
+@pytest.mark.parametrize("dtype,softplus", [(torch.float32, True), (torch.bfloat16, False), (torch.float16, True)])
+def test_scan_many_short_rows(batch, dim, G, N, L, kernel, dtype, softplus):
+    _announce("scan-many-rows", batch, dim, G, N, L, dtype, softplus)
+    args = make_inputs(43, batch, dim, G, N, L, dtype, ss2d_like=True)
+    if not softplus:
+        args = (args[0], args[1].abs() * 0.1, *args[2:6], args[6].abs() * 0.1)
+    if dtype == torch.float32 and L % 4 == 0 and N == 1 and L > 1000:
+        kernel = "row"                                          # whole 16-byte pieces, and the lanes of the last pass well filled
+    assert kernel_of(*args[:5], want_x=False) == kernel_of(*args[:5], want_x=True) == kernel
+    want, xw = orc.selective_scan(*args, softplus, out_float=True, return_x=True)
+    got, x = run_gpu(*args, softplus, True, want_x=True)
+    assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
+    check_states(x, xw, TOL32)
+    assert torch.equal(run_gpu(*args, softplus, True, want_x=False)[0], got)
+
+
 # Rows of no whole 16-byte pieces in the same kernel: a row shorter than a group of four, one that ends 1, 2 and 3 positions into a group, rows on odd
 # elements, cut rows, 4 to 32 states; what the rule leaves to the other kernels beside it.
 ODD_ROWS = [(2, 64, 2, 16, 3, "chan"), (1, 33, 1, 16, 9, "chan"), (2, 47, 1, 8, 49, "chan"), (1, 40, 1, 32, 62, "chan"), (26, 99, 1, 16, 135, "chan"), (25, 99, 1, 16, 135, "row"), (2, 96, 2, 16, 225, "row"),

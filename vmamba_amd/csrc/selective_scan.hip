@@ -633,11 +633,19 @@ static int flat_granularity(const ScanArgs &a, int64_t elem_bytes);
 // groups of two elements or more, and more with single ones, so it is ahead where the row kernel would leave more than 30 % of its lanes idle
 // (12 288 rows: 601 of 1024 positions 29.7 / 23.2 with single elements; 24 576: 418 of 512 in pairs 31.0 / 35.9, 601 40.4 / 42.1, 1003 61.2 / 52.2,
 // 1353 81.0 / 63.9) and, reading pairs or fours, on rows that are no whole 16-byte pieces (24 576 of 484: 30.7 / 37.3).
+// 16 states (groups of fewer than 32 channels; the others are the channel-per-lane kernel's): gathered B and C are most of the work, single elements never
+// pay (24 576 rows of 225 185 / 86), fours and eights do on many short rows (15 360: 56 56 / 41, 100 59 / 54; 20 480: 72 58 / 56, 196 59 / 72, 256 69 / 58; 24 576: 56 57 / 64,
+// 100 59 / 84, 200 64 / 66, 324 97 / 89; 49 152: 100 61 / 161, 208 102 / 127, 256 104 / 131, 324 139 / 174, 400 169 / 139, 576 203 / 248, 784 302 / 261; in fp32 196 92 / 129,
+// 320 138 / 135, 576 265 / 259).
 static bool flat_pays(const ScanArgs &a, bool vec, int in_size) {
+    const int gran = flat_granularity(a, in_size);
+    if (a.N != 1) {
+        if (gran == 1 || a.rows <= 16384) return false;
+        return a.L <= 208 || (a.rows > 40960 && (a.L <= 336 || (in_size == 2 && a.L > kPass && a.L <= 716)));
+    }
     const bool half_full = 10 * (int64_t)a.L < 7 * (((int64_t)a.L + kPass - 1) / kPass * kPass);
     if (a.rows <= 8192 || (vec && in_size == 2 && a.L <= 336 && a.rows <= 12288)) return false;
     if (vec) return half_full;
-    const int gran = flat_granularity(a, in_size);
     if (a.rows <= 16384) return gran == 1 ? a.L < 64 : 4 * (int64_t)a.L < 3 * (((int64_t)a.L + kPass - 1) / kPass * kPass);
     return gran > 1 || half_full;
 }
@@ -673,7 +681,7 @@ static int launch_flat(const ScanArgs &a_in, hipStream_t stream) {
         case 8: SS2D_LAUNCH_FLAT(N, SP, 8, X); break;                \
         case 4: SS2D_LAUNCH_FLAT(N, SP, 4, X); break;                \
         case 2: SS2D_LAUNCH_FLAT(N, SP, 2, X); break;                \
-        default: SS2D_LAUNCH_FLAT(N, SP, 1, X); break;               \
+        default: if constexpr (N == 1) SS2D_LAUNCH_FLAT(N, SP, 1, X); /* (16 states: flat_pays) */ \
     }
 #define SS2D_LAUNCH_FLAT_X(N, SP) \
     if (a.x) { SS2D_LAUNCH_FLAT_G(N, SP, true) } else { SS2D_LAUNCH_FLAT_G(N, SP, false) }
