@@ -69,18 +69,14 @@ struct ChanGeom {
 // A row as a whole, or cut into segments: what a segment leaves from state 0, then its outputs from the state that enters it.
 enum ChanPhase { kWhole, kLocal, kRest };
 
-// kX: the chunk-end states are written as well -- x[row][chunk][2n] = product of a_n since the row's start,
-// x[..][2n + 1] = h_n, after every 2048 positions and at the row's end.  h is what the lane holds; the product is
-// exp2(A_n log2e * sum dl), and the sum is per CHANNEL, not per state: each of a channel's four lanes adds up a quarter of
-// every round's positions (one LDS read, four adds per 16 positions) and the quarters meet when a chunk ends.
-//
-// kMaps: CrossScan folded in.  u is not the (batch, 4 D, L) tensor of the four scan-ordered copies but the map itself,
-// x (batch, D, L), plus its transpose xt (batch, D, L: every H x W map stored as W x H): direction k = the channel's
-// group reads x (k = 0, 2) or xt (k = 1, 3), forwards (k < 2) or backwards -- position t of the scan is element t or
-// L - 1 - t of that row (cross_scan_fwd, classification/models/csm_triton.py:22-29).  A lane's four positions are then
-// the four elements that END at L - 1 - t, taken in reverse; where fewer are left, the row's first four.
-//
-// kDwords: the rows of 16-bit inputs start on dwords (RawGroup).
+// Wavefronts per SIMD to leave registers for.  Four with four states, but for the forms that would then keep 12 to 60 bytes a lane in memory (in single precision with
+// CrossScan folded in or a state that enters; off the dword grid with chunk-end states as well): us with four / three, fp32, 64 x 96 maps of 56 x 56 folded in 300 / 246,
+// 16 x 96 rows of 3136 cut 89 / 84, with chunk-end states 116 / 84.
+template <typename in_t, int kSpw, bool kX, bool kMaps, int kPhase, bool kDwords> constexpr int chan_waves() {
+    if (kSpw != 1) return kSpw == 8 ? 2 : 3;
+    return (kMaps || kPhase == kRest) && (sizeof(in_t) == 4 || (!kDwords && kX)) ? 3 : 4;
+}
+
 // y[i] summed over the four sets of lanes (the banks of four lanes in a row of 16) for every position i of 16: afterwards
 // y[0 .. 3] are positions 4 set .. 4 set + 3.  Two DPP additions, each with its own banks, put two positions into one register:
 // half the additions of a sum that every lane gets, and no selects.
@@ -106,8 +102,20 @@ __device__ __forceinline__ void sum_over_sets(float (&y)[16]) {
 #undef SS2D_ODD
 }
 
+// kX: the chunk-end states are written as well -- x[row][chunk][2n] = product of a_n since the row's start,
+// x[..][2n + 1] = h_n, after every 2048 positions and at the row's end.  h is what the lane holds; the product is
+// exp2(A_n log2e * sum dl), and the sum is per CHANNEL, not per state: each of a channel's four lanes adds up a quarter of
+// every round's positions (one LDS read, four adds per 16 positions) and the quarters meet when a chunk ends.
+//
+// kMaps: CrossScan folded in.  u is not the (batch, 4 D, L) tensor of the four scan-ordered copies but the map itself,
+// x (batch, D, L), plus its transpose xt (batch, D, L: every H x W map stored as W x H): direction k = the channel's
+// group reads x (k = 0, 2) or xt (k = 1, 3), forwards (k < 2) or backwards -- position t of the scan is element t or
+// L - 1 - t of that row (cross_scan_fwd, classification/models/csm_triton.py:22-29).  A lane's four positions are then
+// the four elements that END at L - 1 - t, taken in reverse; where fewer are left, the row's first four.
+//
+// kDwords: the rows of 16-bit inputs start on dwords (RawGroup).
 template <typename in_t, typename out_t, int kSpw, bool kSoftplus, bool kX, bool kMaps, int kPhase, bool kDwords>
-__global__ __launch_bounds__(kBlock, kSpw == 8 ? 2 : kSpw == 1 ? 4 : 3) void scan_chan_kernel(const in_t *__restrict__ u_all, const in_t *__restrict__ dl_all,
+__global__ __launch_bounds__(kBlock, (chan_waves<in_t, kSpw, kX, kMaps, kPhase, kDwords>())) void scan_chan_kernel(const in_t *__restrict__ u_all, const in_t *__restrict__ dl_all,
                                                            const in_t *__restrict__ B_all, const in_t *__restrict__ C_all,
                                                            const float *__restrict__ A_all, out_t *__restrict__ o_all,
                                                            const ScanArgs p, const ChanGeom geo,
