@@ -63,27 +63,9 @@ __device__ __forceinline__ void store2_at(__amdgpu_buffer_rsrc_t buf, uint32_t r
 }
 
 // v[i] summed over the 16 channels (lane / 4) for every i of 16, entry 8 (lane bit 3) + 4 (bit 2) + 2 (bit 5) + (bit 4) left with each
-// lane.  Bits 3 and 2 by pairs of DPP additions with their own banks, bits 5 and 4 by swaps.
+// lane.  Bits 3 and 2 by DPP additions, bits 5 and 4 by swaps.
 __device__ __forceinline__ float sum_over_channels(float (&v)[16]) {
-#define SS2D_ADD(R, S, CTRL) "v_add_f32_dpp %" #R ", %" #S ", %" #S " " CTRL "\n\t"
-#define SS2D_ALL(R) SS2D_ADD(R, R, "row_ror:8 row_mask:0xf bank_mask:0xf")
-#define SS2D_UPPER(R, S) SS2D_ADD(R, S, "row_ror:8 row_mask:0xf bank_mask:0xc")
-#define SS2D_EVEN(R) SS2D_ADD(R, R, "row_shl:4 row_mask:0xf bank_mask:0x5")
-#define SS2D_ODD(R, S) SS2D_ADD(R, S, "row_shr:4 row_mask:0xf bank_mask:0xa")
-    asm("s_nop 1\n\t"
-        SS2D_ALL(0) SS2D_ALL(1) SS2D_ALL(2) SS2D_ALL(3) SS2D_ALL(4) SS2D_ALL(5) SS2D_ALL(6) SS2D_ALL(7)
-        SS2D_UPPER(0, 8) SS2D_UPPER(1, 9) SS2D_UPPER(2, 10) SS2D_UPPER(3, 11)
-        SS2D_UPPER(4, 12) SS2D_UPPER(5, 13) SS2D_UPPER(6, 14) SS2D_UPPER(7, 15)
-        SS2D_EVEN(0) SS2D_EVEN(1) SS2D_EVEN(2) SS2D_EVEN(3)
-        SS2D_ODD(0, 4) SS2D_ODD(1, 5) SS2D_ODD(2, 6) SS2D_ODD(3, 7)
-        "s_nop 1"
-        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
-        : "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]), "v"(v[15]));
-#undef SS2D_ADD
-#undef SS2D_ALL
-#undef SS2D_UPPER
-#undef SS2D_EVEN
-#undef SS2D_ODD
+    sum_over_quads(v);
     auto halves = [](float a, float b) {
         const auto r = __builtin_amdgcn_permlane32_swap(f32_to_bits(a), f32_to_bits(b), false, false);
         return bits_to_f32(r[0]) + bits_to_f32(r[1]);

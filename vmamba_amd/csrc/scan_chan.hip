@@ -77,31 +77,6 @@ template <typename in_t, int kSpw, bool kX, bool kMaps, int kPhase, bool kDwords
     return (kMaps || kPhase == kRest) && (sizeof(in_t) == 4 || (!kDwords && kX)) ? 3 : 4;
 }
 
-// y[i] summed over the four sets of lanes (the banks of four lanes in a row of 16) for every position i of 16: afterwards
-// y[0 .. 3] are positions 4 set .. 4 set + 3.  Two DPP additions, each with its own banks, put two positions into one register:
-// half the additions of a sum that every lane gets, and no selects.
-__device__ __forceinline__ void sum_over_sets(float (&y)[16]) {
-#define SS2D_ADD(R, S, CTRL) "v_add_f32_dpp %" #R ", %" #S ", %" #S " " CTRL "\n\t"
-#define SS2D_ALL(R) SS2D_ADD(R, R, "row_ror:8 row_mask:0xf bank_mask:0xf")
-#define SS2D_UPPER(R, S) SS2D_ADD(R, S, "row_ror:8 row_mask:0xf bank_mask:0xc")
-#define SS2D_EVEN(R) SS2D_ADD(R, R, "row_shl:4 row_mask:0xf bank_mask:0x5")
-#define SS2D_ODD(R, S) SS2D_ADD(R, S, "row_shr:4 row_mask:0xf bank_mask:0xa")
-    asm("s_nop 1\n\t"
-        SS2D_ALL(0) SS2D_ALL(1) SS2D_ALL(2) SS2D_ALL(3) SS2D_ALL(4) SS2D_ALL(5) SS2D_ALL(6) SS2D_ALL(7)
-        SS2D_UPPER(0, 8) SS2D_UPPER(1, 9) SS2D_UPPER(2, 10) SS2D_UPPER(3, 11)
-        SS2D_UPPER(4, 12) SS2D_UPPER(5, 13) SS2D_UPPER(6, 14) SS2D_UPPER(7, 15)
-        SS2D_EVEN(0) SS2D_EVEN(1) SS2D_EVEN(2) SS2D_EVEN(3)
-        SS2D_ODD(0, 4) SS2D_ODD(1, 5) SS2D_ODD(2, 6) SS2D_ODD(3, 7)
-        "s_nop 1"
-        : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(y[4]), "+v"(y[5]), "+v"(y[6]), "+v"(y[7])
-        : "v"(y[8]), "v"(y[9]), "v"(y[10]), "v"(y[11]), "v"(y[12]), "v"(y[13]), "v"(y[14]), "v"(y[15]));
-#undef SS2D_ADD
-#undef SS2D_ALL
-#undef SS2D_UPPER
-#undef SS2D_EVEN
-#undef SS2D_ODD
-}
-
 // kX: the chunk-end states are written as well -- x[row][chunk][2n] = product of a_n since the row's start,
 // x[..][2n + 1] = h_n, after every 2048 positions and at the row's end.  h is what the lane holds; the product is
 // exp2(A_n log2e * sum dl), and the sum is per CHANNEL, not per state: each of a channel's four lanes adds up a quarter of
@@ -342,7 +317,7 @@ __global__ __launch_bounds__(kBlock, (chan_waves<in_t, kSpw, kX, kMaps, kPhase, 
             wave_lds_sync();                                // dl / du, B / C of this round are read
             if constexpr (kPhase != kLocal) {
                 // the four sets' sums: positions 4 set .. + 4 of the lane's channel, into the place of the dl read above
-                sum_over_sets(y);
+                sum_over_quads(y);
                 *reinterpret_cast<float4 *>(my_dl + s * kChanSub + 4 * set) = make_float4(y[0], y[1], y[2], y[3]);
             }
         }

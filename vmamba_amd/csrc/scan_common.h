@@ -428,6 +428,30 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t dwords_of(const void *base, in
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(at & ~(uintptr_t)3), 0, (int)((bytes + 3) & ~3u), kBufferRsrcWord3);
 }
 
+// v[i] summed over the four quads of lanes in a row of 16 (lane bits 2 and 3) for every i of 16: afterwards v[0 .. 3] are entries 4 q .. 4 q + 3 with
+// quad q.  Two DPP additions, each with its own banks, put two entries into one register: half the additions of a sum that every lane gets, and no selects.
+__device__ __forceinline__ void sum_over_quads(float (&v)[16]) {
+#define SS2D_ADD(R, S, CTRL) "v_add_f32_dpp %" #R ", %" #S ", %" #S " " CTRL "\n\t"
+#define SS2D_ALL(R) SS2D_ADD(R, R, "row_ror:8 row_mask:0xf bank_mask:0xf")
+#define SS2D_UPPER(R, S) SS2D_ADD(R, S, "row_ror:8 row_mask:0xf bank_mask:0xc")
+#define SS2D_EVEN(R) SS2D_ADD(R, R, "row_shl:4 row_mask:0xf bank_mask:0x5")
+#define SS2D_ODD(R, S) SS2D_ADD(R, S, "row_shr:4 row_mask:0xf bank_mask:0xa")
+    asm("s_nop 1\n\t"
+        SS2D_ALL(0) SS2D_ALL(1) SS2D_ALL(2) SS2D_ALL(3) SS2D_ALL(4) SS2D_ALL(5) SS2D_ALL(6) SS2D_ALL(7)
+        SS2D_UPPER(0, 8) SS2D_UPPER(1, 9) SS2D_UPPER(2, 10) SS2D_UPPER(3, 11)
+        SS2D_UPPER(4, 12) SS2D_UPPER(5, 13) SS2D_UPPER(6, 14) SS2D_UPPER(7, 15)
+        SS2D_EVEN(0) SS2D_EVEN(1) SS2D_EVEN(2) SS2D_EVEN(3)
+        SS2D_ODD(0, 4) SS2D_ODD(1, 5) SS2D_ODD(2, 6) SS2D_ODD(3, 7)
+        "s_nop 1"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+        : "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]), "v"(v[15]));
+#undef SS2D_ADD
+#undef SS2D_ALL
+#undef SS2D_UPPER
+#undef SS2D_EVEN
+#undef SS2D_ODD
+}
+
 template <bool kSoftplus>
 __device__ __forceinline__ void delta_transform(const float (&raw)[kItems], const float (&bias)[kItems],
                                                 float (&dl)[kItems]) {
