@@ -301,7 +301,7 @@ def _same(got, want):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("N,delta_dim,has_D,has_bias", [(1, 24, True, True), (16, 24, False, True), (2, 24, True, False), (1, 6, False, False)])
-def test_operators_made_in_the_extension_equal_those_made_from_python(N, delta_dim, has_D, has_bias, dtype):
+def test_operators_made_in_the_extension_equal_those_made_from_python(N, delta_dim, has_D, has_bias, dtype, monkeypatch):
     """The three operators forwards and backwards on dense, strided and transposed tensors: the same bits, sizes, strides and types.   (dA, dB, dC and the
     two vectors are sums of atomics over few positions: one wavefront's order.)"""
     from vmamba_amd.csms6s import selective_scan_bwd, selective_scan_fwd
@@ -311,13 +311,25 @@ def test_operators_made_in_the_extension_equal_those_made_from_python(N, delta_d
     delta, A = rand(2, delta_dim, 50) * 0.3, -torch.rand(24, N, generator=g).cuda()
     D, bias = (torch.rand(24, generator=g).cuda() if has_D else None), (torch.rand(delta_dim, generator=g).cuda() if has_bias else None)
     x, ys = rand(2, 6, 5, 10), rand(2, 4, 6, 5, 10)
+    made = []                                                   # of every call of the extension: whether it made the result
+    for name in ("scan_fwd", "scan_bwd", "cross_scan", "cross_merge"):
+        def counted(*args, _native=getattr(_lib.host(), name)):
+            result = _native(*args)
+            made.append(result is not None)
+            return result
+        monkeypatch.setattr(_lib.host(), name, counted)
     calls = [lambda: selective_scan_fwd(u, delta, A, B, C, D, bias, True, 1, True, True), lambda: selective_scan_fwd(u, delta, A, B, C, D, bias, False, 1, False, False),
              lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True)[:2], lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout.float(), None, False)[:2],
              lambda: [va.cross_scan_fn(x)], lambda: [va.cross_scan_fn(x.transpose(2, 3))], lambda: [va.cross_merge_fn(ys)], lambda: [va.cross_merge_fn(ys.transpose(3, 4))]]
-    for call in calls:
+    # the transposed maps are Python's to copy first
+    by_extension = (True, True, delta_dim == 24, delta_dim == 24, True, False, True, False)
+    for call, native in zip(calls, by_extension):
+        made.clear()
         got = call()
+        assert made == [native]
         with _Watching():
             _same(got, call())
+        assert made == [native]                                 # (not asked again)
     sums = lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True)[2:]
     got = sums()
     with _Watching():
