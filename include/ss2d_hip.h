@@ -122,7 +122,7 @@ typedef struct ss2d_scan_params {
 int ss2d_selective_scan_fwd(const ss2d_scan_params *params, void *stream);
 
 /*
- * Which kernel ss2d_selective_scan_fwd would launch for `params` (the same validation, nothing is launched):
+ * Which kind of kernel ss2d_selective_scan_fwd would launch for `params` (the same validation, nothing is launched):
  * one of the ids below, or a negative SS2D_E* code.  Every kernel writes `x` when it is requested, so the answer
  * does not depend on params->x.  No counterpart in the reference (its one kernel template serves every shape,
  * selective_scan_oflex.cpp:224-226); here so that a caller, a benchmark or a test can tell which code path a
@@ -131,11 +131,16 @@ int ss2d_selective_scan_fwd(const ss2d_scan_params *params, void *stream);
 #define SS2D_SCAN_KERNEL_NONE 0  /* empty problem: nothing to launch                                           */
 #define SS2D_SCAN_KERNEL_ROW 1   /* one wavefront per (batch, channel) row                                       */
 #define SS2D_SCAN_KERNEL_ROW4 2  /* few long rows: the four wavefronts of a workgroup share a row                */
-#define SS2D_SCAN_KERNEL_FLAT 3  /* many short rows, or rows off the 16-byte grid: several to a wavefront as one
-                                    stream                                                                      */
+#define SS2D_SCAN_KERNEL_FLAT 3  /* short rows and rows off the 16-byte grid: where there are many, several to
+                                    a wavefront as one stream; few, and long ones, a wavefront each             */
 #define SS2D_SCAN_KERNEL_SMALL 4 /* rows of 49 / 196 positions, one state: a segment of a row per lane           */
 #define SS2D_SCAN_KERNEL_CHAN 5  /* several states per channel: one channel per lane, positions walked serially  */
 int ss2d_selective_scan_kernel(const ss2d_scan_params *params);
+/*
+ * SS2D_SCAN_KERNEL_FLAT above is a class of problems that two kernels share, and the query's answer for all of it.  This one names the
+ * kernel itself: _FLAT where several rows go to a wavefront, _ROW where each has its own, and everywhere else the same as above.
+ */
+int ss2d_selective_scan_launched(const ss2d_scan_params *params);
 
 /*
  * The same forward with CrossScan folded in, for several states per channel: params->u is not the (batch, dim, seqlen)
@@ -182,7 +187,7 @@ int ss2d_selective_scan_bwd(const ss2d_scan_bwd_params *params, void *stream);
 
 /*
  * Which kernel ss2d_selective_scan_bwd launches for these params (>= 0), or the status of a call that launches none.  Nothing is
- * launched; as ss2d_selective_scan_kernel.
+ * launched; as ss2d_selective_scan_launched.
  */
 #define SS2D_SCAN_BWD_KERNEL_NONE 0   /* empty problem                                                            */
 #define SS2D_SCAN_BWD_KERNEL_ROWS 1   /* more than 32 states: one wavefront per (batch, channel) row               */

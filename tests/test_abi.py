@@ -90,8 +90,8 @@ def test_scan_argument_validation():
     assert L.ss2d_selective_scan_fwd(p, None) == _lib.SS2D_EINVAL           # out dtype neither f32 nor input
 
 
-def _scan_plan(batch, dim, L, N, G, in_dtype=_lib.SS2D_BF16, with_x=True, base=1 << 20):
-    """ss2d_selective_scan_kernel for dense tensors of these sizes at made-up, 256-byte aligned addresses (the query
+def _scan_plan(batch, dim, L, N, G, in_dtype=_lib.SS2D_BF16, with_x=True, base=1 << 20, query="ss2d_selective_scan_kernel"):
+    """ss2d_selective_scan_kernel (or another query) for dense tensors of these sizes at made-up, 256-byte aligned addresses (the query
     reads the struct only)."""
     p = _lib.ScanParams()
     p.batch, p.dim, p.seqlen, p.dstate, p.n_groups, p.delta_dim = batch, dim, L, N, G, dim
@@ -104,7 +104,7 @@ def _scan_plan(batch, dim, L, N, G, in_dtype=_lib.SS2D_BF16, with_x=True, base=1
     p.B_batch_stride, p.B_group_stride, p.B_dstate_stride = G * N * L, N * L, L
     p.C_batch_stride, p.C_group_stride, p.C_dstate_stride = G * N * L, N * L, L
     p.out_batch_stride, p.out_d_stride = dim * L, L
-    return _lib.lib().ss2d_selective_scan_kernel(p)
+    return getattr(_lib.lib(), query)(p)
 
 
 def test_scan_kernel_choice_does_not_depend_on_the_chunk_state_output():
@@ -114,9 +114,8 @@ def test_scan_kernel_choice_does_not_depend_on_the_chunk_state_output():
         (128, 384, 3136, 1): _lib.SCAN_KERNEL_ROW, (128, 768, 784, 1): _lib.SCAN_KERNEL_ROW,
         (128, 1536, 196, 1): _lib.SCAN_KERNEL_SMALL, (128, 3072, 49, 1): _lib.SCAN_KERNEL_SMALL,
         (64, 768, 3136, 16): _lib.SCAN_KERNEL_CHAN, (4, 384, 65536, 1): _lib.SCAN_KERNEL_ROW4,
-        (4, 768, 16384, 1): _lib.SCAN_KERNEL_ROW, (48, 384, 3306, 1): _lib.SCAN_KERNEL_ROW,
-        (16, 384, 100, 1): _lib.SCAN_KERNEL_ROW, (128, 384, 100, 1): _lib.SCAN_KERNEL_FLAT, (128, 768, 484, 1): _lib.SCAN_KERNEL_FLAT,
-        (128, 384, 3306, 1): _lib.SCAN_KERNEL_ROW, (1, 768, 3307, 1): _lib.SCAN_KERNEL_ROW4,
+        (4, 768, 16384, 1): _lib.SCAN_KERNEL_ROW, (48, 384, 3306, 1): _lib.SCAN_KERNEL_FLAT,
+        (16, 384, 100, 1): _lib.SCAN_KERNEL_FLAT,
     }
     for (batch, dim, L, N), kernel in shapes.items():
         for with_x in (False, True):
@@ -125,6 +124,24 @@ def test_scan_kernel_choice_does_not_depend_on_the_chunk_state_output():
     assert _scan_plan(2, 384, 3136, 1, 5) == _lib.SS2D_EINVAL
     assert _lib.lib().ss2d_selective_scan_kernel(None) == _lib.SS2D_EINVAL
     assert len(_lib.SCAN_KERNEL_NAMES) == 6
+
+
+def test_scan_kernel_launched():
+    """ss2d_selective_scan_launched names the kernel that runs: where ss2d_selective_scan_kernel says SS2D_SCAN_KERNEL_FLAT for rows that have a wavefront
+    each, it does not; everywhere else the two agree."""
+    flat, row = _lib.SCAN_KERNEL_FLAT, _lib.SCAN_KERNEL_ROW
+    shapes = {  # batch, dim, L, N, groups -> kernel
+        (48, 384, 3306, 1, 4): row, (16, 384, 100, 1, 4): row, (128, 384, 3306, 1, 4): row, (128, 384, 100, 1, 4): flat, (128, 768, 484, 1, 4): flat,
+        (16, 384, 2051, 1, 4): row, (25, 99, 135, 16, 1): row, (1, 48, 1003, 16, 1): row, (131, 128, 36, 16, 8): flat, (131, 128, 33, 16, 8): row,
+        (257, 160, 210, 16, 8): flat,
+    }
+    for (batch, dim, L, N, G), kernel in shapes.items():
+        for with_x in (False, True):
+            assert _scan_plan(batch, dim, L, N, G, with_x=with_x, query="ss2d_selective_scan_launched") == kernel, (batch, dim, L, N, G, with_x)
+            assert _scan_plan(batch, dim, L, N, G, with_x=with_x) == flat
+    for shape in ((128, 384, 3136, 1, 4), (128, 1536, 196, 1, 4), (64, 768, 3136, 16, 4), (4, 384, 65536, 1, 4), (1, 768, 3307, 1, 4), (2, 6, 2309, 3, 1), (0, 384, 9, 1, 4), (2, 384, 9, 1, 5)):
+        assert _scan_plan(*shape) == _scan_plan(*shape, query="ss2d_selective_scan_launched") != flat, shape
+    assert _lib.lib().ss2d_selective_scan_launched(None) == _lib.SS2D_EINVAL
 
 
 def _scan_bwd_plan(batch, dim, L, N, G, dtype=_lib.SS2D_BF16, base=1 << 32):

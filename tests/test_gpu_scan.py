@@ -209,17 +209,15 @@ def test_scan_blocks_of_channels(batch, dim, G, N, L, dtype):
 
 # One state and three: rows of no whole 16-byte pieces read as dwords, a wavefront per row and four; both sides of the lines between a wavefront per
 # row and several rows to one (8192 rows; 16 384 and single elements; rows of two and four).
-ROW_READS = [(2, 8, 4, 1, 1, "row"), (2, 8, 4, 1, 57, "row"), (1, 12, 2, 1, 513, "row"), (1, 6, 2, 3, 335, "row"), (1, 8, 4, 1, 2051, "row4"), (2, 6, 1, 3, 2309, "row4"),
-             (128, 64, 4, 1, 57, "row"), (129, 64, 4, 1, 57, "flat"), (129, 64, 4, 1, 65, "row"), (257, 64, 4, 1, 65, "flat"), (257, 64, 4, 1, 363, "row"), (257, 64, 4, 1, 66, "flat"),
-             (129, 64, 4, 1, 390, "row"), (129, 64, 4, 1, 382, "flat")]
+ROW_READS = [(2, 8, 4, 1, 1), (2, 8, 4, 1, 57), (1, 12, 2, 1, 513), (1, 6, 2, 3, 335), (1, 8, 4, 1, 2051), (2, 6, 1, 3, 2309), (128, 64, 4, 1, 57), (129, 64, 4, 1, 57),
+             (129, 64, 4, 1, 65), (257, 64, 4, 1, 65), (257, 64, 4, 1, 363), (257, 64, 4, 1, 66), (129, 64, 4, 1, 390), (129, 64, 4, 1, 382)]
 
 
-@pytest.mark.parametrize("batch,dim,G,N,L,kernel", ROW_READS)
+@pytest.mark.parametrize("batch,dim,G,N,L", ROW_READS)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-def test_scan_odd_rows(batch, dim, G, N, L, kernel, dtype):
+def test_scan_odd_rows(batch, dim, G, N, L, dtype):
     _announce("scan-row-reads", batch, dim, G, N, L, dtype)
     args = make_inputs(40, batch, dim, G, N, L, dtype, ss2d_like=True)
-    assert kernel_of(*args[:5], want_x=False) == kernel_of(*args[:5], want_x=True) == kernel
     want, xw = orc.selective_scan(*args, True, out_float=True, return_x=True)
     got, x = run_gpu(*args, True, True, want_x=True)
     assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
@@ -229,34 +227,10 @@ def test_scan_odd_rows(batch, dim, G, N, L, kernel, dtype):
         assert torch.allclose(small.float(), want.to(dtype).float(), **TOL16)
 
 
-# Several rows to a wavefront: groups of one, two, four and eight elements within a row, the last wavefront with fewer rows than the others, one state and
-# 16 (of groups of fewer than 32 channels), rows of the shortest and of nearly a chunk; what is on the other side of the rule's lines is a row's own wavefront's.
-MANY_ROWS = [(131, 64, 4, 1, 9, "flat"), (193, 64, 4, 1, 16, "flat"), (193, 64, 4, 1, 72, "flat"), (131, 64, 4, 1, 102, "flat"), (131, 64, 4, 1, 92, "flat"), (17, 1024, 8, 1, 1358, "flat"),
-             (9, 1024, 8, 1, 2044, "row"), (131, 128, 8, 16, 36, "flat"), (131, 128, 8, 16, 24, "flat"), (137, 120, 4, 16, 30, "flat"), (131, 128, 8, 16, 33, "row"), (128, 128, 8, 16, 36, "row"),
-             (131, 128, 8, 16, 212, "row"), (257, 160, 8, 16, 210, "flat")]
-
-
-@pytest.mark.parametrize("batch,dim,G,N,L,kernel", MANY_ROWS)
-@pytest.mark.parametrize("dtype,softplus", [(torch.float32, True), (torch.bfloat16, False), (torch.float16, True)])
-def test_scan_many_short_rows(batch, dim, G, N, L, kernel, dtype, softplus):
-    _announce("scan-many-rows", batch, dim, G, N, L, dtype, softplus)
-    args = make_inputs(43, batch, dim, G, N, L, dtype, ss2d_like=True)
-    if not softplus:
-        args = (args[0], args[1].abs() * 0.1, *args[2:6], args[6].abs() * 0.1)
-    if dtype == torch.float32 and L % 4 == 0 and N == 1 and L > 1000:
-        kernel = "row"                                          # whole 16-byte pieces, and the lanes of the last pass well filled
-    assert kernel_of(*args[:5], want_x=False) == kernel_of(*args[:5], want_x=True) == kernel
-    want, xw = orc.selective_scan(*args, softplus, out_float=True, return_x=True)
-    got, x = run_gpu(*args, softplus, True, want_x=True)
-    assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
-    check_states(x, xw, TOL32)
-    assert torch.equal(run_gpu(*args, softplus, True, want_x=False)[0], got)
-
-
 # Rows of no whole 16-byte pieces in the same kernel: a row shorter than a group of four, one that ends 1, 2 and 3 positions into a group, rows on odd
 # elements, cut rows, 4 to 32 states; what the rule leaves to the other kernels beside it.
-ODD_ROWS = [(2, 64, 2, 16, 3, "chan"), (1, 33, 1, 16, 9, "chan"), (2, 47, 1, 8, 49, "chan"), (1, 40, 1, 32, 62, "chan"), (26, 99, 1, 16, 135, "chan"), (25, 99, 1, 16, 135, "row"), (2, 96, 2, 16, 225, "row"),
-            (1, 48, 1, 16, 1225, "chan"), (1, 48, 1, 16, 1003, "row"), (1, 40, 1, 32, 3306, "chan"), (1, 48, 1, 16, 3306, "row4"), (64, 48, 1, 8, 77, "chan"), (37, 33, 1, 4, 77, "row"),
+ODD_ROWS = [(2, 64, 2, 16, 3, "chan"), (1, 33, 1, 16, 9, "chan"), (2, 47, 1, 8, 49, "chan"), (1, 40, 1, 32, 62, "chan"), (26, 99, 1, 16, 135, "chan"), (25, 99, 1, 16, 135, "flat"), (2, 96, 2, 16, 225, "flat"),
+            (1, 48, 1, 16, 1225, "chan"), (1, 48, 1, 16, 1003, "flat"), (1, 40, 1, 32, 3306, "chan"), (1, 48, 1, 16, 3306, "row4"), (64, 48, 1, 8, 77, "chan"), (37, 33, 1, 4, 77, "row"),
             (39, 33, 1, 4, 77, "chan"), (3, 35, 1, 4, 331, "row"), (1, 64, 1, 4, 3307, "row4")]
 
 
@@ -579,11 +553,11 @@ def test_scan_errors_from_host_api():
 @pytest.mark.parametrize("batch,dim,G,L,dtype", [(16, 384, 4, 2051, torch.bfloat16), (24, 256, 4, 2307, torch.float32),
                                                  (13, 512, 2, 2049, torch.float16)])
 def test_many_long_rows_off_the_vector_grid(batch, dim, G, L, dtype):
-    """6144 rows and more of odd length (no row but the first starts on a 16-byte boundary), a wavefront each.  Every row against the oracle, without
-    and with the chunk states."""
+    """6144 rows and more of odd length (no row but the first starts on a 16-byte boundary): the library walks them eight
+    to a wavefront as one aligned stream.  Every row against the oracle, without and with the chunk states."""
     _announce("scan-long-unaligned", batch, dim, G, L, dtype)
     args = make_inputs(batch * 1000 + L, batch, dim, G, 1, L, dtype, ss2d_like=True)
-    assert kernel_of(*args[:5], want_x=False) == kernel_of(*args[:5], want_x=True) == "row"
+    assert kernel_of(*args[:5], want_x=False) == kernel_of(*args[:5], want_x=True) == "flat"
     want, xw = orc.selective_scan(*args, True, out_float=True, return_x=True)
     for want_x in (False, True):
         got, x = run_gpu(*args, True, True, want_x=want_x)
@@ -600,7 +574,8 @@ def test_full_size_properties(cfg):
     _announce("scan-full", cfg)
     batch, Dn, L, N = dict(stage1=(128, 96, 3136, 1), stage2=(128, 192, 784, 1), stage3=(128, 384, 196, 1),
                            stage4=(128, 768, 49, 1), n16=(64, 192, 3136, 16), hires=(4, 96, 65536, 1),
-                           # many long rows that do not start on 16-byte boundaries (the reference's 57 x 58 check size, an odd map)
+                           # many long rows that do not start on 16-byte boundaries (the reference's 57 x 58 check size,
+                           # an odd map): walked eight rows to a wavefront as one aligned stream
                            rows57x58=(48, 96, 3306, 1), rows75x75=(8, 192, 5625, 1))[cfg]
     K = 4
     g = torch.Generator(device=DEV).manual_seed(28)
@@ -620,3 +595,49 @@ def test_full_size_properties(cfg):
         want = orc.selective_scan(u[b:b + 1].cpu(), delta[b:b + 1].cpu(), A.cpu(), Bm[b:b + 1].cpu(), Cm[b:b + 1].cpu(),
                                   D.cpu(), bias.cpu(), True)
         assert torch.allclose(y[b:b + 1, rows].cpu(), want[:, rows], **TOL32)
+
+
+def launched(u, delta, A, B, C, want_x):
+    """The kernel that runs for these tensors once they sit on the GPU."""
+    from vmamba_amd.csms6s import scan_kernel_launched
+    dev = lambda t: t.to(DEV)
+    x = torch.empty(*u.shape[:2], (u.shape[-1] + _lib.SCAN_CHUNK - 1) // _lib.SCAN_CHUNK, 2 * A.shape[1], device=DEV) if want_x else None
+    return scan_kernel_launched(dev(u), dev(delta), dev(A), dev(B), dev(C), torch.empty(u.shape, device=DEV), x)
+
+
+# The kernel that runs for each of ROW_READS, and of those in ODD_ROWS whose class is that of several rows to a wavefront.
+LAUNCHED = list(zip(ROW_READS, ("row", "row", "row", "row", "row4", "row4", "row", "flat", "row", "flat", "row", "flat", "row", "flat")))
+LAUNCHED += [(case[:5], "row") for case in ODD_ROWS if case[5] == "flat"]
+LAUNCHED += [((16, 384, 4, 1, 2051), "row"), ((13, 512, 2, 1, 2049), "row")]
+
+
+@pytest.mark.parametrize("case,kernel", LAUNCHED)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_scan_odd_rows_kernel_that_runs(case, kernel, dtype):
+    batch, dim, G, N, L = case
+    u, A, B = torch.empty(batch, dim, L, dtype=dtype), torch.empty(dim, N), torch.empty(batch, G, N, L, dtype=dtype)
+    assert launched(u, u, A, B, B, False) == launched(u, u, A, B, B, True) == kernel
+
+
+# Several rows to a wavefront: groups of one, two, four and eight elements within a row, the last wavefront with fewer rows than the others, one state and
+# 16 (of groups of fewer than 32 channels), rows of the shortest and of nearly a chunk; what is on the other side of the rule's lines is a row's own wavefront's.
+MANY_ROWS = [(131, 64, 4, 1, 9, "flat"), (193, 64, 4, 1, 16, "flat"), (193, 64, 4, 1, 72, "flat"), (131, 64, 4, 1, 102, "flat"), (131, 64, 4, 1, 92, "flat"), (17, 1024, 8, 1, 1358, "flat"),
+             (9, 1024, 8, 1, 2044, "row"), (131, 128, 8, 16, 36, "flat"), (131, 128, 8, 16, 24, "flat"), (137, 120, 4, 16, 30, "flat"), (131, 128, 8, 16, 33, "row"), (128, 128, 8, 16, 36, "row"),
+             (131, 128, 8, 16, 212, "row"), (257, 160, 8, 16, 210, "flat")]
+
+
+@pytest.mark.parametrize("batch,dim,G,N,L,kernel", MANY_ROWS)
+@pytest.mark.parametrize("dtype,softplus", [(torch.float32, True), (torch.bfloat16, False), (torch.float16, True)])
+def test_scan_many_short_rows(batch, dim, G, N, L, kernel, dtype, softplus):
+    _announce("scan-many-rows", batch, dim, G, N, L, dtype, softplus)
+    args = make_inputs(43, batch, dim, G, N, L, dtype, ss2d_like=True)
+    if not softplus:
+        args = (args[0], args[1].abs() * 0.1, *args[2:6], args[6].abs() * 0.1)
+    if dtype == torch.float32 and L % 4 == 0 and N == 1 and L > 1000:
+        kernel = "row"                                          # whole 16-byte pieces, and the lanes of the last pass well filled
+    assert launched(*args[:5], want_x=False) == launched(*args[:5], want_x=True) == kernel
+    want, xw = orc.selective_scan(*args, softplus, out_float=True, return_x=True)
+    got, x = run_gpu(*args, softplus, True, want_x=True)
+    assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
+    check_states(x, xw, TOL32)
+    assert torch.equal(run_gpu(*args, softplus, True, want_x=False)[0], got)

@@ -43,13 +43,6 @@ def compare(got, want, tol, what):
         assert err <= tol * scale + tol * 1e-3, f"{what} {name}: max err {err} vs scale {scale}"
 
 
-def bwd_kernel_of(u, delta, A, B, C, dout):
-    """Name of the kernel the library picks for these tensors once they sit on the GPU."""
-    from vmamba_amd.csms6s import scan_bwd_kernel_name
-    u, delta, A, B, C, dout = (t.to(DEV) for t in (u, delta, A, B, C, dout))
-    return scan_bwd_kernel_name(u, delta, A, B, C, dout, torch.empty(u.shape, device=DEV, dtype=u.dtype), torch.empty(u.shape, device=DEV, dtype=u.dtype))
-
-
 CASES = [
     # batch, dim, G, N, L, delta_dim, softplus
     (2, 4, 1, 1, 40, None, True),          # one short pass
@@ -129,15 +122,13 @@ def test_scan_bwd_odd_rows(N, L, dtype, dout_float):
     compare(got, want, 1e-4 if dtype == torch.float32 else 3e-2, "odd rows")
 
 
-# A channel per lane (scan_bwd_chan.hip): rows of one segment (up to 72 positions, many of them), of two, and of many, equal or not; the last chunk of 8 positions with
+# A channel per lane (scan_bwd_chan.hip): rows of one segment (up to 72 positions, many of them), of two, and of many; the last chunk of 8 positions with
 # 1, 3, 7 and 8 of them; 16, 33, 50 and 51 channels per group (1 and 2 in the last wavefront, idle wavefronts); 4, 8 and 16 states; delta rows
 # shared; rows off the dword grid.  Bound in single precision: sums of up to 1030 terms and 51 channels, each term good to a few 2^-23 -- 1e-4 of the largest gradient.
 CHANNEL_CASES = [
     (64, 64, 1, 16, 72, None, True), (64, 64, 1, 16, 73, None, True), (64, 66, 2, 8, 33, None, True), (64, 64, 1, 8, 7, None, False), (128, 64, 1, 4, 57, None, True),
     (64, 64, 1, 16, 128, None, True), (1, 96, 2, 16, 512, None, True), (1, 50, 1, 8, 515, 10, True), (1, 16, 1, 4, 1030, None, True), (2, 51, 1, 16, 779, 17, True),
     (1, 33, 1, 16, 600, None, False), (1, 80, 1, 16, 1000, None, True),
-    # lengths that no equal segments fill: what is left for the last one would be shorter than its states
-    (1, 17, 1, 16, 529, None, True), (1, 32, 2, 16, 729, None, False), (1, 20, 1, 16, 961, 10, True), (1, 16, 1, 8, 585, None, True),
 ]
 
 
@@ -148,7 +139,6 @@ def test_scan_bwd_channel_per_lane(case, dtype):
     print("CASE scan-bwd-chan", case, dtype, flush=True)
     u, delta, A, B, C, D, bias, dout = make(sum(map(int, case[:5])), batch, dim, G, N, L, dtype, delta_dim, softplus)
     dout = dout.to(dtype) if L % 3 == 0 else dout
-    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
     want = torch_ref.selective_scan_grads(u.float(), delta.float(), A, B.float(), C.float(), D, bias, dout.float(), softplus)
     got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, softplus, 1)
     compare(got, want, 1e-4 if dtype == torch.float32 else 3e-2, "channel per lane")
@@ -161,7 +151,6 @@ def test_scan_bwd_channel_per_lane_strided_views(dtype):
     batch, dim, N, L = 2, 50, 16, 600
     u, delta, A, B, C, D, bias, dout = [t.to(DEV) for t in make(3, batch, dim, 1, N, L, dtype)]
     want = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
-    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
 
     def view(t, pitch):
         rows = t.reshape(-1, t.shape[-1])
@@ -185,58 +174,12 @@ def test_scan_bwd_channel_per_lane_keeps_channels_apart():
     last one's constants, included."""
     batch, dim, N, L = 1, 50, 16, 600
     u, delta, A, B, C, D, bias, dout = [t.to(DEV) for t in make(4, batch, dim, 1, N, L, torch.float32)]
-    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
     want = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
     u[0, 49, 300] = float("nan")
     got = va.selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True, 1)
     for i in (0, 1):
         assert torch.equal(got[i][:, :49], want[i][:, :49])
     assert bool(got[1][0, 49, :301].isnan().any()) and bool(got[2][:49].isfinite().all())
-
-
-@pytest.mark.parametrize("L", [600, 72])
-def test_scan_bwd_channel_per_lane_lanes_without_a_channel_add_nothing(L):
-    """33 channels per group: 15 lanes of the third wavefront have none.  The last channel's bias alone would let their decay overflow (softplus off,
-    exp(-20 * -30)), where its own steps are small; an infinite C makes g of a zero dout NaN.  dB and dC are the real channels' sums."""
-    print("CASE scan-bwd-chan-idle-lanes", L, flush=True)
-    batch, dim, N = 96 if L == 72 else 1, 33, 16
-    u, delta, A, B, C, D, bias, dout = make(6, batch, dim, 1, N, L, torch.float32, softplus=False)
-    A[32], bias[32] = -20.0, -30.0
-    delta[:, 32] += 30.0
-    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
-    want = torch_ref.selective_scan_grads(u, delta, A, B, C, D, bias, dout, False)
-    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)
-    compare(got[3:5], want[3:5], 1e-4, "overflowing decay")
-    u, delta, A, B, C, D, bias, dout = make(6, batch, dim, 1, N, L, torch.float32, softplus=False)
-    u, B, C, dout = [t.abs() + 0.1 for t in (u, B, C, dout)]
-    C[0, 0, 5, L - 1] = float("inf")
-    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)
-    assert bool((got[3][0, 0, 5] == float("inf")).all()) and bool(got[3][0, 0, :5].isfinite().all()) and bool(got[4].isfinite().all())
-
-
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("N,L", [(4, 680), (8, 1000), (16, 700)])
-def test_scan_bwd_channel_per_lane_infinite_states(N, L, dtype):
-    """An infinite state and an infinite adjoint go through segments whose decays multiply to 0, as they would position by position (every one of them is
-    above exp(-6)): infinities, not NaN, and only where they belong."""
-    print("CASE scan-bwd-chan-infinite", N, L, dtype, flush=True)
-    dim, inf, first, last = 16, float("inf"), 100, L - 90
-    u, delta, A, B, C, D, bias, dout = make(8, 1, dim, 1, N, L, dtype, softplus=False)
-    u, B, C, dout = [t.abs() + 0.125 for t in (u, B, C, dout)]                  # every sum is one of positive terms
-    A, delta, bias, D = torch.full_like(A, -1.0), 5.0 + delta.abs(), torch.zeros_like(bias), D.abs()
-    call = lambda: [t.double().cpu() for t in va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)]
-    u[0, 3, first] = inf
-    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
-    du, ddelta, dA, dB, dC = call()[:5]
-    assert bool((dC[0, 0, :, first:] == inf).all()) and bool(dC[0, 0, :, :first].isfinite().all())
-    assert bool((dB[0, 0, :, first] == inf).all()) and bool(dB[0, 0, :, :first].isfinite().all()) and bool(dB[0, 0, :, first + 1:].isfinite().all())
-    assert bool(du.isfinite().all()) and bool((ddelta[0, 3, first + 1:] == -inf).all()) and bool(ddelta[0, 3, :first].isfinite().all())
-    assert not bool(dA[3].isfinite().any()) and bool(dA[:3].isfinite().all()) and bool(ddelta[0, 4:].isfinite().all())
-    u[0, 3, first], dout[0, 5, last] = 1.0, inf
-    du, ddelta, dA, dB, dC = call()[:5]
-    assert bool((du[0, 5, :last + 1] == inf).all()) and bool(du[0, 5, last + 1:].isfinite().all()) and bool(du[0, :5].isfinite().all())
-    assert bool((dB[0, 0, :, :last + 1] == inf).all()) and bool(dB[0, 0, :, last + 1:].isfinite().all())
-    assert bool((dC[0, 0, :, last] == inf).all()) and bool(dC[0, 0, :, :last].isfinite().all()) and bool(ddelta[0, :5].isfinite().all())
 
 
 def test_selective_scan_fn_trains():
@@ -301,7 +244,7 @@ def _same(got, want):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("N,delta_dim,has_D,has_bias", [(1, 24, True, True), (16, 24, False, True), (2, 24, True, False), (1, 6, False, False)])
-def test_operators_made_in_the_extension_equal_those_made_from_python(N, delta_dim, has_D, has_bias, dtype, monkeypatch):
+def test_operators_made_in_the_extension_equal_those_made_from_python(N, delta_dim, has_D, has_bias, dtype):
     """The three operators forwards and backwards on dense, strided and transposed tensors: the same bits, sizes, strides and types.   (dA, dB, dC and the
     two vectors are sums of atomics over few positions: one wavefront's order.)"""
     from vmamba_amd.csms6s import selective_scan_bwd, selective_scan_fwd
@@ -311,25 +254,13 @@ def test_operators_made_in_the_extension_equal_those_made_from_python(N, delta_d
     delta, A = rand(2, delta_dim, 50) * 0.3, -torch.rand(24, N, generator=g).cuda()
     D, bias = (torch.rand(24, generator=g).cuda() if has_D else None), (torch.rand(delta_dim, generator=g).cuda() if has_bias else None)
     x, ys = rand(2, 6, 5, 10), rand(2, 4, 6, 5, 10)
-    made = []                                                   # of every call of the extension: whether it made the result
-    for name in ("scan_fwd", "scan_bwd", "cross_scan", "cross_merge"):
-        def counted(*args, _native=getattr(_lib.host(), name)):
-            result = _native(*args)
-            made.append(result is not None)
-            return result
-        monkeypatch.setattr(_lib.host(), name, counted)
     calls = [lambda: selective_scan_fwd(u, delta, A, B, C, D, bias, True, 1, True, True), lambda: selective_scan_fwd(u, delta, A, B, C, D, bias, False, 1, False, False),
              lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True)[:2], lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout.float(), None, False)[:2],
              lambda: [va.cross_scan_fn(x)], lambda: [va.cross_scan_fn(x.transpose(2, 3))], lambda: [va.cross_merge_fn(ys)], lambda: [va.cross_merge_fn(ys.transpose(3, 4))]]
-    # the transposed maps are Python's to copy first
-    by_extension = (True, True, delta_dim == 24, delta_dim == 24, True, False, True, False)
-    for call, native in zip(calls, by_extension):
-        made.clear()
+    for call in calls:
         got = call()
-        assert made == [native]
         with _Watching():
             _same(got, call())
-        assert made == [native]                                 # (not asked again)
     sums = lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True)[2:]
     got = sums()
     with _Watching():
@@ -355,3 +286,100 @@ def test_operators_made_in_the_extension_refuse_what_python_refuses():
         va.cross_scan_fn(u)
     with pytest.raises(TypeError):
         va.cross_merge_fn(torch.zeros(1, 4, 2, 3, 3, device="cuda", dtype=torch.float64))
+
+
+def bwd_kernel_of(u, delta, A, B, C, dout):
+    """Name of the kernel the library picks for these tensors once they sit on the GPU."""
+    from vmamba_amd.csms6s import scan_bwd_kernel_name
+    u, delta, A, B, C, dout = (t.to(DEV) for t in (u, delta, A, B, C, dout))
+    return scan_bwd_kernel_name(u, delta, A, B, C, dout, torch.empty(u.shape, device=DEV, dtype=u.dtype), torch.empty(u.shape, device=DEV, dtype=u.dtype))
+
+
+# lengths that no equal segments fill: what is left for the last one would be shorter than its states
+UNEVEN_CASES = [(1, 17, 1, 16, 529, None, True), (1, 32, 2, 16, 729, None, False), (1, 20, 1, 16, 961, 10, True), (1, 16, 1, 8, 585, None, True)]
+
+
+@pytest.mark.parametrize("case", CHANNEL_CASES + UNEVEN_CASES, ids=lambda c: "x".join(str(v) for v in c))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_bwd_channel_per_lane_is_the_kernel_that_runs(case, dtype):
+    batch, dim, G, N, L, delta_dim, softplus = case
+    u, delta, A, B, C, D, bias, dout = make(sum(map(int, case[:5])), batch, dim, G, N, L, dtype, delta_dim, softplus)
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == bwd_kernel_of(u, delta, A, B, C, dout.to(dtype)) == "chan"
+
+
+@pytest.mark.parametrize("case", UNEVEN_CASES, ids=lambda c: "x".join(str(v) for v in c))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_bwd_channel_per_lane_uneven_segments(case, dtype):
+    test_scan_bwd_channel_per_lane(case, dtype)
+
+
+@pytest.mark.parametrize("L", [600, 72])
+def test_scan_bwd_channel_per_lane_lanes_without_a_channel_add_nothing(L):
+    """33 channels per group: 15 lanes of the third wavefront have none.  The last channel's bias alone would let their decay overflow (softplus off,
+    exp(-20 * -30)), where its own steps are small; an infinite C makes g of a zero dout NaN.  dB and dC are the real channels' sums."""
+    print("CASE scan-bwd-chan-idle-lanes", L, flush=True)
+    batch, dim, N = 96 if L == 72 else 1, 33, 16
+    u, delta, A, B, C, D, bias, dout = make(6, batch, dim, 1, N, L, torch.float32, softplus=False)
+    A[32], bias[32] = -20.0, -30.0
+    delta[:, 32] += 30.0
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
+    want = torch_ref.selective_scan_grads(u, delta, A, B, C, D, bias, dout, False)
+    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)
+    compare(got[3:5], want[3:5], 1e-4, "overflowing decay")
+    u, delta, A, B, C, D, bias, dout = make(6, batch, dim, 1, N, L, torch.float32, softplus=False)
+    u, B, C, dout = [t.abs() + 0.1 for t in (u, B, C, dout)]
+    C[0, 0, 5, L - 1] = float("inf")
+    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)
+    assert bool((got[3][0, 0, 5] == float("inf")).all()) and bool(got[3][0, 0, :5].isfinite().all()) and bool(got[4].isfinite().all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,L", [(4, 680), (8, 1000), (16, 700)])
+def test_scan_bwd_channel_per_lane_infinite_states(N, L, dtype):
+    """An infinite state and an infinite adjoint go through segments whose decays multiply to 0, as they would position by position (every one of them is
+    above exp(-6)): infinities, not NaN, and only where they belong."""
+    print("CASE scan-bwd-chan-infinite", N, L, dtype, flush=True)
+    dim, inf, first, last = 16, float("inf"), 100, L - 90
+    u, delta, A, B, C, D, bias, dout = make(8, 1, dim, 1, N, L, dtype, softplus=False)
+    u, B, C, dout = [t.abs() + 0.125 for t in (u, B, C, dout)]                  # every sum is one of positive terms
+    A, delta, bias, D = torch.full_like(A, -1.0), 5.0 + delta.abs(), torch.zeros_like(bias), D.abs()
+    call = lambda: [t.double().cpu() for t in va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, False, 1)]
+    u[0, 3, first] = inf
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == "chan"
+    du, ddelta, dA, dB, dC = call()[:5]
+    assert bool((dC[0, 0, :, first:] == inf).all()) and bool(dC[0, 0, :, :first].isfinite().all())
+    assert bool((dB[0, 0, :, first] == inf).all()) and bool(dB[0, 0, :, :first].isfinite().all()) and bool(dB[0, 0, :, first + 1:].isfinite().all())
+    assert bool(du.isfinite().all()) and bool((ddelta[0, 3, first + 1:] == -inf).all()) and bool(ddelta[0, 3, :first].isfinite().all())
+    assert not bool(dA[3].isfinite().any()) and bool(dA[:3].isfinite().all()) and bool(ddelta[0, 4:].isfinite().all())
+    u[0, 3, first], dout[0, 5, last] = 1.0, inf
+    du, ddelta, dA, dB, dC = call()[:5]
+    assert bool((du[0, 5, :last + 1] == inf).all()) and bool(du[0, 5, last + 1:].isfinite().all()) and bool(du[0, :5].isfinite().all())
+    assert bool((dB[0, 0, :, :last + 1] == inf).all()) and bool(dB[0, 0, :, last + 1:].isfinite().all())
+    assert bool((dC[0, 0, :, last] == inf).all()) and bool(dC[0, 0, :, :last].isfinite().all()) and bool(ddelta[0, :5].isfinite().all())
+
+
+@pytest.mark.parametrize("N,delta_dim", [(1, 24), (16, 24), (1, 6)])
+def test_operators_are_made_in_the_extension(N, delta_dim, monkeypatch):
+    """The extension makes what it is asked for, strided tensors included; what it leaves to Python are transposed maps and delta rows shared in the backward; and
+    it is not asked where someone follows the operators."""
+    from vmamba_amd.csms6s import selective_scan_bwd, selective_scan_fwd
+    rand = lambda *s: torch.rand(*s, device="cuda")
+    u, B, C, dout = rand(2, 30, 60)[:, 3:27, 8:58], rand(2, 4, N, 50), rand(2, 4, N + 1, 50)[:, :, :N], rand(2, 24, 50)
+    delta, A, D, bias, x, ys = rand(2, delta_dim, 50), -rand(24, N), rand(24), rand(delta_dim), rand(2, 6, 5, 10), rand(2, 4, 6, 5, 10)
+    made = []                                                   # of every call of the extension: whether it made the result
+    for name in ("scan_fwd", "scan_bwd", "cross_scan", "cross_merge"):
+        def counted(*args, _native=getattr(_lib.host(), name)):
+            result = _native(*args)
+            made.append(result is not None)
+            return result
+        monkeypatch.setattr(_lib.host(), name, counted)
+    calls = [(lambda: selective_scan_fwd(u, delta, A, B, C, D, bias, True, 1, True, True), True), (lambda: selective_scan_bwd(u, delta, A, B, C, D, bias, dout, None, True), delta_dim == 24),
+             (lambda: va.cross_scan_fn(x), True), (lambda: va.cross_scan_fn(x.transpose(2, 3)), False), (lambda: va.cross_merge_fn(ys), True),
+             (lambda: va.cross_merge_fn(ys.transpose(3, 4)), False)]
+    for call, native in calls:
+        made.clear()
+        call()
+        assert made == [native]
+        with _Watching():
+            call()
+        assert made == [native]

@@ -22,7 +22,7 @@ SCAN_KERNEL_NAMES = ("none", "row", "row4", "flat", "small", "chan")
 SCAN_BWD_KERNEL_NAMES = ("none", "rows", "one", "states", "chan")
 
 EXPORTS = ("ss2d_abi_version", "ss2d_strerror", "ss2d_cross_scan", "ss2d_cross_merge", "ss2d_selective_scan_fwd",
-           "ss2d_selective_scan_kernel", "ss2d_selective_scan_fwd_maps",
+           "ss2d_selective_scan_kernel", "ss2d_selective_scan_launched", "ss2d_selective_scan_fwd_maps",
            "ss2d_layer_norm", "ss2d_add_layer_norm", "ss2d_bias_layer_norm", "ss2d_layer_norm_cf", "ss2d_layer_norm_cf_crop", "ss2d_dwconv3x3_silu",
            "ss2d_dwconv3x3_silu_f32", "ss2d_dwconv3x3_silu_bwd", "ss2d_dwconv3x3_silu_bwd_workspace_bytes", "ss2d_cross_scan_1b1", "ss2d_core_fwd",
            "ss2d_core_workspace_bytes", "ss2d_core_fwd_ws", "ss2d_forward_core", "ss2d_forward_core_workspace_bytes", "ss2d_block_fwd", "ss2d_block_workspace_bytes", "ss2d_few_rows_bytes", "ss2d_few_applies", "ss2d_x_proj_few", "ss2d_core_few", "ss2d_core_mask_pads", "ss2d_core_embed_maps",
@@ -121,6 +121,8 @@ def lib():
         L.ss2d_selective_scan_fwd_maps.argtypes = [ctypes.POINTER(ScanParams), ctypes.c_void_p, ctypes.c_void_p]
         L.ss2d_selective_scan_kernel.restype = ctypes.c_int
         L.ss2d_selective_scan_kernel.argtypes = [ctypes.POINTER(ScanParams)]
+        L.ss2d_selective_scan_launched.restype = ctypes.c_int
+        L.ss2d_selective_scan_launched.argtypes = [ctypes.POINTER(ScanParams)]
         L.ss2d_layer_norm.restype = ctypes.c_int
         L.ss2d_layer_norm.argtypes = ([ctypes.c_void_p] * 4 + [ctypes.c_int64, ctypes.c_int, ctypes.c_float]
                                       + [ctypes.c_int] * 3 + [ctypes.c_void_p])

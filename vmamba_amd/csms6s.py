@@ -46,10 +46,17 @@ def _scan_params(u, delta, A, B, C, D, delta_bias, delta_softplus, out, x):
 
 
 def scan_kernel_name(u, delta, A, B, C, out, x=None):
-    """Which kernel of the library serves these (already allocated) tensors: one of _lib.SCAN_KERNEL_NAMES.  Nothing
-    is launched (ss2d_selective_scan_kernel)."""
+    """Which kind of kernel of the library serves these (already allocated) tensors: one of _lib.SCAN_KERNEL_NAMES, "flat" for the rows that go several to a
+    wavefront where there are many of them and have one each otherwise.  Nothing is launched (ss2d_selective_scan_kernel)."""
     rc = _lib.lib().ss2d_selective_scan_kernel(_scan_params(u, delta, A, B, C, None, None, True, out, x))
     _lib.check(min(rc, 0), "ss2d_selective_scan_kernel")
+    return _lib.SCAN_KERNEL_NAMES[rc]
+
+
+def scan_kernel_launched(u, delta, A, B, C, out, x=None):
+    """The kernel itself: as scan_kernel_name, but "row" for the rows of its "flat" that have a wavefront each (ss2d_selective_scan_launched)."""
+    rc = _lib.lib().ss2d_selective_scan_launched(_scan_params(u, delta, A, B, C, None, None, True, out, x))
+    _lib.check(min(rc, 0), "ss2d_selective_scan_launched")
     return _lib.SCAN_KERNEL_NAMES[rc]
 
 

@@ -614,15 +614,25 @@ static bool span_fits_u32(const ScanArgs &a, int64_t elem_bytes) {
            span_elems(a, a.B_bs, a.B_gs, a.B_ns) * elem_bytes < lim && span_elems(a, a.C_bs, a.C_gs, a.C_ns) * elem_bytes < lim;
 }
 
-// The flat kernel needs dense u / delta / out (rows adjacent in memory, base 16-byte aligned), one delta row
-// per channel, rows of at least one lane vector and shorter than a chunk (longer ones gather B and C element by element for nothing: 6144 rows of 2051
-// positions, one state in bf16, 62.9 us so and 30.4 a wavefront each, 24 576 of 5625 389 and 262), and dstate 1 or 16.
-static bool flat_eligible(const ScanArgs &a, const ss2d_scan_params *q) {
+// Rows that may be walked as one stream: dense u / delta / out (rows adjacent in memory, base 16-byte aligned), one delta row
+// per channel, rows of at least one lane vector, and dstate 1 or 16.
+static bool one_stream(const ScanArgs &a, const ss2d_scan_params *q) {
     const int64_t L = a.L, KD = a.dim;
-    return L >= kItems && L < 4 * kPass && (a.N == 1 || a.N == 16) && q->delta_dim == q->dim &&
+    return L >= kItems && (a.N == 1 || a.N == 16) && q->delta_dim == q->dim &&
            a.u_ds == L && a.dl_ds == L && a.o_ds == L && a.u_bs == KD * L && a.dl_bs == KD * L && a.o_bs == KD * L &&
            aligned16(q->u) && aligned16(q->delta) && aligned16(q->out) &&
            span_fits_u32(a, q->in_dtype == SS2D_F32 ? 4 : 2);
+}
+
+// The flat kernel takes those shorter than a chunk (longer ones gather B and C element by element for nothing: 6144 rows of 2051
+// positions, one state in bf16, 62.9 us so and 30.4 a wavefront each, 24 576 of 5625 389 and 262).
+static bool flat_eligible(const ScanArgs &a, const ss2d_scan_params *q) { return a.L < 4 * kPass && one_stream(a, q); }
+
+// What ss2d_selective_scan_kernel calls SS2D_SCAN_KERNEL_FLAT: short rows and, one state and many of them, long ones, off the 16-byte grid or with more than
+// 30 % of the lanes of a wavefront per row idle.  A class of problems, and a wider one than the flat kernel's (flat_pays).
+static bool flat_class(const ScanArgs &a, const ss2d_scan_params *q, bool vec) {
+    const bool length_ok = a.L < 4 * kPass || (a.L <= (1 << 24) && a.N == 1 && a.rows >= 6144);
+    return length_ok && one_stream(a, q) && (!vec || 10 * (int64_t)a.L < 7 * (((int64_t)a.L + kPass - 1) / kPass * kPass));
 }
 
 static int flat_granularity(const ScanArgs &a, int64_t elem_bytes);
@@ -750,7 +760,7 @@ static int dispatch_vec(const ScanArgs &a, bool vec, int kernel, hipStream_t str
 
 namespace ss2d {
 
-// Validation and kernel choice shared by the launch and the query entry points.  Returns an SS2D_SCAN_KERNEL_* id
+// Validation and kernel choice shared by the launch and the query entry points.  Returns the SS2D_SCAN_KERNEL_* id of the kernel to launch
 // (SS2D_SCAN_KERNEL_NONE for an empty problem) or a negative status; fills `a` and `vec` for the launch.
 static int plan_scan(const ss2d_scan_params *q, ScanArgs &a, bool &vec) {
     if (!q) return SS2D_EINVAL;
@@ -809,10 +819,17 @@ static int plan_scan(const ss2d_scan_params *q, ScanArgs &a, bool &vec) {
 
 }  // namespace ss2d
 
-extern "C" int ss2d_selective_scan_kernel(const ss2d_scan_params *q) {
+extern "C" int ss2d_selective_scan_launched(const ss2d_scan_params *q) {
     ss2d::ScanArgs a;
     bool vec = false;
     return ss2d::plan_scan(q, a, vec);
+}
+
+extern "C" int ss2d_selective_scan_kernel(const ss2d_scan_params *q) {
+    ss2d::ScanArgs a;
+    bool vec = false;
+    const int kernel = ss2d::plan_scan(q, a, vec);
+    return kernel == SS2D_SCAN_KERNEL_ROW && ss2d::flat_class(a, q, vec) ? SS2D_SCAN_KERNEL_FLAT : kernel;
 }
 
 extern "C" int ss2d_selective_scan_fwd_maps(const ss2d_scan_params *q, const void *x_t, void *stream) {
