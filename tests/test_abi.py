@@ -144,6 +144,20 @@ def test_scan_kernel_launched():
     assert _lib.lib().ss2d_selective_scan_launched(None) == _lib.SS2D_EINVAL
 
 
+def test_scan_channel_per_lane_rule_of_rows_off_the_grid():
+    """Both sides of the lines between a channel per lane and positions in lanes, for rows of an odd number of fours in single precision and of an odd length."""
+    chan = lambda N, L, batch, dtype=_lib.SS2D_F32: _scan_plan(batch, 384, L, N, 4, in_dtype=dtype, query="ss2d_selective_scan_launched") == _lib.SCAN_KERNEL_CHAN
+    for N, L, batches in ((16, 100, (4, 8)), (16, 196, (15, 16)), (16, 484, (49, 50)), (16, 900, (26, 27)), (16, 1332, (31, 32)), (8, 196, (16, 17)), (8, 1028, (31, 32)), (4, 1028, (31, 32)), (4, 1764, (31, 32)),
+                          (32, 900, (26, 27)), (32, 3364, (31, 32)), (4, 3364, (106, 107))):
+        assert [chan(N, L, batch) for batch in batches] == [False, True], (N, L)
+    for N, L, batches in ((4, 1764, (42, 43)), (4, 900, (85, 86)), (16, 1764, (2, 3)), (32, 1332, (2, 3)), (32, 5476, (2, 3))):
+        assert [chan(N, L, batch) for batch in batches] == [True, False], (N, L)
+    assert not any(chan(4, L, 128) for L in range(404, 512, 8)) and all(chan(4, L, 128) for L in (324, 396, 516, 764))
+    assert [chan(16, L, 1) for L in (68, 76, 1028, 1532, 1540, 2044, 2052)] == [True, False, False, False, True, True, False]
+    assert [chan(4, 1301, batch, _lib.SS2D_BF16) for batch in (42, 43, 128)] == [False] * 3 and [chan(4, 961, b, _lib.SS2D_BF16) for b in (42, 43, 85, 86)] == [False, True, True, False]
+    assert all(chan(N, L, batch) for N in (4, 8, 16, 32) for L in (104, 200, 1336, 3360) for batch in (1, 64))      # whole eights: at any size
+
+
 def _scan_bwd_plan(batch, dim, L, N, G, dtype=_lib.SS2D_BF16, base=1 << 32):
     """ss2d_selective_scan_bwd_kernel for dense tensors of these sizes at made-up, 256-byte aligned addresses far apart."""
     p = _lib.ScanBwdParams()

@@ -641,3 +641,19 @@ def test_scan_many_short_rows(batch, dim, G, N, L, kernel, dtype, softplus):
     assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
     check_states(x, xw, TOL32)
     assert torch.equal(run_gpu(*args, softplus, True, want_x=False)[0], got)
+
+
+# Rows of an odd number of fours, which single precision reads in whole pieces whichever kernel it is: both sides of the rule's lines.
+ODD_FOURS = [(2, 64, 2, 16, 68, "chan"), (2, 64, 2, 16, 76, "row"), (3, 48, 1, 16, 1532, "row"), (3, 48, 1, 16, 1540, "chan"), (1, 48, 1, 16, 2052, "row4"), (2, 40, 1, 32, 1332, "chan"), (2, 40, 1, 32, 2116, "row4"),
+             (1, 40, 1, 32, 4100, "chan"), (98, 32, 1, 8, 124, "chan"), (60, 32, 1, 8, 124, "row"), (1040, 32, 1, 4, 404, "row"), (1040, 32, 1, 4, 396, "chan")]
+
+
+@pytest.mark.parametrize("batch,dim,G,N,L,kernel", ODD_FOURS)
+def test_scan_odd_fours(batch, dim, G, N, L, kernel):
+    _announce("scan-odd-fours", batch, dim, G, N, L)
+    args = make_inputs(44, batch, dim, G, N, L, torch.float32, ss2d_like=True)
+    assert launched(*args[:5], want_x=False) == launched(*args[:5], want_x=True) == kernel
+    want, xw = orc.selective_scan(*args, True, out_float=True, return_x=True)
+    got, x = run_gpu(*args, True, True, want_x=True)
+    assert torch.allclose(got, want, **TOL32), f"max abs err {(got - want).abs().max().item()}"
+    check_states(x, xw, TOL32)

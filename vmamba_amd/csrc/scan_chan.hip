@@ -406,33 +406,42 @@ __global__ __launch_bounds__(kBlock) void scan_chan_carry_kernel(const float *__
 // steps of 256 or 512 positions, each in the same time however few the rows, where a wavefront here walks its row serially.  So few wavefronts on 100 to 1000 positions, the more
 // the fewer the states (us, positions / channels in lanes, wavefronts of whole rows in front, bf16: 16 states, 12: 100 positions 12.0 / 12.3, 196 12.1 / 19.9, 324 12.1 / 32.5; 192: 100 17.9 / 12.7,
 // 196 18.4 / 20.5, 324 18.4 / 30.8; 384: 196 27.4 / 21.1, 324 27.9 / 31.3; 768: 324 48.2 / 32.6; 4 states, 192: 77 8.1 / 7.3, 196 8.6 / 12.6; 384: 196 11.9 / 13.0, 324 12.1 / 19.2; 768: 324
-// 21.0 / 20.1), and longer ones of 4 and 8 states (768: 1225 positions of 4 60.9 / 62.1; 12: 3306 of 4 10.9 / 23.1, 16 states 29.2 / 30.7; 96: 70.5 / 54.1); single precision of an odd number of fours
-// they read in whole pieces (16 states, 192: 1764 positions 0.86 of the time here, 768 1.16).
-static bool chan_pays(const ScanArgs &a, bool vec, int in_size) {
-    if (vec && a.L % 8 == 0) return true;
+// 21.0 / 20.1), and longer ones of 8 states (12: 3306 of 4 10.9 / 23.1, 16 states 29.2 / 30.7; 96: 70.5 / 54.1).  Long rows of 4 states only while there is
+// no more than one wavefront to a SIMD (or, whole, many), and above two where the last step over there is less than half of one (time here over the time there, bf16, 1152: 625 .83, 961 1.07, 1225 .94, 1681 .96, 2401 1.32; 1536: .66, .85, .75, 1.02,
+// 1.13; 2304: .62, 1.21, 1.08, 1.13, 1.23; fp32, 768: 1332 .92, 1764 .97, 3364 1.03; 1152: 1.20, 1.22, 1.22; 3072:
+// .97, .96, 2116 .94).
+//
+// Single precision of an odd number of fours (whole): those kernels read it in whole pieces and are ahead longer, by 1808 measured sizes (time here over the time there; 16 states: 96 wavefronts of
+// 68 positions .91, of 100 1.11; 192: 100 .92, 132 1.10; 384: 196 .98; 768: 324 .84; 1152: 484 1.07; 1536: 484 .84; 576: 676 .98, 900 1.12; 768: 900 .88; 8 states, 384: 196 1.17, 576 .85; 4 states, 2304: 324 .85,
+// 484 .98, 3072 .77, 1.14; 1152: 1028 .80, 1332 1.20, 3364 1.22).  Beyond 1024 positions on fewer than 768 wavefronts it wins where there are so few of them that rows are cut, and not
+// right behind a step of 512 or, from 2048 on, of 2048 (16 states, 24: 1028 1.08, 1332 1.23, 1764 .82, 2116 1.32, 3364 1.30; 32 states: 1.02 at most up to 2048, 1.07, 1.05, 5476 .81).
+static bool chan_pays(const ScanArgs &a, bool whole, int in_size, bool maps) {
+    if (whole && a.L % 8 == 0) return true;
     const int64_t units = (int64_t)a.batch * (a.dim / a.dim_per_group) * ((a.dim_per_group + kChanBlock - 1) / kChanBlock);
     const int at = a.N == 4 ? 0 : a.N == 8 ? 1 : a.N == 16 ? 2 : 3;
-    constexpr int kAlways[4] = {56, 64, 104, 104};                // positions up to which a wavefront's walk is as short as a step
-    constexpr int kFrom[4] = {45, 55, 60, 60}, kPerTen[4] = {36, 27, 24, 19};      // wavefronts wanted per 10 positions behind the first ones, up to 512 positions
-    constexpr int kMedium[4] = {1024, 704, 576, 576};             // wavefronts wanted up to 1024 positions
-    if (a.L <= kAlways[at]) return true;
-    if (a.L <= 512) return 10 * units >= (int64_t)kPerTen[at] * (a.L - kFrom[at]);
-    if (a.L <= 1024) return units >= kMedium[at];
-    if (vec && units > 48 && units < 768) return false;
+    const int always[4] = {56, 64, whole ? 72 : 104, 104};        // positions up to which a wavefront's walk is as short as a step
+    const int per_ten[4] = {36, whole && !maps ? 28 : 27, whole ? 28 : 24, 19};         // wavefronts wanted per 10 positions behind the first ones, up to 512 positions
+    constexpr int kFrom[4] = {45, 55, 60, 60};
+    const int medium[4] = {1024, 704, whole ? 640 : 576, whole ? 640 : 576};       // wavefronts wanted up to 1024 positions
+    if (a.L <= always[at]) return true;
+    if (a.N == 4 && !maps && (a.L > 1300 ? units > 1024 && !(whole && units > 2560) : a.L > 512 ? units > 2048 && (a.L - 1) % 512 >= 256 : whole && a.L > 400)) return false;
+    if (a.L <= 512) return 10 * units >= (int64_t)per_ten[at] * (a.L - kFrom[at]);
+    if (a.L <= 1024) return units >= medium[at];
+    if (whole && units < 768) return units <= 48 && (a.N == 16 ? a.L > 1536 && a.L <= 2048 : a.N == 32 && (a.L <= 2048 || a.L > 4096));
     if (a.N == 4) return units >= (in_size == 4 ? 768 : 1024);
     if (a.N == 8) return units >= 576;
     return a.N == 32 || a.L <= 2048 || units >= 64;
 }
 
 bool scan_chan_eligible(const ScanArgs &a, bool vec, int in_size, bool maps) {
-    // With CrossScan folded in the other kernels' lead on few wavefronts is not worth the four copies and another launch (forward_core of 4 x 128 maps of 19 x 19,
-    // 16 states in bf16, 87 us, 106 apart).
     // N/4 states per lane; at least two blocks of channels per group; a block's rows within 32-bit byte offsets
     for (int64_t s : {a.u_ds, a.dl_ds, a.o_ds})
         if (s < 0 || (kChanBlock - 1) * s + a.L > kNowhere / 2 / 4) return false;
     for (int64_t s : {a.B_ns, a.C_ns})
         if (s < 0 || (a.N - 1) * s + a.L > kNowhere / 2 / 4) return false;
-    return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.dim_per_group >= 32 && ((maps && a.N >= 16) || chan_pays(a, vec, in_size));
+    // With CrossScan folded in the other kernels' lead on few wavefronts is not worth the four copies and another launch (forward_core of 4 x 128 maps of 19 x 19,
+    // 16 states in bf16, 87 us, 106 apart).
+    return (a.N == 4 || a.N == 8 || a.N == 16 || a.N == 32) && a.dim_per_group >= 32 && ((maps && a.N >= 16) || chan_pays(a, vec, in_size, maps));
 }
 
 // The number of segments of a row (1: not cut) and the length of all but the last, which has at least 72 positions: a segment's N + 3
