@@ -184,6 +184,8 @@ def test_scan_bwd_kernel_choice():
         assert name(batch, dim, L, N, 4) == kernel, (batch, dim, L, N)
     for L in list(range(512, 2600)) + [3025, 3481, 3844, 3969, 65537]:      # every length of the rule's range, not only those that equal segments fill
         assert all(name(1, 256, L, N, 4, dtype) == "chan" for N in (8, 16) for dtype in (_lib.SS2D_BF16, _lib.SS2D_F32)), L
+    f32, bf16 = _lib.SS2D_F32, _lib.SS2D_BF16           # 8 states: nearly whole passes of 256 positions
+    assert [name(32, 384, L, 8, 4, dtype) for dtype in (f32, bf16) for L in (208, 209, 256, 257)] == ["chan", "states", "states", "chan"] + ["chan"] * 4
     assert name(0, 384, 3136, 1, 4) == "none"
     assert _scan_bwd_plan(2, 384, 3136, 1, 5) == _lib.SS2D_EINVAL
     assert _scan_bwd_plan(1, 16, 400_000, 40, 4) == _lib.SS2D_ENOTSUP

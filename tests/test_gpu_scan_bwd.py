@@ -383,3 +383,15 @@ def test_operators_are_made_in_the_extension(N, delta_dim, monkeypatch):
         with _Watching():
             call()
         assert made == [native]
+
+
+@pytest.mark.parametrize("L", [209, 225, 255, 256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_scan_bwd_eight_states_of_nearly_a_pass(L, dtype):
+    """209 to 256 positions of 8 states: a channel per lane in 16 bits, positions in lanes in single precision.  (Bounds as for CHANNEL_CASES.)"""
+    print("CASE scan-bwd-eight-states", L, dtype, flush=True)
+    u, delta, A, B, C, D, bias, dout = make(9 * L, 216, 48, 1, 8, L, dtype)
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == ("states" if dtype == torch.float32 else "chan")
+    want = torch_ref.selective_scan_grads(u.float(), delta.float(), A, B.float(), C.float(), D, bias, dout.float(), True)
+    got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, True, 1)
+    compare(got, want, 1e-4 if dtype == torch.float32 else 3e-2, "eight states")

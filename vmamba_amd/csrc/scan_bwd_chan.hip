@@ -491,16 +491,17 @@ static_assert(kBcSub * 4 + 1 >= 2 * 16 && kBcSub * 5 >= 2 * (16 + 2), "a segment
 
 // Where a channel per lane is ahead of positions in lanes (scan_bwd_states_kernel).  That one works in passes of 256 positions, and a few
 // images of one or two passes are done before two more kernels have been launched here; many of them or longer rows fill the chip either way,
-// and this kernel has half the instructions per (position, state).  us, positions / channels in lanes, wavefronts of whole rows in front, bf16: 16 states, 12: 196 positions 20 / 44,
-// 400 36 / 46, 576 51 / 46, 3136 202 / 65; 192: 56 31 / 25, 196 44 / 48, 400 74 / 70, 784 140 / 110; 768: 56 76 / 27, 196 109 / 83, 784 422 / 224; 8 states, 1536: 196 99 / 87, 255
-// 110 / 106; 512 of two wavefronts per workgroup (32 channels), in fp32: 130 48 / 45, 1225 209 / 227.  Of 4 states a lane has one, and the work per position is as much as that per state: 192: 784 73 / 51;
-// 768: 56 28 / 17, 196 41 / 46, 784 132 / 133; 1536: 400 114 / 127.
-static bool bwd_chan_pays(const ScanBwdArgs &a) {
+// and this kernel has half the instructions per (position, state).  us, positions / channels in lanes, wavefronts of whole rows in front (bf16: 16 states, 12: 196 positions 20 / 44,
+// 400 36 / 46, 576 51 / 46, 3136 202 / 65; 192: 56 31 / 25, 196 44 / 48, 400 74 / 70, 784 140 / 110; 768: 56 76 / 27, 196 109 / 83, 784 422 / 224; 8 states, 1536: 196 99 / 87;
+// 512 of two wavefronts per workgroup (32 channels), in fp32: 130 48 / 45, 1225 209 / 227).  8 states on 209 to 256 positions, nearly whole passes over there (225 and 255): bf16, 648 wavefronts 80 / 69,
+// 81 / 73, 960 105 / 84, 107 / 89, 1536 105 / 100, 107 / 108, 3072 201 / 179, 205 / 200; fp32, 1536 94 / 111, 96 / 121, 3072 188 / 196, 182 / 217.  Of 4 states a lane has one, and the work per position is as much as that per state (192: 784 73 / 51;
+// 768: 56 28 / 17, 196 41 / 46, 784 132 / 133; 1536: 400 114 / 127).
+static bool bwd_chan_pays(const ScanBwdArgs &a, int in_size) {
     const int64_t units = (int64_t)a.batch * (a.dim / a.dim_per_group) * ((a.dim_per_group + kBcChan - 1) / kBcChan);
     if (a.N == 4) return a.L > 256 ? units <= 192 : a.L <= 96 && units >= 512;
     if (a.dim_per_group < 48 && a.L > 96 && (a.L < 512 || units > 192)) return false;
     if (a.L >= 512) return true;
-    return units >= (a.L > 256 ? 192 : a.L > 128 ? 640 : 256) && (a.N == 16 || a.L <= 208 || a.L > 256);
+    return units >= (a.L > 256 ? 192 : a.L > 128 ? 640 : 256) && (a.N == 16 || a.L <= 208 || a.L > 256 || in_size == 2);
 }
 
 // False: no grid for it.
@@ -521,7 +522,7 @@ static bool bwd_chan_geom(const ScanBwdArgs &a, BwdChanGeom &geo, uint32_t &n_wg
 bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size) {
     BwdChanGeom geo;
     uint32_t n_wg;
-    if ((a.N != 4 && a.N != 8 && a.N != 16) || a.dim_per_group < kBcChan || !bwd_chan_pays(a) || !bwd_chan_geom(a, geo, n_wg)) return false;
+    if ((a.N != 4 && a.N != 8 && a.N != 16) || a.dim_per_group < kBcChan || !bwd_chan_pays(a, in_size) || !bwd_chan_geom(a, geo, n_wg)) return false;
     // the gradients' memory holds the segments' states between the passes
     auto apart = [&](const void *x, int64_t elems, int size) {
         const uintptr_t first = reinterpret_cast<uintptr_t>(x), last = first + (uintptr_t)(elems * size);
