@@ -186,6 +186,11 @@ def test_scan_bwd_kernel_choice():
         assert all(name(1, 256, L, N, 4, dtype) == "chan" for N in (8, 16) for dtype in (_lib.SS2D_BF16, _lib.SS2D_F32)), L
     f32, bf16 = _lib.SS2D_F32, _lib.SS2D_BF16           # 8 states: nearly whole passes of 256 positions
     assert [name(32, 384, L, 8, 4, dtype) for dtype in (f32, bf16) for L in (208, 209, 256, 257)] == ["chan", "states", "states", "chan"] + ["chan"] * 4
+    # 8 states, many long rows: where the other kernel's workgroups and passes are full of positions
+    for shape, dtype, kernel in (((32, 384, 1369), f32, "states"), ((32, 384, 1024), f32, "chan"), ((31, 384, 1369), f32, "chan"), ((64, 384, 1024), f32, "states"), ((64, 384, 784), f32, "chan"),
+                                 ((48, 384, 1024), f32, "chan"), ((64, 768, 484), f32, "states"), ((64, 768, 484), bf16, "states"), ((64, 384, 961), bf16, "chan"), ((64, 768, 441), bf16, "chan")):
+        assert name(*shape, 8, 4, dtype) == kernel, (shape, dtype)
+        assert name(*shape, 16, 4, dtype) == "chan"
     assert name(0, 384, 3136, 1, 4) == "none"
     assert _scan_bwd_plan(2, 384, 3136, 1, 5) == _lib.SS2D_EINVAL
     assert _scan_bwd_plan(1, 16, 400_000, 40, 4) == _lib.SS2D_ENOTSUP

@@ -496,10 +496,15 @@ static_assert(kBcSub * 4 + 1 >= 2 * 16 && kBcSub * 5 >= 2 * (16 + 2), "a segment
 // 512 of two wavefronts per workgroup (32 channels), in fp32: 130 48 / 45, 1225 209 / 227).  8 states on 209 to 256 positions, nearly whole passes over there (225 and 255): bf16, 648 wavefronts 80 / 69,
 // 81 / 73, 960 105 / 84, 107 / 89, 1536 105 / 100, 107 / 108, 3072 201 / 179, 205 / 200; fp32, 1536 94 / 111, 96 / 121, 3072 188 / 196, 182 / 217.  Of 4 states a lane has one, and the work per position is as much as that per state (192: 784 73 / 51;
 // 768: 56 28 / 17, 196 41 / 46, 784 132 / 133; 1536: 400 114 / 127).
-static bool bwd_chan_pays(const ScanBwdArgs &a, int in_size) {
+//
+// 8 states on more than 256 positions, many wavefronts: the other kernel's time depends on how well its grid (1024 workgroups at a time) and its passes are filled, by up to 1.5
+// (fp32, 1024 positions: 1152 wavefronts 433 us, 1536 419).  Full, it is ahead (fp32, 768: 1024 222 / 211, 1369 342 / 399, 2304 503 / 558; 1536: 484 201 / 198, 1024 419 / 463, 1369 634 / 783; 3072: 484 390 / 519;
+// bf16, 1536: 484 214 / 198, 961 472 / 488; 3072: 484 393 / 448, 961 894 / 976), and not where a third of it waits (fp32, 1152: 1024 433 / 357, 2304 995 / 830; 1536: 784 412 / 384; 3072: 784 795 / 738).
+static bool bwd_chan_pays(const ScanBwdArgs &a, int in_size, bool others_full) {
     const int64_t units = (int64_t)a.batch * (a.dim / a.dim_per_group) * ((a.dim_per_group + kBcChan - 1) / kBcChan);
     if (a.N == 4) return a.L > 256 ? units <= 192 : a.L <= 96 && units >= 512;
     if (a.dim_per_group < 48 && a.L > 96 && (a.L < 512 || units > 192)) return false;
+    if (a.N == 8 && a.L > 256 && others_full && (in_size == 4 ? units >= 768 && units * a.L >= 1 << 20 : units >= 2048)) return false;
     if (a.L >= 512) return true;
     return units >= (a.L > 256 ? 192 : a.L > 128 ? 640 : 256) && (a.N == 16 || a.L <= 208 || a.L > 256 || in_size == 2);
 }
@@ -519,10 +524,10 @@ static bool bwd_chan_geom(const ScanBwdArgs &a, BwdChanGeom &geo, uint32_t &n_wg
     return true;
 }
 
-bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size) {
+bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size, bool others_full) {
     BwdChanGeom geo;
     uint32_t n_wg;
-    if ((a.N != 4 && a.N != 8 && a.N != 16) || a.dim_per_group < kBcChan || !bwd_chan_pays(a, in_size) || !bwd_chan_geom(a, geo, n_wg)) return false;
+    if ((a.N != 4 && a.N != 8 && a.N != 16) || a.dim_per_group < kBcChan || !bwd_chan_pays(a, in_size, others_full) || !bwd_chan_geom(a, geo, n_wg)) return false;
     // the gradients' memory holds the segments' states between the passes
     auto apart = [&](const void *x, int64_t elems, int size) {
         const uintptr_t first = reinterpret_cast<uintptr_t>(x), last = first + (uintptr_t)(elems * size);

@@ -45,8 +45,9 @@ struct ScanBwdArgs {
     int64_t g_bs, g_gs, g_ns;      // strides of dB / dC (contiguous (batch, groups, N, L))
 };
 
-// scan_bwd_chan.hip: the backward with a channel per lane, for what scan_bwd_chan_takes.
-bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size);
+// scan_bwd_chan.hip: the backward with a channel per lane, for what scan_bwd_chan_takes (others_full: the kernel with positions in lanes would have 0.88 of its
+// lanes at work or more).
+bool scan_bwd_chan_takes(const ScanBwdArgs &a, int in_size, int dy_size, bool others_full);
 int launch_scan_bwd_chan(const ScanBwdArgs &a, int in_dtype, int dout_dtype, hipStream_t stream);
 
 // Arguments of the fused core kernels (ss2d_core.hip, ss2d_core_small.hip): the C ABI's ss2d_core_params with derived

@@ -896,11 +896,6 @@ static int plan_scan_bwd(const ss2d_scan_bwd_params *q, ScanBwdArgs &a, BwdPlan 
     a.do_bs = q->dout_batch_stride; a.do_ds = q->dout_d_stride;
     a.g_ns = q->seqlen; a.g_gs = (int64_t)q->dstate * q->seqlen; a.g_bs = (int64_t)q->n_groups * a.g_gs;
     const int in_size = q->in_dtype == SS2D_F32 ? 4 : 2, dy_size = q->dout_dtype == SS2D_F32 ? 4 : 2;
-    // several states and enough channels per group: one channel per lane
-    if (scan_bwd_chan_takes(a, in_size, dy_size)) {
-        plan.kernel = SS2D_SCAN_BWD_KERNEL_CHAN;
-        return SS2D_OK;
-    }
     auto dwords_ok = [&](int items) {                            // rows of whole dwords (with one position per lane elements are read)
         if (items == 1) return true;
         auto odd = [](const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 3) != 0; };
@@ -945,6 +940,12 @@ static int plan_scan_bwd(const ss2d_scan_bwd_params *q, ScanBwdArgs &a, BwdPlan 
         chunk = (a.dim_per_group + cpg - 1) / cpg;               // even split
         const int64_t n = images * cpg;
         const size_t smem = smem_of(chunk);
+        // several states and enough channels per group: one channel per lane, unless these workgroups' rounds through the chip are nearly full of positions
+        const bool full = 25 * a.dim_per_group * images * a.L >= 22 * ((n + want_wg - 1) / want_wg * want_wg) * chunk * n_pass * kWave * items;
+        if (scan_bwd_chan_takes(a, in_size, dy_size, full)) {
+            plan.kernel = SS2D_SCAN_BWD_KERNEL_CHAN;
+            return SS2D_OK;
+        }
         plan.items = items; plan.vec = dwords_ok(items);
         plan.n_waves = n_waves; plan.chunk = (int)chunk; plan.cpg = (int)cpg;
         plan.n_wg = n; plan.smem = smem;
