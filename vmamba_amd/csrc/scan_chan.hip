@@ -15,7 +15,7 @@
 //            broadcasts; the four sets' sums meet in DPP additions that leave 4 positions with each set (sum_over_sets);
 //   output   through the dl tile back to lane (r, q), which adds the skip term and stores.
 // What bounds it: vector issue.  64 maps of 192 x 56 x 56 as four directions, 16 states: 624 us, 98 % of it issuing, at 4.8 cycles per vector
-// instruction and 1.9 GHz; 6.5 instructions per (position, state) of which the recurrence is 5 with one exp2 at 8 cycles.  A workgroup of 64
+// instruction and 1.9 GHz; 6.7 instructions per (position, state) of which the recurrence is 5 with one exp2 at 8 cycles.  A workgroup of 64
 // channels whose wavefronts share out the states and meet at four barriers per step, B and C in scalar registers (a fused multiply-add
 // with a scalar operand takes twice the cycles): 641; 16 images of 192 x 28 x 28: 90, now 68, as there are four times as many wavefronts
 // as blocks of 64 channels and each is done on its own.
